@@ -9,7 +9,9 @@ import torch
 from torch import nn
 
 from ..difflogic import GroupSum, LogicLayer
-from ..difflogic.difflogic import logic_layer_group_sum
+from ..difflogic.difflogic import _feature_major, _has_forward_hooks, logic_layer_group_sum
+from ..difflogic.fc_tree import tree_packed, tree_plan, tree_train
+from ..difflogic.packbitstensor import PackBitsTensor
 from .convlogic_layer import ConvLogicLayer
 
 
@@ -21,13 +23,15 @@ _FOLD_PLANS = weakref.WeakKeyDictionary()
 _PREFOLD_MIN_ELEMS = 20 << 19                                     # 512 Ki rows of logits
 
 
-def _prefold(owner, network, x, mode=True):
-    """Folds the logits of all layers of a training step in ONE launch and leaves each layer its (probabilities,
-    coefficients): softmax and fold are then no part of the layers' forward launches -- the LogicLayers run their plain
-    streaming kernel, the deep blocks skip their set-up launch.  Same values as the per-layer folds (tested)."""
+def _prefold(owner, layers, x, mode=True):
+    """Folds the logits of `layers` (a network's, in order) for a training step in ONE launch and leaves each layer its
+    (probabilities, coefficients): softmax and fold are then no part of the layers' forward launches -- the LogicLayers run
+    their plain streaming kernel, the deep blocks skip their set-up launch.  Same values as the per-layer folds (tested)."""
     from ..hip import difflogic_hip
     cache = _FOLD_PLANS.get(owner)
-    if cache is not None and cache[0] == (x.dtype, x.device):
+    if cache is not None and cache[0] != (x.dtype, x.device, len(layers)):
+        cache = None
+    if cache is not None:
         _, picked, plan = cache
         weights = [m._parameters["weights"] for m in picked]
         if plan is None:                                             # nothing to fold when the cache was made: look again
@@ -35,12 +39,11 @@ def _prefold(owner, network, x, mode=True):
         elif not (plan.matches(weights) and all(m.prefold_candidate() is w for m, w in zip(picked, weights))):
             cache = None
     if cache is None:
-        layers = [m for m in network if isinstance(m, (ConvLogicLayer, LogicLayer))]
         picked = [m for m in layers for w in [m.prefold_candidate()] if w is not None and w.dtype == x.dtype and w.device == x.device]
         picked = picked[:difflogic_hip.FOLD_MANY_MAX]
         weights = [m._parameters["weights"] for m in picked]
         plan = difflogic_hip.FoldPlan([w.detach() for w in weights]) if len(picked) >= 2 else None
-        _FOLD_PLANS[owner] = ((x.dtype, x.device), picked, plan)
+        _FOLD_PLANS[owner] = ((x.dtype, x.device, len(layers)), picked, plan)
     if plan is None:
         return
     # An eager step of a small network is bound by the host, where the bookkeeping of this launch costs more than the
@@ -52,17 +55,61 @@ def _prefold(owner, network, x, mode=True):
         m.set_prefold(probs, folded)
 
 
+def _tree_tail(net):
+    """The last four modules of a network -- three LogicLayers and a GroupSum -- when nothing but a call of the modules
+    themselves stands against evaluating them as one operation (difflogic/fc_tree.py), else None."""
+    if len(net) < 4 or net._forward_hooks or net._forward_pre_hooks:
+        return None
+    tail = [net[i] for i in range(len(net) - 4, len(net))]
+    *layers, gs = tail
+    if not all(type(m) is LogicLayer and m.implementation == "cuda" and m.grad_factor == 1.0 for m in layers) or type(gs) is not GroupSum:
+        return None
+    if any(_has_forward_hooks(m) for m in tail) or layers[-1].out_dim % gs.k != 0 or gs.tau == 0:
+        return None
+    for m in layers:
+        w = m._parameters["weights"]
+        if not (w.is_cuda and w.dtype == torch.float32 and w.is_contiguous() and w.device == layers[0]._parameters["weights"].device):
+            return None
+    return layers, gs
+
+
 def _forward(owner, x):
-    """The network on x.  In training on the GPU two things happen that a plain nn.Sequential call would not do: the
-    logits of all layers are folded in one launch where that pays (`prefold`), and the last LogicLayer and the GroupSum
-    behind it run as one autograd node (`fused_tail`, default on), whose backward needs no GroupSum launch."""
+    """The network on x.  Three things happen that a plain nn.Sequential call would not do: the three LogicLayers and the
+    GroupSum at its end are evaluated as one operation where their wiring allows (`tree_tail`, default on; training steps
+    and packed inference); in training the logits of the other layers are folded in one launch where that pays (`prefold`), and a
+    last LogicLayer and GroupSum that do not run as trees run as one autograd node (`fused_tail`, default on), whose
+    backward needs no GroupSum launch."""
     net = owner.network
+    n = len(net)
+    tail = _tree_tail(net) if owner.__dict__.get("tree_tail", True) else None
+    if isinstance(x, PackBitsTensor):
+        plan = tree_plan(*tail[0]) if tail is not None and not owner.training and x.is_cuda and x.bit_count == 64 else None
+        if plan is None:
+            return net(x)
+        h = x
+        for i, m in enumerate(net):
+            if i == n - 4:
+                break
+            h = m(h)
+        if type(h) is not PackBitsTensor or h.image or h.t.shape[0] != tail[0][0].in_dim or not h.t.is_contiguous():
+            return _rest(net, n - 4, h)
+        return tree_packed(tail[0], tail[1].k, h, plan)
     if not (owner.training and isinstance(x, torch.Tensor) and x.is_cuda and torch.is_grad_enabled()):
         return net(x)
+    plan = tree_plan(*tail[0]) if tail is not None and x.dtype == torch.float32 and x.shape[0] % 4 == 0 and x.shape[0] > 0 else None
     mode = owner.__dict__.get("prefold", True)                       # True: where it pays, "always", False
+    layers = [m for m in net if isinstance(m, (ConvLogicLayer, LogicLayer))]
     if mode:
-        _prefold(owner, net, x, mode)
-    n = len(net)
+        _prefold(owner, layers if plan is None else layers[:-3], x, mode)
+    if plan is not None:
+        h = x
+        for i, m in enumerate(net):
+            if i == n - 4:
+                break
+            h = m(h)
+        if h.dim() == 2 and h.shape[1] == tail[0][0].in_dim and h.dtype == torch.float32:
+            return tree_train(tail[0], tail[1], _feature_major(h), plan)
+        return _rest(net, n - 4, h)
     if (owner.__dict__.get("fused_tail", True) and n >= 2 and isinstance(net[n - 2], LogicLayer) and isinstance(net[n - 1], GroupSum)
             and not (net._forward_hooks or net._forward_pre_hooks)):
         h = x
@@ -72,6 +119,13 @@ def _forward(owner, x):
             h = m(h)
         return logic_layer_group_sum(net[n - 2], net[n - 1], h)
     return net(x)
+
+
+def _rest(net, i0, h):
+    for i, m in enumerate(net):
+        if i >= i0:
+            h = m(h)
+    return h
 
 
 def _block(c_in, c_out, implementation, **kw):

@@ -1,0 +1,654 @@
+// The fully connected end of a logic network as ONE operation: a LogicLayer, two halving LogicLayers (2 out_dim = in_dim, every
+// input read by exactly one neuron operand) and the GroupSum behind them (src/convlogic/model.py:49-57,102-107).
+//
+// Where every neuron of the first two layers is read exactly once, neuron j of the third layer is the root of a tree of
+// seven gates -- four of the first layer, two of the second, itself -- over eight rows of the input, and no other root
+// shares any of them.  So the three layers need no activations of their own: a wavefront reads the eight rows of a root,
+// evaluates the tree in registers and adds the root's value to its class.
+//   forward           8 row reads per root instead of 8 + 4 writes + 4 reads + 2 + 2 + 1 + 1 (and the GroupSum's pass)
+//   backward          the tree again; the gradient of the root's row is grad_out[b][class] / tau; the 28 coefficient sums
+//                     give the gradients of the seven neurons' logits, and the gradients of the eight operands go out as
+//                     rows of a buffer ordered by input feature, so that
+//   input gradient    is a sum of consecutive rows per feature: no wiring, no gather, no atomics, fixed order
+//   packed inference  the same tree on 64 samples per word (three bit operations per gate and 32 samples), the class counts
+//                     in vertical counters
+// Measured, first layer to class sums (kernels of the four modules -> here): forward 36 -> 21 us and backward 58 -> 43 us on 4096
+// features, 40960 / 20480 / 10240 neurons, batch 256; 1.31 -> 0.50 ms and 2.19 -> 1.63 ms on 131072 features, 2.62 M / 1.31 M /
+// 655 k neurons, batch 128; packed inference of the former at 65 536 samples 273 -> 78 us.
+// What bounds it: the row reads (2.7 GB of 512-byte pieces through L2 and the last-level cache in 375 us on the large shape) and,
+// backward, the 2.7 GB of operand gradients written once and read once.  Keeping the first layer's output gradient instead (half
+// the bytes to write) needs a gather that reads every row twice plus the other operand's row: 1133 us in place of the
+// 536 us of the sum over consecutive rows.
+// Activations are feature-major with a row pitch that is a multiple of 4; samples from `batch` up to the pitch are computed
+// like any other, carry no gradient and are not written to the result.
+#include <algorithm>
+
+#include "conv_ops.h"
+
+namespace {
+
+constexpr int kTreeWaves = 4;
+constexpr int kTreeBlock = kTreeWaves * kWave;
+
+// the samples of a lane: 1, 2 or 4 consecutive ones, so that a row of 64, 128 or 256 samples fills the wavefront and the
+// root -- indices, coefficients, class -- is uniform (two roots per wavefront on rows of 128 samples need their 28
+// coefficients per lane: 168 registers in the backward kernel against 115)
+template <int V>
+struct Samples {
+    float v[V];
+};
+template <int V>
+struct SamplesRaw;
+template <>
+struct SamplesRaw<1> { using type = float; };
+template <>
+struct SamplesRaw<2> { using type = float2; };
+template <>
+struct SamplesRaw<4> { using type = float4; };
+template <int V>
+__device__ __forceinline__ Samples<V> load_samples(const float *p)
+{
+    return __builtin_bit_cast(Samples<V>, *reinterpret_cast<const typename SamplesRaw<V>::type *>(p));
+}
+template <int V>
+__device__ __forceinline__ void store_samples(float *p, const Samples<V> &v)
+{
+    *reinterpret_cast<typename SamplesRaw<V>::type *>(p) = __builtin_bit_cast(typename SamplesRaw<V>::type, v);
+}
+
+// a of both halves in the low half, b of both halves in the high half (v_permlane32_swap + add), and the same for the even /
+// odd rows of 16 lanes of every half
+__device__ __forceinline__ float swap_add32(float a, float b)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+    return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+__device__ __forceinline__ float swap_add16(float a, float b)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+    return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+
+// ---- coefficients ---------------------------------------------------------------------------------------------------
+// ids [roots][8]: the neurons of a tree, 0..3 of the first layer, 4..5 of the second; the root is neuron j of the third.
+// coef [roots][7][4]: fold16 of the softmax (training) or of the arg-max gate (evaluation) of their logits, in tree order, so
+// that a root's 28 coefficients are one run of 112 bytes.
+struct TreeLogits {
+    const float *l[3];
+};
+__device__ __forceinline__ const float *tree_logits(const TreeLogits &lg, const int32_t *__restrict__ ids, int j, int q)
+{
+    return q < 6 ? (q < 4 ? lg.l[0] : lg.l[1]) + (int64_t)ids[(int64_t)j * 8 + q] * 16 : lg.l[2] + (int64_t)j * 16;
+}
+// index of the first maximum (a NaN counts as the maximum), as clg_gate_argmax
+__device__ __forceinline__ int argmax16(const float *__restrict__ w)
+{
+    float best = w[0];
+    int at = 0;
+#pragma unroll
+    for (int i = 1; i < 16; ++i) {
+        const float v = w[i];
+        if (v > best || (v != v && best == best)) best = v, at = i;
+    }
+    return at;
+}
+__global__ __launch_bounds__(256) void fc_tree_fold_kernel(TreeLogits lg, const int32_t *__restrict__ ids, float *__restrict__ coef,
+                                                         int roots, int hard)
+{
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= (int64_t)roots * 7) return;
+    const int j = (int)(e / 7), q = (int)(e - (int64_t)j * 7);
+    const float *w = tree_logits(lg, ids, j, q);
+    float p[16];
+    if (hard) {
+        const int at = argmax16(w);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) p[i] = i == at ? 1.f : 0.f;
+    } else {
+        softmax16(w, p);
+    }
+    const Coef<float> c = fold16(p);
+    reinterpret_cast<float4 *>(coef)[e] = make_float4(c.ab, c.a, c.b, c.one);
+}
+
+// ---- forward ----------------------------------------------------------------------------------------------------------
+// rows [roots][8]: the input rows of a tree.  A wavefront takes a root at a time, 64 lanes x V samples.
+__device__ __forceinline__ void tree_coefs(const float *__restrict__ coef, int j, Tree<float> &t)
+{
+    const float4 *c = reinterpret_cast<const float4 *>(coef) + (int64_t)j * 7;
+#pragma unroll
+    for (int q = 0; q < 7; ++q) {
+        const float4 v = c[q];
+        t.g[q] = Coef<float>{v.x, v.y, v.z, v.w};
+    }
+}
+template <int V>
+__device__ __forceinline__ void tree_rows(const float *__restrict__ x, const int32_t *__restrict__ rows, int j, int in_dim, int64_t pitch,
+                                          int64_t s, Samples<V> (&v)[8])
+{
+    const int32_t *r = rows + (int64_t)j * 8;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) v[t] = load_samples<V>(x + (int64_t)min((uint32_t)r[t], (uint32_t)in_dim - 1u) * pitch + s);
+}
+
+// grid: (slices of a class, classes, chunks of 64 V samples).  partial [slices][k][pitch]
+template <int V>
+__global__ __launch_bounds__(kTreeBlock) void fc_tree_forward_kernel(const float *__restrict__ x, const int32_t *__restrict__ rows,
+                                                                   const float *__restrict__ coef, float *__restrict__ partial,
+                                                                   int class_rows, int k, int slices, int64_t pitch, int in_dim)
+{
+    __shared__ Samples<V> meet[kTreeWaves][kWave];
+    const int lane = threadIdx.x & (kWave - 1), wave = uniform((int)(threadIdx.x >> 6));
+    const int slice = blockIdx.x, g = blockIdx.y;
+    const int64_t s = ((int64_t)blockIdx.z * kWave + lane) * V, s_at = s < pitch ? s : 0;
+    const int r0 = (int)((int64_t)class_rows * slice / slices), r1 = (int)((int64_t)class_rows * (slice + 1) / slices);
+    Samples<V> acc = {};
+    auto value = [&](int r, Samples<V> &y) {
+        const int j = g * class_rows + r;
+        Tree<float> t;
+        tree_coefs(coef, j, t);
+        Samples<V> v[8];
+        tree_rows<V>(x, rows, j, in_dim, pitch, s_at, v);
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            float tap[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) tap[q] = v[q].v[i];
+            y.v[i] = eval_tree(t, tap).root;
+        }
+    };
+    // four roots of the wavefront in flight; summed in the order of group_sum_fm_kernel
+    int r = r0 + wave;
+    for (; r + 12 < r1; r += 16) {
+        Samples<V> y[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) value(r + 4 * u, y[u]);
+#pragma unroll
+        for (int i = 0; i < V; ++i) acc.v[i] += (y[0].v[i] + y[1].v[i]) + (y[2].v[i] + y[3].v[i]);
+    }
+    for (; r < r1; r += 4) {
+        Samples<V> y;
+        value(r, y);
+#pragma unroll
+        for (int i = 0; i < V; ++i) acc.v[i] += y.v[i];
+    }
+    meet[wave][lane] = acc;
+    __syncthreads();
+    if (wave == 0 && s < pitch) {
+        Samples<V> sum;
+#pragma unroll
+        for (int i = 0; i < V; ++i) sum.v[i] = (meet[0][lane].v[i] + meet[1][lane].v[i]) + (meet[2][lane].v[i] + meet[3][lane].v[i]);
+        store_samples<V>(partial + ((int64_t)slice * k + g) * pitch + s, sum);
+    }
+}
+
+// out[b][g] = inv_tau * sum over the slices in order, eight loads in flight
+__global__ __launch_bounds__(256) void fc_tree_finish_kernel(const float *__restrict__ partial, float *__restrict__ out, int slices, int k,
+                                                           int64_t pitch, int64_t batch, float inv_tau)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;       // sample fastest: the loads of a wavefront are contiguous
+    if (i >= batch * k) return;
+    const int g = (int)(i / batch);
+    const int64_t b = i - (int64_t)g * batch, step = (int64_t)k * pitch;
+    const float *p = partial + (int64_t)g * pitch + b;
+    float acc = 0.f;
+    for (int s = 0; s < slices; s += 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = p[(int64_t)min(s + u, slices - 1) * step];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) acc = s + u < slices ? acc + v[u] : acc;
+    }
+    out[b * k + g] = acc * inv_tau;
+}
+
+// ---- backward -----------------------------------------------------------------------------------------------------------
+// pos [roots][8]: the row of `rowgrad` an operand's gradient goes to: its place in the lists input feature -> operands.
+// The 28 sums of a wavefront are reduced and turned round together: every exchange between lane groups halves the number of
+// values a lane holds instead of repeating each value's full reduction (28 x 6 steps).  They leave as one run of 112 bytes per
+// root; what remains -- 16 gates per neuron, the softmax backward -- needs the logits of seven scattered neurons and is a
+// kernel of its own in neuron order (fc_tree_logit_grad_kernel): done here it held the wavefront for one more round trip and
+// read and wrote 64-byte pieces all over (655360 roots x 128 samples: 1742 us, 978 without it).
+__device__ __forceinline__ void tree_store_sums(float (&v)[28], float *__restrict__ sums, int j, int lane)
+{
+    const int i16 = lane & 15, o = (lane >> 4) & 1, h = lane >> 5;
+    float mine = 0.f;
+#pragma unroll
+    for (int q = 0; q < 7; ++q) {                                     // row (h, o) holds sum 2 o + h of gate q
+        const float u = row16_sum(swap_add16(swap_add32(v[4 * q], v[4 * q + 1]), swap_add32(v[4 * q + 2], v[4 * q + 3])));
+        mine = i16 == q ? u : mine;
+    }
+    if (i16 < 7) sums[(int64_t)j * 28 + 4 * i16 + 2 * o + h] = mine;
+}
+
+template <int V>
+__global__ __launch_bounds__(kTreeBlock) void fc_tree_backward_kernel(const float *__restrict__ x, const int32_t *__restrict__ rows,
+                                                                    const int32_t *__restrict__ pos, const float *__restrict__ coef,
+                                                                    const float *__restrict__ grad_out,
+                                                                    float *__restrict__ sums, float *__restrict__ rowgrad, int roots,
+                                                                    int class_rows, int k, int64_t batch, int64_t pitch, int in_dim,
+                                                                    float inv_tau)
+{
+    const int lane = threadIdx.x & (kWave - 1), wave = uniform((int)(threadIdx.x >> 6));
+    const int64_t total_rows = (int64_t)roots * 8;
+    for (int j = blockIdx.x * kTreeWaves + wave; j < roots; j += gridDim.x * kTreeWaves) {
+        Tree<float> t;
+        tree_coefs(coef, j, t);
+        const int g = j / class_rows;
+        const int32_t *pj = pos + (int64_t)j * 8;
+        float acc[28];
+#pragma unroll
+        for (int q = 0; q < 28; ++q) acc[q] = 0.f;
+        for (int64_t s0 = 0; s0 < pitch; s0 += kWave * V) {
+            const int64_t s = s0 + lane * V;
+            const bool live = s < pitch;
+            Samples<V> v[8];
+            tree_rows<V>(x, rows, j, in_dim, pitch, live ? s : 0, v);
+            float gy[V];
+#pragma unroll
+            for (int i = 0; i < V; ++i) {
+                const int64_t b = s + i;
+                const float go = grad_out[(b < batch ? b : batch - 1) * k + g] * inv_tau;
+                gy[i] = b < batch ? go : 0.f;
+            }
+#pragma unroll
+            for (int i = 0; i < V; ++i) {
+                float tap[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) tap[q] = v[q].v[i];
+                const TreeVals<float> tv = eval_tree(t, tap);
+                auto sums = [&](int q, float gq, float a, float b) {
+                    const float ga = gq * a;
+                    acc[4 * q] = fma_t(ga, b, acc[4 * q]);
+                    acc[4 * q + 1] += ga;
+                    acc[4 * q + 2] = fma_t(gq, b, acc[4 * q + 2]);
+                    acc[4 * q + 3] += gq;
+                };
+                const float g6 = gy[i];
+                sums(6, g6, tv.mid[0], tv.mid[1]);
+                const float gm[2] = {g6 * gate_da(t.g[6], tv.mid[1]), g6 * gate_db(t.g[6], tv.mid[0])};
+#pragma unroll
+                for (int m = 0; m < 2; ++m) {
+                    const float la = tv.leaf[2 * m], lb = tv.leaf[2 * m + 1];
+                    sums(4 + m, gm[m], la, lb);
+                    const float gl[2] = {gm[m] * gate_da(t.g[4 + m], lb), gm[m] * gate_db(t.g[4 + m], la)};
+#pragma unroll
+                    for (int n = 0; n < 2; ++n) {
+                        const int q = 2 * m + n;
+                        sums(q, gl[n], tap[2 * q], tap[2 * q + 1]);
+                        v[2 * q].v[i] = gl[n] * gate_da(t.g[q], tap[2 * q + 1]);
+                        v[2 * q + 1].v[i] = gl[n] * gate_db(t.g[q], tap[2 * q]);
+                    }
+                }
+                // one sample at a time: interleaved, four samples take 169 registers, so 115
+#pragma unroll
+                for (int q = 0; q < 28; ++q) asm volatile("" : "+v"(acc[q]));
+                if (i < V - 1) {
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) asm volatile("" : "+v"(v[q].v[i + 1]));
+                }
+            }
+            if (live) {
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    store_samples<V>(rowgrad + (int64_t)min((uint64_t)(uint32_t)pj[q], (uint64_t)total_rows - 1) * pitch + s, v[q]);
+            }
+        }
+        tree_store_sums(acc, sums, j, lane);
+    }
+}
+
+// Gradients of the logits, one thread per neuron of the three layers in order.  slot: where the neuron's four sums are (root * 7
+// + gate of the tree).
+struct TreeGrads {
+    float *g[3];
+    int64_t end[3];       // neurons of the first one, two, three layers
+};
+__global__ __launch_bounds__(256) void fc_tree_logit_grad_kernel(TreeLogits lg, TreeGrads gr, const float *__restrict__ sums,
+                                                               const int32_t *__restrict__ slot, int64_t slots)
+{
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= gr.end[2]) return;
+    const int layer = e < gr.end[0] ? 0 : (e < gr.end[1] ? 1 : 2);
+    const int64_t n = e - (layer ? gr.end[layer - 1] : 0);
+    const float4 s = reinterpret_cast<const float4 *>(sums)[min((uint64_t)(uint32_t)slot[e], (uint64_t)slots - 1)];
+    const float4 *w = reinterpret_cast<const float4 *>(lg.l[layer] + n * 16);
+    float4 raw[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) raw[i] = w[i];
+    float p[16], gi[16], dot = 0.f;
+    softmax16(reinterpret_cast<const float *>(raw), p);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        gi[i] = coef_transpose_row<float>(i, s.x, s.y, s.z, s.w);
+        dot = fma_t(p[i], gi[i], dot);
+    }
+    float4 *dst = reinterpret_cast<float4 *>(gr.g[layer] + n * 16);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        dst[i] = make_float4(p[4 * i] * (gi[4 * i] - dot), p[4 * i + 1] * (gi[4 * i + 1] - dot), p[4 * i + 2] * (gi[4 * i + 2] - dot),
+                             p[4 * i + 3] * (gi[4 * i + 3] - dot));
+}
+
+// gx[i] = sum of the rows start[i] .. start[i + 1] of rowgrad, eight in flight, four partial sums
+template <int V>
+__global__ __launch_bounds__(kTreeBlock) void fc_tree_gather_kernel(const float *__restrict__ rowgrad, const int64_t *__restrict__ start,
+                                                                  float *__restrict__ gx, int in_dim, int64_t pitch, int64_t total_rows)
+{
+    const int lane = threadIdx.x & (kWave - 1), wave = uniform((int)(threadIdx.x >> 6));
+    const int i = blockIdx.x * kTreeWaves + wave;
+    const int64_t s = ((int64_t)blockIdx.y * kWave + lane) * V;
+    if (i >= in_dim || s >= pitch) return;
+    const int64_t beg = clamp_index(start[i], total_rows + 1), end = clamp_index(start[i + 1], total_rows + 1);
+    Samples<V> part[4] = {};
+    const float *p = rowgrad + beg * pitch + s;
+    int64_t r = beg;
+    for (; r + 8 <= end; r += 8, p += 8 * pitch) {
+        Samples<V> v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = load_samples<V>(p + u * pitch);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+            for (int c = 0; c < V; ++c) part[u & 3].v[c] += v[u].v[c];
+    }
+    if (r < end) {
+        Samples<V> v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = load_samples<V>(p + (r + u < end ? u : 0) * pitch);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+            for (int c = 0; c < V; ++c) part[u & 3].v[c] += r + u < end ? v[u].v[c] : 0.f;
+    }
+    Samples<V> sum;
+#pragma unroll
+    for (int c = 0; c < V; ++c) sum.v[c] = (part[0].v[c] + part[1].v[c]) + (part[2].v[c] + part[3].v[c]);
+    store_samples<V>(gx + (int64_t)i * pitch + s, sum);
+}
+
+int tree_vec(int64_t pitch) { return pitch <= 64 ? 1 : (pitch <= 128 ? 2 : 4); }
+
+int check_tree(const char *name, int64_t in_dim, int64_t roots, int64_t k)
+{
+    CLG_REQUIRE(in_dim > 0 && roots > 0 && k > 0 && roots % k == 0, "%s: in_dim, roots and k must be positive and k divide roots", name);
+    CLG_REQUIRE(in_dim < (1ll << 31) && roots < (1ll << 28) && k <= 65535, "%s: in_dim below 2^31, roots below 2^28 and k up to 65535 only", name);
+    return CLG_OK;
+}
+
+// Row slices of a class, as clg_group_sum cuts them (a class sum of 65 536 values is rounded at 1e-7 of a logit in the
+// thousands: the softmax of the loss then shows the order of the additions, so the order is kept).
+int tree_slices(int64_t class_rows, int64_t batch, int64_t k)
+{
+    int64_t slices = clg_ceil_div(1024, clg_ceil_div(batch, (int64_t)kWave) * k);
+    if (class_rows <= 4096) slices = 64;                              // small classes (where the GroupSum has another kernel): for the parallelism
+    slices = std::min(slices, class_rows / (class_rows <= 4096 ? 16 : 64));
+    return (int)std::min<int64_t>(64, std::max<int64_t>(1, slices));
+}
+
+}  // namespace
+
+extern "C" int clg_fc_tree_fold(const float *logits0, const float *logits1, const float *logits2, const int32_t *ids, float *coef,
+                                int64_t roots, int hard, void *stream)
+{
+    const char *name = "clg_fc_tree_fold";
+    if (int e = check_tree(name, 1, roots, 1)) return e;
+    CLG_REQUIRE(logits0 && logits1 && logits2 && ids && coef, "%s: null pointer argument", name);
+    const TreeLogits lg = {{logits0, logits1, logits2}};
+    hipLaunchKernelGGL(fc_tree_fold_kernel, dim3((unsigned)clg_ceil_div(roots * 7, 256)), dim3(256), 0, clg_stream(stream), lg, ids, coef,
+                       (int)roots, hard);
+    CLG_CHECK_LAUNCH(name);
+    return CLG_OK;
+}
+
+extern "C" int64_t clg_fc_tree_partial_elems(int64_t roots, int64_t k, int64_t batch, int64_t pitch)
+{
+    if (roots <= 0 || k <= 0 || batch <= 0 || pitch < batch) return -1;
+    return (int64_t)tree_slices(roots / k, batch, k) * k * pitch;
+}
+
+extern "C" int clg_fc_tree_forward(const float *x, const int32_t *rows, const float *coef, float *partial, float *out, int64_t in_dim,
+                                   int64_t roots, int64_t k, int64_t batch, int64_t pitch, double tau, void *stream)
+{
+    const char *name = "clg_fc_tree_forward";
+    if (int e = check_tree(name, in_dim, roots, k)) return e;
+    CLG_REQUIRE(x && rows && coef && partial && out, "%s: null pointer argument", name);
+    CLG_REQUIRE(batch > 0 && pitch >= batch && pitch % 4 == 0 && pitch < (1ll << 28) && tau != 0.0,
+                "%s: the row pitch must be a multiple of 4 that holds the batch, tau must not be zero", name);
+    const int slices = tree_slices(roots / k, batch, k);
+    int vec = tree_vec(pitch);                                        // fewer samples per lane where the launch would have less than four wavefronts per SIMD
+    while (vec > 1 && (int64_t)slices * k * clg_ceil_div(pitch, (int64_t)kWave * vec) * kTreeWaves < 4096) vec /= 2;
+    const dim3 grid((unsigned)slices, (unsigned)k, (unsigned)clg_ceil_div(pitch, (int64_t)kWave * vec));
+    CLG_REQUIRE(grid.z <= 65535, "%s: batch too large", name);
+    hipStream_t st = clg_stream(stream);
+#define CLG_TREE_F(V)                                                                                                        \
+    hipLaunchKernelGGL((fc_tree_forward_kernel<V>), grid, dim3(kTreeBlock), 0, st, x, rows, coef, partial, (int)(roots / k), (int)k, \
+                       slices, pitch, (int)in_dim)
+    if (vec == 1) CLG_TREE_F(1);
+    else if (vec == 2) CLG_TREE_F(2);
+    else CLG_TREE_F(4);
+#undef CLG_TREE_F
+    CLG_CHECK_LAUNCH(name);
+    hipLaunchKernelGGL(fc_tree_finish_kernel, dim3((unsigned)clg_ceil_div(batch * k, 256)), dim3(256), 0, st, (const float *)partial, out, slices,
+                       (int)k, pitch, batch, 1.f / (float)tau);
+    CLG_CHECK_LAUNCH(name);
+    return CLG_OK;
+}
+
+extern "C" int clg_fc_tree_backward(const float *x, const int32_t *rows, const int32_t *pos, const int32_t *slot, const float *coef,
+                                    const float *grad_out, const float *logits0, const float *logits1, const float *logits2, float *grad0,
+                                    float *grad1, float *grad2, float *rowgrad, float *sums, const int64_t *start, float *grad_x,
+                                    int64_t in_dim, int64_t roots, int64_t k, int64_t batch, int64_t pitch, double tau, void *stream)
+{
+    const char *name = "clg_fc_tree_backward";
+    if (int e = check_tree(name, in_dim, roots, k)) return e;
+    CLG_REQUIRE(x && rows && pos && slot && coef && grad_out && logits0 && logits1 && logits2 && grad0 && grad1 && grad2 && rowgrad && sums && start &&
+                    grad_x, "%s: null pointer argument", name);
+    CLG_REQUIRE(batch > 0 && pitch >= batch && pitch % 4 == 0 && pitch < (1ll << 28) && tau != 0.0,
+                "%s: the row pitch must be a multiple of 4 that holds the batch, tau must not be zero", name);
+    const int vec = tree_vec(pitch);
+    hipStream_t st = clg_stream(stream);
+    const TreeLogits lg = {{logits0, logits1, logits2}};
+    const TreeGrads gr = {{grad0, grad1, grad2}, {4 * roots, 6 * roots, 7 * roots}};
+    const dim3 grid((unsigned)clg_ceil_div(roots, kTreeWaves));
+    const dim3 ggrid((unsigned)clg_ceil_div(in_dim, kTreeWaves), (unsigned)clg_ceil_div(pitch, (int64_t)kWave * vec));
+    CLG_REQUIRE(ggrid.y <= 65535, "%s: batch too large", name);
+#define CLG_TREE_B(V)                                                                                                            \
+    do {                                                                                                                         \
+        hipLaunchKernelGGL((fc_tree_backward_kernel<V>), grid, dim3(kTreeBlock), 0, st, x, rows, pos, coef, grad_out, sums, rowgrad, (int)roots, \
+                           (int)(roots / k), (int)k, batch, pitch, (int)in_dim, 1.f / (float)tau);                               \
+        hipLaunchKernelGGL((fc_tree_gather_kernel<V>), ggrid, dim3(kTreeBlock), 0, st, (const float *)rowgrad, start, grad_x,    \
+                           (int)in_dim, pitch, roots * 8);                                                                       \
+    } while (0)
+    if (vec == 1) CLG_TREE_B(1);
+    else if (vec == 2) CLG_TREE_B(2);
+    else CLG_TREE_B(4);
+#undef CLG_TREE_B
+    CLG_CHECK_LAUNCH(name);
+    hipLaunchKernelGGL(fc_tree_logit_grad_kernel, dim3((unsigned)clg_ceil_div(7 * roots, 256)), dim3(256), 0, st, lg, gr, (const float *)sums, slot,
+                       7 * roots);
+    CLG_CHECK_LAUNCH(name);
+    return CLG_OK;
+}
+
+// ---- packed inference ---------------------------------------------------------------------------------------------------
+// x int64 words [in_dim, words], 64 samples per word.  codes [roots] = tree_code() of the arg-max gates: three bits per gate
+// and the root's constant, so that a gate is three 3-input bit operations with one mask each.
+//
+// Lanes run along words and, where a row has fewer than 64, along roots as well (cols_log2: log2 of the words a workgroup
+// takes); a lane counts the 64 bit positions of its word over its roots in vertical counters, the workgroup adds the counters
+// as binary numbers and writes (or, with several slices of a class, atomically adds: integers, any order) the class counts.
+// WIDE (64 words): the root is uniform, rows and masks come through the scalar cache.  Workgroups are numbered so that an XCD
+// works on one block of 64 words at a time: in_dim x 512 bytes of input then stay in its L2.
+// 4096 features, 10240 roots, 65 536 samples: 671 MB of row reads from L2 in 78 us = 8.6 TB/s (the three evaluation kernels and
+// the counting kernel: 273 us).
+namespace {
+
+__global__ __launch_bounds__(256) void fc_tree_codes_kernel(TreeLogits lg, const int32_t *__restrict__ ids, uint32_t *__restrict__ codes,
+                                                          int roots, int32_t *__restrict__ counts, int64_t n_counts)
+{
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    for (int64_t i = e; i < n_counts; i += (int64_t)gridDim.x * 256) counts[i] = 0;   // (for the counting kernel's atomics)
+    const int j = (int)(e >> 3), q = (int)(e & 7);                    // eight lanes per root, one gate each
+    int id = 0;
+    if (j < roots && q < 7) id = argmax16(tree_logits(lg, ids, j, q));
+    uint8_t gate[7];
+#pragma unroll
+    for (int t = 0; t < 7; ++t) gate[t] = (uint8_t)__shfl(id, (threadIdx.x & 56) + t, kWave);
+    if (j < roots && q == 0) codes[j] = tree_code(gate);
+}
+
+constexpr int kTreePlanes = 14;                                      // a workgroup takes at most 2^14 - 1 roots
+constexpr int kPackedWaves = 16;
+__device__ __forceinline__ void carry_save(uint32_t &hi, uint32_t &lo, uint32_t a, uint32_t b, uint32_t c)
+{
+    const uint32_t u = a ^ b;
+    hi = (a & b) | (u & c);
+    lo = u ^ c;
+}
+__device__ __forceinline__ void add_counts(uint32_t (&plane)[kTreePlanes], const uint32_t (&other)[kTreePlanes])
+{
+    uint32_t carry = 0;
+#pragma unroll
+    for (int q = 0; q < kTreePlanes; ++q) {
+        const uint32_t b = other[q], u = plane[q] ^ b, c = (plane[q] & b) | (u & carry);
+        plane[q] = u ^ carry;
+        carry = c;
+    }
+}
+
+template <bool WIDE>
+__global__ __launch_bounds__(kPackedWaves *kWave) void fc_tree_packed_kernel(const uint32_t *__restrict__ x, const int32_t *__restrict__ rows,
+                                                                            const uint32_t *__restrict__ codes, int32_t *__restrict__ out,
+                                                                            int class_rows, int k, int slices, uint32_t words,
+                                                                            int64_t samples, int in_dim, int cols_log2, unsigned col_blocks)
+{
+    __shared__ uint32_t meet[kPackedWaves][kTreePlanes][kWave];
+    const int lane = threadIdx.x & (kWave - 1), wave = uniform((int)(threadIdx.x >> 6));
+    const int cols = WIDE ? kWave : 1 << cols_log2, phases = WIDE ? 1 : kWave >> cols_log2, phase = WIDE ? 0 : lane >> cols_log2;
+    // block -> (class, slice, column block): eight column blocks at a time, one per XCD, over all classes and slices
+    const unsigned per_cb = (unsigned)k * slices, group = blockIdx.x / (8 * per_cb), in_group = blockIdx.x - group * 8 * per_cb;
+    const unsigned wide = min(8u, col_blocks - group * 8);           // column blocks of this group
+    const unsigned cs = in_group / wide, cb = group * 8 + in_group % wide;
+    const int g = (int)(cs / slices), slice = (int)(cs % slices);
+    const uint32_t col0 = cb * cols, col = col0 + (lane & (cols - 1)), at = col < words ? col : words - 1;
+    const int part = slice * kPackedWaves + wave, parts = slices * kPackedWaves;
+    const int r0 = (int)((int64_t)class_rows * part / parts), r1 = (int)((int64_t)class_rows * (part + 1) / parts);
+    uint32_t plane[kTreePlanes];
+#pragma unroll
+    for (int q = 0; q < kTreePlanes; ++q) plane[q] = 0;
+    for (int r = r0; r < r1; r += 4 * phases) {                      // four roots of a lane per step
+        uint32_t w[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int rr = r + phase + u * phases;
+            const bool ok = rr < r1;
+            int j = g * class_rows + (ok ? rr : r1 - 1);
+            if constexpr (WIDE) j = uniform(j);
+            const int32_t *row = rows + (int64_t)j * 8;
+            uint32_t v[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) v[t] = x[(uint64_t)min((uint32_t)row[t], (uint32_t)in_dim - 1u) * words + at];
+            const BitOpsAnf::Params pr = BitOpsAnf::unpack(codes[j]);
+            uint32_t leaf[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) leaf[q] = BitOpsAnf::gate32(pr, q, v[2 * q], v[2 * q + 1]);
+            const uint32_t y = BitOpsAnf::gate32(pr, 6, BitOpsAnf::gate32(pr, 4, leaf[0], leaf[1]), BitOpsAnf::gate32(pr, 5, leaf[2], leaf[3]));
+            w[u] = ok ? y ^ pr.inv : 0;
+        }
+        uint32_t two_a, two_b, four;
+        carry_save(two_a, plane[0], plane[0], w[0], w[1]);
+        carry_save(two_b, plane[0], plane[0], w[2], w[3]);
+        carry_save(four, plane[1], plane[1], two_a, two_b);
+#pragma unroll
+        for (int q = 2; q < kTreePlanes; ++q) {
+            const uint32_t t = plane[q] & four;
+            plane[q] ^= four;
+            four = t;
+        }
+    }
+    if constexpr (!WIDE) {
+        for (int by = kWave / 2; by >= cols; by >>= 1) {             // root phases: the first lanes end up with the wavefront's counts
+            uint32_t other[kTreePlanes];
+#pragma unroll
+            for (int q = 0; q < kTreePlanes; ++q) other[q] = (uint32_t)__shfl_down((int)plane[q], by);
+            add_counts(plane, other);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < kTreePlanes; ++q) meet[wave][q][lane] = plane[q];
+    __syncthreads();
+    // the wavefronts' counts in two rounds: wavefront w < 4 adds four of them, then everybody adds those four
+    if (wave < 4) {
+        for (int wv = 4; wv < kPackedWaves; wv += 4) {
+            uint32_t other[kTreePlanes];
+#pragma unroll
+            for (int q = 0; q < kTreePlanes; ++q) other[q] = meet[wave + wv][q][lane];
+            add_counts(plane, other);
+        }
+#pragma unroll
+        for (int q = 0; q < kTreePlanes; ++q) meet[wave][q][lane] = plane[q];
+    }
+    __syncthreads();
+    const int c = threadIdx.x & (cols - 1);
+    uint32_t total[kTreePlanes];
+#pragma unroll
+    for (int q = 0; q < kTreePlanes; ++q) total[q] = meet[0][q][c];
+    for (int wv = 1; wv < 4; ++wv) {
+        uint32_t other[kTreePlanes];
+#pragma unroll
+        for (int q = 0; q < kTreePlanes; ++q) other[q] = meet[wv][q][c];
+        add_counts(total, other);
+    }
+    if (col0 + c >= words) return;
+    const int step = kPackedWaves * kWave / cols;
+    for (int b = threadIdx.x / cols; b < 32; b += step) {
+        const int64_t s = (int64_t)(col0 + c) * 32 + b;
+        if (s >= samples) break;
+        int32_t cnt = 0;
+#pragma unroll
+        for (int q = 0; q < kTreePlanes; ++q) cnt |= (int32_t)((total[q] >> b) & 1) << q;
+        if (slices == 1) out[s * k + g] = cnt;
+        else atomicAdd(out + s * k + g, cnt);
+    }
+}
+
+}  // namespace
+
+extern "C" int clg_fc_tree_packed(const int64_t *x, const int32_t *rows, const int32_t *ids, const float *logits0, const float *logits1,
+                                  const float *logits2, uint32_t *codes, int32_t *out, int64_t in_dim, int64_t roots, int64_t k,
+                                  int64_t words, int64_t samples, void *stream)
+{
+    const char *name = "clg_fc_tree_packed";
+    if (int e = check_tree(name, in_dim, roots, k)) return e;
+    CLG_REQUIRE(x && rows && ids && logits0 && logits1 && logits2 && codes && out, "%s: null pointer argument", name);
+    CLG_REQUIRE(words > 0 && samples > 0 && samples <= words * 64 && words < (1ll << 31), "%s: words %lld, samples %lld", name,
+                (long long)words, (long long)samples);
+    hipStream_t st = clg_stream(stream);
+    const int64_t class_rows = roots / k;
+    const int64_t halves = words * 2;                                // 32-bit words of a row: a lane takes one
+    int cols_log2 = 6;
+    while (cols_log2 > 0 && (1ll << (cols_log2 - 1)) >= halves) --cols_log2;
+    const int64_t col_blocks = clg_ceil_div(halves, 1ll << cols_log2);
+    // One workgroup takes all roots of its columns and class where that gives half of the CUs one; else the classes are sliced
+    // down to two steps of roots per wavefront, and the slices meet in atomics.  (Twelve slices of a class at 65 536 samples:
+    // 7.9 M atomics, 385 us instead of 66.)  A workgroup takes at most 2^14 - 4 roots.
+    const int64_t phases = 64 >> cols_log2;
+    int64_t slices = k * col_blocks >= 128 ? 1 : clg_ceil_div(512, k * col_blocks);
+    slices = std::min(slices, class_rows / (8 * phases * kPackedWaves));
+    slices = std::max<int64_t>(std::max<int64_t>(slices, clg_ceil_div(class_rows, (1 << kTreePlanes) - 4)), 1);
+    const int64_t blocks = k * slices * col_blocks;
+    CLG_REQUIRE(blocks < (1ll << 28) && halves < (1ll << 31), "%s: problem too large for one launch", name);
+    const TreeLogits lg = {{logits0, logits1, logits2}};
+    hipLaunchKernelGGL(fc_tree_codes_kernel, dim3((unsigned)clg_ceil_div(roots * 8, 256)), dim3(256), 0, st, lg, ids, codes, (int)roots, out,
+                       slices > 1 ? samples * k : (int64_t)0);
+    CLG_CHECK_LAUNCH(name);
+#define CLG_TREE_P(WIDE)                                                                                                      \
+    hipLaunchKernelGGL((fc_tree_packed_kernel<WIDE>), dim3((unsigned)blocks), dim3(kPackedWaves * kWave), 0, st, (const uint32_t *)x, rows, \
+                       codes, out, (int)class_rows, (int)k, (int)slices, (uint32_t)halves, samples, (int)in_dim, cols_log2, (unsigned)col_blocks)
+    if (cols_log2 == 6) CLG_TREE_P(true);
+    else CLG_TREE_P(false);
+#undef CLG_TREE_P
+    CLG_CHECK_LAUNCH(name);
+    return CLG_OK;
+}

@@ -1,0 +1,115 @@
+"""A LogicLayer, two halving LogicLayers and a GroupSum -- the end of the reference's networks (src/convlogic/model.py:49-57,
+102-107) -- as one operation.  Where every neuron of the first two layers is read exactly once, each neuron of the third is
+the root of a tree of seven gates over eight input rows that no other root shares, so the three layers are evaluated, and
+differentiated, without activations of their own (csrc/fc_tree.hip)."""
+import weakref
+
+import torch
+
+from ..hip import _lib
+from ..hip._lib import check, stream_ptr
+
+# per first layer: (key, wiring plan); kept outside the modules so that copies and pickles carry no derived buffers
+_PLANS = weakref.WeakKeyDictionary()
+
+
+class TreePlan:
+    """The trees of three layers' wiring: input rows, neuron ids and list positions of every root's eight operands, and the
+    place of every neuron in its tree (int32 on the device; include/convlogic_amd.h).  For layers whose every neuron is read
+    exactly once."""
+
+    def __init__(self, first, second, third):
+        a, b = first._buffers["indices_0"], first._buffers["indices_1"]
+        mid = torch.stack([third._buffers["indices_0"], third._buffers["indices_1"]], 1)                       # [roots, 2]
+        leaf = torch.stack([second._buffers["indices_0"][mid], second._buffers["indices_1"][mid]], 2).flatten(1)   # [roots, 4]
+        operand = torch.stack([a, b], 1)                                                                       # [out, 2]
+        # place of every operand in the lists input feature -> operands: by feature, then by neuron, first operand first (the
+        # order of given_x_indices_of_y)
+        order = torch.argsort(operand.flatten(), stable=True)
+        place = torch.empty_like(order)
+        place[order] = torch.arange(order.numel(), device=order.device)
+        self.roots = third.out_dim
+        self.rows = operand[leaf].flatten(1).to(torch.int32).contiguous()
+        self.pos = place.view(-1, 2)[leaf].flatten(1).to(torch.int32).contiguous()
+        self.ids = torch.cat([leaf, mid, torch.zeros_like(mid)], 1).to(torch.int32).contiguous()
+        # where a neuron's sums are: of the first layer's, of the second's, of the roots
+        slots = torch.arange(7 * self.roots, device=order.device).view(-1, 7)
+        slot = [torch.empty(n, dtype=torch.int64, device=order.device) for n in (first.out_dim, second.out_dim)]
+        slot[0][leaf] = slots[:, :4]
+        slot[1][mid] = slots[:, 4:6]
+        self.slot = torch.cat([slot[0], slot[1], slots[:, 6]]).to(torch.int32)
+
+
+def tree_plan(first, second, third):
+    """The TreePlan of three LogicLayers, or None when their wiring does not make trees.  Rebuilt when a wiring buffer was
+    modified in place, replaced or moved."""
+    if 2 * second.out_dim != second.in_dim or 2 * third.out_dim != third.in_dim or second.in_dim != first.out_dim or third.in_dim != second.out_dim:
+        return None
+    keys = (first._wiring_key(), second._wiring_key(), third._wiring_key())
+    for layer, key in zip((first, second, third), keys):
+        layer._check_wiring(key)
+    cached = _PLANS.get(first)
+    if cached is None or cached[0] != keys:
+        fits = second._sole_consumers(keys[1]) and third._sole_consumers(keys[2])
+        cached = _PLANS[first] = (keys, TreePlan(first, second, third) if fits else None)
+    return cached[1]
+
+
+class _TreeFunction(torch.autograd.Function):
+    """x feature-major [features, B] -> class sums [B, k] / tau of the three layers; gradients of x and of the logits."""
+
+    @staticmethod
+    def forward(ctx, x, l0, l1, l2, start, plan, k, tau):
+        lib, st = _lib.load(), stream_ptr(x)
+        in_dim, batch = x.shape
+        coef = torch.empty((plan.roots, 28), dtype=torch.float32, device=x.device)
+        check(lib.clg_fc_tree_fold(l0.data_ptr(), l1.data_ptr(), l2.data_ptr(), plan.ids.data_ptr(), coef.data_ptr(), plan.roots, 0, st))
+        out = _tree_forward(lib, x, plan, coef, k, tau, st)
+        ctx.save_for_backward(x, l0, l1, l2, start, coef)
+        ctx.plan, ctx.k, ctx.tau = plan, k, tau
+        return out
+
+    @staticmethod
+    def backward(ctx, grad_out):
+        x, l0, l1, l2, start, coef = ctx.saved_tensors
+        plan, k = ctx.plan, ctx.k
+        grad_out = _lib.check_input(grad_out.contiguous(), "grad_out", torch.float32, (x.shape[1], k))
+        _lib.check_same_device(x, grad_out)
+        in_dim, batch = x.shape
+        g0, g1, g2, gx = (torch.empty_like(t) for t in (l0, l1, l2, x))
+        scratch = torch.empty((plan.roots * (8 * batch + 28),), dtype=torch.float32, device=x.device)   # rowgrad, then sums
+        rowgrad, sums = scratch.data_ptr(), scratch.data_ptr() + plan.roots * 8 * batch * 4
+        check(_lib.load().clg_fc_tree_backward(
+            x.data_ptr(), plan.rows.data_ptr(), plan.pos.data_ptr(), plan.slot.data_ptr(), coef.data_ptr(), grad_out.data_ptr(),
+            l0.data_ptr(), l1.data_ptr(), l2.data_ptr(), g0.data_ptr(), g1.data_ptr(), g2.data_ptr(), rowgrad, sums, start.data_ptr(),
+            gx.data_ptr(), in_dim, plan.roots, k, batch, batch, float(ctx.tau), stream_ptr(x)))
+        return gx, g0, g1, g2, None, None, None, None
+
+
+def _tree_forward(lib, x, plan, coef, k, tau, st):
+    in_dim, batch = x.shape
+    out = torch.empty((batch, k), dtype=torch.float32, device=x.device)
+    partial = torch.empty((lib.clg_fc_tree_partial_elems(plan.roots, k, batch, batch),), dtype=torch.float32, device=x.device)
+    check(lib.clg_fc_tree_forward(x.data_ptr(), plan.rows.data_ptr(), coef.data_ptr(), partial.data_ptr(), out.data_ptr(), in_dim,
+                                  plan.roots, k, batch, batch, float(tau), st))
+    return out
+
+
+def tree_train(layers, group_sum, x, plan):
+    """group_sum(third(second(first(x)))) in training; x feature-major [features, B], B a multiple of 4."""
+    first, second, third = layers
+    return _TreeFunction.apply(x, first.weights, second.weights, third.weights, first._buffers["given_x_indices_of_y_start"], plan,
+                               group_sum.k, group_sum.tau)
+
+
+def tree_packed(layers, k, x, plan):
+    """Class counts int32 [samples, k] of packed words x (a PackBitsTensor of 64 samples per word)."""
+    words = x.t
+    lib = _lib.load()
+    samples = words.shape[1] * 64 - x.pad_len
+    out = torch.empty((samples, k), dtype=torch.int32, device=words.device)
+    codes = torch.empty((plan.roots,), dtype=torch.int32, device=words.device)
+    l0, l1, l2 = (layer.weights.detach() for layer in layers)
+    check(lib.clg_fc_tree_packed(words.data_ptr(), plan.rows.data_ptr(), plan.ids.data_ptr(), l0.data_ptr(), l1.data_ptr(), l2.data_ptr(),
+                                 codes.data_ptr(), out.data_ptr(), words.shape[0], plan.roots, k, words.shape[1], samples, stream_ptr(words)))
+    return out

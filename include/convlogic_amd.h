@@ -495,6 +495,35 @@ int clg_convblock_bin_supported(int dtype, const clg_conv_geom *g);
  * without a copy or a synchronisation.  CLG_EINVAL when `host` is not pinned memory mapped for the current device.  No
  * counterpart in the reference (its kernels do not check their inputs). */
 int clg_host_flag_device_pointer(void *host, void **device);
+
+/* ---------------------------------------------------------------------------------
+ * The fully connected end of a network as one operation (float32): a LogicLayer, two halving LogicLayers whose inputs are each
+ * read by exactly one neuron operand, and a GroupSum (src/convlogic/model.py:49-57; the four modules there).  Every neuron
+ * of the third layer is then the root of a tree of seven gates over eight input rows.
+ *   rows [roots, 8]  input rows of a root's tree          ids [roots, 8]  its neurons: 0..3 first layer, 4..5 second
+ *   pos  [roots, 8]  place of each operand in the lists input feature -> operands (CSR, `start` [in_dim + 1])
+ *   slot [7 roots]   of every neuron, first layer first: root * 7 + its place among the tree's gates
+ *   logits0..2       the layers' logits [out, 16]         coef [roots, 7, 4] folded coefficients in tree order
+ * x is feature-major with a row pitch (multiple of 4) >= batch.
+ * ------------------------------------------------------------------------------- */
+/* coef of the softmax (hard = 0) or the arg-max gates (hard = 1) */
+int clg_fc_tree_fold(const float *logits0, const float *logits1, const float *logits2, const int32_t *ids, float *coef,
+                     int64_t roots, int hard, void *stream);
+/* floats of the `partial` buffer of clg_fc_tree_forward; negative for bad arguments */
+int64_t clg_fc_tree_partial_elems(int64_t roots, int64_t k, int64_t batch, int64_t pitch);
+/* out [batch, k] = class sums of the roots' values / tau */
+int clg_fc_tree_forward(const float *x, const int32_t *rows, const float *coef, float *partial, float *out, int64_t in_dim,
+                        int64_t roots, int64_t k, int64_t batch, int64_t pitch, double tau, void *stream);
+/* grad_out [batch, k] -> gradients of the three layers' logits and grad_x [in_dim, pitch]; scratch: rowgrad [8 roots, pitch],
+ * sums [roots, 28] */
+int clg_fc_tree_backward(const float *x, const int32_t *rows, const int32_t *pos, const int32_t *slot, const float *coef,
+                         const float *grad_out, const float *logits0, const float *logits1, const float *logits2, float *grad0,
+                         float *grad1, float *grad2, float *rowgrad, float *sums, const int64_t *start, float *grad_x, int64_t in_dim,
+                         int64_t roots, int64_t k, int64_t batch, int64_t pitch, double tau, void *stream);
+/* packed words [in_dim, words] (64 samples per word) -> int32 class counts [samples, k] with arg-max gates; codes: scratch [roots] */
+int clg_fc_tree_packed(const int64_t *x, const int32_t *rows, const int32_t *ids, const float *logits0, const float *logits1,
+                       const float *logits2, uint32_t *codes, int32_t *out, int64_t in_dim, int64_t roots, int64_t k,
+                       int64_t words, int64_t samples, void *stream);
 int64_t clg_convblock_bin_ctx_bytes(int dtype, const clg_conv_geom *g);
 int clg_convblock_bin_forward(int dtype, const clg_conv_geom *g, const void *x, const void *w, const int32_t *selection, void *y,
                               uint16_t *taps, void *ctx, int flags, int32_t *not_binary, void *stream);

@@ -1,0 +1,112 @@
+"""Three LogicLayers (the last two halving) and a GroupSum as one operation (difflogic/fc_tree.py): training against the float64
+oracle at the edges of its lane layouts (1, 2 and 4 samples per lane, partly filled wavefronts, several passes over a
+row), packed class counts against the modules one after the other."""
+import pytest
+import torch
+
+import convlogic_amd as C
+from convlogic_amd.difflogic import fc_tree
+from oracle import convlogic_oracle as O
+from tests.gpu_util import DEV, assert_grad_close
+
+pytestmark = pytest.mark.gpu
+
+
+def tail(in_dim, roots, k, seed):
+    torch.manual_seed(seed)
+    dims = [in_dim, 4 * roots, 2 * roots, roots]
+    return [C.LogicLayer(a, b, implementation="cuda").to(DEV) for a, b in zip(dims, dims[1:])], C.GroupSum(k, tau=3.0)
+
+
+@pytest.mark.parametrize("batch", [4, 64, 68, 128, 132, 256, 260, 516])
+@pytest.mark.parametrize("in_dim,roots,k", [(8, 2, 1), (40, 130, 10), (700, 663, 3)])
+def test_training_against_the_oracle(batch, in_dim, roots, k):
+    layers, gs = tail(in_dim, roots, k, batch + roots)
+    plan = fc_tree.tree_plan(*layers)
+    assert plan is not None and plan.roots == roots
+    x = torch.rand(in_dim, batch, device=DEV).requires_grad_(True)
+    go = torch.randn(batch, k, device=DEV)
+    y = fc_tree.tree_train(layers, gs, x, plan)
+    y.backward(go)
+    h = xl = x.detach().double().cpu().t().contiguous().requires_grad_(True)
+    ws = [m.weights.detach().double().cpu().requires_grad_(True) for m in layers]
+    for m, w in zip(layers, ws):
+        h = O.logic_fc_forward(h, m.indices_0.cpu(), m.indices_1.cpu(), torch.softmax(w, -1))
+    want = O.group_sum(h, k, gs.tau)
+    want.backward(go.double().cpu())
+    # values: at most roots / k terms of one rounding error each, relative to a sum of as many values around 0.5
+    assert (y.detach().double().cpu() - want.detach()).norm() <= 1e-6 * want.detach().norm()
+    assert_grad_close(x.grad.t(), xl.grad, rel=1e-4, name="grad_x")
+    for i, (m, w) in enumerate(zip(layers, ws)):
+        assert_grad_close(m.weights.grad, w.grad, rel=1e-4, name=f"grad_logits {i}")
+    grads = [x.grad.clone()] + [m.weights.grad.clone() for m in layers]
+    for t in (x, *(m.weights for m in layers)):
+        t.grad = None
+    fc_tree.tree_train(layers, gs, x, plan).backward(go)
+    assert all(torch.equal(a, b) for a, b in zip(grads, [x.grad] + [m.weights.grad for m in layers]))
+
+
+# (words of 64 samples: lanes along roots below 32 of them, one block of columns, a partly filled second one; classes of fewer
+# roots than a workgroup has lanes for, sliced classes, and more roots than a workgroup's counters hold)
+@pytest.mark.parametrize("samples", [1, 64, 100, 1000, 2048, 2112, 20000])
+@pytest.mark.parametrize("in_dim,roots,k", [(8, 3, 3), (100, 640, 10), (3000, 5000, 2), (64, 40000, 1)])
+def test_packed_counts_equal_the_modules(samples, in_dim, roots, k):
+    layers, gs = tail(in_dim, roots, k, samples + roots)
+    for m in layers:
+        m.eval()
+    words = -(-samples // 64)
+    bits = torch.randint(-2**63, 2**63 - 1, (in_dim, words), dtype=torch.int64, device=DEV)
+
+    def packed():
+        p = C.PackBitsTensor.__new__(C.PackBitsTensor)
+        p.t, p.bit_count, p.pad_len, p.image = bits, 64, words * 64 - samples, False
+        return p
+
+    with torch.no_grad():
+        want = torch.nn.Sequential(*layers, gs)(packed())
+        got = fc_tree.tree_packed(layers, k, packed(), fc_tree.tree_plan(*layers))
+    assert got.dtype == torch.int32 and torch.equal(got, want)
+
+
+def test_wiring_that_makes_no_trees_and_rewired_layers():
+    layers, gs = tail(40, 20, 2, 1)
+    assert fc_tree.tree_plan(*layers) is not None
+    with torch.no_grad():                                            # two operands on one neuron: no trees
+        old = layers[1].indices_0[0].item()
+        layers[1].indices_0[0] = layers[1].indices_1[5].item()
+    assert fc_tree.tree_plan(*layers) is None
+    with torch.no_grad():
+        layers[1].indices_0[0] = old
+        layers[0].indices_0.copy_(layers[0].indices_0.flip(0))       # another wiring of the first layer: another plan
+    x = torch.rand(40, 16, device=DEV)
+    y = fc_tree.tree_train(layers, gs, x, fc_tree.tree_plan(*layers))
+    h = x.t()
+    for m in layers:
+        h = m(h)
+    assert torch.allclose(y, gs(h), rtol=1e-5, atol=1e-5)
+    assert fc_tree.tree_plan(layers[0], layers[2], layers[1]) is None   # not a chain of halving layers
+
+
+def test_a_network_takes_its_tail_as_trees_and_equals_its_modules():
+    torch.manual_seed(2)
+    model = C.ConvLogicMnistModel(k_param=2, tau=6.5).to(DEV)
+    x = torch.randint(0, 2, (32, 1, 28, 28), device=DEV).float()
+    labels = torch.randint(0, 10, (32,), device=DEV)
+    results = []
+    for on in (True, False):
+        model.tree_tail = on
+        model.zero_grad()
+        out = model(x)
+        torch.nn.functional.cross_entropy(out, labels).backward()
+        results.append([out.detach()] + [p.grad.clone() for p in model.parameters()])
+        assert ("_Tree" in type(out.grad_fn).__name__) == on
+    for i, (a, b) in enumerate(zip(*results)):
+        assert_grad_close(a, b, rel=1e-4, name=f"result {i}")
+    model.eval()
+    bits = torch.randint(0, 2, (77, 1, 28, 28), device=DEV).bool()
+    with torch.no_grad():
+        counts = []
+        for on in (True, False):
+            model.tree_tail = on
+            counts.append(model(C.PackBitsTensor(bits, 64)))
+    assert torch.equal(*counts)
