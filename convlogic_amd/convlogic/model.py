@@ -9,7 +9,7 @@ import torch
 from torch import nn
 
 from ..difflogic import GroupSum, LogicLayer
-from ..difflogic.difflogic import _feature_major, _has_forward_hooks, logic_layer_group_sum
+from ..difflogic.difflogic import _feature_major, logic_layer_group_sum
 from ..difflogic.fc_tree import tree_packed, tree_plan, tree_train
 from ..difflogic.packbitstensor import PackBitsTensor
 from .convlogic_layer import ConvLogicLayer
@@ -55,16 +55,22 @@ def _prefold(owner, layers, x, mode=True):
         m.set_prefold(probs, folded)
 
 
+def _called_for_itself(module):
+    """True when a call of the module does more than its class's forward: hooks of either pass, a replaced forward."""
+    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+                or "forward" in module.__dict__)
+
+
 def _tree_tail(net):
     """The last four modules of a network -- three LogicLayers and a GroupSum -- when nothing but a call of the modules
     themselves stands against evaluating them as one operation (difflogic/fc_tree.py), else None."""
-    if len(net) < 4 or net._forward_hooks or net._forward_pre_hooks:
+    if len(net) < 4 or _called_for_itself(net) or torch.nn.modules.module._has_any_global_hook():
         return None
     tail = [net[i] for i in range(len(net) - 4, len(net))]
     *layers, gs = tail
     if not all(type(m) is LogicLayer and m.implementation == "cuda" and m.grad_factor == 1.0 for m in layers) or type(gs) is not GroupSum:
         return None
-    if any(_has_forward_hooks(m) for m in tail) or layers[-1].out_dim % gs.k != 0 or gs.tau == 0:
+    if any(_called_for_itself(m) for m in tail) or layers[-1].out_dim % gs.k != 0 or gs.tau == 0:
         return None
     for m in layers:
         w = m._parameters["weights"]

@@ -76,9 +76,10 @@ __device__ __forceinline__ float swap_add16(float a, float b)
 struct TreeLogits {
     const float *l[3];
 };
+__device__ __forceinline__ int64_t tree_neuron(const int32_t *__restrict__ ids, int j, int q) { return q < 6 ? ids[(int64_t)j * 8 + q] : j; }
 __device__ __forceinline__ const float *tree_logits(const TreeLogits &lg, const int32_t *__restrict__ ids, int j, int q)
 {
-    return q < 6 ? (q < 4 ? lg.l[0] : lg.l[1]) + (int64_t)ids[(int64_t)j * 8 + q] * 16 : lg.l[2] + (int64_t)j * 16;
+    return (q < 4 ? lg.l[0] : (q < 6 ? lg.l[1] : lg.l[2])) + tree_neuron(ids, j, q) * 16;
 }
 // index of the first maximum (a NaN counts as the maximum), as clg_gate_argmax
 __device__ __forceinline__ int argmax16(const float *__restrict__ w)
@@ -92,8 +93,10 @@ __device__ __forceinline__ int argmax16(const float *__restrict__ w)
     }
     return at;
 }
+// probs (or null): the probabilities, neurons of the first layer first.  The backward pass reads these: logits that an
+// optimizer updates between the two passes must not reach it.
 __global__ __launch_bounds__(256) void fc_tree_fold_kernel(TreeLogits lg, const int32_t *__restrict__ ids, float *__restrict__ coef,
-                                                         int roots, int hard)
+                                                         float *__restrict__ probs, int roots, int hard)
 {
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (e >= (int64_t)roots * 7) return;
@@ -106,6 +109,11 @@ __global__ __launch_bounds__(256) void fc_tree_fold_kernel(TreeLogits lg, const 
         for (int i = 0; i < 16; ++i) p[i] = i == at ? 1.f : 0.f;
     } else {
         softmax16(w, p);
+    }
+    if (probs) {
+        float4 *dst = reinterpret_cast<float4 *>(probs + (tree_neuron(ids, j, q) + (int64_t)roots * (q < 4 ? 0 : (q < 6 ? 4 : 6))) * 16);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dst[i] = make_float4(p[4 * i], p[4 * i + 1], p[4 * i + 2], p[4 * i + 3]);
     }
     const Coef<float> c = fold16(p);
     reinterpret_cast<float4 *>(coef)[e] = make_float4(c.ab, c.a, c.b, c.one);
@@ -206,7 +214,7 @@ __global__ __launch_bounds__(256) void fc_tree_finish_kernel(const float *__rest
 // pos [roots][8]: the row of `rowgrad` an operand's gradient goes to: its place in the lists input feature -> operands.
 // The 28 sums of a wavefront are reduced and turned round together: every exchange between lane groups halves the number of
 // values a lane holds instead of repeating each value's full reduction (28 x 6 steps).  They leave as one run of 112 bytes per
-// root; what remains -- 16 gates per neuron, the softmax backward -- needs the logits of seven scattered neurons and is a
+// root; what remains -- 16 gates per neuron, the softmax backward -- needs the rows of seven scattered neurons and is a
 // kernel of its own in neuron order (fc_tree_logit_grad_kernel): done here it held the wavefront for one more round trip and
 // read and wrote 64-byte pieces all over (655360 roots x 128 samples: 1742 us, 978 without it).
 __device__ __forceinline__ void tree_store_sums(float (&v)[28], float *__restrict__ sums, int j, int lane)
@@ -304,7 +312,7 @@ struct TreeGrads {
     float *g[3];
     int64_t end[3];       // neurons of the first one, two, three layers
 };
-__global__ __launch_bounds__(256) void fc_tree_logit_grad_kernel(TreeLogits lg, TreeGrads gr, const float *__restrict__ sums,
+__global__ __launch_bounds__(256) void fc_tree_logit_grad_kernel(const float *__restrict__ probs, TreeGrads gr, const float *__restrict__ sums,
                                                                const int32_t *__restrict__ slot, int64_t slots)
 {
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -312,12 +320,13 @@ __global__ __launch_bounds__(256) void fc_tree_logit_grad_kernel(TreeLogits lg, 
     const int layer = e < gr.end[0] ? 0 : (e < gr.end[1] ? 1 : 2);
     const int64_t n = e - (layer ? gr.end[layer - 1] : 0);
     const float4 s = reinterpret_cast<const float4 *>(sums)[min((uint64_t)(uint32_t)slot[e], (uint64_t)slots - 1)];
-    const float4 *w = reinterpret_cast<const float4 *>(lg.l[layer] + n * 16);
-    float4 raw[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) raw[i] = w[i];
+    const float4 *w = reinterpret_cast<const float4 *>(probs + e * 16);
     float p[16], gi[16], dot = 0.f;
-    softmax16(reinterpret_cast<const float *>(raw), p);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float4 v = w[i];
+        p[4 * i] = v.x, p[4 * i + 1] = v.y, p[4 * i + 2] = v.z, p[4 * i + 3] = v.w;
+    }
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         gi[i] = coef_transpose_row<float>(i, s.x, s.y, s.z, s.w);
@@ -389,14 +398,14 @@ int tree_slices(int64_t class_rows, int64_t batch, int64_t k)
 }  // namespace
 
 extern "C" int clg_fc_tree_fold(const float *logits0, const float *logits1, const float *logits2, const int32_t *ids, float *coef,
-                                int64_t roots, int hard, void *stream)
+                                float *probs, int64_t roots, int hard, void *stream)
 {
     const char *name = "clg_fc_tree_fold";
     if (int e = check_tree(name, 1, roots, 1)) return e;
     CLG_REQUIRE(logits0 && logits1 && logits2 && ids && coef, "%s: null pointer argument", name);
     const TreeLogits lg = {{logits0, logits1, logits2}};
     hipLaunchKernelGGL(fc_tree_fold_kernel, dim3((unsigned)clg_ceil_div(roots * 7, 256)), dim3(256), 0, clg_stream(stream), lg, ids, coef,
-                       (int)roots, hard);
+                       probs, (int)roots, hard);
     CLG_CHECK_LAUNCH(name);
     return CLG_OK;
 }
@@ -436,19 +445,17 @@ extern "C" int clg_fc_tree_forward(const float *x, const int32_t *rows, const fl
 }
 
 extern "C" int clg_fc_tree_backward(const float *x, const int32_t *rows, const int32_t *pos, const int32_t *slot, const float *coef,
-                                    const float *grad_out, const float *logits0, const float *logits1, const float *logits2, float *grad0,
-                                    float *grad1, float *grad2, float *rowgrad, float *sums, const int64_t *start, float *grad_x,
-                                    int64_t in_dim, int64_t roots, int64_t k, int64_t batch, int64_t pitch, double tau, void *stream)
+                                    const float *grad_out, const float *probs, float *grad0, float *grad1, float *grad2, float *rowgrad,
+                                    float *sums, const int64_t *start, float *grad_x, int64_t in_dim, int64_t roots, int64_t k, int64_t batch, int64_t pitch, double tau, void *stream)
 {
     const char *name = "clg_fc_tree_backward";
     if (int e = check_tree(name, in_dim, roots, k)) return e;
-    CLG_REQUIRE(x && rows && pos && slot && coef && grad_out && logits0 && logits1 && logits2 && grad0 && grad1 && grad2 && rowgrad && sums && start &&
+    CLG_REQUIRE(x && rows && pos && slot && coef && grad_out && probs && grad0 && grad1 && grad2 && rowgrad && sums && start &&
                     grad_x, "%s: null pointer argument", name);
     CLG_REQUIRE(batch > 0 && pitch >= batch && pitch % 4 == 0 && pitch < (1ll << 28) && tau != 0.0,
                 "%s: the row pitch must be a multiple of 4 that holds the batch, tau must not be zero", name);
     const int vec = tree_vec(pitch);
     hipStream_t st = clg_stream(stream);
-    const TreeLogits lg = {{logits0, logits1, logits2}};
     const TreeGrads gr = {{grad0, grad1, grad2}, {4 * roots, 6 * roots, 7 * roots}};
     const dim3 grid((unsigned)clg_ceil_div(roots, kTreeWaves));
     const dim3 ggrid((unsigned)clg_ceil_div(in_dim, kTreeWaves), (unsigned)clg_ceil_div(pitch, (int64_t)kWave * vec));
@@ -465,7 +472,7 @@ extern "C" int clg_fc_tree_backward(const float *x, const int32_t *rows, const i
     else CLG_TREE_B(4);
 #undef CLG_TREE_B
     CLG_CHECK_LAUNCH(name);
-    hipLaunchKernelGGL(fc_tree_logit_grad_kernel, dim3((unsigned)clg_ceil_div(7 * roots, 256)), dim3(256), 0, st, lg, gr, (const float *)sums, slot,
+    hipLaunchKernelGGL(fc_tree_logit_grad_kernel, dim3((unsigned)clg_ceil_div(7 * roots, 256)), dim3(256), 0, st, probs, gr, (const float *)sums, slot,
                        7 * roots);
     CLG_CHECK_LAUNCH(name);
     return CLG_OK;

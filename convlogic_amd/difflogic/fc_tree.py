@@ -63,25 +63,29 @@ class _TreeFunction(torch.autograd.Function):
         lib, st = _lib.load(), stream_ptr(x)
         in_dim, batch = x.shape
         coef = torch.empty((plan.roots, 28), dtype=torch.float32, device=x.device)
-        check(lib.clg_fc_tree_fold(l0.data_ptr(), l1.data_ptr(), l2.data_ptr(), plan.ids.data_ptr(), coef.data_ptr(), plan.roots, 0, st))
+        probs = torch.empty((7 * plan.roots, 16), dtype=torch.float32, device=x.device)
+        check(lib.clg_fc_tree_fold(l0.data_ptr(), l1.data_ptr(), l2.data_ptr(), plan.ids.data_ptr(), coef.data_ptr(), probs.data_ptr(),
+                                   plan.roots, 0, st))
         out = _tree_forward(lib, x, plan, coef, k, tau, st)
-        ctx.save_for_backward(x, l0, l1, l2, start, coef)
+        # (probabilities, not logits, as in the modules: the logits may be updated between forward and backward)
+        ctx.save_for_backward(x, start, coef, probs)
         ctx.plan, ctx.k, ctx.tau = plan, k, tau
         return out
 
     @staticmethod
     def backward(ctx, grad_out):
-        x, l0, l1, l2, start, coef = ctx.saved_tensors
+        x, start, coef, probs = ctx.saved_tensors
         plan, k = ctx.plan, ctx.k
         grad_out = _lib.check_input(grad_out.contiguous(), "grad_out", torch.float32, (x.shape[1], k))
         _lib.check_same_device(x, grad_out)
         in_dim, batch = x.shape
-        g0, g1, g2, gx = (torch.empty_like(t) for t in (l0, l1, l2, x))
+        gx = torch.empty_like(x)
+        g0, g1, g2 = (torch.empty((n * plan.roots, 16), dtype=torch.float32, device=x.device) for n in (4, 2, 1))
         scratch = torch.empty((plan.roots * (8 * batch + 28),), dtype=torch.float32, device=x.device)   # rowgrad, then sums
         rowgrad, sums = scratch.data_ptr(), scratch.data_ptr() + plan.roots * 8 * batch * 4
         check(_lib.load().clg_fc_tree_backward(
             x.data_ptr(), plan.rows.data_ptr(), plan.pos.data_ptr(), plan.slot.data_ptr(), coef.data_ptr(), grad_out.data_ptr(),
-            l0.data_ptr(), l1.data_ptr(), l2.data_ptr(), g0.data_ptr(), g1.data_ptr(), g2.data_ptr(), rowgrad, sums, start.data_ptr(),
+            probs.data_ptr(), g0.data_ptr(), g1.data_ptr(), g2.data_ptr(), rowgrad, sums, start.data_ptr(),
             gx.data_ptr(), in_dim, plan.roots, k, batch, batch, float(ctx.tau), stream_ptr(x)))
         return gx, g0, g1, g2, None, None, None, None
 

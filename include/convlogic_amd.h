@@ -506,19 +506,20 @@ int clg_host_flag_device_pointer(void *host, void **device);
  *   logits0..2       the layers' logits [out, 16]         coef [roots, 7, 4] folded coefficients in tree order
  * x is feature-major with a row pitch (multiple of 4) >= batch.
  * ------------------------------------------------------------------------------- */
-/* coef of the softmax (hard = 0) or the arg-max gates (hard = 1) */
+/* coef of the softmax (hard = 0) or the arg-max gates (hard = 1); probs [7 roots, 16] takes the probabilities, neurons of the first
+ * layer first (may be NULL) */
 int clg_fc_tree_fold(const float *logits0, const float *logits1, const float *logits2, const int32_t *ids, float *coef,
-                     int64_t roots, int hard, void *stream);
+                     float *probs, int64_t roots, int hard, void *stream);
 /* floats of the `partial` buffer of clg_fc_tree_forward; negative for bad arguments */
 int64_t clg_fc_tree_partial_elems(int64_t roots, int64_t k, int64_t batch, int64_t pitch);
 /* out [batch, k] = class sums of the roots' values / tau */
 int clg_fc_tree_forward(const float *x, const int32_t *rows, const float *coef, float *partial, float *out, int64_t in_dim,
                         int64_t roots, int64_t k, int64_t batch, int64_t pitch, double tau, void *stream);
 /* grad_out [batch, k] -> gradients of the three layers' logits and grad_x [in_dim, pitch]; scratch: rowgrad [8 roots, pitch],
- * sums [roots, 28] */
+ * sums [roots, 28]; probs and coef as clg_fc_tree_fold left them */
 int clg_fc_tree_backward(const float *x, const int32_t *rows, const int32_t *pos, const int32_t *slot, const float *coef,
-                         const float *grad_out, const float *logits0, const float *logits1, const float *logits2, float *grad0,
-                         float *grad1, float *grad2, float *rowgrad, float *sums, const int64_t *start, float *grad_x, int64_t in_dim,
+                         const float *grad_out, const float *probs, float *grad0, float *grad1, float *grad2, float *rowgrad,
+                         float *sums, const int64_t *start, float *grad_x, int64_t in_dim,
                          int64_t roots, int64_t k, int64_t batch, int64_t pitch, double tau, void *stream);
 /* packed words [in_dim, words] (64 samples per word) -> int32 class counts [samples, k] with arg-max gates; codes: scratch [roots] */
 int clg_fc_tree_packed(const int64_t *x, const int32_t *rows, const int32_t *ids, const float *logits0, const float *logits1,

@@ -110,3 +110,40 @@ def test_a_network_takes_its_tail_as_trees_and_equals_its_modules():
             model.tree_tail = on
             counts.append(model(C.PackBitsTensor(bits, 64)))
     assert torch.equal(*counts)
+
+
+def test_logits_updated_between_forward_and_backward_leave_the_gradients_alone():
+    layers, gs = tail(40, 20, 2, 3)
+    x, go = torch.rand(40, 16, device=DEV).requires_grad_(True), torch.randn(16, 2, device=DEV)
+    plan, results = fc_tree.tree_plan(*layers), []
+    for update in (False, True):
+        for t in (x, *(m.weights for m in layers)):
+            t.grad = None
+        y = fc_tree.tree_train(layers, gs, x, plan)
+        if update:
+            with torch.no_grad():
+                for m in layers:
+                    m.weights.add_(1.0).mul_(-2.0)
+        y.backward(go)
+        results.append([x.grad] + [m.weights.grad for m in layers])
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("hook", ["register_forward_hook", "register_full_backward_hook", "register_full_backward_pre_hook", "forward"])
+def test_modules_with_hooks_are_called_themselves(hook):
+    torch.manual_seed(4)
+    model, calls = C.ConvLogicMnistModel(k_param=1).to(DEV), []
+    layer = model.network[-4]
+    if hook == "forward":
+        inner = layer.forward
+        layer.forward = lambda x: (calls.append(1), inner(x))[1]
+    else:
+        getattr(layer, hook)(lambda *a: calls.append(1))
+    model(torch.randint(0, 2, (4, 1, 28, 28), device=DEV).float()).sum().backward()
+    assert calls == [1]
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda m, *a: calls.append(type(m)))
+    try:
+        model(torch.randint(0, 2, (4, 1, 28, 28), device=DEV).float())
+    finally:
+        handle.remove()
+    assert calls.count(C.LogicLayer) >= 2                              # the first two of the three (the last runs with the GroupSum)
