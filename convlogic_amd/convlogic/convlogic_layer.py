@@ -7,7 +7,7 @@ from torch.autograd import Function
 from ..difflogic.functional import GradFactor, bin_op_s
 from ..difflogic.packbitstensor import PackBitsTensor
 from ..hip import convlogic_hip
-from .treelogic_layer import gate_probabilities
+from .treelogic_layer import gate_probabilities, kernel_probabilities
 
 
 class ConvLogicFunction(Function):
@@ -328,7 +328,7 @@ class ConvLogicLayer(nn.Module):
                 raise RuntimeError("ConvLogicLayer(binary_input=True) was given an input with elements other than 0 and 1")
             if self.training and weights.is_contiguous():
                 return _FullConvLogicBinaryFunction.apply(x, weights, sel, *geo, True, flag)
-            w_prob = gate_probabilities(self.weights, self.training, x.dtype).to(x.dtype).contiguous()
+            w_prob = kernel_probabilities(self.weights, self.training, x.dtype)
             return _FullConvLogicBinaryFunction.apply(x, w_prob, sel, *geo, False, flag)
         if (self.complete and self.training and not self.return_intermediate and not self.return_indices and x.is_cuda
                 and weights.dtype == x.dtype and x.dtype in (torch.float32, torch.float64) and weights.is_contiguous()
@@ -336,8 +336,7 @@ class ConvLogicLayer(nn.Module):
             plan = self._backward_plan(x, sel)
             return _FullConvLogicLogitsFunction.apply(x, weights, sel, *geo, self.__dict__.get("feature_major_output", False), plan,
                                                       self._take_prefold(weights) if plan is not None else None)
-        # the kernels read the probabilities in x's element type (the bindings reject any other)
-        w_prob = gate_probabilities(self.weights, self.training, x.dtype).to(x.dtype).contiguous()
+        w_prob = kernel_probabilities(self.weights, self.training, x.dtype)
         if self.complete:
             return FullConvLogicFunction.apply(x, w_prob, sel, *geo, self.return_intermediate, self.return_indices)
         return ConvLogicFunction.apply(x, w_prob, sel, *geo)

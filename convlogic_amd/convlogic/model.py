@@ -10,7 +10,7 @@ from torch import nn
 
 from ..difflogic import GroupSum, LogicLayer
 from ..difflogic.difflogic import _feature_major, logic_layer_group_sum
-from ..difflogic.fc_tree import tree_packed, tree_plan, tree_train
+from ..difflogic.fc_tree import tree_eval, tree_packed, tree_plan, tree_train
 from ..difflogic.packbitstensor import PackBitsTensor
 from .convlogic_layer import ConvLogicLayer
 
@@ -81,39 +81,41 @@ def _tree_tail(net):
 
 def _forward(owner, x):
     """The network on x.  Three things happen that a plain nn.Sequential call would not do: the three LogicLayers and the
-    GroupSum at its end are evaluated as one operation where their wiring allows (`tree_tail`, default on; training steps
-    and packed inference); in training the logits of the other layers are folded in one launch where that pays (`prefold`), and a
+    GroupSum at its end are evaluated as one operation where their wiring allows (`tree_tail`, default on; training steps,
+    evaluation and packed inference); in training the logits of the other layers are folded in one launch where that pays (`prefold`), and a
     last LogicLayer and GroupSum that do not run as trees run as one autograd node (`fused_tail`, default on), whose
     backward needs no GroupSum launch."""
     net = owner.network
     n = len(net)
     tail = _tree_tail(net) if owner.__dict__.get("tree_tail", True) else None
     if isinstance(x, PackBitsTensor):
-        plan = tree_plan(*tail[0]) if tail is not None and not owner.training and x.is_cuda and x.bit_count == 64 else None
+        trees = tail is not None and not any(m.training for m in (owner, *tail[0])) and x.is_cuda and x.bit_count == 64
+        plan = tree_plan(*tail[0]) if trees else None
         if plan is None:
             return net(x)
-        h = x
-        for i, m in enumerate(net):
-            if i == n - 4:
-                break
-            h = m(h)
-        if type(h) is not PackBitsTensor or h.image or h.t.shape[0] != tail[0][0].in_dim or not h.t.is_contiguous():
+        h = _head_of(net, x)
+        if (type(h) is not PackBitsTensor or h.image or h.t.shape[0] != tail[0][0].in_dim or not h.t.is_contiguous()
+                or h.t.device != tail[0][0]._parameters["weights"].device):
             return _rest(net, n - 4, h)
         return tree_packed(tail[0], tail[1].k, h, plan)
-    if not (owner.training and isinstance(x, torch.Tensor) and x.is_cuda and torch.is_grad_enabled()):
+    if not (isinstance(x, torch.Tensor) and x.is_cuda):
         return net(x)
-    plan = tree_plan(*tail[0]) if tail is not None and x.dtype == torch.float32 and x.shape[0] % 4 == 0 and x.shape[0] > 0 else None
+    trees = tail is not None and x.dtype == torch.float32 and x.dim() > 0 and x.shape[0] > 0
+    if not (owner.training and torch.is_grad_enabled()):
+        if not trees or any(m.training for m in tail[0]) or (plan := tree_plan(*tail[0])) is None:
+            return net(x)
+        h = _head_of(net, x)
+        if _trees_take(h, tail[0][0]):
+            return tree_eval(tail[0], tail[1], _feature_major(h.detach()), plan)
+        return _rest(net, n - 4, h)
+    plan = tree_plan(*tail[0]) if trees and all(m.training for m in tail[0]) else None
     mode = owner.__dict__.get("prefold", True)                       # True: where it pays, "always", False
     layers = [m for m in net if isinstance(m, (ConvLogicLayer, LogicLayer))]
     if mode:
         _prefold(owner, layers if plan is None else layers[:-3], x, mode)
     if plan is not None:
-        h = x
-        for i, m in enumerate(net):
-            if i == n - 4:
-                break
-            h = m(h)
-        if h.dim() == 2 and h.shape[1] == tail[0][0].in_dim and h.dtype == torch.float32:
+        h = _head_of(net, x)
+        if _trees_take(h, tail[0][0]):
             return tree_train(tail[0], tail[1], _feature_major(h), plan)
         return _rest(net, n - 4, h)
     if (owner.__dict__.get("fused_tail", True) and n >= 2 and isinstance(net[n - 2], LogicLayer) and isinstance(net[n - 1], GroupSum)
@@ -125,6 +127,20 @@ def _forward(owner, x):
             h = m(h)
         return logic_layer_group_sum(net[n - 2], net[n - 1], h)
     return net(x)
+
+
+def _trees_take(h, first):
+    """True for what the modules themselves would accept (they raise for anything else), up to the kernels' grid"""
+    return (h.dim() == 2 and h.shape[1] == first.in_dim and h.dtype == torch.float32 and h.device == first._parameters["weights"].device
+            and h.shape[0] <= 1 << 20)
+
+
+def _head_of(net, h):
+    """all but the last four modules of a network"""
+    for i, m in enumerate(net):
+        if i == len(net) - 4:
+            return h
+        h = m(h)
 
 
 def _rest(net, i0, h):

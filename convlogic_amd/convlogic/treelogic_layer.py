@@ -6,7 +6,7 @@ from torch.autograd import Function
 
 from ..difflogic.functional import GradFactor, bin_op_s
 from ..difflogic.packbitstensor import PackBitsTensor
-from ..hip import convlogic_hip
+from ..hip import convlogic_hip, difflogic_hip
 
 
 class TreeLogicFunction(Function):
@@ -34,6 +34,13 @@ def gate_probabilities(logits, training, dtype):
     if training:
         return torch.nn.functional.softmax(logits, dim=-1)
     return torch.nn.functional.one_hot(logits.argmax(-1), num_classes=16).to(dtype=dtype)
+
+
+def kernel_probabilities(logits, training, dtype):
+    """gate_probabilities() as the kernels read them: dense, in x's element type (the bindings reject any other)"""
+    if not training:
+        return difflogic_hip.gate_onehot(logits, dtype)
+    return gate_probabilities(logits, training, dtype).to(dtype).contiguous()
 
 
 class TreeLogicLayer(nn.Module):
@@ -66,8 +73,7 @@ class TreeLogicLayer(nn.Module):
         raise ValueError(f"Unknown implementation {self.implementation!r}")
 
     def forward_cuda(self, x):
-        # the kernels read the probabilities in x's element type (the bindings reject any other)
-        w_prob = gate_probabilities(self.weights, self.training, x.dtype).to(x.dtype).contiguous()
+        w_prob = kernel_probabilities(self.weights, self.training, x.dtype)
         return TreeLogicFunction.apply(x, w_prob)
 
     def forward_python(self, x):

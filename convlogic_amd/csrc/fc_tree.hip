@@ -19,8 +19,8 @@
 // backward, the 2.7 GB of operand gradients written once and read once.  Keeping the first layer's output gradient instead (half
 // the bytes to write) needs a gather that reads every row twice plus the other operand's row: 1133 us in place of the
 // 536 us of the sum over consecutive rows.
-// Activations are feature-major with a row pitch that is a multiple of 4; samples from `batch` up to the pitch are computed
-// like any other, carry no gradient and are not written to the result.
+// Activations are feature-major with a row pitch; samples from `batch` up to the pitch are computed like any other, carry no
+// gradient and are not written to the result.
 #include <algorithm>
 
 #include "conv_ops.h"
@@ -376,7 +376,13 @@ __global__ __launch_bounds__(kTreeBlock) void fc_tree_gather_kernel(const float 
     store_samples<V>(gx + (int64_t)i * pitch + s, sum);
 }
 
-int tree_vec(int64_t pitch) { return pitch <= 64 ? 1 : (pitch <= 128 ? 2 : 4); }
+// the widest lanes that a row fills and that its pitch and the buffers' alignment allow
+int tree_vec(int64_t pitch, const void *x, const void *grad_x)
+{
+    const uintptr_t align = (uintptr_t)x | (uintptr_t)grad_x | (uintptr_t)(pitch * 4);
+    const int fit = pitch <= 64 ? 1 : (pitch <= 128 ? 2 : 4);
+    return (align & 15) == 0 ? fit : ((align & 7) == 0 && fit > 1 ? 2 : 1);
+}
 
 int check_tree(const char *name, int64_t in_dim, int64_t roots, int64_t k)
 {
@@ -422,10 +428,10 @@ extern "C" int clg_fc_tree_forward(const float *x, const int32_t *rows, const fl
     const char *name = "clg_fc_tree_forward";
     if (int e = check_tree(name, in_dim, roots, k)) return e;
     CLG_REQUIRE(x && rows && coef && partial && out, "%s: null pointer argument", name);
-    CLG_REQUIRE(batch > 0 && pitch >= batch && pitch % 4 == 0 && pitch < (1ll << 28) && tau != 0.0,
-                "%s: the row pitch must be a multiple of 4 that holds the batch, tau must not be zero", name);
+    CLG_REQUIRE(batch > 0 && pitch >= batch && pitch < (1ll << 28) && tau != 0.0, "%s: the row pitch must hold the batch, tau must not be zero",
+                name);
     const int slices = tree_slices(roots / k, batch, k);
-    int vec = tree_vec(pitch);                                        // fewer samples per lane where the launch would have less than four wavefronts per SIMD
+    int vec = tree_vec(pitch, x, partial);                                        // fewer samples per lane where the launch would have less than four wavefronts per SIMD
     while (vec > 1 && (int64_t)slices * k * clg_ceil_div(pitch, (int64_t)kWave * vec) * kTreeWaves < 4096) vec /= 2;
     const dim3 grid((unsigned)slices, (unsigned)k, (unsigned)clg_ceil_div(pitch, (int64_t)kWave * vec));
     CLG_REQUIRE(grid.z <= 65535, "%s: batch too large", name);
@@ -452,9 +458,9 @@ extern "C" int clg_fc_tree_backward(const float *x, const int32_t *rows, const i
     if (int e = check_tree(name, in_dim, roots, k)) return e;
     CLG_REQUIRE(x && rows && pos && slot && coef && grad_out && probs && grad0 && grad1 && grad2 && rowgrad && sums && start &&
                     grad_x, "%s: null pointer argument", name);
-    CLG_REQUIRE(batch > 0 && pitch >= batch && pitch % 4 == 0 && pitch < (1ll << 28) && tau != 0.0,
-                "%s: the row pitch must be a multiple of 4 that holds the batch, tau must not be zero", name);
-    const int vec = tree_vec(pitch);
+    CLG_REQUIRE(batch > 0 && pitch >= batch && pitch < (1ll << 28) && tau != 0.0, "%s: the row pitch must hold the batch, tau must not be zero",
+                name);
+    const int vec = tree_vec(pitch, (const void *)((uintptr_t)x | (uintptr_t)rowgrad), grad_x);
     hipStream_t st = clg_stream(stream);
     const TreeGrads gr = {{grad0, grad1, grad2}, {4 * roots, 6 * roots, 7 * roots}};
     const dim3 grid((unsigned)clg_ceil_div(roots, kTreeWaves));

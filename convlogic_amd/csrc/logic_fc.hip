@@ -851,6 +851,21 @@ __global__ __launch_bounds__(256) void gate_argmax_kernel(const S *__restrict__ 
     gate[r] = (uint8_t)at;
 }
 
+// probs[r] = one-hot of the arg-max gate of row r, by the same rule: sixteen lanes per row, so that reads and writes are whole
+// lines.  One launch of 4 us in place of argmax, one_hot (fill, scatter) and the conversion, 4 to 8 us each.
+template <typename T>
+__global__ __launch_bounds__(256) void gate_onehot_kernel(const T *__restrict__ logits, T *__restrict__ probs, int64_t rows)
+{
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= rows * 16) return;
+    const T v = logits[e];
+    const T top = row16_max(v != v ? T(0) : v);                      // (unused where the row holds a NaN)
+    const int row0 = threadIdx.x & 48;                               // the row's first lane
+    const unsigned nans = (unsigned)(__ballot(v != v) >> row0) & 0xFFFFu, tops = (unsigned)(__ballot(v == top) >> row0) & 0xFFFFu;
+    const unsigned at = (unsigned)__builtin_ctz(nans ? nans : tops);
+    probs[e] = (threadIdx.x & 15) == at ? T(1) : T(0);
+}
+
 int grid_for(int64_t items)
 {
     const int64_t blocks = clg_ceil_div(items, kWavesPerBlock);
@@ -894,6 +909,19 @@ extern "C" int clg_gate_argmax(int dtype, const void *logits, uint8_t *gate, int
     else if (dtype == CLG_F64) hipLaunchKernelGGL(gate_argmax_kernel<double>, grid, block, 0, st, (const double *)logits, gate, rows);
     else hipLaunchKernelGGL(gate_argmax_kernel<__half>, grid, block, 0, st, (const __half *)logits, gate, rows);
     CLG_CHECK_LAUNCH("clg_gate_argmax");
+    return CLG_OK;
+}
+
+extern "C" int clg_gate_onehot(int dtype, const void *logits, void *probs, int64_t rows, void *stream)
+{
+    CLG_REQUIRE(dtype == CLG_F32 || dtype == CLG_F64, "clg_gate_onehot: dtype must be CLG_F32 or CLG_F64, got %d", dtype);
+    CLG_REQUIRE(logits && probs, "clg_gate_onehot: null pointer argument");
+    CLG_REQUIRE(rows > 0 && rows < (1ll << 35), "clg_gate_onehot: rows must be in 1..2^35-1");
+    const dim3 grid((unsigned)clg_ceil_div(rows, 16)), block(256);
+    hipStream_t st = clg_stream(stream);
+    if (dtype == CLG_F32) hipLaunchKernelGGL(gate_onehot_kernel<float>, grid, block, 0, st, (const float *)logits, (float *)probs, rows);
+    else hipLaunchKernelGGL(gate_onehot_kernel<double>, grid, block, 0, st, (const double *)logits, (double *)probs, rows);
+    CLG_CHECK_LAUNCH("clg_gate_onehot");
     return CLG_OK;
 }
 

@@ -107,7 +107,7 @@ class LogicLayer(torch.nn.Module):
                                                    buffers["given_x_indices_of_y"], self._sole_consumers(key), inside,
                                                    prefolded).transpose(0, 1)
         xt = _feature_major(x)
-        w = self._gate_weights(xt.dtype)
+        w = self._gate_weights(xt.dtype) if self.training else difflogic_hip.gate_onehot(self.weights, xt.dtype)
         args = (xt, self.indices_0, self.indices_1, w, self.given_x_indices_of_y_start, self.given_x_indices_of_y)
         if self.training:
             return LogicLayerCudaFunction.apply(*args).transpose(0, 1)

@@ -99,8 +99,25 @@ def _tree_forward(lib, x, plan, coef, k, tau, st):
     return out
 
 
+class _TreeEvalFunction(torch.autograd.Function):
+    """The same class sums with the arg-max gates: evaluation, which has no gradient."""
+
+    @staticmethod
+    def forward(ctx, x, l0, l1, l2, plan, k, tau):
+        lib, st = _lib.load(), stream_ptr(x)
+        coef = torch.empty((plan.roots, 28), dtype=torch.float32, device=x.device)
+        check(lib.clg_fc_tree_fold(l0.data_ptr(), l1.data_ptr(), l2.data_ptr(), plan.ids.data_ptr(), coef.data_ptr(), None, plan.roots, 1, st))
+        return _tree_forward(lib, x, plan, coef, k, tau, st)
+
+
+def tree_eval(layers, group_sum, x, plan):
+    """group_sum(third(second(first(x)))) of layers in evaluation mode; x feature-major [features, B]."""
+    with torch.no_grad():
+        return _TreeEvalFunction.apply(x, *(layer.weights for layer in layers), plan, group_sum.k, group_sum.tau)
+
+
 def tree_train(layers, group_sum, x, plan):
-    """group_sum(third(second(first(x)))) in training; x feature-major [features, B], B a multiple of 4."""
+    """group_sum(third(second(first(x)))) in training; x feature-major [features, B]."""
     first, second, third = layers
     return _TreeFunction.apply(x, first.weights, second.weights, third.weights, first._buffers["given_x_indices_of_y_start"], plan,
                                group_sum.k, group_sum.tau)

@@ -31,6 +31,7 @@ SIGNATURES = {
     "clg_abi_version": (_i, []),
     "clg_reload_knobs": (None, []),
     "clg_gate_argmax": (_i, [_i, _p, _p, _i64, _p]),
+    "clg_gate_onehot": (_i, [_i, _p, _p, _i64, _p]),
     "clg_fc_forward": (_i, [_i, _p, _p, _p, _p, _p, _i64, _i64, _i64, _p]),
     "clg_fc_backward_w": (_i, [_i, _p, _p, _p, _p, _p, _i64, _i64, _i64, _p]),
     "clg_fc_backward_logits": (_i, [_i, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _p]),

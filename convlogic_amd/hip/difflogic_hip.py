@@ -348,6 +348,18 @@ def gate_argmax(logits):
     return gate
 
 
+def gate_onehot(logits, dtype):
+    """One-hot of the arg-max gate over the last dimension of logits [..., 16], in `dtype`: the probabilities a layer evaluates
+    with.  One launch for dense device logits of that type, torch's operations for any other."""
+    if (logits.is_cuda and logits.is_contiguous() and logits.dtype == dtype and dtype in _lib._DTYPES and logits.shape[-1] == 16
+            and logits.numel()):
+        logits = logits.detach()
+        probs = torch.empty_like(logits)
+        check(_lib.load().clg_gate_onehot(dtype_code(logits), logits.data_ptr(), probs.data_ptr(), logits.numel() // 16, stream_ptr(logits)))
+        return probs
+    return torch.nn.functional.one_hot(logits.argmax(-1), 16).to(dtype)
+
+
 def eval_plan(a, b, in_dim):
     """Walk order of the wiring graph for eval_planned (int32 [out], on the device of `a`).  Host
     computation, done once per wiring."""

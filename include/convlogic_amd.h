@@ -256,6 +256,8 @@ int clg_fc_eval_plan(const int64_t *a_host /*[out_dim]*/, const int64_t *b_host 
  * (fused block); dtype CLG_F32, CLG_F64 or CLG_F16.  Replaces self.weights.argmax(-1).to(torch.uint8) of
  * LogicLayer.forward_cuda_eval (src/difflogic/difflogic.py:161), taken on every packed call as there. */
 int clg_gate_argmax(int dtype, const void *logits /*[rows,16]*/, uint8_t *gate /*[rows]*/, int64_t rows, void *stream);
+/* probs [rows, 16] = one-hot of the same arg-max, in the logits' type (float32 / float64): what the layers evaluate with */
+int clg_gate_onehot(int dtype, const void *logits, void *probs, int64_t rows, void *stream);
 
 /* Same result as clg_fc_eval_packed, evaluated in plan order: the shared input row of consecutive
  * neurons stays in registers, so every input row is fetched about once instead of twice.  plan is
@@ -504,7 +506,7 @@ int clg_host_flag_device_pointer(void *host, void **device);
  *   pos  [roots, 8]  place of each operand in the lists input feature -> operands (CSR, `start` [in_dim + 1])
  *   slot [7 roots]   of every neuron, first layer first: root * 7 + its place among the tree's gates
  *   logits0..2       the layers' logits [out, 16]         coef [roots, 7, 4] folded coefficients in tree order
- * x is feature-major with a row pitch (multiple of 4) >= batch.
+ * x is feature-major with a row pitch >= batch (lanes are 1, 2 or 4 samples wide, whatever pitch and addresses allow).
  * ------------------------------------------------------------------------------- */
 /* coef of the softmax (hard = 0) or the arg-max gates (hard = 1); probs [7 roots, 16] takes the probabilities, neurons of the first
  * layer first (may be NULL) */

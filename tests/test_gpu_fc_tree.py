@@ -18,7 +18,7 @@ def tail(in_dim, roots, k, seed):
     return [C.LogicLayer(a, b, implementation="cuda").to(DEV) for a, b in zip(dims, dims[1:])], C.GroupSum(k, tau=3.0)
 
 
-@pytest.mark.parametrize("batch", [4, 64, 68, 128, 132, 256, 260, 516])
+@pytest.mark.parametrize("batch", [1, 4, 63, 64, 65, 68, 126, 128, 129, 132, 256, 258, 260, 513, 516])
 @pytest.mark.parametrize("in_dim,roots,k", [(8, 2, 1), (40, 130, 10), (700, 663, 3)])
 def test_training_against_the_oracle(batch, in_dim, roots, k):
     layers, gs = tail(in_dim, roots, k, batch + roots)
@@ -147,3 +147,42 @@ def test_modules_with_hooks_are_called_themselves(hook):
     finally:
         handle.remove()
     assert calls.count(C.LogicLayer) >= 2                              # the first two of the three (the last runs with the GroupSum)
+
+
+@pytest.mark.parametrize("batch", [1, 63, 66, 128, 255, 256, 1001])
+def test_evaluation_equals_the_modules(batch):
+    layers, gs = tail(700, 663, 3, batch)
+    net = torch.nn.Sequential(*layers, gs).eval()
+    x = torch.randint(0, 2, (batch, 700), device=DEV).float()
+    got = fc_tree.tree_eval(layers, gs, x.t().contiguous(), fc_tree.tree_plan(*layers))
+    assert not got.requires_grad and torch.equal(got, net(x))          # class sums are whole numbers
+    x = torch.rand(batch, 700, device=DEV)
+    assert torch.allclose(fc_tree.tree_eval(layers, gs, x.t().contiguous(), fc_tree.tree_plan(*layers)), net(x), rtol=2e-6, atol=0)
+
+
+def test_a_network_evaluates_its_tail_as_trees():
+    torch.manual_seed(5)
+    model = C.ConvLogicMnistModel(k_param=2).to(DEV).eval()
+    x, results = torch.randint(0, 2, (33, 1, 28, 28), device=DEV).float(), []
+    for on in (True, False):
+        model.tree_tail = on
+        results.append(model(x))
+    assert torch.equal(*results) and not results[0].requires_grad
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_onehot_of_the_first_maximum(dtype):
+    from convlogic_amd.hip import difflogic_hip
+    logits = torch.randn(37, 7, 16, device=DEV, dtype=dtype)
+    logits[0, 0] = 1.0                                                 # ties, NaN, infinities, zeros of both signs
+    logits[0, 1, 5] = logits[0, 1, 9] = float("nan")
+    logits[0, 2] = -float("inf")
+    logits[0, 3, 7] = logits[0, 3, 11] = float("inf")
+    logits[0, 4] = -0.0
+    logits[0, 4, 6] = 0.0
+    logits[0, 5] = -float("inf")
+    logits[0, 5, 15] = float("nan")
+    logits[0, 6] = torch.finfo(dtype).min
+    got = difflogic_hip.gate_onehot(logits, dtype)
+    assert got.dtype == dtype and torch.equal(got, torch.nn.functional.one_hot(logits.argmax(-1), 16).to(dtype))
+    assert torch.equal(got.argmax(-1).to(torch.uint8), difflogic_hip.gate_argmax(logits))
