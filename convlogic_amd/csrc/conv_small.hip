@@ -16,8 +16,12 @@
 namespace {
 
 constexpr int kLsWaves = 4;                        // wavefronts per workgroup
-constexpr int kLsPlane = 36;                       // padded 6x6 plane
-constexpr int kLsStride = 2 * kLsPlane + 1;        // elements per lane
+// The two planes of a lane with shared halos: the right halo of a row is the left halo of the next, the bottom halo row of the
+// first plane the top one of the second: 56 elements instead of 72, so a wavefront takes 14.6 KB and a CU holds 10 of them, not 8.
+constexpr int kLsRow = 5;                          // row pitch
+constexpr int kLsPlane = 5 * kLsRow;               // top halo row and the four rows of a plane
+constexpr int kLsStride = 2 * kLsPlane + kLsRow + 2;   // elements per lane: the last halo row and its right neighbour; odd
+__host__ __device__ constexpr int ls_at(int row, int col) { return row * kLsRow + col; }   // padded position (1, 1 = first pixel)
 
 // The taps of one kernel, sorted into at most two planes.
 struct LaneTaps {
@@ -98,10 +102,10 @@ __global__ __launch_bounds__(kLsWaves *kWave) void convblock_forward_4x4_kernel(
     while (true) {
         if (live && !tp.wide) {
 #pragma unroll
-            for (int e = 0; e < 16; ++e) mine[((e >> 2) + 1) * 6 + (e & 3) + 1] = pl.v[e];
+            for (int e = 0; e < 16; ++e) mine[ls_at((e >> 2) + 1, (e & 3) + 1)] = pl.v[e];
             if (tp.ch1 != tp.ch0) {
 #pragma unroll
-                for (int e = 0; e < 16; ++e) mine[kLsPlane + ((e >> 2) + 1) * 6 + (e & 3) + 1] = pl.v[16 + e];
+                for (int e = 0; e < 16; ++e) mine[kLsPlane + ls_at((e >> 2) + 1, (e & 3) + 1)] = pl.v[16 + e];
             }
         }
         const typename Ops::Params pr = Ops::load_global(params, c);
@@ -114,7 +118,38 @@ __global__ __launch_bounds__(kLsWaves *kWave) void convblock_forward_4x4_kernel(
         }
         const T *ta[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) ta[k] = mine + (cur.ch[k] != cur.ch0 ? kLsPlane : 0) + cur.ry[k] * 6 + cur.rx[k];
+        for (int k = 0; k < 8; ++k) ta[k] = mine + (cur.ch[k] != cur.ch0 ? kLsPlane : 0) + ls_at(cur.ry[k], cur.rx[k]);
+        const int64_t o = (n * g.c + c) * 4;
+        if (cur.wide) {
+            // taps in more than two channels (caller-made selection): from global memory, cell by cell in a real loop so that
+            // the rare case costs the other one no registers and no waits for the planes in flight
+            const LaneTaps wt = lane_taps(sel, c, tap_limit(g));
+#pragma unroll 1
+            for (int cell = 0; cell < 4; ++cell) {
+                T r[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int oy = 2 * (cell >> 1) + (q >> 1), ox = 2 * (cell & 1) + (q & 1);
+                    T v[8];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) {
+                        const int iy = oy + wt.ry[k] - 1, ix = ox + wt.rx[k] - 1;
+                        v[k] = T(0);
+                        if ((unsigned)iy < 4u && (unsigned)ix < 4u && live) v[k] = xn[wt.ch[k] * 16 + iy * 4 + ix];
+                    }
+                    r[q] = Ops::root(pr, v);
+                }
+                int code;
+                const T best = Ops::pool4(pr, r, code);
+                if (live) {
+                    y[g.y_fm ? ((int64_t)c * 4 + cell) * g.n + n : o + cell] = best;
+                    if (argmax != nullptr) argmax[o + cell] = (uint8_t)code;
+                }
+            }
+            if (!more) break;
+            c = cn;
+            continue;
+        }
         T best[4];
         int codes = 0;
 #pragma unroll
@@ -124,17 +159,8 @@ __global__ __launch_bounds__(kLsWaves *kWave) void convblock_forward_4x4_kernel(
             for (int q = 0; q < 4; ++q) {
                 const int oy = 2 * (cell >> 1) + (q >> 1), ox = 2 * (cell & 1) + (q & 1);
                 T v[8];
-                if (!cur.wide) {
 #pragma unroll
-                    for (int k = 0; k < 8; ++k) v[k] = ta[k][oy * 6 + ox];
-                } else {
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) {
-                        const int iy = oy + cur.ry[k] - 1, ix = ox + cur.rx[k] - 1;
-                        v[k] = T(0);
-                        if ((unsigned)iy < 4u && (unsigned)ix < 4u && live) v[k] = xn[cur.ch[k] * 16 + iy * 4 + ix];
-                    }
-                }
+                for (int k = 0; k < 8; ++k) v[k] = ta[k][ls_at(oy, ox)];
                 r[q] = Ops::root(pr, v);
             }
             int code;
@@ -142,7 +168,6 @@ __global__ __launch_bounds__(kLsWaves *kWave) void convblock_forward_4x4_kernel(
             codes |= code << (8 * cell);
         }
         if (live) {
-            const int64_t o = (n * g.c + c) * 4;
             if (g.y_fm) {                                             // [c, 2, 2, n]: the lanes' samples are neighbours
 #pragma unroll
                 for (int cell = 0; cell < 4; ++cell) y[((int64_t)c * 4 + cell) * g.n + n] = best[cell];
@@ -201,7 +226,7 @@ __global__ __launch_bounds__(kLsWaves *kWave, 2) void convblock_eval_packed_4x4_
     const int piece = lane & 7, sub = lane >> 3;
     const uint64_t *xw = x + ((int64_t)sblock * kWave + sub) * g.cin * 16 + 2 * piece;   // load j: + 8 j groups
     const int64_t group_step = (int64_t)8 * g.cin * 16;
-    uint32_t *put = slices + sub * kLsStride + ((piece >> 1) + 1) * 6 + 2 * (piece & 1) + 1;   // + 8 j slices, + plane
+    uint32_t *put = slices + sub * kLsStride + ls_at((piece >> 1) + 1, 2 * (piece & 1) + 1);   // + 8 j slices, + plane
     PackedPlanes pl;
     // Only the channels of the next kernel are looked at ahead of time (its taps are read again when its turn comes:
     // scalar registers are scarce next to 28 gate masks).  Both planes are always fetched and written, also when a
@@ -222,7 +247,7 @@ __global__ __launch_bounds__(kLsWaves *kWave, 2) void convblock_eval_packed_4x4_
         const bool more = cn < c1;
         const uint32_t *ta[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) ta[k] = mine + (cur.ch[k] != cur.ch0 ? kLsPlane : 0) + cur.ry[k] * 6 + cur.rx[k];
+        for (int k = 0; k < 8; ++k) ta[k] = mine + (cur.ch[k] != cur.ch0 ? kLsPlane : 0) + ls_at(cur.ry[k], cur.rx[k]);
         if (cur.wide) {
             // taps in more than two channels (caller-made selection): 64-bit words straight from global memory, cell by
             // cell in a real loop so that the rare case costs no registers
@@ -274,7 +299,7 @@ __global__ __launch_bounds__(kLsWaves *kWave, 2) void convblock_eval_packed_4x4_
                         const int oy = 2 * (cell >> 1) + (q >> 1), ox = 2 * (cell & 1) + (q & 1);
                         uint32_t v[8];
 #pragma unroll
-                        for (int k = 0; k < 8; ++k) v[k] = ta[k][oy * 6 + ox];
+                        for (int k = 0; k < 8; ++k) v[k] = ta[k][ls_at(oy, ox)];
                         pooled |= BitOps::root32(pr, v);
                     }
                     best[cell] |= (uint64_t)pooled << (32 * half);
@@ -303,26 +328,58 @@ __global__ __launch_bounds__(kLsWaves *kWave, 2) void convblock_eval_packed_4x4_
 //                                      pooled arg-max position of the 4 cells once, accumulates the 28 weight-gradient
 //                                      sums of its kernel over all samples (registers, then DPP and a fixed-order
 //                                      combine of the 4 wavefronts) and writes the 4 x 8 tap gradients of every
-//                                      (kernel, sample) to tg[c][n][cell][tap] (and its 4 arg-max codes to tcodes[c][n]);
+//                                      (kernel, sample) to tg[c][tap][n][cell] (and its 4 arg-max codes to tcodes[c][n]);
 //   convblock_backward_x_4x4_kernel    channel-major: a lane owns the gradient plane of (sample, channel) in its LDS
 //                                      slice and adds the tap gradients of the kernels that read the channel, in
 //                                      increasing kernel order, taps in order -- a fixed summation order.
 // The tree and its derivatives are evaluated once per (kernel, sample, cell) for both gradients.
+// tg is what the pair moves most of (512 B per kernel and sample row of 4 cells, float32).  A tap belongs to ONE of the
+// kernel's two channels, so tap-major rows are read by their channel alone, once, and every access is 16 bytes per lane on
+// consecutive addresses; sample-major pieces of 128 bytes per lane ([c][n][cell][tap]) were fetched whole by both channels.
+// What bounds the first pass is wavefronts: LDS allows 10 per CU (8 with unshared halos), registers 12, and a workgroup has no
+// wavefront that finds no samples.  Second pass: the stream of tg.
+// [128, 16384, 4, 4] -> 32768: 475 + 239 -> 389 + 172 us (1.6 and 3.9 TB/s of tg); [256, 512, 4, 4] -> 1024: 28.5 + 24.9 -> 23.8 + 16.1 us.
 
-constexpr int kGradStride = kLsPlane + 1;          // gradient plane: padded 6x6 (taps of border cells fall into the halo)
+constexpr int kGradStride = kLsPlane + kLsRow + 1; // gradient plane (taps of border cells fall into the halo); odd
 
+// the gradients of a tap at the 4 cells of a sample, as 16-byte pieces
 template <typename T>
-__global__ __launch_bounds__(kLsWaves *kWave) void convblock_backward_4x4_kernel(
+__device__ __forceinline__ void store_cells(T *dst, const T *v)
+{
+    constexpr int PER = 16 / (int)sizeof(T);
+#pragma unroll
+    for (int q = 0; q < 4 / PER; ++q) {
+        u32x4 raw;
+        __builtin_memcpy(&raw, v + q * PER, 16);
+        reinterpret_cast<u32x4 *>(dst)[q] = raw;
+    }
+}
+template <typename T>
+__device__ __forceinline__ void load_cells(T *v, const T *src)
+{
+    constexpr int PER = 16 / (int)sizeof(T);
+#pragma unroll
+    for (int q = 0; q < 4 / PER; ++q) {
+        const u32x4 raw = reinterpret_cast<const u32x4 *>(src)[q];
+        __builtin_memcpy(v + q * PER, &raw, 16);
+    }
+}
+
+// The wavefronts of a workgroup (1, 2 or 4) deal the 64-sample blocks among themselves.
+template <typename T>
+__global__ __launch_bounds__(kLsWaves *kWave, sizeof(T) == 4 ? 3 : 1) void convblock_backward_4x4_kernel(
     const T *__restrict__ x, const T *__restrict__ folded, const int32_t *__restrict__ sel, const T *__restrict__ gy,
     const uint8_t *__restrict__ argmax, T *__restrict__ tg, uint32_t *__restrict__ tcodes, T *__restrict__ gw,
     const T *__restrict__ probs, Geom g, int ct)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ T meet[kLsWaves][28];
-    const int lane = threadIdx.x & (kWave - 1), wave = uniform((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & (kWave - 1), wave = uniform((int)(threadIdx.x >> 6)), waves = blockDim.x >> 6;
     T *mine = reinterpret_cast<T *>(smem) + ((size_t)wave * kWave + lane) * kLsStride;
 #pragma unroll
     for (int e = 0; e < kLsStride; ++e) mine[e] = T(0);
+    for (int e = threadIdx.x; e < kLsWaves * 28; e += blockDim.x) meet[e / 28][e % 28] = T(0);   // wavefronts that are not there
+    __syncthreads();
     const int sblocks = (g.n + kWave - 1) / kWave;
     const int c0 = blockIdx.x * ct, c1 = min(g.c, c0 + ct);
     for (int c = c0; c < c1; ++c) {
@@ -333,97 +390,103 @@ __global__ __launch_bounds__(kLsWaves *kWave) void convblock_backward_4x4_kernel
         for (int q = 0; q < 7; ++q) tr.g[q] = Coef<T>{fc[4 * q], fc[4 * q + 1], fc[4 * q + 2], fc[4 * q + 3]};
         const T *ta[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) ta[k] = mine + (tp.ch[k] != tp.ch0 ? kLsPlane : 0) + tp.ry[k] * 6 + tp.rx[k];
+        for (int k = 0; k < 8; ++k) ta[k] = mine + (tp.ch[k] != tp.ch0 ? kLsPlane : 0) + ls_at(tp.ry[k], tp.rx[k]);
         T acc[28];
 #pragma unroll
         for (int k = 0; k < 28; ++k) acc[k] = T(0);
-        // the wavefronts of the workgroup deal the 64-sample blocks among themselves; planes one block ahead
-        int sb = wave;
-        Planes<T> pl;
-        {
-            const int64_t n = (int64_t)sb * kWave + lane;
-            if (sb < sblocks) fetch_planes(pl, tp, x + (n < g.n ? n : 0) * g.cin * 16, n < g.n);
-        }
-        for (; sb < sblocks; sb += kLsWaves) {
+        // the tree and its derivatives at one cell: adds to the 28 sums, leaves the tap gradients in v
+        auto cell_gradients = [&](T (&v)[8], T go) {
+            const TreeVals<T> tv = eval_tree(tr, v);
+            const T g_m[2] = {go * gate_da(tr.g[6], tv.mid[1]), go * gate_db(tr.g[6], tv.mid[0])};
+            T g_l[4];
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                g_l[2 * m] = g_m[m] * gate_da(tr.g[4 + m], tv.leaf[2 * m + 1]);
+                g_l[2 * m + 1] = g_m[m] * gate_db(tr.g[4 + m], tv.leaf[2 * m]);
+            }
+            // weight-gradient sums: (g a b, g a, g b, g) per gate
+            auto add = [&](int q, T gg, T a, T b) {
+                acc[4 * q] = fma_t(gg, a * b, acc[4 * q]);
+                acc[4 * q + 1] = fma_t(gg, a, acc[4 * q + 1]);
+                acc[4 * q + 2] = fma_t(gg, b, acc[4 * q + 2]);
+                acc[4 * q + 3] += gg;
+            };
+            add(6, go, tv.mid[0], tv.mid[1]);
+            add(4, g_m[0], tv.leaf[0], tv.leaf[1]);
+            add(5, g_m[1], tv.leaf[2], tv.leaf[3]);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const T a = v[2 * q], b = v[2 * q + 1];
+                add(q, g_l[q], a, b);
+                v[2 * q] = g_l[q] * gate_da(tr.g[q], b);
+                v[2 * q + 1] = g_l[q] * gate_db(tr.g[q], a);
+            }
+        };
+        for (int sb = wave; sb < sblocks; sb += waves) {
             const int64_t n = (int64_t)sb * kWave + lane;
             const bool live = n < g.n;
-            const T *xn = x + (live ? n : 0) * g.cin * 16;
-            if (!tp.wide) {
+            const int64_t ns = live ? n : g.n - 1;                    // lanes without a sample: the last one's values, gradient 0
+            const T *xn = x + ns * g.cin * 16;
+            const int64_t o = (ns * g.c + c) * 4;
+            T gout[4];
+            const uint32_t codes = *reinterpret_cast<const uint32_t *>(argmax + o);
 #pragma unroll
-                for (int e = 0; e < 16; ++e) mine[((e >> 2) + 1) * 6 + (e & 3) + 1] = live ? pl.v[e] : T(0);
-                if (tp.ch1 != tp.ch0) {
+            for (int cell = 0; cell < 4; ++cell) gout[cell] = g.y_fm ? gy[((int64_t)c * 4 + cell) * g.n + ns] : gy[o + cell];
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) mine[kLsPlane + ((e >> 2) + 1) * 6 + (e & 3) + 1] = live ? pl.v[16 + e] : T(0);
+            for (int cell = 0; cell < 4; ++cell) gout[cell] = live ? gout[cell] : T(0);
+            T *dst = tg != nullptr && live ? tg + ((int64_t)c * 8 * g.n + n) * 4 : nullptr;
+            const int64_t tap_step = (int64_t)g.n * 4;
+            if (dst) tcodes[(int64_t)c * g.n + n] = codes;            // kernel-major copy: the second pass reads it coalesced
+            if (tp.wide) {
+                // taps in more than two channels (caller-made selection): from global memory, cell by cell in a real loop so
+                // that the rare case costs the other one no registers and no waits
+                const LaneTaps wt = lane_taps(sel, c, tap_limit(g));
+#pragma unroll 1
+                for (int cell = 0; cell < 4; ++cell) {
+                    const int code = (codes >> (8 * cell)) & 3;
+                    const int oy = 2 * (cell >> 1) + (code >> 1), ox = 2 * (cell & 1) + (code & 1);
+                    T v[8];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) {
+                        const int iy = oy + wt.ry[k] - 1, ix = ox + wt.rx[k] - 1;
+                        const bool in = (unsigned)iy < 4u && (unsigned)ix < 4u;
+                        v[k] = in ? xn[wt.ch[k] * 16 + iy * 4 + ix] : T(0);
+                    }
+                    const T go = cell < 2 ? (cell == 0 ? gout[0] : gout[1]) : (cell == 2 ? gout[2] : gout[3]);
+                    cell_gradients(v, go);
+                    if (dst) {
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) dst[k * tap_step + cell] = v[k];
+                    }
                 }
+                continue;
             }
-            const int64_t o = (n * g.c + c) * 4;
-            T gout[4] = {T(0), T(0), T(0), T(0)};
-            uint32_t codes = 0;
-            if (live) {
+            Planes<T> pl;
+            load_plane(pl.v, 0, xn + tp.ch0 * 16);
+            load_plane(pl.v, 16, xn + tp.ch1 * 16);
 #pragma unroll
-                for (int cell = 0; cell < 4; ++cell) gout[cell] = g.y_fm ? gy[((int64_t)c * 4 + cell) * g.n + n] : gy[o + cell];
-                codes = *reinterpret_cast<const uint32_t *>(argmax + o);
-            }
-            {
-                const int sn = sb + kLsWaves;                          // next block's planes, in flight during the cells
-                const int64_t nn = (int64_t)sn * kWave + lane;
-                if (sn < sblocks) fetch_planes(pl, tp, x + (nn < g.n ? nn : 0) * g.cin * 16, nn < g.n);
+            for (int e = 0; e < 16; ++e) {
+                mine[ls_at((e >> 2) + 1, (e & 3) + 1)] = pl.v[e];
+                mine[kLsPlane + ls_at((e >> 2) + 1, (e & 3) + 1)] = pl.v[16 + e];
             }
             T gt[32];
 #pragma unroll
             for (int cell = 0; cell < 4; ++cell) {
                 const int code = (codes >> (8 * cell)) & 3;
-                const int oy = 2 * (cell >> 1) + (code >> 1), ox = 2 * (cell & 1) + (code & 1);
+                const int po = ls_at(2 * (cell >> 1) + (code >> 1), 2 * (cell & 1) + (code & 1));   // per lane: the pooled maximum's position
                 T v[8];
-                if (!tp.wide) {
-                    const int po = oy * 6 + ox;                        // per lane: the pooled maximum's position
 #pragma unroll
-                    for (int k = 0; k < 8; ++k) v[k] = ta[k][po];
-                } else {
+                for (int k = 0; k < 8; ++k) v[k] = ta[k][po];
+                cell_gradients(v, gout[cell]);
 #pragma unroll
-                    for (int k = 0; k < 8; ++k) {
-                        const int iy = oy + tp.ry[k] - 1, ix = ox + tp.rx[k] - 1;
-                        v[k] = T(0);
-                        if ((unsigned)iy < 4u && (unsigned)ix < 4u && live) v[k] = xn[tp.ch[k] * 16 + iy * 4 + ix];
-                    }
-                }
-                const TreeVals<T> tv = eval_tree(tr, v);
-                const T go = gout[cell];                               // 0 for lanes without a sample
-                const T g_m[2] = {go * gate_da(tr.g[6], tv.mid[1]), go * gate_db(tr.g[6], tv.mid[0])};
-                T g_l[4];
+                for (int k = 0; k < 8; ++k) gt[4 * k + cell] = v[k];
+                // one cell at a time: interleaved, the four take 199 registers and leave two wavefronts per SIMD
 #pragma unroll
-                for (int m = 0; m < 2; ++m) {
-                    g_l[2 * m] = g_m[m] * gate_da(tr.g[4 + m], tv.leaf[2 * m + 1]);
-                    g_l[2 * m + 1] = g_m[m] * gate_db(tr.g[4 + m], tv.leaf[2 * m]);
-                }
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    gt[cell * 8 + 2 * q] = g_l[q] * gate_da(tr.g[q], v[2 * q + 1]);
-                    gt[cell * 8 + 2 * q + 1] = g_l[q] * gate_db(tr.g[q], v[2 * q]);
-                }
-                // weight-gradient sums: (g a b, g a, g b, g) per gate
-                auto add = [&](int q, T gg, T a, T b) {
-                    acc[4 * q] = fma_t(gg, a * b, acc[4 * q]);
-                    acc[4 * q + 1] = fma_t(gg, a, acc[4 * q + 1]);
-                    acc[4 * q + 2] = fma_t(gg, b, acc[4 * q + 2]);
-                    acc[4 * q + 3] += gg;
-                };
-#pragma unroll
-                for (int q = 0; q < 4; ++q) add(q, g_l[q], v[2 * q], v[2 * q + 1]);
-                add(4, g_m[0], tv.leaf[0], tv.leaf[1]);
-                add(5, g_m[1], tv.leaf[2], tv.leaf[3]);
-                add(6, go, tv.mid[0], tv.mid[1]);
+                for (int k = 0; k < 28; ++k) asm volatile("" : "+v"(acc[k]));
             }
-            if (tg != nullptr && live) {
-                T *dst = tg + ((int64_t)c * g.n + n) * 32;
-                tcodes[(int64_t)c * g.n + n] = codes;                  // kernel-major copy: the second pass reads it coalesced
-                constexpr int PER = 16 / (int)sizeof(T);
+            if (dst) {
 #pragma unroll
-                for (int q = 0; q < 32 / PER; ++q) {
-                    u32x4 raw;
-                    __builtin_memcpy(&raw, &gt[q * PER], 16);
-                    reinterpret_cast<u32x4 *>(dst)[q] = raw;
-                }
+                for (int k = 0; k < 8; ++k) store_cells(dst + k * tap_step, &gt[4 * k]);
             }
         }
         // 28 sums of this kernel: lanes, then the wavefronts in order
@@ -433,15 +496,15 @@ __global__ __launch_bounds__(kLsWaves *kWave) void convblock_backward_4x4_kernel
             if (lane == 0) meet[wave][k] = t;
         }
         __syncthreads();
-        if (threadIdx.x < 7 * 16) {
-            const int q = threadIdx.x >> 4, i = threadIdx.x & 15;
+        for (int e = threadIdx.x; e < 7 * 16; e += blockDim.x) {
+            const int q = e >> 4, i = e & 15;
             T sums[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k) sums[k] = (meet[0][4 * q + k] + meet[1][4 * q + k]) + (meet[2][4 * q + k] + meet[3][4 * q + k]);
             T gi = coef_transpose_row<T>(i, sums[0], sums[1], sums[2], sums[3]);
-            const int64_t e = ((int64_t)c * 7 + q) * 16 + i;
-            if (probs != nullptr) gi = softmax16_backward(gi, probs[e]);       // gradient w.r.t. the logits
-            gw[e] = gi;
+            const int64_t at = (int64_t)c * 112 + e;
+            if (probs != nullptr) gi = softmax16_backward(gi, probs[at]);      // gradient w.r.t. the logits
+            gw[at] = gi;
         }
         __syncthreads();
     }
@@ -471,61 +534,81 @@ __global__ __launch_bounds__(kLsWaves *kWave) void convblock_backward_x_4x4_kern
     for (int e = 0; e < kGradStride; ++e) plane[e] = T(0);
     const int nhits = count[2 * ch];
     const int32_t *hit = hits + count[2 * ch + 1];
-    constexpr int PER = 16 / (int)sizeof(T);
-    auto fetch = [&](int k, T (&gt)[32], uint32_t &codes) {
-        const int c = hit[k] & 0xFFFF;
-        const T *src = tg + ((int64_t)c * g.n + ns) * 32;
-#pragma unroll
-        for (int q = 0; q < 32 / PER; ++q) {
-            const u32x4 raw = reinterpret_cast<const u32x4 *>(src)[q];
-            T part[PER];
-            __builtin_memcpy(part, &raw, 16);
-#pragma unroll
-            for (int e = 0; e < PER; ++e) gt[q * PER + e] = part[e];
-        }
-        codes = tcodes[(int64_t)c * g.n + ns];
+    // Eight kernels of the list at a time: lane 8 h + t looks tap t of kernel h up, so the set bits of the vote are the
+    // (kernel, tap) pairs that read this channel, in the order of the additions.  The pairs go through a ring of kRing
+    // requests; the pairs of the next eight kernels are looked up meanwhile.
+    constexpr int kRing = sizeof(T) == 4 ? 8 : 4;
+    const int slot = lane >> 3, tap = lane & 7;
+    auto entry = [&](int k0) { return k0 + slot < nhits ? hit[k0 + slot] : 0; };
+    auto look_up = [&](int ent) {                                     // kernel, tap, offset in the plane; -1: no such pair
+        const int c = ent & 0xFFFF;
+        const Tap tp = unpack_tap(sel[c * 8 + tap], tap_limit(g));
+        return (ent >> (16 + tap)) & 1 ? (c << 16 | tap << 8 | ls_at(tp.ry, tp.rx)) : -1;
     };
-    T cur[32], nxt[32];
-    uint32_t cur_codes = 0, nxt_codes = 0;
-    if (nhits > 0) fetch(0, cur, cur_codes);
-    for (int k = 0; k < nhits; ++k) {
-        if (k + 1 < nhits) fetch(k + 1, nxt, nxt_codes);              // in flight during the updates of hit k
-        const int ent = hit[k];
-        const int c = ent & 0xFFFF, mask = (ent >> 16) & 0xFF;
-        int pc[4];                                                    // padded position of every cell's maximum
-#pragma unroll
-        for (int cell = 0; cell < 4; ++cell) {
-            const int code = (cur_codes >> (8 * cell)) & 3;
-            pc[cell] = (2 * (cell >> 1) + (code >> 1)) * 6 + 2 * (cell & 1) + (code & 1);
+    int pair = -1, ent_next = 0;
+    if (nhits > 0) {
+        pair = look_up(entry(0));
+        ent_next = entry(8);
+    }
+    for (int k0 = 0; k0 < nhits; k0 += 8) {
+        uint64_t todo = __ballot(pair != -1);
+        const int total = __popcll(todo);
+        const int pair_next = look_up(ent_next);                      // entry() past the list has no tap: -1
+        ent_next = entry(k0 + 16);
+        if (total == 0) {
+            pair = pair_next;
+            continue;
         }
+        T val[kRing][4];
+        uint32_t code[kRing];
+        int off[kRing], last = 0;
+        auto request = [&](int u) {                                   // past the last pair: that pair again
+            if (todo) {
+                last = __builtin_ctzll(todo);
+                todo &= todo - 1;
+            }
+            const uint32_t p = (uint32_t)__builtin_amdgcn_readlane(pair, last);
+            const int c = p >> 16, t = (p >> 8) & 7;
+            off[u] = p & 0xFF;
+            load_cells(val[u], tg + (((int64_t)c * 8 + t) * g.n + ns) * 4);
+            code[u] = tcodes[(int64_t)c * g.n + ns];
+        };
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            if ((mask >> t) & 1) {                                    // wave-uniform: tap t of kernel c reads this channel
-                const Tap tp = unpack_tap(sel[c * 8 + t], tap_limit(g));
-                const int off = tp.ry * 6 + tp.rx;
-                T old[4];
-                // the four cells' targets of one tap are distinct elements; taps are applied one after the other
+        for (int u = 0; u < kRing; ++u) request(u);
+        auto add = [&](int u) {
+            int at[4];
+            T old[4];
+            // the four cells' targets of one tap are distinct elements (or halo, never read); taps are applied one after the other
 #pragma unroll
-                for (int cell = 0; cell < 4; ++cell) old[cell] = plane[pc[cell] + off];
+            for (int cell = 0; cell < 4; ++cell) {
+                const int cd = (code[u] >> (8 * cell)) & 3;
+                at[cell] = ls_at(2 * (cell >> 1) + (cd >> 1), 2 * (cell & 1) + (cd & 1)) + off[u];
+            }
 #pragma unroll
-                for (int cell = 0; cell < 4; ++cell) plane[pc[cell] + off] = old[cell] + cur[cell * 8 + t];
+            for (int cell = 0; cell < 4; ++cell) old[cell] = plane[at[cell]];
+#pragma unroll
+            for (int cell = 0; cell < 4; ++cell) plane[at[cell]] = old[cell] + val[u][cell];
+        };
+        int i = 0;
+        for (; i + kRing < total; i += kRing) {
+#pragma unroll
+            for (int u = 0; u < kRing; ++u) {
+                add(u);
+                request(u);
             }
         }
 #pragma unroll
-        for (int e = 0; e < 32; ++e) cur[e] = nxt[e];
-        cur_codes = nxt_codes;
+        for (int u = 0; u < kRing; ++u)
+            if (i + u < total) add(u);
+        pair = pair_next;
     }
     if (live) {
         T out[16];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) out[e] = plane[((e >> 2) + 1) * 6 + (e & 3) + 1];
+        for (int e = 0; e < 16; ++e) out[e] = plane[ls_at((e >> 2) + 1, (e & 3) + 1)];
         T *dst = gx + (n * g.cin + ch) * 16;
 #pragma unroll
-        for (int q = 0; q < 16 / PER; ++q) {
-            u32x4 raw;
-            __builtin_memcpy(&raw, &out[q * PER], 16);
-            reinterpret_cast<u32x4 *>(dst)[q] = raw;
-        }
+        for (int q = 0; q < 4; ++q) store_cells(dst + 4 * q, &out[4 * q]);
     }
 }
 
@@ -588,7 +671,7 @@ int clg_convblock_eval_packed_4x4(const Geom &g, const uint64_t *x, const uint8_
 }
 
 // ---- gradients: launchers (the caller has run the prepare kernel: folded coefficients and per-channel kernel lists) ----
-// tap gradients [c][n][32] followed by the arg-max codes [c][n] of the same (kernel, sample) pairs
+// tap gradients [c][8][n][4] followed by the arg-max codes [c][n] of the same (kernel, sample) pairs
 static size_t tg_elems_bytes(int dtype, const Geom &g) { return (size_t)g.c * g.n * 32 * (dtype == CLG_F64 ? 8 : 4); }
 size_t clg_convblock_backward_4x4_tg_bytes(int dtype, const Geom &g) { return tg_elems_bytes(dtype, g) + (size_t)g.c * g.n * 4; }
 
@@ -599,10 +682,11 @@ static int launch_backward_4x4(const Geom &g, const void *x, const void *folded,
 {
     int ct = 16;                                                      // kernels per workgroup, at least ~1024 workgroups
     while (ct > 1 && (g.c + ct - 1) / ct < 1024) ct >>= 1;
-    const size_t lds = (size_t)kLsWaves * kWave * kLsStride * sizeof(T);
+    const int sblocks = (g.n + kWave - 1) / kWave, waves = sblocks >= 4 ? 4 : (sblocks >= 2 ? 2 : 1);   // none without samples
+    const size_t lds = (size_t)waves * kWave * kLsStride * sizeof(T);
     if (int e = allow_lds(convblock_backward_4x4_kernel<T>, lds + 1024, name)) return e;
     uint32_t *tcodes = reinterpret_cast<uint32_t *>(reinterpret_cast<unsigned char *>(tg) + tg_elems_bytes(sizeof(T) == 8 ? CLG_F64 : CLG_F32, g));
-    hipLaunchKernelGGL(convblock_backward_4x4_kernel<T>, dim3((unsigned)((g.c + ct - 1) / ct)), dim3(kLsWaves * kWave), lds, st,
+    hipLaunchKernelGGL(convblock_backward_4x4_kernel<T>, dim3((unsigned)((g.c + ct - 1) / ct)), dim3(waves * kWave), lds, st,
                        (const T *)x, (const T *)folded, sel, (const T *)gy, argmax, gx != nullptr ? (T *)tg : (T *)nullptr, tcodes, (T *)gw,
                        (const T *)probs, g, ct);
     CLG_CHECK_LAUNCH(name);

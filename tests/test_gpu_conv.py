@@ -412,6 +412,24 @@ def test_block_4x4_one_sample_per_lane_gradients(n, cin, cout, dtype, monkeypatc
                 assert (a - b).abs().max().item() <= tol * scale, key
 
 
+@pytest.mark.parametrize("n,cin,cout", [(33, 2, 70), (64, 1, 9), (65, 5, 41), (193, 3, 24), (256, 9, 33)])
+def test_block_4x4_input_gradient_over_long_kernel_lists(n, cin, cout, monkeypatch):
+    # the per-channel pass takes its list eight kernels at a time and the taps of those through a ring of requests: lists of
+    # 8 and fewer, just above 8 and of many rounds, 1, 2 and 4 wavefronts of samples and ragged ones.  Taps are added in the
+    # order of the staged kernels; their tree gradients differ in rounding (2e-5 of the largest sum, as above).
+    torch.manual_seed(n + cin)
+    x = torch.rand(n, cin, 4, 4, device=DEV)
+    layer = C.ConvLogicLayer(cin, cout, padding=1, complete=True, implementation="cuda").to(DEV)
+    wp = torch.softmax(layer.weights.detach(), -1)
+    y, am = convlogic_hip.full_convlogic_forward(x, wp, layer.selection, 1, 1, 1, 1, 3, 3)
+    gy = torch.randn_like(y)
+    got = convlogic_hip.full_convlogic_backward(gy, x, wp, am, layer.selection, 1, 1, 1, 1)
+    set_knobs(monkeypatch, CLG_BWD_4X4="0")
+    want = convlogic_hip.full_convlogic_backward(gy, x, wp, am, layer.selection, 1, 1, 1, 1)
+    for a, b in zip(got, want):
+        assert (a - b).abs().max().item() <= 2e-5 * b.abs().max().item()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("n,cin,cout", [(32, 3, 5), (100, 24, 48), (130, 40, 17)])
 def test_block_4x4_feature_major_output(n, cin, cout, dtype):
