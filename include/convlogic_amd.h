@@ -278,6 +278,13 @@ int clg_fc_eval_packed_planned_logits(int elem_size, const void *x /*[in_dim,wor
                                       const float *logits /*[out_dim,16]*/, const int32_t *plan /*[out_dim]*/,
                                       void *y /*[out_dim,words]*/, int64_t in_dim, int64_t out_dim, int64_t words, void *stream);
 
+/* clg_gate_argmax + clg_fc_eval_packed in ONE launch, for rows the walk kernel does not take: the same gate ids from the 16
+ * float32 logits of a neuron.  Rows must be whole 4-byte words at 4-byte aligned addresses (CLG_EINVAL otherwise; use the
+ * two calls then).  Replaces the same lines of LogicLayer.forward_cuda_eval as clg_fc_eval_packed_planned_logits. */
+int clg_fc_eval_packed_logits(int elem_size, const void *x /*[in_dim,words]*/, const int64_t *a, const int64_t *b,
+                              const float *logits /*[out_dim,16]*/, void *y /*[out_dim,words]*/, int64_t in_dim, int64_t out_dim,
+                              int64_t words, void *stream);
+
 /* out[s][g] = number of features of class g (features/k consecutive rows) whose sample-s bit is set,
  * for s < words*8*elem_size - pad_len.  features must be divisible by k.
  * Replaces difflogic_cuda.groupbitsum -- src/difflogic/cuda/difflogic.cpp:22-33,

@@ -224,6 +224,25 @@ def test_eval_planned_logits_entry_point_rejects_rows_the_walk_kernel_does_not_t
     assert rc != 0 and b"clg_fc_eval_walk_fits" in lib.clg_last_error()
 
 
+@pytest.mark.parametrize("words,bits", [(1, 32), (63, 32), (129, 32), (313, 32), (1025, 32), (2, 64), (9, 64), (65, 64), (5, 16),
+                                        (6, 16), (3, 8), (12, 8)])
+def test_eval_from_logits_on_short_and_odd_rows(words, bits):
+    # one launch for rows of whole 4-byte words (4-, 8- and 16-byte vectors), the two-launch route for the others
+    in_dim, out_dim = 37, 51
+    rng = np.random.default_rng(words)
+    torch.manual_seed(words)
+    info = np.iinfo(O.NP_WORD[bits])
+    x = rng.integers(info.min, info.max, (in_dim, words), dtype=O.NP_WORD[bits])
+    idx0, idx1 = torch.randint(0, in_dim, (out_dim,)), torch.randint(0, in_dim, (out_dim,))
+    logits = torch.randn(out_dim, 16)
+    logits[0], logits[1, 4], logits[1, 9] = 0.0, 9.0, 9.0
+    logits[2, 3], logits[2, 7] = float("inf"), float("nan")
+    xd, a, b = torch.from_numpy(x).to(DEV), idx0.to(DEV), idx1.to(DEV)
+    got = difflogic_hip.eval_planned_logits(xd, a, b, logits.to(DEV), difflogic_hip.eval_plan(a, b, in_dim))
+    want = O.eval_packed(x, idx0.numpy(), idx1.numpy(), logits.argmax(-1).numpy().astype(np.uint8))
+    assert np.array_equal(got.cpu().numpy(), want)
+
+
 def test_eval_plan_follows_in_place_rewiring():
     torch.manual_seed(4)
     layer = C.LogicLayer(40, 60, implementation="cuda").to(DEV).eval()
