@@ -91,7 +91,7 @@ __global__ __launch_bounds__(256) void convblock_prepare_kernel(const T *__restr
                                                               TapLimit lim)
 {
     if ((int)blockIdx.x >= pad_block0) {                            // tail of the launch: the padded copy of x
-        pad_image_elem(pad, (int64_t)(blockIdx.x - pad_block0) * 256 + threadIdx.x);
+        pad_image_elems(pad, blockIdx.x - pad_block0);
         return;
     }
     if ((int)blockIdx.x < fold_blocks) {

@@ -217,6 +217,31 @@ def test_block_deep_and_wide_shapes_vs_oracle(shape, dtype):
     assert_grad_close(layer.weights.grad, ll.grad, name="grad_logits")
 
 
+@pytest.mark.parametrize("n,cin,cout,h,w,pad,kernel", [(1, 1, 4, 2, 2, 1, 3), (3, 2, 5, 4, 6, (0, 1), 3), (5, 3, 9, 8, 10, (1, 0), 3),
+                                                      (2, 5, 6, 12, 6, 1, 3), (7, 3, 8, 10, 14, 0, 3), (3, 3, 7, 5, 7, 0, 2)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_padded_copy_of_odd_images(n, cin, cout, h, w, pad, kernel, dtype, monkeypatch):
+    # the kernels that read the zero-padded copy: samples, planes and rows that end inside a thread's four elements
+    stride, pad, kernel = (1, 1), pad if isinstance(pad, tuple) else (pad, pad), (kernel, kernel)
+    torch.manual_seed(h * w)
+    layer = C.ConvLogicLayer(cin, cout, stride=stride, padding=pad, kernel=kernel, complete=True, implementation="cuda").to(DEV, dtype)
+    x = torch.rand(n, cin, h, w, device=DEV, dtype=dtype)
+    results = []
+    for direct in ("1", "0"):
+        set_knobs(monkeypatch, CLG_FWD_DIRECT=direct, CLG_BWDX_DIRECT=direct)
+        xd = x.clone().requires_grad_(True)
+        layer.weights.grad = None
+        y = layer(xd)
+        y.backward(torch.cos(torch.arange(y.numel(), device=DEV, dtype=dtype)).view_as(y))
+        results.append((y.detach(), xd.grad, layer.weights.grad))
+    set_knobs(monkeypatch, CLG_FWD_DIRECT=None, CLG_BWDX_DIRECT=None)
+    (y1, gx1, gw1), (y0, gx0, gw0) = results
+    # at most a few hundred terms per sum: their order changes a sum by that many rounding errors at most
+    tol = 512 * torch.finfo(dtype).eps
+    assert torch.equal(y1, y0)
+    assert torch.allclose(gx1, gx0, rtol=tol, atol=tol) and torch.allclose(gw1, gw0, rtol=tol, atol=tol)
+
+
 def test_block_config4_full_size_properties():
     # BASELINE config 4 at full size: determinism (bitwise) and linearity of the backward in grad_y
     torch.manual_seed(5)
