@@ -370,16 +370,12 @@ class ConvLogicLayer(nn.Module):
             raise RuntimeError("packed evaluation needs implementation='cuda'")
         assert x.image and x.t.dim() == 4 and x.t.shape[1] == self.in_channels, (x.image, tuple(x.t.shape), self.in_channels)
         self._check_selection()
-        x.t = convlogic_hip.full_convlogic_eval_packed(x.t.contiguous(), self._eval_gates(), self.selection.contiguous(),
-                                                       *self.stride, *self.padding, *self.kernel,
-                                                       feature_major=getattr(self, "feature_major_output", False))
+        # gate ids = arg-max of the logits, taken on every call: nothing cached that an in-place update of `weights.data`
+        # could leave stale
+        x.t = convlogic_hip.full_convlogic_eval_packed_logits(x.t.contiguous(), self.weights.detach().contiguous(), self.selection.contiguous(),
+                                                              (*self.stride, *self.padding, *self.kernel),
+                                                              feature_major=getattr(self, "feature_major_output", False))
         return x
-
-    def _eval_gates(self):
-        """uint8 [C, 7] arg-max gate ids, taken from the logits on every call (one small launch; nothing cached that an
-        in-place update of `weights.data` could leave stale)."""
-        from ..hip import difflogic_hip
-        return difflogic_hip.gate_argmax(self.weights.detach().contiguous())
 
     def extra_repr(self):
         return f"in_channels={self.in_channels}, out_channels={self.out_channels}, groups={self.groups}"

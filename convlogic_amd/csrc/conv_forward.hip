@@ -1035,3 +1035,28 @@ extern "C" int clg_convblock_eval_packed_ws(const clg_conv_geom *gg, const uint6
     return launch_forward_direct<BitOps, float>(g, dp, x, gates, selection, y, nullptr, scratch, clg_stream(stream),
                                                 "clg_convblock_eval_packed_ws");
 }
+
+// The packed block from the logits: the scratch starts with the gate ids [c_out, 7], what the evaluation itself needs follows.
+static size_t packed_gates_bytes(const Geom &g) { return ((size_t)g.c * 7 + 255) & ~(size_t)255; }
+
+extern "C" int64_t clg_convblock_eval_packed_logits_scratch_bytes(const clg_conv_geom *gg)
+{
+    Geom g;
+    if (clg_convblock_check(gg, &g, CLG_F64, "clg_convblock_eval_packed_logits_scratch_bytes")) return -1;
+    const int64_t eval = clg_convblock_eval_packed_scratch_bytes(gg);
+    return eval < 0 ? eval : (int64_t)packed_gates_bytes(g) + eval;
+}
+
+extern "C" int clg_convblock_eval_packed_logits(int dtype, const clg_conv_geom *gg, const uint64_t *x, const void *logits,
+                                                const int32_t *selection, uint64_t *y, int feature_major, void *scratch, void *stream)
+{
+    const char *name = "clg_convblock_eval_packed_logits";
+    Geom g;
+    if (int e = clg_convblock_check(gg, &g, CLG_F64, name)) return e;
+    CLG_REQUIRE(x && logits && selection && y && scratch, "%s: null pointer argument", name);
+    CLG_REQUIRE(x != y, "%s: x and y must not overlap", name);
+    uint8_t *gates = reinterpret_cast<uint8_t *>(scratch);
+    if (int e = clg_gate_argmax(dtype, logits, gates, (int64_t)g.c * 7, stream)) return e;
+    if (feature_major) return clg_convblock_eval_packed_fm(gg, x, gates, selection, y, stream);
+    return clg_convblock_eval_packed_ws(gg, x, gates, selection, y, gates + packed_gates_bytes(g), stream);
+}

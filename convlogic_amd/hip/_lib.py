@@ -94,6 +94,8 @@ SIGNATURES = {
     "clg_convblock_forward_padded": (_i, [_i, _GP, _p, _p, _p, _p, _p, _p, _i, _p, _p, _p]),
     "clg_convblock_eval_packed_fm_supported": (_i, [_GP]),
     "clg_convblock_eval_packed_fm": (_i, [_GP, _p, _p, _p, _p, _p]),
+    "clg_convblock_eval_packed_logits_scratch_bytes": (_i64, [_GP]),
+    "clg_convblock_eval_packed_logits": (_i, [_i, _GP, _p, _p, _p, _p, _i, _p, _p]),
     "clg_convblock_forward_fm": (_i, [_i, _GP, _p, _p, _p, _p, _p, _p, _p]),
     "clg_convblock_backward_fm": (_i, [_i, _GP, _p, _p, _p, _p, _p, _p, _p, _i, _p, _p]),
     "clg_convblock_backward_scratch_bytes": (_i64, [_i, _GP]),

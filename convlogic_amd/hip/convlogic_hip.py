@@ -207,6 +207,31 @@ def full_convlogic_eval_packed(x, gates, selection, stride_h, stride_w, pad_h, p
     return y
 
 
+def full_convlogic_eval_packed_logits(x, logits, selection, geo, feature_major=False):
+    """full_convlogic_eval_packed(x, gate_argmax(logits), selection, *geo, feature_major) in one call; logits float [C, 7, 16],
+    contiguous.  (Python spends 7 us on the separate arg-max call, of 43 us per block of a request of 256 images.)"""
+    check_input(x, "x")
+    check_input(logits, "weights")
+    if x.dtype != torch.int64 or x.dim() != 4:
+        raise RuntimeError("full_convlogic_eval_packed expects int64 words [G, C, H, W] and uint8 gate ids [C, 7]")
+    c = logits.shape[0] if logits.dim() else -1
+    if tuple(logits.shape) != (c, 7, 16):
+        raise RuntimeError(f"full_convlogic_eval_packed expects logits of shape [C, 7, 16], got {tuple(logits.shape)}")
+    _selection_arg(x, selection, c)
+    _lib.check_same_device(x, logits)
+    dt = dtype_code(logits, half_ok=True)
+    g = _geom(x, c, *geo)
+    ho, wo = _out_size(g)
+    lib, ref = _lib.load(), ctypes.byref(g)
+    fm = bool(feature_major and lib.clg_convblock_eval_packed_fm_supported(ref))
+    shape = (c, ho // 2, wo // 2, g.n) if fm else (g.n, c, max(ho, 0) // 2, max(wo, 0) // 2)
+    y = torch.empty(shape, dtype=torch.int64, device=x.device)
+    scratch = _scratch(lib.clg_convblock_eval_packed_logits_scratch_bytes(ref), x.device)
+    check(lib.clg_convblock_eval_packed_logits(dt, ref, x.data_ptr(), logits.data_ptr(), selection.data_ptr(), y.data_ptr(), int(fm),
+                                               scratch.data_ptr(), stream_ptr(x)))
+    return y.permute(3, 0, 1, 2) if fm else y
+
+
 def full_convlogic_intermediates(x, weight, selection, stride_h, stride_w, pad_h, pad_w, kernel_h, kernel_w):
     """-> (x2 [N,C,Ho,Wo,4], x3 [N,C,Ho,Wo,2]), the second and third result of the reference's
     full_convlogic_forward (full_convlogic_kernel.cu:172,194)."""

@@ -440,6 +440,11 @@ int clg_convblock_forward_ex(int dtype, const clg_conv_geom *g, const void *x, c
 int clg_convblock_eval_packed_fm_supported(const clg_conv_geom *g);
 int clg_convblock_eval_packed_fm(const clg_conv_geom *g, const uint64_t *x, const uint8_t *gates, const int32_t *selection,
                                  uint64_t *y /*[c_out,ho/2,wo/2,groups]*/, void *stream);
+/* clg_gate_argmax on logits [c_out, 7, 16] (dtype as there), then clg_convblock_eval_packed_ws, or with feature_major != 0
+ * clg_convblock_eval_packed_fm: one call, the gate ids in the scratch. */
+int64_t clg_convblock_eval_packed_logits_scratch_bytes(const clg_conv_geom *g);
+int clg_convblock_eval_packed_logits(int dtype, const clg_conv_geom *g, const uint64_t *x, const void *logits, const int32_t *selection,
+                                     uint64_t *y, int feature_major, void *scratch, void *stream);
 int clg_convblock_forward_fm(int dtype, const clg_conv_geom *g, const void *x, const void *w, const int32_t *selection,
                              void *y /*[c_out,ho/2,wo/2,n]*/, uint8_t *argmax, void *scratch, void *stream);
 int clg_convblock_backward_fm(int dtype, const clg_conv_geom *g, const void *grad_y /*[c_out,ho/2,wo/2,n]*/, const void *x,
