@@ -1060,7 +1060,15 @@ BwdXMode choose_backward_x(const Geom &g, int elem, TilePlan *p, int *sample_ele
     // when there are thousands of such owners with short kernel lists (48 vs 88 us at [256,32,16,16] -> 128,
     // 74 vs 164 us at [256,64,16,16] -> 256; few channels with long lists stay tiled: 141 vs 248 us at C4).
     const int64_t owners = clg_ceil_div(g.n, pd.G) * g.cin, avg_hits = (2 * (int64_t)g.c) / g.cin;
-    bool use_direct = direct && (!tiled || lanes(pd) >= 2 * lanes(pt) || (owners >= 4096 && avg_hits <= 16));
+    // float32, by the chain of cell blocks that an owner walks (hits x blocks of 64 cells; the tiled kernel's wavefronts take
+    // several channels each, and a small batch leaves most CUs without a workgroup).  Whole block, forward + backward, tiled ->
+    // direct: chains up to 16 from 4 channels on 1.0 to 3.6 times faster, however few owners ([100,32,12,12] -> 96: 100 -> 56 us,
+    // [16,32,8,8] -> 16: 83 -> 23, [2,64,8,8] -> 256: 128 -> 36); up to 32 from 16 channels on, where no wavefronts share a
+    // plane ([64,16,8,8] -> 256 87 -> 61, at 8 channels 86 -> 95); up to 64 from 2048 owners on (178 -> 161 at
+    // [64,32,28,28] -> 256, but 102 -> 123 at half its channels); longer chains are the tiled kernel's ([16,32,28,28] -> 512: 139 -> 215).
+    const int64_t chain = avg_hits * clg_ceil_div((int64_t)pd.G * I, kWave);
+    const bool short_chain = elem == 4 && g.cin >= 4 && (chain <= 16 || (g.cin >= 16 && ((chain <= 32 && owners >= 64) || (chain <= 64 && owners >= 2048))));
+    bool use_direct = direct && (!tiled || lanes(pd) >= 2 * lanes(pt) || (owners >= 4096 && avg_hits <= 16) || short_chain);
     if (const char *e = clg_knob(K_BWDX_DIRECT)) use_direct = direct && (atoi(e) != 0 || !tiled);
     if (use_direct) {
         *p = pd;

@@ -242,6 +242,30 @@ def test_padded_copy_of_odd_images(n, cin, cout, h, w, pad, kernel, dtype, monke
     assert torch.allclose(gx1, gx0, rtol=tol, atol=tol) and torch.allclose(gw1, gw0, rtol=tol, atol=tol)
 
 
+@pytest.mark.parametrize("n,cin,cout,side", [(2, 4, 32, 8), (2, 4, 34, 8), (2, 3, 16, 8), (1, 16, 16, 2), (16, 16, 256, 8), (12, 16, 256, 8),
+                                             (9, 32, 96, 12), (3, 5, 8, 20)])
+def test_input_gradient_on_both_sides_of_the_kernel_choice(n, cin, cout, side, monkeypatch):
+    # float32: short chains of cell blocks take the kernel with one wavefront per channel, longer ones the staged one; both
+    # add an element's terms in the order of the kernels that read it
+    torch.manual_seed(n * cout)
+    layer = C.ConvLogicLayer(cin, cout, kernel=3, padding=1, complete=True, implementation="cuda").to(DEV)
+    x = torch.rand(n, cin, side, side, device=DEV)
+    grads = []
+    for direct in (None, "1", "0"):
+        set_knobs(monkeypatch, CLG_BWDX_DIRECT=direct)
+        xd = x.clone().requires_grad_(True)
+        layer.weights.grad = None
+        y = layer(xd)
+        y.backward(torch.cos(torch.arange(y.numel(), device=DEV, dtype=torch.float32)).view_as(y))
+        grads.append((xd.grad, layer.weights.grad))
+    set_knobs(monkeypatch, CLG_BWDX_DIRECT=None)
+    # terms of one input element: at most 9 taps of each of its kernels; of one logit: one per pooled cell
+    eps = torch.finfo(torch.float32).eps
+    for gx, gw in grads[1:]:
+        assert torch.allclose(grads[0][0], gx, rtol=9 * cout * eps, atol=9 * cout * eps)
+        assert torch.allclose(grads[0][1], gw, rtol=n * side * side * eps, atol=n * side * side * eps)
+
+
 def test_block_config4_full_size_properties():
     # BASELINE config 4 at full size: determinism (bitwise) and linearity of the backward in grad_y
     torch.manual_seed(5)
