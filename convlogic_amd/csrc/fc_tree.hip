@@ -76,10 +76,14 @@ __device__ __forceinline__ float swap_add16(float a, float b)
 struct TreeLogits {
     const float *l[3];
 };
-__device__ __forceinline__ int64_t tree_neuron(const int32_t *__restrict__ ids, int j, int q) { return q < 6 ? ids[(int64_t)j * 8 + q] : j; }
-__device__ __forceinline__ const float *tree_logits(const TreeLogits &lg, const int32_t *__restrict__ ids, int j, int q)
+// (A bad id names a wrong neuron; it never leaves the logits or the probabilities, which are written at the same place.)
+__device__ __forceinline__ int64_t tree_neuron(const int32_t *__restrict__ ids, int j, int q, int roots)
 {
-    return (q < 4 ? lg.l[0] : (q < 6 ? lg.l[1] : lg.l[2])) + tree_neuron(ids, j, q) * 16;
+    return q < 6 ? min((uint32_t)ids[(int64_t)j * 8 + q], (q < 4 ? 4u : 2u) * (uint32_t)roots - 1u) : (uint32_t)j;
+}
+__device__ __forceinline__ const float *tree_logits(const TreeLogits &lg, const int32_t *__restrict__ ids, int j, int q, int roots)
+{
+    return (q < 4 ? lg.l[0] : (q < 6 ? lg.l[1] : lg.l[2])) + tree_neuron(ids, j, q, roots) * 16;
 }
 // index of the first maximum (a NaN counts as the maximum), as clg_gate_argmax
 __device__ __forceinline__ int argmax16(const float *__restrict__ w)
@@ -101,7 +105,7 @@ __global__ __launch_bounds__(256) void fc_tree_fold_kernel(TreeLogits lg, const 
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (e >= (int64_t)roots * 7) return;
     const int j = (int)(e / 7), q = (int)(e - (int64_t)j * 7);
-    const float *w = tree_logits(lg, ids, j, q);
+    const float *w = tree_logits(lg, ids, j, q, roots);
     float p[16];
     if (hard) {
         const int at = argmax16(w);
@@ -111,7 +115,7 @@ __global__ __launch_bounds__(256) void fc_tree_fold_kernel(TreeLogits lg, const 
         softmax16(w, p);
     }
     if (probs) {
-        float4 *dst = reinterpret_cast<float4 *>(probs + (tree_neuron(ids, j, q) + (int64_t)roots * (q < 4 ? 0 : (q < 6 ? 4 : 6))) * 16);
+        float4 *dst = reinterpret_cast<float4 *>(probs + (tree_neuron(ids, j, q, roots) + (int64_t)roots * (q < 4 ? 0 : (q < 6 ? 4 : 6))) * 16);
 #pragma unroll
         for (int i = 0; i < 4; ++i) dst[i] = make_float4(p[4 * i], p[4 * i + 1], p[4 * i + 2], p[4 * i + 3]);
     }
@@ -504,7 +508,7 @@ __global__ __launch_bounds__(256) void fc_tree_codes_kernel(TreeLogits lg, const
     for (int64_t i = e; i < n_counts; i += (int64_t)gridDim.x * 256) counts[i] = 0;   // (for the counting kernel's atomics)
     const int j = (int)(e >> 3), q = (int)(e & 7);                    // eight lanes per root, one gate each
     int id = 0;
-    if (j < roots && q < 7) id = argmax16(tree_logits(lg, ids, j, q));
+    if (j < roots && q < 7) id = argmax16(tree_logits(lg, ids, j, q, roots));
     uint8_t gate[7];
 #pragma unroll
     for (int t = 0; t < 7; ++t) gate[t] = (uint8_t)__shfl(id, (threadIdx.x & 56) + t, kWave);

@@ -519,6 +519,7 @@ int clg_host_flag_device_pointer(void *host, void **device);
  *   slot [7 roots]   of every neuron, first layer first: root * 7 + its place among the tree's gates
  *   logits0..2       the layers' logits [out, 16]         coef [roots, 7, 4] folded coefficients in tree order
  * x is feature-major with a row pitch >= batch (lanes are 1, 2 or 4 samples wide, whatever pitch and addresses allow).
+ * An entry of rows, ids, pos or slot out of range is taken as the last one: a wrong result, no access outside the buffers.
  * ------------------------------------------------------------------------------- */
 /* coef of the softmax (hard = 0) or the arg-max gates (hard = 1); probs [7 roots, 16] takes the probabilities, neurons of the first
  * layer first (may be NULL) */

@@ -186,3 +186,23 @@ def test_onehot_of_the_first_maximum(dtype):
     got = difflogic_hip.gate_onehot(logits, dtype)
     assert got.dtype == dtype and torch.equal(got, torch.nn.functional.one_hot(logits.argmax(-1), 16).to(dtype))
     assert torch.equal(got.argmax(-1).to(torch.uint8), difflogic_hip.gate_argmax(logits))
+
+
+@pytest.mark.parametrize("hard", [0, 1])
+def test_ids_out_of_range_stay_inside_the_logits_and_the_probabilities(hard):
+    from convlogic_amd.hip import _lib
+    roots = 70
+    logits = [torch.randn(n * roots, 16, device=DEV) for n in (4, 2, 1)]
+    ids = torch.stack([torch.randint(0, (4 if q < 4 else 2) * roots, (roots,), dtype=torch.int32) for q in range(8)], 1)
+    ids[3, 1], ids[5, 4], ids[9, 0], ids[11, 5] = 4 * roots, 2 * roots, -1, -2**31
+    inside = torch.stack([ids[:, q].long().where((ids[:, q] >= 0) & (ids[:, q] < n * roots), torch.tensor(n * roots - 1))
+                          for q, n in enumerate((4, 4, 4, 4, 2, 2))], 1).to(DEV)
+    coef = torch.empty(roots, 7, 4, device=DEV)
+    probs = torch.full((7 * roots + 64, 16), 7.0, device=DEV)             # (the rows behind the last one stay as they are)
+    on_device = ids.to(DEV)
+    _lib.check(_lib.load().clg_fc_tree_fold(*(l.data_ptr() for l in logits), on_device.data_ptr(), coef.data_ptr(), probs.data_ptr(), roots,
+                                            hard, _lib.stream_ptr(coef)))
+    tree = torch.cat([logits[0][inside[:, :4]], logits[1][inside[:, 4:]], logits[2][:, None]], 1).cpu().double()      # [roots, 7, 16]
+    want = O.fold_coefficients(torch.nn.functional.one_hot(tree.argmax(-1), 16).double() if hard else torch.softmax(tree, -1))
+    # a coefficient is a sum of at most 16 probabilities times 1 or 2, each a few roundings off
+    assert (coef.cpu().double() - want).abs().max() <= 1e-5 and (probs[7 * roots:] == 7).all()
