@@ -74,7 +74,8 @@ def _tree_tail(net):
         return None
     for m in layers:
         w = m._parameters["weights"]
-        if not (w.is_cuda and w.dtype == torch.float32 and w.is_contiguous() and w.device == layers[0]._parameters["weights"].device):
+        if not (w.is_cuda and w.dtype == torch.float32 and w.shape == (m.out_dim, 16) and w.is_contiguous()
+                and w.device == layers[0]._parameters["weights"].device):
             return None
     return layers, gs
 

@@ -206,3 +206,15 @@ def test_ids_out_of_range_stay_inside_the_logits_and_the_probabilities(hard):
     want = O.fold_coefficients(torch.nn.functional.one_hot(tree.argmax(-1), 16).double() if hard else torch.softmax(tree, -1))
     # a coefficient is a sum of at most 16 probabilities times 1 or 2, each a few roundings off
     assert (coef.cpu().double() - want).abs().max() <= 1e-5 and (probs[7 * roots:] == 7).all()
+
+
+@pytest.mark.parametrize("at", [4, 5, 6])
+def test_logits_of_another_size_are_refused(at):
+    torch.manual_seed(6)
+    model = C.ConvLogicMnistModel(k_param=2).to(DEV).eval()
+    layer = model.network[at]
+    layer.weights = torch.nn.Parameter(layer.weights.detach()[:-1].clone())
+    with torch.no_grad(), pytest.raises(RuntimeError, match="shape|logits|neurons"):
+        model(torch.zeros(8, 1, 28, 28, device=DEV))
+    with torch.no_grad(), pytest.raises(RuntimeError, match="shape|logits|neurons"):
+        model(C.PackBitsTensor(torch.zeros(8, 1, 28, 28, dtype=torch.bool, device=DEV), 64))
