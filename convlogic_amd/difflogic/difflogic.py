@@ -6,12 +6,19 @@ implementation="cuda" runs the HIP kernels (on ROCm builds of torch the device t
 reference's second, explicitly selected backend: plain torch ops on whatever device the tensors
 live on.
 """
+import weakref
+
 import numpy as np
 import torch
 
 from ..hip import difflogic_hip
 from .functional import GradFactor, bin_op_s, get_unique_connections
 from .packbitstensor import PackBitsTensor
+
+# per layer: the wiring buffers its last check was of.  While these live no other buffer can have their addresses, so a wiring
+# key (versions and addresses) that is equal to the checked one is of the checked wiring.  Outside the modules: copies and
+# pickles carry no buffers of an earlier device.
+_CHECKED_BUFFERS = weakref.WeakKeyDictionary()
 
 
 def _reverse_wiring(idx0, idx1, in_dim):
@@ -93,8 +100,7 @@ class LogicLayer(torch.nn.Module):
             assert x.is_cuda, f"x must be a CUDA tensor, got device: {x.device}"
         assert x.ndim == 2, x.ndim
         assert x.shape[1] == self.in_dim, (tuple(x.shape[::-1]), self.in_dim)
-        key = self._wiring_key()
-        self._check_wiring(key)
+        key = self._check_wiring()
         weights, buffers = self._parameters["weights"], self._buffers
         if (self.training and weights.dtype == x.dtype and x.dtype in (torch.float32, torch.float64)
                 and weights.is_contiguous() and weights.device == x.device):
@@ -149,15 +155,25 @@ class LogicLayer(torch.nn.Module):
         # (buffers and parameters straight from their dicts: nn.Module.__getattr__ costs a microsecond per lookup, and
         # this key is taken on every call)
         a, b = self._buffers["indices_0"], self._buffers["indices_1"]
-        return (a._version, b._version, a.data_ptr(), b.data_ptr(), self._parameters["weights"].device)
+        return (a._version, b._version, a.data_ptr(), b.data_ptr(), self._parameters["weights"].device, self.__dict__.get("_wiring_epoch", 0))
 
-    def _check_wiring(self, key=None):
-        """The kernels index x with indices_0 / indices_1 without bounds checks: an index outside [0, in_dim) must
+    def __getstate__(self):                                          # a copy's buffers are its own: checked for themselves
+        state = self.__dict__.copy()
+        state.pop("_wiring_checked", None)
+        return state
+
+    def _new_wiring_epoch(self):
+        """No key taken before is equal to one taken after: whatever was derived from the wiring is derived again."""
+        self.__dict__["_wiring_epoch"] = self.__dict__.get("_wiring_epoch", 0) + 1
+
+    def _check_wiring(self):
+        """Returns the key of the wiring, which what is derived from it (here and in fc_tree) is kept under.  The kernels index x with indices_0 / indices_1 without bounds checks: an index outside [0, in_dim) must
         raise here instead of faulting the GPU.  Checked on the first launch and again whenever the buffers were
         modified in place (version counter) or replaced; writes through `.data` bypass the counter -- call
         invalidate() after those."""
-        key = key or self._wiring_key()
+        key = self._wiring_key()
         if self.__dict__.get("_wiring_checked") != key:
+            self._new_wiring_epoch()
             for name, idx in (("indices_0", self.indices_0), ("indices_1", self.indices_1)):
                 if idx.dtype != torch.int64 or tuple(idx.shape) != (self.out_dim,):
                     raise ValueError(f"{name} must be int64 [{self.out_dim}], got {idx.dtype} {tuple(idx.shape)}")
@@ -181,12 +197,25 @@ class LogicLayer(torch.nn.Module):
                         self.given_x_indices_of_y_start.copy_(start)
                         self.given_x_indices_of_y.copy_(flat)
                     self._reverse_built = built
-            self._wiring_checked = key
+            _CHECKED_BUFFERS[self] = (self._buffers["indices_0"], self._buffers["indices_1"])
+            self._wiring_checked = key = self._wiring_key()
+        return key
 
     def invalidate(self):
-        """Drops everything derived from the wiring buffers (range check, consumer analysis, packed walk plan, reverse map).  Needed only after writing indices_0 / indices_1 through `.data`, which the version
-        counters do not see."""
+        """Drops everything derived from the wiring buffers (range check, consumer analysis, packed walk plan, reverse map, the
+        trees of three layers that this one belongs to).  Needed only after writing indices_0 / indices_1 through `.data`, which
+        the version counters do not see."""
         self._wiring_checked = self._sole_cache = self._plan_cache = self._reverse_built = None
+        self._new_wiring_epoch()
+        _CHECKED_BUFFERS.pop(self, None)
+
+    def _apply(self, fn, *args, **kwargs):
+        a, b = self._buffers["indices_0"], self._buffers["indices_1"]
+        super()._apply(fn, *args, **kwargs)
+        if self._buffers["indices_0"] is not a or self._buffers["indices_1"] is not b:   # moved to another device
+            self._new_wiring_epoch()
+            _CHECKED_BUFFERS.pop(self, None)
+        return self
 
     def _load_from_state_dict(self, *args, **kwargs):
         super()._load_from_state_dict(*args, **kwargs)
@@ -198,7 +227,7 @@ class LogicLayer(torch.nn.Module):
         wiring buffers were modified in place or moved."""
         if 2 * self.out_dim != self.in_dim:
             return False
-        key = key or self._wiring_key()
+        key = key or self._check_wiring()
         cached = self.__dict__.get("_sole_cache")
         if cached is None or cached[0] != key:
             uses = torch.bincount(torch.cat([self.indices_0, self.indices_1]), minlength=self.in_dim)
@@ -209,8 +238,7 @@ class LogicLayer(torch.nn.Module):
     def _eval_plan(self):
         """Walk order of the wiring graph for the packed evaluation kernel; rebuilt when the wiring
         buffers were modified in place or moved to another device."""
-        self._check_wiring()
-        key = self._wiring_key()
+        key = self._check_wiring()
         cached = getattr(self, "_plan_cache", None)
         if cached is None or cached[0] != key:
             cached = (key, difflogic_hip.eval_plan(self.indices_0, self.indices_1, self.in_dim))
@@ -420,8 +448,7 @@ def logic_layer_group_sum(layer, group_sum, x):
             and layer.grad_factor == 1.0 and weights.dtype == x.dtype and x.dtype in (torch.float32, torch.float64)
             and weights.is_contiguous() and weights.device == x.device and layer.out_dim % group_sum.k == 0 and x.shape[0] > 0
             and group_sum.tau != 0 and not _has_forward_hooks(layer) and not _has_forward_hooks(group_sum)):
-        key = layer._wiring_key()
-        layer._check_wiring(key)
+        key = layer._check_wiring()
         if layer._sole_consumers(key):
             buffers = layer._buffers
             return _LogicLayerGroupSumFunction.apply(_feature_major(x), buffers["indices_0"], buffers["indices_1"], weights,

@@ -9,7 +9,8 @@ import torch
 from ..hip import _lib
 from ..hip._lib import check, stream_ptr
 
-# per first layer: (key, wiring plan); kept outside the modules so that copies and pickles carry no derived buffers
+# per first layer: (keys of the three wirings, weak references to the other two layers, plan); kept outside the modules so that
+# copies and pickles carry no derived buffers
 _PLANS = weakref.WeakKeyDictionary()
 
 
@@ -42,17 +43,15 @@ class TreePlan:
 
 def tree_plan(first, second, third):
     """The TreePlan of three LogicLayers, or None when their wiring does not make trees.  Rebuilt when a wiring buffer was
-    modified in place, replaced or moved."""
+    modified in place, replaced or moved, when invalidate() was called on one of the layers, and for other layers."""
     if 2 * second.out_dim != second.in_dim or 2 * third.out_dim != third.in_dim or second.in_dim != first.out_dim or third.in_dim != second.out_dim:
         return None
-    keys = (first._wiring_key(), second._wiring_key(), third._wiring_key())
-    for layer, key in zip((first, second, third), keys):
-        layer._check_wiring(key)
+    keys = (first._check_wiring(), second._check_wiring(), third._check_wiring())
     cached = _PLANS.get(first)
-    if cached is None or cached[0] != keys:
+    if cached is None or cached[0] != keys or cached[1]() is not second or cached[2]() is not third:
         fits = second._sole_consumers(keys[1]) and third._sole_consumers(keys[2])
-        cached = _PLANS[first] = (keys, TreePlan(first, second, third) if fits else None)
-    return cached[1]
+        cached = _PLANS[first] = (keys, weakref.ref(second), weakref.ref(third), TreePlan(first, second, third) if fits else None)
+    return cached[3]
 
 
 class _TreeFunction(torch.autograd.Function):

@@ -218,3 +218,42 @@ def test_logits_of_another_size_are_refused(at):
         model(torch.zeros(8, 1, 28, 28, device=DEV))
     with torch.no_grad(), pytest.raises(RuntimeError, match="shape|logits|neurons"):
         model(C.PackBitsTensor(torch.zeros(8, 1, 28, 28, dtype=torch.bool, device=DEV), 64))
+
+
+def assert_tail_equals_modules(model):
+    """training, evaluation and packed counts with the trees and with the modules called themselves"""
+    x = torch.randint(0, 2, (32, 1, 28, 28), device=DEV).float()
+    results = []
+    for on in (True, False):
+        model.tree_tail = on
+        model.train().zero_grad()
+        out = model(x)
+        assert ("_Tree" in type(out.grad_fn).__name__) == on
+        out.square().sum().backward()
+        grads = [p.grad.clone() for p in model.parameters()]
+        with torch.no_grad():
+            results.append([out.detach(), *grads, model.eval()(x), model(C.PackBitsTensor(x.bool(), 64))])
+    # One element: a sum over 32 samples and up to 144 positions of products through seven layers, whose terms may be ten times the
+    # mean element and cancel: 7 roundings of 6e-8 on each of them, sqrt(32 * 144) of a kind, 10 * 7 * 6e-8 * 68 = 3e-4 of the
+    # mean.  (A wiring that did not arrive is off by the mean itself.)
+    for i, (a, b) in enumerate(zip(*results)):
+        assert_grad_close(a, b, rel=1e-4, rel_elem=3e-4, name=f"result {i}")
+
+
+@pytest.mark.parametrize("route", ["data", "loaded on the cpu", "other layer"])
+@pytest.mark.parametrize("at", [4, 5, 6])
+def test_another_wiring_reaches_the_trees(route, at):
+    torch.manual_seed(at)
+    model = C.ConvLogicMnistModel(k_param=2).to(DEV)
+    assert_tail_equals_modules(model)
+    layer = model.network[at]
+    if route == "data":
+        layer.indices_0.data.copy_(layer.indices_0.flip(0))
+        layer.invalidate()
+    elif route == "other layer":
+        model.network[at] = C.LogicLayer(layer.in_dim, layer.out_dim, implementation="cuda").to(DEV)
+    else:
+        state = C.ConvLogicMnistModel(k_param=2).state_dict()
+        model.cpu().load_state_dict(state)
+        model.to(DEV)
+    assert_tail_equals_modules(model)

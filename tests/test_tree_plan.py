@@ -1,0 +1,101 @@
+"""When the trees of three LogicLayers (difflogic/fc_tree.py) are derived again: after every way in which a wiring can change.
+On the CPU, with a stand-in for the tables that notes the wiring it was made from."""
+import copy
+import pickle
+
+import pytest
+import torch
+
+import convlogic_amd as C
+from convlogic_amd.difflogic import fc_tree
+
+
+class Noted:
+    def __init__(self, *layers):
+        self.wiring = [t.clone() for m in layers for t in (m.indices_0, m.indices_1)]
+
+    def of(self, layers):
+        return all(torch.equal(t, w) for t, w in zip((t for m in layers for t in (m.indices_0, m.indices_1)), self.wiring))
+
+
+@pytest.fixture
+def layers(monkeypatch):
+    monkeypatch.setattr(fc_tree, "TreePlan", Noted)
+    return chain(0)
+
+
+def chain(seed):
+    torch.manual_seed(seed)
+    return [C.LogicLayer(a, b, implementation="cuda") for a, b in ((24, 40), (40, 20), (20, 10))]
+
+
+def swapped(layer):
+    """another wiring of the layer in which every input is read as often as before"""
+    return layer.indices_0.flip(0)
+
+
+def test_the_plan_is_kept(layers):
+    plan = fc_tree.tree_plan(*layers)
+    assert plan.of(layers) and fc_tree.tree_plan(*layers) is plan
+    for m in layers:                                                   # no move: the same buffers
+        m.to("cpu").float().train()
+    assert fc_tree.tree_plan(*layers) is plan
+
+
+@pytest.mark.parametrize("at", [0, 1, 2])
+def test_invalidate_after_a_write_through_data(layers, at):
+    fc_tree.tree_plan(*layers)
+    layers[at].indices_0.data.copy_(swapped(layers[at]))
+    layers[at].invalidate()
+    assert fc_tree.tree_plan(*layers).of(layers)
+
+
+@pytest.mark.parametrize("at", [0, 1, 2])
+def test_writes_in_place_and_other_buffers(layers, at):
+    fc_tree.tree_plan(*layers)
+    layers[at].indices_0.copy_(swapped(layers[at]))
+    assert fc_tree.tree_plan(*layers).of(layers)
+    layers[at].indices_0 = swapped(layers[at])
+    assert fc_tree.tree_plan(*layers).of(layers)
+    for _ in range(20):                                                # (the allocator hands the last buffer's address out again)
+        new = swapped(layers[at])
+        layers[at].indices_0 = torch.empty(0, dtype=torch.int64)
+        del layers[at].indices_0
+        layers[at].register_buffer("indices_0", new)
+        assert fc_tree.tree_plan(*layers).of(layers)
+
+
+@pytest.mark.parametrize("at", [0, 1, 2])
+def test_a_key_that_is_the_same_after_a_move(layers, at, monkeypatch):
+    # buffers that went to another device and came back have version 0 again and may have the old addresses
+    fc_tree.tree_plan(*layers)
+    old = [layers[at].indices_0, layers[at].indices_1]
+    key = layers[at]._wiring_key()
+    layers[at]._apply(lambda t: t.clone())
+    for name, t in zip(("indices_0", "indices_1"), old):
+        t.data.copy_(swapped(layers[at]) if name == "indices_0" else t)
+        layers[at]._buffers[name] = t                                  # the old address, the old version, another wiring
+    assert layers[at]._wiring_key()[:5] == key[:5]
+    assert fc_tree.tree_plan(*layers).of(layers)
+
+
+def test_other_layers_behind_the_first(layers):
+    fc_tree.tree_plan(*layers)
+    other = chain(1)
+    key = layers[1]._wiring_key()
+    other[1]._wiring_key = lambda: key                                 # as if the new layer's buffers had the old addresses
+    other[1]._wiring_checked = key
+    assert fc_tree.tree_plan(layers[0], other[1], layers[2]).of([layers[0], other[1], layers[2]])
+    assert fc_tree.tree_plan(*layers).of(layers)
+    assert fc_tree.tree_plan(layers[0], layers[1], other[2]).of([layers[0], layers[1], other[2]])
+
+
+def test_a_loaded_wiring_and_copies(layers):
+    plan = fc_tree.tree_plan(*layers)
+    for copies in (copy.deepcopy(layers), pickle.loads(pickle.dumps(layers))):
+        for m in copies:
+            assert "_wiring_checked" not in m.__dict__
+        assert fc_tree.tree_plan(*copies) is not plan and fc_tree.tree_plan(*copies).of(copies)
+    for m, o in zip(layers, chain(1)):
+        m.load_state_dict(o.state_dict())
+    assert fc_tree.tree_plan(*layers).of(layers)
