@@ -16,29 +16,18 @@ _PLANS = weakref.WeakKeyDictionary()
 
 class TreePlan:
     """The trees of three layers' wiring: input rows, neuron ids and list positions of every root's eight operands, and the
-    place of every neuron in its tree (int32 on the device; include/convlogic_amd.h).  For layers whose every neuron is read
-    exactly once."""
+    place of every neuron in its tree (int32 on the device; include/convlogic_amd.h).  `fits`: every neuron of the first two
+    layers is read exactly once, so there are trees."""
 
     def __init__(self, first, second, third):
-        a, b = first._buffers["indices_0"], first._buffers["indices_1"]
-        mid = torch.stack([third._buffers["indices_0"], third._buffers["indices_1"]], 1)                       # [roots, 2]
-        leaf = torch.stack([second._buffers["indices_0"][mid], second._buffers["indices_1"][mid]], 2).flatten(1)   # [roots, 4]
-        operand = torch.stack([a, b], 1)                                                                       # [out, 2]
-        # place of every operand in the lists input feature -> operands: by feature, then by neuron, first operand first (the
-        # order of given_x_indices_of_y)
-        order = torch.argsort(operand.flatten(), stable=True)
-        place = torch.empty_like(order)
-        place[order] = torch.arange(order.numel(), device=order.device)
-        self.roots = third.out_dim
-        self.rows = operand[leaf].flatten(1).to(torch.int32).contiguous()
-        self.pos = place.view(-1, 2)[leaf].flatten(1).to(torch.int32).contiguous()
-        self.ids = torch.cat([leaf, mid, torch.zeros_like(mid)], 1).to(torch.int32).contiguous()
-        # where a neuron's sums are: of the first layer's, of the second's, of the roots
-        slots = torch.arange(7 * self.roots, device=order.device).view(-1, 7)
-        slot = [torch.empty(n, dtype=torch.int64, device=order.device) for n in (first.out_dim, second.out_dim)]
-        slot[0][leaf] = slots[:, :4]
-        slot[1][mid] = slots[:, 4:6]
-        self.slot = torch.cat([slot[0], slot[1], slots[:, 6]]).to(torch.int32)
+        roots = self.roots = third.out_dim
+        tables = torch.empty((31 * roots,), dtype=torch.int32, device=first._buffers["indices_0"].device)
+        self.rows, self.pos, self.ids, self.slot = tables.split([8 * roots, 8 * roots, 8 * roots, 7 * roots])
+        wiring = [m._buffers[name] for m in (first, second, third) for name in ("indices_0", "indices_1")]
+        wiring += [first._buffers[name] for name in ("given_x_indices_of_y_start", "given_x_indices_of_y")]
+        check(_lib.load().clg_fc_tree_plan(*(t.data_ptr() for t in wiring), *(t.data_ptr() for t in (self.rows, self.pos, self.ids, self.slot)),
+                                           first.in_dim, roots, stream_ptr(tables)))
+        self.fits = int(self.slot.min()) >= 0
 
 
 def tree_plan(first, second, third):
@@ -49,8 +38,8 @@ def tree_plan(first, second, third):
     keys = (first._check_wiring(), second._check_wiring(), third._check_wiring())
     cached = _PLANS.get(first)
     if cached is None or cached[0] != keys or cached[1]() is not second or cached[2]() is not third:
-        fits = second._sole_consumers(keys[1]) and third._sole_consumers(keys[2])
-        cached = _PLANS[first] = (keys, weakref.ref(second), weakref.ref(third), TreePlan(first, second, third) if fits else None)
+        plan = TreePlan(first, second, third)
+        cached = _PLANS[first] = (keys, weakref.ref(second), weakref.ref(third), plan if plan.fits else None)
     return cached[3]
 
 

@@ -109,6 +109,7 @@ SIGNATURES = {
     "clg_convblock_bin_backward_scratch_bytes": (_i64, [_i, _GP]),
     "clg_convblock_bin_backward": (_i, [_i, _GP, _p, _p, _p, _p, _p, _i, _p, _p]),
     "clg_host_flag_device_pointer": (_i, [_p, _p]),
+    "clg_fc_tree_plan": (_i, [_p] * 12 + [_i64, _i64, _p]),
     "clg_fc_tree_fold": (_i, [_p, _p, _p, _p, _p, _p, _i64, _i, _p]),
     "clg_fc_tree_partial_elems": (_i64, [_i64, _i64, _i64, _i64]),
     "clg_fc_tree_forward": (_i, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _f64, _p]),

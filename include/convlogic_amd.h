@@ -521,6 +521,12 @@ int clg_host_flag_device_pointer(void *host, void **device);
  * x is feature-major with a row pitch >= batch (lanes are 1, 2 or 4 samples wide, whatever pitch and addresses allow).
  * An entry of rows, ids, pos or slot out of range is taken as the last one: a wrong result, no access outside the buffers.
  * ------------------------------------------------------------------------------- */
+/* the four tables from the layers' wirings (a / b of the three, start / flat = given_x_indices_of_y_start / given_x_indices_of_y
+ * of the first, neurons increasing in every list).  Where a neuron of the first two layers is read by no operand, or by several, a slot
+ * is -1 afterwards: the wiring makes no trees. */
+int clg_fc_tree_plan(const int64_t *a0, const int64_t *b0, const int64_t *a1, const int64_t *b1, const int64_t *a2, const int64_t *b2,
+                     const int64_t *start, const int64_t *flat, int32_t *rows, int32_t *pos, int32_t *ids, int32_t *slot, int64_t in_dim,
+                     int64_t roots, void *stream);
 /* coef of the softmax (hard = 0) or the arg-max gates (hard = 1); probs [7 roots, 16] takes the probabilities, neurons of the first
  * layer first (may be NULL) */
 int clg_fc_tree_fold(const float *logits0, const float *logits1, const float *logits2, const int32_t *ids, float *coef,

@@ -257,3 +257,26 @@ def test_another_wiring_reaches_the_trees(route, at):
         model.cpu().load_state_dict(state)
         model.to(DEV)
     assert_tail_equals_modules(model)
+
+
+@pytest.mark.parametrize("in_dim,roots", [(1, 1), (2, 1), (8, 1), (3, 31), (40, 32), (64, 33), (700, 663), (2000, 250), (5, 5000)])
+def test_the_tables_of_a_wiring(in_dim, roots):
+    torch.manual_seed(in_dim + roots)
+    layers = [C.LogicLayer(a, b, implementation="cuda").to(DEV) for a, b in ((in_dim, 4 * roots), (4 * roots, 2 * roots), (2 * roots, roots))]
+    with torch.no_grad():                                              # some neurons read one feature twice, some features are not read
+        layers[0].indices_1[::3] = layers[0].indices_0[::3]
+        layers[0].indices_1[1::5] = in_dim // 2
+    plan = fc_tree.tree_plan(*layers)
+    a, b = ([getattr(m, name).cpu() for m in layers] for name in ("indices_0", "indices_1"))
+    mid = torch.stack([a[2], b[2]], 1)
+    leaf = torch.stack([a[1][mid], b[1][mid]], 2).flatten(1)
+    operand = torch.stack([a[0], b[0]], 1)
+    order = torch.argsort(operand.flatten(), stable=True)              # by feature, then by neuron, the first operand first
+    place = torch.empty_like(order)
+    place[order] = torch.arange(order.numel())
+    slots = torch.arange(7 * roots).view(-1, 7)
+    slot = torch.full((7 * roots,), -1)
+    slot[leaf], slot[4 * roots + mid], slot[6 * roots:] = slots[:, :4], slots[:, 4:6], slots[:, 6]
+    want = operand[leaf].flatten(1), place.view(-1, 2)[leaf].flatten(1), torch.cat([leaf, mid, torch.zeros_like(mid)], 1), slot
+    for got, table in zip((plan.rows, plan.pos, plan.ids, plan.slot), want):
+        assert torch.equal(got.cpu().long(), table.flatten())

@@ -11,6 +11,8 @@ from convlogic_amd.difflogic import fc_tree
 
 
 class Noted:
+    fits = True
+
     def __init__(self, *layers):
         self.wiring = [t.clone() for m in layers for t in (m.indices_0, m.indices_1)]
 
