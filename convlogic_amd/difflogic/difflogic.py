@@ -12,6 +12,7 @@ import numpy as np
 import torch
 
 from ..hip import difflogic_hip
+from . import fc_tree
 from .functional import GradFactor, bin_op_s, get_unique_connections
 from .packbitstensor import PackBitsTensor
 
@@ -220,6 +221,7 @@ class LogicLayer(torch.nn.Module):
     def _load_from_state_dict(self, *args, **kwargs):
         super()._load_from_state_dict(*args, **kwargs)
         self.invalidate()
+        fc_tree.refresh(self)
 
     def _sole_consumers(self, key=None):
         """True when every input feature is read by exactly one neuron operand (the halving layers of the

@@ -2,6 +2,7 @@
 102-107) -- as one operation.  Where every neuron of the first two layers is read exactly once, each neuron of the third is
 the root of a tree of seven gates over eight input rows that no other root shares, so the three layers are evaluated, and
 differentiated, without activations of their own (csrc/fc_tree.hip)."""
+import threading
 import weakref
 
 import torch
@@ -9,45 +10,103 @@ import torch
 from ..hip import _lib
 from ..hip._lib import check, stream_ptr
 
-# per first layer: (keys of the three wirings, weak references to the other two layers, plan); kept outside the modules so that
-# copies and pickles carry no derived buffers
+# per first layer: the _Entry of every pair of layers that was seen behind it; kept outside the modules so that copies and pickles
+# carry no derived buffers
 _PLANS = weakref.WeakKeyDictionary()
+_BUILDING = threading.Lock()
 
 
 class TreePlan:
     """The trees of three layers' wiring: input rows, neuron ids and list positions of every root's eight operands, and the
-    place of every neuron in its tree (int32 on the device; include/convlogic_amd.h).  `fits`: every neuron of the first two
-    layers is read exactly once, so there are trees."""
+    place of every neuron in its tree (int32 on the device; include/convlogic_amd.h).  The tables stay where they are for the
+    plan's life: a recorded HIP graph reads them at these addresses."""
 
     def __init__(self, first, second, third):
-        roots = self.roots = third.out_dim
-        tables = torch.empty((31 * roots,), dtype=torch.int32, device=first._buffers["indices_0"].device)
-        self.rows, self.pos, self.ids, self.slot = tables.split([8 * roots, 8 * roots, 8 * roots, 7 * roots])
-        wiring = [m._buffers[name] for m in (first, second, third) for name in ("indices_0", "indices_1")]
+        self.roots, self.device = third.out_dim, first._buffers["indices_0"].device
+        tables = torch.empty((31 * self.roots,), dtype=torch.int32, device=self.device)
+        self.rows, self.pos, self.ids, self.slot = tables.split([n * self.roots for n in (8, 8, 8, 7)])
+        self.build(first, second, third)
+
+    def build(self, first, second, third):
+        wiring = wiring_of(first, second, third)
         wiring += [first._buffers[name] for name in ("given_x_indices_of_y_start", "given_x_indices_of_y")]
         check(_lib.load().clg_fc_tree_plan(*(t.data_ptr() for t in wiring), *(t.data_ptr() for t in (self.rows, self.pos, self.ids, self.slot)),
-                                           first.in_dim, roots, stream_ptr(tables)))
-        self.fits = int(self.slot.min()) >= 0
+                                           first.in_dim, self.roots, stream_ptr(self.slot)))
+
+    def fits(self):
+        """True when every neuron of the first two layers is read exactly once, so that there are trees.  Waits for the tables."""
+        return int(self.slot.min()) >= 0
+
+
+class _Entry:
+    def __init__(self, second, third):
+        self.second, self.third = weakref.ref(second), weakref.ref(third)
+        self.keys = self.plan = None
+        self.fits = False
+
+    def is_of(self, second, third):
+        return self.second() is second and self.third() is third
+
+
+def wiring_of(*layers):
+    return [m._buffers[name] for m in layers for name in ("indices_0", "indices_1")]
 
 
 def tree_plan(first, second, third):
-    """The TreePlan of three LogicLayers, or None when their wiring does not make trees.  Rebuilt when a wiring buffer was
-    modified in place, replaced or moved, when invalidate() was called on one of the layers, and for other layers."""
+    """The TreePlan of three LogicLayers, or None when their wiring does not make trees.  Made again, in the same tables, when
+    a wiring buffer was modified in place, replaced or moved and when invalidate() was called on one of the layers.  (Made
+    outside a recording only: making it waits for the device.)"""
     if 2 * second.out_dim != second.in_dim or 2 * third.out_dim != third.in_dim or second.in_dim != first.out_dim or third.in_dim != second.out_dim:
         return None
     keys = (first._check_wiring(), second._check_wiring(), third._check_wiring())
-    cached = _PLANS.get(first)
-    if cached is None or cached[0] != keys or cached[1]() is not second or cached[2]() is not third:
-        plan = TreePlan(first, second, third)
-        cached = _PLANS[first] = (keys, weakref.ref(second), weakref.ref(third), plan if plan.fits else None)
-    return cached[3]
+    entry = next((e for e in _PLANS.get(first, ()) if e.is_of(second, third)), None)
+    if entry is None or entry.keys != keys:
+        if first._buffers["indices_0"].is_cuda and torch.cuda.is_current_stream_capturing():
+            return None
+        with _BUILDING:
+            entry = _make(first, second, third, keys)
+    return entry.plan if entry.fits else None
+
+
+def _make(first, second, third, keys):
+    entries = _PLANS.setdefault(first, [])
+    entry = next((e for e in entries if e.is_of(second, third)), None)
+    if entry is None:
+        entry = _Entry(second, third)
+    elif entry.keys == keys:                                          # another thread made it meanwhile
+        return entry
+    entry.keys = None
+    if entry.plan is None or entry.plan.device != first._buffers["indices_0"].device:
+        entry.plan, had = TreePlan(first, second, third), False
+    else:
+        entry.plan.build(first, second, third)
+        had = True
+    entry.fits = entry.plan.fits()
+    if not (entry.fits or had):
+        entry.plan = None                                             # no trees, and nothing recorded with them
+    entry.keys = keys
+    _PLANS[first] = [e for e in entries if e.second() is not None and e.third() is not None and e is not entry] + [entry]
+    return entry
+
+
+def refresh(layer):
+    """Makes the tables of the plans that `layer` belongs to again (a state was loaded into it): a step that was recorded with
+    them replays the loaded wiring.  In the stream's order, no wait; the next tree_plan() looks at the result."""
+    with _BUILDING:
+        for first, entries in list(_PLANS.items()):
+            for e in entries:
+                second, third = e.second(), e.third()
+                if e.plan is None or second is None or third is None or layer not in (first, second, third):
+                    continue
+                if all(t.device == e.plan.device for t in wiring_of(first, second, third)):
+                    e.plan.build(first, second, third)
 
 
 class _TreeFunction(torch.autograd.Function):
     """x feature-major [features, B] -> class sums [B, k] / tau of the three layers; gradients of x and of the logits."""
 
     @staticmethod
-    def forward(ctx, x, l0, l1, l2, start, plan, k, tau):
+    def forward(ctx, x, l0, l1, l2, start, wiring, plan, k, tau):
         lib, st = _lib.load(), stream_ptr(x)
         in_dim, batch = x.shape
         coef = torch.empty((plan.roots, 28), dtype=torch.float32, device=x.device)
@@ -55,14 +114,15 @@ class _TreeFunction(torch.autograd.Function):
         check(lib.clg_fc_tree_fold(l0.data_ptr(), l1.data_ptr(), l2.data_ptr(), plan.ids.data_ptr(), coef.data_ptr(), probs.data_ptr(),
                                    plan.roots, 0, st))
         out = _tree_forward(lib, x, plan, coef, k, tau, st)
-        # (probabilities, not logits, as in the modules: the logits may be updated between forward and backward)
-        ctx.save_for_backward(x, start, coef, probs)
+        # (probabilities, not logits, as in the modules: the logits may be updated between forward and backward; the wiring for
+        # autograd's check that it was not)
+        ctx.save_for_backward(x, start, coef, probs, *wiring)
         ctx.plan, ctx.k, ctx.tau = plan, k, tau
         return out
 
     @staticmethod
     def backward(ctx, grad_out):
-        x, start, coef, probs = ctx.saved_tensors
+        x, start, coef, probs = ctx.saved_tensors[:4]
         plan, k = ctx.plan, ctx.k
         grad_out = _lib.check_input(grad_out.contiguous(), "grad_out", torch.float32, (x.shape[1], k))
         _lib.check_same_device(x, grad_out)
@@ -75,7 +135,7 @@ class _TreeFunction(torch.autograd.Function):
             x.data_ptr(), plan.rows.data_ptr(), plan.pos.data_ptr(), plan.slot.data_ptr(), coef.data_ptr(), grad_out.data_ptr(),
             probs.data_ptr(), g0.data_ptr(), g1.data_ptr(), g2.data_ptr(), rowgrad, sums, start.data_ptr(),
             gx.data_ptr(), in_dim, plan.roots, k, batch, batch, float(ctx.tau), stream_ptr(x)))
-        return gx, g0, g1, g2, None, None, None, None
+        return gx, g0, g1, g2, None, None, None, None, None
 
 
 def _tree_forward(lib, x, plan, coef, k, tau, st):
@@ -107,8 +167,8 @@ def tree_eval(layers, group_sum, x, plan):
 def tree_train(layers, group_sum, x, plan):
     """group_sum(third(second(first(x)))) in training; x feature-major [features, B]."""
     first, second, third = layers
-    return _TreeFunction.apply(x, first.weights, second.weights, third.weights, first._buffers["given_x_indices_of_y_start"], plan,
-                               group_sum.k, group_sum.tau)
+    return _TreeFunction.apply(x, first.weights, second.weights, third.weights, first._buffers["given_x_indices_of_y_start"],
+                               wiring_of(*layers), plan, group_sum.k, group_sum.tau)
 
 
 def tree_packed(layers, k, x, plan):

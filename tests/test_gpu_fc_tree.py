@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import convlogic_amd as C
+from convlogic_amd.convlogic.model import _forward
 from convlogic_amd.difflogic import fc_tree
 from oracle import convlogic_oracle as O
 from tests.gpu_util import DEV, assert_grad_close
@@ -280,3 +281,81 @@ def test_the_tables_of_a_wiring(in_dim, roots):
     want = operand[leaf].flatten(1), place.view(-1, 2)[leaf].flatten(1), torch.cat([leaf, mid, torch.zeros_like(mid)], 1), slot
     for got, table in zip((plan.rows, plan.pos, plan.ids, plan.slot), want):
         assert torch.equal(got.cpu().long(), table.flatten())
+
+
+class Head(torch.nn.Module):
+    """a network that is nothing but its fully connected end"""
+
+    def __init__(self, in_dim=40, roots=20, k=2):
+        super().__init__()
+        layers = [C.LogicLayer(a, b, implementation="cuda") for a, b in ((in_dim, 4 * roots), (4 * roots, 2 * roots), (2 * roots, roots))]
+        self.network = torch.nn.Sequential(torch.nn.Flatten(), *layers, C.GroupSum(k, tau=3.0))
+
+    def forward(self, x):
+        return _forward(self, x)
+
+
+def test_a_recorded_step_replays_the_loaded_wiring():
+    torch.manual_seed(7)
+    model, other = Head().to(DEV), Head().to(DEV)
+    batches = [(torch.rand(32, 40, device=DEV), torch.randint(0, 2, (32,), device=DEV)) for _ in range(3)]
+    loss_of = lambda x, y: torch.nn.functional.cross_entropy(model(x), y)
+    step = C.GraphedStep(loss_of, batches[0], model.parameters())
+    plan = fc_tree.tree_plan(*model.network[1:4])
+    addresses = [t.data_ptr() for t in (plan.rows, plan.pos, plan.ids, plan.slot)]
+    own, another = ({k: v.clone() for k, v in m.state_dict().items()} for m in (model, other))
+    for state, between in ((own, True), (another, False), (own, False), (another, True)):
+        model.load_state_dict(state)
+        if between:                                                    # an eager pass on the loaded state before the replays
+            with torch.no_grad():
+                model.eval()(batches[0][0])
+            model.train()
+        other = [torch.randint(0, 2**31 - 1, (1 << 12,), dtype=torch.int32, device=DEV) for _ in range(32)]   # (takes freed memory)
+        replayed = []
+        for x, y in batches:
+            loss = step(x, y)
+            torch.cuda.synchronize()
+            replayed.append([loss.clone()] + [p.grad.clone() for p in model.parameters()])
+        for (x, y), got in zip(batches, replayed):
+            grads = [p.grad for p in model.parameters()]
+            for p in model.parameters():
+                p.grad = None
+            loss = loss_of(x, y)
+            loss.backward()
+            assert all(torch.equal(a, b) for a, b in zip(got, [loss.detach()] + [p.grad for p in model.parameters()]))
+            for p, g in zip(model.parameters(), grads):
+                p.grad = g                                              # the step's own
+        assert fc_tree.tree_plan(*model.network[1:4]) is plan
+    assert addresses == [t.data_ptr() for t in (plan.rows, plan.pos, plan.ids, plan.slot)]
+
+
+def test_a_wiring_changed_between_forward_and_backward_is_refused():
+    torch.manual_seed(8)
+    model = C.ConvLogicMnistModel(k_param=2).to(DEV)
+    for at in (4, 5, 6):
+        out = model(torch.zeros(4, 1, 28, 28, device=DEV))
+        with torch.no_grad():
+            model.network[at].indices_0.copy_(model.network[at].indices_0.flip(0))
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            out.sum().backward()
+
+
+def test_a_recording_without_the_tables_takes_the_modules():
+    torch.manual_seed(9)
+    model, x = Head().to(DEV).eval(), torch.randint(0, 2, (64, 40), device=DEV).float()
+    with torch.no_grad():
+        want = model.network(x)                                        # the modules have checked their wirings, no tables yet
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            model.network(x)
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got = model(x)
+        for _ in range(3):
+            x.copy_(torch.randint(0, 2, x.shape, device=DEV).float())
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(got, model.network(x))
+            assert torch.equal(got, model(x))

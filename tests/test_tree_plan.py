@@ -11,9 +11,15 @@ from convlogic_amd.difflogic import fc_tree
 
 
 class Noted:
-    fits = True
+    device = torch.device("cpu")
 
     def __init__(self, *layers):
+        self.build(*layers)
+
+    def fits(self):
+        return True
+
+    def build(self, *layers):
         self.wiring = [t.clone() for m in layers for t in (m.indices_0, m.indices_1)]
 
     def of(self, layers):
@@ -100,4 +106,22 @@ def test_a_loaded_wiring_and_copies(layers):
         assert fc_tree.tree_plan(*copies) is not plan and fc_tree.tree_plan(*copies).of(copies)
     for m, o in zip(layers, chain(1)):
         m.load_state_dict(o.state_dict())
-    assert fc_tree.tree_plan(*layers).of(layers)
+        assert plan.of(layers)                                          # at once: a recorded step reads these tables
+    assert fc_tree.tree_plan(*layers) is plan
+
+
+def test_the_tables_of_a_recorded_step_stay(layers):
+    plan = fc_tree.tree_plan(*layers)
+    other = chain(1)
+    assert fc_tree.tree_plan(layers[0], other[1], layers[2]) is not plan    # a second network over the same first layer
+    for m in layers:
+        m.load_state_dict(m.state_dict())
+    layers[1].indices_0.copy_(swapped(layers[1]))
+    layers[2].invalidate()
+    assert fc_tree.tree_plan(*layers) is plan and plan.of(layers)
+    plan.fits = lambda: False                                          # a wiring that makes no trees: not used, not freed
+    layers[0].invalidate()
+    assert fc_tree.tree_plan(*layers) is None
+    plan.fits = lambda: True
+    layers[0].invalidate()
+    assert fc_tree.tree_plan(*layers) is plan
