@@ -231,15 +231,21 @@ class ConvLogicLayer(nn.Module):
         """(plan bytes, signature) of this layer's backward pass for inputs like x: the reverse map input channel ->
         kernels and the tap offsets of the kernels' image layout, which depend only on the selection and the geometry.
         Built on the first training step with a shape and kept (the reference's LogicLayer builds its reverse map at
-        construction, src/difflogic/difflogic.py:71-87); rebuilt when the selection buffer or the library's knobs change."""
+        construction, src/difflogic/difflogic.py:71-87); rebuilt when the selection buffer or the library's knobs change.
+        A kept plan is complete: a call on any other stream or thread may use it.  One that is made inside a recording is the
+        recording's own, which makes it again in every replay."""
         from ..hip import _lib
         key = (tuple(x.shape), x.dtype, x.device, sel._version, sel.data_ptr(), _lib.knob_generation())
         plans = self.__dict__.setdefault("_plans", {})
         plan = plans.get(key)
         if plan is None:
+            plan = convlogic_hip.make_backward_plan(x, self.out_channels, sel, *self.stride, *self.padding, *self.kernel)
+            if torch.cuda.is_current_stream_capturing():
+                return plan
+            torch.cuda.current_stream(x.device).synchronize()
             if len(plans) >= 4:                                      # a few batch shapes (training, last partial batch, evaluation)
                 plans.pop(next(iter(plans)))
-            plan = plans[key] = convlogic_hip.make_backward_plan(x, self.out_channels, sel, *self.stride, *self.padding, *self.kernel)
+            plans[key] = plan
         return plan
 
     def prefold_candidate(self):

@@ -8,6 +8,7 @@ import pytest
 import torch
 
 import convlogic_amd as C
+from convlogic_amd.difflogic import fc_tree
 from convlogic_amd.hip import _lib, convlogic_hip
 from tests.gpu_util import DEV, assert_grad_close, block_oracle, set_knobs
 
@@ -113,3 +114,44 @@ def test_module_training_path_uses_the_plan_and_matches_the_oracle(shape):
     # another batch size gets a plan of its own; an in-place edit of the selection drops the old ones on the next call
     layer(x[:3].detach()).sum().backward()
     assert len(layer._plans) == 2
+
+
+def test_a_kept_plan_is_complete():
+    # what a first call leaves for calls on other streams: the tables of a block's plan and of a network's trees
+    torch.manual_seed(5)
+    layer, x = C.ConvLogicLayer(8, 16, padding=1, complete=True, implementation="cuda").to(DEV), torch.rand(4, 8, 8, 8, device=DEV)
+    chain = [C.LogicLayer(a, b, implementation="cuda").to(DEV) for a, b in ((40, 80), (80, 40), (40, 20))]
+    busy = torch.randn(4096, 4096, device=DEV)
+    torch.cuda.synchronize()
+    for make in (lambda: layer._backward_plan(x, layer.selection), lambda: fc_tree.tree_plan(*chain)):
+        side = torch.cuda.Stream()
+        with torch.cuda.stream(side):
+            for _ in range(20):                                        # the stream is behind when the plan is asked for
+                busy @ busy
+            assert make() is not None and side.query()
+
+
+def test_a_plan_made_in_a_recording_is_the_recordings_own():
+    torch.manual_seed(6)
+    layer = C.ConvLogicLayer(8, 16, padding=1, complete=True, implementation="cuda").to(DEV)
+    static = torch.rand(4, 8, 8, 8, device=DEV)
+    layer(static[:2]).sum().backward()                                 # (the selection is checked, no plan for four samples)
+
+    def step():
+        layer.weights.grad = None
+        layer(static).square().sum().backward()
+        return layer.weights.grad
+
+    graph = torch.cuda.CUDAGraph()
+    layer.weights.grad = None
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        layer(static).square().sum().backward()
+    recorded = layer.weights.grad
+    assert [key[0][0] for key in layer._plans] == [2]
+    for _ in range(3):
+        static.copy_(torch.rand_like(static))
+        eager = step().clone()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(recorded, eager)
