@@ -1,5 +1,8 @@
 """ConvLogicLayer, its autograd functions and PoolLogicLayer.
 Interface of the reference's src/convlogic/convlogic_layer.py, on HIP kernels for gfx950."""
+import threading
+import types
+
 import torch
 from torch import nn
 from torch.autograd import Function
@@ -166,6 +169,22 @@ def _pair(v):
     return (v, v) if isinstance(v, int) else tuple(v)
 
 
+_MAKING_PLANS = threading.Lock()
+
+
+class _KeptPlan:
+    """A backward plan of a layer, the selection it was made from (version and address) and whether a recording reads it."""
+
+    def __init__(self):
+        self.plan = self.wiring = None
+        self.recorded = False
+
+    def make(self, like, sel, layer):
+        """In place where there are tables already: a recorded step reads them at their addresses."""
+        tables = None if self.plan is None else self.plan[0]
+        self.plan = convlogic_hip.make_backward_plan(like, layer.out_channels, sel, *layer.stride, *layer.padding, *layer.kernel, into=tables)
+
+
 class ConvLogicLayer(nn.Module):
     """Logic-gate convolution: every output channel reads 8 taps (from at most two input channels of
     its group) inside its receptive field and combines them with 4 gates, or with the complete
@@ -222,31 +241,52 @@ class ConvLogicLayer(nn.Module):
         self._selection_checked = key
 
     def invalidate(self):
-        """Forces the next call to check the selection buffer again and to rebuild the backward plans (after a write
+        """Forces the next call to check the selection buffer again and to make the backward plans again (after a write
         through `.data`)."""
         self._selection_checked = None
-        self._plans = {}
+        for kept in self.__dict__.get("_plans", {}).values():
+            kept.wiring = None
 
     def _backward_plan(self, x, sel):
         """(plan bytes, signature) of this layer's backward pass for inputs like x: the reverse map input channel ->
         kernels and the tap offsets of the kernels' image layout, which depend only on the selection and the geometry.
         Built on the first training step with a shape and kept (the reference's LogicLayer builds its reverse map at
-        construction, src/difflogic/difflogic.py:71-87); rebuilt when the selection buffer or the library's knobs change.
-        A kept plan is complete: a call on any other stream or thread may use it.  One that is made inside a recording is the
-        recording's own, which makes it again in every replay."""
+        construction, src/difflogic/difflogic.py:71-87); made again, in the same tables, when the selection buffer changes.
+        A kept plan is complete: a call on any other stream or thread may use it.  One that was taken in a recording is kept
+        for the layer's life, as the replays read it; one that is made inside a recording is the recording's own, which makes
+        it again in every replay."""
         from ..hip import _lib
-        key = (tuple(x.shape), x.dtype, x.device, sel._version, sel.data_ptr(), _lib.knob_generation())
+        key = (tuple(x.shape), x.dtype, x.device, _lib.knob_generation())
+        wiring = (sel._version, sel.data_ptr())
         plans = self.__dict__.setdefault("_plans", {})
-        plan = plans.get(key)
-        if plan is None:
-            plan = convlogic_hip.make_backward_plan(x, self.out_channels, sel, *self.stride, *self.padding, *self.kernel)
-            if torch.cuda.is_current_stream_capturing():
-                return plan
-            torch.cuda.current_stream(x.device).synchronize()
-            if len(plans) >= 4:                                      # a few batch shapes (training, last partial batch, evaluation)
-                plans.pop(next(iter(plans)))
-            plans[key] = plan
-        return plan
+        kept, recording = plans.get(key), torch.cuda.is_current_stream_capturing()
+        if kept is not None and kept.wiring == wiring:
+            kept.recorded |= recording
+            return kept.plan
+        if recording:
+            return convlogic_hip.make_backward_plan(x, self.out_channels, sel, *self.stride, *self.padding, *self.kernel)
+        with _MAKING_PLANS:
+            kept = plans.get(key)
+            if kept is None:
+                self._make_room(plans, x.device)
+                kept = _KeptPlan()
+            if kept.wiring != wiring:                                # (else another thread made it meanwhile)
+                kept.wiring = None
+                kept.make(x, sel, self)
+                torch.cuda.current_stream(x.device).synchronize()
+                kept.wiring = wiring
+                plans[key] = kept
+            return kept.plan
+
+    @staticmethod
+    def _make_room(plans, device, most=16):
+        """At most `most` plans beside the recorded ones.  (A few batch shapes: training, last partial batch, evaluation; a program
+        that goes round more of them makes one plan per call, and waits for the device, as kernels in flight may read the plan
+        that goes.)"""
+        idle = [key for key, kept in plans.items() if not kept.recorded]
+        if len(idle) >= most:
+            torch.cuda.synchronize(device)
+            plans.pop(idle[0])
 
     def prefold_candidate(self):
         """The logits a network may fold for this layer ahead of its forward call (one launch for all its layers,
@@ -269,9 +309,19 @@ class ConvLogicLayer(nn.Module):
             return pf[2], pf[3]
         return None
 
+    def __getstate__(self):                                          # copies and pickles make plans of their own
+        return {name: value for name, value in self.__dict__.items() if name != "_plans"}
+
+    def __setstate__(self, state):
+        super().__setstate__({name: value for name, value in state.items() if name != "_plans"})
+
     def _load_from_state_dict(self, *args, **kwargs):
         super()._load_from_state_dict(*args, **kwargs)
         self.invalidate()
+        sel = self._buffers["selection"]
+        for (shape, dtype, device, _), kept in self.__dict__.get("_plans", {}).items():
+            if kept.recorded and sel.device == device:               # a recorded step replays the loaded selection
+                kept.make(types.SimpleNamespace(shape=shape, dtype=dtype, device=device), sel.contiguous(), self)
 
     def forward(self, x):
         if isinstance(x, PackBitsTensor):

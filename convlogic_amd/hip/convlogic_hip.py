@@ -390,19 +390,22 @@ def full_convlogic_forward_logits(x, logits, selection, stride_h, stride_w, pad_
     return y, argmax, probs
 
 
-def make_backward_plan(x, c_out, selection, stride_h, stride_w, pad_h, pad_w, kernel_h, kernel_w):
+def make_backward_plan(x, c_out, selection, stride_h, stride_w, pad_h, pad_w, kernel_h, kernel_w, into=None):
     """Per-layer plan of the block's backward pass for inputs of x's shape and dtype: -> (plan bytes on the device,
     signature).  Depends only on the selection and the geometry; built once and reused by every
     full_convlogic_backward_planned() call of the layer (the reverse map the reference's LogicLayer builds at
-    construction, src/difflogic/difflogic.py:71-87, for the fused block)."""
-    check_input(x, "x")
-    if x.dim() != 4:
-        raise RuntimeError(f"Expected x to be 4D (N, C, H, W), but got {x.dim()}")
+    construction, src/difflogic/difflogic.py:71-87, for the fused block).  Of x only shape, dtype and device are looked at.
+    into: the bytes of an earlier plan for the same geometry, which are written again."""
+    if isinstance(x, torch.Tensor):
+        check_input(x, "x")
+    if len(x.shape) != 4:
+        raise RuntimeError(f"Expected x to be 4D (N, C, H, W), but got {len(x.shape)}")
     _selection_arg(x, selection, c_out)
     g = _geom(x, c_out, stride_h, stride_w, pad_h, pad_w, kernel_h, kernel_w)
     lib = _lib.load()
     dt = dtype_code(x)
-    plan = _scratch(lib.clg_convblock_plan_bytes(dt, ctypes.byref(g)), x.device)
+    nbytes = lib.clg_convblock_plan_bytes(dt, ctypes.byref(g))
+    plan = into if into is not None and into.numel() >= nbytes and into.device == x.device else _scratch(nbytes, x.device)
     sig = ctypes.c_int64(0)
     check(lib.clg_convblock_plan(dt, ctypes.byref(g), selection.data_ptr(), plan.data_ptr(), ctypes.byref(sig), stream_ptr(x)))
     return plan, sig.value

@@ -2,7 +2,9 @@
 that depend only on the selection are built once; a planned call gives the gradients of the unplanned entry points on
 every kernel family (images in LDS, padded global copy, 4x4 one-sample-per-lane, any-shape gather), twice in a row,
 with and without the coefficients folded by the forward launch."""
+import copy
 import ctypes
+import pickle
 
 import pytest
 import torch
@@ -155,3 +157,51 @@ def test_a_plan_made_in_a_recording_is_the_recordings_own():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(recorded, eager)
+
+
+def test_a_recorded_step_replays_the_loaded_selection_and_its_plan_stays():
+    torch.manual_seed(7)
+    model, other = (C.ConvLogicMnistModel(k_param=2).to(DEV) for _ in range(2))
+    batches = [(torch.randint(0, 2, (32, 1, 28, 28), device=DEV).float(), torch.randint(0, 10, (32,), device=DEV)) for _ in range(2)]
+    loss_of = lambda x, y: torch.nn.functional.cross_entropy(model(x), y)
+    step = C.GraphedStep(loss_of, batches[0], model.parameters())
+    blocks = [m for m in model.network if isinstance(m, C.ConvLogicLayer) and m.__dict__.get("_plans")]
+    recorded = [kept for m in blocks for kept in m._plans.values() if kept.recorded]
+    assert len(recorded) == len(blocks) >= 2
+    addresses = [kept.plan[0].data_ptr() for kept in recorded]
+    own, another = ({k: v.clone() for k, v in m.state_dict().items()} for m in (model, other))
+    for state, eager_first in ((own, True), (another, False), (own, False), (another, True)):
+        model.load_state_dict(state)
+        for n in range(1, 21) if eager_first else ():                  # more batch sizes than plans are kept
+            model(batches[0][0][:n])
+        taken = [torch.randint(0, 2**31 - 1, (1 << 12,), dtype=torch.int32, device=DEV) for _ in range(32)]   # (takes freed memory)
+        replayed = []
+        for x, y in batches:
+            loss = step(x, y)
+            torch.cuda.synchronize()
+            replayed.append([loss.clone()] + [p.grad.clone() for p in model.parameters()])
+        for (x, y), got in zip(batches, replayed):
+            grads = [p.grad for p in model.parameters()]
+            for p in model.parameters():
+                p.grad = None
+            loss = loss_of(x, y)
+            loss.backward()
+            assert all(torch.equal(a, b) for a, b in zip(got, [loss.detach()] + [p.grad for p in model.parameters()]))
+            for p, g in zip(model.parameters(), grads):
+                p.grad = g                                              # the step's own
+        del taken
+    assert addresses == [kept.plan[0].data_ptr() for kept in recorded]
+    assert all(any(kept is own for own in m._plans.values()) for m, kept in zip(blocks, recorded))
+    assert all(len(m._plans) <= 17 for m in blocks)
+
+
+def test_copies_and_pickles_carry_no_plans():
+    layer = C.ConvLogicLayer(2, 4, complete=True, implementation="cuda")
+    layer._plans = {"left by an earlier process": (None, 0)}
+    for other in (copy.deepcopy(layer), pickle.loads(pickle.dumps(layer))):
+        assert "_plans" not in other.__dict__ and torch.equal(other.weights, layer.weights)
+    state = dict(layer.__dict__)                                       # as a pickle of an earlier version holds it
+    other = C.ConvLogicLayer.__new__(C.ConvLogicLayer)
+    other.__setstate__(state)
+    assert "_plans" not in other.__dict__
+    other.invalidate()
