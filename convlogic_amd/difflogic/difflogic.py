@@ -206,7 +206,7 @@ class LogicLayer(torch.nn.Module):
         """Drops everything derived from the wiring buffers (range check, consumer analysis, packed walk plan, reverse map, the
         trees of three layers that this one belongs to).  Needed only after writing indices_0 / indices_1 through `.data`, which
         the version counters do not see."""
-        self._wiring_checked = self._sole_cache = self._plan_cache = self._reverse_built = None
+        self._wiring_checked = self._sole_cache = self._reverse_built = None
         self._new_wiring_epoch()
         _CHECKED_BUFFERS.pop(self, None)
 
@@ -238,12 +238,17 @@ class LogicLayer(torch.nn.Module):
         return cached[1]
 
     def _eval_plan(self):
-        """Walk order of the wiring graph for the packed evaluation kernel; rebuilt when the wiring
-        buffers were modified in place or moved to another device."""
+        """Walk order of the wiring graph for the packed evaluation kernel; rebuilt when the wiring buffers were modified in
+        place or moved to another device -- in the same memory where it can be: a recorded HIP graph reads it there."""
         key = self._check_wiring()
         cached = getattr(self, "_plan_cache", None)
         if cached is None or cached[0] != key:
-            cached = (key, difflogic_hip.eval_plan(self.indices_0, self.indices_1, self.in_dim))
+            plan = difflogic_hip.eval_plan(self.indices_0, self.indices_1, self.in_dim)
+            if cached is not None and cached[1].shape == plan.shape and cached[1].device == plan.device:
+                plan = cached[1].copy_(plan)
+                if plan.is_cuda:                                     # complete before a call on another stream takes it
+                    torch.cuda.current_stream(plan.device).synchronize()
+            cached = (key, plan)
             self._plan_cache = cached
         return cached[1]
 

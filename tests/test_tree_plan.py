@@ -125,3 +125,16 @@ def test_the_tables_of_a_recorded_step_stay(layers):
     plan.fits = lambda: True
     layers[0].invalidate()
     assert fc_tree.tree_plan(*layers) is plan
+
+
+def test_the_walk_plan_of_a_recorded_packed_layer_stays():
+    from convlogic_amd.hip import difflogic_hip
+    layer, other = chain(0)[0], chain(1)[0]
+    address = layer._eval_plan().data_ptr()
+    for change in (lambda: layer.load_state_dict(layer.state_dict()), lambda: layer.load_state_dict(other.state_dict()),
+                   lambda: layer.indices_0.copy_(swapped(layer)), layer.invalidate):
+        change()
+        keep = [torch.full((40,), -1, dtype=torch.int32) for _ in range(64)]   # (takes freed memory)
+        assert layer._eval_plan().data_ptr() == address
+        assert torch.equal(layer._eval_plan(), difflogic_hip.eval_plan(layer.indices_0, layer.indices_1, layer.in_dim))
+        del keep
