@@ -64,8 +64,8 @@ def _called_for_itself(module):
 def _tree_tail(net):
     """The last four modules of a network -- three LogicLayers and a GroupSum -- when nothing but a call of the modules
     themselves stands against evaluating them as one operation (difflogic/fc_tree.py), else None."""
-    if len(net) < 4 or _called_for_itself(net) or torch.nn.modules.module._has_any_global_hook():
-        return None
+    if type(net) is not nn.Sequential or len(net) < 4 or _called_for_itself(net) or torch.nn.modules.module._has_any_global_hook():
+        return None                                                   # (a wrapped network, or one with a forward of its own, is called)
     tail = [net[i] for i in range(len(net) - 4, len(net))]
     *layers, gs = tail
     if not all(type(m) is LogicLayer and m.implementation == "cuda" and m.grad_factor == 1.0 for m in layers) or type(gs) is not GroupSum:
@@ -87,7 +87,6 @@ def _forward(owner, x):
     last LogicLayer and GroupSum that do not run as trees run as one autograd node (`fused_tail`, default on), whose
     backward needs no GroupSum launch."""
     net = owner.network
-    n = len(net)
     tail = _tree_tail(net) if owner.__dict__.get("tree_tail", True) else None
     if isinstance(x, PackBitsTensor):
         trees = tail is not None and not any(m.training for m in (owner, *tail[0])) and x.is_cuda and x.bit_count == 64
@@ -97,7 +96,7 @@ def _forward(owner, x):
         h = _head_of(net, x)
         if (type(h) is not PackBitsTensor or h.image or h.t.shape[0] != tail[0][0].in_dim or not h.t.is_contiguous()
                 or h.t.device != tail[0][0]._parameters["weights"].device):
-            return _rest(net, n - 4, h)
+            return _rest(net, h)
         return tree_packed(tail[0], tail[1].k, h, plan)
     if not (isinstance(x, torch.Tensor) and x.is_cuda):
         return net(x)
@@ -108,17 +107,18 @@ def _forward(owner, x):
         h = _head_of(net, x)
         if _trees_take(h, tail[0][0]):
             return tree_eval(tail[0], tail[1], _feature_major(h.detach()), plan)
-        return _rest(net, n - 4, h)
+        return _rest(net, h)
     plan = tree_plan(*tail[0]) if trees and all(m.training for m in tail[0]) else None
     mode = owner.__dict__.get("prefold", True)                       # True: where it pays, "always", False
-    layers = [m for m in net if isinstance(m, (ConvLogicLayer, LogicLayer))]
     if mode:
+        layers = [m for m in net if isinstance(m, (ConvLogicLayer, LogicLayer))]
         _prefold(owner, layers if plan is None else layers[:-3], x, mode)
     if plan is not None:
         h = _head_of(net, x)
         if _trees_take(h, tail[0][0]):
             return tree_train(tail[0], tail[1], _feature_major(h), plan)
-        return _rest(net, n - 4, h)
+        return _rest(net, h)
+    n = len(net)
     if (owner.__dict__.get("fused_tail", True) and n >= 2 and isinstance(net[n - 2], LogicLayer) and isinstance(net[n - 1], GroupSum)
             and not (net._forward_hooks or net._forward_pre_hooks)):
         h = x
@@ -144,10 +144,10 @@ def _head_of(net, h):
         h = m(h)
 
 
-def _rest(net, i0, h):
-    for i, m in enumerate(net):
-        if i >= i0:
-            h = m(h)
+def _rest(net, h):
+    """the last four"""
+    for i in range(len(net) - 4, len(net)):
+        h = net[i](h)
     return h
 
 

@@ -359,3 +359,26 @@ def test_a_recording_without_the_tables_takes_the_modules():
             torch.cuda.synchronize()
             assert torch.equal(got, model.network(x))
             assert torch.equal(got, model(x))
+
+
+def test_a_wrapped_network_and_one_with_a_forward_of_its_own_are_called():
+    class Doubled(torch.nn.Sequential):
+        def forward(self, x):
+            return 2 * super().forward(x)
+
+    class Wrapped(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        def forward(self, x):
+            return self.inner(x)
+
+    torch.manual_seed(10)
+    model, x = Head().to(DEV).eval(), torch.randint(0, 2, (64, 40), device=DEV).float()
+    with torch.no_grad():
+        want, network = model(x), model.network
+        model.network = Doubled(*network)
+        assert torch.equal(model(x), 2 * want)
+        model.network = Wrapped(network)
+        assert torch.equal(model(x), want)

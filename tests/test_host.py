@@ -357,3 +357,20 @@ def test_python_path_rejects_an_index_rewired_out_of_range_through_data():
     layer.indices_0.data[3] = 8
     with pytest.raises((IndexError, RuntimeError)):
         layer(x)
+
+
+def test_a_wrapped_network_is_called():
+    # `network` inside a module that is no sequence (a data-parallel or compiling wrapper): the call goes to the wrapper
+    class Wrapped(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        def forward(self, x):
+            return self.inner(x)
+
+    torch.manual_seed(0)
+    model, x = C.ConvLogicMnistModel(k_param=1, implementation="python"), torch.randint(0, 2, (2, 1, 28, 28)).float()
+    want = [model.train()(x), model.eval()(x)]
+    model.network = Wrapped(model.network)
+    assert torch.equal(model.train()(x), want[0]) and torch.equal(model.eval()(x), want[1])
