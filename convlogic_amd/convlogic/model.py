@@ -72,6 +72,8 @@ def _tree_tail(net):
         return None
     if any(_called_for_itself(m) for m in tail) or layers[-1].out_dim % gs.k != 0 or gs.tau == 0:
         return None
+    if gs.k > 65535 or layers[0].in_dim >= 1 << 31 or layers[-1].out_dim >= 1 << 28:   # (what the tree kernels' indices hold)
+        return None
     for m in layers:
         w = m._parameters["weights"]
         if not (w.is_cuda and w.dtype == torch.float32 and w.shape == (m.out_dim, 16) and w.is_contiguous()

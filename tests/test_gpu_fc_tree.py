@@ -382,3 +382,13 @@ def test_a_wrapped_network_and_one_with_a_forward_of_its_own_are_called():
         assert torch.equal(model(x), 2 * want)
         model.network = Wrapped(network)
         assert torch.equal(model(x), want)
+
+
+def test_more_classes_than_the_tree_kernels_take():
+    # (the float class sums take no more either: they refuse, as for the modules)
+    torch.manual_seed(11)
+    model, bits = Head(140000, 70000, 70000).to(DEV).eval(), torch.rand(3, 140000, device=DEV) < 0.5
+    with torch.no_grad():
+        assert torch.equal(model(C.PackBitsTensor(bits, 64)), model.network(C.PackBitsTensor(bits, 64)))
+        with pytest.raises(RuntimeError, match="k <= 65535"):
+            model(bits.float())
