@@ -277,7 +277,8 @@ __device__ __forceinline__ void tree_store_sums(float (&v)[28], float *__restric
     if (i16 < 7) sums[(int64_t)j * 28 + 4 * i16 + 2 * o + h] = mine;
 }
 
-template <int V>
+// SUMS, ROWS: for the gradients of the logits, of the input (a frozen end and an input without a gradient need one of them).
+template <int V, bool SUMS, bool ROWS>
 __global__ __launch_bounds__(kTreeBlock) void fc_tree_backward_kernel(const float *__restrict__ x, const int32_t *__restrict__ rows,
                                                                     const int32_t *__restrict__ pos, const float *__restrict__ coef,
                                                                     const float *__restrict__ grad_out,
@@ -313,7 +314,8 @@ __global__ __launch_bounds__(kTreeBlock) void fc_tree_backward_kernel(const floa
 #pragma unroll
                 for (int q = 0; q < 8; ++q) tap[q] = v[q].v[i];
                 const TreeVals<float> tv = eval_tree(t, tap);
-                auto sums = [&](int q, float gq, float a, float b) {
+                auto add = [&](int q, float gq, float a, float b) {
+                    if constexpr (!SUMS) return;
                     const float ga = gq * a;
                     acc[4 * q] = fma_t(ga, b, acc[4 * q]);
                     acc[4 * q + 1] += ga;
@@ -321,17 +323,17 @@ __global__ __launch_bounds__(kTreeBlock) void fc_tree_backward_kernel(const floa
                     acc[4 * q + 3] += gq;
                 };
                 const float g6 = gy[i];
-                sums(6, g6, tv.mid[0], tv.mid[1]);
+                add(6, g6, tv.mid[0], tv.mid[1]);
                 const float gm[2] = {g6 * gate_da(t.g[6], tv.mid[1]), g6 * gate_db(t.g[6], tv.mid[0])};
 #pragma unroll
                 for (int m = 0; m < 2; ++m) {
                     const float la = tv.leaf[2 * m], lb = tv.leaf[2 * m + 1];
-                    sums(4 + m, gm[m], la, lb);
+                    add(4 + m, gm[m], la, lb);
                     const float gl[2] = {gm[m] * gate_da(t.g[4 + m], lb), gm[m] * gate_db(t.g[4 + m], la)};
 #pragma unroll
                     for (int n = 0; n < 2; ++n) {
                         const int q = 2 * m + n;
-                        sums(q, gl[n], tap[2 * q], tap[2 * q + 1]);
+                        add(q, gl[n], tap[2 * q], tap[2 * q + 1]);
                         v[2 * q].v[i] = gl[n] * gate_da(t.g[q], tap[2 * q + 1]);
                         v[2 * q + 1].v[i] = gl[n] * gate_db(t.g[q], tap[2 * q]);
                     }
@@ -344,18 +346,18 @@ __global__ __launch_bounds__(kTreeBlock) void fc_tree_backward_kernel(const floa
                     for (int q = 0; q < 8; ++q) asm volatile("" : "+v"(v[q].v[i + 1]));
                 }
             }
-            if (live) {
+            if (ROWS && live) {
 #pragma unroll
                 for (int q = 0; q < 8; ++q)
                     store_samples<V>(rowgrad + (int64_t)min((uint64_t)(uint32_t)pj[q], (uint64_t)total_rows - 1) * pitch + s, v[q]);
             }
         }
-        tree_store_sums(acc, sums, j, lane);
+        if constexpr (SUMS) tree_store_sums(acc, sums, j, lane);
     }
 }
 
 // Gradients of the logits, one thread per neuron of the three layers in order.  slot: where the neuron's four sums are (root * 7
-// + gate of the tree).
+// + gate of the tree).  A layer whose gradient is not wanted has a null pointer.
 struct TreeGrads {
     float *g[3];
     int64_t end[3];       // neurons of the first one, two, three layers
@@ -367,6 +369,7 @@ __global__ __launch_bounds__(256) void fc_tree_logit_grad_kernel(const float *__
     if (e >= gr.end[2]) return;
     const int layer = e < gr.end[0] ? 0 : (e < gr.end[1] ? 1 : 2);
     const int64_t n = e - (layer ? gr.end[layer - 1] : 0);
+    if (gr.g[layer] == nullptr) return;
     const float4 s = reinterpret_cast<const float4 *>(sums)[min((uint64_t)(uint32_t)slot[e], (uint64_t)slots - 1)];
     const float4 *w = reinterpret_cast<const float4 *>(probs + e * 16);
     float p[16], gi[16], dot = 0.f;
@@ -520,8 +523,10 @@ extern "C" int clg_fc_tree_backward(const float *x, const int32_t *rows, const i
 {
     const char *name = "clg_fc_tree_backward";
     if (int e = check_tree(name, in_dim, roots, k)) return e;
-    CLG_REQUIRE(x && rows && pos && slot && coef && grad_out && probs && grad0 && grad1 && grad2 && rowgrad && sums && start &&
-                    grad_x, "%s: null pointer argument", name);
+    const bool logits = grad0 || grad1 || grad2;
+    CLG_REQUIRE(x && rows && coef && grad_out && (logits || grad_x), "%s: null pointer argument", name);
+    CLG_REQUIRE(!logits || (slot && probs && sums), "%s: gradients of logits need slot, probs and sums", name);
+    CLG_REQUIRE(!grad_x || (pos && rowgrad && start), "%s: the gradient of x needs pos, rowgrad and start", name);
     CLG_REQUIRE(batch > 0 && pitch >= batch && pitch < (1ll << 28) && tau != 0.0, "%s: the row pitch must hold the batch, tau must not be zero",
                 name);
     const int vec = tree_vec(pitch, (const void *)((uintptr_t)x | (uintptr_t)rowgrad), grad_x);
@@ -530,18 +535,25 @@ extern "C" int clg_fc_tree_backward(const float *x, const int32_t *rows, const i
     const dim3 grid((unsigned)clg_ceil_div(roots, kTreeWaves));
     const dim3 ggrid((unsigned)clg_ceil_div(in_dim, kTreeWaves), (unsigned)clg_ceil_div(pitch, (int64_t)kWave * vec));
     CLG_REQUIRE(ggrid.y <= 65535, "%s: batch too large", name);
+#define CLG_TREE_K(V, SUMS, ROWS)                                                                                                \
+    hipLaunchKernelGGL((fc_tree_backward_kernel<V, SUMS, ROWS>), grid, dim3(kTreeBlock), 0, st, x, rows, pos, coef, grad_out, sums, rowgrad, \
+                       (int)roots, (int)(roots / k), (int)k, batch, pitch, (int)in_dim, 1.f / (float)tau)
 #define CLG_TREE_B(V)                                                                                                            \
     do {                                                                                                                         \
-        hipLaunchKernelGGL((fc_tree_backward_kernel<V>), grid, dim3(kTreeBlock), 0, st, x, rows, pos, coef, grad_out, sums, rowgrad, (int)roots, \
-                           (int)(roots / k), (int)k, batch, pitch, (int)in_dim, 1.f / (float)tau);                               \
-        hipLaunchKernelGGL((fc_tree_gather_kernel<V>), ggrid, dim3(kTreeBlock), 0, st, (const float *)rowgrad, start, grad_x,    \
-                           (int)in_dim, pitch, roots * 8);                                                                       \
+        if (logits && grad_x) CLG_TREE_K(V, true, true);                                                                         \
+        else if (logits) CLG_TREE_K(V, true, false);                                                                             \
+        else CLG_TREE_K(V, false, true);                                                                                         \
+        if (grad_x)                                                                                                              \
+            hipLaunchKernelGGL((fc_tree_gather_kernel<V>), ggrid, dim3(kTreeBlock), 0, st, (const float *)rowgrad, start, grad_x, \
+                               (int)in_dim, pitch, roots * 8);                                                                   \
     } while (0)
     if (vec == 1) CLG_TREE_B(1);
     else if (vec == 2) CLG_TREE_B(2);
     else CLG_TREE_B(4);
 #undef CLG_TREE_B
+#undef CLG_TREE_K
     CLG_CHECK_LAUNCH(name);
+    if (!logits) return CLG_OK;
     hipLaunchKernelGGL(fc_tree_logit_grad_kernel, dim3((unsigned)clg_ceil_div(7 * roots, 256)), dim3(256), 0, st, probs, gr, (const float *)sums, slot,
                        7 * roots);
     CLG_CHECK_LAUNCH(name);

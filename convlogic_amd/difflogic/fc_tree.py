@@ -110,9 +110,8 @@ class _TreeFunction(torch.autograd.Function):
         lib, st = _lib.load(), stream_ptr(x)
         in_dim, batch = x.shape
         coef = torch.empty((plan.roots, 28), dtype=torch.float32, device=x.device)
-        probs = torch.empty((7 * plan.roots, 16), dtype=torch.float32, device=x.device)
-        check(lib.clg_fc_tree_fold(l0.data_ptr(), l1.data_ptr(), l2.data_ptr(), plan.ids.data_ptr(), coef.data_ptr(), probs.data_ptr(),
-                                   plan.roots, 0, st))
+        probs = torch.empty((7 * plan.roots, 16), dtype=torch.float32, device=x.device) if any(ctx.needs_input_grad[1:4]) else None
+        check(lib.clg_fc_tree_fold(l0.data_ptr(), l1.data_ptr(), l2.data_ptr(), plan.ids.data_ptr(), coef.data_ptr(), _ptr(probs), plan.roots, 0, st))
         out = _tree_forward(lib, x, plan, coef, k, tau, st)
         # (probabilities, not logits, as in the modules: the logits may be updated between forward and backward; the wiring for
         # autograd's check that it was not)
@@ -126,16 +125,21 @@ class _TreeFunction(torch.autograd.Function):
         plan, k = ctx.plan, ctx.k
         grad_out = _lib.check_input(grad_out.contiguous(), "grad_out", torch.float32, (x.shape[1], k))
         _lib.check_same_device(x, grad_out)
-        in_dim, batch = x.shape
-        gx = torch.empty_like(x)
-        g0, g1, g2 = (torch.empty((n * plan.roots, 16), dtype=torch.float32, device=x.device) for n in (4, 2, 1))
-        scratch = torch.empty((plan.roots * (8 * batch + 28),), dtype=torch.float32, device=x.device)   # rowgrad, then sums
-        rowgrad, sums = scratch.data_ptr(), scratch.data_ptr() + plan.roots * 8 * batch * 4
+        (in_dim, batch), roots = x.shape, plan.roots
+        need_x, need = ctx.needs_input_grad[0], ctx.needs_input_grad[1:4]
+        gx = torch.empty_like(x) if need_x else None
+        grads = [torch.empty((n * roots, 16), dtype=torch.float32, device=x.device) if needed else None for n, needed in zip((4, 2, 1), need)]
+        rows = 8 * roots * batch if need_x else 0
+        scratch = torch.empty((rows + 28 * roots,), dtype=torch.float32, device=x.device)       # rowgrad, then sums
         check(_lib.load().clg_fc_tree_backward(
-            x.data_ptr(), plan.rows.data_ptr(), plan.pos.data_ptr(), plan.slot.data_ptr(), coef.data_ptr(), grad_out.data_ptr(),
-            probs.data_ptr(), g0.data_ptr(), g1.data_ptr(), g2.data_ptr(), rowgrad, sums, start.data_ptr(),
-            gx.data_ptr(), in_dim, plan.roots, k, batch, batch, float(ctx.tau), stream_ptr(x)))
-        return gx, g0, g1, g2, None, None, None, None, None
+            x.data_ptr(), plan.rows.data_ptr(), plan.pos.data_ptr(), plan.slot.data_ptr(), coef.data_ptr(), grad_out.data_ptr(), _ptr(probs),
+            *(_ptr(g) for g in grads), scratch.data_ptr(), scratch.data_ptr() + 4 * rows, start.data_ptr(), _ptr(gx), in_dim, roots, k, batch,
+            batch, float(ctx.tau), stream_ptr(x)))
+        return gx, *grads, None, None, None, None, None
+
+
+def _ptr(t):
+    return None if t is None else t.data_ptr()
 
 
 def _tree_forward(lib, x, plan, coef, k, tau, st):

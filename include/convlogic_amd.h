@@ -537,7 +537,8 @@ int64_t clg_fc_tree_partial_elems(int64_t roots, int64_t k, int64_t batch, int64
 int clg_fc_tree_forward(const float *x, const int32_t *rows, const float *coef, float *partial, float *out, int64_t in_dim,
                         int64_t roots, int64_t k, int64_t batch, int64_t pitch, double tau, void *stream);
 /* grad_out [batch, k] -> gradients of the three layers' logits and grad_x [in_dim, pitch]; scratch: rowgrad [8 roots, pitch],
- * sums [roots, 28]; probs and coef as clg_fc_tree_fold left them */
+ * sums [roots, 28]; probs and coef as clg_fc_tree_fold left them.  A gradient that is not wanted is NULL; without grad_x pos,
+ * rowgrad and start are not read, without the other three slot, probs and sums. */
 int clg_fc_tree_backward(const float *x, const int32_t *rows, const int32_t *pos, const int32_t *slot, const float *coef,
                          const float *grad_out, const float *probs, float *grad0, float *grad1, float *grad2, float *rowgrad,
                          float *sums, const int64_t *start, float *grad_x, int64_t in_dim,

@@ -392,3 +392,30 @@ def test_more_classes_than_the_tree_kernels_take():
         assert torch.equal(model(C.PackBitsTensor(bits, 64)), model.network(C.PackBitsTensor(bits, 64)))
         with pytest.raises(RuntimeError, match="k <= 65535"):
             model(bits.float())
+
+
+@pytest.mark.parametrize("batch", [3, 66, 256])
+@pytest.mark.parametrize("wanted", [(1, 0, 0, 0), (0, 1, 1, 1), (0, 0, 1, 0), (1, 1, 0, 1)])
+def test_gradients_that_are_not_wanted_are_not_made(wanted, batch):
+    layers, gs = tail(40, 130, 10, batch)
+    x, go = torch.rand(40, batch, device=DEV), torch.randn(batch, 10, device=DEV)
+    inputs = [x] + [m.weights for m in layers]
+    results = []
+    for some in ((1, 1, 1, 1), wanted):
+        for t, want in zip(inputs, some):
+            t.grad = None
+            t.requires_grad_(bool(want))
+        fc_tree.tree_train(layers, gs, x, fc_tree.tree_plan(*layers)).backward(go)
+        results.append([t.grad for t in inputs])
+    for all_of_them, some, want in zip(*results, wanted):
+        assert torch.equal(all_of_them, some) if want else some is None
+
+
+def test_a_frozen_end_allocates_no_gradients():
+    layers, gs = tail(40, 1300, 10, 1)
+    x, go = torch.rand(40, 256, device=DEV), torch.randn(256, 10, device=DEV)
+    y = fc_tree.tree_train(layers, gs, x, fc_tree.tree_plan(*layers))
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    y.backward(go)                                                     # x needs no gradient: no operand gradients [8 roots, batch]
+    assert torch.cuda.max_memory_allocated() - before < 8 * 1300 * 256 * 4
