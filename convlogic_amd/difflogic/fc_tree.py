@@ -91,15 +91,25 @@ def _make(first, second, third, keys):
 
 def refresh(layer):
     """Makes the tables of the plans that `layer` belongs to again (a state was loaded into it): a step that was recorded with
-    them replays the loaded wiring.  In the stream's order, no wait; the next tree_plan() looks at the result."""
+    them replays the loaded wiring.  In the stream's order; the next tree_plan() looks at the result.  A wiring that the next
+    call refuses (load_state_dict(assign=True) takes any type and stride) is not read: the tables stay as they were."""
     with _BUILDING:
         for first, entries in list(_PLANS.items()):
             for e in entries:
                 second, third = e.second(), e.third()
                 if e.plan is None or second is None or third is None or layer not in (first, second, third):
                     continue
-                if all(t.device == e.plan.device for t in wiring_of(first, second, third)):
+                if all(t.device == e.plan.device for t in wiring_of(first, second, third)) and _checked(first, second, third):
                     e.plan.build(first, second, third)
+
+
+def _checked(*layers):
+    try:
+        for m in layers:
+            m._check_wiring()
+    except ValueError:
+        return False
+    return True
 
 
 class _TreeFunction(torch.autograd.Function):

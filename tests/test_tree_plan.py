@@ -21,6 +21,7 @@ class Noted:
 
     def build(self, *layers):
         self.wiring = [t.clone() for m in layers for t in (m.indices_0, m.indices_1)]
+        self.start, self.flat = layers[0].given_x_indices_of_y_start.clone(), layers[0].given_x_indices_of_y.clone()
 
     def of(self, layers):
         return all(torch.equal(t, w) for t, w in zip((t for m in layers for t in (m.indices_0, m.indices_1)), self.wiring))
@@ -108,6 +109,32 @@ def test_a_loaded_wiring_and_copies(layers):
         m.load_state_dict(o.state_dict())
         assert plan.of(layers)                                          # at once: a recorded step reads these tables
     assert fc_tree.tree_plan(*layers) is plan
+
+
+@pytest.mark.parametrize("at", [0, 1, 2])
+def test_a_loaded_wiring_that_is_refused_is_not_read(layers, at):
+    # load_state_dict(assign=True) takes buffers of any type and stride: the tables are made from what a call accepts alone
+    plan = fc_tree.tree_plan(*layers)
+    before = copy.deepcopy(layers)
+    for name in ("indices_0", "indices_1", "given_x_indices_of_y_start", "given_x_indices_of_y"):
+        good = {k: v.clone() for k, v in layers[at].state_dict().items()}
+        for bad in (good[name].int(), good[name].repeat_interleave(2)[::2], torch.full_like(good[name], 1 << 40)):
+            if bad.dtype == torch.int64 and bad.is_contiguous() and name.startswith("given"):
+                continue                                               # (these lists are made again from the wiring)
+            layers[at].load_state_dict({**good, name: bad}, assign=True)
+            assert plan.of(before)
+            with pytest.raises(ValueError, match=name if name.startswith("given") else "indices"):
+                fc_tree.tree_plan(*layers)
+        layers[at].load_state_dict(good, assign=True)
+        assert fc_tree.tree_plan(*layers) is plan and plan.of(before)
+
+
+def test_the_reverse_lists_of_a_loaded_wiring(layers):
+    # a state without the reverse lists: the tables are made with the lists of the loaded wiring
+    plan = fc_tree.tree_plan(*layers)
+    state = {k: v for k, v in chain(1)[0].state_dict().items() if not k.startswith("given")}
+    layers[0].load_state_dict(state, strict=False)
+    assert plan.of(layers) and torch.equal(plan.start, chain(1)[0].given_x_indices_of_y_start) and torch.equal(plan.flat, chain(1)[0].given_x_indices_of_y)
 
 
 def test_the_tables_of_a_recorded_step_stay(layers):
