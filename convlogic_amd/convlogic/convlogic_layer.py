@@ -319,9 +319,15 @@ class ConvLogicLayer(nn.Module):
         super()._load_from_state_dict(*args, **kwargs)
         self.invalidate()
         sel = self._buffers["selection"]
-        for (shape, dtype, device, _), kept in self.__dict__.get("_plans", {}).items():
-            if kept.recorded and sel.device == device:               # a recorded step replays the loaded selection
-                kept.make(types.SimpleNamespace(shape=shape, dtype=dtype, device=device), sel.contiguous(), self)
+        recorded = [(key, kept) for key, kept in self.__dict__.get("_plans", {}).items() if kept.recorded and sel.device == key[2]]
+        if not recorded:
+            return
+        try:
+            self._check_selection()
+        except ValueError:                                           # the next call raises; the plans stay as they were
+            return
+        for (shape, dtype, device, _), kept in recorded:             # a recorded step replays the loaded selection
+            kept.make(types.SimpleNamespace(shape=shape, dtype=dtype, device=device), sel.contiguous(), self)
 
     def forward(self, x):
         if isinstance(x, PackBitsTensor):

@@ -374,3 +374,25 @@ def test_a_wrapped_network_is_called():
     want = [model.train()(x), model.eval()(x)]
     model.network = Wrapped(model.network)
     assert torch.equal(model.train()(x), want[0]) and torch.equal(model.eval()(x), want[1])
+
+
+def test_a_loaded_selection_is_checked_before_recorded_plans_are_made_from_it():
+    class Kept:
+        recorded, made = True, 0
+
+        def make(self, like, sel, layer):
+            assert sel.dtype == torch.int32 and sel.is_contiguous()
+            self.made += 1
+
+    torch.manual_seed(0)
+    layer = C.ConvLogicLayer(2, 4, complete=True, implementation="python")
+    kept = Kept()
+    layer._plans = {((8, 2, 8, 8), torch.float32, torch.device("cpu"), 0): kept}
+    good = {k: v.clone() for k, v in layer.state_dict().items()}
+    for bad in (good["selection"].long(), good["selection"] + (2 << 16)):    # another type; a channel that is not there
+        layer.load_state_dict({**good, "selection": bad}, assign=True)
+        assert kept.made == 0
+        with pytest.raises(ValueError, match="selection"):
+            layer._check_selection()
+    layer.load_state_dict(good)
+    assert kept.made == 1
