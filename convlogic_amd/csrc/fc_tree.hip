@@ -301,6 +301,13 @@ __global__ __launch_bounds__(kTreeBlock) void fc_tree_backward_kernel(const floa
             const bool live = s < pitch;
             Samples<V> v[8];
             tree_rows<V>(x, rows, j, in_dim, pitch, live ? s : 0, v);
+            if (s0 + kWave * V > batch) {                             // values without a sample: zeros, whatever the row holds there
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+#pragma unroll
+                    for (int i = 0; i < V; ++i) v[q].v[i] = s + i < batch ? v[q].v[i] : 0.f;
+                }
+            }
             float gy[V];
 #pragma unroll
             for (int i = 0; i < V; ++i) {

@@ -419,3 +419,28 @@ def test_a_frozen_end_allocates_no_gradients():
     before = torch.cuda.memory_allocated()
     y.backward(go)                                                     # x needs no gradient: no operand gradients [8 roots, batch]
     assert torch.cuda.max_memory_allocated() - before < 8 * 1300 * 256 * 4
+
+
+@pytest.mark.parametrize("batch,pitch", [(3, 64), (100, 128), (60, 96), (200, 256), (257, 512), (300, 304)])
+def test_what_a_row_holds_behind_the_batch_adds_nothing(batch, pitch):
+    from convlogic_amd.hip import _lib
+    lib, ptr = _lib.load(), lambda t: t.data_ptr()
+    layers, _ = tail(40, 130, 10, batch)
+    plan, (in_dim, roots, k) = fc_tree.tree_plan(*layers), (40, 130, 10)
+    x, go = torch.rand(in_dim, pitch, device=DEV), torch.randn(batch, k, device=DEV)
+    start = layers[0].given_x_indices_of_y_start
+    results = []
+    for behind in (0.0, float("nan"), float("inf")):
+        x[:, batch:] = behind
+        coef, probs, out = (torch.empty(*s, device=DEV) for s in ((roots, 28), (7 * roots, 16), (batch, k)))
+        _lib.check(lib.clg_fc_tree_fold(*(ptr(m.weights) for m in layers), ptr(plan.ids), ptr(coef), ptr(probs), roots, 0, _lib.stream_ptr(x)))
+        partial = torch.empty(lib.clg_fc_tree_partial_elems(roots, k, batch, pitch), device=DEV)
+        _lib.check(lib.clg_fc_tree_forward(ptr(x), ptr(plan.rows), ptr(coef), ptr(partial), ptr(out), in_dim, roots, k, batch, pitch, 3.0, _lib.stream_ptr(x)))
+        grads, gx = [torch.empty(n * roots, 16, device=DEV) for n in (4, 2, 1)], torch.empty(in_dim, pitch, device=DEV)
+        rowgrad, sums = torch.empty(8 * roots, pitch, device=DEV), torch.empty(roots, 28, device=DEV)
+        _lib.check(lib.clg_fc_tree_backward(ptr(x), ptr(plan.rows), ptr(plan.pos), ptr(plan.slot), ptr(coef), ptr(go), ptr(probs), *map(ptr, grads),
+                                            ptr(rowgrad), ptr(sums), ptr(start), ptr(gx), in_dim, roots, k, batch, pitch, 3.0, _lib.stream_ptr(x)))
+        results.append([out, *grads, gx[:, :batch].clone()])
+    for other in results[1:]:
+        for i, (a, b) in enumerate(zip(results[0], other)):
+            assert torch.isfinite(a).all() and torch.equal(a, b), f"result {i}"
