@@ -22,7 +22,9 @@
 // into halo elements that are never read back).  The order of additions is program order.
 #include <stdlib.h>
 
+#include <memory>
 #include <mutex>
+#include <new>
 
 #include "conv_tile.h"
 
@@ -1048,7 +1050,8 @@ enum BwdXMode { kBwdXGather = 0, kBwdXTiled = 1, kBwdXDirect = 2 };
 
 // Tiled (input image in LDS) when a wavefront pass is reasonably full there; the direct kernel when the
 // image does not fit or fills at least twice as many lanes; the per-element gather for everything else.
-BwdXMode choose_backward_x(const Geom &g, int elem, TilePlan *p, int *sample_elems)
+// long_lists: some channel's kernel list is known to be much longer than the average, see lists_are_long.
+BwdXMode choose_backward_x(const Geom &g, int elem, TilePlan *p, int *sample_elems, bool long_lists = false)
 {
     TilePlan pt, pd;
     int se = 0;
@@ -1067,7 +1070,10 @@ BwdXMode choose_backward_x(const Geom &g, int elem, TilePlan *p, int *sample_ele
     // plane ([64,16,8,8] -> 256 87 -> 61, at 8 channels 86 -> 95); up to 64 from 2048 owners on (178 -> 161 at
     // [64,32,28,28] -> 256, but 102 -> 123 at half its channels); longer chains are the tiled kernel's ([16,32,28,28] -> 512: 139 -> 215).
     const int64_t chain = avg_hits * clg_ceil_div((int64_t)pd.G * I, kWave);
-    const bool short_chain = elem == 4 && g.cin >= 4 && (chain <= 16 || (g.cin >= 16 && ((chain <= 32 && owners >= 64) || (chain <= 64 && owners >= 2048))));
+    // (The price is memory: the padded copy of x that the direct kernel reads lives from the forward call to the backward one.)
+    // All of this goes by the average list, as random taps make them; one channel's long list is one wavefront's chain, so
+    // where the lists are known it is not taken for those.
+    const bool short_chain = !long_lists && elem == 4 && g.cin >= 4 && (chain <= 16 || (g.cin >= 16 && ((chain <= 32 && owners >= 64) || (chain <= 64 && owners >= 2048))));
     bool use_direct = direct && (!tiled || lanes(pd) >= 2 * lanes(pt) || (owners >= 4096 && avg_hits <= 16) || short_chain);
     if (const char *e = clg_knob(K_BWDX_DIRECT)) use_direct = direct && (atoi(e) != 0 || !tiled);
     if (use_direct) {
@@ -1080,6 +1086,24 @@ BwdXMode choose_backward_x(const Geom &g, int elem, TilePlan *p, int *sample_ele
         return kBwdXTiled;
     }
     return kBwdXGather;
+}
+
+// A channel whose list is so long that the tiled kernel is the better one: not a list as random taps make them (of the average m
+// one in a million has more than 2 m + 8 kernels), and its chain grows by more than what the direct kernel is ahead by.
+// Measured with up to all kernels on one channel: a kernel of the list takes 0.83 us per block of 64 cells in the direct kernel and twice
+// that in the tiled one, which shares a list among `spread` wavefronts; at lists of random taps the direct kernel is 7 to 72 us ahead
+// where spread is above 2, the 40 us taken here are at most an eighth off either way ([64,32,28,28] -> 256 at a list of 40:
+// 192 / 171 us direct / tiled, of 136: 507 / 277; [32,64,14,14] -> 512 at 40: 80 / 142, at 264: 261 / 230).
+bool lists_are_long(const Geom &g, int elem, const int32_t *count)
+{
+    TilePlan pt, pd;
+    int se = 0;
+    if (!plan_backward_x(g, elem, &pt) || !plan_backward_x_direct(g, elem, &pd, &se)) return false;
+    int64_t longest = 0;
+    for (int ch = 0; ch < g.cin; ++ch) longest = count[2 * ch] > longest ? count[2 * ch] : longest;
+    const int64_t avg = (2 * (int64_t)g.c) / g.cin, blocks = clg_ceil_div((int64_t)pd.G * (g.ho / 2) * (g.wo / 2), kWave);
+    const int64_t spread = (int64_t)pt.hit_split * pt.hsw * pt.bands;
+    return longest > 2 * avg + 8 && (longest - avg) * blocks * (spread - 2) > 48 * spread;
 }
 
 size_t bwd_x_direct_xp_off(const BwdScratch &lay) { return (lay.total + 255) & ~(size_t)255; }
@@ -1444,16 +1468,20 @@ int clg_allow_lds(const void *kernel, size_t bytes, const char *name)
     return CLG_OK;
 }
 
-extern "C" int64_t clg_convblock_backward_x_scratch_bytes(int dtype, const clg_conv_geom *gg)
+static int64_t backward_x_scratch_bytes(const char *name, int dtype, const clg_conv_geom *gg, bool long_lists)
 {
     Geom g;
-    if (clg_convblock_check(gg, &g, dtype, "clg_convblock_backward_x_scratch_bytes")) return -1;
+    if (clg_convblock_check(gg, &g, dtype, name)) return -1;
     TilePlan p;
     int se = 0;
-    const BwdXMode mode = choose_backward_x(g, elem_size(dtype), &p, &se);
+    const BwdXMode mode = choose_backward_x(g, elem_size(dtype), &p, &se, long_lists);
     const BwdScratch lay = bwd_scratch_layout(g, elem_size(dtype), mode == kBwdXTiled ? p.hit_split : 1);
     if (mode == kBwdXDirect) return (int64_t)(bwd_x_direct_xp_off(lay) + (size_t)se * g.n * elem_size(dtype));
     return (int64_t)lay.total;
+}
+extern "C" int64_t clg_convblock_backward_x_scratch_bytes(int dtype, const clg_conv_geom *gg)
+{
+    return backward_x_scratch_bytes("clg_convblock_backward_x_scratch_bytes", dtype, gg, false);
 }
 
 // What the tiled input gradient sets up for a padded weight gradient that follows in the same call: its prepare launch
@@ -1479,14 +1507,14 @@ PadJob<T> share_from_tiled(const Geom &g, const TilePlan &p, const void *x, void
 
 static int convblock_backward_x_impl(int dtype, const clg_conv_geom *gg, const void *grad_y, const void *x, const void *w,
                                      const int32_t *selection, const uint8_t *argmax, void *grad_x, void *scratch, void *stream,
-                                     SharedPad *shared, void *w_scratch = nullptr, const PlanView *pv = nullptr)
+                                     SharedPad *shared, void *w_scratch = nullptr, const PlanView *pv = nullptr, bool long_lists = false)
 {
     Geom g;
     if (int e = clg_convblock_check(gg, &g, dtype, "clg_convblock_backward_x")) return e;
     CLG_REQUIRE(grad_y && x && w && selection && argmax && grad_x && scratch, "clg_convblock_backward_x: null pointer argument");
     TilePlan p;
     int se = 0;
-    const BwdXMode mode = choose_backward_x(g, elem_size(dtype), &p, &se);
+    const BwdXMode mode = choose_backward_x(g, elem_size(dtype), &p, &se, long_lists);
     hipStream_t st = clg_stream(stream);
     if (mode == kBwdXTiled) {
         BwdTables tb;
@@ -1601,18 +1629,26 @@ static int convblock_backward_4x4(int dtype, const Geom &g, const void *grad_y, 
                                       tb.count, tb.hits, grad_x, st, name);
 }
 
-extern "C" int64_t clg_convblock_backward_scratch_bytes(int dtype, const clg_conv_geom *gg)
+static int64_t backward_scratch_bytes(const char *name, int dtype, const clg_conv_geom *gg, bool long_lists)
 {
-    const int64_t a = clg_convblock_backward_x_scratch_bytes(dtype, gg), b = clg_convblock_backward_w_scratch_bytes(dtype, gg);
+    const int64_t a = backward_x_scratch_bytes(name, dtype, gg, long_lists), b = clg_convblock_backward_w_scratch_bytes(dtype, gg);
     if (a < 0 || b < 0) return -1;
     int64_t total = ((a + 255) & ~255ll) + b;
     Geom g;
-    if (clg_convblock_check(gg, &g, dtype, "clg_convblock_backward_scratch_bytes")) return -1;
+    if (clg_convblock_check(gg, &g, dtype, name)) return -1;
     if (backward_4x4_wanted(g)) {
         const int64_t small = (int64_t)(backward_4x4_tg_off(g, dtype) + clg_convblock_backward_4x4_tg_bytes(dtype, g));
         if (small > total) total = small;
     }
     return total;
+}
+extern "C" int64_t clg_convblock_backward_scratch_bytes(int dtype, const clg_conv_geom *gg)
+{
+    return backward_scratch_bytes("clg_convblock_backward_scratch_bytes", dtype, gg, false);
+}
+extern "C" int64_t clg_convblock_backward_planned_scratch_bytes(int dtype, const clg_conv_geom *gg, int64_t signature)
+{
+    return backward_scratch_bytes("clg_convblock_backward_planned_scratch_bytes", dtype, gg, (signature & 1) != 0);
 }
 
 extern "C" int clg_convblock_backward(int dtype, const clg_conv_geom *gg, const void *grad_y, const void *x, const void *w,
@@ -1685,7 +1721,8 @@ struct PlanInfo {
     size_t total;
     int64_t signature;
 };
-PlanInfo plan_info(const Geom &g, int dtype)
+// long_lists is the lowest bit of the signature (0 where it makes no difference), so a planned call finds the kernels again.
+PlanInfo plan_info(const Geom &g, int dtype, bool long_lists)
 {
     PlanInfo pi;
     const int elem = elem_size(dtype);
@@ -1694,7 +1731,14 @@ PlanInfo plan_info(const Geom &g, int dtype)
         TilePlan p;
         int se = 0;
         mode = (int)choose_backward_x(g, elem, &p, &se);
+        if (long_lists) {
+            const int other = (int)choose_backward_x(g, elem, &p, &se, true);
+            long_lists = other != mode;
+            mode = other;
+        }
         if (mode != kBwdXGather) rs = p.rs, chs = p.chs;
+    } else {
+        long_lists = false;
     }
     pi.lay = bwd_scratch_layout(g, elem, 1);
     pi.rs = rs, pi.chs = chs;
@@ -1706,7 +1750,7 @@ PlanInfo plan_info(const Geom &g, int dtype)
         h ^= (uint64_t)f;
         h *= 1099511628211ull;
     }
-    pi.signature = (int64_t)(h & 0x7fffffffffffffffull);
+    pi.signature = (int64_t)(h & 0x7ffffffffffffffeull) | (long_lists ? 1 : 0);
     return pi;
 }
 }  // namespace
@@ -1715,25 +1759,47 @@ extern "C" int64_t clg_convblock_plan_bytes(int dtype, const clg_conv_geom *gg)
 {
     Geom g;
     if (clg_convblock_check(gg, &g, dtype, "clg_convblock_plan_bytes")) return -1;
-    return (int64_t)plan_info(g, dtype).total;
+    return (int64_t)plan_info(g, dtype, false).total;                 // (the same tables for lists of any length)
+}
+
+// lists and tap offsets by the set-up launch of the unplanned path (no weights: nothing is folded)
+static int make_plan(const Geom &g, int dtype, const PlanInfo &pi, const int32_t *selection, void *plan, hipStream_t st)
+{
+    if (dtype == CLG_F32) return launch_prepare<float>(g, pi.lay, pi.rs, pi.chs, nullptr, selection, plan, st, no_pad_job<float>());
+    return launch_prepare<double>(g, pi.lay, pi.rs, pi.chs, nullptr, selection, plan, st, no_pad_job<double>());
+}
+
+extern "C" int clg_convblock_plan_lists(int dtype, const clg_conv_geom *gg, const int32_t *selection, void *plan, int lists,
+                                        int64_t *signature, void *stream)
+{
+    const char *name = "clg_convblock_plan_lists";
+    Geom g;
+    if (int e = clg_convblock_check(gg, &g, dtype, name)) return e;
+    CLG_REQUIRE(selection && plan && signature, "%s: null pointer argument", name);
+    CLG_REQUIRE(lists >= CLG_LISTS_LOOK && lists <= CLG_LISTS_LONG, "%s: lists must be a CLG_LISTS_ value, got %d", name, lists);
+    hipStream_t st = clg_stream(stream);
+    const PlanInfo pi = plan_info(g, dtype, lists == CLG_LISTS_LONG);
+    if (int e = make_plan(g, dtype, pi, selection, plan, st)) return e;
+    *signature = pi.signature;
+    if (lists != CLG_LISTS_LOOK) return CLG_OK;
+    const PlanInfo other = plan_info(g, dtype, true);
+    if (other.signature == pi.signature) return CLG_OK;
+    const size_t entries = 2 * (size_t)g.cin;
+    const std::unique_ptr<int32_t[]> count(new (std::nothrow) int32_t[entries]);
+    CLG_REQUIRE(count != nullptr, "%s: out of host memory", name);
+    hipError_t err = hipMemcpyAsync(count.get(), reinterpret_cast<unsigned char *>(plan) + pi.lay.count_off, entries * 4, hipMemcpyDeviceToHost, st);
+    if (err == hipSuccess) err = hipStreamSynchronize(st);
+    CLG_REQUIRE(err == hipSuccess, "%s: the lists cannot be read (%s); inside a recording lists cannot be CLG_LISTS_LOOK", name, hipGetErrorString(err));
+    if (!lists_are_long(g, elem_size(dtype), count.get())) return CLG_OK;
+    if (int e = make_plan(g, dtype, other, selection, plan, st)) return e;
+    *signature = other.signature;
+    return CLG_OK;
 }
 
 extern "C" int clg_convblock_plan(int dtype, const clg_conv_geom *gg, const int32_t *selection, void *plan, int64_t *signature,
                                   void *stream)
 {
-    Geom g;
-    if (int e = clg_convblock_check(gg, &g, dtype, "clg_convblock_plan")) return e;
-    CLG_REQUIRE(selection && plan && signature, "clg_convblock_plan: null pointer argument");
-    const PlanInfo pi = plan_info(g, dtype);
-    hipStream_t st = clg_stream(stream);
-    // lists and tap offsets by the set-up launch of the unplanned path (no weights: nothing is folded)
-    if (dtype == CLG_F32) {
-        if (int e = launch_prepare<float>(g, pi.lay, pi.rs, pi.chs, nullptr, selection, plan, st, no_pad_job<float>())) return e;
-    } else {
-        if (int e = launch_prepare<double>(g, pi.lay, pi.rs, pi.chs, nullptr, selection, plan, st, no_pad_job<double>())) return e;
-    }
-    *signature = pi.signature;
-    return CLG_OK;
+    return clg_convblock_plan_lists(dtype, gg, selection, plan, CLG_LISTS_SHORT, signature, stream);
 }
 
 // One sample of the padded copy the planned backward pass reads when its input gradient is the direct kernel, else 0.
@@ -1756,7 +1822,8 @@ static int backward_planned_impl(const char *name, int dtype, const clg_conv_geo
     const bool wrt_logits = (flags & CLG_BWD_WRT_LOGITS) != 0, fm = (flags & CLG_BWD_GY_FEATURE_MAJOR) != 0;
     CLG_REQUIRE(!fm || clg_convblock_fm_supported(dtype, gg), "%s: CLG_BWD_GY_FEATURE_MAJOR needs a shape for which "
                 "clg_convblock_fm_supported() holds (4x4 images, 3x3 kernel, stride 1, padding 1, n >= 32)", name);
-    const PlanInfo pi = plan_info(g, dtype);
+    const bool long_lists = (signature & 1) != 0;
+    const PlanInfo pi = plan_info(g, dtype, long_lists);
     CLG_REQUIRE(signature == pi.signature, "%s: the plan was made for another geometry, element type or kernel choice (make a new one "
                 "with clg_convblock_plan; the CLG_* knobs are part of the choice)", name);
     unsigned char *pb = reinterpret_cast<unsigned char *>(plan);
@@ -1771,12 +1838,13 @@ static int backward_planned_impl(const char *name, int dtype, const clg_conv_geo
         g.y_fm = fm ? 1 : 0;
         return convblock_backward_4x4(dtype, g, grad_y, x, w, selection, argmax, grad_x, grad_w, scratch, stream, probs, name, &pv);
     }
-    const int64_t a = clg_convblock_backward_x_scratch_bytes(dtype, gg);
+    const int64_t a = backward_x_scratch_bytes(name, dtype, gg, long_lists);
     if (a < 0) return CLG_EINVAL;
     SharedPad shared;
     void *w_scratch = reinterpret_cast<unsigned char *>(scratch) + ((a + 255) & ~255ll);
     if (grad_x != nullptr)
-        if (int e = convblock_backward_x_impl(dtype, gg, grad_y, x, w, selection, argmax, grad_x, scratch, stream, &shared, w_scratch, &pv))
+        if (int e = convblock_backward_x_impl(dtype, gg, grad_y, x, w, selection, argmax, grad_x, scratch, stream, &shared, w_scratch, &pv,
+                                              long_lists))
             return e;
     return convblock_backward_w_impl(dtype, gg, grad_y, x, w, selection, argmax, grad_w, w_scratch, stream, probs, name, &shared);
 }
@@ -1797,8 +1865,8 @@ extern "C" int clg_convblock_backward_planned_padded(int dtype, const clg_conv_g
     const char *name = "clg_convblock_backward_planned_padded";
     Geom g;
     if (int e = clg_convblock_check(gg, &g, dtype, name)) return e;
-    CLG_REQUIRE(padded == nullptr || (grad_x != nullptr && clg_convblock_backward_padded_sample_elems(dtype, g) > 0),
-                "%s: a padded copy is only taken with grad_x and where clg_convblock_padded_elems() is not 0", name);
+    CLG_REQUIRE(padded == nullptr || (grad_x != nullptr && clg_convblock_backward_padded_sample_elems(dtype, g) > 0 && (signature & 1) == 0),
+                "%s: a padded copy is only taken with grad_x, where clg_convblock_padded_elems() is not 0 and for a plan of short lists", name);
     return backward_planned_impl(name, dtype, gg, grad_y, x, w, folded, padded, selection, argmax, plan, signature, grad_x, grad_w, flags,
                                  scratch, stream);
 }

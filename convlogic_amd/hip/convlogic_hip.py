@@ -390,12 +390,16 @@ def full_convlogic_forward_logits(x, logits, selection, stride_h, stride_w, pad_
     return y, argmax, probs
 
 
-def make_backward_plan(x, c_out, selection, stride_h, stride_w, pad_h, pad_w, kernel_h, kernel_w, into=None):
+LISTS_LOOK, LISTS_SHORT = -1, 0                                       # CLG_LISTS_* (include/convlogic_amd.h)
+
+
+def make_backward_plan(x, c_out, selection, stride_h, stride_w, pad_h, pad_w, kernel_h, kernel_w, into=None, lists=LISTS_SHORT):
     """Per-layer plan of the block's backward pass for inputs of x's shape and dtype: -> (plan bytes on the device,
     signature).  Depends only on the selection and the geometry; built once and reused by every
     full_convlogic_backward_planned() call of the layer (the reverse map the reference's LogicLayer builds at
     construction, src/difflogic/difflogic.py:71-87, for the fused block).  Of x only shape, dtype and device are looked at.
-    into: the bytes of an earlier plan for the same geometry, which are written again."""
+    into: the bytes of an earlier plan for the same geometry, which are written again.  lists: LISTS_SHORT, LISTS_LOOK (waits for the
+    stream) or lists_of() an earlier plan."""
     if isinstance(x, torch.Tensor):
         check_input(x, "x")
     if len(x.shape) != 4:
@@ -407,8 +411,13 @@ def make_backward_plan(x, c_out, selection, stride_h, stride_w, pad_h, pad_w, ke
     nbytes = lib.clg_convblock_plan_bytes(dt, ctypes.byref(g))
     plan = into if into is not None and into.numel() >= nbytes and into.device == x.device else _scratch(nbytes, x.device)
     sig = ctypes.c_int64(0)
-    check(lib.clg_convblock_plan(dt, ctypes.byref(g), selection.data_ptr(), plan.data_ptr(), ctypes.byref(sig), stream_ptr(x)))
+    check(lib.clg_convblock_plan_lists(dt, ctypes.byref(g), selection.data_ptr(), plan.data_ptr(), lists, ctypes.byref(sig), stream_ptr(x)))
     return plan, sig.value
+
+
+def lists_of(signature):
+    """What a plan's kernels were chosen for: LISTS_SHORT, or 1 for a channel that many kernels read (they take no padded copy of x)."""
+    return signature & 1
 
 
 def full_convlogic_backward_planned(grad_y, x, weight, folded, argmax, selection, plan, signature, stride_h, stride_w, pad_h, pad_w,
@@ -437,7 +446,7 @@ def full_convlogic_backward_planned(grad_y, x, weight, folded, argmax, selection
         check_input(plan, "plan", torch.uint8)
         if plan.numel() < lib.clg_convblock_plan_bytes(dt, ctypes.byref(g)):
             raise RuntimeError("plan is smaller than clg_convblock_plan_bytes() for this geometry")
-    scratch = _scratch(lib.clg_convblock_backward_scratch_bytes(dt, ctypes.byref(g)), x.device)
+    scratch = _scratch(lib.clg_convblock_backward_planned_scratch_bytes(dt, ctypes.byref(g), signature), x.device)
     gx = torch.empty_like(x) if need_grad_x else None
     gw = torch.empty((g.c_out, 7, 16), dtype=x.dtype, device=x.device)
     flags = (1 if wrt_logits else 0) | (2 if feature_major else 0)

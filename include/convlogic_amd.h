@@ -461,11 +461,22 @@ int clg_convblock_backward_fm(int dtype, const clg_conv_geom *g, const void *gra
  * only read a plan. */
 int64_t clg_convblock_plan_bytes(int dtype, const clg_conv_geom *g);
 int clg_convblock_plan(int dtype, const clg_conv_geom *g, const int32_t *selection, void *plan, int64_t *signature, void *stream);
+/* The same, where the caller knows more of the selection than that its taps are spread over the channels like random ones.
+ * CLG_LISTS_LONG: so many kernels read one channel that the kernels for short lists, where a list is one wavefront's work,
+ * are the slower ones.  CLG_LISTS_LOOK: looks at the lists and chooses (waits for the stream; not inside a recording).  The choice is the lowest bit
+ * of the signature; plans made again in the memory of one that is in use must be given it as `lists`. */
+#define CLG_LISTS_LOOK -1
+#define CLG_LISTS_SHORT 0
+#define CLG_LISTS_LONG 1
+int clg_convblock_plan_lists(int dtype, const clg_conv_geom *g, const int32_t *selection, void *plan, int lists, int64_t *signature,
+                             void *stream);
+/* scratch of the planned calls (clg_convblock_backward_scratch_bytes for a plan of short lists) */
+int64_t clg_convblock_backward_planned_scratch_bytes(int dtype, const clg_conv_geom *g, int64_t signature);
 #define CLG_BWD_WRT_LOGITS 1       /* w = softmax(logits): grad_w is the gradient w.r.t. the logits */
 #define CLG_BWD_GY_FEATURE_MAJOR 2 /* grad_y laid out [c_out, ho/2, wo/2, n] (shapes of clg_convblock_fm_supported) */
 /* clg_convblock_backward / clg_convblock_backward_logits / clg_convblock_backward_fm (chosen by flags) with a plan: no list building per call, and with folded [c_out, 7, 4] (written by clg_convblock_forward_ex with
  * CLG_FWD_FOLDED_OUT for the same w; may be NULL) no set-up launch is left for blocks whose images fit LDS.  grad_x may
- * be NULL.  scratch: clg_convblock_backward_scratch_bytes().  Same values as the unplanned entry points.
+ * be NULL.  scratch: clg_convblock_backward_planned_scratch_bytes().  Same values as the unplanned entry points.
  * Replaces full_convlogic_backward_x + full_convlogic_backward_weight (src/convlogic/convlogic_layer.py:71-82). */
 int clg_convblock_backward_planned(int dtype, const clg_conv_geom *g, const void *grad_y, const void *x, const void *w,
                                    const void *folded, const int32_t *selection, const uint8_t *argmax, void *plan,

@@ -118,6 +118,54 @@ def test_module_training_path_uses_the_plan_and_matches_the_oracle(shape):
     assert len(layer._plans) == 2
 
 
+def crowded(sel, half=True):
+    """the selection with channel 0 in place of the first channel of every second kernel (or of every kernel)"""
+    ch, first = sel >> 16, (sel >> 16)[:, :1]
+    there = (ch == first) & ((torch.arange(sel.shape[0], device=sel.device) % 2 == 0).view(-1, 1) | (not half))
+    return (torch.where(there, torch.zeros_like(ch), ch) << 16) | (sel & 0xFFFF)
+
+
+@pytest.mark.parametrize("shape", [(64, 16, 256, 8), (64, 32, 256, 28)])
+def test_a_channel_that_many_kernels_read_keeps_the_kernels_of_long_lists(shape, monkeypatch):
+    n, cin, cout, side = shape
+    torch.manual_seed(n)
+    layer = C.ConvLogicLayer(cin, cout, padding=1, complete=True, implementation="cuda").to(DEV)
+    x, geo = torch.rand(n, cin, side, side, device=DEV), (1, 1, 1, 1)
+    for sel, is_long in ((layer.selection, False), (crowded(layer.selection), True)):
+        y, am, probs, folded = convlogic_hip.full_convlogic_forward_logits(x, layer.weights.detach(), sel, *geo, 3, 3, want_folded=True)
+        gy = torch.randn_like(y)
+        plans = [convlogic_hip.make_backward_plan(x, cout, sel, *geo, 3, 3, lists=how) for how in (-1, 0, 1)]
+        assert [convlogic_hip.lists_of(sig) for _, sig in plans] == [is_long, 0, 1]
+        # the kernels of long lists are those that the knob takes at this shape, bit for bit
+        set_knobs(monkeypatch, CLG_BWDX_DIRECT="0")
+        want = convlogic_hip.full_convlogic_backward_logits(gy, x, probs, am, sel, *geo)
+        set_knobs(monkeypatch, CLG_BWDX_DIRECT=None)
+        for plan, sig in plans:
+            got = convlogic_hip.full_convlogic_backward_planned(gy, x, probs, folded, am, sel, plan, sig, *geo)
+            if convlogic_hip.lists_of(sig):
+                assert torch.equal(got[0], want[0])
+            for a, b in zip(got, want):
+                assert_grad_close(a, b, rel=1e-4)
+        padded = torch.empty(_lib.load().clg_convblock_padded_elems(0, ctypes.byref(convlogic_hip._geom(x, cout, *geo, 3, 3)), 1), device=DEV)
+        if padded.numel():
+            with pytest.raises(RuntimeError, match="short lists"):
+                convlogic_hip.full_convlogic_backward_planned(gy, x, probs, folded, am, sel, *plans[2], *geo, padded=padded)
+    # a plan that is in use keeps its kernels when it is made again for another selection
+    layer(x.requires_grad_(True)).sum().backward()
+    with torch.no_grad():
+        layer.selection.copy_(crowded(layer.selection))
+    x.grad = None
+    layer(x).backward(gy)
+    (kept,) = layer._plans.values()
+    assert convlogic_hip.lists_of(kept.plan[1]) == 0
+    again = copy.deepcopy(layer)
+    gx, x.grad = x.grad, None
+    again(x).backward(gy)
+    (kept,) = again._plans.values()
+    assert convlogic_hip.lists_of(kept.plan[1]) == 1
+    assert_grad_close(gx, x.grad, rel=1e-4)
+
+
 def test_a_kept_plan_is_complete():
     # what a first call leaves for calls on other streams: the tables of a block's plan and of a network's trees
     torch.manual_seed(5)
