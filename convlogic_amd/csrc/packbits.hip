@@ -396,7 +396,7 @@ void launch_pack_smv(const uint8_t *t, void *words, int64_t features, int64_t ba
 // split the rows.  Every thread counts the bit positions of its column with vertical counters (plane p holds bit p of the
 // running counts): four words are combined by three carry-save adders and the resulting "fours" word ripples into planes 2
 // and up.  The row phases of a wavefront are added as binary numbers through lane shuffles, the wavefronts through LDS, and
-// every wavefront expands its share of the bit positions into counts: no atomics, no zero fill, rows in a fixed order.
+// every wavefront expands its share of the bit positions into counts: no atomics and no zero fill unless a class is sliced.
 // Wide rows are bound by their reads: 5.1 TB/s on [64000, 1024] 8-byte words (103 us); narrow ones by the additions of the
 // counters.  Rows that are not whole 8-byte words, or shorter than 512 bytes, used to take one wavefront per 8-byte column
 // that read them byte by byte and met the others in atomics: [8000, 313] 4-byte words 279 -> 7.7 us, [8000, 1251] bytes
@@ -445,6 +445,31 @@ __device__ __forceinline__ uint64_t shuffle_down(uint64_t v, int by)
     return ((uint64_t)(uint32_t)__shfl_down((int)(uint32_t)(v >> 32), by) << 32) | (uint32_t)__shfl_down((int)(uint32_t)v, by);
 }
 __device__ __forceinline__ uint32_t shuffle_down(uint32_t v, int by) { return (uint32_t)__shfl_down((int)v, by); }
+
+// Classes of few rows: a wavefront per class and 8 bytes of its rows, lane = sample bit, so that nothing has to meet.  (The counters'
+// additions above cost as much for one row as for a hundred: 100000 classes of one 8-byte word 758 us in place of 35, 10000
+// classes of one row of four 74 in place of 21.)
+__global__ __launch_bounds__(256) void group_bit_sum_few_kernel(const uint8_t *__restrict__ x, int32_t *__restrict__ out, int class_rows,
+                                                              int64_t row_bytes, int64_t samples, int64_t k, int64_t cols8)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t item = (int64_t)blockIdx.x * 4 + uniform((int)(threadIdx.x >> 6));
+    if (item >= k * cols8) return;
+    const int64_t g = item / cols8, col = item - g * cols8, s = col * 64 + lane;
+    if (s >= samples) return;                                         // (its byte may lie behind the row)
+    const uint8_t *p = x + g * class_rows * row_bytes + (s >> 3);
+    int32_t acc = 0;
+    int r = 0;
+    for (; r + 8 <= class_rows; r += 8, p += 8 * row_bytes) {
+        uint32_t v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = p[j * row_bytes];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc += (v[j] >> (lane & 7)) & 1;
+    }
+    for (; r < class_rows; ++r, p += row_bytes) acc += (*p >> (lane & 7)) & 1;
+    out[s * k + g] = acc;
+}
 
 // S: the stored piece of a row, V: the register it is counted in.  cols_log2: log2 of C.
 template <typename S, typename V, int WAVES>
@@ -659,12 +684,26 @@ extern "C" int clg_group_bit_sum(int elem_size, const void *x, int32_t *out, int
     const int64_t row_bytes = words * elem_size, samples = row_bytes * 8 - pad_len;
     CLG_REQUIRE(pad_len >= 0 && samples > 0, "clg_group_bit_sum: pad_len %lld leaves no samples", (long long)pad_len);
     CLG_REQUIRE(k < (1 << 20), "clg_group_bit_sum: k too large");
-    CLG_REQUIRE(k < (1 << 20), "clg_group_bit_sum: k too large");
     const int64_t class_rows = features / k;
     hipStream_t st = clg_stream(stream);
     const uintptr_t align = (uintptr_t)x | (uintptr_t)row_bytes;
     const int piece = (align & 7) == 0 ? 8 : ((align & 3) == 0 ? 4 : 1);
-    const int64_t pieces = row_bytes / piece;
+    const int64_t pieces = row_bytes / piece, cols8 = clg_ceil_div(row_bytes, 8);
+    // A wavefront per class and 8 bytes: up to 96 rows where the GPU is not filled by them (0.4 to 1.0 times the time of the counters, at
+    // 256 rows 1.1 to 1.7 times), up to 128 or 256 where there are few columns (0.02 to 0.9), else up to 24 (0.4 to 1.0; at 64
+    // 1.0 to 1.4).  Not for full GPUs of wide 8-byte rows, which the counters read 512 bytes at a time (0.8 to 1.6), unless there
+    // are so many classes that what counts is the writes (0.5 to 1.1).
+    const int64_t rows_max = cols8 == 1 ? (piece == 8 || k >= 1000 ? 256 : 128)
+                                        : (cols8 <= 4 && piece == 8 ? 128 : (cols8 <= 8 || k * cols8 <= 4096 ? 96 : 0));
+    const bool by_bit = class_rows <= rows_max || (class_rows <= 24 && (cols8 < 64 || piece == 4)) ||
+                        (class_rows <= 8 && k >= 8192) || (piece == 1 && class_rows <= (cols8 < 512 ? 24 : 2));
+    if (by_bit && !clg_knob(K_GSUM_SLICES)) {
+        CLG_REQUIRE(clg_ceil_div(k * cols8, 4) < (1ll << 31), "clg_group_bit_sum: problem too large for one launch");
+        hipLaunchKernelGGL(group_bit_sum_few_kernel, dim3((unsigned)clg_ceil_div(k * cols8, 4)), dim3(256), 0, st, (const uint8_t *)x, out,
+                           (int)class_rows, row_bytes, samples, k, cols8);
+        CLG_CHECK_LAUNCH("clg_group_bit_sum");
+        return CLG_OK;
+    }
     // Columns per workgroup: a whole wavefront of them where that gives half of the CUs a workgroup (64 lanes x 8 bytes = 512
     // contiguous bytes of a row: 103 us at [64000, 1024] 8-byte words, 135 with 32 columns), fewer -- and more row phases --
     // where it does not, as long as the columns make 64-byte runs ([81920, 64]: 95 us with 64 columns, 22 with 8), and never

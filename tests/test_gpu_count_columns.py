@@ -7,7 +7,7 @@ import torch
 
 from convlogic_amd.hip import difflogic_hip
 from oracle import convlogic_oracle as O
-from tests.gpu_util import DEV
+from tests.gpu_util import DEV, set_knobs
 
 pytestmark = pytest.mark.gpu
 
@@ -31,3 +31,17 @@ def test_counts_of_classes_beyond_the_counter_range(bits, words):
     x[16400:16411] = 0
     got = difflogic_hip.groupbitsum(torch.from_numpy(x).to(DEV), 1, 2).cpu().numpy()
     assert got.shape == (words * bits - 1, 2) and (got[:, 0] == 16400).all() and (got[:, 1] == 16400 - 11).all()
+
+
+# Few rows per class take a wavefront per class and 8 bytes of a row: at the ends of its range, columns that are partly behind the row,
+# more (class, column) pairs than fill the GPU, and the column kernel at the same sizes (the knob takes it).
+@pytest.mark.parametrize("bits,words", [(64, 1), (64, 9), (64, 63), (32, 1), (32, 15), (16, 5), (8, 1), (8, 77), (8, 1251)])
+@pytest.mark.parametrize("class_rows,k", [(1, 700), (8, 3), (9, 100), (24, 70), (25, 70), (96, 2), (97, 2), (128, 3), (256, 2)])
+def test_counts_of_classes_of_few_rows(bits, words, class_rows, k, monkeypatch):
+    torch.manual_seed(bits + words + class_rows)
+    x = torch.randint(-128, 128, (class_rows * k, words * bits // 8), dtype=torch.int8).view({8: torch.int8, 16: torch.int16, 32: torch.int32, 64: torch.int64}[bits])
+    pad = int(torch.randint(0, bits, (1,))) if words > 1 else 0
+    want = O.group_bit_sum(x.numpy(), pad, k)
+    for slices in (None, "1"):
+        set_knobs(monkeypatch, CLG_GSUM_SLICES=slices)
+        assert np.array_equal(difflogic_hip.groupbitsum(x.to(DEV), pad, k).cpu().numpy(), want)
