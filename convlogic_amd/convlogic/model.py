@@ -97,7 +97,7 @@ def _forward(owner, x):
             return net(x)
         h = _head_of(net, x)
         if (type(h) is not PackBitsTensor or h.image or h.t.shape[0] != tail[0][0].in_dim or not h.t.is_contiguous()
-                or h.t.device != tail[0][0]._parameters["weights"].device):
+                or h.t.device != tail[0][0]._parameters["weights"].device or _many_small_classes(plan.roots, tail[1].k, h)):
             return _rest(net, h)
         return tree_packed(tail[0], tail[1].k, h, plan)
     if not (isinstance(x, torch.Tensor) and x.is_cuda):
@@ -130,6 +130,14 @@ def _forward(owner, x):
             h = m(h)
         return logic_layer_group_sum(net[n - 2], net[n - 1], h)
     return net(x)
+
+
+def _many_small_classes(roots, k, words):
+    """True for packed words on which the modules are the faster ones: the trees' workgroups each add up the counts of a class,
+    which costs as much for one root as for hundreds (1000 classes of one root, 256 samples: 22 us, 13 by the modules; of
+    16 roots: 34 and 37; of one root, 20 000 samples: 149 and 288)."""
+    rows = roots // k
+    return k >= 512 and rows <= 16 and rows * words.t.shape[1] * 64 <= 4096
 
 
 def _trees_take(h, first):

@@ -384,6 +384,19 @@ def test_a_wrapped_network_and_one_with_a_forward_of_its_own_are_called():
         assert torch.equal(model(x), want)
 
 
+@pytest.mark.parametrize("k,rows,samples,by_trees", [(600, 1, 64, False), (600, 1, 4096, False), (600, 1, 4097, True), (511, 1, 64, True),
+                                                     (600, 16, 256, False), (600, 17, 64, True), (600, 16, 257, True)])
+def test_many_small_classes_take_the_modules(k, rows, samples, by_trees, monkeypatch):
+    from convlogic_amd.convlogic import model as M
+    torch.manual_seed(12)
+    model, bits = Head(k * rows, k * rows, k).to(DEV).eval(), torch.rand(samples, k * rows, device=DEV) < 0.5
+    calls = []
+    monkeypatch.setattr(M, "tree_packed", lambda *a: calls.append(1) or fc_tree.tree_packed(*a))
+    with torch.no_grad():
+        assert torch.equal(model(C.PackBitsTensor(bits, 64)), model.network(C.PackBitsTensor(bits, 64)))
+    assert bool(calls) == by_trees
+
+
 def test_more_classes_than_the_tree_kernels_take():
     # (the float class sums take no more either: they refuse, as for the modules)
     torch.manual_seed(11)
