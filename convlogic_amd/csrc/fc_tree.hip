@@ -238,7 +238,8 @@ __global__ __launch_bounds__(kTreeBlock) void fc_tree_forward_kernel(const float
     }
 }
 
-// out[b][g] = inv_tau * sum over the slices in order, eight loads in flight
+// out[b][g] = inv_tau * sum over the slices in order, FLIGHT loads in flight
+template <int FLIGHT>
 __global__ __launch_bounds__(256) void fc_tree_finish_kernel(const float *__restrict__ partial, float *__restrict__ out, int slices, int k,
                                                            int64_t pitch, int64_t batch, float inv_tau)
 {
@@ -248,12 +249,12 @@ __global__ __launch_bounds__(256) void fc_tree_finish_kernel(const float *__rest
     const int64_t b = i - (int64_t)g * batch, step = (int64_t)k * pitch;
     const float *p = partial + (int64_t)g * pitch + b;
     float acc = 0.f;
-    for (int s = 0; s < slices; s += 8) {
-        float v[8];
+    for (int s = 0; s < slices; s += FLIGHT) {
+        float v[FLIGHT];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = p[(int64_t)min(s + u, slices - 1) * step];
+        for (int u = 0; u < FLIGHT; ++u) v[u] = p[(int64_t)min(s + u, slices - 1) * step];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) acc = s + u < slices ? acc + v[u] : acc;
+        for (int u = 0; u < FLIGHT; ++u) acc = s + u < slices ? acc + v[u] : acc;
     }
     out[b * k + g] = acc * inv_tau;
 }
@@ -450,13 +451,14 @@ int check_tree(const char *name, int64_t in_dim, int64_t roots, int64_t k)
 }
 
 // Row slices of a class, as clg_group_sum cuts them (a class sum of 65 536 values is rounded at 1e-7 of a logit in the
-// thousands: the softmax of the loss then shows the order of the additions, so the order is kept).
+// thousands: the softmax of the loss then shows the order of the additions, so the order is kept).  Only one or two large classes of a
+// small batch are cut into more slices than its 64, which would be the launch's only 64 or 128 workgroups.
 int tree_slices(int64_t class_rows, int64_t batch, int64_t k)
 {
     int64_t slices = clg_ceil_div(1024, clg_ceil_div(batch, (int64_t)kWave) * k);
     if (class_rows <= 4096) slices = 64;                              // small classes (where the GroupSum has another kernel): for the parallelism
     slices = std::min(slices, class_rows / (class_rows <= 4096 ? 16 : 64));
-    return (int)std::min<int64_t>(64, std::max<int64_t>(1, slices));
+    return (int)std::min<int64_t>(512, std::max<int64_t>(1, slices));
 }
 
 }  // namespace
@@ -518,8 +520,12 @@ extern "C" int clg_fc_tree_forward(const float *x, const int32_t *rows, const fl
     else CLG_TREE_F(4);
 #undef CLG_TREE_F
     CLG_CHECK_LAUNCH(name);
-    hipLaunchKernelGGL(fc_tree_finish_kernel, dim3((unsigned)clg_ceil_div(batch * k, 256)), dim3(256), 0, st, (const float *)partial, out, slices,
-                       (int)k, pitch, batch, 1.f / (float)tau);
+#define CLG_TREE_S(FLIGHT)                                                                                                    \
+    hipLaunchKernelGGL((fc_tree_finish_kernel<FLIGHT>), dim3((unsigned)clg_ceil_div(batch * k, 256)), dim3(256), 0, st, (const float *)partial, \
+                       out, slices, (int)k, pitch, batch, 1.f / (float)tau)
+    if (slices > 64) CLG_TREE_S(32);
+    else CLG_TREE_S(8);
+#undef CLG_TREE_S
     CLG_CHECK_LAUNCH(name);
     return CLG_OK;
 }

@@ -457,3 +457,29 @@ def test_what_a_row_holds_behind_the_batch_adds_nothing(batch, pitch):
     for other in results[1:]:
         for i, (a, b) in enumerate(zip(results[0], other)):
             assert torch.isfinite(a).all() and torch.equal(a, b), f"result {i}"
+
+
+@pytest.mark.parametrize("batch", [1, 3, 64, 100])
+@pytest.mark.parametrize("roots,k", [(4097, 1), (9000, 1), (40000, 1), (20000, 2)])
+def test_one_or_two_large_classes(roots, k, batch):
+    # more slices of a class than the 64 of larger launches: the sums against float64, the gradients against the modules
+    model = Head(50, roots, k).to(DEV)
+    x, go = torch.rand(batch, 50, device=DEV).requires_grad_(True), torch.randn(batch, k, device=DEV)
+    results = []
+    for on in (True, False):
+        model.tree_tail = on
+        model.train().zero_grad()
+        x.grad = None
+        out = model(x)
+        out.backward(go)
+        results.append([out.detach(), x.grad] + [p.grad for p in model.parameters()])
+    h = x.detach().double()
+    for m in list(model.network)[1:4]:
+        a, b = h[:, m.indices_0], h[:, m.indices_1]
+        c = O.fold_coefficients(torch.softmax(m.weights.detach().double(), -1).cpu()).to(DEV)
+        h = c[:, 0] * a * b + c[:, 1] * a + c[:, 2] * b + c[:, 3]
+    want = h.view(batch, k, -1).sum(-1) / 3.0
+    # at most 512 + 40 additions in a row of values around 0.5, each a rounding of the sum so far: 0.5 * 552 * 6e-8 of it at worst
+    assert ((results[0][0].double() - want).abs() <= 2e-5 * want).all()
+    for i, (a, b) in enumerate(zip(*results)):
+        assert_grad_close(a, b, rel=1e-4, name=f"result {i}")
