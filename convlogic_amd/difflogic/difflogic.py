@@ -6,6 +6,7 @@ implementation="cuda" runs the HIP kernels (on ROCm builds of torch the device t
 reference's second, explicitly selected backend: plain torch ops on whatever device the tensors
 live on.
 """
+import threading
 import weakref
 
 import numpy as np
@@ -20,6 +21,7 @@ from .packbitstensor import PackBitsTensor
 # key (versions and addresses) that is equal to the checked one is of the checked wiring.  Outside the modules: copies and
 # pickles carry no buffers of an earlier device.
 _CHECKED_BUFFERS = weakref.WeakKeyDictionary()
+_CHECKING = threading.Lock()                                          # one thread checks: two would count the same wiring twice
 
 
 def _reverse_wiring(idx0, idx1, in_dim):
@@ -168,38 +170,45 @@ class LogicLayer(torch.nn.Module):
         self.__dict__["_wiring_epoch"] = self.__dict__.get("_wiring_epoch", 0) + 1
 
     def _check_wiring(self):
-        """Returns the key of the wiring, which what is derived from it (here and in fc_tree) is kept under.  The kernels index x with indices_0 / indices_1 without bounds checks: an index outside [0, in_dim) must
-        raise here instead of faulting the GPU.  Checked on the first launch and again whenever the buffers were
-        modified in place (version counter) or replaced; writes through `.data` bypass the counter -- call
-        invalidate() after those."""
+        """Returns the key of the wiring, which what is derived from it (here and in fc_tree) is kept under.  The kernels index
+        x with indices_0 / indices_1 without bounds checks: an index outside [0, in_dim) must raise here instead of faulting
+        the GPU.  Checked on the first launch and again whenever the buffers were modified in place (version counter) or
+        replaced; writes through `.data` bypass the counter -- call invalidate() after those."""
         key = self._wiring_key()
         if self.__dict__.get("_wiring_checked") != key:
-            self._new_wiring_epoch()
-            for name, idx in (("indices_0", self.indices_0), ("indices_1", self.indices_1)):
-                if idx.dtype != torch.int64 or tuple(idx.shape) != (self.out_dim,):
-                    raise ValueError(f"{name} must be int64 [{self.out_dim}], got {idx.dtype} {tuple(idx.shape)}")
-                if idx.numel() and (int(idx.min()) < 0 or int(idx.max()) >= self.in_dim):
-                    raise ValueError(f"{name} holds an input index outside [0, {self.in_dim})")
-            if self.implementation == "cuda":                        # the reverse map of the input gradient
-                for name, n in (("given_x_indices_of_y_start", self.in_dim + 1), ("given_x_indices_of_y", 2 * self.out_dim)):
-                    t = getattr(self, name)
-                    if t.dtype != torch.int64 or tuple(t.shape) != (n,) or t.device != self.indices_0.device or not t.is_contiguous():
-                        raise ValueError(f"{name} must be a contiguous int64 [{n}] on the device of the wiring")
-                if not (self.indices_0.is_contiguous() and self.indices_1.is_contiguous()
-                        and self.indices_0.device == self.indices_1.device == self.weights.device):
-                    raise ValueError("indices_0 / indices_1 must be contiguous and on the device of the weights")
-                # The reverse map belongs to the wiring it was built from: after an in-place rewiring or a state_dict
-                # that replaced the indices it is rebuilt here (into the same buffers), so the input gradient never walks
-                # the lists of an older wiring.  (The reference builds it once, src/difflogic/difflogic.py:71-87.)
-                built = (self.indices_0._version, self.indices_1._version)
-                if self.__dict__.get("_reverse_built") != built:
-                    start, flat = _reverse_wiring(self.indices_0.cpu().numpy(), self.indices_1.cpu().numpy(), self.in_dim)
-                    with torch.no_grad():
-                        self.given_x_indices_of_y_start.copy_(start)
-                        self.given_x_indices_of_y.copy_(flat)
-                    self._reverse_built = built
-            _CHECKED_BUFFERS[self] = (self._buffers["indices_0"], self._buffers["indices_1"])
-            self._wiring_checked = key = self._wiring_key()
+            with _CHECKING:
+                key = self._wiring_key()
+                if self.__dict__.get("_wiring_checked") != key:       # (else another thread checked it meanwhile)
+                    key = self._check_new_wiring()
+        return key
+
+    def _check_new_wiring(self):
+        self._new_wiring_epoch()
+        for name, idx in (("indices_0", self.indices_0), ("indices_1", self.indices_1)):
+            if idx.dtype != torch.int64 or tuple(idx.shape) != (self.out_dim,):
+                raise ValueError(f"{name} must be int64 [{self.out_dim}], got {idx.dtype} {tuple(idx.shape)}")
+            if idx.numel() and (int(idx.min()) < 0 or int(idx.max()) >= self.in_dim):
+                raise ValueError(f"{name} holds an input index outside [0, {self.in_dim})")
+        if self.implementation == "cuda":                            # the reverse map of the input gradient
+            for name, n in (("given_x_indices_of_y_start", self.in_dim + 1), ("given_x_indices_of_y", 2 * self.out_dim)):
+                t = getattr(self, name)
+                if t.dtype != torch.int64 or tuple(t.shape) != (n,) or t.device != self.indices_0.device or not t.is_contiguous():
+                    raise ValueError(f"{name} must be a contiguous int64 [{n}] on the device of the wiring")
+            if not (self.indices_0.is_contiguous() and self.indices_1.is_contiguous()
+                    and self.indices_0.device == self.indices_1.device == self.weights.device):
+                raise ValueError("indices_0 / indices_1 must be contiguous and on the device of the weights")
+            # The reverse map belongs to the wiring it was built from: after an in-place rewiring or a state_dict
+            # that replaced the indices it is rebuilt here (into the same buffers), so the input gradient never walks
+            # the lists of an older wiring.  (The reference builds it once, src/difflogic/difflogic.py:71-87.)
+            built = (self.indices_0._version, self.indices_1._version)
+            if self.__dict__.get("_reverse_built") != built:
+                start, flat = _reverse_wiring(self.indices_0.cpu().numpy(), self.indices_1.cpu().numpy(), self.in_dim)
+                with torch.no_grad():
+                    self.given_x_indices_of_y_start.copy_(start)
+                    self.given_x_indices_of_y.copy_(flat)
+                self._reverse_built = built
+        _CHECKED_BUFFERS[self] = (self._buffers["indices_0"], self._buffers["indices_1"])
+        self._wiring_checked = key = self._wiring_key()
         return key
 
     def invalidate(self):

@@ -2,6 +2,8 @@
 On the CPU, with a stand-in for the tables that notes the wiring it was made from."""
 import copy
 import pickle
+import threading
+import time
 
 import pytest
 import torch
@@ -152,6 +154,26 @@ def test_the_tables_of_a_recorded_step_stay(layers):
     plan.fits = lambda: True
     layers[0].invalidate()
     assert fc_tree.tree_plan(*layers) is plan
+
+
+def test_two_threads_check_a_wiring_once(layers):
+    # a wiring that counts as new a second time would make the tables again under the kernels of the first thread
+    layer, entered = layers[0], []
+    check = layer._check_new_wiring
+
+    def slowly():
+        entered.append(1)
+        time.sleep(0.2)
+        return check()
+
+    layer._check_new_wiring = slowly
+    keys = []
+    threads = [threading.Thread(target=lambda: keys.append(layer._check_wiring())) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(entered) == 1 and len(set(keys)) == 1 and layer._wiring_epoch == 1
 
 
 def test_the_walk_plan_of_a_recorded_packed_layer_stays():
