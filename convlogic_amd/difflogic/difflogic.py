@@ -66,7 +66,7 @@ class LogicLayer(torch.nn.Module):
             start, flat = _reverse_wiring(self.indices_0.cpu().numpy(), self.indices_1.cpu().numpy(), in_dim)
             self.register_buffer("given_x_indices_of_y_start", start)
             self.register_buffer("given_x_indices_of_y", flat)
-            self._reverse_built = (self.indices_0._version, self.indices_1._version)
+            self._reverse_built = self._index_buffers()
 
         self.num_neurons = out_dim
         self.num_weights = out_dim
@@ -165,6 +165,16 @@ class LogicLayer(torch.nn.Module):
         state.pop("_wiring_checked", None)
         return state
 
+    def _index_buffers(self):
+        """The wiring buffers and their versions: what the reverse map is of.  (The buffers themselves: versions alone are those
+        of any buffer that was never written.)"""
+        a, b = self._buffers["indices_0"], self._buffers["indices_1"]
+        return a, b, a._version, b._version
+
+    def _reverse_is_current(self):
+        of, now = self.__dict__.get("_reverse_built"), self._index_buffers()
+        return of is not None and of[0] is now[0] and of[1] is now[1] and of[2:] == now[2:]
+
     def _new_wiring_epoch(self):
         """No key taken before is equal to one taken after: whatever was derived from the wiring is derived again."""
         self.__dict__["_wiring_epoch"] = self.__dict__.get("_wiring_epoch", 0) + 1
@@ -197,16 +207,15 @@ class LogicLayer(torch.nn.Module):
             if not (self.indices_0.is_contiguous() and self.indices_1.is_contiguous()
                     and self.indices_0.device == self.indices_1.device == self.weights.device):
                 raise ValueError("indices_0 / indices_1 must be contiguous and on the device of the weights")
-            # The reverse map belongs to the wiring it was built from: after an in-place rewiring or a state_dict
-            # that replaced the indices it is rebuilt here (into the same buffers), so the input gradient never walks
+            # The reverse map belongs to the wiring it was built from: after an in-place rewiring, a state_dict or an
+            # assignment that replaced the indices it is rebuilt here (into the same buffers), so the input gradient never walks
             # the lists of an older wiring.  (The reference builds it once, src/difflogic/difflogic.py:71-87.)
-            built = (self.indices_0._version, self.indices_1._version)
-            if self.__dict__.get("_reverse_built") != built:
+            if not self._reverse_is_current():
                 start, flat = _reverse_wiring(self.indices_0.cpu().numpy(), self.indices_1.cpu().numpy(), self.in_dim)
                 with torch.no_grad():
                     self.given_x_indices_of_y_start.copy_(start)
                     self.given_x_indices_of_y.copy_(flat)
-                self._reverse_built = built
+                self._reverse_built = self._index_buffers()
         _CHECKED_BUFFERS[self] = (self._buffers["indices_0"], self._buffers["indices_1"])
         self._wiring_checked = key = self._wiring_key()
         return key
@@ -221,7 +230,10 @@ class LogicLayer(torch.nn.Module):
 
     def _apply(self, fn, *args, **kwargs):
         a, b = self._buffers["indices_0"], self._buffers["indices_1"]
+        current = self._reverse_is_current()
         super()._apply(fn, *args, **kwargs)
+        if current:                                                  # (the reverse map moves with its wiring)
+            self._reverse_built = self._index_buffers()
         if self._buffers["indices_0"] is not a or self._buffers["indices_1"] is not b:   # moved to another device
             self._new_wiring_epoch()
             _CHECKED_BUFFERS.pop(self, None)

@@ -396,3 +396,35 @@ def test_a_loaded_selection_is_checked_before_recorded_plans_are_made_from_it():
             layer._check_selection()
     layer.load_state_dict(good)
     assert kept.made == 1
+
+
+def test_the_reverse_lists_follow_the_wiring_buffers(monkeypatch):
+    import copy
+    import pickle
+    from convlogic_amd.difflogic import difflogic as D
+    made = []
+    monkeypatch.setattr(D, "_reverse_wiring", lambda *a: made.append(1) or _reverse_wiring(*a))
+
+    def check(layer, remade):
+        made.clear()
+        layer._check_wiring()
+        start, flat = _reverse_wiring(layer.indices_0.numpy(), layer.indices_1.numpy(), layer.in_dim)
+        assert torch.equal(layer.given_x_indices_of_y_start, start) and torch.equal(layer.given_x_indices_of_y, flat)
+        assert len(made) == remade
+
+    torch.manual_seed(0)
+    layer = C.LogicLayer(24, 40, implementation="cuda")
+    layer.indices_0 = layer.indices_0.flip(0)                          # a wiring of the caller's, before the first call ...
+    check(layer, 1)
+    layer.indices_1 = layer.indices_1.flip(0)                          # ... and after one: new buffers, version 0 as the old ones
+    check(layer, 1)
+    layer._apply(lambda t: t.clone())                                  # a move brings the lists along
+    check(layer, 0)
+    for other in (copy.deepcopy(layer), pickle.loads(pickle.dumps(layer))):
+        check(other, 1)                                                # (torch counts the buffers of a copy as written)
+    layer.indices_0[:2] = layer.indices_0[:2].flip(0)
+    layer._apply(lambda t: t.clone())                                  # written, then moved before a call
+    check(layer, 1)
+    layer.load_state_dict(C.LogicLayer(24, 40, implementation="cuda").state_dict())
+    check(layer, 1)
+    check(C.LogicLayer(24, 40, implementation="cuda"), 0)
