@@ -1058,6 +1058,7 @@ BwdXMode choose_backward_x(const Geom &g, int elem, TilePlan *p, int *sample_ele
     const bool tiled = plan_backward_x(g, elem, &pt);
     const bool direct = plan_backward_x_direct(g, elem, &pd, &se);
     const int I = (g.ho / 2) * (g.wo / 2);
+    if (!direct) pd.G = 1;                                            // (not made: G only divides below)
     auto lanes = [&](const TilePlan &q) { return q.G * I < kWave ? q.G * I : kWave; };
     // The direct kernel has one independent wavefront per (sample group, channel) and no barriers: it also wins
     // when there are thousands of such owners with short kernel lists (48 vs 88 us at [256,32,16,16] -> 128,

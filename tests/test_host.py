@@ -428,3 +428,19 @@ def test_the_reverse_lists_follow_the_wiring_buffers(monkeypatch):
     layer.load_state_dict(C.LogicLayer(24, 40, implementation="cuda").state_dict())
     check(layer, 1)
     check(C.LogicLayer(24, 40, implementation="cuda"), 0)
+
+
+@pytest.mark.parametrize("c_out", [1, 65535, 65536, 66000, 100000])
+def test_blocks_of_any_number_of_kernels_are_planned_on_the_host(c_out):
+    # the choice of the gradient kernels where one of them takes no such block: it used to divide by that one's unset plan
+    import ctypes
+    import types
+    from convlogic_amd.hip import convlogic_hip
+    lib = _lib.load()
+    for shape in ((2, 2, 6, 6), (2, 2, 4, 4), (64, 2, 4, 4), (3, 1, 28, 28), (100, 16, 8, 8)):
+        g = convlogic_hip._geom(types.SimpleNamespace(shape=shape), c_out, 1, 1, 1, 1, 3, 3)
+        for dtype in (0, 1):
+            for poison in range(4):                                    # (other calls leave other values on the stack)
+                assert lib.clg_convblock_backward_scratch_bytes(dtype, ctypes.byref(g)) > 0
+                assert lib.clg_convblock_plan_bytes(dtype, ctypes.byref(g)) > 0
+                lib.clg_fc_tree_partial_elems(1 + poison, 1, 1, 1)
