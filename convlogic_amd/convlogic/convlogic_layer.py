@@ -169,11 +169,17 @@ def _pair(v):
     return (v, v) if isinstance(v, int) else tuple(v)
 
 
+def _same_buffer(of, buffer):
+    """True when `of` = (buffer, version) is of this buffer as it is now.  The buffer itself is compared (and so held): another
+    one may have its address and version, for instance after a move to another device and back."""
+    return of is not None and of[0] is buffer and of[1] == buffer._version
+
+
 _MAKING_PLANS = threading.Lock()
 
 
 class _KeptPlan:
-    """A backward plan of a layer, the selection it was made from (version and address) and whether a recording reads it."""
+    """A backward plan of a layer, the selection it was made from (buffer and version) and whether a recording reads it."""
 
     def __init__(self):
         self.plan = self.wiring = None
@@ -230,8 +236,7 @@ class ConvLogicLayer(nn.Module):
         Checked at construction, on the first launch and whenever the buffer was modified in place (version counter)
         or replaced; writes through `.data` bypass the counter -- call invalidate() after those."""
         sel = self._buffers["selection"]                             # (not through nn.Module.__getattr__: taken on every call)
-        key = (sel._version, sel.data_ptr())
-        if self.__dict__.get("_selection_checked") == key:
+        if _same_buffer(self.__dict__.get("_selection_checked"), sel):
             return
         if sel.dtype != torch.int32 or tuple(sel.shape) != (self.out_channels, 8):
             raise ValueError(f"selection must be int32 [{self.out_channels}, 8], got {sel.dtype} {tuple(sel.shape)}")
@@ -239,7 +244,7 @@ class ConvLogicLayer(nn.Module):
         if sel.numel() and (int(ch.max()) >= self.in_channels or int(row.max()) >= self.kernel[0] or int(col.max()) >= self.kernel[1]):
             raise ValueError(f"selection names a tap outside {self.in_channels} input channels and a "
                              f"{self.kernel[0]}x{self.kernel[1]} receptive field")
-        self._selection_checked = key
+        self._selection_checked = (sel, sel._version)
 
     def invalidate(self):
         """Forces the next call to check the selection buffer again and to make the backward plans again (after a write
@@ -258,10 +263,10 @@ class ConvLogicLayer(nn.Module):
         it again in every replay."""
         from ..hip import _lib
         key = (tuple(x.shape), x.dtype, x.device, _lib.knob_generation())
-        wiring = (sel._version, sel.data_ptr())
+        buffer = self._buffers["selection"]                          # (sel: the same, or a contiguous copy for this call)
         plans = self.__dict__.setdefault("_plans", {})
         kept, recording = plans.get(key), torch.cuda.is_current_stream_capturing()
-        if kept is not None and kept.wiring == wiring:
+        if kept is not None and _same_buffer(kept.wiring, buffer):
             kept.recorded |= recording
             return kept.plan
         if recording:
@@ -271,11 +276,11 @@ class ConvLogicLayer(nn.Module):
             if kept is None:
                 self._make_room(plans, x.device)
                 kept = _KeptPlan()
-            if kept.wiring != wiring:                                # (else another thread made it meanwhile)
-                kept.wiring = None
+            if not _same_buffer(kept.wiring, buffer):                # (else another thread made it meanwhile)
+                kept.wiring, version = None, buffer._version
                 kept.make(x, sel, self)
                 torch.cuda.current_stream(x.device).synchronize()
-                kept.wiring = wiring
+                kept.wiring = (buffer, version)
                 plans[key] = kept
             return kept.plan
 
@@ -310,11 +315,11 @@ class ConvLogicLayer(nn.Module):
             return pf[2], pf[3]
         return None
 
-    def __getstate__(self):                                          # copies and pickles make plans of their own
-        return {name: value for name, value in self.__dict__.items() if name != "_plans"}
+    def __getstate__(self):                                          # copies and pickles make plans and checks of their own
+        return {name: value for name, value in self.__dict__.items() if name not in ("_plans", "_selection_checked")}
 
     def __setstate__(self, state):
-        super().__setstate__({name: value for name, value in state.items() if name != "_plans"})
+        super().__setstate__({name: value for name, value in state.items() if name not in ("_plans", "_selection_checked")})
 
     def _load_from_state_dict(self, *args, **kwargs):
         super()._load_from_state_dict(*args, **kwargs)

@@ -253,3 +253,26 @@ def test_copies_and_pickles_carry_no_plans():
     other.__setstate__(state)
     assert "_plans" not in other.__dict__
     other.invalidate()
+
+
+@pytest.mark.parametrize("route", ["moved", "dense copy"])
+def test_another_selection_at_the_same_address_reaches_the_plan(route):
+    torch.manual_seed(8)
+    layer, other = (C.ConvLogicLayer(8, 16, padding=1, complete=True, implementation="cuda").to(DEV) for _ in range(2))
+    other.weights.data.copy_(layer.weights)
+    x = torch.rand(4, 8, 8, 8, device=DEV, requires_grad=True)
+    if route == "dense copy":                                          # every call makes a contiguous copy of such a buffer
+        layer.selection = layer.selection.t().contiguous().t()
+    layer(x).sum().backward()
+    if route == "moved":
+        layer.cpu()
+        layer.selection.copy_(other.selection)
+        layer.to(DEV)
+    else:
+        layer.selection.copy_(other.selection)
+    grads = []
+    for m in (layer, other):
+        x.grad = m.weights.grad = None
+        m(x).square().sum().backward()
+        grads.append((x.grad, m.weights.grad))
+    assert all(torch.equal(a, b) for a, b in zip(*grads))

@@ -430,6 +430,20 @@ def test_the_reverse_lists_follow_the_wiring_buffers(monkeypatch):
     check(C.LogicLayer(24, 40, implementation="cuda"), 0)
 
 
+def test_the_check_of_a_selection_is_of_its_buffer():
+    # a buffer at the address of an earlier one, with its version, as after a move to another device and back
+    layer = C.ConvLogicLayer(2, 4, complete=True, implementation="python")
+    memory = layer.selection.numpy().copy()
+    layer.selection = torch.from_numpy(memory)
+    layer._check_selection()
+    memory[0, 0] = 2 << 16                                             # a channel that is not there
+    other = torch.from_numpy(memory)
+    assert (other.data_ptr(), other._version) == (layer.selection.data_ptr(), layer.selection._version)
+    layer.selection = other
+    with pytest.raises(ValueError, match="selection"):
+        layer._check_selection()
+
+
 @pytest.mark.parametrize("c_out", [1, 65535, 65536, 66000, 100000])
 def test_blocks_of_any_number_of_kernels_are_planned_on_the_host(c_out):
     # the choice of the gradient kernels where one of them takes no such block: it used to divide by that one's unset plan
