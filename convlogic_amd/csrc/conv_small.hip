@@ -17,7 +17,8 @@ namespace {
 
 constexpr int kLsWaves = 4;                        // wavefronts per workgroup
 // The two planes of a lane with shared halos: the right halo of a row is the left halo of the next, the bottom halo row of the
-// first plane the top one of the second: 56 elements instead of 72, so a wavefront takes 14.6 KB and a CU holds 10 of them, not 8.
+// first plane the top one of the second: 57 elements (an odd stride) instead of 73, 14.6 KB for a wavefront's 64 slices instead of 18.7.
+// A CU's 160 KB hold two workgroups of four wavefronts either way, five instead of four of two, eleven instead of eight of one.
 constexpr int kLsRow = 5;                          // row pitch
 constexpr int kLsPlane = 5 * kLsRow;               // top halo row and the four rows of a plane
 constexpr int kLsStride = 2 * kLsPlane + kLsRow + 2;   // elements per lane: the last halo row and its right neighbour; odd
@@ -336,8 +337,8 @@ __global__ __launch_bounds__(kLsWaves *kWave, 2) void convblock_eval_packed_4x4_
 // tg is what the pair moves most of (512 B per kernel and sample row of 4 cells, float32).  A tap belongs to ONE of the
 // kernel's two channels, so tap-major rows are read by their channel alone, once, and every access is 16 bytes per lane on
 // consecutive addresses; sample-major pieces of 128 bytes per lane ([c][n][cell][tap]) were fetched whole by both channels.
-// What bounds the first pass is wavefronts: LDS allows 10 per CU (8 with unshared halos), registers 12, and a workgroup has no
-// wavefront that finds no samples.  Second pass: the stream of tg.
+// What bounds the first pass is wavefronts: LDS allows 8 per CU in workgroups of four, 10 in workgroups of two (batches up to 192),
+// registers 12, and a workgroup has no wavefront that finds no samples.  Second pass: the stream of tg.
 // [128, 16384, 4, 4] -> 32768: 475 + 239 -> 389 + 172 us (1.6 and 3.9 TB/s of tg); [256, 512, 4, 4] -> 1024: 28.5 + 24.9 -> 23.8 + 16.1 us.
 
 constexpr int kGradStride = kLsPlane + kLsRow + 1; // gradient plane (taps of border cells fall into the halo); odd

@@ -483,3 +483,32 @@ def test_one_or_two_large_classes(roots, k, batch):
     assert ((results[0][0].double() - want).abs() <= 2e-5 * want).all()
     for i, (a, b) in enumerate(zip(*results)):
         assert_grad_close(a, b, rel=1e-4, name=f"result {i}")
+
+
+def test_one_network_first_used_by_several_threads_and_streams():
+    # every thread's first call meets a wiring that nobody has checked, tables that nobody has made, or those of another stream
+    import threading
+    torch.manual_seed(13)
+    model = Head(300, 2000, 10).to(DEV).eval()
+    x = [torch.randint(0, 2, (n, 300), device=DEV).float() for n in (64, 100, 257, 1000)]
+    with torch.no_grad():
+        want = [(model.network(t), model.network(C.PackBitsTensor(t.bool(), 64))) for t in x]
+    for _ in range(5):
+        for m in list(model.network)[1:4]:
+            m.invalidate()
+        got, start = [None] * len(x), threading.Barrier(len(x))
+
+        def work(i):
+            with torch.cuda.stream(torch.cuda.Stream()), torch.no_grad():
+                start.wait()
+                got[i] = model(x[i]), model(C.PackBitsTensor(x[i].bool(), 64))
+                torch.cuda.current_stream().synchronize()
+
+        torch.cuda.synchronize()
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(len(x))]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        for (a, b), (c, d) in zip(got, want):
+            assert torch.equal(a, c) and torch.equal(b, d)
