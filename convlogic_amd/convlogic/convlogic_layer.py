@@ -265,11 +265,11 @@ class ConvLogicLayer(nn.Module):
         key = (tuple(x.shape), x.dtype, x.device, _lib.knob_generation())
         buffer = self._buffers["selection"]                          # (sel: the same, or a contiguous copy for this call)
         plans = self.__dict__.setdefault("_plans", {})
-        kept, recording = plans.get(key), torch.cuda.is_current_stream_capturing()
+        kept = plans.get(key)
         if kept is not None and _same_buffer(kept.wiring, buffer):
-            kept.recorded |= recording
+            kept.recorded = kept.recorded or torch.cuda.is_current_stream_capturing()
             return kept.plan
-        if recording:
+        if torch.cuda.is_current_stream_capturing():
             return convlogic_hip.make_backward_plan(x, self.out_channels, sel, *self.stride, *self.padding, *self.kernel)
         with _MAKING_PLANS:
             kept = plans.get(key)

@@ -64,21 +64,23 @@ def _called_for_itself(module):
 def _tree_tail(net):
     """The last four modules of a network -- three LogicLayers and a GroupSum -- when nothing but a call of the modules
     themselves stands against evaluating them as one operation (difflogic/fc_tree.py), else None."""
-    if type(net) is not nn.Sequential or len(net) < 4 or _called_for_itself(net) or torch.nn.modules.module._has_any_global_hook():
+    if type(net) is not nn.Sequential or len(net._modules) < 4 or _called_for_itself(net) or torch.nn.modules.module._has_any_global_hook():
         return None                                                   # (a wrapped network, or one with a forward of its own, is called)
-    tail = [net[i] for i in range(len(net) - 4, len(net))]
-    *layers, gs = tail
-    if not all(type(m) is LogicLayer and m.implementation == "cuda" and m.grad_factor == 1.0 for m in layers) or type(gs) is not GroupSum:
+    *layers, gs = list(net._modules.values())[-4:]
+    if type(gs) is not GroupSum or _called_for_itself(gs):
         return None
-    if any(_called_for_itself(m) for m in tail) or layers[-1].out_dim % gs.k != 0 or gs.tau == 0:
+    device = None
+    for m in layers:
+        if type(m) is not LogicLayer or m.implementation != "cuda" or m.grad_factor != 1.0 or _called_for_itself(m):
+            return None
+        w = m._parameters["weights"]
+        device = device or w.device
+        if not (w.is_cuda and w.dtype == torch.float32 and w.shape == (m.out_dim, 16) and w.is_contiguous() and w.device == device):
+            return None
+    if layers[-1].out_dim % gs.k != 0 or gs.tau == 0:
         return None
     if gs.k > 65535 or layers[0].in_dim >= 1 << 31 or layers[-1].out_dim >= 1 << 28:   # (what the tree kernels' indices hold)
         return None
-    for m in layers:
-        w = m._parameters["weights"]
-        if not (w.is_cuda and w.dtype == torch.float32 and w.shape == (m.out_dim, 16) and w.is_contiguous()
-                and w.device == layers[0]._parameters["weights"].device):
-            return None
     return layers, gs
 
 
@@ -148,16 +150,15 @@ def _trees_take(h, first):
 
 def _head_of(net, h):
     """all but the last four modules of a network"""
-    for i, m in enumerate(net):
-        if i == len(net) - 4:
-            return h
+    for m in list(net._modules.values())[:-4]:
         h = m(h)
+    return h
 
 
 def _rest(net, h):
     """the last four"""
-    for i in range(len(net) - 4, len(net)):
-        h = net[i](h)
+    for m in list(net._modules.values())[-4:]:
+        h = m(h)
     return h
 
 

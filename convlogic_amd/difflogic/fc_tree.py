@@ -59,8 +59,10 @@ def tree_plan(first, second, third):
     if 2 * second.out_dim != second.in_dim or 2 * third.out_dim != third.in_dim or second.in_dim != first.out_dim or third.in_dim != second.out_dim:
         return None
     keys = (first._check_wiring(), second._check_wiring(), third._check_wiring())
-    entry = next((e for e in _PLANS.get(first, ()) if e.is_of(second, third)), None)
-    if entry is None or entry.keys != keys:
+    for entry in _PLANS.get(first, ()):
+        if entry.keys == keys and entry.is_of(second, third):
+            break
+    else:
         if first._buffers["indices_0"].is_cuda and torch.cuda.is_current_stream_capturing():
             return None
         with _BUILDING:
