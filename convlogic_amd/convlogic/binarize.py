@@ -44,6 +44,8 @@ def pack_thresholds(x: torch.Tensor, thresholds: torch.Tensor) -> PackBitsTensor
     thresholding and bit packing in one pass over the pixels."""
     if not x.is_cuda:
         raise NotImplementedError(f"pack_thresholds only supports GPU tensors, but got {x.device}.")
-    words, pad_len = convlogic_hip.threshold_pack_images(x.float().contiguous(),
-                                                         thresholds.to(x.device, torch.float32).contiguous())
+    thresholds = thresholds.float().contiguous()
+    if thresholds.numel() > convlogic_hip.THRESHOLDS_HOST_MAX or torch.cuda.is_current_stream_capturing():
+        thresholds = thresholds.to(x.device)                         # (a recording must not keep the values of this call)
+    words, pad_len = convlogic_hip.threshold_pack_images(x.float().contiguous(), thresholds)
     return PackBitsTensor.from_image_words(words, pad_len)

@@ -6,37 +6,87 @@
 
 namespace {
 
-constexpr int kLevelsPerPass = 4;
+template <int SAMPLES>
+struct PartWord;
+template <>
+struct PartWord<64> {
+    typedef uint64_t type;
+};
+template <>
+struct PartWord<16> {
+    typedef uint16_t type;
+};
 
-// thread = one element of the [c0, h*w] plane set, blockIdx.y = group of 64 samples, blockIdx.z = pass over
-// four thresholds: lanes read consecutive pixels of one sample (coalesced), 64 samples fill a word.
-__global__ __launch_bounds__(256) void threshold_pack_kernel(const float *__restrict__ x, const float *__restrict__ thr,
+constexpr int kLevelsPerPass = 8;
+
+// Thresholds that the host has at hand travel in the kernel's arguments (no copy to the device, nothing to wait for)
+constexpr int kHostLevels = 64;
+struct HostThresholds {
+    float t[kHostLevels];
+};
+
+// A workgroup takes 256 / SPLIT elements of the [c0, h*w] plane set (blockIdx.x) of one group of 64 samples (blockIdx.y) and up to
+// L thresholds (blockIdx.z); wavefront lanes read consecutive pixels of one sample (coalesced).  SPLIT threads share an
+// element, 64 / SPLIT samples each, and meet in LDS.  Bound by the read of the images; L is the number of thresholds where it is
+// small, so that none is compared in vain (an L of 4 for all cost 165 us at 3 levels, and from 5 levels on a second read of the
+// images).
+template <int L, int SPLIT>
+__global__ __launch_bounds__(256) void threshold_pack_kernel(const float *__restrict__ x, const float *__restrict__ thr, const HostThresholds host,
                                                            uint64_t *__restrict__ words, int64_t n, int64_t plane_elems, int levels)
 {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= plane_elems) return;
+    constexpr int kElems = 256 / SPLIT, kSamples = 64 / SPLIT, kBatch = 16;
+    typedef typename PartWord<kSamples>::type Part;
+    __shared__ Part part[SPLIT > 1 ? SPLIT : 1][SPLIT > 1 ? L : 1][SPLIT > 1 ? kElems : 1];
+    const int lane = threadIdx.x % kElems, q = uniform((int)threadIdx.x / kElems);
+    const int64_t e = (int64_t)blockIdx.x * kElems + lane;
+    const bool live = e < plane_elems;
     const int64_t g = blockIdx.y;
     const int l0 = blockIdx.z * kLevelsPerPass;
-    float t[kLevelsPerPass];
+    float t[L];
 #pragma unroll
-    for (int l = 0; l < kLevelsPerPass; ++l) t[l] = l0 + l < levels ? thr[l0 + l] : 0.0f;
-    uint64_t w[kLevelsPerPass] = {0, 0, 0, 0};
-    const int64_t s0 = g * 64;
-    const int count = n - s0 < 64 ? (int)(n - s0) : 64;
+    for (int l = 0; l < L; ++l) t[l] = l0 + l < levels ? (thr ? thr[l0 + l] : host.t[l0 + l]) : 0.0f;
+    Part w[L];
+#pragma unroll
+    for (int l = 0; l < L; ++l) w[l] = 0;
+    const int64_t s0 = g * 64 + q * kSamples, left = n - s0;
     const float *src = x + s0 * plane_elems + e;
-    for (int s = 0; s < count; s += 8) {
-        float v[8];
+    if (live && left >= kSamples) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = s + j < count ? src[(int64_t)(s + j) * plane_elems] : 0.0f;
+        for (int s = 0; s < kSamples; s += kBatch) {
+            float v[kBatch];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+            for (int j = 0; j < kBatch; ++j) v[j] = src[(int64_t)(s + j) * plane_elems];
 #pragma unroll
-            for (int l = 0; l < kLevelsPerPass; ++l) w[l] |= (uint64_t)(s + j < count && v[j] > t[l]) << (s + j);
+            for (int j = 0; j < kBatch; ++j)
+#pragma unroll
+                for (int l = 0; l < L; ++l) w[l] |= (Part)(v[j] > t[l] ? 1 : 0) << (s + j);
+        }
+    } else if (live) {
+        for (int s = 0; s < left; ++s) {
+            const float v = src[(int64_t)s * plane_elems];
+#pragma unroll
+            for (int l = 0; l < L; ++l) w[l] |= (Part)(v > t[l] ? 1 : 0) << s;
         }
     }
+    if constexpr (SPLIT == 1) {
+        if (!live) return;
 #pragma unroll
-    for (int l = 0; l < kLevelsPerPass; ++l)
-        if (l0 + l < levels) __builtin_nontemporal_store(w[l], &words[(g * levels + l0 + l) * plane_elems + e]);
+        for (int l = 0; l < L; ++l)
+            if (l0 + l < levels) __builtin_nontemporal_store((uint64_t)w[l], &words[(g * levels + l0 + l) * plane_elems + e]);
+    } else {
+#pragma unroll
+        for (int l = 0; l < L; ++l) part[q][l][lane] = w[l];
+        __syncthreads();
+        for (int i = threadIdx.x; i < L * kElems; i += 256) {
+            const int l = i / kElems, el = i % kElems;
+            const int64_t at = (int64_t)blockIdx.x * kElems + el;
+            if (l0 + l >= levels || at >= plane_elems) continue;
+            uint64_t word = 0;
+#pragma unroll
+            for (int j = 0; j < SPLIT; ++j) word |= (uint64_t)part[j][l][el] << (j * kSamples);
+            __builtin_nontemporal_store(word, &words[(g * levels + l0 + l) * plane_elems + at]);
+        }
+    }
 }
 
 __global__ __launch_bounds__(256) void threshold_float_kernel(const float *__restrict__ x, const float *__restrict__ thr,
@@ -60,22 +110,62 @@ int check_threshold_args(const void *x, const void *thr, const void *out, int64_
 
 }  // namespace
 
+namespace {
+template <int L>
+void launch_threshold_pack(const float *x, const float *thr, const HostThresholds &host, uint64_t *words, int64_t n, int64_t plane_elems,
+                           int levels, int64_t groups, hipStream_t st)
+{
+    const unsigned passes = (unsigned)clg_ceil_div(levels, kLevelsPerPass);
+    // Four threads per element: 161 -> 153 us on [65536, 3, 32, 32] with 3 levels (5.8 TB/s), 9.0 -> 4.8 us with 256 images;
+    // one where a level's words alone leave LDS nothing to save and the elements fill the GPU (36 against 40 us on
+    // [65536, 1, 28, 28] with 1 level).
+    const bool split = levels > 1 || clg_ceil_div(plane_elems, 256) * groups < 2048;
+    if (split)
+        hipLaunchKernelGGL((threshold_pack_kernel<L, 4>), dim3((unsigned)clg_ceil_div(plane_elems, 64), (unsigned)groups, passes), dim3(256), 0, st,
+                           x, thr, host, words, n, plane_elems, levels);
+    else
+        hipLaunchKernelGGL((threshold_pack_kernel<L, 1>), dim3((unsigned)clg_ceil_div(plane_elems, 256), (unsigned)groups, passes), dim3(256), 0, st,
+                           x, thr, host, words, n, plane_elems, levels);
+}
+
+int threshold_pack(const char *name, const float *x, const float *thr, const HostThresholds &host, uint64_t *words, int64_t n, int64_t c0,
+                   int64_t hw, int64_t levels, void *stream)
+{
+    const int64_t groups = clg_ceil_div(n, 64), plane_elems = c0 * hw;
+    CLG_REQUIRE(groups <= 65535 * 64ll, "%s: batch too large for one launch", name);
+    // the grid's y extent is limited to 65535: larger batches go in slabs of 65535 groups
+    for (int64_t g0 = 0; g0 < groups; g0 += 65535) {
+        const int64_t gs = groups - g0 < 65535 ? groups - g0 : 65535, left = n - g0 * 64;
+        const float *xs = x + g0 * 64 * plane_elems;
+        uint64_t *ws = words + g0 * levels * plane_elems;
+        if (levels == 1) launch_threshold_pack<1>(xs, thr, host, ws, left, plane_elems, (int)levels, gs, clg_stream(stream));
+        else if (levels == 2) launch_threshold_pack<2>(xs, thr, host, ws, left, plane_elems, (int)levels, gs, clg_stream(stream));
+        else if (levels == 3) launch_threshold_pack<3>(xs, thr, host, ws, left, plane_elems, (int)levels, gs, clg_stream(stream));
+        else if (levels <= 5) launch_threshold_pack<5>(xs, thr, host, ws, left, plane_elems, (int)levels, gs, clg_stream(stream));
+        else launch_threshold_pack<kLevelsPerPass>(xs, thr, host, ws, left, plane_elems, (int)levels, gs, clg_stream(stream));
+        CLG_CHECK_LAUNCH(name);
+    }
+    return CLG_OK;
+}
+}  // namespace
+
 extern "C" int clg_threshold_pack_images(const float *x, const float *thresholds, uint64_t *words, int64_t n, int64_t c0,
                                          int64_t hw, int64_t levels, void *stream)
 {
-    if (int e = check_threshold_args(x, thresholds, words, n, c0, hw, levels, "clg_threshold_pack_images")) return e;
-    const int64_t groups = clg_ceil_div(n, 64), passes = clg_ceil_div(levels, kLevelsPerPass);
-    CLG_REQUIRE(groups <= 65535 * 64ll, "clg_threshold_pack_images: batch too large for one launch");
-    const int64_t plane_elems = c0 * hw;
-    // the grid's y extent is limited to 65535: larger batches go in slabs of 65535 groups
-    for (int64_t g0 = 0; g0 < groups; g0 += 65535) {
-        const int64_t gs = groups - g0 < 65535 ? groups - g0 : 65535;
-        hipLaunchKernelGGL(threshold_pack_kernel, dim3((unsigned)clg_ceil_div(plane_elems, 256), (unsigned)gs, (unsigned)passes),
-                           dim3(256), 0, clg_stream(stream), x + g0 * 64 * plane_elems, thresholds,
-                           words + g0 * levels * plane_elems, n - g0 * 64, plane_elems, (int)levels);
-        CLG_CHECK_LAUNCH("clg_threshold_pack_images");
-    }
-    return CLG_OK;
+    const char *name = "clg_threshold_pack_images";
+    if (int e = check_threshold_args(x, thresholds, words, n, c0, hw, levels, name)) return e;
+    return threshold_pack(name, x, thresholds, HostThresholds{}, words, n, c0, hw, levels, stream);
+}
+
+extern "C" int clg_threshold_pack_images_host(const float *x, const float *thresholds, uint64_t *words, int64_t n, int64_t c0,
+                                              int64_t hw, int64_t levels, void *stream)
+{
+    const char *name = "clg_threshold_pack_images_host";
+    if (int e = check_threshold_args(x, thresholds, words, n, c0, hw, levels, name)) return e;
+    CLG_REQUIRE(levels <= kHostLevels, "%s: at most %d levels", name, kHostLevels);
+    HostThresholds host{};
+    for (int64_t l = 0; l < levels; ++l) host.t[l] = thresholds[l];
+    return threshold_pack(name, x, nullptr, host, words, n, c0, hw, levels, stream);
 }
 
 extern "C" int clg_threshold_images(const float *x, const float *thresholds, float *out, int64_t n, int64_t c0, int64_t hw,

@@ -76,6 +76,7 @@ SIGNATURES = {
     "clg_convblock_forward": (_i, [_i, _GP, _p, _p, _p, _p, _p, _p]),
     "clg_threshold_images": (_i, [_p, _p, _p, _i64, _i64, _i64, _i64, _p]),
     "clg_threshold_pack_images": (_i, [_p, _p, _p, _i64, _i64, _i64, _i64, _p]),
+    "clg_threshold_pack_images_host": (_i, [_p, _p, _p, _i64, _i64, _i64, _i64, _p]),
     "clg_convblock_eval_packed": (_i, [_GP, _p, _p, _p, _p, _p]),
     "clg_convblock_eval_packed_ws": (_i, [_GP, _p, _p, _p, _p, _p, _p]),
     "clg_convblock_eval_packed_scratch_bytes": (_i64, [_GP]),

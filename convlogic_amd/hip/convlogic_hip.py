@@ -485,9 +485,13 @@ def full_convlogic_backward_fm(grad_y_fm, x, weight, argmax, selection, stride_h
 
 
 # ---- input binarisation -------------------------------------------------------------------------
-def _threshold_args(x, thresholds):
+THRESHOLDS_HOST_MAX = 64
+
+
+def _threshold_args(x, thresholds, host=False):
     check_input(x, "x")
-    check_input(thresholds, "thresholds")
+    if not host:
+        check_input(thresholds, "thresholds")
     if x.dtype != torch.float32 or thresholds.dtype != torch.float32 or x.dim() != 4 or thresholds.dim() != 1:
         raise RuntimeError("expected float32 images [N, C, H, W] and float32 thresholds [L]")
     n, c0, h, w = x.shape
@@ -507,13 +511,16 @@ def threshold_images(x, thresholds):
 
 def threshold_pack_images(x, thresholds):
     """float32 [N, C, H, W] -> (int64 words [ceil(N/64), L*C, H, W], pad_len): the thresholded channels
-    packed 64 samples per word, group-major, without materialising them as floats."""
-    n, c0, h, w, levels = _threshold_args(x, thresholds)
+    packed 64 samples per word, group-major, without materialising them as floats.  thresholds: on x's device, or up to
+    THRESHOLDS_HOST_MAX of them in host memory, which then travel in the launch."""
+    host = thresholds.device.type == "cpu" and thresholds.is_contiguous() and thresholds.numel() <= THRESHOLDS_HOST_MAX
+    n, c0, h, w, levels = _threshold_args(x, thresholds, host)
     groups = -(-n // 64)
     out = torch.empty((groups, levels * c0, h, w), dtype=torch.int64, device=x.device)
     if out.numel():
-        check(_lib.load().clg_threshold_pack_images(x.data_ptr(), thresholds.data_ptr(), out.data_ptr(), n, c0, h * w, levels,
-                                                    stream_ptr(x)))
+        lib = _lib.load()
+        call = lib.clg_threshold_pack_images_host if host else lib.clg_threshold_pack_images
+        check(call(x.data_ptr(), thresholds.data_ptr(), out.data_ptr(), n, c0, h * w, levels, stream_ptr(x)))
     return out, groups * 64 - n
 
 

@@ -581,6 +581,10 @@ int clg_threshold_images(const float *x, const float *thresholds, float *out /*[
  * src/difflogic/packbitstensor.py:12-21; the float {0,1} tensor is never materialised. */
 int clg_threshold_pack_images(const float *x, const float *thresholds, uint64_t *words, int64_t n, int64_t c0,
                               int64_t hw, int64_t levels, void *stream);
+/* The same with `thresholds` in HOST memory, at most 64 of them: they are read before the call returns and travel in the
+ * launch itself. */
+int clg_threshold_pack_images_host(const float *x, const float *thresholds, uint64_t *words, int64_t n, int64_t c0,
+                                   int64_t hw, int64_t levels, void *stream);
 
 #ifdef __cplusplus
 }

@@ -32,6 +32,21 @@ def test_threshold_float_and_packed_match_oracle(n, c0, h, w, levels):
     assert torch.equal(ref.t, p.t)
 
 
+@pytest.mark.parametrize("n,side,levels", [(65, 5, 1), (63, 9, 2), (130, 16, 3), (64, 8, 4), (193, 7, 5), (70, 3, 8), (33, 4, 9), (90, 2, 65), (24000, 32, 1)])
+def test_thresholds_in_host_memory_and_on_the_device(n, side, levels):
+    # up to 64 host thresholds travel in the launch; more, and those of a recording, are copied
+    torch.manual_seed(n)
+    x = torch.rand((n, 2, side, side), device=DEV)
+    thr = O.thresholds_uniform(levels)
+    x[0, 0, 0, 0] = thr[-1]
+    want = C.PackBitsTensor(binarize.apply_thresholds(x, thr).bool(), 64).t
+    assert torch.equal(binarize.pack_thresholds(x, thr).t, want)
+    assert torch.equal(binarize.pack_thresholds(x, thr.to(DEV)).t, want)
+    assert torch.equal(binarize.pack_thresholds(x, thr.double()).t, want)
+    strided = torch.stack([thr, thr], 1)[:, 0]
+    assert torch.equal(convlogic_hip.threshold_pack_images(x, thr.to(DEV))[0], want) and torch.equal(binarize.pack_thresholds(x, strided).t, want)
+
+
 def test_thresholds_and_network_input():
     torch.manual_seed(1)
     assert torch.equal(binarize.uniform_thresholds(3), O.thresholds_uniform(3))
