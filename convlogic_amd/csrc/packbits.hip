@@ -380,6 +380,67 @@ __global__ __launch_bounds__(FL *SG) void pack_bits_tile_kernel(const uint8_t *_
     }
 }
 
+// The same for any feature count and alignment, and for batches too small to fill the GPU with 64 samples per thread: lane =
+// sample.  A wavefront reads 64 bytes of 64 consecutive rows (16 bytes per lane and load, at any alignment), and the
+// comparison of one byte in all lanes IS the feature's word, which lane f keeps; SG wavefronts of consecutive sample groups then write
+// runs of 8 SG bytes of every feature row.  Tiles that are neighbours along the features share lines of the input, so every
+// XCD takes a contiguous run of them ([20000, 3000]: 33 -> 22 us).  Bound by latency where there is little to read
+// (bool [10000, 784]: 18.5 us by tiles of 64 samples per thread, 5.9 here; [10000, 785], a byte at a time: 43, 6.2) and by the reads
+// of 64-byte pieces where there is much (3 TB/s).
+template <int SG>
+__global__ __launch_bounds__(SG *kWave) void pack_bits_ballot_kernel(const uint8_t *__restrict__ t, uint8_t *__restrict__ out, int64_t features,
+                                                                    int64_t batch, int64_t row_bytes, unsigned feature_blocks, unsigned per_xcd,
+                                                                    unsigned tiles)
+{
+    constexpr int F = 64;
+    __shared__ uint64_t tile[F][SG + 1];
+    const int lane = threadIdx.x & (kWave - 1), sg = uniform((int)(threadIdx.x >> 6));
+    const unsigned at = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;  // workgroups go round the XCDs
+    if (at >= tiles) return;
+    const int64_t f0 = (int64_t)(at % feature_blocks) * F, grp0 = (int64_t)(at / feature_blocks) * SG;
+    const int64_t s = (grp0 + sg) * 64 + lane;
+    const int count = features - f0 < F ? (int)(features - f0) : F;   // features of this workgroup
+    u32x4 v[F / 16];
+#pragma unroll
+    for (int i = 0; i < F / 16; ++i) v[i] = (u32x4)0u;
+    if (s < batch) {
+        const uint8_t *p = t + s * features + f0;
+#pragma unroll
+        for (int i = 0; i < F / 16; ++i) {
+            if (16 * i + 16 <= count) {                               // uniform
+                __builtin_memcpy(&v[i], p + 16 * i, 16);
+            } else {
+#pragma unroll
+                for (int b = 0; b < 16; ++b)
+                    if (16 * i + b < count) v[i][b / 4] |= (uint32_t)p[16 * i + b] << (8 * (b % 4));
+            }
+        }
+    }
+    uint32_t lo = 0, hi = 0;
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+        const uint64_t word = __ballot((v[f / 16][(f % 16) / 4] & (0xFFu << (8 * (f % 4)))) != 0);
+        lo = lane == f ? (uint32_t)word : lo;
+        hi = lane == f ? (uint32_t)(word >> 32) : hi;
+    }
+    tile[lane][sg] = ((uint64_t)hi << 32) | lo;
+    __syncthreads();
+    const int64_t byte0 = grp0 * 8, run = row_bytes - byte0 < 8 * SG ? row_bytes - byte0 : 8 * SG;
+    if ((row_bytes & 3) == 0 && ((uintptr_t)out & 3) == 0) {          // runs of whole 4-byte pieces
+        for (int i = threadIdx.x; i < F * 2 * SG; i += SG * kWave) {
+            const int f = i / (2 * SG), piece = i % (2 * SG);
+            if (f >= count || 4 * piece >= run) continue;
+            const uint32_t bits = (uint32_t)(tile[f][piece / 2] >> (32 * (piece % 2)));
+            *reinterpret_cast<uint32_t *>(out + (f0 + f) * row_bytes + byte0 + 4 * piece) = bits;
+        }
+    } else {
+        for (int i = threadIdx.x; i < F * 8 * SG; i += SG * kWave) {
+            const int f = i / (8 * SG), b = i % (8 * SG);
+            if (f < count && b < run) out[(f0 + f) * row_bytes + byte0 + b] = (uint8_t)(tile[f][b / 8] >> (8 * (b % 8)));
+        }
+    }
+}
+
 template <int V, int G>
 void launch_pack_smv(const uint8_t *t, void *words, int64_t features, int64_t batch, int64_t row_bytes, int64_t groups, hipStream_t st)
 {
@@ -649,13 +710,22 @@ extern "C" int clg_pack_bits_sample_major(const uint8_t *t, void *words, int64_t
     if (int e = check_pack(t, words, features, batch, bit_count, "clg_pack_bits_sample_major")) return e;
     const int64_t row_bytes = clg_ceil_div(batch, bit_count) * (bit_count / 8);
     const int64_t groups = clg_ceil_div(batch, 64);
-    if (features % 16 == 0 && ((uintptr_t)t & 15) == 0 && ((uintptr_t)words & 7) == 0 && groups <= 65535) {
-        // 16 features per lane, 2 groups per thread: best of 4..16 features x 2..16 groups (3.8 TB/s on bool [8192, 64000])
-        // from 8 groups of 64 samples on, the words go through LDS and leave as 64 (8..15 groups) or 128 contiguous bytes per
-        // feature row: 155 -> 121 us on bool [8192, 64000], 101 -> 52 us on [65536, 4096] with 32 feature lanes x 16 groups
-        // (512 threads; 16 x 16 and 64 x 8 are 8 % slower); CLG_PACK_TILE=0 keeps the direct stores
-        const char *e_tile = clg_knob(K_PACK_TILE);
+    // Large batches of 16-byte aligned rows: 16 features x 64 samples per thread, the words through LDS from 8 groups on (bool
+    // [8192, 64000]: 155 us with direct stores, 121; CLG_PACK_TILE=0 keeps the direct stores).  What does not give these
+    // kernels enough threads, or has rows that are not whole 8-byte words, is faster by ballots.  The lines, tile against
+    // ballot: 67 MB as [65536, 1024] 19.0 and 20.5 us, 60 MB as [20000, 2992] 27 and 20 (rows of 4-byte words: 78 MB 34 and
+    // 24, 157 MB 46 and 43), 32 MB as [2000, 16000] 14.7 and 12.2; direct stores against ballot: [128, 500000] 22 and 26,
+    // [200, 200000] 20 and 15, [64, 200000] 8.5 and 12.
+    const int64_t bytes = features * batch;
+    const char *e_tile = clg_knob(K_PACK_TILE);
+    const bool vectors = features % 16 == 0 && ((uintptr_t)t & 15) == 0 && ((uintptr_t)words & 7) == 0 && groups <= 65535;
+    CLG_REQUIRE(vectors || groups <= 65535ll * kPackGroups, "clg_pack_bits_sample_major: batch above %lld samples is not supported",
+                65535ll * kPackGroups * 64);
+    const bool large = groups >= 8 ? bytes >= ((row_bytes & 7) == 0 ? 48ll << 20 : 160ll << 20)
+                                   : bytes >= 48ll << 20 || (groups == 1 && features > 98304);
+    if (vectors && (e_tile || large)) {
         const bool tiled = !e_tile || atoi(e_tile) != 0;
+        // 32 feature lanes x 16 groups: 101 -> 52 us on [65536, 4096] (512 threads; 16 x 16 and 64 x 8 are 8 % slower)
         if (tiled && groups >= 16)
             hipLaunchKernelGGL((pack_bits_tile_kernel<32, 16>), dim3((unsigned)clg_ceil_div(features, 32 * 16), (unsigned)clg_ceil_div(groups, 16)),
                                dim3(512), 0, clg_stream(stream), t, (uint8_t *)words, features, batch, row_bytes);
@@ -664,11 +734,22 @@ extern "C" int clg_pack_bits_sample_major(const uint8_t *t, void *words, int64_t
                                dim3(256), 0, clg_stream(stream), t, (uint8_t *)words, features, batch, row_bytes);
         else
             launch_pack_smv<4, 2>(t, words, features, batch, row_bytes, groups, clg_stream(stream));
-    } else {
-        const int64_t gy = clg_ceil_div(groups, kPackGroups);
-        CLG_REQUIRE(gy <= 65535, "clg_pack_bits_sample_major: batch above %lld samples is not supported", 65535ll * kPackGroups * 64);
-        hipLaunchKernelGGL(pack_bits_sm_kernel, dim3((unsigned)clg_ceil_div(features, 256), (unsigned)gy), dim3(256), 0,
+    } else if (!vectors && groups <= 4 && features >= 32768) {
+        // few groups of very many features fill the GPU with a thread per feature ([64, 95233]: 4.1 us, 7.3 by ballots)
+        hipLaunchKernelGGL(pack_bits_sm_kernel, dim3((unsigned)clg_ceil_div(features, 256), (unsigned)clg_ceil_div(groups, kPackGroups)), dim3(256), 0,
                            clg_stream(stream), t, (uint8_t *)words, features, batch, row_bytes);
+    } else {
+        // eight groups per workgroup where there are plenty ([65536, 4097]: 155 us with four, 142; [10000, 784]: 5.9 and 6.7)
+        const bool wide = bytes >= 96ll << 20;
+        const int64_t feature_blocks = clg_ceil_div(features, 64), tiles = feature_blocks * clg_ceil_div(groups, wide ? 8 : 4), per_xcd = clg_ceil_div(tiles, 8);
+        CLG_REQUIRE(tiles < (1ll << 28), "clg_pack_bits_sample_major: problem too large for one launch");
+        const dim3 grid((unsigned)(8 * per_xcd));
+        if (wide)
+            hipLaunchKernelGGL((pack_bits_ballot_kernel<8>), grid, dim3(8 * kWave), 0, clg_stream(stream), t, (uint8_t *)words, features, batch,
+                               row_bytes, (unsigned)feature_blocks, (unsigned)per_xcd, (unsigned)tiles);
+        else
+            hipLaunchKernelGGL((pack_bits_ballot_kernel<4>), grid, dim3(4 * kWave), 0, clg_stream(stream), t, (uint8_t *)words, features, batch,
+                               row_bytes, (unsigned)feature_blocks, (unsigned)per_xcd, (unsigned)tiles);
     }
     CLG_CHECK_LAUNCH("clg_pack_bits_sample_major");
     return CLG_OK;

@@ -8,7 +8,7 @@ import torch
 import convlogic_amd as C
 from convlogic_amd.hip import _lib, difflogic_hip
 from oracle import convlogic_oracle as O
-from tests.gpu_util import DEV
+from tests.gpu_util import DEV, set_knobs
 
 pytestmark = pytest.mark.gpu
 TORCH_WORD = {8: torch.int8, 16: torch.int16, 32: torch.int32, 64: torch.int64}
@@ -31,6 +31,39 @@ def test_pack_bits_both_layouts(bits, batch, features):
     assert np.array_equal(w1.cpu().numpy(), want) and np.array_equal(w2.cpu().numpy(), want)
     p = C.PackBitsTensor(tt, bits)
     assert p.pad_len == pad and np.array_equal(p.t.cpu().numpy(), want)
+
+
+def _packed_bytes(t, bits):
+    """words of bool [batch, features] as bytes [features, row bytes], by integer sums"""
+    batch, features = t.shape
+    words = -(-batch // bits)
+    rows = torch.zeros((words * bits, features), dtype=torch.int32, device=t.device)
+    rows[:batch] = t
+    return (rows.view(-1, 8, features) << torch.arange(8, device=t.device, dtype=torch.int32).view(1, 8, 1)).sum(1).to(torch.uint8).t()
+
+
+@pytest.mark.parametrize("tile", [None, "0", "1"])
+@pytest.mark.parametrize("bits,batch,features,offset", [(8, 65, 63, 1), (16, 255, 64, 3), (32, 256, 65, 0), (64, 257, 129, 15), (8, 1030, 48, 0),
+                                                        (32, 2049, 528, 0), (64, 513, 2001, 7), (64, 70, 32769, 0), (64, 300, 33000, 5)])
+def test_pack_bits_ballots_and_tiles(monkeypatch, tile, bits, batch, features, offset):
+    # odd feature counts and addresses, partial last words, groups and feature blocks; the tiles of long aligned rows on the same
+    set_knobs(monkeypatch, CLG_PACK_TILE=tile)
+    torch.manual_seed(batch + features)
+    raw = torch.randint(0, 4, (offset + batch * features,), device=DEV, dtype=torch.uint8)   # any non-zero byte counts as true
+    t = raw.view(torch.bool)[offset:].view(batch, features)
+    want = _packed_bytes(raw[offset:].view(batch, features) != 0, bits)
+    got, pad = difflogic_hip.tensor_packbits_sample_major(t, bits)
+    monkeypatch.undo()
+    _lib.reload_knobs()
+    assert pad == -batch % bits and torch.equal(got.view(torch.uint8).view(features, -1), want)
+
+
+@pytest.mark.parametrize("bits,batch,features", [(64, 1100, 92000), (32, 30020, 3360), (64, 400, 130000), (64, 20001, 5100)])
+def test_pack_bits_large(bits, batch, features):
+    # either side of the lines between ballots of four and eight groups, tiles and direct stores
+    t = torch.rand((batch, features), device=DEV) < 0.5
+    got, _ = difflogic_hip.tensor_packbits_sample_major(t, bits)
+    assert torch.equal(got.view(torch.uint8).view(features, -1), _packed_bytes(t, bits))
 
 
 @pytest.mark.parametrize("bits,batch", [(64, 4096), (64, 100), (32, 1000), (16, 48), (8, 8), (8, 24), (32, 96)])
