@@ -390,10 +390,7 @@ class ConvLogicLayer(nn.Module):
         if (self.__dict__.get("binary_input") and self.complete and not self.return_intermediate and not self.return_indices
                 and x.is_cuda and x.dtype == torch.float32 and weights.dtype == torch.float32 and weights.device == x.device
                 and sel.device == x.device and convlogic_hip.bin_supported(x, self.out_channels, *geo)):
-            flag = self._binary_flag()
-            if flag.raised():
-                flag.clear()
-                raise RuntimeError("ConvLogicLayer(binary_input=True) was given an input with elements other than 0 and 1")
+            flag = self.binary_flag_checked()
             if self.training and weights.is_contiguous():
                 return _FullConvLogicBinaryFunction.apply(x, weights, sel, *geo, True, flag)
             w_prob = kernel_probabilities(self.weights, self.training, x.dtype)
@@ -408,6 +405,14 @@ class ConvLogicLayer(nn.Module):
         if self.complete:
             return FullConvLogicFunction.apply(x, w_prob, sel, *geo, self.return_intermediate, self.return_indices)
         return ConvLogicFunction.apply(x, w_prob, sel, *geo)
+
+    def binary_flag_checked(self):
+        """The layer's flag; raises when an earlier call has set it."""
+        flag = self._binary_flag()
+        if flag.raised():
+            flag.clear()
+            raise RuntimeError("ConvLogicLayer(binary_input=True) was given an input with elements other than 0 and 1")
+        return flag
 
     def _binary_flag(self):
         flag = self.__dict__.get("_bin_flag")

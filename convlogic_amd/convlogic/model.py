@@ -12,6 +12,8 @@ from ..difflogic import GroupSum, LogicLayer
 from ..difflogic.difflogic import _feature_major, logic_layer_group_sum
 from ..difflogic.fc_tree import tree_eval, tree_packed, tree_plan, tree_train
 from ..difflogic.packbitstensor import PackBitsTensor
+from ..hip.convlogic_hip import bin_supported
+from . import packed_net
 from .convlogic_layer import ConvLogicLayer
 
 
@@ -97,9 +99,12 @@ def _forward(owner, x):
         plan = tree_plan(*tail[0]) if trees else None
         if plan is None:
             return net(x)
+        counts = _counts_at_once(net, tail, plan, x)
+        if counts is not None:
+            return counts
         h = _head_of(net, x)
         if (type(h) is not PackBitsTensor or h.image or h.t.shape[0] != tail[0][0].in_dim or not h.t.is_contiguous()
-                or h.t.device != tail[0][0]._parameters["weights"].device or _many_small_classes(plan.roots, tail[1].k, h)):
+                or h.t.device != tail[0][0]._parameters["weights"].device or _many_small_classes(plan.roots, tail[1].k, h.t.shape[1])):
             return _rest(net, h)
         return tree_packed(tail[0], tail[1].k, h, plan)
     if not (isinstance(x, torch.Tensor) and x.is_cuda):
@@ -108,6 +113,9 @@ def _forward(owner, x):
     if not (owner.training and torch.is_grad_enabled()):
         if not trees or any(m.training for m in tail[0]) or (plan := tree_plan(*tail[0])) is None:
             return net(x)
+        out = _sums_at_once(net, tail, plan, x)
+        if out is not None:
+            return out
         h = _head_of(net, x)
         if _trees_take(h, tail[0][0]):
             return tree_eval(tail[0], tail[1], _feature_major(h.detach()), plan)
@@ -134,12 +142,49 @@ def _forward(owner, x):
     return net(x)
 
 
+def _counts_at_once(net, tail, plan, x):
+    """Class counts of packed images with every module of the network in one call (packed_net), or None where the modules have to be
+    called.  x holds the words in front of the trees afterwards, as after the modules."""
+    t, (layers, gs) = x.t, tail
+    if not (type(x) is PackBitsTensor and x.image and t.dim() == 4 and t.dtype == torch.int64 and t.is_contiguous() and t.shape[0] > 0
+            and 0 <= x.pad_len < 64):
+        return None
+    blocks = packed_net.blocks_of(net, _called_for_itself)
+    if blocks is None or t.device != blocks[0]._parameters["weights"].device or t.device != layers[0]._parameters["weights"].device:
+        return None
+    geoms = packed_net.geometries(blocks, *t.shape, layers[0].in_dim)
+    if geoms is None or _many_small_classes(plan.roots, gs.k, t.shape[0]):
+        return None
+    x.t, counts = packed_net.evaluate(blocks, geoms, t, layers, plan, gs.k, t.shape[0] * 64 - x.pad_len)
+    x.image = False
+    return counts
+
+
+def _sums_at_once(net, tail, plan, x):
+    """Class sums of 0/1 images (the first block's binary_input, verified by the kernels) on packed bits, or None.  Against the float
+    kernels: 245 -> 90 us of device time for 1000 images of the k = 32 CIFAR network, 1365 -> 160 at k = 128; small batches of the
+    smallest networks leave the words' kernels short of work (k = 8, 128 images: 58 and 63 us)."""
+    layers, gs = tail
+    if x.dim() != 4 or not (x.shape[0] >= 192 or plan.roots >= 8192) or x.shape[0] > 65535 * 64 or gs.k >= 512:
+        return None
+    blocks = packed_net.blocks_of(net, _called_for_itself)
+    if blocks is None or not blocks[0].__dict__.get("binary_input") or not (
+            x.device == blocks[0]._parameters["weights"].device == layers[0]._parameters["weights"].device):
+        return None
+    n, c, h, w = x.shape
+    first = blocks[0]
+    geoms = packed_net.geometries(blocks, -(-n // 64), c, h, w, layers[0].in_dim)
+    if geoms is None or not bin_supported(x, first.out_channels, *first.stride, *first.padding, *first.kernel):
+        return None
+    return packed_net.evaluate_images(blocks, geoms, x.contiguous(), layers, gs, plan)
+
+
 def _many_small_classes(roots, k, words):
     """True for packed words on which the modules are the faster ones: the trees' workgroups each add up the counts of a class,
     which costs as much for one root as for hundreds (1000 classes of one root, 256 samples: 22 us, 13 by the modules; of
     16 roots: 34 and 37; of one root, 20 000 samples: 149 and 288)."""
     rows = roots // k
-    return k >= 512 and rows <= 16 and rows * words.t.shape[1] * 64 <= 4096
+    return k >= 512 and rows <= 16 and rows * words * 64 <= 4096
 
 
 def _trees_take(h, first):

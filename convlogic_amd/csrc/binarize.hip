@@ -30,9 +30,11 @@ struct HostThresholds {
 // element, 64 / SPLIT samples each, and meet in LDS.  Bound by the read of the images; L is the number of thresholds where it is
 // small, so that none is compared in vain (an L of 4 for all cost 165 us at 3 levels, and from 5 levels on a second read of the
 // images).
-template <int L, int SPLIT>
+// BINARY: images that hold 0 and 1 already (any other value is a 1 and sets *bad).
+template <int L, int SPLIT, bool BINARY = false>
 __global__ __launch_bounds__(256) void threshold_pack_kernel(const float *__restrict__ x, const float *__restrict__ thr, const HostThresholds host,
-                                                           uint64_t *__restrict__ words, int64_t n, int64_t plane_elems, int levels)
+                                                           uint64_t *__restrict__ words, int64_t n, int64_t plane_elems, int levels,
+                                                           int32_t *__restrict__ bad = nullptr)
 {
     constexpr int kElems = 256 / SPLIT, kSamples = 64 / SPLIT, kBatch = 16;
     typedef typename PartWord<kSamples>::type Part;
@@ -50,6 +52,15 @@ __global__ __launch_bounds__(256) void threshold_pack_kernel(const float *__rest
     for (int l = 0; l < L; ++l) w[l] = 0;
     const int64_t s0 = g * 64 + q * kSamples, left = n - s0;
     const float *src = x + s0 * plane_elems + e;
+    bool other = false;
+    auto bit = [&](float v, float threshold) {
+        if constexpr (BINARY) {
+            other = other || (v != 0.f && v != 1.f);
+            return v != 0.f;
+        } else {
+            return v > threshold;
+        }
+    };
     if (live && left >= kSamples) {
 #pragma unroll
         for (int s = 0; s < kSamples; s += kBatch) {
@@ -59,15 +70,16 @@ __global__ __launch_bounds__(256) void threshold_pack_kernel(const float *__rest
 #pragma unroll
             for (int j = 0; j < kBatch; ++j)
 #pragma unroll
-                for (int l = 0; l < L; ++l) w[l] |= (Part)(v[j] > t[l] ? 1 : 0) << (s + j);
+                for (int l = 0; l < L; ++l) w[l] |= (Part)(bit(v[j], t[l]) ? 1 : 0) << (s + j);
         }
     } else if (live) {
         for (int s = 0; s < left; ++s) {
             const float v = src[(int64_t)s * plane_elems];
 #pragma unroll
-            for (int l = 0; l < L; ++l) w[l] |= (Part)(v > t[l] ? 1 : 0) << s;
+            for (int l = 0; l < L; ++l) w[l] |= (Part)(bit(v, t[l]) ? 1 : 0) << s;
         }
     }
+    if (BINARY && other) *bad = 1;
     if constexpr (SPLIT == 1) {
         if (!live) return;
 #pragma unroll
@@ -122,10 +134,10 @@ void launch_threshold_pack(const float *x, const float *thr, const HostThreshold
     const bool split = levels > 1 || clg_ceil_div(plane_elems, 256) * groups < 2048;
     if (split)
         hipLaunchKernelGGL((threshold_pack_kernel<L, 4>), dim3((unsigned)clg_ceil_div(plane_elems, 64), (unsigned)groups, passes), dim3(256), 0, st,
-                           x, thr, host, words, n, plane_elems, levels);
+                           x, thr, host, words, n, plane_elems, levels, (int32_t *)nullptr);
     else
         hipLaunchKernelGGL((threshold_pack_kernel<L, 1>), dim3((unsigned)clg_ceil_div(plane_elems, 256), (unsigned)groups, passes), dim3(256), 0, st,
-                           x, thr, host, words, n, plane_elems, levels);
+                           x, thr, host, words, n, plane_elems, levels, (int32_t *)nullptr);
 }
 
 int threshold_pack(const char *name, const float *x, const float *thr, const HostThresholds &host, uint64_t *words, int64_t n, int64_t c0,
@@ -166,6 +178,22 @@ extern "C" int clg_threshold_pack_images_host(const float *x, const float *thres
     HostThresholds host{};
     for (int64_t l = 0; l < levels; ++l) host.t[l] = thresholds[l];
     return threshold_pack(name, x, nullptr, host, words, n, c0, hw, levels, stream);
+}
+
+extern "C" int clg_pack_binary_images(const float *x, uint64_t *words, int64_t n, int64_t c0, int64_t hw, int32_t *not_binary, void *stream)
+{
+    const char *name = "clg_pack_binary_images";
+    if (int e = check_threshold_args(x, not_binary, words, n, c0, hw, 1, name)) return e;
+    const int64_t groups = clg_ceil_div(n, 64), plane_elems = c0 * hw;
+    CLG_REQUIRE(groups <= 65535, "%s: batch too large for one launch", name);
+    if (clg_ceil_div(plane_elems, 256) * groups < 2048)              // (the split as for one threshold)
+        hipLaunchKernelGGL((threshold_pack_kernel<1, 4, true>), dim3((unsigned)clg_ceil_div(plane_elems, 64), (unsigned)groups), dim3(256), 0,
+                           clg_stream(stream), x, (const float *)nullptr, HostThresholds{}, words, n, plane_elems, 1, not_binary);
+    else
+        hipLaunchKernelGGL((threshold_pack_kernel<1, 1, true>), dim3((unsigned)clg_ceil_div(plane_elems, 256), (unsigned)groups), dim3(256), 0,
+                           clg_stream(stream), x, (const float *)nullptr, HostThresholds{}, words, n, plane_elems, 1, not_binary);
+    CLG_CHECK_LAUNCH(name);
+    return CLG_OK;
 }
 
 extern "C" int clg_threshold_images(const float *x, const float *thresholds, float *out, int64_t n, int64_t c0, int64_t hw,

@@ -586,11 +586,29 @@ extern "C" int clg_fc_tree_backward(const float *x, const int32_t *rows, const i
 // the counting kernel: 273 us).
 namespace {
 
+// The logits of the blocks in front of the trees, whose gate ids the same launch finds (one thread per gate, in the workgroups from
+// tree_blocks on): one launch of 5 us for a network in place of one per block.
+constexpr int kMaxNetBlocks = 16;
+struct NetGates {
+    const float *logits[kMaxNetBlocks];
+    uint8_t *ids[kMaxNetBlocks];
+    int64_t end[kMaxNetBlocks];   // gates up to and including the block's
+    int blocks, tree_blocks;
+};
 __global__ __launch_bounds__(256) void fc_tree_codes_kernel(TreeLogits lg, const int32_t *__restrict__ ids, uint32_t *__restrict__ codes,
-                                                          int roots, int32_t *__restrict__ counts, int64_t n_counts)
+                                                          int roots, int32_t *__restrict__ counts, int64_t n_counts, NetGates net)
 {
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
     for (int64_t i = e; i < n_counts; i += (int64_t)gridDim.x * 256) counts[i] = 0;   // (for the counting kernel's atomics)
+    if ((int)blockIdx.x >= net.tree_blocks) {
+        const int64_t at = e - (int64_t)net.tree_blocks * 256;
+        int64_t first = 0;
+        for (int b = 0; b < net.blocks; ++b) {
+            if (at >= first && at < net.end[b]) net.ids[b][at - first] = (uint8_t)argmax16(net.logits[b] + (at - first) * 16);
+            first = net.end[b];
+        }
+        return;
+    }
     const int j = (int)(e >> 3), q = (int)(e & 7);                    // eight lanes per root, one gate each
     int id = 0;
     if (j < roots && q < 7) id = argmax16(tree_logits(lg, ids, j, q, roots));
@@ -622,6 +640,7 @@ __device__ __forceinline__ void add_counts(uint32_t (&plane)[kTreePlanes], const
 template <bool WIDE>
 __global__ __launch_bounds__(kPackedWaves *kWave) void fc_tree_packed_kernel(const uint32_t *__restrict__ x, const int32_t *__restrict__ rows,
                                                                             const uint32_t *__restrict__ codes, int32_t *__restrict__ out,
+                                                                            float *__restrict__ sums, float inv_tau,
                                                                             int class_rows, int k, int slices, uint32_t words,
                                                                             int64_t samples, int in_dim, int cols_log2, unsigned col_blocks)
 {
@@ -710,9 +729,76 @@ __global__ __launch_bounds__(kPackedWaves *kWave) void fc_tree_packed_kernel(con
         int32_t cnt = 0;
 #pragma unroll
         for (int q = 0; q < kTreePlanes; ++q) cnt |= (int32_t)((total[q] >> b) & 1) << q;
-        if (slices == 1) out[s * k + g] = cnt;
-        else atomicAdd(out + s * k + g, cnt);
+        if (slices > 1) atomicAdd(out + s * k + g, cnt);
+        else if (sums != nullptr) sums[s * k + g] = (float)cnt * inv_tau;
+        else out[s * k + g] = cnt;
     }
+}
+
+__global__ __launch_bounds__(256) void fc_tree_sums_kernel(const int32_t *__restrict__ counts, float *__restrict__ sums, int64_t n, float inv_tau)
+{
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e < n) sums[e] = (float)counts[e] * inv_tau;
+}
+
+// How a launch is cut: columns of 32-bit words per workgroup, slices of a class
+struct PackedCut {
+    int cols_log2;
+    int64_t col_blocks, slices;
+};
+PackedCut cut_packed(int64_t roots, int64_t k, int64_t words)
+{
+    const int64_t class_rows = roots / k, halves = words * 2;        // 32-bit words of a row: a lane takes one
+    PackedCut c;
+    c.cols_log2 = 6;
+    while (c.cols_log2 > 0 && (1ll << (c.cols_log2 - 1)) >= halves) --c.cols_log2;
+    c.col_blocks = clg_ceil_div(halves, 1ll << c.cols_log2);
+    // One workgroup takes all roots of its columns and class where that gives half of the CUs one; else the classes are sliced
+    // down to two steps of roots per wavefront, and the slices meet in atomics.  (Twelve slices of a class at 65 536 samples:
+    // 7.9 M atomics, 385 us instead of 66.)  A workgroup takes at most 2^14 - 4 roots.
+    const int64_t phases = 64 >> c.cols_log2;
+    int64_t slices = k * c.col_blocks >= 128 ? 1 : clg_ceil_div(512, k * c.col_blocks);
+    slices = std::min(slices, class_rows / (8 * phases * kPackedWaves));
+    c.slices = std::max<int64_t>(std::max<int64_t>(slices, clg_ceil_div(class_rows, (1 << kTreePlanes) - 4)), 1);
+    return c;
+}
+
+// counts (int32) or sums (float, counts / tau; where classes are sliced, counts are scratch then) of packed words
+int count_packed(const char *name, const int64_t *x, const int32_t *rows, const uint32_t *codes, int32_t *counts,
+                 float *sums, float inv_tau, int64_t in_dim, int64_t roots, int64_t k, int64_t words, int64_t samples, const PackedCut &c,
+                 hipStream_t st)
+{
+#define CLG_TREE_P(WIDE)                                                                                                      \
+    hipLaunchKernelGGL((fc_tree_packed_kernel<WIDE>), dim3((unsigned)(k * c.slices * c.col_blocks)), dim3(kPackedWaves * kWave), 0, st, \
+                       (const uint32_t *)x, rows, codes, counts, sums, inv_tau, (int)(roots / k), (int)k, (int)c.slices, (uint32_t)(words * 2), \
+                       samples, (int)in_dim, c.cols_log2, (unsigned)c.col_blocks)
+    if (c.cols_log2 == 6) CLG_TREE_P(true);
+    else CLG_TREE_P(false);
+#undef CLG_TREE_P
+    CLG_CHECK_LAUNCH(name);
+    if (sums != nullptr && c.slices > 1) {
+        hipLaunchKernelGGL(fc_tree_sums_kernel, dim3((unsigned)clg_ceil_div(samples * k, 256)), dim3(256), 0, st, (const int32_t *)counts, sums,
+                           samples * k, inv_tau);
+        CLG_CHECK_LAUNCH(name);
+    }
+    return CLG_OK;
+}
+
+int make_codes(const char *name, const TreeLogits &lg, const int32_t *ids, uint32_t *codes, int64_t roots, int32_t *counts, int64_t n_counts,
+               NetGates net, hipStream_t st)
+{
+    net.tree_blocks = (int)clg_ceil_div(roots * 8, 256);
+    const int64_t gate_blocks = net.blocks ? clg_ceil_div(net.end[net.blocks - 1], 256) : 0;
+    hipLaunchKernelGGL(fc_tree_codes_kernel, dim3((unsigned)(net.tree_blocks + gate_blocks)), dim3(256), 0, st, lg, ids, codes, (int)roots,
+                       counts, n_counts, net);
+    CLG_CHECK_LAUNCH(name);
+    return CLG_OK;
+}
+
+int check_packed(const char *name, int64_t k, int64_t words, const PackedCut &c)
+{
+    CLG_REQUIRE(k * c.slices * c.col_blocks < (1ll << 28) && words < (1ll << 30), "%s: problem too large for one launch", name);
+    return CLG_OK;
 }
 
 }  // namespace
@@ -726,31 +812,109 @@ extern "C" int clg_fc_tree_packed(const int64_t *x, const int32_t *rows, const i
     CLG_REQUIRE(x && rows && ids && logits0 && logits1 && logits2 && codes && out, "%s: null pointer argument", name);
     CLG_REQUIRE(words > 0 && samples > 0 && samples <= words * 64 && words < (1ll << 31), "%s: words %lld, samples %lld", name,
                 (long long)words, (long long)samples);
+    const PackedCut c = cut_packed(roots, k, words);
+    if (int e = check_packed(name, k, words, c)) return e;
     hipStream_t st = clg_stream(stream);
-    const int64_t class_rows = roots / k;
-    const int64_t halves = words * 2;                                // 32-bit words of a row: a lane takes one
-    int cols_log2 = 6;
-    while (cols_log2 > 0 && (1ll << (cols_log2 - 1)) >= halves) --cols_log2;
-    const int64_t col_blocks = clg_ceil_div(halves, 1ll << cols_log2);
-    // One workgroup takes all roots of its columns and class where that gives half of the CUs one; else the classes are sliced
-    // down to two steps of roots per wavefront, and the slices meet in atomics.  (Twelve slices of a class at 65 536 samples:
-    // 7.9 M atomics, 385 us instead of 66.)  A workgroup takes at most 2^14 - 4 roots.
-    const int64_t phases = 64 >> cols_log2;
-    int64_t slices = k * col_blocks >= 128 ? 1 : clg_ceil_div(512, k * col_blocks);
-    slices = std::min(slices, class_rows / (8 * phases * kPackedWaves));
-    slices = std::max<int64_t>(std::max<int64_t>(slices, clg_ceil_div(class_rows, (1 << kTreePlanes) - 4)), 1);
-    const int64_t blocks = k * slices * col_blocks;
-    CLG_REQUIRE(blocks < (1ll << 28) && halves < (1ll << 31), "%s: problem too large for one launch", name);
     const TreeLogits lg = {{logits0, logits1, logits2}};
-    hipLaunchKernelGGL(fc_tree_codes_kernel, dim3((unsigned)clg_ceil_div(roots * 8, 256)), dim3(256), 0, st, lg, ids, codes, (int)roots, out,
-                       slices > 1 ? samples * k : (int64_t)0);
-    CLG_CHECK_LAUNCH(name);
-#define CLG_TREE_P(WIDE)                                                                                                      \
-    hipLaunchKernelGGL((fc_tree_packed_kernel<WIDE>), dim3((unsigned)blocks), dim3(kPackedWaves * kWave), 0, st, (const uint32_t *)x, rows, \
-                       codes, out, (int)class_rows, (int)k, (int)slices, (uint32_t)halves, samples, (int)in_dim, cols_log2, (unsigned)col_blocks)
-    if (cols_log2 == 6) CLG_TREE_P(true);
-    else CLG_TREE_P(false);
-#undef CLG_TREE_P
-    CLG_CHECK_LAUNCH(name);
+    if (int e = make_codes(name, lg, ids, codes, roots, out, c.slices > 1 ? samples * k : (int64_t)0, NetGates{}, st)) return e;
+    return count_packed(name, x, rows, codes, out, nullptr, 0.f, in_dim, roots, k, words, samples, c, st);
+}
+
+// ---- a whole network on packed words -----------------------------------------------------------------------------------------
+// Blocks, flattening and trees in one call: the launches of the modules without the host's work between them, and the gate ids
+// of all blocks and trees in one launch.
+namespace {
+
+size_t net_up(size_t v) { return (v + 255) & ~(size_t)255; }
+struct NetLayout {
+    size_t gates_off[kMaxNetBlocks], codes_off, counts_off, ping_off, pong_off, ws_off, total;
+};
+
+// checks the blocks against each other and lays the scratch out: gate ids | codes | counts | two activations | a block's scratch
+int net_layout(const char *name, const clg_packed_block *blocks, int n_blocks, int64_t in_dim, int64_t roots, int64_t k, int64_t samples,
+               NetLayout *l)
+{
+    CLG_REQUIRE(blocks && n_blocks > 0 && n_blocks <= kMaxNetBlocks, "%s: 1 to %d blocks", name, kMaxNetBlocks);
+    size_t at = 0, act[2] = {0, 0}, ws = 0;
+    int64_t c = 0, h = 0, w = 0;
+    for (int b = 0; b < n_blocks; ++b) {
+        const clg_conv_geom &gg = blocks[b].geom;
+        CLG_REQUIRE(b == 0 || (gg.n == blocks[0].geom.n && gg.c_in == c && gg.h == h && gg.w == w), "%s: block %d does not take the output of the one before",
+                    name, b);
+        const int64_t need = clg_convblock_eval_packed_scratch_bytes(&gg);
+        if (need < 0) return CLG_EINVAL;
+        ws = std::max(ws, (size_t)need);
+        c = gg.c_out;
+        h = ((gg.h + 2 * gg.pad_h - gg.kernel_h) / gg.stride_h + 1) / 2;
+        w = ((gg.w + 2 * gg.pad_w - gg.kernel_w) / gg.stride_w + 1) / 2;
+        l->gates_off[b] = at;
+        at += net_up((size_t)c * 7);
+        act[b & 1] = std::max(act[b & 1], (size_t)gg.n * c * h * w * 8);
+    }
+    CLG_REQUIRE(c * h * w == in_dim, "%s: the last block gives %lld features, the trees take %lld", name, (long long)(c * h * w), (long long)in_dim);
+    const PackedCut cut = cut_packed(roots, k, blocks[0].geom.n);
+    l->codes_off = at;
+    l->counts_off = l->codes_off + net_up((size_t)roots * 4);
+    l->ping_off = l->counts_off + (cut.slices > 1 ? net_up((size_t)samples * k * 4) : 0);
+    l->pong_off = l->ping_off + net_up(act[0]);
+    l->ws_off = l->pong_off + net_up(act[1]);
+    l->total = l->ws_off + net_up(ws);
     return CLG_OK;
+}
+
+}  // namespace
+
+extern "C" int64_t clg_net_packed_scratch_bytes(const clg_packed_block *blocks, int n_blocks, int64_t in_dim, int64_t roots, int64_t k,
+                                                int64_t samples)
+{
+    const char *name = "clg_net_packed_scratch_bytes";
+    if (check_tree(name, in_dim, roots, k)) return -1;
+    NetLayout l;
+    return net_layout(name, blocks, n_blocks, in_dim, roots, k, samples, &l) ? -1 : (int64_t)l.total;
+}
+
+extern "C" int clg_net_packed(const clg_packed_block *blocks, int n_blocks, const int64_t *x, const int32_t *rows, const int32_t *ids,
+                              const float *logits0, const float *logits1, const float *logits2, int64_t *features, int32_t *counts, float *sums,
+                              double tau, int64_t in_dim, int64_t roots, int64_t k, int64_t samples, void *scratch, void *stream)
+{
+    const char *name = "clg_net_packed";
+    if (int e = check_tree(name, in_dim, roots, k)) return e;
+    NetLayout l;
+    if (int e = net_layout(name, blocks, n_blocks, in_dim, roots, k, samples, &l)) return e;
+    const int64_t words = blocks[0].geom.n;
+    CLG_REQUIRE(x && rows && ids && logits0 && logits1 && logits2 && features && scratch && (counts != nullptr) != (sums != nullptr),
+                "%s: null pointer argument, or both or neither of counts and sums", name);
+    CLG_REQUIRE(samples > 0 && samples <= words * 64 && (sums == nullptr || tau != 0.0), "%s: words %lld, samples %lld, tau %g", name,
+                (long long)words, (long long)samples, tau);
+    const PackedCut c = cut_packed(roots, k, words);
+    if (int e = check_packed(name, k, words, c)) return e;
+    unsigned char *base = reinterpret_cast<unsigned char *>(scratch);
+    NetGates net{};
+    net.blocks = n_blocks;
+    int64_t gates = 0;
+    for (int b = 0; b < n_blocks; ++b) {
+        CLG_REQUIRE(blocks[b].logits && blocks[b].selection, "%s: null pointer in block %d", name, b);
+        net.logits[b] = blocks[b].logits;
+        net.ids[b] = base + l.gates_off[b];
+        net.end[b] = gates += (int64_t)blocks[b].geom.c_out * 7;
+    }
+    hipStream_t st = clg_stream(stream);
+    const TreeLogits lg = {{logits0, logits1, logits2}};
+    uint32_t *codes = reinterpret_cast<uint32_t *>(base + l.codes_off);
+    int32_t *meet = counts != nullptr ? counts : reinterpret_cast<int32_t *>(base + l.counts_off);
+    if (int e = make_codes(name, lg, ids, codes, roots, meet, c.slices > 1 ? samples * k : (int64_t)0, net, st)) return e;
+    const uint64_t *in = reinterpret_cast<const uint64_t *>(x);
+    bool flat = false;                                                // the last block wrote its words feature-major
+    for (int b = 0; b < n_blocks; ++b) {
+        const clg_packed_block &bl = blocks[b];
+        uint64_t *out = reinterpret_cast<uint64_t *>(base + ((b & 1) ? l.pong_off : l.ping_off));
+        flat = b == n_blocks - 1 && clg_convblock_eval_packed_fm_supported(&bl.geom);
+        const int e = flat ? clg_convblock_eval_packed_fm(&bl.geom, in, net.ids[b], bl.selection, reinterpret_cast<uint64_t *>(features), stream)
+                           : clg_convblock_eval_packed_ws(&bl.geom, in, net.ids[b], bl.selection, out, base + l.ws_off, stream);
+        if (e) return e;
+        in = out;
+    }
+    if (!flat)
+        if (int e = clg_transpose_2d(8, in, features, words, in_dim, stream)) return e;
+    return count_packed(name, features, rows, codes, meet, sums, sums != nullptr ? 1.f / (float)tau : 0.f, in_dim, roots, k, words, samples, c, st);
 }

@@ -25,6 +25,11 @@ class ConvGeom(ctypes.Structure):
 
 _GP = ctypes.POINTER(ConvGeom)
 
+
+class PackedBlock(ctypes.Structure):
+    _fields_ = [("geom", ConvGeom), ("logits", _p), ("selection", _p)]
+
+
 # name -> (restype, argtypes); every symbol include/convlogic_amd.h declares
 SIGNATURES = {
     "clg_last_error": (ctypes.c_char_p, []),
@@ -76,6 +81,7 @@ SIGNATURES = {
     "clg_convblock_forward": (_i, [_i, _GP, _p, _p, _p, _p, _p, _p]),
     "clg_threshold_images": (_i, [_p, _p, _p, _i64, _i64, _i64, _i64, _p]),
     "clg_threshold_pack_images": (_i, [_p, _p, _p, _i64, _i64, _i64, _i64, _p]),
+    "clg_pack_binary_images": (_i, [_p, _p, _i64, _i64, _i64, _p, _p]),
     "clg_threshold_pack_images_host": (_i, [_p, _p, _p, _i64, _i64, _i64, _i64, _p]),
     "clg_convblock_eval_packed": (_i, [_GP, _p, _p, _p, _p, _p]),
     "clg_convblock_eval_packed_ws": (_i, [_GP, _p, _p, _p, _p, _p, _p]),
@@ -118,6 +124,8 @@ SIGNATURES = {
     "clg_fc_tree_forward": (_i, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _f64, _p]),
     "clg_fc_tree_backward": (_i, [_p] * 14 + [_i64, _i64, _i64, _i64, _i64, _f64, _p]),
     "clg_fc_tree_packed": (_i, [_p] * 8 + [_i64, _i64, _i64, _i64, _i64, _p]),
+    "clg_net_packed_scratch_bytes": (_i64, [_p, _i, _i64, _i64, _i64, _i64]),
+    "clg_net_packed": (_i, [_p, _i] + [_p] * 9 + [_f64, _i64, _i64, _i64, _i64, _p, _p]),
 }
 
 _lib = None

@@ -558,6 +558,22 @@ int clg_fc_tree_backward(const float *x, const int32_t *rows, const int32_t *pos
 int clg_fc_tree_packed(const int64_t *x, const int32_t *rows, const int32_t *ids, const float *logits0, const float *logits1,
                        const float *logits2, uint32_t *codes, int32_t *out, int64_t in_dim, int64_t roots, int64_t k,
                        int64_t words, int64_t samples, void *stream);
+
+/* A whole network on packed words in one call: blocks (arg-max gates), flattening, trees and class counts. */
+typedef struct clg_packed_block {
+    clg_conv_geom geom;       /* n = groups of 64 samples; each block takes the output of the one before */
+    const float *logits;      /* [c_out, 7, 16] */
+    const int32_t *selection; /* [c_out, 8] */
+} clg_packed_block;
+/* bytes of `scratch` of clg_net_packed; negative for bad arguments */
+int64_t clg_net_packed_scratch_bytes(const clg_packed_block *blocks, int n_blocks, int64_t in_dim, int64_t roots, int64_t k, int64_t samples);
+/* x: words [n, c_in, h, w] of the first block; rows, ids, logits0..2: the trees, as for clg_fc_tree_packed.  features takes the words
+ * between blocks and trees, [in_dim, n]; counts int32 [samples, k], or sums float [samples, k] = counts / tau, the other one NULL.
+ * At most 16 blocks. */
+int clg_net_packed(const clg_packed_block *blocks, int n_blocks, const int64_t *x, const int32_t *rows, const int32_t *ids,
+                   const float *logits0, const float *logits1, const float *logits2, int64_t *features, int32_t *counts, float *sums,
+                   double tau, int64_t in_dim, int64_t roots, int64_t k, int64_t samples, void *scratch, void *stream);
+
 int64_t clg_convblock_bin_ctx_bytes(int dtype, const clg_conv_geom *g);
 int clg_convblock_bin_forward(int dtype, const clg_conv_geom *g, const void *x, const void *w, const int32_t *selection, void *y,
                               uint16_t *taps, void *ctx, int flags, int32_t *not_binary, void *stream);
@@ -581,8 +597,11 @@ int clg_threshold_images(const float *x, const float *thresholds, float *out /*[
  * src/difflogic/packbitstensor.py:12-21; the float {0,1} tensor is never materialised. */
 int clg_threshold_pack_images(const float *x, const float *thresholds, uint64_t *words, int64_t n, int64_t c0,
                               int64_t hw, int64_t levels, void *stream);
-/* The same with `thresholds` in HOST memory, at most 64 of them: they are read before the call returns and travel in the
- * launch itself. */
+/* Images of 0 and 1 into the same words: a bit is set where x is not 0; an x that is neither sets *not_binary to 1 (device memory, or
+ * pinned host memory by clg_host_flag_device_pointer).  At most 65535 groups. */
+int clg_pack_binary_images(const float *x, uint64_t *words, int64_t n, int64_t c0, int64_t hw, int32_t *not_binary, void *stream);
+/* clg_threshold_pack_images with `thresholds` in HOST memory, at most 64 of them: they are read before the call returns and
+ * travel in the launch itself. */
 int clg_threshold_pack_images_host(const float *x, const float *thresholds, uint64_t *words, int64_t n, int64_t c0,
                                    int64_t hw, int64_t levels, void *stream);
 
