@@ -9,7 +9,7 @@ from torch.autograd import Function
 
 from ..difflogic.functional import GradFactor, bin_op_s
 from ..difflogic.packbitstensor import PackBitsTensor
-from ..hip import convlogic_hip
+from ..hip import _lib, convlogic_hip
 from .treelogic_layer import gate_probabilities, kernel_probabilities
 
 
@@ -261,7 +261,6 @@ class ConvLogicLayer(nn.Module):
         A kept plan is complete: a call on any other stream or thread may use it.  One that was taken in a recording is kept
         for the layer's life, as the replays read it; one that is made inside a recording is the recording's own, which makes
         it again in every replay."""
-        from ..hip import _lib
         key = (tuple(x.shape), x.dtype, x.device, _lib.knob_generation())
         buffer = self._buffers["selection"]                          # (sel: the same, or a contiguous copy for this call)
         plans = self.__dict__.setdefault("_plans", {})
@@ -392,6 +391,8 @@ class ConvLogicLayer(nn.Module):
                 and sel.device == x.device and convlogic_hip.bin_supported(x, self.out_channels, *geo)):
             flag = self.binary_flag_checked()
             if self.training and weights.is_contiguous():
+                if not _lib.traced():
+                    return _lib.nodes().binary_block(x, weights, sel, geo, flag.device_ptr)
                 return _FullConvLogicBinaryFunction.apply(x, weights, sel, *geo, True, flag)
             w_prob = kernel_probabilities(self.weights, self.training, x.dtype)
             return _FullConvLogicBinaryFunction.apply(x, w_prob, sel, *geo, False, flag)
@@ -399,6 +400,8 @@ class ConvLogicLayer(nn.Module):
                 and weights.dtype == x.dtype and x.dtype in (torch.float32, torch.float64) and weights.is_contiguous()
                 and weights.device == x.device and sel.device == x.device):
             plan = self._backward_plan(x, sel)
+            if x.dtype == torch.float32 and not _lib.traced():
+                return _lib.nodes().block(x, weights, sel, geo, self.__dict__.get("feature_major_output", False), *plan, self._take_prefold(weights))
             return _FullConvLogicLogitsFunction.apply(x, weights, sel, *geo, self.__dict__.get("feature_major_output", False), plan,
                                                       self._take_prefold(weights) if plan is not None else None)
         w_prob = kernel_probabilities(self.weights, self.training, x.dtype)

@@ -1,0 +1,395 @@
+// Autograd nodes of the float32 training path in C++: the same calls of the C ABI, tensors and checks as the Python functions of
+// the modules (difflogic/difflogic.py, difflogic/fc_tree.py, convlogic/convlogic_layer.py), which serve every other case.
+// What they are for: the backward pass runs on autograd's device thread, where a Python function first has to take the
+// interpreter from the thread that waits for it, and an eager step of a small network is bound by that and by the interpreter's time
+// per launch.  Forward and backward of one block 82 us on a quiet host and 146 with the hand-off by the Python
+// functions, of a LogicLayer 64 and 124.
+#include <ATen/ATen.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_cpp_function.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include "convlogic_amd.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+void check(int rc)
+{
+    TORCH_CHECK(rc == CLG_OK, clg_last_error());
+}
+void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
+void *ptr(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
+const int64_t *idx(const Tensor &t) { return static_cast<const int64_t *>(t.data_ptr()); }
+Tensor floats(const Tensor &like, at::IntArrayRef shape) { return at::empty(shape, like.options()); }
+Tensor bytes(const Tensor &like, int64_t n)
+{
+    TORCH_CHECK(n >= 0, clg_last_error());
+    return at::empty({n < 8 ? 8 : n}, like.options().dtype(at::kByte));
+}
+// what the kernels read as raw float32 memory of `like`'s device
+void need(const Tensor &t, const Tensor &like, const char *name, at::IntArrayRef shape)
+{
+    TORCH_CHECK(t.device() == like.device(), "all tensors must be on one device, got ", like.device(), " and ", t.device());
+    TORCH_CHECK(t.scalar_type() == at::kFloat, name, " must have dtype torch.float32, got ", t.scalar_type());
+    TORCH_CHECK(t.is_contiguous(), name, " must be contiguous");
+    TORCH_CHECK(t.sizes() == shape, name, " must have shape ", shape, ", got ", t.sizes());
+}
+Tensor transposed(const Tensor &x)
+{
+    Tensor out = at::empty({x.size(1), x.size(0)}, x.options());
+    if (out.numel()) check(clg_transpose_2d((int)x.element_size(), x.data_ptr(), out.data_ptr(), x.size(0), x.size(1), stream_of(x)));
+    return out;
+}
+Tensor contiguous_2d(const Tensor &t)
+{
+    if (t.is_contiguous()) return t;
+    if (t.is_cuda() && t.dim() == 2 && t.transpose(0, 1).is_contiguous()) return transposed(t.transpose(0, 1));
+    return t.contiguous();
+}
+
+// ---- layouts -----------------------------------------------------------------------------------------------------------
+// [batch, features] -> contiguous [features, batch], and the same for the gradient
+struct FeatureMajor : torch::autograd::Function<FeatureMajor> {
+    static Tensor forward(AutogradContext *, const Tensor &x) { return transposed(x); }
+    static variable_list backward(AutogradContext *, variable_list grads)
+    {
+        const Tensor &g = grads[0];
+        return {g.is_cuda() && g.is_contiguous() ? transposed(g) : g.transpose(0, 1)};
+    }
+};
+Tensor feature_major(const Tensor &x) { return FeatureMajor::apply(x); }
+
+// ---- LogicLayer ------------------------------------------------------------------------------------------------------------
+struct FcLayer : torch::autograd::Function<FcLayer> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x_in, const Tensor &a, const Tensor &b, const Tensor &logits, const Tensor &start,
+                          const Tensor &flat, bool sole, bool sample_major)
+    {
+        const int64_t out_dim = logits.size(0), in_dim = x_in.size(sample_major ? 1 : 0), batch = x_in.size(sample_major ? 0 : 1);
+        Tensor y = floats(x_in, {out_dim, batch}), probs = floats(x_in, {out_dim, 16}), folded = floats(x_in, {out_dim, 4}), x = x_in;
+        if (sample_major) {
+            x = floats(x_in, {in_dim, batch});
+            check(clg_fc_forward_logits_ex(CLG_F32, x_in.data_ptr(), idx(a), idx(b), logits.data_ptr(), probs.data_ptr(), folded.data_ptr(),
+                                           y.data_ptr(), in_dim, out_dim, batch, CLG_FC_X_SAMPLE_MAJOR, x.data_ptr(), stream_of(x)));
+        } else {
+            check(clg_fc_forward_logits(CLG_F32, x.data_ptr(), idx(a), idx(b), logits.data_ptr(), probs.data_ptr(), folded.data_ptr(), y.data_ptr(),
+                                        in_dim, out_dim, batch, stream_of(x)));
+        }
+        ctx->save_for_backward({x, a, b, probs, folded, start, flat});
+        ctx->saved_data["sole"] = sole;
+        ctx->saved_data["sample_major"] = sample_major;
+        return y;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &x = saved[0], &a = saved[1], &b = saved[2], &probs = saved[3], &folded = saved[4], &start = saved[5], &flat = saved[6];
+        const bool sole = ctx->saved_data["sole"].toBool(), sample_major = ctx->saved_data["sample_major"].toBool();
+        const bool need_x = ctx->needs_input_grad(0), need_l = ctx->needs_input_grad(3);
+        const int64_t in_dim = x.size(0), batch = x.size(1), out_dim = folded.size(0);
+        const bool fused = !sole && need_x && need_l && clg_fc_backward_fused_fits(CLG_F32, batch);
+        Tensor gy = grads[0], gx, gl;
+        // a gradient that arrives as a transposed view: its feature-major copy is made by the call that computes both gradients
+        const bool gy_sample_major = fused && !gy.is_contiguous() && gy.is_cuda() && gy.dim() == 2 && gy.transpose(0, 1).is_contiguous();
+        if (gy_sample_major) {
+            gy = gy.transpose(0, 1);
+            need(gy, x, "grad_y", {batch, out_dim});
+        } else {
+            gy = contiguous_2d(gy);
+            need(gy, x, "grad_y", {out_dim, batch});
+        }
+        if (need_l) gl = floats(x, {out_dim, 16});
+        if (fused) {
+            gx = sample_major ? floats(x, {batch, in_dim}) : floats(x, {in_dim, batch});
+            Tensor copy;
+            if (gy_sample_major) copy = floats(x, {out_dim, batch});
+            check(clg_fc_backward_fused_ex(CLG_F32, x.data_ptr(), idx(a), idx(b), folded.data_ptr(), probs.data_ptr(), gy.data_ptr(), idx(start),
+                                           idx(flat), gx.data_ptr(), gl.data_ptr(), in_dim, out_dim, batch,
+                                           (sample_major ? CLG_FC_GX_SAMPLE_MAJOR : 0) | (gy_sample_major ? CLG_FC_GY_SAMPLE_MAJOR : 0), ptr(copy),
+                                           stream_of(x)));
+            return {gx, Tensor(), Tensor(), gl, Tensor(), Tensor(), Tensor(), Tensor()};
+        }
+        if (need_x) gx = at::empty_like(x);
+        if (sole && need_x && need_l) {
+            check(clg_fc_backward_sole(CLG_F32, x.data_ptr(), idx(a), idx(b), folded.data_ptr(), probs.data_ptr(), gy.data_ptr(), gx.data_ptr(),
+                                       gl.data_ptr(), in_dim, out_dim, batch, stream_of(x)));
+        } else {
+            if (need_x)
+                check(clg_fc_backward_x_folded(CLG_F32, x.data_ptr(), idx(a), idx(b), folded.data_ptr(), gy.data_ptr(), idx(start), idx(flat),
+                                               gx.data_ptr(), in_dim, out_dim, batch, stream_of(x)));
+            if (need_l)
+                check(clg_fc_backward_logits(CLG_F32, x.data_ptr(), idx(a), idx(b), probs.data_ptr(), gy.data_ptr(), gl.data_ptr(), in_dim, out_dim,
+                                             batch, stream_of(x)));
+        }
+        if (sample_major && need_x) gx = transposed(gx);
+        return {gx, Tensor(), Tensor(), gl, Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+// x [batch, in] where sample_major, else [in, batch]; -> [batch, out], a transposed view of [out, batch]
+Tensor fc_layer(const Tensor &x, const Tensor &a, const Tensor &b, const Tensor &logits, const Tensor &start, const Tensor &flat, bool sole,
+                bool sample_major)
+{
+    need(logits, x, "weights", {a.numel(), 16});
+    return FcLayer::apply(x, a, b, logits, start, flat, sole, sample_major).transpose(0, 1);
+}
+
+// ---- complete blocks -----------------------------------------------------------------------------------------------------
+struct Conv {                                                         // stride, padding and kernel of a block
+    int64_t sh, sw, ph, pw, kh, kw;
+    clg_conv_geom geom(const Tensor &x, int64_t c_out) const
+    {
+        return {(int32_t)x.size(0), (int32_t)x.size(1), (int32_t)x.size(2), (int32_t)x.size(3), (int32_t)c_out, (int32_t)sh, (int32_t)sw,
+                (int32_t)ph, (int32_t)pw, (int32_t)kh, (int32_t)kw};
+    }
+    c10::IValue saved(std::vector<int64_t> more) const
+    {
+        std::vector<int64_t> l{sh, sw, ph, pw, kh, kw};
+        l.insert(l.end(), more.begin(), more.end());
+        return c10::IValue(std::move(l));
+    }
+    static Conv from(const std::vector<int64_t> &l) { return {l[0], l[1], l[2], l[3], l[4], l[5]}; }
+};
+std::vector<int64_t> pooled(const clg_conv_geom &g)
+{
+    const int64_t ho = (g.h + 2 * g.pad_h - g.kernel_h) / g.stride_h + 1, wo = (g.w + 2 * g.pad_w - g.kernel_w) / g.stride_w + 1;
+    return {g.n, g.c_out, std::max<int64_t>(ho, 0) / 2, std::max<int64_t>(wo, 0) / 2};
+}
+
+// plan, signature: the layer's backward plan.  pair: probabilities and folded coefficients [c, 7, 16], [c, 7, 4] in one buffer
+// that a network made for all its layers (or null).
+struct Block : torch::autograd::Function<Block> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x_in, const Tensor &logits, const Tensor &sel_in, const Conv *conv, bool want_fm,
+                          const Tensor *plan, int64_t signature, const std::pair<Tensor, Tensor> *pair, bool need_x)
+    {
+        const Tensor x = x_in.contiguous(), sel = sel_in.contiguous();
+        const int64_t c = logits.size(0);
+        const clg_conv_geom g = conv->geom(x, c);
+        const auto s = pooled(g);
+        const bool fm = want_fm && clg_convblock_fm_supported(CLG_F32, &g);
+        Tensor y = fm ? floats(x, {s[1], s[2], s[3], s[0]}) : floats(x, s), argmax = at::empty(s, x.options().dtype(at::kByte));
+        Tensor probs, folded;                                         // without a pair: probabilities and coefficients in one tensor, no folded
+        if (pair != nullptr) {
+            probs = pair->first, folded = pair->second;
+            need(probs, x, "prefolded probabilities", {c, 7, 16});
+            need(folded, x, "prefolded coefficients", {c, 7, 4});
+            TORCH_CHECK(folded.data_ptr<float>() == probs.data_ptr<float>() + probs.numel(),
+                        "prefolded: the folded coefficients must follow the probabilities in one buffer (fold_many)");
+        } else {
+            probs = floats(x, {c * (112 + 28)});
+        }
+        const Tensor scratch = bytes(x, clg_convblock_forward_scratch_bytes(CLG_F32, &g));
+        const int flags = CLG_FWD_W_LOGITS | (fm ? CLG_FWD_Y_FEATURE_MAJOR : 0) | CLG_FWD_FOLDED_OUT | (pair != nullptr ? CLG_FWD_FOLDED_IN : 0);
+        Tensor padded;
+        if (need_x && (signature & 1) == CLG_LISTS_SHORT && !fm) {    // the copy of x that the forward kernels stage and the backward reads
+            const int64_t elems = clg_convblock_padded_elems(CLG_F32, &g, 1);
+            if (elems > 0) padded = floats(x, {elems});
+        }
+        const int32_t *selection = static_cast<const int32_t *>(sel.data_ptr());
+        uint8_t *codes = static_cast<uint8_t *>(argmax.data_ptr());
+        if (padded.defined())
+            check(clg_convblock_forward_padded(CLG_F32, &g, x.data_ptr(), logits.data_ptr(), selection, y.data_ptr(), codes, probs.data_ptr(), flags,
+                                               scratch.data_ptr(), padded.data_ptr(), stream_of(x)));
+        else
+            check(clg_convblock_forward_ex(CLG_F32, &g, x.data_ptr(), logits.data_ptr(), selection, y.data_ptr(), codes, probs.data_ptr(), flags,
+                                           scratch.data_ptr(), stream_of(x)));
+        ctx->save_for_backward({x, probs, sel, argmax, folded, padded});
+        ctx->saved_data["conv"] = conv->saved({fm, signature});
+        ctx->saved_data["plan"] = *plan;
+        return fm ? y.permute({3, 0, 1, 2}) : y;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &x = saved[0], &probs = saved[1], &sel = saved[2], &argmax = saved[3];
+        const auto ints = ctx->saved_data["conv"].toIntVector();
+        const Conv conv = Conv::from(ints);
+        const bool need_x = ctx->needs_input_grad(0), need_l = ctx->needs_input_grad(1);
+        const int64_t c = sel.size(0), signature = ints[7];
+        const float *folded = saved[4].defined() ? saved[4].data_ptr<float>() : probs.data_ptr<float>() + c * 112;
+        const int32_t *selection = static_cast<const int32_t *>(sel.data_ptr());
+        const uint8_t *codes = static_cast<const uint8_t *>(argmax.data_ptr());
+        const clg_conv_geom g = conv.geom(x, c);
+        Tensor gy = grads[0], gx, gl;
+        if (need_x) gx = at::empty_like(x);
+        if (need_l) {
+            const bool fm = ints[6] && !gy.is_contiguous() && gy.permute({1, 2, 3, 0}).is_contiguous();
+            const auto s = pooled(g);
+            if (fm) {
+                gy = gy.permute({1, 2, 3, 0});
+                need(gy, x, "grad_y", {s[1], s[2], s[3], s[0]});
+            } else {
+                gy = gy.contiguous();
+                need(gy, x, "grad_y", s);
+            }
+            gl = floats(x, {c, 7, 16});
+            const Tensor plan = ctx->saved_data["plan"].toTensor(),
+                         scratch = bytes(x, clg_convblock_backward_planned_scratch_bytes(CLG_F32, &g, signature));
+            const Tensor padded = fm || !need_x ? Tensor() : saved[5];
+            const int flags = CLG_BWD_WRT_LOGITS | (fm ? CLG_BWD_GY_FEATURE_MAJOR : 0);
+            if (padded.defined())
+                check(clg_convblock_backward_planned_padded(CLG_F32, &g, gy.data_ptr(), x.data_ptr(), probs.data_ptr(), folded,
+                                                            padded.data_ptr(), selection, codes, plan.data_ptr(), signature, gx.data_ptr(),
+                                                            gl.data_ptr(), flags, scratch.data_ptr(), stream_of(x)));
+            else
+                check(clg_convblock_backward_planned(CLG_F32, &g, gy.data_ptr(), x.data_ptr(), probs.data_ptr(), folded, selection, codes,
+                                                     plan.data_ptr(), signature, ptr(gx), gl.data_ptr(), flags, scratch.data_ptr(), stream_of(x)));
+        } else if (need_x) {
+            gy = gy.contiguous();
+            need(gy, x, "grad_y", pooled(g));
+            const Tensor scratch = bytes(x, clg_convblock_backward_x_scratch_bytes(CLG_F32, &g));
+            check(clg_convblock_backward_x(CLG_F32, &g, gy.data_ptr(), x.data_ptr(), probs.data_ptr(), selection, codes, gx.data_ptr(),
+                                           scratch.data_ptr(), stream_of(x)));
+        }
+        return {gx, gl, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+Tensor block(const Tensor &x, const Tensor &logits, const Tensor &sel, std::array<int64_t, 6> conv, bool want_fm, const Tensor &plan,
+             int64_t signature, const std::optional<std::pair<Tensor, Tensor>> &prefolded)
+{
+    need(logits, x, "weights", {sel.size(0), 7, 16});
+    const Conv cv{conv[0], conv[1], conv[2], conv[3], conv[4], conv[5]};
+    return Block::apply(x, logits, sel, &cv, want_fm, &plan, signature, prefolded ? &*prefolded : nullptr, at::GradMode::is_enabled() && x.requires_grad());
+}
+
+// The block on 0/1 inputs, from the logits.  flag: device address of the layer's BinaryFlag.
+struct BinaryBlock : torch::autograd::Function<BinaryBlock> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x_in, const Tensor &logits, const Tensor &sel_in, const Conv *conv, int64_t flag)
+    {
+        const Tensor x = x_in.contiguous(), sel = sel_in.contiguous();
+        const clg_conv_geom g = conv->geom(x, logits.size(0));
+        const Tensor keep = bytes(x, clg_convblock_bin_ctx_bytes(CLG_F32, &g));
+        const auto s = pooled(g);
+        Tensor y = floats(x, s), taps = at::empty(s, x.options().dtype(at::kShort));
+        check(clg_convblock_bin_forward(CLG_F32, &g, x.data_ptr(), logits.data_ptr(), static_cast<const int32_t *>(sel.data_ptr()), y.data_ptr(),
+                                        static_cast<uint16_t *>(taps.data_ptr()), keep.data_ptr(), CLG_FWD_W_LOGITS,
+                                        reinterpret_cast<int32_t *>(flag), stream_of(x)));
+        ctx->save_for_backward({taps, keep});                        // x itself is not needed again
+        ctx->saved_data["conv"] = conv->saved(x.sizes().vec());
+        return y;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &taps = saved[0], &keep = saved[1], gy = grads[0].contiguous();
+        TORCH_CHECK(gy.is_cuda(), "grad_y must be a CUDA tensor");
+        TORCH_CHECK(gy.device() == taps.device(), "all tensors must be on one device, got ", taps.device(), " and ", gy.device());
+        need(gy, gy, "grad_y", taps.sizes());
+        const auto ints = ctx->saved_data["conv"].toIntVector();
+        const Conv cv = Conv::from(ints);
+        const std::vector<int64_t> xs(ints.begin() + 6, ints.end());
+        const int64_t c = gy.size(1);
+        const clg_conv_geom g = {(int32_t)xs[0], (int32_t)xs[1], (int32_t)xs[2], (int32_t)xs[3], (int32_t)c, (int32_t)cv.sh, (int32_t)cv.sw,
+                                 (int32_t)cv.ph, (int32_t)cv.pw, (int32_t)cv.kh, (int32_t)cv.kw};
+        const bool need_x = ctx->needs_input_grad(0), need_l = ctx->needs_input_grad(1);
+        Tensor gx, gl, scratch;
+        if (need_x) gx = floats(gy, xs);
+        if (need_l) {
+            gl = floats(gy, {c, 7, 16});
+            scratch = bytes(gy, clg_convblock_bin_backward_scratch_bytes(CLG_F32, &g));
+        }
+        if (need_x || need_l)
+            check(clg_convblock_bin_backward(CLG_F32, &g, gy.data_ptr(), static_cast<const uint16_t *>(taps.data_ptr()), keep.data_ptr(), ptr(gx),
+                                             ptr(gl), CLG_BWD_WRT_LOGITS, ptr(scratch), stream_of(gy)));
+        return {gx, gl, Tensor(), Tensor(), Tensor()};
+    }
+};
+Tensor binary_block(const Tensor &x, const Tensor &logits, const Tensor &sel, std::array<int64_t, 6> conv, int64_t flag)
+{
+    need(logits, x, "weights", {sel.size(0), 7, 16});
+    const Conv cv{conv[0], conv[1], conv[2], conv[3], conv[4], conv[5]};
+    return BinaryBlock::apply(x, logits, sel, &cv, flag);
+}
+
+// ---- three LogicLayers and a GroupSum as trees --------------------------------------------------------------------------------
+// wiring: indices_0 and indices_1 of the three layers, saved for autograd's check that they were not written in between;
+// rows, pos, ids, slot: the tables of the wiring.
+struct TreeArgs {
+    Tensor start, rows, pos, ids, slot;
+    std::vector<Tensor> wiring;
+    int64_t roots, k;
+    double tau;
+};
+struct Trees : torch::autograd::Function<Trees> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &l0, const Tensor &l1, const Tensor &l2, const TreeArgs *t, bool need_l)
+    {
+        const int64_t in_dim = x.size(0), batch = x.size(1);
+        const auto i32 = [](const Tensor &v) { return static_cast<const int32_t *>(v.data_ptr()); };
+        Tensor coef = floats(x, {t->roots, 28}), probs;
+        if (need_l) probs = floats(x, {7 * t->roots, 16});            // (the logits may be updated between forward and backward)
+        check(clg_fc_tree_fold(l0.data_ptr<float>(), l1.data_ptr<float>(), l2.data_ptr<float>(), i32(t->ids), coef.data_ptr<float>(),
+                               static_cast<float *>(ptr(probs)), t->roots, 0, stream_of(x)));
+        const int64_t elems = clg_fc_tree_partial_elems(t->roots, t->k, batch, batch);
+        Tensor out = floats(x, {batch, t->k}), partial = floats(x, {elems < 0 ? 0 : elems});
+        check(clg_fc_tree_forward(x.data_ptr<float>(), i32(t->rows), coef.data_ptr<float>(), partial.data_ptr<float>(), out.data_ptr<float>(), in_dim,
+                                  t->roots, t->k, batch, batch, t->tau, stream_of(x)));
+        variable_list saved = {x, t->start, coef, probs};
+        saved.insert(saved.end(), t->wiring.begin(), t->wiring.end());
+        ctx->save_for_backward(std::move(saved));
+        ctx->saved_data["tables"] = std::vector<Tensor>{t->rows, t->pos, t->slot};
+        ctx->saved_data["k"] = t->k;
+        ctx->saved_data["tau"] = t->tau;
+        return out;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &x = saved[0], &start = saved[1], &coef = saved[2], &probs = saved[3];
+        const auto tables = ctx->saved_data["tables"].toTensorVector();
+        const int64_t k = ctx->saved_data["k"].toInt(), in_dim = x.size(0), batch = x.size(1), roots = coef.size(0);
+        const auto i32 = [](const Tensor &v) { return static_cast<const int32_t *>(v.data_ptr()); };
+        const auto f32 = [](const Tensor &v) { return static_cast<float *>(ptr(v)); };
+        const Tensor go = grads[0].contiguous();
+        need(go, x, "grad_out", {batch, k});
+        Tensor gx, g[3];
+        if (ctx->needs_input_grad(0)) gx = at::empty_like(x);
+        const int64_t neurons[3] = {4 * roots, 2 * roots, roots};
+        for (int i = 0; i < 3; ++i)
+            if (ctx->needs_input_grad(1 + i)) g[i] = floats(x, {neurons[i], 16});
+        const int64_t rows = gx.defined() ? 8 * roots * batch : 0;
+        const Tensor scratch = floats(x, {rows + 28 * roots});       // operand gradients, then sums
+        check(clg_fc_tree_backward(f32(x), i32(tables[0]), i32(tables[1]), i32(tables[2]), f32(coef), f32(go), f32(probs), f32(g[0]), f32(g[1]),
+                                   f32(g[2]), f32(scratch), f32(scratch) + rows, idx(start), f32(gx), in_dim, roots, k, batch, batch,
+                                   ctx->saved_data["tau"].toDouble(), stream_of(x)));
+        return {gx, g[0], g[1], g[2], Tensor(), Tensor()};
+    }
+};
+Tensor trees(const Tensor &x, const Tensor &l0, const Tensor &l1, const Tensor &l2, const Tensor &start, std::vector<Tensor> wiring, const Tensor &rows,
+             const Tensor &pos, const Tensor &ids, const Tensor &slot, int64_t roots, int64_t k, double tau)
+{
+    need(l0, x, "weights", {4 * roots, 16});
+    need(l1, x, "weights", {2 * roots, 16});
+    need(l2, x, "weights", {roots, 16});
+    const TreeArgs t{start, rows, pos, ids, slot, std::move(wiring), roots, k, tau};
+    return Trees::apply(x, l0, l1, l2, &t, at::GradMode::is_enabled() && (l0.requires_grad() || l1.requires_grad() || l2.requires_grad()));
+}
+
+// grad_fn of a node's output in Python: a type of the name that the Python function's node has
+template <typename F>
+void name_node(const char *name)
+{
+    static PyTypeObject type;
+    torch::autograd::_initFunctionPyTypeObject(type, name, nullptr, nullptr);
+    torch::autograd::registerCppFunction(typeid(torch::autograd::CppNode<F>), &type);
+}
+
+}  // namespace
+
+// (the interpreter is given up while a node works: the launches wait for nothing, but another thread may)
+PYBIND11_MODULE(_nodes, m)
+{
+    const auto no_gil = py::call_guard<py::gil_scoped_release>();
+    name_node<FeatureMajor>("_FeatureMajorBackward");
+    name_node<FcLayer>("_LogicLayerLogitsFunctionBackward");
+    name_node<Block>("_FullConvLogicLogitsFunctionBackward");
+    name_node<BinaryBlock>("_FullConvLogicBinaryFunctionBackward");
+    name_node<Trees>("_TreeFunctionBackward");
+    m.def("feature_major", &feature_major, no_gil);
+    m.def("fc_layer", &fc_layer, no_gil);
+    m.def("block", &block, no_gil);
+    m.def("binary_block", &binary_block, no_gil);
+    m.def("trees", &trees, no_gil);
+}

@@ -12,7 +12,7 @@ import weakref
 import numpy as np
 import torch
 
-from ..hip import difflogic_hip
+from ..hip import _lib, difflogic_hip
 from . import fc_tree
 from .functional import GradFactor, bin_op_s, get_unique_connections
 from .packbitstensor import PackBitsTensor
@@ -111,6 +111,10 @@ class LogicLayer(torch.nn.Module):
             # node per layer instead of two
             prefolded = self._take_prefold(weights)
             inside = prefolded is None and _transposes_with_kernel(x)
+            if prefolded is None and x.dtype == torch.float32 and not _lib.traced():
+                return _lib.nodes().fc_layer(x if inside else _feature_major(x), buffers["indices_0"], buffers["indices_1"], weights,
+                                             buffers["given_x_indices_of_y_start"], buffers["given_x_indices_of_y"], self._sole_consumers(key),
+                                             inside)
             return _LogicLayerLogitsFunction.apply(x if inside else _feature_major(x), buffers["indices_0"], buffers["indices_1"],
                                                    weights, buffers["given_x_indices_of_y_start"],
                                                    buffers["given_x_indices_of_y"], self._sole_consumers(key), inside,
@@ -321,7 +325,7 @@ def _feature_major(x):
     if xt.is_contiguous():
         return xt
     if _transposes_with_kernel(x):
-        return _FeatureMajor.apply(x)
+        return _FeatureMajor.apply(x) if _lib.traced() else _lib.nodes().feature_major(x)
     return xt.contiguous()
 
 

@@ -183,6 +183,9 @@ def tree_eval(layers, group_sum, x, plan):
 def tree_train(layers, group_sum, x, plan):
     """group_sum(third(second(first(x)))) in training; x feature-major [features, B]."""
     first, second, third = layers
+    if not _lib.traced():
+        return _lib.nodes().trees(x, first.weights, second.weights, third.weights, first._buffers["given_x_indices_of_y_start"], wiring_of(*layers),
+                                  plan.rows, plan.pos, plan.ids, plan.slot, plan.roots, group_sum.k, float(group_sum.tau))
     return _TreeFunction.apply(x, first.weights, second.weights, third.weights, first._buffers["given_x_indices_of_y_start"],
                                wiring_of(*layers), plan, group_sum.k, group_sum.tau)
 

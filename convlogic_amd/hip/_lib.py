@@ -147,6 +147,31 @@ def load():
     return _lib
 
 
+_nodes = None
+
+
+def nodes():
+    """The autograd nodes of the float32 training path (csrc/nodes.cpp)."""
+    global _nodes
+    if _nodes is None:
+        load()
+        try:
+            from .. import _nodes as module
+        except ImportError as e:
+            raise RuntimeError(f"convlogic_amd: _nodes.so is missing or does not load ({e}). Build it with `python -m convlogic_amd.build`; there "
+                               "is no fallback for the 'cuda' implementation.") from e
+        _nodes = module
+    return _nodes
+
+
+def traced():
+    """True while torch.jit records a trace: the Python functions leave a node in it, calls of the C++ ones would not."""
+    return _tracing_state() is not None
+
+
+_tracing_state = torch._C._get_tracing_state
+
+
 def available():
     return os.path.exists(LIB_PATH)
 

@@ -543,6 +543,7 @@ class BinaryFlag:
         dev = ctypes.c_void_p(0)
         check(_lib.load().clg_host_flag_device_pointer(self.host.data_ptr(), ctypes.byref(dev)))
         self.device_ptr = dev.value
+        self._word = ctypes.c_int32.from_address(self.host.data_ptr())   # (read on every call: a tensor element costs 3 us)
 
     def __deepcopy__(self, memo):                                    # a copied layer gets a flag of its own
         return BinaryFlag()
@@ -551,10 +552,10 @@ class BinaryFlag:
         return (BinaryFlag, ())
 
     def raised(self):
-        return bool(self.host[0].item())
+        return self._word.value != 0
 
     def clear(self):
-        self.host.zero_()
+        self._word.value = 0
 
 
 def bin_forward(x, w, selection, stride_h, stride_w, pad_h, pad_w, kernel_h, kernel_w, flag, logits=False, validate=True):
