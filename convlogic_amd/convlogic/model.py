@@ -162,10 +162,10 @@ def _counts_at_once(net, tail, plan, x):
 
 def _sums_at_once(net, tail, plan, x):
     """Class sums of 0/1 images (the first block's binary_input, verified by the kernels) on packed bits, or None.  Against the float
-    kernels: 245 -> 90 us of device time for 1000 images of the k = 32 CIFAR network, 1365 -> 160 at k = 128; small batches of the
-    smallest networks leave the words' kernels short of work (k = 8, 128 images: 58 and 63 us)."""
+    kernels: 245 -> 79 us for 1000 images of the k = 32 CIFAR network, 1365 -> 160 at k = 128; one image of the smallest networks 36 to 55
+    -> 35 to 60 us in a recorded graph, 130 to 165 -> 60 to 68 called eagerly."""
     layers, gs = tail
-    if x.dim() != 4 or not (x.shape[0] >= 192 or plan.roots >= 8192) or x.shape[0] > 65535 * 64 or gs.k >= 512:
+    if x.dim() != 4 or x.shape[0] > 65535 * 64 or gs.k >= 512:
         return None
     blocks = packed_net.blocks_of(net, _called_for_itself)
     if blocks is None or not blocks[0].__dict__.get("binary_input") or not (

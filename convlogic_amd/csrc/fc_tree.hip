@@ -37,14 +37,17 @@ template <int V>
 struct Samples {
     float v[V];
 };
+// (vectors at any 4-byte boundary, which is all that a wide access to global memory needs: rows of an odd number of samples)
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
 template <int V>
 struct SamplesRaw;
 template <>
 struct SamplesRaw<1> { using type = float; };
 template <>
-struct SamplesRaw<2> { using type = float2; };
+struct SamplesRaw<2> { using type = f32x2u; };
 template <>
-struct SamplesRaw<4> { using type = float4; };
+struct SamplesRaw<4> { using type = f32x4u; };
 template <int V>
 __device__ __forceinline__ Samples<V> load_samples(const float *p)
 {
@@ -54,6 +57,13 @@ template <int V>
 __device__ __forceinline__ void store_samples(float *p, const Samples<V> &v)
 {
     *reinterpret_cast<typename SamplesRaw<V>::type *>(p) = __builtin_bit_cast(typename SamplesRaw<V>::type, v);
+}
+// Where the lane whose samples begin at s reads and writes: the last lane of a row whose length V does not divide steps back to the
+// last V samples, which it shares with its neighbour (the same values, computed twice); lanes behind the row: 0.
+template <int V>
+__device__ __forceinline__ int64_t samples_at(int64_t s, int64_t pitch)
+{
+    return s >= pitch ? 0 : (s + V <= pitch ? s : pitch - V);
 }
 
 // a of both halves in the low half, b of both halves in the high half (v_permlane32_swap + add), and the same for the even /
@@ -129,42 +139,84 @@ __device__ __forceinline__ const float *tree_logits(const TreeLogits &lg, const 
 {
     return (q < 4 ? lg.l[0] : (q < 6 ? lg.l[1] : lg.l[2])) + tree_neuron(ids, j, q, roots) * 16;
 }
-// index of the first maximum (a NaN counts as the maximum), as clg_gate_argmax
-__device__ __forceinline__ int argmax16(const float *__restrict__ w)
+// Index of the first maximum of 16 logits (a NaN counts as the maximum), as clg_gate_argmax, by four lanes: `mine` are the logits 4 (lane
+// & 3) .. + 3.  Valid in all four.  Values compare as integers: -0 and +0 equal, NaN on top.
+__device__ __forceinline__ int argmax16_quad(f32x4u mine)
 {
-    float best = w[0];
+    const float v[4] = {mine.x, mine.y, mine.z, mine.w};
+    uint32_t best = 0;
     int at = 0;
 #pragma unroll
-    for (int i = 1; i < 16; ++i) {
-        const float v = w[i];
-        if (v > best || (v != v && best == best)) best = v, at = i;
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t u = __builtin_bit_cast(uint32_t, v[i] + 0.0f);
+        const uint32_t key = v[i] != v[i] ? 0xFFFFFFFFu : (u ^ ((u >> 31) ? 0xFFFFFFFFu : 0x80000000u));
+        if (i == 0 || key > best) best = key, at = i;
+    }
+    at += 4 * (threadIdx.x & 3);
+#pragma unroll
+    for (int by = 1; by <= 2; by <<= 1) {
+        const uint32_t key = by == 1 ? dpp_zero<0xB1, 0xF>(best) : dpp_zero<0x4E, 0xF>(best);
+        const int other = (int)(by == 1 ? dpp_zero<0xB1, 0xF>((uint32_t)at) : dpp_zero<0x4E, 0xF>((uint32_t)at));
+        if (key > best || (key == best && other < at)) best = key, at = other;
     }
     return at;
 }
 // probs (or null): the probabilities, neurons of the first layer first.  The backward pass reads these: logits that an
 // optimizer updates between the two passes must not reach it.
+// A lane per gate does the arithmetic, four lanes per gate move its 64 bytes: the 16-byte pieces of a row go through LDS, so that an
+// access of a wavefront is 16 rows in place of 64 pieces of 64 rows (131072 features, 655360 roots: 211 -> 188 us, 94080 roots 38 -> 28; what is left
+// are 0.66 GB of rows, read and written in tree order).
+constexpr int kFoldPitch = 20;                                       // floats of a row in LDS: 16-byte pieces, lanes spread over the banks
 __global__ __launch_bounds__(256) void fc_tree_fold_kernel(TreeLogits lg, const int32_t *__restrict__ ids, float *__restrict__ coef,
                                                          float *__restrict__ probs, int roots, int hard)
 {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= (int64_t)roots * 7) return;
-    const int j = (int)(e / 7), q = (int)(e - (int64_t)j * 7);
-    const float *w = tree_logits(lg, ids, j, q, roots);
-    float p[16];
+    __shared__ __align__(16) float rows[256 / kWave][kWave * kFoldPitch];
+    const int lane = threadIdx.x & (kWave - 1);
+    float *mine = rows[threadIdx.x >> 6];
+    const int64_t gates = (int64_t)roots * 7, e0 = (int64_t)blockIdx.x * 256 + (threadIdx.x & ~(kWave - 1)), e = e0 + lane;
+    if (e0 >= gates) return;                                          // (a whole wavefront; none meets another one)
+    const int64_t ec = e < gates ? e : gates - 1;
+    const int j = (int)(ec / 7), q = (int)(ec - (int64_t)j * 7);
+    const int layer = q < 4 ? 0 : (q < 6 ? 1 : 2);
+    const int neuron = (int)tree_neuron(ids, j, q, roots);
+    const int place = neuron + roots * (layer == 0 ? 0 : (layer == 1 ? 4 : 6));   // of the neuron among all (below 2^31: roots < 2^28)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int from = 16 * i + (lane >> 2), l = __shfl(layer, from, kWave), n = __shfl(neuron, from, kWave);
+        const float *w = l == 0 ? lg.l[0] : (l == 1 ? lg.l[1] : lg.l[2]);
+        const f32x4u v = reinterpret_cast<const f32x4u *>(w + (int64_t)n * 16)[lane & 3];
+        // (logits at any 4-byte boundary)
+        *reinterpret_cast<float4 *>(mine + from * kFoldPitch + 4 * (lane & 3)) = make_float4(v.x, v.y, v.z, v.w);
+    }
+    float w[16], p[16];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float4 v = *reinterpret_cast<const float4 *>(mine + lane * kFoldPitch + 4 * i);
+        w[4 * i] = v.x, w[4 * i + 1] = v.y, w[4 * i + 2] = v.z, w[4 * i + 3] = v.w;
+    }
     if (hard) {
-        const int at = argmax16(w);
+        float best = w[0];
+        int at = 0;
+#pragma unroll
+        for (int i = 1; i < 16; ++i)
+            if (w[i] > best || (w[i] != w[i] && best == best)) best = w[i], at = i;
 #pragma unroll
         for (int i = 0; i < 16; ++i) p[i] = i == at ? 1.f : 0.f;
     } else {
         softmax16(w, p);
     }
-    if (probs) {
-        float4 *dst = reinterpret_cast<float4 *>(probs + (tree_neuron(ids, j, q, roots) + (int64_t)roots * (q < 4 ? 0 : (q < 6 ? 4 : 6))) * 16);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) dst[i] = make_float4(p[4 * i], p[4 * i + 1], p[4 * i + 2], p[4 * i + 3]);
-    }
     const Coef<float> c = fold16(p);
-    reinterpret_cast<float4 *>(coef)[e] = make_float4(c.ab, c.a, c.b, c.one);
+    if (e < gates) reinterpret_cast<float4 *>(coef)[e] = make_float4(c.ab, c.a, c.b, c.one);
+    if (probs == nullptr) return;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<float4 *>(mine + lane * kFoldPitch + 4 * i) = make_float4(p[4 * i], p[4 * i + 1], p[4 * i + 2], p[4 * i + 3]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int from = 16 * i + (lane >> 2), at = __shfl(place, from, kWave);
+        const float4 v = *reinterpret_cast<const float4 *>(mine + from * kFoldPitch + 4 * (lane & 3));
+        if (e0 + from < gates) reinterpret_cast<float4 *>(probs + (int64_t)at * 16)[lane & 3] = v;
+    }
 }
 
 // ---- forward ----------------------------------------------------------------------------------------------------------
@@ -196,7 +248,7 @@ __global__ __launch_bounds__(kTreeBlock) void fc_tree_forward_kernel(const float
     __shared__ Samples<V> meet[kTreeWaves][kWave];
     const int lane = threadIdx.x & (kWave - 1), wave = uniform((int)(threadIdx.x >> 6));
     const int slice = blockIdx.x, g = blockIdx.y;
-    const int64_t s = ((int64_t)blockIdx.z * kWave + lane) * V, s_at = s < pitch ? s : 0;
+    const int64_t s = ((int64_t)blockIdx.z * kWave + lane) * V, s_at = samples_at<V>(s, pitch);
     const int r0 = (int)((int64_t)class_rows * slice / slices), r1 = (int)((int64_t)class_rows * (slice + 1) / slices);
     Samples<V> acc = {};
     auto value = [&](int r, Samples<V> &y) {
@@ -234,7 +286,7 @@ __global__ __launch_bounds__(kTreeBlock) void fc_tree_forward_kernel(const float
         Samples<V> sum;
 #pragma unroll
         for (int i = 0; i < V; ++i) sum.v[i] = (meet[0][lane].v[i] + meet[1][lane].v[i]) + (meet[2][lane].v[i] + meet[3][lane].v[i]);
-        store_samples<V>(partial + ((int64_t)slice * k + g) * pitch + s, sum);
+        store_samples<V>(partial + ((int64_t)slice * k + g) * pitch + s_at, sum);
     }
 }
 
@@ -405,8 +457,8 @@ __global__ __launch_bounds__(kTreeBlock) void fc_tree_gather_kernel(const float 
 {
     const int lane = threadIdx.x & (kWave - 1), wave = uniform((int)(threadIdx.x >> 6));
     const int i = blockIdx.x * kTreeWaves + wave;
-    const int64_t s = ((int64_t)blockIdx.y * kWave + lane) * V;
-    if (i >= in_dim || s >= pitch) return;
+    const int64_t s_lane = ((int64_t)blockIdx.y * kWave + lane) * V, s = samples_at<V>(s_lane, pitch);
+    if (i >= in_dim || s_lane >= pitch) return;
     const int64_t beg = clamp_index(start[i], total_rows + 1), end = clamp_index(start[i + 1], total_rows + 1);
     Samples<V> part[4] = {};
     const float *p = rowgrad + beg * pitch + s;
@@ -435,11 +487,15 @@ __global__ __launch_bounds__(kTreeBlock) void fc_tree_gather_kernel(const float 
     store_samples<V>(gx + (int64_t)i * pitch + s, sum);
 }
 
-// the widest lanes that a row fills and that its pitch and the buffers' alignment allow
-int tree_vec(int64_t pitch, const void *x, const void *grad_x)
+// The widest lanes that a row fills: a pass of 64 lanes x V samples over rows of up to 64, 128 and 256.  The kernels that only read rows and
+// write whole sums take them for any row length (211 samples, 10 roots of 3200: forward 26.9 -> 23.4 us, input gradient 48.5 ->
+// 32.8, in place of one sample per lane); the backward kernel, bound by the operand gradients that it writes, where V divides the row
+// and the buffers are aligned (83 samples: 107 us with one sample per lane, 114 with two; 211: 77 and 75 with four).
+int tree_vec(int64_t pitch) { return pitch <= 64 ? 1 : (pitch <= 128 ? 2 : 4); }
+int tree_vec_dividing(int64_t pitch, const void *x, const void *rowgrad)
 {
-    const uintptr_t align = (uintptr_t)x | (uintptr_t)grad_x | (uintptr_t)(pitch * 4);
-    const int fit = pitch <= 64 ? 1 : (pitch <= 128 ? 2 : 4);
+    const uintptr_t align = (uintptr_t)x | (uintptr_t)rowgrad | (uintptr_t)(pitch * 4);
+    const int fit = tree_vec(pitch);
     return (align & 15) == 0 ? fit : ((align & 7) == 0 && fit > 1 ? 2 : 1);
 }
 
@@ -507,7 +563,7 @@ extern "C" int clg_fc_tree_forward(const float *x, const int32_t *rows, const fl
     CLG_REQUIRE(batch > 0 && pitch >= batch && pitch < (1ll << 28) && tau != 0.0, "%s: the row pitch must hold the batch, tau must not be zero",
                 name);
     const int slices = tree_slices(roots / k, batch, k);
-    int vec = tree_vec(pitch, x, partial);                                        // fewer samples per lane where the launch would have less than four wavefronts per SIMD
+    int vec = tree_vec(pitch);                                        // fewer samples per lane where the launch would have less than four wavefronts per SIMD
     while (vec > 1 && (int64_t)slices * k * clg_ceil_div(pitch, (int64_t)kWave * vec) * kTreeWaves < 4096) vec /= 2;
     const dim3 grid((unsigned)slices, (unsigned)k, (unsigned)clg_ceil_div(pitch, (int64_t)kWave * vec));
     CLG_REQUIRE(grid.z <= 65535, "%s: batch too large", name);
@@ -542,11 +598,11 @@ extern "C" int clg_fc_tree_backward(const float *x, const int32_t *rows, const i
     CLG_REQUIRE(!grad_x || (pos && rowgrad && start), "%s: the gradient of x needs pos, rowgrad and start", name);
     CLG_REQUIRE(batch > 0 && pitch >= batch && pitch < (1ll << 28) && tau != 0.0, "%s: the row pitch must hold the batch, tau must not be zero",
                 name);
-    const int vec = tree_vec(pitch, (const void *)((uintptr_t)x | (uintptr_t)rowgrad), grad_x);
+    const int vec = tree_vec_dividing(pitch, x, rowgrad), gvec = tree_vec(pitch);
     hipStream_t st = clg_stream(stream);
     const TreeGrads gr = {{grad0, grad1, grad2}, {4 * roots, 6 * roots, 7 * roots}};
     const dim3 grid((unsigned)clg_ceil_div(roots, kTreeWaves));
-    const dim3 ggrid((unsigned)clg_ceil_div(in_dim, kTreeWaves), (unsigned)clg_ceil_div(pitch, (int64_t)kWave * vec));
+    const dim3 ggrid((unsigned)clg_ceil_div(in_dim, kTreeWaves), (unsigned)clg_ceil_div(pitch, (int64_t)kWave * gvec));
     CLG_REQUIRE(ggrid.y <= 65535, "%s: batch too large", name);
 #define CLG_TREE_K(V, SUMS, ROWS)                                                                                                \
     hipLaunchKernelGGL((fc_tree_backward_kernel<V, SUMS, ROWS>), grid, dim3(kTreeBlock), 0, st, x, rows, pos, coef, grad_out, sums, rowgrad, \
@@ -556,13 +612,19 @@ extern "C" int clg_fc_tree_backward(const float *x, const int32_t *rows, const i
         if (logits && grad_x) CLG_TREE_K(V, true, true);                                                                         \
         else if (logits) CLG_TREE_K(V, true, false);                                                                             \
         else CLG_TREE_K(V, false, true);                                                                                         \
-        if (grad_x)                                                                                                              \
-            hipLaunchKernelGGL((fc_tree_gather_kernel<V>), ggrid, dim3(kTreeBlock), 0, st, (const float *)rowgrad, start, grad_x, \
-                               (int)in_dim, pitch, roots * 8);                                                                   \
     } while (0)
+#define CLG_TREE_G(V)                                                                                                            \
+    hipLaunchKernelGGL((fc_tree_gather_kernel<V>), ggrid, dim3(kTreeBlock), 0, st, (const float *)rowgrad, start, grad_x, (int)in_dim, pitch, \
+                       roots * 8)
     if (vec == 1) CLG_TREE_B(1);
     else if (vec == 2) CLG_TREE_B(2);
     else CLG_TREE_B(4);
+    if (grad_x) {
+        if (gvec == 1) CLG_TREE_G(1);
+        else if (gvec == 2) CLG_TREE_G(2);
+        else CLG_TREE_G(4);
+    }
+#undef CLG_TREE_G
 #undef CLG_TREE_B
 #undef CLG_TREE_K
     CLG_CHECK_LAUNCH(name);
@@ -586,8 +648,9 @@ extern "C" int clg_fc_tree_backward(const float *x, const int32_t *rows, const i
 // the counting kernel: 273 us).
 namespace {
 
-// The logits of the blocks in front of the trees, whose gate ids the same launch finds (one thread per gate, in the workgroups from
-// tree_blocks on): one launch of 5 us for a network in place of one per block.
+// The logits of the blocks in front of the trees, whose gate ids the same launch finds (in the workgroups from tree_blocks on): one
+// launch for a network in place of one of 4 us per block.  Four lanes per gate, 16 bytes each: a lane that read the 16 logits of a
+// gate by itself waited for one after the other (75520 roots: 87 us, now 18).
 constexpr int kMaxNetBlocks = 16;
 struct NetGates {
     const float *logits[kMaxNetBlocks];
@@ -600,26 +663,29 @@ __global__ __launch_bounds__(256) void fc_tree_codes_kernel(TreeLogits lg, const
 {
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
     for (int64_t i = e; i < n_counts; i += (int64_t)gridDim.x * 256) counts[i] = 0;   // (for the counting kernel's atomics)
+    const int part = threadIdx.x & 3;
     if ((int)blockIdx.x >= net.tree_blocks) {
-        const int64_t at = e - (int64_t)net.tree_blocks * 256;
+        const int64_t at = (e - (int64_t)net.tree_blocks * 256) >> 2;
         int64_t first = 0;
-        for (int b = 0; b < net.blocks; ++b) {
-            if (at >= first && at < net.end[b]) net.ids[b][at - first] = (uint8_t)argmax16(net.logits[b] + (at - first) * 16);
+        for (int b = 0; b < net.blocks; ++b) {                        // (four lanes together)
+            if (at >= first && at < net.end[b]) {
+                const int id = argmax16_quad(reinterpret_cast<const f32x4u *>(net.logits[b] + (at - first) * 16)[part]);
+                if (part == 0) net.ids[b][at - first] = (uint8_t)id;
+            }
             first = net.end[b];
         }
         return;
     }
-    const int j = (int)(e >> 3), q = (int)(e & 7);                    // eight lanes per root, one gate each
+    const int j = (int)(e >> 5), q = (int)(e >> 2) & 7;               // 32 lanes per root, four per gate
     int id = 0;
-    if (j < roots && q < 7) id = argmax16(tree_logits(lg, ids, j, q, roots));
+    if (j < roots && q < 7) id = argmax16_quad(reinterpret_cast<const f32x4u *>(tree_logits(lg, ids, j, q, roots))[part]);
     uint8_t gate[7];
 #pragma unroll
-    for (int t = 0; t < 7; ++t) gate[t] = (uint8_t)__shfl(id, (threadIdx.x & 56) + t, kWave);
-    if (j < roots && q == 0) codes[j] = tree_code(gate);
+    for (int t = 0; t < 7; ++t) gate[t] = (uint8_t)__shfl(id, (threadIdx.x & 32) + 4 * t, kWave);
+    if (j < roots && q == 0 && part == 0) codes[j] = tree_code(gate);
 }
 
 constexpr int kTreePlanes = 14;                                      // a workgroup takes at most 2^14 - 1 roots
-constexpr int kPackedWaves = 16;
 __device__ __forceinline__ void carry_save(uint32_t &hi, uint32_t &lo, uint32_t a, uint32_t b, uint32_t c)
 {
     const uint32_t u = a ^ b;
@@ -637,14 +703,17 @@ __device__ __forceinline__ void add_counts(uint32_t (&plane)[kTreePlanes], const
     }
 }
 
-template <bool WIDE>
-__global__ __launch_bounds__(kPackedWaves *kWave) void fc_tree_packed_kernel(const uint32_t *__restrict__ x, const int32_t *__restrict__ rows,
+// Slices of a class meet in atomics on `out`, or, where the caller has room, in partial [slices][k][samples] that fc_tree_meet_kernel
+// adds: 985 000 atomics of 52 slices were half of the time at 75520 roots and 1894 samples (97 us, now 23 and 5; 10240
+// roots and 256 samples 14 -> 9 us).
+template <bool WIDE, int WAVES>
+__global__ __launch_bounds__(WAVES *kWave) void fc_tree_packed_kernel(const uint32_t *__restrict__ x, const int32_t *__restrict__ rows,
                                                                             const uint32_t *__restrict__ codes, int32_t *__restrict__ out,
-                                                                            float *__restrict__ sums, float inv_tau,
+                                                                            float *__restrict__ sums, float inv_tau, int32_t *__restrict__ partial,
                                                                             int class_rows, int k, int slices, uint32_t words,
                                                                             int64_t samples, int in_dim, int cols_log2, unsigned col_blocks)
 {
-    __shared__ uint32_t meet[kPackedWaves][kTreePlanes][kWave];
+    __shared__ uint32_t meet[WAVES][kTreePlanes][kWave];
     const int lane = threadIdx.x & (kWave - 1), wave = uniform((int)(threadIdx.x >> 6));
     const int cols = WIDE ? kWave : 1 << cols_log2, phases = WIDE ? 1 : kWave >> cols_log2, phase = WIDE ? 0 : lane >> cols_log2;
     // block -> (class, slice, column block): eight column blocks at a time, one per XCD, over all classes and slices
@@ -653,7 +722,7 @@ __global__ __launch_bounds__(kPackedWaves *kWave) void fc_tree_packed_kernel(con
     const unsigned cs = in_group / wide, cb = group * 8 + in_group % wide;
     const int g = (int)(cs / slices), slice = (int)(cs % slices);
     const uint32_t col0 = cb * cols, col = col0 + (lane & (cols - 1)), at = col < words ? col : words - 1;
-    const int part = slice * kPackedWaves + wave, parts = slices * kPackedWaves;
+    const int part = slice * WAVES + wave, parts = slices * WAVES;
     const int r0 = (int)((int64_t)class_rows * part / parts), r1 = (int)((int64_t)class_rows * (part + 1) / parts);
     uint32_t plane[kTreePlanes];
 #pragma unroll
@@ -699,54 +768,75 @@ __global__ __launch_bounds__(kPackedWaves *kWave) void fc_tree_packed_kernel(con
 #pragma unroll
     for (int q = 0; q < kTreePlanes; ++q) meet[wave][q][lane] = plane[q];
     __syncthreads();
-    // the wavefronts' counts in two rounds: wavefront w < 4 adds four of them, then everybody adds those four
-    if (wave < 4) {
-        for (int wv = 4; wv < kPackedWaves; wv += 4) {
+    // the wavefronts' counts in two rounds: wavefront w < 4 adds every fourth of them, then a thread per column those four
+    if constexpr (WAVES > 4) {
+        if (wave < 4) {
+            for (int wv = 4; wv < WAVES; wv += 4) {
+                uint32_t other[kTreePlanes];
+#pragma unroll
+                for (int q = 0; q < kTreePlanes; ++q) other[q] = meet[wave + wv][q][lane];
+                add_counts(plane, other);
+            }
+#pragma unroll
+            for (int q = 0; q < kTreePlanes; ++q) meet[wave][q][lane] = plane[q];
+        }
+        __syncthreads();
+    }
+    if (wave == 0) {
+#pragma unroll
+        for (int wv = 1; wv < 4; ++wv) {
             uint32_t other[kTreePlanes];
 #pragma unroll
-            for (int q = 0; q < kTreePlanes; ++q) other[q] = meet[wave + wv][q][lane];
+            for (int q = 0; q < kTreePlanes; ++q) other[q] = meet[wv][q][lane];
             add_counts(plane, other);
         }
 #pragma unroll
-        for (int q = 0; q < kTreePlanes; ++q) meet[wave][q][lane] = plane[q];
+        for (int q = 0; q < kTreePlanes; ++q) meet[0][q][lane] = plane[q];
     }
     __syncthreads();
-    const int c = threadIdx.x & (cols - 1);
-    uint32_t total[kTreePlanes];
-#pragma unroll
-    for (int q = 0; q < kTreePlanes; ++q) total[q] = meet[0][q][c];
-    for (int wv = 1; wv < 4; ++wv) {
-        uint32_t other[kTreePlanes];
-#pragma unroll
-        for (int q = 0; q < kTreePlanes; ++q) other[q] = meet[wv][q][c];
-        add_counts(total, other);
-    }
-    if (col0 + c >= words) return;
-    const int step = kPackedWaves * kWave / cols;
-    for (int b = threadIdx.x / cols; b < 32; b += step) {
+    // consecutive threads take consecutive samples
+    const int b = threadIdx.x & 31;
+    for (int c = threadIdx.x >> 5; c < cols; c += WAVES * 2) {
         const int64_t s = (int64_t)(col0 + c) * 32 + b;
-        if (s >= samples) break;
+        if (s >= samples) break;                                      // (so is every later one; columns past the row as well)
         int32_t cnt = 0;
 #pragma unroll
-        for (int q = 0; q < kTreePlanes; ++q) cnt |= (int32_t)((total[q] >> b) & 1) << q;
-        if (slices > 1) atomicAdd(out + s * k + g, cnt);
+        for (int q = 0; q < kTreePlanes; ++q) cnt |= (int32_t)((meet[0][q][c] >> b) & 1) << q;
+        if (partial != nullptr) partial[((int64_t)slice * k + g) * samples + s] = cnt;
+        else if (slices > 1) atomicAdd(out + s * k + g, cnt);
         else if (sums != nullptr) sums[s * k + g] = (float)cnt * inv_tau;
         else out[s * k + g] = cnt;
     }
 }
 
-__global__ __launch_bounds__(256) void fc_tree_sums_kernel(const int32_t *__restrict__ counts, float *__restrict__ sums, int64_t n, float inv_tau)
+// out or sums [samples][k] = sum over the slices of partial [slices][k][samples]
+__global__ __launch_bounds__(256) void fc_tree_meet_kernel(const int32_t *__restrict__ partial, int32_t *__restrict__ out, float *__restrict__ sums,
+                                                         int slices, int k, int64_t samples, float inv_tau)
 {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e < n) sums[e] = (float)counts[e] * inv_tau;
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x, n = samples * k;
+    if (e >= n) return;
+    const int64_t g = e / samples, s = e - g * samples;
+    int32_t cnt = 0;
+    int i = 0;
+    for (; i + 8 <= slices; i += 8) {
+        int32_t v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = partial[(i + u) * n + e];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) cnt += v[u];
+    }
+    for (; i < slices; ++i) cnt += partial[i * n + e];
+    if (sums != nullptr) sums[s * k + g] = (float)cnt * inv_tau;
+    else out[s * k + g] = cnt;
 }
 
-// How a launch is cut: columns of 32-bit words per workgroup, slices of a class
+// How a launch is cut: columns of 32-bit words per workgroup, slices of a class, wavefronts of a workgroup
 struct PackedCut {
-    int cols_log2;
+    int cols_log2, waves;
     int64_t col_blocks, slices;
 };
-PackedCut cut_packed(int64_t roots, int64_t k, int64_t words)
+// meet: the slices meet in a partial buffer, not in atomics
+PackedCut cut_packed(int64_t roots, int64_t k, int64_t words, bool meet)
 {
     const int64_t class_rows = roots / k, halves = words * 2;        // 32-bit words of a row: a lane takes one
     PackedCut c;
@@ -754,31 +844,38 @@ PackedCut cut_packed(int64_t roots, int64_t k, int64_t words)
     while (c.cols_log2 > 0 && (1ll << (c.cols_log2 - 1)) >= halves) --c.cols_log2;
     c.col_blocks = clg_ceil_div(halves, 1ll << c.cols_log2);
     // One workgroup takes all roots of its columns and class where that gives half of the CUs one; else the classes are sliced
-    // down to two steps of roots per wavefront, and the slices meet in atomics.  (Twelve slices of a class at 65 536 samples:
-    // 7.9 M atomics, 385 us instead of 66.)  A workgroup takes at most 2^14 - 4 roots.
-    const int64_t phases = 64 >> c.cols_log2;
-    int64_t slices = k * c.col_blocks >= 128 ? 1 : clg_ceil_div(512, k * c.col_blocks);
-    slices = std::min(slices, class_rows / (8 * phases * kPackedWaves));
+    // down to two steps of roots per wavefront, two workgroups per CU (what LDS holds of them).  (Twelve slices of a class at 65 536
+    // samples: 7.9 M atomics, 385 us instead of 66.)  A workgroup takes at most 2^14 - 4 roots.
+    const int64_t phases = 64 >> c.cols_log2, per_slice = k * c.col_blocks;
+    c.waves = 16;
+    int64_t slices = per_slice >= 128 ? 1 : (meet ? 512 / per_slice : clg_ceil_div(512, per_slice));
+    slices = std::min(slices, class_rows / (8 * phases * c.waves));
+    if (meet && std::max<int64_t>(slices, 1) * per_slice < 64) {      // small classes: workgroups of four wavefronts, one step each
+        c.waves = 4;
+        slices = std::min<int64_t>(512 / per_slice, class_rows / (4 * phases * c.waves));
+    }
     c.slices = std::max<int64_t>(std::max<int64_t>(slices, clg_ceil_div(class_rows, (1 << kTreePlanes) - 4)), 1);
     return c;
 }
 
-// counts (int32) or sums (float, counts / tau; where classes are sliced, counts are scratch then) of packed words
-int count_packed(const char *name, const int64_t *x, const int32_t *rows, const uint32_t *codes, int32_t *counts,
-                 float *sums, float inv_tau, int64_t in_dim, int64_t roots, int64_t k, int64_t words, int64_t samples, const PackedCut &c,
-                 hipStream_t st)
+// counts (int32) or sums (float, counts / tau) of packed words; partial: room for slices x k x samples, or null
+int count_packed(const char *name, const int64_t *x, const int32_t *rows, const uint32_t *codes, int32_t *counts, float *sums, float inv_tau,
+                 int32_t *partial, int64_t in_dim, int64_t roots, int64_t k, int64_t words, int64_t samples, const PackedCut &c, hipStream_t st)
 {
-#define CLG_TREE_P(WIDE)                                                                                                      \
-    hipLaunchKernelGGL((fc_tree_packed_kernel<WIDE>), dim3((unsigned)(k * c.slices * c.col_blocks)), dim3(kPackedWaves * kWave), 0, st, \
-                       (const uint32_t *)x, rows, codes, counts, sums, inv_tau, (int)(roots / k), (int)k, (int)c.slices, (uint32_t)(words * 2), \
-                       samples, (int)in_dim, c.cols_log2, (unsigned)c.col_blocks)
-    if (c.cols_log2 == 6) CLG_TREE_P(true);
-    else CLG_TREE_P(false);
+    if (c.slices == 1) partial = nullptr;
+#define CLG_TREE_P(WIDE, WAVES)                                                                                               \
+    hipLaunchKernelGGL((fc_tree_packed_kernel<WIDE, WAVES>), dim3((unsigned)(k * c.slices * c.col_blocks)), dim3(WAVES * kWave), 0, st, \
+                       (const uint32_t *)x, rows, codes, counts, sums, inv_tau, partial, (int)(roots / k), (int)k, (int)c.slices, \
+                       (uint32_t)(words * 2), samples, (int)in_dim, c.cols_log2, (unsigned)c.col_blocks)
+    if (c.waves == 4 && c.cols_log2 == 6) CLG_TREE_P(true, 4);
+    else if (c.waves == 4) CLG_TREE_P(false, 4);
+    else if (c.cols_log2 == 6) CLG_TREE_P(true, 16);
+    else CLG_TREE_P(false, 16);
 #undef CLG_TREE_P
     CLG_CHECK_LAUNCH(name);
-    if (sums != nullptr && c.slices > 1) {
-        hipLaunchKernelGGL(fc_tree_sums_kernel, dim3((unsigned)clg_ceil_div(samples * k, 256)), dim3(256), 0, st, (const int32_t *)counts, sums,
-                           samples * k, inv_tau);
+    if (partial != nullptr) {
+        hipLaunchKernelGGL(fc_tree_meet_kernel, dim3((unsigned)clg_ceil_div(samples * k, 256)), dim3(256), 0, st, (const int32_t *)partial, counts,
+                           sums, (int)c.slices, (int)k, samples, inv_tau);
         CLG_CHECK_LAUNCH(name);
     }
     return CLG_OK;
@@ -787,8 +884,8 @@ int count_packed(const char *name, const int64_t *x, const int32_t *rows, const 
 int make_codes(const char *name, const TreeLogits &lg, const int32_t *ids, uint32_t *codes, int64_t roots, int32_t *counts, int64_t n_counts,
                NetGates net, hipStream_t st)
 {
-    net.tree_blocks = (int)clg_ceil_div(roots * 8, 256);
-    const int64_t gate_blocks = net.blocks ? clg_ceil_div(net.end[net.blocks - 1], 256) : 0;
+    net.tree_blocks = (int)clg_ceil_div(roots * 32, 256);
+    const int64_t gate_blocks = net.blocks ? clg_ceil_div(net.end[net.blocks - 1] * 4, 256) : 0;
     hipLaunchKernelGGL(fc_tree_codes_kernel, dim3((unsigned)(net.tree_blocks + gate_blocks)), dim3(256), 0, st, lg, ids, codes, (int)roots,
                        counts, n_counts, net);
     CLG_CHECK_LAUNCH(name);
@@ -812,12 +909,12 @@ extern "C" int clg_fc_tree_packed(const int64_t *x, const int32_t *rows, const i
     CLG_REQUIRE(x && rows && ids && logits0 && logits1 && logits2 && codes && out, "%s: null pointer argument", name);
     CLG_REQUIRE(words > 0 && samples > 0 && samples <= words * 64 && words < (1ll << 31), "%s: words %lld, samples %lld", name,
                 (long long)words, (long long)samples);
-    const PackedCut c = cut_packed(roots, k, words);
+    const PackedCut c = cut_packed(roots, k, words, false);
     if (int e = check_packed(name, k, words, c)) return e;
     hipStream_t st = clg_stream(stream);
     const TreeLogits lg = {{logits0, logits1, logits2}};
     if (int e = make_codes(name, lg, ids, codes, roots, out, c.slices > 1 ? samples * k : (int64_t)0, NetGates{}, st)) return e;
-    return count_packed(name, x, rows, codes, out, nullptr, 0.f, in_dim, roots, k, words, samples, c, st);
+    return count_packed(name, x, rows, codes, out, nullptr, 0.f, nullptr, in_dim, roots, k, words, samples, c, st);
 }
 
 // ---- a whole network on packed words -----------------------------------------------------------------------------------------
@@ -827,10 +924,10 @@ namespace {
 
 size_t net_up(size_t v) { return (v + 255) & ~(size_t)255; }
 struct NetLayout {
-    size_t gates_off[kMaxNetBlocks], codes_off, counts_off, ping_off, pong_off, ws_off, total;
+    size_t gates_off[kMaxNetBlocks], codes_off, partial_off, ping_off, pong_off, ws_off, total;
 };
 
-// checks the blocks against each other and lays the scratch out: gate ids | codes | counts | two activations | a block's scratch
+// checks the blocks against each other and lays the scratch out: gate ids | codes | slices' counts | two activations | a block's scratch
 int net_layout(const char *name, const clg_packed_block *blocks, int n_blocks, int64_t in_dim, int64_t roots, int64_t k, int64_t samples,
                NetLayout *l)
 {
@@ -852,10 +949,10 @@ int net_layout(const char *name, const clg_packed_block *blocks, int n_blocks, i
         act[b & 1] = std::max(act[b & 1], (size_t)gg.n * c * h * w * 8);
     }
     CLG_REQUIRE(c * h * w == in_dim, "%s: the last block gives %lld features, the trees take %lld", name, (long long)(c * h * w), (long long)in_dim);
-    const PackedCut cut = cut_packed(roots, k, blocks[0].geom.n);
+    const PackedCut cut = cut_packed(roots, k, blocks[0].geom.n, true);
     l->codes_off = at;
-    l->counts_off = l->codes_off + net_up((size_t)roots * 4);
-    l->ping_off = l->counts_off + (cut.slices > 1 ? net_up((size_t)samples * k * 4) : 0);
+    l->partial_off = l->codes_off + net_up((size_t)roots * 4);
+    l->ping_off = l->partial_off + (cut.slices > 1 ? net_up((size_t)cut.slices * samples * k * 4) : 0);
     l->pong_off = l->ping_off + net_up(act[0]);
     l->ws_off = l->pong_off + net_up(act[1]);
     l->total = l->ws_off + net_up(ws);
@@ -886,7 +983,7 @@ extern "C" int clg_net_packed(const clg_packed_block *blocks, int n_blocks, cons
                 "%s: null pointer argument, or both or neither of counts and sums", name);
     CLG_REQUIRE(samples > 0 && samples <= words * 64 && (sums == nullptr || tau != 0.0), "%s: words %lld, samples %lld, tau %g", name,
                 (long long)words, (long long)samples, tau);
-    const PackedCut c = cut_packed(roots, k, words);
+    const PackedCut c = cut_packed(roots, k, words, true);
     if (int e = check_packed(name, k, words, c)) return e;
     unsigned char *base = reinterpret_cast<unsigned char *>(scratch);
     NetGates net{};
@@ -901,8 +998,7 @@ extern "C" int clg_net_packed(const clg_packed_block *blocks, int n_blocks, cons
     hipStream_t st = clg_stream(stream);
     const TreeLogits lg = {{logits0, logits1, logits2}};
     uint32_t *codes = reinterpret_cast<uint32_t *>(base + l.codes_off);
-    int32_t *meet = counts != nullptr ? counts : reinterpret_cast<int32_t *>(base + l.counts_off);
-    if (int e = make_codes(name, lg, ids, codes, roots, meet, c.slices > 1 ? samples * k : (int64_t)0, net, st)) return e;
+    if (int e = make_codes(name, lg, ids, codes, roots, nullptr, 0, net, st)) return e;
     const uint64_t *in = reinterpret_cast<const uint64_t *>(x);
     bool flat = false;                                                // the last block wrote its words feature-major
     for (int b = 0; b < n_blocks; ++b) {
@@ -916,5 +1012,6 @@ extern "C" int clg_net_packed(const clg_packed_block *blocks, int n_blocks, cons
     }
     if (!flat)
         if (int e = clg_transpose_2d(8, in, features, words, in_dim, stream)) return e;
-    return count_packed(name, features, rows, codes, meet, sums, sums != nullptr ? 1.f / (float)tau : 0.f, in_dim, roots, k, words, samples, c, st);
+    return count_packed(name, features, rows, codes, counts, sums, sums != nullptr ? 1.f / (float)tau : 0.f,
+                        reinterpret_cast<int32_t *>(base + l.partial_off), in_dim, roots, k, words, samples, c, st);
 }

@@ -38,7 +38,8 @@ def at_once(monkeypatch):
 # samples at the ends of words and of the 32 groups from which the last CIFAR block writes feature-major; classes in one slice and in several
 @pytest.mark.parametrize("topology,k,channels,samples", [("cifar", 8, 3, 1), ("cifar", 8, 9, 64), ("cifar", 32, 9, 65), ("cifar", 16, 3, 1983),
                                                          ("cifar", 16, 3, 1985), ("cifar", 8, 1, 8200), ("mnist", 8, 1, 63), ("mnist", 24, 1, 1000),
-                                                         ("mnist", 9, 2, 4097), ("cifar", 100, 6, 130), ("mnist", 300, 1, 70)])
+                                                         ("mnist", 9, 2, 4097), ("cifar", 100, 6, 130), ("mnist", 300, 1, 70),
+                                                         ("cifar", 64, 3, 1900), ("mnist", 300, 1, 500)])
 def test_counts_and_sums_are_those_of_the_modules(at_once, topology, k, channels, samples):
     model, side = network(topology, k, channels)
     x = (torch.rand(samples, channels, side, side, device=DEV) < 0.5).float()
@@ -52,7 +53,7 @@ def test_counts_and_sums_are_those_of_the_modules(at_once, topology, k, channels
     at_once.clear()
     with torch.no_grad():
         sums = model(x)
-    assert bool(at_once) == (samples >= 192 or model.network[-2].out_dim >= 8192)
+    assert at_once
     # counts are whole numbers in either; the modules' division by tau may round once more
     assert sums.dtype == torch.float32 and torch.equal((sums * model.network[-1].tau).round().int(), want)
     assert torch.allclose(sums, by_modules(model, x), rtol=2e-7, atol=0)
