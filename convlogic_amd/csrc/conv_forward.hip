@@ -14,12 +14,14 @@
 // with a caller-made selection) reads its taps from global memory instead.  Lanes run along conv-output
 // columns, each lane evaluates the tree at conv rows 2r and 2r+1, the horizontal neighbour comes over
 // DPP, and the even lane pools and writes.  The kernel index is uniform per wavefront, so gate
-// parameters and tap offsets sit in scalar registers.
+// parameters and tap offsets sit in scalar registers.  Many channels with enough samples take the
+// wavefront-private staging of conv_pair.hip; choose_forward below has the rule.
 #include <stdlib.h>
 
 #include <algorithm>
 
 #include "conv_ops.h"
+#include "conv_pair.h"
 
 int clg_convblock_check(const clg_conv_geom *gg, Geom *g, int dtype, const char *name);
 int clg_convblock_forward_generic(int dtype, const Geom &g, const void *x, const void *w, const int32_t *selection, void *y,
@@ -594,16 +596,40 @@ bool plan_forward_direct(const Geom &g, int elem, bool needs_folded, DirectPlan 
     return true;
 }
 
+bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
+
 // Which forward path a shape takes: 0 = tiled (all channels in LDS), 1 = tiled with channel subsets,
 // 2 = direct from a padded copy (needs scratch), 3 = any-shape kernel, 4 = one sample per lane on 4x4 images
 // (float gates; needs scratch for the folded coefficients), 5 = one kernel per lane (float gates, at most 16 pooled
-// cells, all planes of a sample in LDS, at least 256 kernels; needs scratch for the folded coefficients).
-int choose_forward(const Geom &g, int elem, int params_per_kernel, bool have_scratch, TilePlan *tp, DirectPlan *dp)
+// cells, all planes of a sample in LDS, at least 256 kernels; needs scratch for the folded coefficients), 6 = two planes per
+// wavefront (pair != null: x starts at a 16-byte boundary; needs scratch for coefficients and tap table).
+int choose_forward(const Geom &g, int elem, int params_per_kernel, bool have_scratch, TilePlan *tp, DirectPlan *dp, PairPlan *pair = nullptr)
 {
     bool lane_sample = have_scratch && params_per_kernel > 1 && clg_convblock_is_4x4(g);
     if (const char *e = clg_knob(K_FWD_4X4)) lane_sample = lane_sample && atoi(e) != 0;
     if (lane_sample) return 4;
     const bool tiled = plan_forward(g, elem, params_per_kernel, tp);
+    if (pair != nullptr && have_scratch && (params_per_kernel == 1) == (elem == 8) && clg_plan_pair(g, elem, pair)) {
+        // Two planes per wavefront, against what the shape takes otherwise (us with the launch that makes the tables).  Where a
+        // sample's channels do not fit LDS it is better at every batch for float gates ([54,1204,8,8] -> 4816 50.8 -> 39.4,
+        // [176,380,8,8] -> 1520 82.8 -> 37.5, [18,46,32,32] -> 571 28.7 -> 25.4) and, its second launch paid for, from
+        // 2^18 wavefronts x channels on for words ([272,105,16,16] -> 420 186 -> 79, [8,105,16,16] -> 420 15.2 -> 13.1, but 4 groups of
+        // them 12.2 -> 12.9).  Where they fit, the tiled kernels stage every channel for every tile of kernels and this one only what
+        // it reads: float gates from 16 channels (24 where the cells of a sample are more than a wavefront) and 2^17 wavefronts x
+        // channels on ([256,128,8,8] -> 512 27.8 -> 22.0, [100,32,12,12] -> 96 20.4 -> 13.3, [64,144,6,6] -> 432 19.0 -> 12.8; [64,16,16,16]
+        // -> 64 9.5 -> 10.5 and [256,16,28,28] -> 64 29 -> 37 stay), words up to 16 cells ([1024,128,8,8] -> 512 97 -> 86; [1024,32,16,16] ->
+        // 128 73 -> 82 stays: staging a pair writes as many words as its kernel reads).
+        const int I = (g.ho / 2) * (g.wo / 2);
+        const bool fits = tiled && !tp->subset, words = elem == 8;
+        const int64_t work = (int64_t)pair->groups * g.c * clg_ceil_div((int64_t)pair->G * I, kWave) * g.cin;
+        bool use = words ? work >= (1 << 18) && (!fits || I <= 16) : !fits || (work > (1 << 17) && g.cin >= (I > kWave ? 24 : 16));
+        use = use && !clg_knob(K_FWD_DIRECT) && !clg_knob(K_FWD_SUBSET) && !clg_knob(K_FWD_KPL);   // (a path that is asked for)
+        if (const char *e = clg_knob(K_FWD_PAIR)) use = atoi(e) != 0;
+        if (use) {
+            plan_common(g, tp);
+            return 6;
+        }
+    }
     {
         // one kernel per lane: 40.4 -> 21.2 us (+ 3.9 us for the launch that folds the coefficients) at [256,128,8,8] -> 512
         const int I = (g.ho / 2) * (g.wo / 2);
@@ -767,9 +793,11 @@ extern "C" int64_t clg_convblock_forward_scratch_bytes(int dtype, const clg_conv
     if (clg_convblock_check(gg, &g, dtype, "clg_convblock_forward_scratch_bytes")) return -1;
     TilePlan tp;
     DirectPlan dp;
+    PairPlan pp;
     const int elem = dtype == CLG_F64 ? 8 : 4;
     const int path = choose_forward(g, elem, 28, true, &tp, &dp);
-    return path == 2 ? (int64_t)dp.total : (path == 4 || path == 5 ? (int64_t)g.c * 28 * elem : 0);
+    const int64_t bytes = path == 2 ? (int64_t)dp.total : (path == 4 || path == 5 ? (int64_t)g.c * 28 * elem : 0);
+    return choose_forward(g, elem, 28, true, &tp, &dp, &pp) == 6 ? std::max(bytes, (int64_t)pp.total_bytes) : bytes;   // (6 depends on x's address)
 }
 
 extern "C" int clg_convblock_forward_ws(int dtype, const clg_conv_geom *gg, const void *x, const void *w, const int32_t *selection,
@@ -781,8 +809,12 @@ extern "C" int clg_convblock_forward_ws(int dtype, const clg_conv_geom *gg, cons
     TilePlan tp;
     DirectPlan dp;
     const int elem = dtype == CLG_F64 ? 8 : 4;
-    const int path = choose_forward(g, elem, 28, scratch != nullptr, &tp, &dp);
+    PairPlan pp;
+    const int path = choose_forward(g, elem, 28, scratch != nullptr, &tp, &dp, aligned16(x) ? &pp : nullptr);
     hipStream_t st = clg_stream(stream);
+    if (path == 6)
+        return clg_forward_pair_f32(g, pp, (const float *)x, (const float *)w, selection, (float *)y, argmax, scratch, false, nullptr, nullptr, nullptr,
+                                    0, 0, 0, st, "clg_convblock_forward_ws");
     if (path == 4 || path == 5) {
         const dim3 pgrid((unsigned)clg_ceil_div((int64_t)g.c * 7, 256));
         if (dtype == CLG_F32)
@@ -843,7 +875,8 @@ static int forward_ex_impl(const char *name, int dtype, const clg_conv_geom *gg,
     TilePlan tp;
     DirectPlan dp;
     const int elem = dtype == CLG_F64 ? 8 : 4;
-    const int path = fm ? 4 : choose_forward(g, elem, 28, scratch != nullptr, &tp, &dp);
+    PairPlan pp;
+    const int path = fm ? 4 : choose_forward(g, elem, 28, scratch != nullptr, &tp, &dp, aligned16(x) ? &pp : nullptr);
     hipStream_t st = clg_stream(stream);
     // the folded coefficients [c_out, 7, 4] follow the probabilities in probs_out
     void *folded_out = want_folded ? reinterpret_cast<unsigned char *>(probs_out) + (size_t)g.c * 112 * elem : nullptr;
@@ -861,6 +894,12 @@ static int forward_ex_impl(const char *name, int dtype, const clg_conv_geom *gg,
         CLG_CHECK_LAUNCH(name);
         return CLG_OK;
     };
+    if (path == 6) {
+        float *probs = (float *)probs_out;
+        return clg_forward_pair_f32(g, pp, (const float *)x, (const float *)w, selection, (float *)y, argmax, scratch, logits && !given, probs,
+                                    given ? (const float *)folded_out : nullptr, (float *)padded_out, tp.rs, tp.chs,
+                                    g.cin * tp.chs + g.ph * tp.rs + g.pw, st, name, want_folded && !given ? (float *)folded_out : nullptr);
+    }
     if (path == 4 || path == 5) {
         g.y_fm = fm ? 1 : 0;
         void *fold_to = want_folded ? folded_out : scratch;             // the kernels read them from wherever they are
@@ -942,7 +981,7 @@ extern "C" int64_t clg_convblock_padded_elems(int dtype, const clg_conv_geom *gg
     DirectPlan dp;
     const int elem = dtype == CLG_F64 ? 8 : 4;
     const int path = choose_forward(g, elem, 28, have_scratch != 0, &tp, &dp);
-    if (path != 0 && path != 2 && path != 5) return 0;
+    if (path != 0 && path != 2 && path != 5) return 0;                // (of an x that does not start at a 16-byte boundary)
     const int64_t se = clg_convblock_backward_padded_sample_elems(dtype, g);
     if (se <= 0) return 0;
     const int64_t mine = path == 2 ? dp.sample_elems : (int64_t)g.cin * tp.chs + g.ph * tp.rs + g.pw;
@@ -1019,7 +1058,9 @@ extern "C" int64_t clg_convblock_eval_packed_scratch_bytes(const clg_conv_geom *
     if (clg_convblock_check(gg, &g, CLG_F64, "clg_convblock_eval_packed_scratch_bytes")) return -1;
     TilePlan tp;
     DirectPlan dp;
-    return choose_forward(g, 8, 1, true, &tp, &dp) == 2 ? (int64_t)dp.total : 0;
+    PairPlan pp;
+    const int64_t bytes = choose_forward(g, 8, 1, true, &tp, &dp) == 2 ? (int64_t)dp.total : 0;
+    return choose_forward(g, 8, 1, true, &tp, &dp, &pp) == 6 ? std::max(bytes, (int64_t)pp.total_bytes) : bytes;
 }
 
 extern "C" int clg_convblock_eval_packed_ws(const clg_conv_geom *gg, const uint64_t *x, const uint8_t *gates, const int32_t *selection,
@@ -1031,7 +1072,10 @@ extern "C" int clg_convblock_eval_packed_ws(const clg_conv_geom *gg, const uint6
     CLG_REQUIRE(x != y, "clg_convblock_eval_packed_ws: x and y must not overlap");
     TilePlan tp;
     DirectPlan dp;
-    if (choose_forward(g, 8, 1, scratch != nullptr, &tp, &dp) != 2) return clg_convblock_eval_packed(gg, x, gates, selection, y, stream);
+    PairPlan pp;
+    const int path = choose_forward(g, 8, 1, scratch != nullptr, &tp, &dp, aligned16(x) ? &pp : nullptr);
+    if (path == 6) return clg_forward_pair_packed(g, pp, x, gates, selection, y, scratch, clg_stream(stream), "clg_convblock_eval_packed_ws");
+    if (path != 2) return clg_convblock_eval_packed(gg, x, gates, selection, y, stream);
     return launch_forward_direct<BitOps, float>(g, dp, x, gates, selection, y, nullptr, scratch, clg_stream(stream),
                                                 "clg_convblock_eval_packed_ws");
 }

@@ -1,0 +1,339 @@
+// Fused conv-logic block, forward, a wavefront at a time: a kernel's taps lie in at most two input planes, so a wavefront copies the two
+// planes of its kernel for the samples of 64 pooled cells into LDS of its own and evaluates the kernel there, lane = pooled
+// cell, the four positions of the window in registers.  No image of all channels (which does not fit LDS from some hundred
+// channels on), no padded copy of x, no barriers.  Element policies of conv_ops.h: float gates with a max pool and its arg-max code, or
+// bitwise gates on 64 samples per word with an OR pool.
+//
+// The planes arrive as 16-byte pieces, requested while the kernel before is evaluated, and go to LDS with shared halos that are
+// zeroed once: a row is `lead` zeros (16 bytes of them, at least the padding) and the w pixels, so that a piece is stored whole
+// where w is a multiple of it; the right halo of a row is the lead of the next, the bottom halo of a plane the top of the next.  A tap is
+// one offset added to the lane's position; the window's other positions are immediate offsets of the same reads, two values each.
+//
+// Bound by the vector ALU and, next to it, by LDS issue: per kernel and 64 cells 97 vector instructions of float gates and 16
+// two-value reads ([128,4096,8,8] -> 16384: 257 us of 111 us that the vector instructions alone take; the kernel before read its taps
+// from a padded copy, 355 us), 181 of words and 16 ([272,420,8,8] -> 1680: 77 us, before 226).  Which shapes come here:
+// choose_forward in conv_forward.hip.
+#include <algorithm>
+
+#include "conv_ops.h"
+#include "conv_pair.h"
+
+namespace {
+
+constexpr int kPairWaves = 4;
+constexpr int kPairTable = 12;                                        // per kernel: channel 0, channel 1 (-1: more than two), code, -, 8 taps;
+                                                                      // behind the last one the geometry, for the rare path that needs all of it
+
+// What a launch needs besides x and the selection, in one launch: table, folded coefficients (float gates; the softmax of logits
+// first), the zero-padded copy of x that the backward pass reads.
+template <typename Ops, typename P, typename T>
+__global__ __launch_bounds__(256) void pair_prepare_kernel(const P *__restrict__ w, const int32_t *__restrict__ sel, T *__restrict__ folded,
+                                                         int32_t *__restrict__ table, PairPlan p, Geom g, PadJob<T> pad,
+                                                         int pad_block0, int from_logits, T *__restrict__ probs_out)
+{
+    if ((int)blockIdx.x >= pad_block0) {
+        pad_image_elems(pad, blockIdx.x - pad_block0);
+        return;
+    }
+    const int C = g.c;
+    const TapLimit lim = tap_limit(g);
+    const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if constexpr (!Ops::kOrPool) {
+        if (folded != nullptr && q < (int64_t)C * 7) {
+            T pr[16];
+            if (from_logits) {
+                softmax16(w + q * 16, pr);
+                if (probs_out != nullptr) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) probs_out[q * 16 + i] = pr[i];
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) pr[i] = w[q * 16 + i];
+            }
+            const Coef<T> cf = fold16(pr);
+            folded[q * 4 + 0] = cf.ab;
+            folded[q * 4 + 1] = cf.a;
+            folded[q * 4 + 2] = cf.b;
+            folded[q * 4 + 3] = cf.one;
+        }
+    }
+    if (q == 0) *reinterpret_cast<Geom *>(table + (int64_t)C * kPairTable) = g;
+    if (q < C) {
+        Tap tp[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) tp[t] = unpack_tap(sel[q * 8 + t], lim);
+        const int ch0 = tp[0].ch;
+        int ch1 = ch0;
+#pragma unroll
+        for (int t = 7; t >= 1; --t) ch1 = tp[t].ch != ch0 ? tp[t].ch : ch1;   // first channel that differs
+        bool wide = false;
+        int32_t *row = table + q * kPairTable;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            wide |= tp[t].ch != ch0 && tp[t].ch != ch1;
+            row[4 + t] = (tp[t].ch != ch0 ? p.plane : 0) + tp[t].ry * p.rs + tp[t].rx + p.lead - p.pw;
+        }
+        row[0] = ch0;
+        row[1] = wide ? -1 : ch1;
+        if constexpr (Ops::kOrPool) row[2] = (int32_t)tree_code(w + q * 7);
+    }
+}
+
+// LDS that the lanes of one wavefront share: its accesses complete in order, the compiler has to keep them so
+__device__ __forceinline__ void wave_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <typename Ops>
+__device__ __forceinline__ typename Ops::Params pair_params(const void *__restrict__ folded, const int32_t *__restrict__ row, int c)
+{
+    if constexpr (Ops::kOrPool) {
+        return Ops::unpack((uint32_t)row[2]);
+    } else {
+        typename Ops::Params pr = Ops::load_global(folded, c);
+        pin_addends(pr.tr);
+        return pr;
+    }
+}
+
+// NL: 16-byte pieces per lane.  RS: the row stride where it is known at compile time (else 0).  ROWS: no piece crosses a row.  ONE: the
+// cells of a group of samples are at most 64.  What a lane needs per kernel is worked out once, and the geometry's fields are
+// read again where a kernel's taps are in more than two channels: with them in scalar registers all along the loop spilled some.
+template <typename Ops, int NL, int RS, bool ROWS, bool ONE>
+__global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kernel(const typename Ops::Elem *__restrict__ x, const void *__restrict__ folded,
+                                                                                 const int32_t *__restrict__ table, const int32_t *__restrict__ sel,
+                                                                                 typename Ops::Elem *__restrict__ y, uint8_t *__restrict__ argmax,
+                                                                                 Geom g, PairPlan p)
+{
+    using T = typename Ops::Elem;
+    constexpr int PER = 16 / (int)sizeof(T);
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int lane = threadIdx.x & (kWave - 1), wave = uniform((int)(threadIdx.x >> 6));
+    T *mine = reinterpret_cast<T *>(smem) + wave * p.wave_elems;
+    for (int i = lane * PER; i < p.wave_elems; i += kWave * PER) *reinterpret_cast<u32x4 *>(mine + i) = (u32x4)0u;
+    // the kernel tiles of a group of samples follow each other on one XCD: its L2 holds their planes
+    const unsigned logical = xcd_contiguous_block(blockIdx.x, gridDim.x);
+    const int grp = uniform((int)fdiv(logical, p.d_tiles)), tile = uniform((int)logical) - grp * p.tiles;
+    const int n0 = grp * p.G, g_here = min(p.G, g.n - n0);
+    const int hw = g.h * g.w, wp = g.wo >> 1, I = (g.ho >> 1) * wp;
+    const int row_step = RS ? RS : p.rs;
+    // pieces of this lane: sample s, plane 0 or 1, elements e .. of it; where they go in LDS (a lane without one reads the first
+    // and writes behind the planes)
+    uint32_t from[NL], second[NL];
+    int to[NL][ROWS ? 1 : PER];
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+        const uint32_t v = lane + i * kWave, pl = fdiv(v, p.d_pieces), e = (v - pl * p.pieces) * PER, s = pl >> 1;
+        const bool have = (int)s < g_here;
+        second[i] = have ? pl & 1 : 0;
+        from[i] = have ? (s * (uint32_t)(g.cin * hw) + e) * (uint32_t)sizeof(T) : 0;
+#pragma unroll
+        for (int j = 0; j < (ROWS ? 1 : PER); ++j) {
+            const uint32_t r = fdiv(e + j, p.d_w), col = e + j - r * (uint32_t)g.w;
+            to[i][j] = have ? (int)(s * p.sample + (pl & 1) * p.plane + (r + g.ph) * row_step + p.lead + col) : p.wave_elems - PER + j;
+        }
+    }
+    // cell of this lane: where its window begins in LDS, where its value goes
+    struct Cell {
+        int at;
+        uint32_t out, s, py, px;
+        bool live;
+    };
+    auto cell_of = [&](uint32_t u) {
+        Cell r;
+        r.live = (int)u < g_here * I;
+        const uint32_t uu = r.live ? u : 0;
+        r.s = fdiv(uu, p.d_cells);
+        const uint32_t cell = uu - r.s * (uint32_t)I;
+        r.py = fdiv(cell, p.d_wp), r.px = cell - r.py * (uint32_t)wp;
+        r.at = (int)(r.s * p.sample + 2 * r.py * row_step + 2 * r.px);
+        r.out = r.s * (uint32_t)(g.c * I) + cell;
+        return r;
+    };
+    const T *xg = x + (int64_t)n0 * g.cin * hw;
+    T *yg = y + (int64_t)n0 * g.c * I;
+    uint8_t *ag = argmax + (int64_t)n0 * g.c * I;
+    const int cells = g_here * I, blocks = ONE ? 1 : (cells + kWave - 1) / kWave;
+    const uint32_t plane_bytes = (uint32_t)hw * (uint32_t)sizeof(T);
+    u32x4 piece[NL];
+    auto fetch = [&](int c) {
+        const int32_t *row = table + c * kPairTable;
+        const uint32_t o0 = (uint32_t)row[0] * plane_bytes, d = (uint32_t)max(row[1], 0) * plane_bytes - o0;
+#pragma unroll
+        for (int i = 0; i < NL; ++i)
+            piece[i] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const char *>(xg) + (size_t)(from[i] + o0 + second[i] * d));
+    };
+    const int c_end = min(g.c, (tile + 1) * p.ct);
+    int c = tile * p.ct + wave;
+    if (c >= c_end) return;
+    fetch(c);
+    const Cell first = cell_of(lane);
+    for (;;) {
+        const int32_t *row = table + c * kPairTable;
+        wave_fence();
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            if constexpr (ROWS) {
+                *reinterpret_cast<u32x4 *>(mine + to[i][0]) = piece[i];
+            } else {
+                T part[PER];
+                __builtin_memcpy(part, &piece[i], 16);
+#pragma unroll
+                for (int j = 0; j < PER; ++j) mine[to[i][j]] = part[j];
+            }
+        }
+        wave_fence();
+        const typename Ops::Params pr = pair_params<Ops>(folded, row, c);
+        int off[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) off[t] = row[4 + t];
+        const bool wide = row[1] < 0;
+        const int cn = c + kPairWaves;
+        if (cn < c_end) fetch(cn);                                    // in flight while this kernel is evaluated
+        for (int b = 0; b < blocks; ++b) {
+            const Cell cell = ONE ? first : cell_of(b * kWave + lane);
+            T r[4];
+            if (!wide) {
+                const T *at = mine + cell.at;
+                T v[4][8];
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    const T *q = at + off[t];
+                    v[0][t] = q[0];
+                    v[1][t] = q[1];
+                    v[2][t] = q[row_step];
+                    v[3][t] = q[row_step + 1];
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) r[k] = Ops::root(pr, v[k]);
+            } else {
+                // taps in more than two channels (caller-made selection): from global memory, a position at a time
+                const Geom &full = *reinterpret_cast<const Geom *>(table + g.c * kPairTable);
+                const T *xn = xg + (int64_t)cell.s * full.cin * full.h * full.w;
+#pragma unroll 1
+                for (int k = 0; k < 4; ++k) {
+                    T v[8];
+#pragma unroll
+                    for (int t = 0; t < 8; ++t)
+                        v[t] = read_tap(xn, full, unpack_tap(sel[c * 8 + t], tap_limit(full)), (int)(2 * cell.py) + (k >> 1), (int)(2 * cell.px) + (k & 1));
+                    const T rk = Ops::root(pr, v);
+                    r[0] = k == 0 ? rk : r[0], r[1] = k == 1 ? rk : r[1], r[2] = k == 2 ? rk : r[2], r[3] = k == 3 ? rk : r[3];
+                }
+            }
+            int code;
+            const T best = Ops::pool4(pr, r, code);
+            if (cell.live) {
+                reinterpret_cast<T *>(reinterpret_cast<char *>(yg + (int64_t)c * I) + (size_t)(cell.out * (uint32_t)sizeof(T)))[0] = best;
+                if constexpr (!Ops::kOrPool) (ag + (int64_t)c * I)[cell.out] = (uint8_t)code;
+            }
+        }
+        if (cn >= c_end) return;
+        c = cn;
+    }
+}
+
+template <typename Ops, int NL, int RS, bool ROWS, bool ONE>
+int launch_pair_one(const Geom &g, const PairPlan &p, const void *x, const void *folded, const int32_t *table, const int32_t *sel, void *y, uint8_t *argmax,
+                hipStream_t st, const char *name)
+{
+    using T = typename Ops::Elem;
+    const size_t lds = (size_t)kPairWaves * p.wave_elems * sizeof(T);
+    if (int e = allow_lds(convblock_forward_pair_kernel<Ops, NL, RS, ROWS, ONE>, lds, name)) return e;
+    hipLaunchKernelGGL((convblock_forward_pair_kernel<Ops, NL, RS, ROWS, ONE>), dim3((unsigned)(p.tiles * p.groups)), dim3(kPairWaves * kWave), lds, st,
+                       (const T *)x, folded, table, sel, (T *)y, argmax, g, p);
+    CLG_CHECK_LAUNCH(name);
+    return CLG_OK;
+}
+template <typename Ops, int NL, int RS, bool ROWS>
+int launch_pair(const Geom &g, const PairPlan &p, const void *x, const void *folded, const int32_t *table, const int32_t *sel, void *y, uint8_t *argmax,
+                hipStream_t st, const char *name)
+{
+    if (p.G * (g.ho / 2) * (g.wo / 2) <= kWave) return launch_pair_one<Ops, NL, RS, ROWS, true>(g, p, x, folded, table, sel, y, argmax, st, name);
+    return launch_pair_one<Ops, NL, RS, ROWS, false>(g, p, x, folded, table, sel, y, argmax, st, name);
+}
+template <typename Ops, int NL>
+int launch_pair_nl(const Geom &g, const PairPlan &p, const void *x, const void *folded, const int32_t *table, const int32_t *sel, void *y,
+                   uint8_t *argmax, hipStream_t st, const char *name)
+{
+    constexpr int PER = 16 / (int)sizeof(typename Ops::Elem);
+    if (g.w % PER != 0) return launch_pair<Ops, NL, 0, false>(g, p, x, folded, table, sel, y, argmax, st, name);
+    if (p.rs == 16 + PER) return launch_pair<Ops, NL, 16 + PER, true>(g, p, x, folded, table, sel, y, argmax, st, name);
+    if (p.rs == 8 + PER) return launch_pair<Ops, NL, 8 + PER, true>(g, p, x, folded, table, sel, y, argmax, st, name);
+    return launch_pair<Ops, NL, 0, true>(g, p, x, folded, table, sel, y, argmax, st, name);
+}
+
+}  // namespace
+
+bool clg_plan_pair(const Geom &g, int elem, PairPlan *p)
+{
+    const int per = 16 / elem;
+    if (g.sh != 1 || g.sw != 1 || !taps_inside(g) || g.ho % 2 || g.wo % 2 || g.pw > per || (g.h * g.w) % per) return false;
+    const int I = (g.ho / 2) * (g.wo / 2);
+    p->lead = per;
+    p->pw = g.pw;
+    p->rs = g.w + per;
+    p->plane = (g.h + g.ph) * p->rs;
+    p->G = std::max(1, std::min(kWave / I, g.n));
+    p->pieces = (uint32_t)(g.h * g.w / per);
+    p->loads = (int)clg_ceil_div((int64_t)2 * p->G * p->pieces, kWave);
+    if (p->loads > 8 || (elem == 8 && p->loads > 4)) return false;
+    // samples 16 words apart modulo the 64 banks, so that the rows of neighbouring samples do not meet there
+    p->sample = 2 * p->plane;
+    if (p->G > 1)
+        while (p->sample * (elem / 4) % 64 != 16 || p->sample % per) p->sample += elem == 8 ? 2 : 4;
+    p->wave_elems = (int)(clg_ceil_div((int64_t)p->G * p->sample + g.ph * p->rs + per + g.kw, per) * per + per);   // (the last piece takes what lanes without one write)
+    if ((int64_t)kPairWaves * p->wave_elems * elem > 64 * 1024) return false;
+    p->groups = (int)clg_ceil_div(g.n, p->G);
+    // 32-bit offsets inside a group of samples and in the table
+    if ((int64_t)p->G * g.cin * g.h * g.w * elem >= (1ll << 32) || (int64_t)p->G * g.c * I * elem >= (1ll << 32) || g.c > 65535) return false;
+    // kernels per workgroup: many, for the planes of a sample to be found in L2, as long as there are 8192 wavefronts
+    int64_t ct = 64;
+        while (ct > 4 * kPairWaves && p->groups * clg_ceil_div(g.c, ct) < 2048) ct /= 2;
+    p->ct = (int)ct;
+    p->tiles = (int)clg_ceil_div(g.c, ct);
+    if ((int64_t)p->tiles * p->groups >= (1ll << 31)) return false;
+    p->d_tiles = make_fastdiv((uint32_t)p->tiles);
+    p->d_pieces = make_fastdiv(p->pieces);
+    p->d_w = make_fastdiv((uint32_t)g.w);
+    p->d_wp = make_fastdiv((uint32_t)(g.wo / 2));
+    p->d_cells = make_fastdiv((uint32_t)I);
+    p->folded_bytes = elem == 4 ? ((size_t)g.c * 28 * 4 + 255) & ~(size_t)255 : 0;
+    p->total_bytes = p->folded_bytes + (size_t)g.c * kPairTable * 4 + sizeof(Geom);
+    return true;
+}
+
+// float: w = probabilities or, with from_logits, logits; folded_in: coefficients that are made already, folded_out: where they go
+// (null: scratch).  padded_out: where the zero-padded copy of x goes (strides rs, chs), or null.
+int clg_forward_pair_f32(const Geom &g, const PairPlan &p, const float *x, const float *w, const int32_t *sel, float *y, uint8_t *argmax, void *scratch,
+                         bool from_logits, float *probs_out, const float *folded_in, float *padded_out, int pad_rs, int pad_chs, int pad_sample,
+                         hipStream_t st, const char *name, float *folded_out)
+{
+    unsigned char *base = reinterpret_cast<unsigned char *>(scratch);
+    float *folded = folded_out ? folded_out : reinterpret_cast<float *>(base);
+    int32_t *table = reinterpret_cast<int32_t *>(base + p.folded_bytes);
+    const PadJob<float> job = padded_out ? make_pad_job(x, padded_out, g, pad_rs, pad_chs, pad_sample) : no_pad_job<float>();
+    const unsigned prep = (unsigned)clg_ceil_div((int64_t)g.c * (folded_in ? 1 : 7), 256);
+    hipLaunchKernelGGL((pair_prepare_kernel<FloatOps<float>, float, float>), dim3(prep + pad_blocks(job)), dim3(256), 0, st, w, sel,
+                       folded_in ? (float *)nullptr : folded, table, p, g, job, (int)prep, from_logits ? 1 : 0, probs_out);
+    CLG_CHECK_LAUNCH(name);
+    const void *fc = folded_in ? (const void *)folded_in : (const void *)folded;
+    using Ops = FloatOps<float>;
+    if (p.loads <= 2) return launch_pair_nl<Ops, 2>(g, p, x, fc, table, sel, y, argmax, st, name);
+    if (p.loads <= 4) return launch_pair_nl<Ops, 4>(g, p, x, fc, table, sel, y, argmax, st, name);
+    return launch_pair_nl<Ops, 8>(g, p, x, fc, table, sel, y, argmax, st, name);
+}
+
+int clg_forward_pair_packed(const Geom &g, const PairPlan &p, const uint64_t *x, const uint8_t *gates, const int32_t *sel, uint64_t *y, void *scratch,
+                            hipStream_t st, const char *name)
+{
+    int32_t *table = reinterpret_cast<int32_t *>(scratch);
+    const unsigned prep = (unsigned)clg_ceil_div(g.c, 256);
+    hipLaunchKernelGGL((pair_prepare_kernel<BitOpsAnf, uint8_t, float>), dim3(prep), dim3(256), 0, st, gates, sel, (float *)nullptr, table, p, g,
+                       no_pad_job<float>(), (int)prep, 0, (float *)nullptr);
+    CLG_CHECK_LAUNCH(name);
+    if (p.loads <= 2) return launch_pair_nl<BitOpsAnf, 2>(g, p, x, nullptr, table, sel, y, nullptr, st, name);
+    return launch_pair_nl<BitOpsAnf, 4>(g, p, x, nullptr, table, sel, y, nullptr, st, name);
+}

@@ -1,0 +1,130 @@
+"""The forward kernels that stage the two planes of a kernel per wavefront (csrc/conv_pair.hip), float and packed: the same gates
+on the same values as the staged and the padded-copy kernels, so everything is compared bit for bit with those, at the edges of
+the tiles (samples per wavefront, kernels per workgroup, 16-byte pieces that end in a row), and once with the oracle."""
+import numpy as np
+import pytest
+import torch
+
+import convlogic_amd as C
+from convlogic_amd.hip import convlogic_hip as H
+from oracle import convlogic_oracle as O
+from tests.gpu_util import DEV, check_pool_route, set_knobs
+
+pytestmark = pytest.mark.gpu
+# n, cin, h, w, cout, kernel, padding
+SHAPES = [(1, 3, 8, 8, 5, 3, 1),          # one group that is not full
+          (9, 5, 8, 8, 67, 3, 1),         # 2 groups of 4 samples and one; 67 kernels: the last tile has 3
+          (3, 17, 16, 16, 33, 3, 1),      # one sample per wavefront
+          (15, 6, 6, 6, 18, 3, 1),        # 7 samples of 9 cells: a lane without a cell; rows of 6: pieces cross rows
+          (5, 4, 12, 12, 16, 3, 1),       # 36 cells
+          (2, 3, 14, 14, 9, 3, 1),        # 49 cells, rows of 14
+          (2, 3, 28, 28, 7, 5, 2),        # four blocks of cells, the last of 4
+          (2, 5, 32, 32, 6, 3, 1),        # rows of 32
+          (3, 4, 8, 16, 10, 3, 1),        # not square
+          (3, 4, 16, 8, 10, 5, 2),
+          (4, 3, 10, 10, 8, 3, 0),        # no padding: the top halo is empty
+          (2, 2, 8, 8, 4, 8, 4),          # padding as wide as a piece of floats: (even sizes 9 - 1)
+          (33, 4, 2, 2, 6, 3, 1),         # one cell per sample: 64 samples in a group
+          (2, 1, 20, 12, 4, 3, 1)]        # one channel: both planes are the same
+
+
+def _selection(layer, wide):
+    sel = layer.selection.clone()
+    if wide:                                                          # taps of every third kernel in up to eight channels
+        g = torch.Generator().manual_seed(7)
+        perm = torch.randint(0, sel.shape[0], tuple(sel.shape), generator=g).to(sel.device)
+        mixed = torch.gather(sel, 0, perm)
+        sel[::3] = mixed[::3]
+    return sel.contiguous()
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("n,cin,h,w,c,k,pad", SHAPES)
+def test_float_forward_equals_the_other_kernels_bit_for_bit(n, cin, h, w, c, k, pad, wide, monkeypatch):
+    torch.manual_seed(n * 100 + h)
+    if (h + 2 * pad - k + 1) % 2 or (w + 2 * pad - k + 1) % 2:
+        h, w = h + 1, w + 1                                           # (even conv outputs)
+    layer = C.ConvLogicLayer(cin, c, kernel=k, padding=pad, complete=True, implementation="cuda").to(DEV)
+    sel = _selection(layer, wide)
+    x, logits = torch.randn(n, cin, h, w, device=DEV), layer.weights.detach()
+    probs, geo = torch.softmax(logits, -1), (1, 1, pad, pad, k, k)
+
+    def everything(x):
+        res = [H.full_convlogic_forward_logits(x, logits, sel, *geo, want_folded=True, want_padded=True), H.full_convlogic_forward(x, probs, sel, *geo),
+               H.full_convlogic_forward_logits(x, logits, sel, *geo)]
+        both = torch.cat((res[0][2].reshape(-1), res[0][3].reshape(-1)))
+        given = both[:c * 112].view(c, 7, 16), both[c * 112:].view(c, 7, 4)
+        res.append(H.full_convlogic_forward_logits(x, logits, sel, *geo, want_folded=True, want_padded=True, prefolded=given))
+        return res
+
+    set_knobs(monkeypatch, CLG_FWD_PAIR="0")
+    want = everything(x)
+    set_knobs(monkeypatch, CLG_FWD_PAIR="1")
+    got = everything(x)
+    # and an x that starts 4 bytes behind a 16-byte boundary: the other kernels again, whatever the copy for the backward pass says
+    shifted = torch.empty(x.numel() + 1, device=DEV)[1:].view_as(x).copy_(x)
+    for other in (got, everything(shifted)):
+        for a, b in zip(want, other):
+            assert len(a) == len(b)
+            for u, v in zip(a, b):
+                assert (u is None and v is None) or torch.equal(u, v)
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("n,cin,h,w,c,k,pad", SHAPES)
+def test_packed_forward_equals_the_other_kernels(n, cin, h, w, c, k, pad, wide, monkeypatch):
+    torch.manual_seed(n * 100 + w)
+    if (h + 2 * pad - k + 1) % 2 or (w + 2 * pad - k + 1) % 2:
+        h, w = h + 1, w + 1
+    layer = C.ConvLogicLayer(cin, c, kernel=k, padding=pad, complete=True, implementation="cuda").to(DEV)
+    sel, logits, geo = _selection(layer, wide), torch.randn_like(layer.weights), (1, 1, pad, pad, k, k)
+    x = torch.randint(-2**62, 2**62, (n, cin, h, w), device=DEV)
+    set_knobs(monkeypatch, CLG_FWD_PAIR="0")
+    want = H.full_convlogic_eval_packed_logits(x, logits, sel, geo)
+    set_knobs(monkeypatch, CLG_FWD_PAIR="1")
+    assert torch.equal(want, H.full_convlogic_eval_packed_logits(x, logits, sel, geo))
+    assert np.array_equal(want.cpu().numpy(), O.conv_block_eval_packed(x.cpu().numpy(), logits.argmax(-1).to(torch.uint8).cpu().numpy(), sel.cpu().numpy(),
+                                                                       (1, 1), (pad, pad), (k, k)))
+    shifted = torch.empty(x.numel() + 1, dtype=torch.int64, device=DEV)[1:].view_as(x).copy_(x)
+    assert torch.equal(want, H.full_convlogic_eval_packed_logits(shifted, logits, sel, geo))
+
+
+def test_float_forward_at_values_that_are_not_finite_and_replayed_in_a_graph(monkeypatch):
+    # infinities and NaN take the same way through gates and pool as in the staged kernel; a replay reads what x holds then
+    torch.manual_seed(3)
+    n, cin, h, c = 24, 24, 16, 128                                    # the default choice at this shape
+    layer = C.ConvLogicLayer(cin, c, complete=True, implementation="cuda").to(DEV)
+    x = torch.randn(n, cin, h, h, device=DEV)
+    special = torch.tensor([float("inf"), float("-inf"), float("nan"), -0.0, 3e38, 1e-42], device=DEV)
+    hit = torch.rand_like(x) < 0.02
+    x[hit] = special[torch.randint(0, 6, (int(hit.sum()),), device=DEV)]
+    run = lambda: H.full_convlogic_forward_logits(x, layer.weights.detach(), layer.selection, 1, 1, 1, 1, 3, 3)
+    set_knobs(monkeypatch, CLG_FWD_PAIR="0")
+    want = run()
+    set_knobs(monkeypatch, CLG_FWD_PAIR=None)
+    same = lambda a, b: all(torch.equal(torch.nan_to_num(u.float(), nan=7.0), torch.nan_to_num(v.float(), nan=7.0)) and torch.equal(u.isnan(), v.isnan())
+                            for u, v in zip(a, b))
+    assert same(want, run())
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        run()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        out = run()
+    for seed in (11, 12, 13):
+        x.copy_(torch.rand(x.shape, generator=torch.Generator().manual_seed(seed)))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert same(run(), out)
+
+
+def test_module_against_the_oracle_at_a_shape_of_the_default_choice():
+    torch.manual_seed(4)
+    layer = C.ConvLogicLayer(32, 128, complete=True, implementation="cuda", return_indices=True).to(DEV)
+    x = torch.rand(40, 32, 12, 12, device=DEV)
+    y, idx = layer(x)
+    from tests.gpu_util import block_oracle
+    routed, _, idx_ref, _, _, _, _, x4 = block_oracle(x, layer.weights, layer.selection, (1, 1), (1, 1), (3, 3), idx)
+    check_pool_route(idx, idx_ref, x4)
+    assert (y.detach().cpu() - routed).abs().max().item() <= 1e-5
