@@ -596,20 +596,18 @@ bool plan_forward_direct(const Geom &g, int elem, bool needs_folded, DirectPlan 
     return true;
 }
 
-bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
-
 // Which forward path a shape takes: 0 = tiled (all channels in LDS), 1 = tiled with channel subsets,
 // 2 = direct from a padded copy (needs scratch), 3 = any-shape kernel, 4 = one sample per lane on 4x4 images
 // (float gates; needs scratch for the folded coefficients), 5 = one kernel per lane (float gates, at most 16 pooled
 // cells, all planes of a sample in LDS, at least 256 kernels; needs scratch for the folded coefficients), 6 = two planes per
-// wavefront (pair != null: x starts at a 16-byte boundary; needs scratch for coefficients and tap table).
-int choose_forward(const Geom &g, int elem, int params_per_kernel, bool have_scratch, TilePlan *tp, DirectPlan *dp, PairPlan *pair = nullptr)
+// wavefront (needs scratch for coefficients and tap table).
+int choose_forward(const Geom &g, int elem, int params_per_kernel, bool have_scratch, TilePlan *tp, DirectPlan *dp, PairPlan *pair)
 {
     bool lane_sample = have_scratch && params_per_kernel > 1 && clg_convblock_is_4x4(g);
     if (const char *e = clg_knob(K_FWD_4X4)) lane_sample = lane_sample && atoi(e) != 0;
     if (lane_sample) return 4;
     const bool tiled = plan_forward(g, elem, params_per_kernel, tp);
-    if (pair != nullptr && have_scratch && (params_per_kernel == 1) == (elem == 8) && clg_plan_pair(g, elem, pair)) {
+    if (have_scratch && (params_per_kernel == 1) == (elem == 8) && clg_plan_pair(g, elem, pair)) {
         // Two planes per wavefront, against what the shape takes otherwise (us with the launch that makes the tables).  Where a
         // sample's channels do not fit LDS it is better at every batch for float gates ([54,1204,8,8] -> 4816 50.8 -> 39.4,
         // [176,380,8,8] -> 1520 82.8 -> 37.5, [18,46,32,32] -> 571 28.7 -> 25.4) and, its second launch paid for, from
@@ -795,9 +793,9 @@ extern "C" int64_t clg_convblock_forward_scratch_bytes(int dtype, const clg_conv
     DirectPlan dp;
     PairPlan pp;
     const int elem = dtype == CLG_F64 ? 8 : 4;
-    const int path = choose_forward(g, elem, 28, true, &tp, &dp);
-    const int64_t bytes = path == 2 ? (int64_t)dp.total : (path == 4 || path == 5 ? (int64_t)g.c * 28 * elem : 0);
-    return choose_forward(g, elem, 28, true, &tp, &dp, &pp) == 6 ? std::max(bytes, (int64_t)pp.total_bytes) : bytes;   // (6 depends on x's address)
+    const int path = choose_forward(g, elem, 28, true, &tp, &dp, &pp);
+    if (path == 6) return (int64_t)pp.total_bytes;
+    return path == 2 ? (int64_t)dp.total : (path == 4 || path == 5 ? (int64_t)g.c * 28 * elem : 0);
 }
 
 extern "C" int clg_convblock_forward_ws(int dtype, const clg_conv_geom *gg, const void *x, const void *w, const int32_t *selection,
@@ -810,7 +808,7 @@ extern "C" int clg_convblock_forward_ws(int dtype, const clg_conv_geom *gg, cons
     DirectPlan dp;
     const int elem = dtype == CLG_F64 ? 8 : 4;
     PairPlan pp;
-    const int path = choose_forward(g, elem, 28, scratch != nullptr, &tp, &dp, aligned16(x) ? &pp : nullptr);
+    const int path = choose_forward(g, elem, 28, scratch != nullptr, &tp, &dp, &pp);
     hipStream_t st = clg_stream(stream);
     if (path == 6)
         return clg_forward_pair_f32(g, pp, (const float *)x, (const float *)w, selection, (float *)y, argmax, scratch, false, nullptr, nullptr, nullptr,
@@ -876,7 +874,7 @@ static int forward_ex_impl(const char *name, int dtype, const clg_conv_geom *gg,
     DirectPlan dp;
     const int elem = dtype == CLG_F64 ? 8 : 4;
     PairPlan pp;
-    const int path = fm ? 4 : choose_forward(g, elem, 28, scratch != nullptr, &tp, &dp, aligned16(x) ? &pp : nullptr);
+    const int path = fm ? 4 : choose_forward(g, elem, 28, scratch != nullptr, &tp, &dp, &pp);
     hipStream_t st = clg_stream(stream);
     // the folded coefficients [c_out, 7, 4] follow the probabilities in probs_out
     void *folded_out = want_folded ? reinterpret_cast<unsigned char *>(probs_out) + (size_t)g.c * 112 * elem : nullptr;
@@ -980,8 +978,9 @@ extern "C" int64_t clg_convblock_padded_elems(int dtype, const clg_conv_geom *gg
     TilePlan tp;
     DirectPlan dp;
     const int elem = dtype == CLG_F64 ? 8 : 4;
-    const int path = choose_forward(g, elem, 28, have_scratch != 0, &tp, &dp);
-    if (path != 0 && path != 2 && path != 5) return 0;                // (of an x that does not start at a 16-byte boundary)
+    PairPlan pp;
+    const int path = choose_forward(g, elem, 28, have_scratch != 0, &tp, &dp, &pp);
+    if (path != 0 && path != 2 && path != 5 && path != 6) return 0;
     const int64_t se = clg_convblock_backward_padded_sample_elems(dtype, g);
     if (se <= 0) return 0;
     const int64_t mine = path == 2 ? dp.sample_elems : (int64_t)g.cin * tp.chs + g.ph * tp.rs + g.pw;
@@ -1059,8 +1058,8 @@ extern "C" int64_t clg_convblock_eval_packed_scratch_bytes(const clg_conv_geom *
     TilePlan tp;
     DirectPlan dp;
     PairPlan pp;
-    const int64_t bytes = choose_forward(g, 8, 1, true, &tp, &dp) == 2 ? (int64_t)dp.total : 0;
-    return choose_forward(g, 8, 1, true, &tp, &dp, &pp) == 6 ? std::max(bytes, (int64_t)pp.total_bytes) : bytes;
+    const int path = choose_forward(g, 8, 1, true, &tp, &dp, &pp);
+    return path == 6 ? (int64_t)pp.total_bytes : (path == 2 ? (int64_t)dp.total : 0);
 }
 
 extern "C" int clg_convblock_eval_packed_ws(const clg_conv_geom *gg, const uint64_t *x, const uint8_t *gates, const int32_t *selection,
@@ -1073,7 +1072,7 @@ extern "C" int clg_convblock_eval_packed_ws(const clg_conv_geom *gg, const uint6
     TilePlan tp;
     DirectPlan dp;
     PairPlan pp;
-    const int path = choose_forward(g, 8, 1, scratch != nullptr, &tp, &dp, aligned16(x) ? &pp : nullptr);
+    const int path = choose_forward(g, 8, 1, scratch != nullptr, &tp, &dp, &pp);
     if (path == 6) return clg_forward_pair_packed(g, pp, x, gates, selection, y, scratch, clg_stream(stream), "clg_convblock_eval_packed_ws");
     if (path != 2) return clg_convblock_eval_packed(gg, x, gates, selection, y, stream);
     return launch_forward_direct<BitOps, float>(g, dp, x, gates, selection, y, nullptr, scratch, clg_stream(stream),

@@ -19,3 +19,72 @@ int clg_forward_pair_f32(const Geom &g, const PairPlan &p, const float *x, const
                          hipStream_t st, const char *name, float *folded_out = nullptr);
 int clg_forward_pair_packed(const Geom &g, const PairPlan &p, const uint64_t *x, const uint8_t *gates, const int32_t *sel, uint64_t *y, void *scratch,
                             hipStream_t st, const char *name);
+
+constexpr int kPairWaves = 4;
+// The 28 sums per kernel of a float block's weight gradient by the same staging (conv_pair_grad.hip): partial [c][nb][28].
+int clg_pair_grad_w_parts(const Geom &g, const PairPlan &p);          // nb, at most 64
+int clg_pair_grad_w(const Geom &g, const PairPlan &p, int nb, const float *gy, const float *x, const float *folded, const int32_t *sel,
+                    const uint8_t *argmax, float *partial, hipStream_t st, const char *name);
+
+#if defined(__HIPCC__)
+namespace {
+
+// LDS that the lanes of one wavefront share: its accesses complete in order, the compiler has to keep them so
+__device__ __forceinline__ void wave_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The 16-byte pieces of two planes of a group of samples on their way to LDS: fetch() requests those of two channels, store() puts them
+// into the rows of the image.  ROWS: no piece crosses a row.  A lane without a piece reads the first one and writes
+// behind the planes.
+typedef u32x4 u32x4_any __attribute__((aligned(4)));                  // (global memory takes 16 bytes at every multiple of four)
+template <typename T, int NL, bool ROWS>
+struct PairPieces {
+    static constexpr int PER = 16 / (int)sizeof(T);
+    uint32_t from[NL], second[NL];                                   // second: all ones for a piece of channel 1
+    int to[NL][ROWS ? 1 : PER];
+    u32x4 piece[NL];
+    __device__ __forceinline__ void place(const Geom &g, const PairPlan &p, int row_step, int g_here, int lane)
+    {
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const uint32_t v = lane + i * kWave, pl = fdiv(v, p.d_pieces), e = (v - pl * p.pieces) * PER, s = pl >> 1, plane = pl & 1;
+            const bool have = (int)s < g_here;
+            second[i] = have && plane ? ~0u : 0u;
+            from[i] = have ? (s * (uint32_t)(g.cin * g.h * g.w) + e) * (uint32_t)sizeof(T) : 0;
+#pragma unroll
+            for (int j = 0; j < (ROWS ? 1 : PER); ++j) {
+                const uint32_t r = fdiv(e + j, p.d_w), col = e + j - r * (uint32_t)g.w;
+                to[i][j] = have ? (int)(s * p.sample + plane * p.plane + (r + g.ph) * row_step + p.lead + col) : p.wave_elems - PER + j;
+            }
+        }
+    }
+    // o0: bytes from the group's first sample to its channel 0, d: from there to channel 1 (modulo 2^32)
+    __device__ __forceinline__ void fetch(const T *__restrict__ xg, uint32_t o0, uint32_t d)
+    {
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const uint32_t o = from[i] + o0 + (second[i] & d);
+            piece[i] = *reinterpret_cast<const u32x4_any *>(reinterpret_cast<const char *>(xg) + (size_t)o);
+        }
+    }
+    __device__ __forceinline__ void store(T *__restrict__ image)
+    {
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            if constexpr (ROWS) {
+                *reinterpret_cast<u32x4 *>(image + to[i][0]) = piece[i];
+            } else {
+                T part[PER];
+                __builtin_memcpy(part, &piece[i], 16);
+#pragma unroll
+                for (int j = 0; j < PER; ++j) image[to[i][j]] = part[j];
+            }
+        }
+    }
+};
+
+}  // namespace
+#endif

@@ -20,7 +20,6 @@
 
 namespace {
 
-constexpr int kPairWaves = 4;
 constexpr int kPairTable = 12;                                        // per kernel: channel 0, channel 1 (-1: more than two), code, -, 8 taps;
                                                                       // behind the last one the geometry, for the rare path that needs all of it
 
@@ -80,13 +79,6 @@ __global__ __launch_bounds__(256) void pair_prepare_kernel(const P *__restrict__
     }
 }
 
-// LDS that the lanes of one wavefront share: its accesses complete in order, the compiler has to keep them so
-__device__ __forceinline__ void wave_fence()
-{
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 template <typename Ops>
 __device__ __forceinline__ typename Ops::Params pair_params(const void *__restrict__ folded, const int32_t *__restrict__ row, int c)
 {
@@ -120,22 +112,8 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kern
     const int n0 = grp * p.G, g_here = min(p.G, g.n - n0);
     const int hw = g.h * g.w, wp = g.wo >> 1, I = (g.ho >> 1) * wp;
     const int row_step = RS ? RS : p.rs;
-    // pieces of this lane: sample s, plane 0 or 1, elements e .. of it; where they go in LDS (a lane without one reads the first
-    // and writes behind the planes)
-    uint32_t from[NL], second[NL];
-    int to[NL][ROWS ? 1 : PER];
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-        const uint32_t v = lane + i * kWave, pl = fdiv(v, p.d_pieces), e = (v - pl * p.pieces) * PER, s = pl >> 1;
-        const bool have = (int)s < g_here;
-        second[i] = have ? pl & 1 : 0;
-        from[i] = have ? (s * (uint32_t)(g.cin * hw) + e) * (uint32_t)sizeof(T) : 0;
-#pragma unroll
-        for (int j = 0; j < (ROWS ? 1 : PER); ++j) {
-            const uint32_t r = fdiv(e + j, p.d_w), col = e + j - r * (uint32_t)g.w;
-            to[i][j] = have ? (int)(s * p.sample + (pl & 1) * p.plane + (r + g.ph) * row_step + p.lead + col) : p.wave_elems - PER + j;
-        }
-    }
+    PairPieces<T, NL, ROWS> in;
+    in.place(g, p, row_step, g_here, lane);
     // cell of this lane: where its window begins in LDS, where its value goes
     struct Cell {
         int at;
@@ -158,13 +136,10 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kern
     uint8_t *ag = argmax + (int64_t)n0 * g.c * I;
     const int cells = g_here * I, blocks = ONE ? 1 : (cells + kWave - 1) / kWave;
     const uint32_t plane_bytes = (uint32_t)hw * (uint32_t)sizeof(T);
-    u32x4 piece[NL];
     auto fetch = [&](int c) {
         const int32_t *row = table + c * kPairTable;
-        const uint32_t o0 = (uint32_t)row[0] * plane_bytes, d = (uint32_t)max(row[1], 0) * plane_bytes - o0;
-#pragma unroll
-        for (int i = 0; i < NL; ++i)
-            piece[i] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const char *>(xg) + (size_t)(from[i] + o0 + second[i] * d));
+        const uint32_t o0 = (uint32_t)row[0] * plane_bytes;
+        in.fetch(xg, o0, (uint32_t)max(row[1], 0) * plane_bytes - o0);
     };
     const int c_end = min(g.c, (tile + 1) * p.ct);
     int c = tile * p.ct + wave;
@@ -174,17 +149,7 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kern
     for (;;) {
         const int32_t *row = table + c * kPairTable;
         wave_fence();
-#pragma unroll
-        for (int i = 0; i < NL; ++i) {
-            if constexpr (ROWS) {
-                *reinterpret_cast<u32x4 *>(mine + to[i][0]) = piece[i];
-            } else {
-                T part[PER];
-                __builtin_memcpy(part, &piece[i], 16);
-#pragma unroll
-                for (int j = 0; j < PER; ++j) mine[to[i][j]] = part[j];
-            }
-        }
+        in.store(mine);
         wave_fence();
         const typename Ops::Params pr = pair_params<Ops>(folded, row, c);
         int off[8];
@@ -281,7 +246,7 @@ bool clg_plan_pair(const Geom &g, int elem, PairPlan *p)
     p->loads = (int)clg_ceil_div((int64_t)2 * p->G * p->pieces, kWave);
     if (p->loads > 8 || (elem == 8 && p->loads > 4)) return false;
     // samples 16 words apart modulo the 64 banks, so that the rows of neighbouring samples do not meet there
-    p->sample = 2 * p->plane;
+    p->sample = (int)clg_ceil_div(2 * p->plane, per) * per;
     if (p->G > 1)
         while (p->sample * (elem / 4) % 64 != 16 || p->sample % per) p->sample += elem == 8 ? 2 : 4;
     p->wave_elems = (int)(clg_ceil_div((int64_t)p->G * p->sample + g.ph * p->rs + per + g.kw, per) * per + per);   // (the last piece takes what lanes without one write)

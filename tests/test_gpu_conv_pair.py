@@ -25,7 +25,13 @@ SHAPES = [(1, 3, 8, 8, 5, 3, 1),          # one group that is not full
           (4, 3, 10, 10, 8, 3, 0),        # no padding: the top halo is empty
           (2, 2, 8, 8, 4, 8, 4),          # padding as wide as a piece of floats: (even sizes 9 - 1)
           (33, 4, 2, 2, 6, 3, 1),         # one cell per sample: 64 samples in a group
-          (2, 1, 20, 12, 4, 3, 1)]        # one channel: both planes are the same
+          (2, 1, 20, 12, 4, 3, 1),        # one channel: both planes are the same
+          (5, 3, 8, 7, 6, (3, 4), 1)]     # odd rows: a sample's planes are no whole number of pieces
+
+
+def _even_outputs(h, w, k, pad):
+    kh, kw = k if isinstance(k, tuple) else (k, k)
+    return h + (h + 2 * pad - kh + 1) % 2, w + (w + 2 * pad - kw + 1) % 2, (kh, kw)
 
 
 def _selection(layer, wide):
@@ -42,12 +48,11 @@ def _selection(layer, wide):
 @pytest.mark.parametrize("n,cin,h,w,c,k,pad", SHAPES)
 def test_float_forward_equals_the_other_kernels_bit_for_bit(n, cin, h, w, c, k, pad, wide, monkeypatch):
     torch.manual_seed(n * 100 + h)
-    if (h + 2 * pad - k + 1) % 2 or (w + 2 * pad - k + 1) % 2:
-        h, w = h + 1, w + 1                                           # (even conv outputs)
+    h, w, (kh, kw) = _even_outputs(h, w, k, pad)
     layer = C.ConvLogicLayer(cin, c, kernel=k, padding=pad, complete=True, implementation="cuda").to(DEV)
     sel = _selection(layer, wide)
     x, logits = torch.randn(n, cin, h, w, device=DEV), layer.weights.detach()
-    probs, geo = torch.softmax(logits, -1), (1, 1, pad, pad, k, k)
+    probs, geo = torch.softmax(logits, -1), (1, 1, pad, pad, kh, kw)
 
     def everything(x):
         res = [H.full_convlogic_forward_logits(x, logits, sel, *geo, want_folded=True, want_padded=True), H.full_convlogic_forward(x, probs, sel, *geo),
@@ -61,7 +66,7 @@ def test_float_forward_equals_the_other_kernels_bit_for_bit(n, cin, h, w, c, k, 
     want = everything(x)
     set_knobs(monkeypatch, CLG_FWD_PAIR="1")
     got = everything(x)
-    # and an x that starts 4 bytes behind a 16-byte boundary: the other kernels again, whatever the copy for the backward pass says
+    # and an x that starts 4 bytes behind a 16-byte boundary
     shifted = torch.empty(x.numel() + 1, device=DEV)[1:].view_as(x).copy_(x)
     for other in (got, everything(shifted)):
         for a, b in zip(want, other):
@@ -74,17 +79,16 @@ def test_float_forward_equals_the_other_kernels_bit_for_bit(n, cin, h, w, c, k, 
 @pytest.mark.parametrize("n,cin,h,w,c,k,pad", SHAPES)
 def test_packed_forward_equals_the_other_kernels(n, cin, h, w, c, k, pad, wide, monkeypatch):
     torch.manual_seed(n * 100 + w)
-    if (h + 2 * pad - k + 1) % 2 or (w + 2 * pad - k + 1) % 2:
-        h, w = h + 1, w + 1
+    h, w, (kh, kw) = _even_outputs(h, w, k, pad)
     layer = C.ConvLogicLayer(cin, c, kernel=k, padding=pad, complete=True, implementation="cuda").to(DEV)
-    sel, logits, geo = _selection(layer, wide), torch.randn_like(layer.weights), (1, 1, pad, pad, k, k)
+    sel, logits, geo = _selection(layer, wide), torch.randn_like(layer.weights), (1, 1, pad, pad, kh, kw)
     x = torch.randint(-2**62, 2**62, (n, cin, h, w), device=DEV)
     set_knobs(monkeypatch, CLG_FWD_PAIR="0")
     want = H.full_convlogic_eval_packed_logits(x, logits, sel, geo)
     set_knobs(monkeypatch, CLG_FWD_PAIR="1")
     assert torch.equal(want, H.full_convlogic_eval_packed_logits(x, logits, sel, geo))
     assert np.array_equal(want.cpu().numpy(), O.conv_block_eval_packed(x.cpu().numpy(), logits.argmax(-1).to(torch.uint8).cpu().numpy(), sel.cpu().numpy(),
-                                                                       (1, 1), (pad, pad), (k, k)))
+                                                                       (1, 1), (pad, pad), (kh, kw)))
     shifted = torch.empty(x.numel() + 1, dtype=torch.int64, device=DEV)[1:].view_as(x).copy_(x)
     assert torch.equal(want, H.full_convlogic_eval_packed_logits(shifted, logits, sel, geo))
 
