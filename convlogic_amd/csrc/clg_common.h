@@ -35,7 +35,7 @@ void clg_set_error(const char *fmt, ...);
     X(BWDW_CELLS) X(BWDW_PADDED) X(BWDX_BANDS) X(BWDX_CSR) X(BWDX_DIRECT) X(BWDX_HSW) X(BWDX_SPLIT) X(BWD_4X4)         \
     X(EVAL_CHUNK_BYTES) X(EVAL_NPW) X(EVAL_WALK_R) X(EVAL_WALK_SEG) X(FWD_4X4) X(FWD_CT) X(FWD_DIRECT) X(FWD_NW)       \
     X(FWD_ONE_ROW) X(FWD_S) X(FWD_SOFTMAX_IN_KERNEL) X(FWD_SUBSET) X(GSUM_SLICES) X(PACKED_4X4_HALVES) X(PACK_TILE)    \
-    X(BWDW_LDS) X(BIN_CT) X(BIN_S) X(BIN_NW) X(BIN_HSW) X(BIN_PARTS) X(BIN_PIECE) X(BIN_HL) X(FWD_KPL) X(FWD_PAIR)
+    X(BWDW_LDS) X(BIN_CT) X(BIN_S) X(BIN_NW) X(BIN_HSW) X(BIN_PARTS) X(BIN_PIECE) X(BIN_HL) X(FWD_KPL) X(FWD_PAIR) X(BWDW_PAIR)
 enum ClgKnob {
 #define CLG_KNOB_ENUM(name) K_##name,
     CLG_KNOBS(CLG_KNOB_ENUM)
@@ -165,6 +165,19 @@ __device__ __forceinline__ T wave_sum(T v)
         const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), 63);
         return __builtin_bit_cast(T, ((uint64_t)hi << 32) | lo);
     }
+}
+
+// a of both halves in the low half, b of both halves in the high half (v_permlane32_swap + add), and the same for the even /
+// odd rows of 16 lanes of every half
+__device__ __forceinline__ float swap_add32(float a, float b)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+    return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+__device__ __forceinline__ float swap_add16(float a, float b)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+    return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
 }
 
 // Sum over each row of 16 lanes, valid in all of its lanes (the first four steps of wave_sum).

@@ -26,6 +26,7 @@
 #include <mutex>
 #include <new>
 
+#include "conv_pair.h"
 #include "conv_tile.h"
 
 int clg_convblock_check(const clg_conv_geom *gg, Geom *g, int dtype, const char *name);
@@ -1265,6 +1266,7 @@ struct SharedPad {
     const void *xp = nullptr, *folded = nullptr;
     const int32_t *taps = nullptr;
     int sample_elems = 0;
+    bool direct = false;                                             // the input gradient was the direct kernel
     TilePlan p;
 };
 
@@ -1286,6 +1288,7 @@ int launch_backward_x_direct(const Geom &g, const TilePlan &p, int sample_elems,
         shared->folded = tb.folded;
         shared->taps = tb.taps;
         shared->sample_elems = sample_elems;
+        shared->direct = true;
         shared->p = p;
     }
     if (int e = allow_lds(convblock_backward_x_direct_kernel<T>, p.lds_bytes, "clg_convblock_backward_x")) return e;
@@ -1577,6 +1580,19 @@ static int convblock_backward_w_impl(int dtype, const clg_conv_geom *gg, const v
     Geom g;
     if (int e = clg_convblock_check(gg, &g, dtype, name)) return e;
     CLG_REQUIRE(grad_y && x && w && selection && argmax && grad_w && scratch, "%s: null pointer argument", name);
+    // Behind the direct input gradient (many channels, or few samples): planes staged two at a time where the shape allows it, from
+    // x itself ([256,128,8,8] -> 512, both gradients: 51.4 -> 47.3 us; behind the tiled input gradient 112 -> 115 at [64,32,28,28] -> 256).
+    PairPlan pp;
+    bool pair = shared != nullptr && shared->direct && dtype == CLG_F32 && clg_plan_pair(g, 4, &pp);
+    if (const char *e = clg_knob(K_BWDW_PAIR)) pair = pair && atoi(e) != 0;
+    if (pair) {
+        const int nb = clg_pair_grad_w_parts(g, pp);
+        hipStream_t st = clg_stream(stream);
+        if (int e = clg_pair_grad_w(g, pp, nb, (const float *)grad_y, (const float *)x, (const float *)shared->folded, selection, argmax, (float *)scratch,
+                                    st, "clg_convblock_backward_w(two planes)"))
+            return e;
+        return clg_launch_reduce_coef(CLG_F32, scratch, grad_w, g.c, nb, 7, st, "clg_convblock_backward_w(reduce)", probs);
+    }
     if (shared != nullptr && shared->xp != nullptr && g.c <= 65535) {
         if (dtype == CLG_F32) return launch_backward_w_shared<float>(g, *shared, grad_y, argmax, grad_w, scratch, clg_stream(stream), probs);
         return launch_backward_w_shared<double>(g, *shared, grad_y, argmax, grad_w, scratch, clg_stream(stream), probs);

@@ -1,0 +1,203 @@
+// Weight gradient of the fused float32 conv-logic block from planes that a wavefront stages for itself (conv_pair.h; the forward pass in
+// conv_pair.hip has the layout): the tree is recomputed at the arg-max position of a window, lane = pooled cell.
+//
+// The kernel with lanes along a padded copy of x asks the vector cache for eight addresses per lane and cell, 16 clocks each of the
+// one that four SIMDs share: 128 of the 270 clocks it takes per 64 cells.  Here they come as two 16-byte loads of a
+// lane.  102 vector instructions per 64 cells bound it from there ([128,4096,8,8] -> 16384: 253 -> 172 us, 81 of them those;
+// [128,1024,16,16] -> 4096: 191 -> 157; [256,128,8,8] -> 512: 16.9 -> 14).
+// The input gradient was built the same way (own planes resident, the other channel's staged per kernel, gradient planes in LDS) and
+// taken back: 620 to 640 us for both gradients against 597 with the kernel that gathers; a chain of scalar loads, staging
+// and read-add-write rounds per kernel of a list bounds both.
+#include <algorithm>
+
+#include "conv_ops.h"
+#include "conv_pair.h"
+
+namespace {
+
+// A pooled cell of a group of samples: where its window begins in LDS, its place in grad_y (in elements, from the group's first sample).
+struct PairCell {
+    int at;
+    uint32_t out, s, py, px;
+    bool live;
+};
+__device__ __forceinline__ PairCell pair_cell(const Geom &g, const PairPlan &p, int row_step, uint32_t u, int cells, int I, int wp)
+{
+    PairCell r;
+    r.live = (int)u < cells;
+    const uint32_t uu = r.live ? u : 0;
+    r.s = fdiv(uu, p.d_cells);
+    const uint32_t cell = uu - r.s * (uint32_t)I;
+    r.py = fdiv(cell, p.d_wp), r.px = cell - r.py * (uint32_t)wp;
+    r.at = (int)(r.s * p.sample + 2 * r.py * row_step + 2 * r.px);
+    r.out = r.s * (uint32_t)(g.c * I) + cell;
+    return r;
+}
+
+// The 28 sums of a workgroup: every exchange between lane groups halves the number of values a lane holds, then the wavefronts meet in LDS.
+__device__ __forceinline__ void pair_block_sums(float (&v)[28], float *__restrict__ meet, float *__restrict__ dst, int lane, int wave)
+{
+    const int i16 = lane & 15, o = (lane >> 4) & 1, h = lane >> 5;
+    float mine = 0.f;
+#pragma unroll
+    for (int q = 0; q < 7; ++q) {                                     // row (h, o) holds sum 2 o + h of gate q
+        const float u = row16_sum(swap_add16(swap_add32(v[4 * q], v[4 * q + 1]), swap_add32(v[4 * q + 2], v[4 * q + 3])));
+        mine = i16 == q ? u : mine;
+    }
+    __syncthreads();                                                 // (the planes are done with)
+    if (i16 < 7) meet[wave * 28 + 4 * i16 + 2 * o + h] = mine;
+    __syncthreads();
+    if (threadIdx.x < 28) {
+        float s = meet[threadIdx.x];
+#pragma unroll
+        for (int w = 1; w < kPairWaves; ++w) s += meet[w * 28 + threadIdx.x];
+        dst[threadIdx.x] = s;
+    }
+}
+
+// A wavefront owns a kernel and every 4 nb-th group of samples; the planes, grad_y and arg-max codes of the next
+// group are in flight while the current one is evaluated, and the 28 sums (7 gates x (ab, a, b, 1)) stay in registers over all of
+// them.  partial [c][nb][28], added in order by reduce_coef_partials.
+template <int NL, int RS, bool ROWS, bool ONE>
+__global__ __launch_bounds__(kPairWaves *kWave) void convblock_backward_w_pair_kernel(const float *__restrict__ gy, const float *__restrict__ x,
+                                                                                    const float *__restrict__ folded, const int32_t *__restrict__ sel,
+                                                                                    const uint8_t *__restrict__ argmax, float *__restrict__ partial,
+                                                                                    Geom g, PairPlan p, int nb)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int lane = threadIdx.x & (kWave - 1), wave = uniform((int)(threadIdx.x >> 6));
+    float *mine = reinterpret_cast<float *>(smem) + wave * p.wave_elems;
+    for (int i = lane * 4; i < p.wave_elems; i += kWave * 4) *reinterpret_cast<u32x4 *>(mine + i) = (u32x4)0u;
+    // workgroups that read the same samples (one part, every kernel) follow each other on one XCD and share its L2
+    const unsigned logical = xcd_contiguous_block(blockIdx.x, gridDim.x);
+    const int bx = uniform((int)(logical / (unsigned)g.c)), c = uniform((int)logical) - bx * g.c;
+    const int wp = g.wo >> 1, I = (g.ho >> 1) * wp, cells = p.G * I, blocks = ONE ? 1 : (cells + kWave - 1) / kWave;
+    const int row_step = RS ? RS : p.rs;
+    const float *fc = folded + (int64_t)c * 28;
+    Tree<float> tr;
+#pragma unroll
+    for (int q = 0; q < 7; ++q) tr.g[q] = Coef<float>{fc[4 * q], fc[4 * q + 1], fc[4 * q + 2], fc[4 * q + 3]};
+    int ch0, ch1, off[8];
+    bool wide = false;                                               // (taps in more than two channels, by a caller-made selection)
+    {
+        Tap tp[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) tp[t] = unpack_tap(sel[c * 8 + t], tap_limit(g));
+        ch0 = ch1 = tp[0].ch;
+#pragma unroll
+        for (int t = 7; t >= 1; --t) ch1 = tp[t].ch != ch0 ? tp[t].ch : ch1;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            wide |= tp[t].ch != ch0 && tp[t].ch != ch1;
+            off[t] = uniform((tp[t].ch != ch0 ? p.plane : 0) + tp[t].ry * row_step + tp[t].rx + p.lead - p.pw);
+        }
+    }
+    const uint32_t plane_bytes = (uint32_t)(g.h * g.w) * 4u, o0 = (uint32_t)ch0 * plane_bytes, d = (uint32_t)ch1 * plane_bytes - o0;
+    PairPieces<float, NL, ROWS> in;
+    in.place(g, p, row_step, p.G, lane);
+    const PairCell first = pair_cell(g, p, row_step, lane, cells, I, wp);
+    float acc[28];
+#pragma unroll
+    for (int k = 0; k < 28; ++k) acc[k] = 0.f;
+    // the last group is moved back so that it is full; what it shares with the one before does not count again
+    const int step = kPairWaves * nb, sample = g.cin * g.h * g.w;
+    auto start_of = [&](int q) { return min(q * p.G, g.n - p.G); };
+    auto fetch = [&](int q) { in.fetch(x + (int64_t)start_of(q) * sample, o0, d); };
+    int code = 0;
+    float gout = 0.f;
+    auto load_cell = [&](int q, const PairCell &cell) {
+        const int64_t row = ((int64_t)start_of(q) * g.c + c) * I;
+        code = argmax[row + cell.out];
+        gout = gy[row + cell.out];
+    };
+    int q = bx * kPairWaves + wave;
+    if (q < p.groups) {
+        fetch(q);
+        load_cell(q, first);
+    }
+    for (; q < p.groups; q += step) {
+        wave_fence();
+        in.store(mine);
+        wave_fence();
+        const int qn = q + step, n0 = start_of(q);
+        if (qn < p.groups) fetch(qn);
+        for (int b = 0; b < blocks; ++b) {
+            const PairCell cell = ONE ? first : pair_cell(g, p, row_step, b * kWave + lane, cells, I, wp);
+            const int code_now = code;
+            const float gq = gout;
+            if (b + 1 < blocks) load_cell(q, pair_cell(g, p, row_step, (b + 1) * kWave + lane, cells, I, wp));
+            else if (qn < p.groups) load_cell(qn, first);
+            if (!(cell.live && n0 + (int)cell.s >= q * p.G)) continue;
+            float tap[8];
+            if (!wide) {
+                const float *at = mine + cell.at + (code_now >> 1) * row_step + (code_now & 1);
+#pragma unroll
+                for (int t = 0; t < 8; ++t) tap[t] = at[off[t]];
+            } else {
+                const float *xn = x + (int64_t)(n0 + (int)cell.s) * sample;
+#pragma unroll
+                for (int t = 0; t < 8; ++t) 
+                    tap[t] = read_tap(xn, g, unpack_tap(sel[c * 8 + t], tap_limit(g)), (int)(2 * cell.py) + (code_now >> 1), (int)(2 * cell.px) + (code_now & 1));
+            }
+            const TreeVals<float> tv = eval_tree(tr, tap);
+            auto add = [&](int k, float gk, float a, float b2) {
+                const float ga = gk * a;
+                acc[4 * k] = fma_t(ga, b2, acc[4 * k]);
+                acc[4 * k + 1] += ga;
+                acc[4 * k + 2] = fma_t(gk, b2, acc[4 * k + 2]);
+                acc[4 * k + 3] += gk;
+            };
+            add(6, gq, tv.mid[0], tv.mid[1]);
+            const float gm[2] = {gq * gate_da(tr.g[6], tv.mid[1]), gq * gate_db(tr.g[6], tv.mid[0])};
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                const float la = tv.leaf[2 * m], lb = tv.leaf[2 * m + 1];
+                add(4 + m, gm[m], la, lb);
+                add(2 * m, gm[m] * gate_da(tr.g[4 + m], lb), tap[4 * m], tap[4 * m + 1]);
+                add(2 * m + 1, gm[m] * gate_db(tr.g[4 + m], la), tap[4 * m + 2], tap[4 * m + 3]);
+            }
+        }
+    }
+    pair_block_sums(acc, reinterpret_cast<float *>(smem), partial + ((int64_t)c * nb + bx) * 28, lane, wave);
+}
+
+}  // namespace
+
+template <int NL, int RS, bool ROWS, bool ONE>
+static int launch_pair_w(const Geom &g, const PairPlan &p, int nb, const float *gy, const float *x, const float *folded, const int32_t *sel,
+                         const uint8_t *argmax, float *partial, hipStream_t st, const char *name)
+{
+    const size_t lds = (size_t)kPairWaves * p.wave_elems * 4;
+    if (int e = allow_lds(convblock_backward_w_pair_kernel<NL, RS, ROWS, ONE>, lds, name)) return e;
+    hipLaunchKernelGGL((convblock_backward_w_pair_kernel<NL, RS, ROWS, ONE>), dim3((unsigned)(g.c * nb)), dim3(kPairWaves *kWave), lds, st, gy, x,
+                       folded, sel, argmax, partial, g, p, nb);
+    CLG_CHECK_LAUNCH(name);
+    return CLG_OK;
+}
+template <int NL>
+static int launch_pair_w_nl(const Geom &g, const PairPlan &p, int nb, const float *gy, const float *x, const float *folded, const int32_t *sel,
+                            const uint8_t *argmax, float *partial, hipStream_t st, const char *name)
+{
+    const bool one = p.G * (g.ho / 2) * (g.wo / 2) <= kWave;
+    auto *launch = launch_pair_w<NL, 0, true, false>;
+    if (g.w % 4 != 0) launch = one ? launch_pair_w<NL, 0, false, true> : launch_pair_w<NL, 0, false, false>;
+    else if (one) launch = p.rs == 20 ? launch_pair_w<NL, 20, true, true> : (p.rs == 12 ? launch_pair_w<NL, 12, true, true> : launch_pair_w<NL, 0, true, true>);
+    return launch(g, p, nb, gy, x, folded, sel, argmax, partial, st, name);
+}
+
+// Workgroups per kernel: 1024 of them are enough ([256,32,16,16] -> 128, both gradients: 52.7 us without this kernel, 46.9 with 8 per kernel,
+// 50.8 with 16, 63 with 2; [128,4096,8,8] -> 16384: 691, 597 with 1, 617 with 2), and a wavefront takes at least four blocks of cells for its
+// 28 reductions.
+int clg_pair_grad_w_parts(const Geom &g, const PairPlan &p)
+{
+    const int64_t blocks = (int64_t)p.groups * clg_ceil_div((int64_t)p.G * (g.ho / 2) * (g.wo / 2), kWave);
+    return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(64, clg_ceil_div(1024, g.c)), blocks / (4 * kPairWaves)));
+}
+
+int clg_pair_grad_w(const Geom &g, const PairPlan &p, int nb, const float *gy, const float *x, const float *folded, const int32_t *sel,
+                    const uint8_t *argmax, float *partial, hipStream_t st, const char *name)
+{
+    if (p.loads <= 2) return launch_pair_w_nl<2>(g, p, nb, gy, x, folded, sel, argmax, partial, st, name);
+    if (p.loads <= 4) return launch_pair_w_nl<4>(g, p, nb, gy, x, folded, sel, argmax, partial, st, name);
+    return launch_pair_w_nl<8>(g, p, nb, gy, x, folded, sel, argmax, partial, st, name);
+}

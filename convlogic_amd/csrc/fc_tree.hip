@@ -66,19 +66,6 @@ __device__ __forceinline__ int64_t samples_at(int64_t s, int64_t pitch)
     return s >= pitch ? 0 : (s + V <= pitch ? s : pitch - V);
 }
 
-// a of both halves in the low half, b of both halves in the high half (v_permlane32_swap + add), and the same for the even /
-// odd rows of 16 lanes of every half
-__device__ __forceinline__ float swap_add32(float a, float b)
-{
-    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
-    return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
-}
-__device__ __forceinline__ float swap_add16(float a, float b)
-{
-    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
-    return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
-}
-
 // ---- the trees of a wiring ----------------------------------------------------------------------------------------------
 // a / b of the three layers; start / flat: the lists input feature -> neurons of the first layer, increasing in every list, the
 // first operand before the second where a neuron reads a feature twice.

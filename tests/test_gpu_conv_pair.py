@@ -132,3 +132,34 @@ def test_module_against_the_oracle_at_a_shape_of_the_default_choice():
     routed, _, idx_ref, _, _, _, _, x4 = block_oracle(x, layer.weights, layer.selection, (1, 1), (1, 1), (3, 3), idx)
     check_pool_route(idx, idx_ref, x4)
     assert (y.detach().cpu() - routed).abs().max().item() <= 1e-5
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("n,cin,h,w,c,k,pad", SHAPES)
+def test_weight_gradient_against_float64_at_the_same_arg_max(n, cin, h, w, c, k, pad, wide, monkeypatch):
+    # the last group of samples overlaps the one before; parts of a kernel without a block of cells; many parts per kernel
+    torch.manual_seed(n * 100 + h)
+    h, w, (kh, kw) = _even_outputs(h, w, k, pad)
+    layer = C.ConvLogicLayer(cin, c, kernel=k, padding=pad, complete=True, implementation="cuda").to(DEV)
+    sel, geo = _selection(layer, wide), (1, 1, pad, pad)
+    set_knobs(monkeypatch, CLG_BWDX_DIRECT="1")                       # (the kernel stands behind the direct input gradient)
+    for rep in (1, 40):
+        x = torch.rand(n * rep, cin, h, w, device=DEV)
+        probs = torch.softmax(layer.weights.detach(), -1)
+        y, am = H.full_convlogic_forward(x, probs, sel, *geo, kh, kw)
+        gy = torch.randn_like(y)
+        _, ref = H.full_convlogic_backward(gy.double(), x.double(), probs.double(), am, sel, *geo)
+        gx1, gw1 = H.full_convlogic_backward(gy, x, probs, am, sel, *geo)
+        set_knobs(monkeypatch, CLG_BWDW_PAIR="0")
+        gx0, gw0 = H.full_convlogic_backward(gy, x, probs, am, sel, *geo)
+        set_knobs(monkeypatch, CLG_BWDW_PAIR=None)
+        assert torch.equal(gx0, gx1)
+        # every term of the four sums of a gate is at most |grad_y| (values and partial derivatives of gates lie in [-1, 1]); a
+        # gradient adds them with coefficients of absolute sum <= 5.  Rounding: 12 steps make a term, a lane adds one per block of
+        # cells (at least one cell in use each), 6 + 3 + 64 additions join lanes, wavefronts and parts.
+        bound = 5 * (12 + y[:, 0].numel() + 73) * 2.0**-24 * gy.abs().double().sum((0, 2, 3))
+        err = (gw1.double() - ref).abs().amax((1, 2))
+        assert (err <= bound).all(), (rep, (err / bound).max().item())
+        assert err.max() <= 2 * (gw0.double() - ref).abs().max() + 1e-6 * gy.abs().max()
+        if wide and rep == 1:
+            break
