@@ -601,7 +601,7 @@ bool plan_forward_direct(const Geom &g, int elem, bool needs_folded, DirectPlan 
 // (float gates; needs scratch for the folded coefficients), 5 = one kernel per lane (float gates, at most 16 pooled
 // cells, all planes of a sample in LDS, at least 256 kernels; needs scratch for the folded coefficients), 6 = two planes per
 // wavefront (needs scratch for coefficients and tap table).
-int choose_forward(const Geom &g, int elem, int params_per_kernel, bool have_scratch, TilePlan *tp, DirectPlan *dp, PairPlan *pair)
+int choose_forward(const Geom &g, int elem, int params_per_kernel, bool have_scratch, TilePlan *tp, DirectPlan *dp, PairPlan *pair, bool table_ready = false)
 {
     bool lane_sample = have_scratch && params_per_kernel > 1 && clg_convblock_is_4x4(g);
     if (const char *e = clg_knob(K_FWD_4X4)) lane_sample = lane_sample && atoi(e) != 0;
@@ -616,11 +616,16 @@ int choose_forward(const Geom &g, int elem, int params_per_kernel, bool have_scr
         // it reads: float gates from 16 channels (24 where the cells of a sample are more than a wavefront) and 2^17 wavefronts x
         // channels on ([256,128,8,8] -> 512 27.8 -> 22.0, [100,32,12,12] -> 96 20.4 -> 13.3, [64,144,6,6] -> 432 19.0 -> 12.8; [64,16,16,16]
         // -> 64 9.5 -> 10.5 and [256,16,28,28] -> 64 29 -> 37 stay), words up to 16 cells ([1024,128,8,8] -> 512 97 -> 86; [1024,32,16,16] ->
-        // 128 73 -> 82 stays: staging a pair writes as many words as its kernel reads).
+        // 128 73 -> 82 stays: staging a pair writes as many words as its kernel reads) and where one workgroup's image fills a
+        // CU ([141,100,12,12] -> 300 54 -> 30).  table_ready: the table comes from a launch that is made anyway (a whole network): at any
+        // batch ([4,128,8,8] -> 512 11.3 -> 4.5, [4,32,16,16] -> 128 6.4 -> 4.5, [128,32,16,16] -> 128 19 -> 18, but 512 of them 43 -> 47).
         const int I = (g.ho / 2) * (g.wo / 2);
         const bool fits = tiled && !tp->subset, words = elem == 8;
         const int64_t work = (int64_t)pair->groups * g.c * clg_ceil_div((int64_t)pair->G * I, kWave) * g.cin;
-        bool use = words ? work >= (1 << 18) && (!fits || I <= 16) : !fits || (work > (1 << 17) && g.cin >= (I > kWave ? 24 : 16));
+        bool use = !fits || (work > (1 << 17) && g.cin >= (I > kWave ? 24 : 16));
+        if (words)
+            use = (work >= (1 << 18) || table_ready) &&
+                  (!fits || I <= 16 || tp->lds_bytes > 80 * 1024 || (table_ready && (int64_t)pair->groups * g.c <= (1 << 14)));
         use = use && !clg_knob(K_FWD_DIRECT) && !clg_knob(K_FWD_SUBSET) && !clg_knob(K_FWD_KPL);   // (a path that is asked for)
         if (const char *e = clg_knob(K_FWD_PAIR)) use = atoi(e) != 0;
         if (use) {
@@ -1060,6 +1065,13 @@ extern "C" int64_t clg_convblock_eval_packed_scratch_bytes(const clg_conv_geom *
     PairPlan pp;
     const int path = choose_forward(g, 8, 1, true, &tp, &dp, &pp);
     return path == 6 ? (int64_t)pp.total_bytes : (path == 2 ? (int64_t)dp.total : 0);
+}
+
+bool clg_packed_pair(const Geom &g, PairPlan *p)
+{
+    TilePlan tp;
+    DirectPlan dp;
+    return choose_forward(g, 8, 1, true, &tp, &dp, p, true) == 6;
 }
 
 extern "C" int clg_convblock_eval_packed_ws(const clg_conv_geom *gg, const uint64_t *x, const uint8_t *gates, const int32_t *selection,

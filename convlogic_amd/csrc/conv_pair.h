@@ -11,14 +11,20 @@ struct PairPlan {
     uint32_t pieces;          // per plane
     FastDiv d_tiles, d_pieces, d_w, d_wp, d_cells;
     size_t folded_bytes, total_bytes;   // scratch: folded coefficients | table and geometry
+    int out_sample, out_cell;           // the output: elements between samples, between cells of a kernel (whose cells follow those of the kernel before)
 };
+constexpr int kPairTable = 12;          // per kernel: channel 0, channel 1 (-1: more than two), code, -, 8 taps;
+                                        // behind the last one the geometry, for the rare path that needs all of it
 // elem: 4 (float) or 8 (words).  False where the shape is another kernel's.
 bool clg_plan_pair(const Geom &g, int elem, PairPlan *p);
 int clg_forward_pair_f32(const Geom &g, const PairPlan &p, const float *x, const float *w, const int32_t *sel, float *y, uint8_t *argmax, void *scratch,
                          bool from_logits, float *probs_out, const float *folded_in, float *padded_out, int pad_rs, int pad_chs, int pad_sample,
                          hipStream_t st, const char *name, float *folded_out = nullptr);
+// gates: null where the table at the start of the scratch is made already
 int clg_forward_pair_packed(const Geom &g, const PairPlan &p, const uint64_t *x, const uint8_t *gates, const int32_t *sel, uint64_t *y, void *scratch,
                             hipStream_t st, const char *name);
+// Whether a packed block comes here when its table costs no launch of its own (conv_forward.hip).
+bool clg_packed_pair(const Geom &g, PairPlan *p);
 
 constexpr int kPairWaves = 4;
 // The 28 sums per kernel of a float block's weight gradient by the same staging (conv_pair_grad.hip): partial [c][nb][28].

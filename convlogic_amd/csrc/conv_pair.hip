@@ -20,9 +20,6 @@
 
 namespace {
 
-constexpr int kPairTable = 12;                                        // per kernel: channel 0, channel 1 (-1: more than two), code, -, 8 taps;
-                                                                      // behind the last one the geometry, for the rare path that needs all of it
-
 // What a launch needs besides x and the selection, in one launch: table, folded coefficients (float gates; the softmax of logits
 // first), the zero-padded copy of x that the backward pass reads.
 template <typename Ops, typename P, typename T>
@@ -128,12 +125,13 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kern
         const uint32_t cell = uu - r.s * (uint32_t)I;
         r.py = fdiv(cell, p.d_wp), r.px = cell - r.py * (uint32_t)wp;
         r.at = (int)(r.s * p.sample + 2 * r.py * row_step + 2 * r.px);
-        r.out = r.s * (uint32_t)(g.c * I) + cell;
+        r.out = r.s * (uint32_t)p.out_sample + cell * (uint32_t)p.out_cell;
         return r;
     };
     const T *xg = x + (int64_t)n0 * g.cin * hw;
-    T *yg = y + (int64_t)n0 * g.c * I;
-    uint8_t *ag = argmax + (int64_t)n0 * g.c * I;
+    T *yg = y + (int64_t)n0 * p.out_sample;
+    uint8_t *ag = argmax + (int64_t)n0 * p.out_sample;
+    const int kernel_cells = I * p.out_cell;
     const int cells = g_here * I, blocks = ONE ? 1 : (cells + kWave - 1) / kWave;
     const uint32_t plane_bytes = (uint32_t)hw * (uint32_t)sizeof(T);
     auto fetch = [&](int c) {
@@ -191,8 +189,8 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kern
             int code;
             const T best = Ops::pool4(pr, r, code);
             if (cell.live) {
-                reinterpret_cast<T *>(reinterpret_cast<char *>(yg + (int64_t)c * I) + (size_t)(cell.out * (uint32_t)sizeof(T)))[0] = best;
-                if constexpr (!Ops::kOrPool) (ag + (int64_t)c * I)[cell.out] = (uint8_t)code;
+                reinterpret_cast<T *>(reinterpret_cast<char *>(yg + (int64_t)c * kernel_cells) + (size_t)(cell.out * (uint32_t)sizeof(T)))[0] = best;
+                if constexpr (!Ops::kOrPool) (ag + (int64_t)c * kernel_cells)[cell.out] = (uint8_t)code;
             }
         }
         if (cn >= c_end) return;
@@ -235,6 +233,7 @@ int launch_pair_nl(const Geom &g, const PairPlan &p, const void *x, const void *
 bool clg_plan_pair(const Geom &g, int elem, PairPlan *p)
 {
     const int per = 16 / elem;
+    *p = PairPlan{};
     if (g.sh != 1 || g.sw != 1 || !taps_inside(g) || g.ho % 2 || g.wo % 2 || g.pw > per || (g.h * g.w) % per) return false;
     const int I = (g.ho / 2) * (g.wo / 2);
     p->lead = per;
@@ -254,9 +253,13 @@ bool clg_plan_pair(const Geom &g, int elem, PairPlan *p)
     p->groups = (int)clg_ceil_div(g.n, p->G);
     // 32-bit offsets inside a group of samples and in the table
     if ((int64_t)p->G * g.cin * g.h * g.w * elem >= (1ll << 32) || (int64_t)p->G * g.c * I * elem >= (1ll << 32) || g.c > 65535) return false;
+    p->out_sample = g.y_fm ? 1 : g.c * I;
+    p->out_cell = g.y_fm ? g.n : 1;
+    if (g.y_fm && (int64_t)I * g.n * elem >= (1ll << 31)) return false;
     // kernels per workgroup: many, for the planes of a sample to be found in L2, as long as there are 8192 wavefronts
     int64_t ct = 64;
-        while (ct > 4 * kPairWaves && p->groups * clg_ceil_div(g.c, ct) < 2048) ct /= 2;
+    while (ct > 4 * kPairWaves && p->groups * clg_ceil_div(g.c, ct) < 2048) ct /= 2;
+    while (ct > kPairWaves && p->groups * clg_ceil_div(g.c, ct) < 512) ct /= 2;
     p->ct = (int)ct;
     p->tiles = (int)clg_ceil_div(g.c, ct);
     if ((int64_t)p->tiles * p->groups >= (1ll << 31)) return false;
@@ -296,7 +299,8 @@ int clg_forward_pair_packed(const Geom &g, const PairPlan &p, const uint64_t *x,
 {
     int32_t *table = reinterpret_cast<int32_t *>(scratch);
     const unsigned prep = (unsigned)clg_ceil_div(g.c, 256);
-    hipLaunchKernelGGL((pair_prepare_kernel<BitOpsAnf, uint8_t, float>), dim3(prep), dim3(256), 0, st, gates, sel, (float *)nullptr, table, p, g,
+    if (gates != nullptr)
+        hipLaunchKernelGGL((pair_prepare_kernel<BitOpsAnf, uint8_t, float>), dim3(prep), dim3(256), 0, st, gates, sel, (float *)nullptr, table, p, g,
                        no_pad_job<float>(), (int)prep, 0, (float *)nullptr);
     CLG_CHECK_LAUNCH(name);
     if (p.loads <= 2) return launch_pair_nl<BitOpsAnf, 2>(g, p, x, nullptr, table, sel, y, nullptr, st, name);

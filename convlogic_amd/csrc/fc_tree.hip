@@ -24,6 +24,9 @@
 #include <algorithm>
 
 #include "conv_ops.h"
+#include "conv_pair.h"
+
+int clg_convblock_check(const clg_conv_geom *gg, Geom *g, int dtype, const char *name);
 
 namespace {
 
@@ -635,16 +638,52 @@ extern "C" int clg_fc_tree_backward(const float *x, const int32_t *rows, const i
 // the counting kernel: 273 us).
 namespace {
 
-// The logits of the blocks in front of the trees, whose gate ids the same launch finds (in the workgroups from tree_blocks on): one
-// launch for a network in place of one of 4 us per block.  Four lanes per gate, 16 bytes each: a lane that read the 16 logits of a
-// gate by itself waited for one after the other (75520 roots: 87 us, now 18).
+// The blocks in front of the trees: the same launch finds the gate ids of their kernels (in the workgroups from tree_blocks on), or the table
+// of kernels and taps that a block's own kernel reads -- one launch for a network in place of one of 4 us per block and another of 2 to
+// 4 us per table.  Four lanes per gate, 16 bytes each: a lane that read the 16 logits of a gate by itself waited for one
+// after the other (75520 roots: 87 us, now 18).
 constexpr int kMaxNetBlocks = 16;
+struct NetBlock {
+    const float *logits;
+    const int32_t *sel;
+    uint8_t *ids;                 // gate ids [c, 7], or
+    int32_t *table;               // rows of conv_pair.h
+    int end;                      // kernels up to and including the block's
+    int plane, rs, shift;         // of the table's offsets
+    Geom geom;
+};
 struct NetGates {
-    const float *logits[kMaxNetBlocks];
-    uint8_t *ids[kMaxNetBlocks];
-    int64_t end[kMaxNetBlocks];   // gates up to and including the block's
+    NetBlock block[kMaxNetBlocks];
     int blocks, tree_blocks;
 };
+// 32 lanes per kernel, four per gate; the kernel's eight taps are the first eight lanes'
+__device__ __forceinline__ void net_kernel(const NetBlock &b, int64_t c, int lane)
+{
+    const int part = lane & 3, q = (lane >> 2) & 7, half = lane & 32, t = lane & 31;
+    const int32_t tap = b.sel[c * 8 + (t & 7)];                       // (on its way while the gates are found)
+    int id = 0;
+    if (q < 7) id = argmax16_quad(reinterpret_cast<const f32x4u *>(b.logits + (c * 7 + q) * 16)[part]);
+    if (b.table == nullptr) {
+        if (q < 7 && part == 0) b.ids[c * 7 + q] = (uint8_t)id;
+        return;
+    }
+    uint8_t gate[7];
+#pragma unroll
+    for (int u = 0; u < 7; ++u) gate[u] = (uint8_t)__shfl(id, half + 4 * u, kWave);
+    const Tap tp = unpack_tap(tap, tap_limit(b.geom));
+    const int ch0 = __shfl(tp.ch, half, kWave);
+    const uint32_t differ = (uint32_t)(__ballot(tp.ch != ch0) >> half) & 0xFFu;
+    const int ch1 = __shfl(tp.ch, half + (differ ? __builtin_ctz(differ) : 0), kWave);
+    const bool wide = ((uint32_t)(__ballot(tp.ch != ch0 && tp.ch != ch1) >> half) & 0xFFu) != 0;
+    int32_t *row = b.table + c * kPairTable;
+    if (t < 8) row[4 + t] = (tp.ch != ch0 ? b.plane : 0) + tp.ry * b.rs + tp.rx + b.shift;
+    if (t == 0) {
+        row[0] = ch0;
+        row[1] = wide ? -1 : ch1;
+        row[2] = (int32_t)tree_code(gate);
+        if (c == 0) *reinterpret_cast<Geom *>(b.table + (int64_t)b.geom.c * kPairTable) = b.geom;
+    }
+}
 __global__ __launch_bounds__(256) void fc_tree_codes_kernel(TreeLogits lg, const int32_t *__restrict__ ids, uint32_t *__restrict__ codes,
                                                           int roots, int32_t *__restrict__ counts, int64_t n_counts, NetGates net)
 {
@@ -652,14 +691,11 @@ __global__ __launch_bounds__(256) void fc_tree_codes_kernel(TreeLogits lg, const
     for (int64_t i = e; i < n_counts; i += (int64_t)gridDim.x * 256) counts[i] = 0;   // (for the counting kernel's atomics)
     const int part = threadIdx.x & 3;
     if ((int)blockIdx.x >= net.tree_blocks) {
-        const int64_t at = (e - (int64_t)net.tree_blocks * 256) >> 2;
-        int64_t first = 0;
-        for (int b = 0; b < net.blocks; ++b) {                        // (four lanes together)
-            if (at >= first && at < net.end[b]) {
-                const int id = argmax16_quad(reinterpret_cast<const f32x4u *>(net.logits[b] + (at - first) * 16)[part]);
-                if (part == 0) net.ids[b][at - first] = (uint8_t)id;
-            }
-            first = net.end[b];
+        const int64_t at = (e - (int64_t)net.tree_blocks * 256) >> 5;
+        int first = 0;
+        for (int b = 0; b < net.blocks; ++b) {                        // (32 lanes together)
+            if (at >= first && at < net.block[b].end) net_kernel(net.block[b], at - first, threadIdx.x & (kWave - 1));
+            first = net.block[b].end;
         }
         return;
     }
@@ -869,10 +905,10 @@ int count_packed(const char *name, const int64_t *x, const int32_t *rows, const 
 }
 
 int make_codes(const char *name, const TreeLogits &lg, const int32_t *ids, uint32_t *codes, int64_t roots, int32_t *counts, int64_t n_counts,
-               NetGates net, hipStream_t st)
+               NetGates &net, hipStream_t st)
 {
     net.tree_blocks = (int)clg_ceil_div(roots * 32, 256);
-    const int64_t gate_blocks = net.blocks ? clg_ceil_div(net.end[net.blocks - 1] * 4, 256) : 0;
+    const int64_t gate_blocks = net.blocks ? clg_ceil_div((int64_t)net.block[net.blocks - 1].end * 32, 256) : 0;
     hipLaunchKernelGGL(fc_tree_codes_kernel, dim3((unsigned)(net.tree_blocks + gate_blocks)), dim3(256), 0, st, lg, ids, codes, (int)roots,
                        counts, n_counts, net);
     CLG_CHECK_LAUNCH(name);
@@ -900,7 +936,8 @@ extern "C" int clg_fc_tree_packed(const int64_t *x, const int32_t *rows, const i
     if (int e = check_packed(name, k, words, c)) return e;
     hipStream_t st = clg_stream(stream);
     const TreeLogits lg = {{logits0, logits1, logits2}};
-    if (int e = make_codes(name, lg, ids, codes, roots, out, c.slices > 1 ? samples * k : (int64_t)0, NetGates{}, st)) return e;
+    NetGates none{};
+    if (int e = make_codes(name, lg, ids, codes, roots, out, c.slices > 1 ? samples * k : (int64_t)0, none, st)) return e;
     return count_packed(name, x, rows, codes, out, nullptr, 0.f, nullptr, in_dim, roots, k, words, samples, c, st);
 }
 
@@ -914,7 +951,17 @@ struct NetLayout {
     size_t gates_off[kMaxNetBlocks], codes_off, partial_off, ping_off, pong_off, ws_off, total;
 };
 
-// checks the blocks against each other and lays the scratch out: gate ids | codes | slices' counts | two activations | a block's scratch
+// a block's geometry in a network and, where it is staged two planes at a time, its plan; the last one writes its words feature-major
+int net_pair(const char *name, const clg_packed_block *blocks, int n_blocks, int b, Geom *g, PairPlan *p, bool *pair)
+{
+    if (int e = clg_convblock_check(&blocks[b].geom, g, CLG_F64, name)) return e;
+    g->y_fm = b == n_blocks - 1 ? 1 : 0;
+    *pair = !(g->y_fm && clg_convblock_eval_packed_fm_supported(&blocks[b].geom)) && clg_packed_pair(*g, p);
+    if (!*pair) g->y_fm = 0;
+    return CLG_OK;
+}
+
+// checks the blocks against each other and lays the scratch out: gate ids or tables | codes | slices' counts | two activations | a block's scratch
 int net_layout(const char *name, const clg_packed_block *blocks, int n_blocks, int64_t in_dim, int64_t roots, int64_t k, int64_t samples,
                NetLayout *l)
 {
@@ -932,7 +979,11 @@ int net_layout(const char *name, const clg_packed_block *blocks, int n_blocks, i
         h = ((gg.h + 2 * gg.pad_h - gg.kernel_h) / gg.stride_h + 1) / 2;
         w = ((gg.w + 2 * gg.pad_w - gg.kernel_w) / gg.stride_w + 1) / 2;
         l->gates_off[b] = at;
-        at += net_up((size_t)c * 7);
+        Geom g;
+        PairPlan p;
+        bool pair = false;
+        if (int e = net_pair(name, blocks, n_blocks, b, &g, &p, &pair)) return e;
+        at += net_up(pair ? p.total_bytes : (size_t)c * 7);
         act[b & 1] = std::max(act[b & 1], (size_t)gg.n * c * h * w * 8);
     }
     CLG_REQUIRE(c * h * w == in_dim, "%s: the last block gives %lld features, the trees take %lld", name, (long long)(c * h * w), (long long)in_dim);
@@ -975,12 +1026,26 @@ extern "C" int clg_net_packed(const clg_packed_block *blocks, int n_blocks, cons
     unsigned char *base = reinterpret_cast<unsigned char *>(scratch);
     NetGates net{};
     net.blocks = n_blocks;
-    int64_t gates = 0;
+    PairPlan plan[kMaxNetBlocks];
+    int64_t kernels = 0;
     for (int b = 0; b < n_blocks; ++b) {
         CLG_REQUIRE(blocks[b].logits && blocks[b].selection, "%s: null pointer in block %d", name, b);
-        net.logits[b] = blocks[b].logits;
-        net.ids[b] = base + l.gates_off[b];
-        net.end[b] = gates += (int64_t)blocks[b].geom.c_out * 7;
+        NetBlock &nb = net.block[b];
+        bool pair = false;
+        if (int e = net_pair(name, blocks, n_blocks, b, &nb.geom, &plan[b], &pair)) return e;
+        nb.logits = blocks[b].logits;
+        nb.sel = blocks[b].selection;
+        kernels += nb.geom.c;
+        CLG_REQUIRE(kernels < (1ll << 28), "%s: problem too large for one launch", name);
+        nb.end = (int)kernels;
+        if (pair) {
+            nb.table = reinterpret_cast<int32_t *>(base + l.gates_off[b]);
+            nb.plane = plan[b].plane;
+            nb.rs = plan[b].rs;
+            nb.shift = plan[b].lead - plan[b].pw;
+        } else {
+            nb.ids = base + l.gates_off[b];
+        }
     }
     hipStream_t st = clg_stream(stream);
     const TreeLogits lg = {{logits0, logits1, logits2}};
@@ -991,9 +1056,13 @@ extern "C" int clg_net_packed(const clg_packed_block *blocks, int n_blocks, cons
     for (int b = 0; b < n_blocks; ++b) {
         const clg_packed_block &bl = blocks[b];
         uint64_t *out = reinterpret_cast<uint64_t *>(base + ((b & 1) ? l.pong_off : l.ping_off));
-        flat = b == n_blocks - 1 && clg_convblock_eval_packed_fm_supported(&bl.geom);
-        const int e = flat ? clg_convblock_eval_packed_fm(&bl.geom, in, net.ids[b], bl.selection, reinterpret_cast<uint64_t *>(features), stream)
-                           : clg_convblock_eval_packed_ws(&bl.geom, in, net.ids[b], bl.selection, out, base + l.ws_off, stream);
+        const NetBlock &nb = net.block[b];
+        const bool last = b == n_blocks - 1, pair = nb.table != nullptr;
+        flat = last && (pair || clg_convblock_eval_packed_fm_supported(&bl.geom));
+        if (flat) out = reinterpret_cast<uint64_t *>(features);
+        const int e = pair ? clg_forward_pair_packed(nb.geom, plan[b], in, nullptr, bl.selection, out, nb.table, st, name)
+                           : (flat ? clg_convblock_eval_packed_fm(&bl.geom, in, nb.ids, bl.selection, out, stream)
+                                   : clg_convblock_eval_packed_ws(&bl.geom, in, nb.ids, bl.selection, out, base + l.ws_off, stream));
         if (e) return e;
         in = out;
     }

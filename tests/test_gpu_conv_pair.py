@@ -163,3 +163,29 @@ def test_weight_gradient_against_float64_at_the_same_arg_max(n, cin, h, w, c, k,
         assert err.max() <= 2 * (gw0.double() - ref).abs().max() + 1e-6 * gy.abs().max()
         if wide and rep == 1:
             break
+
+
+@pytest.mark.parametrize("topology,k,channels,samples", [("cifar", 9, 3, 70), ("cifar", 16, 6, 640), ("cifar", 8, 3, 2049), ("mnist", 10, 1, 500)])
+@pytest.mark.parametrize("wide", [False, True])
+def test_networks_with_tables_from_the_launch_of_the_codes(topology, k, channels, samples, wide, monkeypatch):
+    # the tables come from the launch that finds the gates of blocks and trees, the last block writes feature-major (also where its
+    # samples do not fill a group): class counts and the words in front of the trees against the other kernels
+    torch.manual_seed(samples)
+    model = (C.ConvLogicCifarModel(k_param=k, input_channels=channels, tau=6.5) if topology == "cifar"
+             else C.ConvLogicMnistModel(k_param=k, input_channels=channels)).to(DEV).eval()
+    side = 32 if topology == "cifar" else 28
+    with torch.no_grad():
+        for p in model.parameters():
+            p.add_(torch.randn_like(p), alpha=2.0)
+        for m in model.network:
+            if isinstance(m, C.ConvLogicLayer):
+                m.selection.copy_(_selection(m, wide))
+    x = torch.rand(samples, channels, side, side, device=DEV) < 0.5
+    seen = []
+    for knob in ("0", None, "1"):
+        set_knobs(monkeypatch, CLG_FWD_PAIR=knob)
+        packed = C.PackBitsTensor(x, 64)
+        with torch.no_grad():
+            seen.append((model(packed), packed.t))
+    for counts, words in seen[1:]:
+        assert torch.equal(counts, seen[0][0]) and torch.equal(words, seen[0][1])
