@@ -2,6 +2,8 @@
 // arg-max code, or bitwise gates on 64 packed samples per uint64 word with an OR pool.
 #pragma once
 
+#include <type_traits>
+
 #include "conv_tile.h"
 
 #if defined(__HIPCC__)
@@ -79,6 +81,19 @@ struct FloatOps {
         return pr;
     }
     static __device__ __forceinline__ Elem root(const Params &pr, const Elem (&v)[8]) { return eval_tree(pr.tr, v).root; }
+    // the four positions of a window; read(t, out): tap t at each
+    template <typename Read>
+    static __device__ __forceinline__ void root4(const Params &pr, Read read, Elem (&r)[4])
+    {
+        Elem v[8][4];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) read(t, v[t]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const Elem tap[8] = {v[0][k], v[1][k], v[2][k], v[3][k], v[4][k], v[5][k], v[6][k], v[7][k]};
+            r[k] = root(pr, tap);
+        }
+    }
     // strict > in window order (0,0),(0,1),(1,0),(1,1): the first maximum wins
     static __device__ __forceinline__ void pool_store(Elem r0, Elem r0o, Elem r1, Elem r1o, Elem *__restrict__ yb,
                                                       uint8_t *__restrict__ ab, int idx)
@@ -203,6 +218,7 @@ struct BitOpsAnf {
     static constexpr bool kOrPool = true;                            // the pool is an OR: any order, no arg-max
     struct Params {
         uint32_t c1[7], c2[7], c3[7], inv;                           // all-ones / all-zeros
+        uint32_t code;
     };
     static __device__ __forceinline__ Params unpack(uint32_t code)
     {
@@ -214,6 +230,7 @@ struct BitOpsAnf {
             pr.c3[k] = 0u - ((code >> (3 * k + 2)) & 1u);
         }
         pr.inv = 0u - ((code >> 21) & 1u);
+        pr.code = code;
         return pr;
     }
     // params = gate ids uint8 [c_out, 7]
@@ -257,6 +274,48 @@ struct BitOpsAnf {
     static __device__ __forceinline__ Elem root_true(const Params &pr, const Elem (&v)[8])
     {
         return root(pr, v) ^ (((uint64_t)pr.inv << 32) | pr.inv);
+    }
+    // The four positions of a window at once.  Enough work per gate for a branch on its kind, which the wavefront takes as one: of the eight
+    // functions that are 0 at (0, 0), two each are one 3-input operation with c2 as the mask -- a third of the operations
+    // of root() ([272,105,16,16] -> 420: 73 us there, 62 here).
+    template <int K>
+    static __device__ __forceinline__ void gate4(uint32_t code, const Elem (&a)[4], const Elem (&b)[4], Elem (&y)[4])
+    {
+        const uint32_t m = 0u - ((code >> (3 * K + 1)) & 1u);
+        auto all = [&](auto table) {
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const uint32_t lo = __builtin_amdgcn_bitop3_b32((uint32_t)a[p], (uint32_t)b[p], m, decltype(table)::value);
+                const uint32_t hi = __builtin_amdgcn_bitop3_b32((uint32_t)(a[p] >> 32), (uint32_t)(b[p] >> 32), m, decltype(table)::value);
+                y[p] = ((uint64_t)hi << 32) | lo;
+            }
+            asm volatile("");                                        // (branches stay branches)
+        };
+        // 0xF0 = a, 0xCC = b, 0xAA = c2
+        if ((code >> (3 * K)) & 1u) {
+            if ((code >> (3 * K + 2)) & 1u) all(std::integral_constant<int, 0xB8>{});        // c2 ? a | b : a & ~b
+            else all(std::integral_constant<int, 0x78>{});                                   // c2 ? a ^ b : a
+        } else {
+            if ((code >> (3 * K + 2)) & 1u) all(std::integral_constant<int, 0x48>{});        // c2 ? ~a & b : a & b
+            else all(std::integral_constant<int, 0x88>{});                                   // c2 ? b : 0
+        }
+    }
+    // (the second subtree's values are read when the first one's leaves are made: 64 registers less at a time)
+    template <typename Read>
+    static __device__ __forceinline__ void root4(const Params &pr, Read read, Elem (&r)[4])
+    {
+        Elem t[4][4], leaf[2][4], mid[2][4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) read(q, t[q]);
+        gate4<0>(pr.code, t[0], t[1], leaf[0]);
+        gate4<1>(pr.code, t[2], t[3], leaf[1]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) read(4 + q, t[q]);
+        gate4<4>(pr.code, leaf[0], leaf[1], mid[0]);
+        gate4<2>(pr.code, t[0], t[1], leaf[0]);
+        gate4<3>(pr.code, t[2], t[3], leaf[1]);
+        gate4<5>(pr.code, leaf[0], leaf[1], mid[1]);
+        gate4<6>(pr.code, mid[0], mid[1], r);
     }
     template <int TABLE>
     static __device__ __forceinline__ Elem join_as(const Params &pr, Elem a, Elem b)

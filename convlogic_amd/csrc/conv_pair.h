@@ -7,16 +7,25 @@ struct PairPlan {
     int G, groups;            // samples per wavefront, groups of them
     int ct, tiles;            // kernels per workgroup, tiles of them
     int lead, pw, rs, plane, sample, wave_elems;   // LDS, in elements: zeros in front of a row, row / plane / sample stride, all of a wavefront
+    int odd;                  // from a row's even columns to its odd ones where they are kept apart, else 0
     int loads;                // 16-byte pieces per lane
     uint32_t pieces;          // per plane
     FastDiv d_tiles, d_pieces, d_w, d_wp, d_cells;
     size_t folded_bytes, total_bytes;   // scratch: folded coefficients | table and geometry
     int out_sample, out_cell;           // the output: elements between samples, between cells of a kernel (whose cells follow those of the kernel before)
 };
+// Of a tap (plane, row, column) from a window's first position: the offset of the window's first column in the low half, of its second in
+// the high one; shift: what the rows' zeros put in front of column 0.
+__host__ __device__ inline int32_t pair_tap(int plane, int rs, int odd, int shift, bool second, int ry, int rx)
+{
+    const int row = (second ? plane : 0) + ry * rs, a = rx + shift, b = a + 1;
+    return (row + (a & 1) * odd + (a >> 1)) | (row + (b & 1) * odd + (b >> 1)) << 16;
+}
 constexpr int kPairTable = 12;          // per kernel: channel 0, channel 1 (-1: more than two), code, -, 8 taps;
                                         // behind the last one the geometry, for the rare path that needs all of it
-// elem: 4 (float) or 8 (words).  False where the shape is another kernel's.
-bool clg_plan_pair(const Geom &g, int elem, PairPlan *p);
+// elem: 4 (float) or 8 (words).  False where the shape is another kernel's.  split: even and odd columns apart, as the forward kernel
+// reads them.
+bool clg_plan_pair(const Geom &g, int elem, PairPlan *p, bool split = true);
 int clg_forward_pair_f32(const Geom &g, const PairPlan &p, const float *x, const float *w, const int32_t *sel, float *y, uint8_t *argmax, void *scratch,
                          bool from_logits, float *probs_out, const float *folded_in, float *padded_out, int pad_rs, int pad_chs, int pad_sample,
                          hipStream_t st, const char *name, float *folded_out = nullptr);
@@ -43,10 +52,10 @@ __device__ __forceinline__ void wave_fence()
 }
 
 // The 16-byte pieces of two planes of a group of samples on their way to LDS: fetch() requests those of two channels, store() puts them
-// into the rows of the image.  ROWS: no piece crosses a row.  A lane without a piece reads the first one and writes
-// behind the planes.
+// into the rows of the image.  ROWS: no piece crosses a row.  SPLIT: even and odd columns apart.  A lane without a piece
+// reads the first one and writes behind the planes.
 typedef u32x4 u32x4_any __attribute__((aligned(4)));                  // (global memory takes 16 bytes at every multiple of four)
-template <typename T, int NL, bool ROWS>
+template <typename T, int NL, bool ROWS, bool SPLIT>
 struct PairPieces {
     static constexpr int PER = 16 / (int)sizeof(T);
     uint32_t from[NL], second[NL];                                   // second: all ones for a piece of channel 1
@@ -63,7 +72,8 @@ struct PairPieces {
 #pragma unroll
             for (int j = 0; j < (ROWS ? 1 : PER); ++j) {
                 const uint32_t r = fdiv(e + j, p.d_w), col = e + j - r * (uint32_t)g.w;
-                to[i][j] = have ? (int)(s * p.sample + plane * p.plane + (r + g.ph) * row_step + p.lead + col) : p.wave_elems - PER + j;
+                const uint32_t at = p.lead + col, place = SPLIT ? (at & 1) * p.odd + (at >> 1) : at;
+                to[i][j] = have ? (int)(s * p.sample + plane * p.plane + (r + g.ph) * row_step + place) : p.wave_elems - PER - (SPLIT ? p.odd : 0) + j;
             }
         }
     }
@@ -76,11 +86,17 @@ struct PairPieces {
             piece[i] = *reinterpret_cast<const u32x4_any *>(reinterpret_cast<const char *>(xg) + (size_t)o);
         }
     }
-    __device__ __forceinline__ void store(T *__restrict__ image)
+    __device__ __forceinline__ void store(T *__restrict__ image, int odd = 0)
     {
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
-            if constexpr (ROWS) {
+            if constexpr (ROWS && SPLIT && PER == 4) {
+                *reinterpret_cast<u32x2 *>(image + to[i][0]) = u32x2{piece[i].x, piece[i].z};
+                *reinterpret_cast<u32x2 *>(image + to[i][0] + odd) = u32x2{piece[i].y, piece[i].w};
+            } else if constexpr (ROWS && SPLIT) {
+                *reinterpret_cast<u32x2 *>(image + to[i][0]) = u32x2{piece[i].x, piece[i].y};
+                *reinterpret_cast<u32x2 *>(image + to[i][0] + odd) = u32x2{piece[i].z, piece[i].w};
+            } else if constexpr (ROWS) {
                 *reinterpret_cast<u32x4 *>(image + to[i][0]) = piece[i];
             } else {
                 T part[PER];

@@ -4,15 +4,15 @@
 // channels on), no padded copy of x, no barriers.  Element policies of conv_ops.h: float gates with a max pool and its arg-max code, or
 // bitwise gates on 64 samples per word with an OR pool.
 //
-// The planes arrive as 16-byte pieces, requested while the kernel before is evaluated, and go to LDS with shared halos that are
-// zeroed once: a row is `lead` zeros (16 bytes of them, at least the padding) and the w pixels, so that a piece is stored whole
-// where w is a multiple of it; the right halo of a row is the lead of the next, the bottom halo of a plane the top of the next.  A tap is
-// one offset added to the lane's position; the window's other positions are immediate offsets of the same reads, two values each.
+// The planes arrive as 16-byte pieces, requested while the kernel before is evaluated, and go to LDS with halos that are zeroed once: a row
+// is `lead` zeros (16 bytes of them, at least the padding), the w pixels and the zeros behind, even columns and odd ones apart; the
+// bottom halo of a plane is the top of the next.  A tap is two offsets added to the lane's position, of a window's first and
+// second column; the second row is an immediate offset of the same read.
 //
-// Bound by the vector ALU and, next to it, by LDS issue: per kernel and 64 cells 97 vector instructions of float gates and 16
-// two-value reads ([128,4096,8,8] -> 16384: 257 us of 111 us that the vector instructions alone take; the kernel before read its taps
-// from a padded copy, 355 us), 181 of words and 16 ([272,420,8,8] -> 1680: 77 us, before 226).  Which shapes come here:
-// choose_forward in conv_forward.hip.
+// Bound by LDS and the vector ALU together: per kernel and 64 cells 97 vector instructions of float gates and 16 two-value reads
+// ([128,4096,8,8] -> 16384: 240 us, the vector instructions alone 111; the kernel before read its taps from a padded copy, 355 us), 56 + 30 of
+// words ([1024,128,8,8] -> 512: 66 us).  With even and odd columns in one row the lanes of a read were two elements apart and met in
+// the banks two to four times: 265 and 84 us.  Which shapes come here: choose_forward in conv_forward.hip.
 #include <algorithm>
 
 #include "conv_ops.h"
@@ -68,7 +68,7 @@ __global__ __launch_bounds__(256) void pair_prepare_kernel(const P *__restrict__
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             wide |= tp[t].ch != ch0 && tp[t].ch != ch1;
-            row[4 + t] = (tp[t].ch != ch0 ? p.plane : 0) + tp[t].ry * p.rs + tp[t].rx + p.lead - p.pw;
+            row[4 + t] = pair_tap(p.plane, p.rs, p.odd, p.lead - p.pw, tp[t].ch != ch0, tp[t].ry, tp[t].rx);
         }
         row[0] = ch0;
         row[1] = wide ? -1 : ch1;
@@ -109,7 +109,9 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kern
     const int n0 = grp * p.G, g_here = min(p.G, g.n - n0);
     const int hw = g.h * g.w, wp = g.wo >> 1, I = (g.ho >> 1) * wp;
     const int row_step = RS ? RS : p.rs;
-    PairPieces<T, NL, ROWS> in;
+    // the row strides that have an instantiation come with their offset of the odd columns
+    const int odd = RS ? (RS / 2 + 1) & ~1 : p.odd;
+    PairPieces<T, NL, ROWS, true> in;
     in.place(g, p, row_step, g_here, lane);
     // cell of this lane: where its window begins in LDS, where its value goes
     struct Cell {
@@ -124,7 +126,7 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kern
         r.s = fdiv(uu, p.d_cells);
         const uint32_t cell = uu - r.s * (uint32_t)I;
         r.py = fdiv(cell, p.d_wp), r.px = cell - r.py * (uint32_t)wp;
-        r.at = (int)(r.s * p.sample + 2 * r.py * row_step + 2 * r.px);
+        r.at = (int)(r.s * p.sample + 2 * r.py * row_step + r.px);
         r.out = r.s * (uint32_t)p.out_sample + cell * (uint32_t)p.out_cell;
         return r;
     };
@@ -147,7 +149,7 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kern
     for (;;) {
         const int32_t *row = table + c * kPairTable;
         wave_fence();
-        in.store(mine);
+        in.store(mine, odd);
         wave_fence();
         const typename Ops::Params pr = pair_params<Ops>(folded, row, c);
         int off[8];
@@ -161,17 +163,13 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kern
             T r[4];
             if (!wide) {
                 const T *at = mine + cell.at;
-                T v[4][8];
-#pragma unroll
-                for (int t = 0; t < 8; ++t) {
-                    const T *q = at + off[t];
-                    v[0][t] = q[0];
-                    v[1][t] = q[1];
-                    v[2][t] = q[row_step];
-                    v[3][t] = q[row_step + 1];
-                }
-#pragma unroll
-                for (int k = 0; k < 4; ++k) r[k] = Ops::root(pr, v[k]);
+                Ops::root4(pr, [&](int t, T (&v)[4]) {
+                    const T *q = at + (off[t] & 0xFFFF), *q1 = at + ((uint32_t)off[t] >> 16);
+                    v[0] = q[0];
+                    v[1] = q1[0];
+                    v[2] = q[row_step];
+                    v[3] = q1[row_step];
+                }, r);
             } else {
                 // taps in more than two channels (caller-made selection): from global memory, a position at a time
                 const Geom &full = *reinterpret_cast<const Geom *>(table + g.c * kPairTable);
@@ -223,14 +221,38 @@ int launch_pair_nl(const Geom &g, const PairPlan &p, const void *x, const void *
 {
     constexpr int PER = 16 / (int)sizeof(typename Ops::Elem);
     if (g.w % PER != 0) return launch_pair<Ops, NL, 0, false>(g, p, x, folded, table, sel, y, argmax, st, name);
-    if (p.rs == 16 + PER) return launch_pair<Ops, NL, 16 + PER, true>(g, p, x, folded, table, sel, y, argmax, st, name);
-    if (p.rs == 8 + PER) return launch_pair<Ops, NL, 8 + PER, true>(g, p, x, folded, table, sel, y, argmax, st, name);
+    constexpr int kWide = PER == 4 ? 28 : 20, kNarrow = PER == 4 ? 18 : 14;    // 3 x 3 kernels on rows of 16 and of 8
+    if (p.rs == kWide) return launch_pair<Ops, NL, kWide, true>(g, p, x, folded, table, sel, y, argmax, st, name);
+    if (p.rs == kNarrow) return launch_pair<Ops, NL, kNarrow, true>(g, p, x, folded, table, sel, y, argmax, st, name);
     return launch_pair<Ops, NL, 0, true>(g, p, x, folded, table, sel, y, argmax, st, name);
 }
 
 }  // namespace
 
-bool clg_plan_pair(const Geom &g, int elem, PairPlan *p)
+// Split rows: a window's two columns are read by instructions of their own, so that the lanes of one (cells of a row) read consecutive
+// elements; with both in one row they were two apart and met in the 64 banks of LDS at least twice.  Row and sample strides put
+// the rows and samples of a wavefront next to each other modulo the banks where their numbers are powers of two (an access of
+// floats takes 64 lanes, of words 32): conflicts of a read 2 -> 1 for floats on 16 x 16 and 8 x 8, 4 and 3 -> 1 for words.
+static bool split_rows(const Geom &g, int elem, PairPlan *p)
+{
+    const int hp = g.ho / 2, wp = g.wo / 2, half = (p->lead + g.w + g.pw + 1) / 2, step = elem == 4 ? 2 : 1, banks = elem == 4 ? 64 : 32;
+    int wp2 = 1, hp2 = 1;
+    while (wp2 < wp) wp2 *= 2;
+    while (hp2 < hp) hp2 *= 2;
+    const bool align = wp2 >= 2 * step;                               // (floats are stored in pairs: even strides)
+    for (p->rs = (2 * half + step - 1) / step * step; ; p->rs += step) {
+        p->odd = (p->rs / 2 + 1) & ~1;
+        if (p->odd >= half && p->odd + half <= p->rs && (!align || p->rs % wp2 == wp2 / 2)) break;
+    }
+    p->plane = (g.h + g.ph) * p->rs;
+    p->sample = 2 * p->plane;
+    const int tile = wp2 * hp2;
+    if (p->G > 1 && tile < banks && tile % step == 0)
+        while (p->sample % (2 * tile) != tile) p->sample += step;
+    return p->plane + p->sample < (1 << 15);                          // (offsets of 16 bits)
+}
+
+bool clg_plan_pair(const Geom &g, int elem, PairPlan *p, bool split)
 {
     const int per = 16 / elem;
     *p = PairPlan{};
@@ -238,17 +260,21 @@ bool clg_plan_pair(const Geom &g, int elem, PairPlan *p)
     const int I = (g.ho / 2) * (g.wo / 2);
     p->lead = per;
     p->pw = g.pw;
-    p->rs = g.w + per;
-    p->plane = (g.h + g.ph) * p->rs;
     p->G = std::max(1, std::min(kWave / I, g.n));
     p->pieces = (uint32_t)(g.h * g.w / per);
     p->loads = (int)clg_ceil_div((int64_t)2 * p->G * p->pieces, kWave);
     if (p->loads > 8 || (elem == 8 && p->loads > 4)) return false;
-    // samples 16 words apart modulo the 64 banks, so that the rows of neighbouring samples do not meet there
-    p->sample = (int)clg_ceil_div(2 * p->plane, per) * per;
-    if (p->G > 1)
-        while (p->sample * (elem / 4) % 64 != 16 || p->sample % per) p->sample += elem == 8 ? 2 : 4;
-    p->wave_elems = (int)(clg_ceil_div((int64_t)p->G * p->sample + g.ph * p->rs + per + g.kw, per) * per + per);   // (the last piece takes what lanes without one write)
+    if (split) {
+        if (!split_rows(g, elem, p)) return false;
+    } else {
+        p->rs = g.w + per;
+        p->plane = (g.h + g.ph) * p->rs;
+        // samples 16 words apart modulo the 64 banks, so that the rows of neighbouring samples do not meet there
+        p->sample = (int)clg_ceil_div(2 * p->plane, per) * per;
+        if (p->G > 1)
+            while (p->sample * (elem / 4) % 64 != 16 || p->sample % per) p->sample += elem == 8 ? 2 : 4;
+    }
+    p->wave_elems = (int)(clg_ceil_div((int64_t)p->G * p->sample + g.ph * p->rs + per + g.kw, per) * per + per + (p->odd + per) / per * per);   // (the end takes what lanes without a piece write)
     if ((int64_t)kPairWaves * p->wave_elems * elem > 64 * 1024) return false;
     p->groups = (int)clg_ceil_div(g.n, p->G);
     // 32-bit offsets inside a group of samples and in the table

@@ -93,7 +93,7 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_backward_w_pair_k
         }
     }
     const uint32_t plane_bytes = (uint32_t)(g.h * g.w) * 4u, o0 = (uint32_t)ch0 * plane_bytes, d = (uint32_t)ch1 * plane_bytes - o0;
-    PairPieces<float, NL, ROWS> in;
+    PairPieces<float, NL, ROWS, false> in;
     in.place(g, p, row_step, p.G, lane);
     const PairCell first = pair_cell(g, p, row_step, lane, cells, I, wp);
     float acc[28];

@@ -649,7 +649,7 @@ struct NetBlock {
     uint8_t *ids;                 // gate ids [c, 7], or
     int32_t *table;               // rows of conv_pair.h
     int end;                      // kernels up to and including the block's
-    int plane, rs, shift;         // of the table's offsets
+    int plane, rs, odd, shift;    // of the table's offsets
     Geom geom;
 };
 struct NetGates {
@@ -676,7 +676,7 @@ __device__ __forceinline__ void net_kernel(const NetBlock &b, int64_t c, int lan
     const int ch1 = __shfl(tp.ch, half + (differ ? __builtin_ctz(differ) : 0), kWave);
     const bool wide = ((uint32_t)(__ballot(tp.ch != ch0 && tp.ch != ch1) >> half) & 0xFFu) != 0;
     int32_t *row = b.table + c * kPairTable;
-    if (t < 8) row[4 + t] = (tp.ch != ch0 ? b.plane : 0) + tp.ry * b.rs + tp.rx + b.shift;
+    if (t < 8) row[4 + t] = pair_tap(b.plane, b.rs, b.odd, b.shift, tp.ch != ch0, tp.ry, tp.rx);
     if (t == 0) {
         row[0] = ch0;
         row[1] = wide ? -1 : ch1;
@@ -1042,6 +1042,7 @@ extern "C" int clg_net_packed(const clg_packed_block *blocks, int n_blocks, cons
             nb.table = reinterpret_cast<int32_t *>(base + l.gates_off[b]);
             nb.plane = plan[b].plane;
             nb.rs = plan[b].rs;
+            nb.odd = plan[b].odd;
             nb.shift = plan[b].lead - plan[b].pw;
         } else {
             nb.ids = base + l.gates_off[b];
