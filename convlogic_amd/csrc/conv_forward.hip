@@ -610,17 +610,20 @@ int choose_forward(const Geom &g, int elem, int params_per_kernel, bool have_scr
     if (have_scratch && (params_per_kernel == 1) == (elem == 8) && clg_plan_pair(g, elem, pair)) {
         // Two planes per wavefront, against what the shape takes otherwise (us with the launch that makes the tables).  Float gates: where a
         // sample's channels do not fit LDS it is better at every batch ([54,1204,8,8] -> 4816 50.8 -> 37, [176,380,8,8] -> 1520
-        // 82.8 -> 35, [18,46,32,32] -> 571 28.7 -> 27).  Where they fit, the tiled kernels stage every channel for every tile of
+        // 82.8 -> 35, [18,46,32,32] -> 571 28.7 -> 23).  Where they fit, the tiled kernels stage every channel for every tile of
         // kernels and this one only what it reads: from 16 channels (24 where the cells of a sample are more than a wavefront) and
         // 2^17 wavefronts x channels on ([256,128,8,8] -> 512 27.1 -> 20.7, [100,32,12,12] -> 96 20.3 -> 11.8, [64,144,6,6] -> 432
-        // 19.0 -> 12.8; [64,16,16,16] -> 64 9.5 -> 10.5 and [256,16,28,28] -> 64 28.5 -> 35 stay).  Words: from 2^18 wavefronts x
+        // 19.0 -> 12.8; [64,16,16,16] -> 64 9.5 -> 10.5 and [256,16,28,28] -> 64 28.5 -> 35 stay; [64,24,32,32] -> 128 28 -> 20).  Words: from 2^18 wavefronts x
         // channels on, where the second launch is paid for ([272,105,16,16] -> 420 187 -> 64, [1024,32,16,16] -> 128 73 -> 65,
         // [8,105,16,16] -> 420 15.2 -> 13; 4 groups of them 12.2 -> 12.9).  table_ready: the table comes from a launch that is made anyway (a
         // whole network): at any batch ([4,128,8,8] -> 512 11.3 -> 4.5, [4,32,16,16] -> 128 6.4 -> 4.5).
         const int I = (g.ho / 2) * (g.wo / 2);
         const bool fits = tiled && !tp->subset;
-        const int64_t work = (int64_t)pair->groups * g.c * clg_ceil_div((int64_t)pair->G * I, kWave) * g.cin;
-        bool use = elem == 8 ? work >= (1 << 18) || table_ready : !fits || (work > (1 << 17) && g.cin >= (I > kWave ? 24 : 16));
+        // words in bands that leave lanes idle (28 x 28 images: 196 cells in 4 times 64) or restage a few channels over and over, from a thousand
+        // wavefronts on: [512,16,28,28] -> 64 71 -> 83, [500,1,28,28] -> 32 29 -> 39, but [1024,9,32,32] -> 32 88 -> 76
+        const bool bands_lose = pair->bands && (8 * I < 7 * kWave * pair->bands || g.cin < 4) && (int64_t)g.n * g.c > 1024;
+        const int64_t work = (int64_t)pair->groups * g.c * (pair->bands ? 1 : clg_ceil_div((int64_t)pair->G * I, kWave)) * g.cin;
+        bool use = elem == 8 ? (work >= (1 << 18) || table_ready) && !(bands_lose && fits) : !fits || (work > (1 << 17) && g.cin >= (I > kWave ? 24 : 16));
         use = use && !clg_knob(K_FWD_DIRECT) && !clg_knob(K_FWD_SUBSET) && !clg_knob(K_FWD_KPL);   // (a path that is asked for)
         if (const char *e = clg_knob(K_FWD_PAIR)) use = atoi(e) != 0;
         if (use) {

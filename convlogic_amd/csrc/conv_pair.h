@@ -4,13 +4,14 @@
 #include "conv_tile.h"
 
 struct PairPlan {
-    int G, groups;            // samples per wavefront, groups of them
+    int G, groups;            // samples per wavefront, groups of them; or
+    int bands, band_rows;     // a sample of more than 64 cells in bands of so many rows of them (bands > 0; a group is a band)
     int ct, tiles;            // kernels per workgroup, tiles of them
     int lead, pw, rs, plane, sample, wave_elems;   // LDS, in elements: zeros in front of a row, row / plane / sample stride, all of a wavefront
     int odd;                  // from a row's even columns to its odd ones where they are kept apart, else 0
     int loads;                // 16-byte pieces per lane
-    uint32_t pieces;          // per plane
-    FastDiv d_tiles, d_pieces, d_w, d_wp, d_cells;
+    uint32_t pieces;          // per plane, or per band of one
+    FastDiv d_tiles, d_pieces, d_w, d_wp, d_cells, d_bands;
     size_t folded_bytes, total_bytes;   // scratch: folded coefficients | table and geometry
     int out_sample, out_cell;           // the output: elements between samples, between cells of a kernel (whose cells follow those of the kernel before)
 };
@@ -75,6 +76,21 @@ struct PairPieces {
                 const uint32_t at = p.lead + col, place = SPLIT ? (at & 1) * p.odd + (at >> 1) : at;
                 to[i][j] = have ? (int)(s * p.sample + plane * p.plane + (r + g.ph) * row_step + place) : p.wave_elems - PER - (SPLIT ? p.odd : 0) + j;
             }
+        }
+    }
+    // a band of one sample: its rows begin at row y0 of the image, those outside it stay the zeros they are
+    __device__ __forceinline__ void place_band(const Geom &g, const PairPlan &p, int row_step, int y0, int lane)
+    {
+        static_assert(ROWS && SPLIT, "whole pieces per row");
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const uint32_t v = lane + i * kWave, plane = fdiv(v, p.d_pieces), e = (v - plane * p.pieces) * PER, r = fdiv(e, p.d_w);
+            const uint32_t col = e - r * (uint32_t)g.w, at = p.lead + col;
+            const int y = y0 + (int)r;
+            const bool have = plane < 2 && y >= 0 && y < g.h;
+            second[i] = have && plane ? ~0u : 0u;
+            from[i] = have ? (uint32_t)(y * g.w + (int)col) * (uint32_t)sizeof(T) : 0;
+            to[i][0] = have ? (int)(plane * p.plane + r * row_step + (at >> 1)) : p.wave_elems - PER - p.odd;
         }
     }
     // o0: bytes from the group's first sample to its channel 0, d: from there to channel 1 (modulo 2^32)

@@ -6,7 +6,8 @@
 //
 // The planes arrive as 16-byte pieces, requested while the kernel before is evaluated, and go to LDS with halos that are zeroed once: a row
 // is `lead` zeros (16 bytes of them, at least the padding), the w pixels and the zeros behind, even columns and odd ones apart; the
-// bottom halo of a plane is the top of the next.  A tap is two offsets added to the lane's position, of a window's first and
+// bottom halo of a plane is the top of the next.  An image of more than 64 cells is staged in bands of whole rows of cells with halo rows of
+// their own.  A tap is two offsets added to the lane's position, of a window's first and
 // second column; the second row is an immediate offset of the same read.
 //
 // Bound by LDS and the vector ALU together: per kernel and 64 cells 97 vector instructions of float gates and 16 two-value reads
@@ -89,7 +90,7 @@ __device__ __forceinline__ typename Ops::Params pair_params(const void *__restri
 }
 
 // NL: 16-byte pieces per lane.  RS: the row stride where it is known at compile time (else 0).  ROWS: no piece crosses a row.  ONE: the
-// cells of a group of samples are at most 64.  What a lane needs per kernel is worked out once, and the geometry's fields are
+// cells of a group of samples are at most 64; else, with ROWS, a group is a band of a sample, and without, 64 cells after the other.  What a lane needs per kernel is worked out once, and the geometry's fields are
 // read again where a kernel's taps are in more than two channels: with them in scalar registers all along the loop spilled some.
 template <typename Ops, int NL, int RS, bool ROWS, bool ONE>
 __global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kernel(const typename Ops::Elem *__restrict__ x, const void *__restrict__ folded,
@@ -106,13 +107,16 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kern
     // the kernel tiles of a group of samples follow each other on one XCD: its L2 holds their planes
     const unsigned logical = xcd_contiguous_block(blockIdx.x, gridDim.x);
     const int grp = uniform((int)fdiv(logical, p.d_tiles)), tile = uniform((int)logical) - grp * p.tiles;
-    const int n0 = grp * p.G, g_here = min(p.G, g.n - n0);
+    constexpr bool BAND = ROWS && !ONE;
+    const int n0 = BAND ? uniform((int)fdiv(grp, p.d_bands)) : grp * p.G, g_here = BAND ? 1 : min(p.G, g.n - n0);
+    const int r0 = BAND ? (grp - n0 * p.bands) * p.band_rows : 0;     // a band's first row of cells
     const int hw = g.h * g.w, wp = g.wo >> 1, I = (g.ho >> 1) * wp;
     const int row_step = RS ? RS : p.rs;
     // the row strides that have an instantiation come with their offset of the odd columns
     const int odd = RS ? (RS / 2 + 1) & ~1 : p.odd;
     PairPieces<T, NL, ROWS, true> in;
-    in.place(g, p, row_step, g_here, lane);
+    if constexpr (BAND) in.place_band(g, p, row_step, 2 * r0 - g.ph, lane);
+    else in.place(g, p, row_step, g_here, lane);
     // cell of this lane: where its window begins in LDS, where its value goes
     struct Cell {
         int at;
@@ -121,12 +125,16 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kern
     };
     auto cell_of = [&](uint32_t u) {
         Cell r;
-        r.live = (int)u < g_here * I;
+        r.live = (int)u < (BAND ? min(p.band_rows, (g.ho >> 1) - r0) * wp : g_here * I);
         const uint32_t uu = r.live ? u : 0;
-        r.s = fdiv(uu, p.d_cells);
-        const uint32_t cell = uu - r.s * (uint32_t)I;
+        r.s = BAND ? 0 : fdiv(uu, p.d_cells);
+        uint32_t cell = uu - r.s * (uint32_t)I;
         r.py = fdiv(cell, p.d_wp), r.px = cell - r.py * (uint32_t)wp;
         r.at = (int)(r.s * p.sample + 2 * r.py * row_step + r.px);
+        if (BAND) {
+            r.py += r0;
+            cell += r0 * wp;
+        }
         r.out = r.s * (uint32_t)p.out_sample + cell * (uint32_t)p.out_cell;
         return r;
     };
@@ -134,7 +142,7 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kern
     T *yg = y + (int64_t)n0 * p.out_sample;
     uint8_t *ag = argmax + (int64_t)n0 * p.out_sample;
     const int kernel_cells = I * p.out_cell;
-    const int cells = g_here * I, blocks = ONE ? 1 : (cells + kWave - 1) / kWave;
+    const int blocks = ONE || BAND ? 1 : (g_here * I + kWave - 1) / kWave;
     const uint32_t plane_bytes = (uint32_t)hw * (uint32_t)sizeof(T);
     auto fetch = [&](int c) {
         const int32_t *row = table + c * kPairTable;
@@ -159,7 +167,7 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kern
         const int cn = c + kPairWaves;
         if (cn < c_end) fetch(cn);                                    // in flight while this kernel is evaluated
         for (int b = 0; b < blocks; ++b) {
-            const Cell cell = ONE ? first : cell_of(b * kWave + lane);
+            const Cell cell = ONE || BAND ? first : cell_of(b * kWave + lane);
             T r[4];
             if (!wide) {
                 const T *at = mine + cell.at;
@@ -222,6 +230,7 @@ int launch_pair_nl(const Geom &g, const PairPlan &p, const void *x, const void *
     constexpr int PER = 16 / (int)sizeof(typename Ops::Elem);
     if (g.w % PER != 0) return launch_pair<Ops, NL, 0, false>(g, p, x, folded, table, sel, y, argmax, st, name);
     constexpr int kWide = PER == 4 ? 28 : 20, kNarrow = PER == 4 ? 18 : 14;    // 3 x 3 kernels on rows of 16 and of 8
+    if (p.rs == 40 && p.bands) return launch_pair_one<Ops, NL, 40, true, false>(g, p, x, folded, table, sel, y, argmax, st, name);   // of 28 and 32
     if (p.rs == kWide) return launch_pair<Ops, NL, kWide, true>(g, p, x, folded, table, sel, y, argmax, st, name);
     if (p.rs == kNarrow) return launch_pair<Ops, NL, kNarrow, true>(g, p, x, folded, table, sel, y, argmax, st, name);
     return launch_pair<Ops, NL, 0, true>(g, p, x, folded, table, sel, y, argmax, st, name);
@@ -244,7 +253,7 @@ static bool split_rows(const Geom &g, int elem, PairPlan *p)
         p->odd = (p->rs / 2 + 1) & ~1;
         if (p->odd >= half && p->odd + half <= p->rs && (!align || p->rs % wp2 == wp2 / 2)) break;
     }
-    p->plane = (g.h + g.ph) * p->rs;
+    p->plane = (p->bands ? 2 * p->band_rows + g.kh - 1 : g.h + g.ph) * p->rs;   // (a band has its halo rows itself)
     p->sample = 2 * p->plane;
     const int tile = wp2 * hp2;
     if (p->G > 1 && tile < banks && tile % step == 0)
@@ -262,8 +271,14 @@ bool clg_plan_pair(const Geom &g, int elem, PairPlan *p, bool split)
     p->pw = g.pw;
     p->G = std::max(1, std::min(kWave / I, g.n));
     p->pieces = (uint32_t)(g.h * g.w / per);
+    if (split && I > kWave && g.wo / 2 <= kWave && g.w % per == 0) {
+        const int rows = kWave / (g.wo / 2), hp = g.ho / 2;
+        p->bands = (int)clg_ceil_div(hp, rows);
+        p->band_rows = (int)clg_ceil_div(hp, p->bands);
+        p->pieces = (uint32_t)((2 * p->band_rows + g.kh - 1) * (g.w / per));
+    }
     p->loads = (int)clg_ceil_div((int64_t)2 * p->G * p->pieces, kWave);
-    if (p->loads > 8 || (elem == 8 && p->loads > 4)) return false;
+    if (p->loads > 8 || (elem == 8 && p->loads > 6)) return false;
     if (split) {
         if (!split_rows(g, elem, p)) return false;
     } else {
@@ -276,7 +291,8 @@ bool clg_plan_pair(const Geom &g, int elem, PairPlan *p, bool split)
     }
     p->wave_elems = (int)(clg_ceil_div((int64_t)p->G * p->sample + g.ph * p->rs + per + g.kw, per) * per + per + (p->odd + per) / per * per);   // (the end takes what lanes without a piece write)
     if ((int64_t)kPairWaves * p->wave_elems * elem > 64 * 1024) return false;
-    p->groups = (int)clg_ceil_div(g.n, p->G);
+    if (p->bands && (int64_t)g.n * p->bands >= (1ll << 31)) return false;
+    p->groups = p->bands ? g.n * p->bands : (int)clg_ceil_div(g.n, p->G);
     // 32-bit offsets inside a group of samples and in the table
     if ((int64_t)p->G * g.cin * g.h * g.w * elem >= (1ll << 32) || (int64_t)p->G * g.c * I * elem >= (1ll << 32) || g.c > 65535) return false;
     p->out_sample = g.y_fm ? 1 : g.c * I;
@@ -284,12 +300,13 @@ bool clg_plan_pair(const Geom &g, int elem, PairPlan *p, bool split)
     if (g.y_fm && (int64_t)I * g.n * elem >= (1ll << 31)) return false;
     // kernels per workgroup: many, for the planes of a sample to be found in L2, as long as there are 8192 wavefronts
     int64_t ct = 64;
-    while (ct > 4 * kPairWaves && p->groups * clg_ceil_div(g.c, ct) < 2048) ct /= 2;
-    while (ct > kPairWaves && p->groups * clg_ceil_div(g.c, ct) < 512) ct /= 2;
+    while (ct > 4 * kPairWaves && (int64_t)p->groups * clg_ceil_div(g.c, ct) < 2048) ct /= 2;
+    while (ct > kPairWaves && (int64_t)p->groups * clg_ceil_div(g.c, ct) < 512) ct /= 2;
     p->ct = (int)ct;
     p->tiles = (int)clg_ceil_div(g.c, ct);
     if ((int64_t)p->tiles * p->groups >= (1ll << 31)) return false;
     p->d_tiles = make_fastdiv((uint32_t)p->tiles);
+    p->d_bands = make_fastdiv((uint32_t)std::max(1, p->bands));
     p->d_pieces = make_fastdiv(p->pieces);
     p->d_w = make_fastdiv((uint32_t)g.w);
     p->d_wp = make_fastdiv((uint32_t)(g.wo / 2));
@@ -330,5 +347,6 @@ int clg_forward_pair_packed(const Geom &g, const PairPlan &p, const uint64_t *x,
                        no_pad_job<float>(), (int)prep, 0, (float *)nullptr);
     CLG_CHECK_LAUNCH(name);
     if (p.loads <= 2) return launch_pair_nl<BitOpsAnf, 2>(g, p, x, nullptr, table, sel, y, nullptr, st, name);
-    return launch_pair_nl<BitOpsAnf, 4>(g, p, x, nullptr, table, sel, y, nullptr, st, name);
+    if (p.loads <= 4) return launch_pair_nl<BitOpsAnf, 4>(g, p, x, nullptr, table, sel, y, nullptr, st, name);
+    return launch_pair_nl<BitOpsAnf, 6>(g, p, x, nullptr, table, sel, y, nullptr, st, name);
 }
