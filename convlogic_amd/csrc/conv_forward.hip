@@ -605,7 +605,7 @@ int choose_forward(const Geom &g, int elem, int params_per_kernel, bool have_scr
 {
     bool lane_sample = have_scratch && params_per_kernel > 1 && clg_convblock_is_4x4(g);
     if (const char *e = clg_knob(K_FWD_4X4)) lane_sample = lane_sample && atoi(e) != 0;
-    if (lane_sample) return 4;
+    if (lane_sample && elem != 4) return 4;
     const bool tiled = plan_forward(g, elem, params_per_kernel, tp);
     if (have_scratch && (params_per_kernel == 1) == (elem == 8) && clg_plan_pair(g, elem, pair)) {
         // Two planes per wavefront, against what the shape takes otherwise (us with the launch that makes the tables).  Float gates: where a
@@ -623,7 +623,10 @@ int choose_forward(const Geom &g, int elem, int params_per_kernel, bool have_scr
         // wavefronts on: [512,16,28,28] -> 64 71 -> 83, [500,1,28,28] -> 32 29 -> 39, but [1024,9,32,32] -> 32 88 -> 76
         const bool bands_lose = pair->bands && (8 * I < 7 * kWave * pair->bands || g.cin < 4) && (int64_t)g.n * g.c > 1024;
         const int64_t work = (int64_t)pair->groups * g.c * (pair->bands ? 1 : clg_ceil_div((int64_t)pair->G * I, kWave)) * g.cin;
-        bool use = elem == 8 ? (work >= (1 << 18) || table_ready) && !(bands_lose && fits) : !fits || (work > (1 << 17) && g.cin >= (I > kWave ? 24 : 16));
+        // 4 x 4 images, against a sample per lane: [128,16384,4,4] -> 32768 191 -> 164, but [256,512,4,4] -> 1024 15.0 either way and
+        // [64,512,4,4] -> 1024 8.8 -> 9.8; words are better here at every size
+        // ([1024,512,4,4] -> 1024 57 -> 44, [141,1600,4,4] -> 3200 83 and 20 -> 26).
+        bool use = lane_sample ? (int64_t)pair->groups * g.c > (1 << 16) : elem == 8 ? (work >= (1 << 18) || table_ready) && !(bands_lose && fits) : !fits || (work > (1 << 17) && g.cin >= (I > kWave ? 24 : 16));
         use = use && !clg_knob(K_FWD_DIRECT) && !clg_knob(K_FWD_SUBSET) && !clg_knob(K_FWD_KPL);   // (a path that is asked for)
         if (const char *e = clg_knob(K_FWD_PAIR)) use = atoi(e) != 0;
         if (use) {
@@ -631,6 +634,7 @@ int choose_forward(const Geom &g, int elem, int params_per_kernel, bool have_scr
             return 6;
         }
     }
+    if (lane_sample) return 4;
     {
         // one kernel per lane: 40.4 -> 21.2 us (+ 3.9 us for the launch that folds the coefficients) at [256,128,8,8] -> 512
         const int I = (g.ho / 2) * (g.wo / 2);
@@ -877,7 +881,8 @@ static int forward_ex_impl(const char *name, int dtype, const clg_conv_geom *gg,
     DirectPlan dp;
     const int elem = dtype == CLG_F64 ? 8 : 4;
     PairPlan pp;
-    const int path = fm ? 4 : choose_forward(g, elem, 28, scratch != nullptr, &tp, &dp, &pp);
+    g.y_fm = fm ? 1 : 0;
+    const int path = choose_forward(g, elem, 28, scratch != nullptr, &tp, &dp, &pp);   // (4 or 6 where fm)
     hipStream_t st = clg_stream(stream);
     // the folded coefficients [c_out, 7, 4] follow the probabilities in probs_out
     void *folded_out = want_folded ? reinterpret_cast<unsigned char *>(probs_out) + (size_t)g.c * 112 * elem : nullptr;
@@ -902,7 +907,6 @@ static int forward_ex_impl(const char *name, int dtype, const clg_conv_geom *gg,
                                     g.cin * tp.chs + g.ph * tp.rs + g.pw, st, name, want_folded && !given ? (float *)folded_out : nullptr);
     }
     if (path == 4 || path == 5) {
-        g.y_fm = fm ? 1 : 0;
         void *fold_to = want_folded ? folded_out : scratch;             // the kernels read them from wherever they are
         const dim3 pgrid((unsigned)clg_ceil_div((int64_t)g.c * 7, 256));
         if (given) {
@@ -1110,6 +1114,14 @@ extern "C" int clg_convblock_eval_packed_logits(int dtype, const clg_conv_geom *
     CLG_REQUIRE(x != y, "%s: x and y must not overlap", name);
     uint8_t *gates = reinterpret_cast<uint8_t *>(scratch);
     if (int e = clg_gate_argmax(dtype, logits, gates, (int64_t)g.c * 7, stream)) return e;
-    if (feature_major) return clg_convblock_eval_packed_fm(gg, x, gates, selection, y, stream);
+    PairPlan pp;
+    if (feature_major) {
+        TilePlan tp;
+        DirectPlan dp;
+        g.y_fm = 1;
+        if (clg_convblock_eval_packed_fm_supported(gg) && choose_forward(g, 8, 1, true, &tp, &dp, &pp) == 6)
+            return clg_forward_pair_packed(g, pp, x, gates, selection, y, gates + packed_gates_bytes(g), clg_stream(stream), name);
+        return clg_convblock_eval_packed_fm(gg, x, gates, selection, y, stream);
+    }
     return clg_convblock_eval_packed_ws(gg, x, gates, selection, y, gates + packed_gates_bytes(g), stream);
 }

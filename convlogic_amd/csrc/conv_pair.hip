@@ -120,7 +120,7 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kern
     // cell of this lane: where its window begins in LDS, where its value goes
     struct Cell {
         int at;
-        uint32_t out, s, py, px;
+        uint32_t out, code, s, py, px;
         bool live;
     };
     auto cell_of = [&](uint32_t u) {
@@ -136,11 +136,12 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kern
             cell += r0 * wp;
         }
         r.out = r.s * (uint32_t)p.out_sample + cell * (uint32_t)p.out_cell;
+        r.code = r.s * (uint32_t)(g.c * I) + cell;                    // (arg-max codes stay sample by sample)
         return r;
     };
     const T *xg = x + (int64_t)n0 * g.cin * hw;
     T *yg = y + (int64_t)n0 * p.out_sample;
-    uint8_t *ag = argmax + (int64_t)n0 * p.out_sample;
+    uint8_t *ag = argmax + (int64_t)n0 * g.c * I;
     const int kernel_cells = I * p.out_cell;
     const int blocks = ONE || BAND ? 1 : (g_here * I + kWave - 1) / kWave;
     const uint32_t plane_bytes = (uint32_t)hw * (uint32_t)sizeof(T);
@@ -196,7 +197,7 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kern
             const T best = Ops::pool4(pr, r, code);
             if (cell.live) {
                 reinterpret_cast<T *>(reinterpret_cast<char *>(yg + (int64_t)c * kernel_cells) + (size_t)(cell.out * (uint32_t)sizeof(T)))[0] = best;
-                if constexpr (!Ops::kOrPool) (ag + (int64_t)c * kernel_cells)[cell.out] = (uint8_t)code;
+                if constexpr (!Ops::kOrPool) (ag + (int64_t)c * I)[cell.code] = (uint8_t)code;
             }
         }
         if (cn >= c_end) return;
@@ -230,6 +231,7 @@ int launch_pair_nl(const Geom &g, const PairPlan &p, const void *x, const void *
     constexpr int PER = 16 / (int)sizeof(typename Ops::Elem);
     if (g.w % PER != 0) return launch_pair<Ops, NL, 0, false>(g, p, x, folded, table, sel, y, argmax, st, name);
     constexpr int kWide = PER == 4 ? 28 : 20, kNarrow = PER == 4 ? 18 : 14;    // 3 x 3 kernels on rows of 16 and of 8
+    if (PER == 2 && p.rs == 9 && !p.bands) return launch_pair_one<Ops, NL, PER == 2 ? 9 : 0, true, true>(g, p, x, folded, table, sel, y, argmax, st, name);   // of 4
     if (p.rs == 40 && p.bands) return launch_pair_one<Ops, NL, 40, true, false>(g, p, x, folded, table, sel, y, argmax, st, name);   // of 28 and 32
     if (p.rs == kWide) return launch_pair<Ops, NL, kWide, true>(g, p, x, folded, table, sel, y, argmax, st, name);
     if (p.rs == kNarrow) return launch_pair<Ops, NL, kNarrow, true>(g, p, x, folded, table, sel, y, argmax, st, name);

@@ -956,7 +956,7 @@ int net_pair(const char *name, const clg_packed_block *blocks, int n_blocks, int
 {
     if (int e = clg_convblock_check(&blocks[b].geom, g, CLG_F64, name)) return e;
     g->y_fm = b == n_blocks - 1 ? 1 : 0;
-    *pair = !(g->y_fm && clg_convblock_eval_packed_fm_supported(&blocks[b].geom)) && clg_packed_pair(*g, p);
+    *pair = clg_packed_pair(*g, p);
     if (!*pair) g->y_fm = 0;
     return CLG_OK;
 }

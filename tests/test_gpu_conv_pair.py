@@ -189,3 +189,19 @@ def test_networks_with_tables_from_the_launch_of_the_codes(topology, k, channels
             seen.append((model(packed), packed.t))
     for counts, words in seen[1:]:
         assert torch.equal(counts, seen[0][0]) and torch.equal(words, seen[0][1])
+
+
+@pytest.mark.parametrize("feature_major", [False, True])
+@pytest.mark.parametrize("n,cin,c,wide", [(32, 6, 9, False), (33, 20, 70, True), (50, 3, 130, False)])
+def test_images_of_4x4_against_the_kernels_with_a_sample_per_lane(n, cin, c, wide, feature_major, monkeypatch):
+    torch.manual_seed(n)
+    layer = C.ConvLogicLayer(cin, c, complete=True, implementation="cuda").to(DEV)
+    sel, logits = _selection(layer, wide), torch.randn_like(layer.weights)
+    x, words = torch.randn(n, cin, 4, 4, device=DEV), torch.randint(-2**62, 2**62, (n, cin, 4, 4), device=DEV)
+    run = lambda: (*H.full_convlogic_forward_logits(x, logits, sel, 1, 1, 1, 1, 3, 3, feature_major=feature_major, want_folded=True),
+                   H.full_convlogic_eval_packed_logits(words, logits, sel, (1, 1, 1, 1, 3, 3), feature_major=feature_major))
+    set_knobs(monkeypatch, CLG_FWD_PAIR="0")
+    want = run()
+    set_knobs(monkeypatch, CLG_FWD_PAIR="1")
+    for a, b in zip(want, run()):
+        assert a.shape == b.shape and torch.equal(a, b)
