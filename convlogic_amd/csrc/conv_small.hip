@@ -9,6 +9,7 @@
 // once and stays zero), a plane arrives as four 16-byte loads per lane that are requested one kernel ahead, and the
 // 16 positions x 8 taps are LDS reads at (tap address + immediate position offset).  No barriers, no bounds checks.
 // A kernel whose taps name more than two channels (possible with a caller-made selection) reads global memory.
+// (Large float blocks, and words wherever the caller has scratch for a tap table, run forward in conv_pair.hip: choose_forward.)
 #include <stdlib.h>
 
 #include "conv_ops.h"
