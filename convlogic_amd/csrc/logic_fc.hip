@@ -83,6 +83,24 @@ __device__ __forceinline__ void store_vec(S *p, const Pack<typename ComputeOf<S>
         *reinterpret_cast<V *>(p) = __builtin_bit_cast(V, v);
     }
 }
+
+// Rows of any number of samples (at least VEC): a wide access to global memory needs 4-byte alignment only, and the last lane of a row
+// that VEC does not divide steps back to the last VEC samples, which it shares with its neighbour (the same values, twice).
+typedef float f32x4_row __attribute__((ext_vector_type(4), aligned(4)));
+template <typename S, int VEC>
+__device__ __forceinline__ Pack<typename ComputeOf<S>::type, VEC> load_row(const S *p)
+{
+    if constexpr (sizeof(S) == 4 && VEC == 4) return __builtin_bit_cast(Pack<S, VEC>, *reinterpret_cast<const f32x4_row *>(p));
+    else return load_vec<S, VEC>(p);
+}
+template <typename T, int VEC>
+__device__ __forceinline__ void store_row(T *p, const Pack<T, VEC> &v)
+{
+    if constexpr (sizeof(T) == 4 && VEC == 4) *reinterpret_cast<f32x4_row *>(p) = __builtin_bit_cast(f32x4_row, v);
+    else store_vec<T, VEC>(p, v);
+}
+template <int VEC>
+__device__ __forceinline__ int64_t row_at(int64_t s, int64_t batch) { return s + VEC <= batch ? s : batch - VEC; }
 template <typename S>
 __device__ __forceinline__ typename ComputeOf<S>::type load_one(const S *p)
 {
@@ -386,11 +404,12 @@ __global__ __launch_bounds__(kBlock) void fc_forward_folded_kernel(const T *__re
         const T *xb = x + clamp_index(b[j], in_dim) * batch;
         T *yj = y + j * batch;
         for (int64_t s = (int64_t)l * VEC; s < batch; s += pass) {
-            const Pack<T, VEC> va = load_vec<T, VEC>(xa + s), vb = load_vec<T, VEC>(xb + s);
+            const int64_t at = row_at<VEC>(s, batch);
+            const Pack<T, VEC> va = load_row<T, VEC>(xa + at), vb = load_row<T, VEC>(xb + at);
             Pack<T, VEC> r;
 #pragma unroll
             for (int k = 0; k < VEC; ++k) r.v[k] = gate(c, va.v[k], vb.v[k]);
-            store_vec<T, VEC>(yj + s, r);
+            store_row<T, VEC>(yj + at, r);
         }
     }
 }
@@ -443,11 +462,12 @@ __global__ __launch_bounds__(kBlock) void fc_forward_logits_kernel(const T *__re
         const T *xb = x + clamp_index(b[j], in_dim) * batch;
         T *yj = y + j * batch;
         for (int64_t s = (int64_t)l * VEC; s < batch; s += pass) {
-            const Pack<T, VEC> va = load_vec<T, VEC>(xa + s), vb = load_vec<T, VEC>(xb + s);
+            const int64_t at = row_at<VEC>(s, batch);
+            const Pack<T, VEC> va = load_row<T, VEC>(xa + at), vb = load_row<T, VEC>(xb + at);
             Pack<T, VEC> r;
 #pragma unroll
             for (int k = 0; k < VEC; ++k) r.v[k] = gate(c, va.v[k], vb.v[k]);
-            store_vec<T, VEC>(yj + s, r);
+            store_row<T, VEC>(yj + at, r);
         }
     }
 }
@@ -534,8 +554,8 @@ __device__ __forceinline__ Pack<T, VEC> fc_walk_consumers(const T *__restrict__ 
         Pack<T, VEC> vo[4], vg[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            vo[u] = load_vec<T, VEC>(x + (int64_t)cur_m.io[u] * batch + s_at);
-            vg[u] = load_vec<T, VEC>(gy + (int64_t)(cur_m.j[u] < 0 ? 0 : cur_m.j[u]) * batch + s_at);
+            vo[u] = load_row<T, VEC>(x + (int64_t)cur_m.io[u] * batch + s_at);
+            vg[u] = load_row<T, VEC>(gy + (int64_t)(cur_m.j[u] < 0 ? 0 : cur_m.j[u]) * batch + s_at);
         }
         if (kAlwaysAhead || cur + 4 < end) {
             wiring(j_next, cur_m.j[3], next_m);
@@ -598,11 +618,12 @@ __global__ __launch_bounds__(kBlock) void fc_backward_x_folded_kernel(
         const int64_t i = (it / batch_chunks) * rows + sub;
         const int64_t s = (((it % batch_chunks) << lpr_log2) + l) * VEC;
         if (i >= in_dim || s >= batch) continue;
+        const int64_t at = row_at<VEC>(s, batch);
         const int64_t beg = clamp_index(csr_start[i], 2 * (int64_t)out_dim + 1), end = clamp_index(csr_start[i + 1], 2 * (int64_t)out_dim + 1);
         const Pack<T, VEC> none{};
         const Pack<T, VEC> acc = fc_walk_consumers<T, VEC, 0>(x, a, b, folded, gy, csr_list, (T *)nullptr, (const T *)nullptr, in_dim, out_dim,
-                                                              batch, i, beg, end, s, true, none, lane);
-        store_vec<T, VEC>(gx + i * batch + s, acc);
+                                                              batch, i, beg, end, at, true, none, lane);
+        store_row<T, VEC>(gx + i * batch + at, acc);
     }
 }
 
@@ -876,6 +897,12 @@ template <typename T>
 constexpr int vec_width() { return 16 / sizeof(T); }
 
 // log2 of the lanes one row of `batch` samples takes at `vec` samples per lane: 16, 32 or 64 lanes
+// Four samples per lane for rows of any length from 17 samples on (up to 16, one per lane is one pass as well: 4.0 us against 5.2 for
+// the input gradient of 300 features, batch 5).  Input gradient, one -> four samples per lane: 8000 -> 8000 neurons 27.2 -> 12.0 us at batch 255,
+// 33.0 -> 19.0 at 266; 30000 -> 30000 at 599 208 -> 88; forward 18.8 -> 12.7 at 30000 -> 45000, batch 102.
+// (Sums over the batch would have to leave the shared samples out: the weight gradient lost 4.6 -> 5.9 us at batch 256 by the test for it.)
+bool wide_rows(int64_t batch) { return batch % 4 == 0 || batch > 16; }
+
 int lanes_per_row_log2(int64_t batch, int vec)
 {
     const int64_t lanes = clg_ceil_div(batch, (int64_t)vec);
@@ -1111,7 +1138,7 @@ extern "C" int clg_fc_forward_folded(int dtype, const void *x, const int64_t *a,
                            block, 0, st, (const T *)x, a, b, (const T *)folded, (T *)y, (int)out_dim, batch, lg, (int)in_dim);       \
     } while (0)
     if (dtype == CLG_F32) {
-        if (batch % 4 == 0) CLG_LAUNCH_FF(float, 4);
+        if (wide_rows(batch)) CLG_LAUNCH_FF(float, 4);
         else CLG_LAUNCH_FF(float, 1);
     } else {
         if (batch % 2 == 0) CLG_LAUNCH_FF(double, 2);
@@ -1153,7 +1180,7 @@ extern "C" int clg_fc_forward_logits(int dtype, const void *x, const int64_t *a,
                            (int)out_dim, batch, lg, (int)in_dim);                                                              \
     } while (0)
     if (dtype == CLG_F32) {
-        if (batch % 4 == 0) CLG_LAUNCH_FL(float, 4);
+        if (wide_rows(batch)) CLG_LAUNCH_FL(float, 4);
         else CLG_LAUNCH_FL(float, 1);
     } else {
         if (batch % 2 == 0) CLG_LAUNCH_FL(double, 2);
@@ -1183,7 +1210,7 @@ extern "C" int clg_fc_backward_x_folded(int dtype, const void *x, const int64_t 
                            chunks, lg, (int)out_dim);                                                                        \
     } while (0)
     if (dtype == CLG_F32) {
-        if (batch % 4 == 0) CLG_LAUNCH_BXF(float, 4);
+        if (wide_rows(batch)) CLG_LAUNCH_BXF(float, 4);
         else CLG_LAUNCH_BXF(float, 1);
     } else {
         if (batch % 2 == 0) CLG_LAUNCH_BXF(double, 2);
