@@ -19,6 +19,8 @@
 #include "conv_ops.h"
 #include "conv_pair.h"
 
+int clg_convblock_check(const clg_conv_geom *gg, Geom *g, int dtype, const char *name);
+
 namespace {
 
 // What a launch needs besides x and the selection, in one launch: table, folded coefficients (float gates; the softmax of logits
@@ -90,8 +92,10 @@ __device__ __forceinline__ typename Ops::Params pair_params(const void *__restri
 }
 
 // NL: 16-byte pieces per lane.  RS: the row stride where it is known at compile time (else 0).  ROWS: no piece crosses a row.  ONE: the
-// cells of a group of samples are at most 64; else, with ROWS, a group is a band of a sample, and without, 64 cells after the other.  What a lane needs per kernel is worked out once, and the geometry's fields are
-// read again where a kernel's taps are in more than two channels: with them in scalar registers all along the loop spilled some.
+// cells of a group of samples are at most 64; else, with ROWS, a group is a band of a sample (the launch checks that the plan has bands
+// then, and only then), and without, 64 cells after the other.  What a lane needs per kernel is worked out once, and the geometry's
+// fields are read again where a kernel's taps are in more than two channels: with them in scalar registers all along the loop spilled
+// some.
 template <typename Ops, int NL, int RS, bool ROWS, bool ONE>
 __global__ __launch_bounds__(kPairWaves *kWave) void convblock_forward_pair_kernel(const typename Ops::Elem *__restrict__ x, const void *__restrict__ folded,
                                                                                  const int32_t *__restrict__ table, const int32_t *__restrict__ sel,
@@ -210,6 +214,7 @@ int launch_pair_one(const Geom &g, const PairPlan &p, const void *x, const void 
                 hipStream_t st, const char *name)
 {
     using T = typename Ops::Elem;
+    CLG_REQUIRE((p.bands > 0) == (ROWS && !ONE), "%s: a plan of %d bands for another kernel", name, p.bands);
     const size_t lds = (size_t)kPairWaves * p.wave_elems * sizeof(T);
     if (int e = allow_lds(convblock_forward_pair_kernel<Ops, NL, RS, ROWS, ONE>, lds, name)) return e;
     hipLaunchKernelGGL((convblock_forward_pair_kernel<Ops, NL, RS, ROWS, ONE>), dim3((unsigned)(p.tiles * p.groups)), dim3(kPairWaves * kWave), lds, st,
@@ -273,7 +278,9 @@ bool clg_plan_pair(const Geom &g, int elem, PairPlan *p, bool split)
     p->pw = g.pw;
     p->G = std::max(1, std::min(kWave / I, g.n));
     p->pieces = (uint32_t)(g.h * g.w / per);
-    if (split && I > kWave && g.wo / 2 <= kWave && g.w % per == 0) {
+    // an image of more than 64 cells whose rows are whole pieces goes in bands of whole rows of cells, or not at all
+    if (split && I > kWave && g.w % per == 0) {
+        if (g.wo / 2 > kWave) return false;
         const int rows = kWave / (g.wo / 2), hp = g.ho / 2;
         p->bands = (int)clg_ceil_div(hp, rows);
         p->band_rows = (int)clg_ceil_div(hp, p->bands);
@@ -351,4 +358,20 @@ int clg_forward_pair_packed(const Geom &g, const PairPlan &p, const uint64_t *x,
     if (p.loads <= 2) return launch_pair_nl<BitOpsAnf, 2>(g, p, x, nullptr, table, sel, y, nullptr, st, name);
     if (p.loads <= 4) return launch_pair_nl<BitOpsAnf, 4>(g, p, x, nullptr, table, sel, y, nullptr, st, name);
     return launch_pair_nl<BitOpsAnf, 6>(g, p, x, nullptr, table, sel, y, nullptr, st, name);
+}
+
+extern "C" int clg_convblock_pair_plan(int dtype, const clg_conv_geom *gg, int weight_gradient, int64_t *plan)
+{
+    const char *name = "clg_convblock_pair_plan";
+    Geom g;
+    if (int e = clg_convblock_check(gg, &g, dtype, name)) return e;
+    CLG_REQUIRE(plan && !(weight_gradient && dtype != CLG_F32), "%s: null pointer argument, or a weight gradient of words", name);
+    PairPlan p;
+    if (!clg_plan_pair(g, dtype == CLG_F64 ? 8 : 4, &p, !weight_gradient)) return 0;
+    plan[0] = p.G;
+    plan[1] = p.groups;
+    plan[2] = p.bands;
+    plan[3] = p.band_rows;
+    plan[4] = (int64_t)kPairWaves * p.wave_elems * (dtype == CLG_F64 ? 8 : 4);
+    return 1;
 }

@@ -86,6 +86,7 @@ SIGNATURES = {
     "clg_convblock_eval_packed": (_i, [_GP, _p, _p, _p, _p, _p]),
     "clg_convblock_eval_packed_ws": (_i, [_GP, _p, _p, _p, _p, _p, _p]),
     "clg_convblock_eval_packed_scratch_bytes": (_i64, [_GP]),
+    "clg_convblock_pair_plan": (_i, [_i, _GP, _i, _p]),
     "clg_convblock_forward_ws": (_i, [_i, _GP, _p, _p, _p, _p, _p, _p, _p]),
     "clg_convblock_forward_scratch_bytes": (_i64, [_i, _GP]),
     "clg_convblock_intermediates": (_i, [_i, _GP, _p, _p, _p, _p, _p, _p]),

@@ -26,6 +26,10 @@ SHAPES = [(1, 3, 8, 8, 5, 3, 1),          # one group that is not full
           (2, 2, 8, 8, 4, 8, 4),          # padding as wide as a piece of floats: (even sizes 9 - 1)
           (33, 4, 2, 2, 6, 3, 1),         # one cell per sample: 64 samples in a group
           (2, 1, 20, 12, 4, 3, 1),        # one channel: both planes are the same
+          (2, 3, 4, 128, 6, 3, 1),        # a row of 64 cells is a band
+          (2, 3, 4, 256, 9, 3, 1),        # rows of more cells than a wavefront has lanes: whole pieces are left to the other kernels,
+          (3, 4, 2, 132, 10, 3, 1),
+          (3, 4, 2, 130, 10, 3, 1),       # others are walked 64 cells at a time
           (5, 3, 8, 7, 6, (3, 4), 1)]     # odd rows: a sample's planes are no whole number of pieces
 
 
