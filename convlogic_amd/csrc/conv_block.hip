@@ -1583,7 +1583,7 @@ static int convblock_backward_w_impl(int dtype, const clg_conv_geom *gg, const v
     // Behind the direct input gradient (many channels, or few samples): planes staged two at a time where the shape allows it, from
     // x itself ([256,128,8,8] -> 512, both gradients: 51.4 -> 47.3 us; behind the tiled input gradient 112 -> 115 at [64,32,28,28] -> 256).
     PairPlan pp;
-    bool pair = shared != nullptr && shared->direct && dtype == CLG_F32 && clg_plan_pair(g, 4, &pp, false);
+    bool pair = shared != nullptr && shared->direct && dtype == CLG_F32 && clg_plan_pair(g, 4, &pp, false) && clg_pair_grad_w_wanted(g, pp);
     if (const char *e = clg_knob(K_BWDW_PAIR)) pair = pair && atoi(e) != 0;
     if (pair) {
         const int nb = clg_pair_grad_w_parts(g, pp);

@@ -39,6 +39,7 @@ bool clg_packed_pair(const Geom &g, PairPlan *p);
 constexpr int kPairWaves = 4;
 // The 28 sums per kernel of a float block's weight gradient by the same staging (conv_pair_grad.hip): partial [c][nb][28].
 int clg_pair_grad_w_parts(const Geom &g, const PairPlan &p);          // nb, at most 64
+bool clg_pair_grad_w_wanted(const Geom &g, const PairPlan &p);        // false where it is not the kernel to take
 int clg_pair_grad_w(const Geom &g, const PairPlan &p, int nb, const float *gy, const float *x, const float *folded, const int32_t *sel,
                     const uint8_t *argmax, float *partial, hipStream_t st, const char *name);
 

@@ -373,5 +373,6 @@ extern "C" int clg_convblock_pair_plan(int dtype, const clg_conv_geom *gg, int w
     plan[2] = p.bands;
     plan[3] = p.band_rows;
     plan[4] = (int64_t)kPairWaves * p.wave_elems * (dtype == CLG_F64 ? 8 : 4);
+    plan[5] = weight_gradient ? clg_pair_grad_w_parts(g, p) : 0;
     return 1;
 }

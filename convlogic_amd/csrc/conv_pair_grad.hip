@@ -4,7 +4,7 @@
 // The kernel with lanes along a padded copy of x asks the vector cache for eight addresses per lane and cell, 16 clocks each of the
 // one that four SIMDs share: 128 of the 270 clocks it takes per 64 cells.  Here they come as two 16-byte loads of a
 // lane.  102 vector instructions per 64 cells bound it from there ([128,4096,8,8] -> 16384: 253 -> 172 us, 81 of them those;
-// [128,1024,16,16] -> 4096: 191 -> 157; [256,128,8,8] -> 512: 16.9 -> 14).
+// [128,1024,16,16] -> 4096: 191 -> 165; [256,128,8,8] -> 512: 16.9 -> 14).
 // The input gradient was built the same way (own planes resident, the other channel's staged per kernel, gradient planes in LDS) and
 // taken back: 620 to 640 us for both gradients against 597 with the kernel that gathers; a chain of scalar loads, staging
 // and read-add-write rounds per kernel of a list bounds both.
@@ -185,13 +185,25 @@ static int launch_pair_w_nl(const Geom &g, const PairPlan &p, int nb, const floa
     return launch(g, p, nb, gy, x, folded, sel, argmax, partial, st, name);
 }
 
-// Workgroups per kernel: 1024 of them are enough ([256,32,16,16] -> 128, both gradients: 52.7 us without this kernel, 46.9 with 8 per kernel,
-// 50.8 with 16, 63 with 2; [128,4096,8,8] -> 16384: 691, 597 with 1, 617 with 2), and a wavefront takes at least four blocks of cells for its
-// 28 reductions.
+// Workgroups per kernel.  A lane adds one term per block of cells it visits to the same sum, so there are as many as keep that chain where the
+// kernel of the padded copy has it: 8 terms, 16 from 65536 cells of a kernel on (one part for each of 4096 kernels had 32 terms and an
+// error 1.2 times as large at [128,1024,16,16] -> 4096, 161 us where four take 169; 1.5 times at [1000,40,8,8] -> 2000).  More of them up to 1024 workgroups in all ([256,32,16,16] -> 128, both gradients: 52.7 us without
+// this kernel, 46.9 with 8 per kernel, 50.8 with 16, 63 with 2), as long as a wavefront has four blocks of cells for its 28
+// reductions.
+constexpr int kMaxParts = 64;                                        // (what the scratch holds)
+static int64_t cell_blocks(const Geom &g, const PairPlan &p) { return (int64_t)p.groups * clg_ceil_div((int64_t)p.G * (g.ho / 2) * (g.wo / 2), kWave); }
 int clg_pair_grad_w_parts(const Geom &g, const PairPlan &p)
 {
-    const int64_t blocks = (int64_t)p.groups * clg_ceil_div((int64_t)p.G * (g.ho / 2) * (g.wo / 2), kWave);
-    return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(64, clg_ceil_div(1024, g.c)), blocks / (4 * kPairWaves)));
+    const int64_t cells = (int64_t)(g.ho / 2) * (g.wo / 2) * g.n, blocks = cell_blocks(g, p), terms = cells >= 65536 ? 16 : 8;
+    const int64_t fill = std::min<int64_t>(clg_ceil_div(1024, g.c), blocks / (4 * kPairWaves));
+    return (int)std::max<int64_t>(1, std::min<int64_t>(kMaxParts, std::max(fill, clg_ceil_div(blocks, terms * kPairWaves))));
+}
+// From the most parts on the kernel of the padded copy has longer chains as well: one term per 256 threads and 64 parts.
+bool clg_pair_grad_w_wanted(const Geom &g, const PairPlan &p)
+{
+    const int nb = clg_pair_grad_w_parts(g, p);
+    const int64_t cells = (int64_t)(g.ho / 2) * (g.wo / 2) * g.n;
+    return nb < kMaxParts || clg_ceil_div(cell_blocks(g, p), (int64_t)nb * kPairWaves) <= clg_ceil_div(cells, (int64_t)kMaxParts * 256);
 }
 
 int clg_pair_grad_w(const Geom &g, const PairPlan &p, int nb, const float *gy, const float *x, const float *folded, const int32_t *sel,

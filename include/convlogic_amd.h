@@ -367,8 +367,9 @@ int clg_convblock_eval_packed(const clg_conv_geom *g, const uint64_t *x, const u
 /* clg_convblock_eval_packed with a workspace, as clg_convblock_forward_ws. */
 int64_t clg_convblock_eval_packed_scratch_bytes(const clg_conv_geom *g);
 /* The plan of the kernels that stage two planes of a block per wavefront, to look at: returns 1 where they can take the shape, 0 where they
- * cannot, negative for bad arguments.  dtype: CLG_F32, or CLG_F64 for words; weight_gradient: 0 for the forward.  plan[0..4]: samples
- * per group, groups, bands of a sample (0: a group is whole samples), rows of pooled cells of a band, bytes of LDS per workgroup. */
+ * cannot, negative for bad arguments.  dtype: CLG_F32, or CLG_F64 for words; weight_gradient: 0 for the forward.  plan[0..5]: samples
+ * per group, groups, bands of a sample (0: a group is whole samples), rows of pooled cells of a band, bytes of LDS per workgroup,
+ * workgroups that share a kernel's weight gradient (0 for the forward). */
 int clg_convblock_pair_plan(int dtype, const clg_conv_geom *g, int weight_gradient, int64_t *plan);
 int clg_convblock_eval_packed_ws(const clg_conv_geom *g, const uint64_t *x, const uint8_t *gates,
                                  const int32_t *selection, uint64_t *y, void *scratch, void *stream);

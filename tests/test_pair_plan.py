@@ -32,13 +32,13 @@ def _check(lib, n, c_in, h, w, c_out, kh, kw, ph, pw, seen):
         for size in (lib.clg_convblock_forward_scratch_bytes, lib.clg_convblock_backward_scratch_bytes):
             assert (size(dtype, ctypes.byref(g)) >= 0) == fine
     assert (lib.clg_convblock_eval_packed_scratch_bytes(ctypes.byref(g)) >= 0) == fine
-    plan = (ctypes.c_int64 * 5)()
+    plan = (ctypes.c_int64 * 6)()
     for dtype, weight_gradient in ((0, 0), (1, 0), (0, 1)):
         took = lib.clg_convblock_pair_plan(dtype, ctypes.byref(g), weight_gradient, plan)
         assert (took >= 0) == fine
         if took != 1:
             continue
-        samples, groups, bands, rows, lds = plan
+        samples, groups, bands, rows, lds, parts = plan
         cells, pieces_in_rows = (ho // 2) * (wo // 2), w % (4 if dtype == 0 else 2) == 0
         assert 0 < lds <= 64 * 1024
         if bands:                                                     # a lane per cell of a band, the bands cover the rows, none is empty
@@ -47,6 +47,9 @@ def _check(lib, n, c_in, h, w, c_out, kh, kw, ph, pw, seen):
         else:                                                         # more cells than lanes: only the kernels that walk a group
             assert samples * groups >= n > samples * (groups - 1)
             assert samples * cells <= 64 or weight_gradient or not pieces_in_rows
+        if weight_gradient:                                           # terms a lane adds to one sum: as many as in the kernel of the padded copy
+            blocks, limit = groups * -(-samples * cells // 64), 16 if n * cells >= 65536 else 8
+            assert 1 <= parts <= 64 and (parts == 64 or -(-blocks // (4 * parts)) <= limit)
         seen.add((dtype, weight_gradient, bands > 0, samples * cells > 64))
 
 
@@ -65,6 +68,16 @@ def test_plans_of_all_small_geometries():
                         _check(lib, n, 5, h, w, 40, *kernel, seen)
     _in_a_thread(work)
     assert {(0, 0, True, True), (0, 0, False, False), (0, 0, False, True), (1, 0, True, True), (0, 1, False, True)} <= seen
+
+
+def test_parts_of_a_weight_gradient_of_many_kernels():
+    def work():
+        lib = _lib.load()
+        for n in (1, 16, 33, 90, 128, 300, 400, 1000, 4096, 20000):
+            for side in (4, 6, 8, 12, 16, 20, 24, 32):
+                for c_out in (3, 64, 600, 1024, 4096, 65535):
+                    _check(lib, n, 16, side, side, c_out, 3, 3, 1, 1, set())
+    _in_a_thread(work)
 
 
 def test_plans_of_wide_images():
