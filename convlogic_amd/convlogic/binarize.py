@@ -45,7 +45,8 @@ def pack_thresholds(x: torch.Tensor, thresholds: torch.Tensor) -> PackBitsTensor
     if not x.is_cuda:
         raise NotImplementedError(f"pack_thresholds only supports GPU tensors, but got {x.device}.")
     thresholds = thresholds.float().contiguous()
-    if thresholds.numel() > convlogic_hip.THRESHOLDS_HOST_MAX or torch.cuda.is_current_stream_capturing():
-        thresholds = thresholds.to(x.device)                         # (a recording must not keep the values of this call)
+    # few of them in host memory travel in the launch (but a recording must not keep the values of this call); the rest go to x's device
+    if thresholds.device.type != "cpu" or thresholds.numel() > convlogic_hip.THRESHOLDS_HOST_MAX or torch.cuda.is_current_stream_capturing():
+        thresholds = thresholds.to(x.device)
     words, pad_len = convlogic_hip.threshold_pack_images(x.float().contiguous(), thresholds)
     return PackBitsTensor.from_image_words(words, pad_len)

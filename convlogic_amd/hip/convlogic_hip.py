@@ -492,6 +492,7 @@ def _threshold_args(x, thresholds, host=False):
     check_input(x, "x")
     if not host:
         check_input(thresholds, "thresholds")
+        _lib.check_same_device(x, thresholds)
     if x.dtype != torch.float32 or thresholds.dtype != torch.float32 or x.dim() != 4 or thresholds.dim() != 1:
         raise RuntimeError("expected float32 images [N, C, H, W] and float32 thresholds [L]")
     n, c0, h, w = x.shape

@@ -458,3 +458,32 @@ def test_blocks_of_any_number_of_kernels_are_planned_on_the_host(c_out):
                 assert lib.clg_convblock_backward_scratch_bytes(dtype, ctypes.byref(g)) > 0
                 assert lib.clg_convblock_plan_bytes(dtype, ctypes.byref(g)) > 0
                 lib.clg_fc_tree_partial_elems(1 + poison, 1, 1, 1)
+
+
+@pytest.mark.parametrize("where,count,recording,moved", [("cpu", 3, False, False), ("cpu", 64, False, False), ("cpu", 65, False, True), ("cpu", 3, True, True),
+                                                         ("cuda:0", 3, False, True), ("cuda:1", 3, False, True), ("cuda:1", 65, False, True)])
+def test_thresholds_reach_the_kernel_in_host_memory_or_on_the_device_of_the_images(monkeypatch, where, count, recording, moved):
+    # (stand-ins for tensors: there is no second GPU to put thresholds on)
+    from convlogic_amd.convlogic import binarize
+
+    class Stand:
+        is_cuda = True
+
+        def __init__(self, device):
+            self.device = torch.device(device)
+
+        def float(self):
+            return self
+        contiguous = float
+
+        def numel(self):
+            return count
+
+        def to(self, device):
+            return Stand(device)
+    took = []
+    monkeypatch.setattr(binarize.convlogic_hip, "threshold_pack_images", lambda x, thr: took.append(thr.device) or (None, 0))
+    monkeypatch.setattr(binarize.PackBitsTensor, "from_image_words", lambda *a: None)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: recording)
+    binarize.pack_thresholds(Stand("cuda:0"), Stand(where))
+    assert took == [torch.device("cuda:0" if moved else "cpu")]
