@@ -185,25 +185,34 @@ static int launch_pair_w_nl(const Geom &g, const PairPlan &p, int nb, const floa
     return launch(g, p, nb, gy, x, folded, sel, argmax, partial, st, name);
 }
 
-// Workgroups per kernel.  A lane adds one term per block of cells it visits to the same sum, so there are as many as keep that chain where the
-// kernel of the padded copy has it: 8 terms, 16 from 65536 cells of a kernel on (one part for each of 4096 kernels had 32 terms and an
-// error 1.2 times as large at [128,1024,16,16] -> 4096, 161 us where four take 169; 1.5 times at [1000,40,8,8] -> 2000).  More of them up to 1024 workgroups in all ([256,32,16,16] -> 128, both gradients: 52.7 us without
-// this kernel, 46.9 with 8 per kernel, 50.8 with 16, 63 with 2), as long as a wavefront has four blocks of cells for its 28
-// reductions.
+// Workgroups per kernel.  A lane adds one term per block of cells it visits to the same sum, so there are as many as keep that chain no longer
+// than in the kernel of the padded copy, which gives a thread 8 terms, 16 from 65536 cells of a kernel on, in at most 64 parts (one
+// part for each of 4096 kernels had 32 terms and an error 1.2 times as large at [128,1024,16,16] -> 4096, 161 us where four
+// take 169; 1.5 times at [1000,40,8,8] -> 2000).  A group's blocks of cells stay together, so a lane takes whole groups.  More workgroups up to
+// 1024 in all ([256,32,16,16] -> 128, both gradients: 52.7 us without this kernel, 46.9 with 8 per kernel, 50.8 with
+// 16, 63 with 2), as long as a wavefront has four blocks of cells for its 28 reductions.
 constexpr int kMaxParts = 64;                                        // (what the scratch holds)
-static int64_t cell_blocks(const Geom &g, const PairPlan &p) { return (int64_t)p.groups * clg_ceil_div((int64_t)p.G * (g.ho / 2) * (g.wo / 2), kWave); }
+struct Chain {
+    int64_t blocks, limit;                                           // blocks of 64 cells of a group; terms of the other kernel
+};
+static Chain chain_of(const Geom &g, const PairPlan &p)
+{
+    const int64_t I = (int64_t)(g.ho / 2) * (g.wo / 2), cells = I * g.n, terms = cells >= 65536 ? 16 : 8;
+    const int64_t parts = std::min<int64_t>(kMaxParts, clg_ceil_div(cells, 256 * terms));
+    return {clg_ceil_div(p.G * I, kWave), clg_ceil_div(cells, 256 * parts)};
+}
 int clg_pair_grad_w_parts(const Geom &g, const PairPlan &p)
 {
-    const int64_t cells = (int64_t)(g.ho / 2) * (g.wo / 2) * g.n, blocks = cell_blocks(g, p), terms = cells >= 65536 ? 16 : 8;
-    const int64_t fill = std::min<int64_t>(clg_ceil_div(1024, g.c), blocks / (4 * kPairWaves));
-    return (int)std::max<int64_t>(1, std::min<int64_t>(kMaxParts, std::max(fill, clg_ceil_div(blocks, terms * kPairWaves))));
+    const Chain ch = chain_of(g, p);
+    const int64_t groups = std::max<int64_t>(1, ch.limit / ch.blocks);      // of a wavefront
+    const int64_t fill = std::min<int64_t>(clg_ceil_div(1024, g.c), p.groups * ch.blocks / (4 * kPairWaves));
+    return (int)std::max<int64_t>(1, std::min<int64_t>(kMaxParts, std::max(fill, clg_ceil_div(p.groups, groups * kPairWaves))));
 }
-// From the most parts on the kernel of the padded copy has longer chains as well: one term per 256 threads and 64 parts.
+// Lanes that idle in every block of cells can make the chain longer than the other kernel's even with the most parts.
 bool clg_pair_grad_w_wanted(const Geom &g, const PairPlan &p)
 {
-    const int nb = clg_pair_grad_w_parts(g, p);
-    const int64_t cells = (int64_t)(g.ho / 2) * (g.wo / 2) * g.n;
-    return nb < kMaxParts || clg_ceil_div(cell_blocks(g, p), (int64_t)nb * kPairWaves) <= clg_ceil_div(cells, (int64_t)kMaxParts * 256);
+    const Chain ch = chain_of(g, p);
+    return clg_ceil_div(p.groups, (int64_t)clg_pair_grad_w_parts(g, p) * kPairWaves) * ch.blocks <= std::max(ch.limit, ch.blocks);
 }
 
 int clg_pair_grad_w(const Geom &g, const PairPlan &p, int nb, const float *gy, const float *x, const float *folded, const int32_t *sel,

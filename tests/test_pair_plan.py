@@ -47,9 +47,10 @@ def _check(lib, n, c_in, h, w, c_out, kh, kw, ph, pw, seen):
         else:                                                         # more cells than lanes: only the kernels that walk a group
             assert samples * groups >= n > samples * (groups - 1)
             assert samples * cells <= 64 or weight_gradient or not pieces_in_rows
-        if weight_gradient:                                           # terms a lane adds to one sum: as many as in the kernel of the padded copy
-            blocks, limit = groups * -(-samples * cells // 64), 16 if n * cells >= 65536 else 8
-            assert 1 <= parts <= 64 and (parts == 64 or -(-blocks // (4 * parts)) <= limit)
+        if weight_gradient:                                           # terms a lane adds to one sum: no more than in the kernel of the padded copy
+            blocks, total = -(-samples * cells // 64), n * cells
+            other = -(-total // (256 * min(64, -(-total // (256 * (16 if total >= 65536 else 8))))))
+            assert 1 <= parts <= 64 and (parts == 64 or -(-groups // (4 * parts)) * blocks <= max(other, blocks))
         seen.add((dtype, weight_gradient, bands > 0, samples * cells > 64))
 
 
