@@ -699,13 +699,16 @@ __global__ __launch_bounds__(256) void fc_tree_codes_kernel(TreeLogits lg, const
         }
         return;
     }
-    const int j = (int)(e >> 5), q = (int)(e >> 2) & 7;               // 32 lanes per root, four per gate
-    int id = 0;
-    if (j < roots && q < 7) id = argmax16_quad(reinterpret_cast<const f32x4u *>(tree_logits(lg, ids, j, q, roots))[part]);
-    uint8_t gate[7];
+    const int q = (threadIdx.x >> 2) & 7;                             // 32 lanes per root, four per gate
+    for (int j0 = blockIdx.x * 8; j0 < roots; j0 += net.tree_blocks * 8) {
+        const int j = j0 + (int)(threadIdx.x >> 5);
+        int id = 0;
+        if (j < roots && q < 7) id = argmax16_quad(reinterpret_cast<const f32x4u *>(tree_logits(lg, ids, j, q, roots))[part]);
+        uint8_t gate[7];
 #pragma unroll
-    for (int t = 0; t < 7; ++t) gate[t] = (uint8_t)__shfl(id, (threadIdx.x & 32) + 4 * t, kWave);
-    if (j < roots && q == 0 && part == 0) codes[j] = tree_code(gate);
+        for (int t = 0; t < 7; ++t) gate[t] = (uint8_t)__shfl(id, (threadIdx.x & 32) + 4 * t, kWave);
+        if (j < roots && q == 0 && part == 0) codes[j] = tree_code(gate);
+    }
 }
 
 constexpr int kTreePlanes = 14;                                      // a workgroup takes at most 2^14 - 1 roots
@@ -907,7 +910,8 @@ int count_packed(const char *name, const int64_t *x, const int32_t *rows, const 
 int make_codes(const char *name, const TreeLogits &lg, const int32_t *ids, uint32_t *codes, int64_t roots, int32_t *counts, int64_t n_counts,
                NetGates &net, hipStream_t st)
 {
-    net.tree_blocks = (int)clg_ceil_div(roots * 32, 256);
+    // 2^18 workgroups fill the GPU many times over; a launch of 32 lanes for each of 2^27 roots would be of more threads than there can be
+    net.tree_blocks = (int)std::min<int64_t>(clg_ceil_div(roots * 32, 256), 1 << 18);
     const int64_t gate_blocks = net.blocks ? clg_ceil_div((int64_t)net.block[net.blocks - 1].end * 32, 256) : 0;
     hipLaunchKernelGGL(fc_tree_codes_kernel, dim3((unsigned)(net.tree_blocks + gate_blocks)), dim3(256), 0, st, lg, ids, codes, (int)roots,
                        counts, n_counts, net);

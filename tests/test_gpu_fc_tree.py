@@ -189,6 +189,25 @@ def test_onehot_of_the_first_maximum(dtype):
     assert torch.equal(got.argmax(-1).to(torch.uint8), difflogic_hip.gate_argmax(logits))
 
 
+# (the gate ids of more roots than one pass of a launch takes; 2^27 of them, 32 lanes each, were once refused)
+@pytest.mark.parametrize("class_rows,k", [(1, 3), (129, 16257), (4096, 32768)])
+def test_packed_counts_of_many_roots(class_rows, k):
+    from convlogic_amd.hip import _lib
+    roots = class_rows * k
+    # every tree's leaves and middle gates are neuron 0 of their layer; the root's gate is "0" or, where logit 15 is above the others, "1"
+    zero = torch.zeros(roots, 8, dtype=torch.int32, device=DEV)
+    first = torch.zeros(1, 16, device=DEV)
+    last = torch.zeros(roots, 16, device=DEV)
+    last[:, 15] = torch.randn(roots, device=DEV)
+    words = torch.randint(-2**63, 2**63 - 1, (5, 1), dtype=torch.int64, device=DEV)
+    codes = torch.empty(roots, dtype=torch.int32, device=DEV)
+    out = torch.empty(64, k, dtype=torch.int32, device=DEV)
+    _lib.check(_lib.load().clg_fc_tree_packed(words.data_ptr(), zero.data_ptr(), zero.data_ptr(), first.data_ptr(), first.data_ptr(), last.data_ptr(),
+                                              codes.data_ptr(), out.data_ptr(), 5, roots, k, 1, 64, _lib.stream_ptr(words)))
+    want = (last[:, 15] > 0).view(k, class_rows).sum(1).int()
+    assert torch.equal(out, want.expand(64, k))
+
+
 @pytest.mark.parametrize("hard", [0, 1])
 def test_ids_out_of_range_stay_inside_the_logits_and_the_probabilities(hard):
     from convlogic_amd.hip import _lib
