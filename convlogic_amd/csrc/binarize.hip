@@ -130,8 +130,8 @@ void launch_threshold_pack(const float *x, const float *thr, const HostThreshold
     const unsigned passes = (unsigned)clg_ceil_div(levels, kLevelsPerPass);
     // Four threads per element: 161 -> 153 us on [65536, 3, 32, 32] with 3 levels (5.8 TB/s), 9.0 -> 4.8 us with 256 images;
     // one where a level's words alone leave LDS nothing to save and the elements fill the GPU (36 against 40 us on
-    // [65536, 1, 28, 28] with 1 level).
-    const bool split = levels > 1 || clg_ceil_div(plane_elems, 256) * groups < 2048;
+    // [65536, 1, 28, 28] with 1 level), and where four would be more threads than a launch can have.
+    const bool split = (levels > 1 || clg_ceil_div(plane_elems, 256) * groups < 2048) && clg_ceil_div(plane_elems, 64) < (1 << 24);
     if (split)
         hipLaunchKernelGGL((threshold_pack_kernel<L, 4>), dim3((unsigned)clg_ceil_div(plane_elems, 64), (unsigned)groups, passes), dim3(256), 0, st,
                            x, thr, host, words, n, plane_elems, levels, (int32_t *)nullptr);

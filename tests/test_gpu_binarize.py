@@ -47,6 +47,14 @@ def test_thresholds_in_host_memory_and_on_the_device(n, side, levels):
     assert torch.equal(convlogic_hip.threshold_pack_images(x, thr.to(DEV))[0], want) and torch.equal(binarize.pack_thresholds(x, strided).t, want)
 
 
+def test_thresholds_of_an_image_of_many_pixels():
+    # 2^30 pixels: four threads per pixel, as more than one level takes, would be a launch of 2^32
+    x = torch.rand((1, 1, 32768, 32768), device=DEV)
+    words = binarize.pack_thresholds(x, torch.tensor([0.25, 0.75])).t
+    for level, thr in enumerate((0.25, 0.75)):
+        assert torch.equal(words[0, level], (x[0, 0] > thr).long())
+
+
 def test_thresholds_and_network_input():
     torch.manual_seed(1)
     assert torch.equal(binarize.uniform_thresholds(3), O.thresholds_uniform(3))
