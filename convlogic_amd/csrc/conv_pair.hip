@@ -313,7 +313,7 @@ bool clg_plan_pair(const Geom &g, int elem, PairPlan *p, bool split)
     while (ct > kPairWaves && (int64_t)p->groups * clg_ceil_div(g.c, ct) < 512) ct /= 2;
     p->ct = (int)ct;
     p->tiles = (int)clg_ceil_div(g.c, ct);
-    if ((int64_t)p->tiles * p->groups >= (1ll << 31)) return false;
+    if (split && (int64_t)p->tiles * p->groups >= (1ll << 24)) return false;   // (workgroups of 256: fewer than 2^32 threads)
     p->d_tiles = make_fastdiv((uint32_t)p->tiles);
     p->d_bands = make_fastdiv((uint32_t)std::max(1, p->bands));
     p->d_pieces = make_fastdiv(p->pieces);

@@ -41,6 +41,7 @@ def _check(lib, n, c_in, h, w, c_out, kh, kw, ph, pw, seen):
         samples, groups, bands, rows, lds, parts = plan
         cells, pieces_in_rows = (ho // 2) * (wo // 2), w % (4 if dtype == 0 else 2) == 0
         assert 0 < lds <= 64 * 1024
+        assert weight_gradient or groups * -(-c_out // 64) < 2**24    # (workgroups of 256 threads; at most 64 kernels each)
         if bands:                                                     # a lane per cell of a band, the bands cover the rows, none is empty
             assert weight_gradient == 0 and samples == 1 and groups == n * bands
             assert rows * (wo // 2) <= 64 and bands * rows >= ho // 2 > (bands - 1) * rows
@@ -87,7 +88,7 @@ def test_plans_of_wide_images():
 
     def work():
         lib = _lib.load()
-        for n, c_in, c_out in ((1, 3, 8), (64, 32, 64)):
+        for n, c_in, c_out in ((1, 3, 8), (64, 32, 64), (2**23, 3, 8)):
             for h in (2, 3, 4, 5, 6, 8, 16):
                 for w in (*range(60, 70), *range(120, 140), 160, 200, *range(250, 264), 384, 512, 520):
                     for kernel in ((3, 3, 1, 1), (5, 5, 2, 2), (2, 2, 0, 0), (3, 4, 1, 1)):
