@@ -178,6 +178,7 @@ __global__ __launch_bounds__(256) void fc_tree_fold_kernel(TreeLogits lg, const 
         // (logits at any 4-byte boundary)
         *reinterpret_cast<float4 *>(mine + from * kFoldPitch + 4 * (lane & 3)) = make_float4(v.x, v.y, v.z, v.w);
     }
+    wave_fence();                                                     // (lanes read what others wrote)
     float w[16], p[16];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -198,9 +199,11 @@ __global__ __launch_bounds__(256) void fc_tree_fold_kernel(TreeLogits lg, const 
     const Coef<float> c = fold16(p);
     if (e < gates) reinterpret_cast<float4 *>(coef)[e] = make_float4(c.ab, c.a, c.b, c.one);
     if (probs == nullptr) return;
+    wave_fence();
 #pragma unroll
     for (int i = 0; i < 4; ++i)
         *reinterpret_cast<float4 *>(mine + lane * kFoldPitch + 4 * i) = make_float4(p[4 * i], p[4 * i + 1], p[4 * i + 2], p[4 * i + 3]);
+    wave_fence();
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int from = 16 * i + (lane >> 2), at = __shfl(place, from, kWave);
