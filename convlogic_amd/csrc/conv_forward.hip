@@ -596,6 +596,37 @@ bool plan_forward_direct(const Geom &g, int elem, bool needs_folded, DirectPlan 
     return true;
 }
 
+// Whether a shape that two planes per wavefront can take is faster there than on the path it has otherwise; all figures are us with the
+// launch that makes the tables.  fits: the tiled kernels hold all channels of a sample in LDS.
+bool pair_is_faster(const Geom &g, int elem, const PairPlan &p, bool is_4x4, bool fits, bool table_ready)
+{
+    const int64_t I = (int64_t)(g.ho / 2) * (g.wo / 2);
+    const int64_t waves = (int64_t)p.groups * g.c * (p.bands ? 1 : clg_ceil_div(p.G * I, kWave));
+    if (elem == 8) {
+        // Words in bands that leave lanes idle (28 x 28 images: 196 cells in 4 times 64) or restage a few channels over and over, from a
+        // thousand wavefronts on: [512,16,28,28] -> 64 71 -> 83, [500,1,28,28] -> 32 29 -> 39, but [1024,9,32,32] -> 32 88 -> 76.
+        const bool idle = 8 * I < 7 * kWave * p.bands, few_channels = g.cin < 4;
+        if (fits && p.bands && (idle || few_channels) && (int64_t)g.n * g.c > 1024) return false;
+        // The table from a launch that is made anyway (a whole network): at any batch ([4,128,8,8] -> 512 11.3 -> 4.5,
+        // [4,32,16,16] -> 128 6.4 -> 4.5; 4 x 4 images [1024,512,4,4] -> 1024 57 -> 44, [141,1600,4,4] -> 3200 83 and 20 -> 26).
+        if (table_ready) return true;
+        // Otherwise from 2^18 wavefronts x channels on, where the second launch is paid for ([272,105,16,16] -> 420 187 -> 64,
+        // [1024,32,16,16] -> 128 73 -> 65, [8,105,16,16] -> 420 15.2 -> 13; 4 groups of them 12.2 -> 12.9).
+        return waves * g.cin >= (1 << 18);
+    }
+    // 4 x 4 images, against a sample per lane: [128,16384,4,4] -> 32768 191 -> 164, but [256,512,4,4] -> 1024 15.0 either way and
+    // [64,512,4,4] -> 1024 8.8 -> 9.8.
+    if (is_4x4) return (int64_t)p.groups * g.c > (1 << 16);
+    // Where a sample's channels do not fit LDS, at every batch ([54,1204,8,8] -> 4816 50.8 -> 37, [176,380,8,8] -> 1520 82.8 -> 35,
+    // [18,46,32,32] -> 571 28.7 -> 23).
+    if (!fits) return true;
+    // Where they fit, the tiled kernels stage every channel for every tile of kernels and this one only what it reads: from 16 channels (24
+    // where the cells of a sample are more than a wavefront) and 2^17 wavefronts x channels on ([256,128,8,8] -> 512 27.1 -> 20.7,
+    // [100,32,12,12] -> 96 20.3 -> 11.8, [64,144,6,6] -> 432 19.0 -> 12.8; [64,16,16,16] -> 64 9.5 -> 10.5 and
+    // [256,16,28,28] -> 64 28.5 -> 35 stay; [64,24,32,32] -> 128 28 -> 20).
+    return g.cin >= (I > kWave ? 24 : 16) && waves * g.cin > (1 << 17);
+}
+
 // Which forward path a shape takes: 0 = tiled (all channels in LDS), 1 = tiled with channel subsets,
 // 2 = direct from a padded copy (needs scratch), 3 = any-shape kernel, 4 = one sample per lane on 4x4 images
 // (float gates; needs scratch for the folded coefficients), 5 = one kernel per lane (float gates, at most 16 pooled
@@ -608,25 +639,7 @@ int choose_forward(const Geom &g, int elem, int params_per_kernel, bool have_scr
     if (lane_sample && elem != 4) return 4;
     const bool tiled = plan_forward(g, elem, params_per_kernel, tp);
     if (have_scratch && (params_per_kernel == 1) == (elem == 8) && clg_plan_pair(g, elem, pair)) {
-        // Two planes per wavefront, against what the shape takes otherwise (us with the launch that makes the tables).  Float gates: where a
-        // sample's channels do not fit LDS it is better at every batch ([54,1204,8,8] -> 4816 50.8 -> 37, [176,380,8,8] -> 1520
-        // 82.8 -> 35, [18,46,32,32] -> 571 28.7 -> 23).  Where they fit, the tiled kernels stage every channel for every tile of
-        // kernels and this one only what it reads: from 16 channels (24 where the cells of a sample are more than a wavefront) and
-        // 2^17 wavefronts x channels on ([256,128,8,8] -> 512 27.1 -> 20.7, [100,32,12,12] -> 96 20.3 -> 11.8, [64,144,6,6] -> 432
-        // 19.0 -> 12.8; [64,16,16,16] -> 64 9.5 -> 10.5 and [256,16,28,28] -> 64 28.5 -> 35 stay; [64,24,32,32] -> 128 28 -> 20).  Words: from 2^18 wavefronts x
-        // channels on, where the second launch is paid for ([272,105,16,16] -> 420 187 -> 64, [1024,32,16,16] -> 128 73 -> 65,
-        // [8,105,16,16] -> 420 15.2 -> 13; 4 groups of them 12.2 -> 12.9).  table_ready: the table comes from a launch that is made anyway (a
-        // whole network): at any batch ([4,128,8,8] -> 512 11.3 -> 4.5, [4,32,16,16] -> 128 6.4 -> 4.5).
-        const int I = (g.ho / 2) * (g.wo / 2);
-        const bool fits = tiled && !tp->subset;
-        // words in bands that leave lanes idle (28 x 28 images: 196 cells in 4 times 64) or restage a few channels over and over, from a thousand
-        // wavefronts on: [512,16,28,28] -> 64 71 -> 83, [500,1,28,28] -> 32 29 -> 39, but [1024,9,32,32] -> 32 88 -> 76
-        const bool bands_lose = pair->bands && (8 * I < 7 * kWave * pair->bands || g.cin < 4) && (int64_t)g.n * g.c > 1024;
-        const int64_t work = (int64_t)pair->groups * g.c * (pair->bands ? 1 : clg_ceil_div((int64_t)pair->G * I, kWave)) * g.cin;
-        // 4 x 4 images, against a sample per lane: [128,16384,4,4] -> 32768 191 -> 164, but [256,512,4,4] -> 1024 15.0 either way and
-        // [64,512,4,4] -> 1024 8.8 -> 9.8; words are better here at every size
-        // ([1024,512,4,4] -> 1024 57 -> 44, [141,1600,4,4] -> 3200 83 and 20 -> 26).
-        bool use = lane_sample ? (int64_t)pair->groups * g.c > (1 << 16) : elem == 8 ? (work >= (1 << 18) || table_ready) && !(bands_lose && fits) : !fits || (work > (1 << 17) && g.cin >= (I > kWave ? 24 : 16));
+        bool use = pair_is_faster(g, elem, *pair, lane_sample, tiled && !tp->subset, table_ready);
         use = use && !clg_knob(K_FWD_DIRECT) && !clg_knob(K_FWD_SUBSET) && !clg_knob(K_FWD_KPL);   // (a path that is asked for)
         if (const char *e = clg_knob(K_FWD_PAIR)) use = atoi(e) != 0;
         if (use) {
