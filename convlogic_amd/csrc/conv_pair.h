@@ -24,8 +24,8 @@ __host__ __device__ inline int32_t pair_tap(int plane, int rs, int odd, int shif
 }
 constexpr int kPairTable = 12;          // per kernel: channel 0, channel 1 (-1: more than two), code, -, 8 taps;
                                         // behind the last one the geometry, for the rare path that needs all of it
-// elem: 4 (float) or 8 (words).  False where the shape is another kernel's.  split: even and odd columns apart, as the forward kernel
-// reads them.
+// elem: 4 (float) or 8 (words).  False where the shape is another kernel's.  split: even and odd columns apart, as the forward kernels
+// read them; without, as the weight gradient of floats does.
 bool clg_plan_pair(const Geom &g, int elem, PairPlan *p, bool split = true);
 int clg_forward_pair_f32(const Geom &g, const PairPlan &p, const float *x, const float *w, const int32_t *sel, float *y, uint8_t *argmax, void *scratch,
                          bool from_logits, float *probs_out, const float *folded_in, float *padded_out, int pad_rs, int pad_chs, int pad_sample,

@@ -272,6 +272,7 @@ bool clg_plan_pair(const Geom &g, int elem, PairPlan *p, bool split)
 {
     const int per = 16 / elem;
     *p = PairPlan{};
+    if (!split && elem != 4) return false;                           // (the weight gradient, which words do not have)
     if (g.sh != 1 || g.sw != 1 || !taps_inside(g) || g.ho % 2 || g.wo % 2 || g.pw > per || (g.h * g.w) % per) return false;
     const int I = (g.ho / 2) * (g.wo / 2);
     p->lead = per;
@@ -293,10 +294,10 @@ bool clg_plan_pair(const Geom &g, int elem, PairPlan *p, bool split)
     } else {
         p->rs = g.w + per;
         p->plane = (g.h + g.ph) * p->rs;
-        // samples 16 words apart modulo the 64 banks, so that the rows of neighbouring samples do not meet there
+        // samples 16 floats apart modulo the 64 banks, so that the rows of neighbouring samples do not meet there
         p->sample = (int)clg_ceil_div(2 * p->plane, per) * per;
         if (p->G > 1)
-            while (p->sample * (elem / 4) % 64 != 16 || p->sample % per) p->sample += elem == 8 ? 2 : 4;
+            while (p->sample % 64 != 16) p->sample += per;
     }
     p->wave_elems = (int)(clg_ceil_div((int64_t)p->G * p->sample + g.ph * p->rs + per + g.kw, per) * per + per + (p->odd + per) / per * per);   // (the end takes what lanes without a piece write)
     if ((int64_t)kPairWaves * p->wave_elems * elem > 64 * 1024) return false;
