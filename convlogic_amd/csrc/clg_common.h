@@ -190,6 +190,20 @@ __device__ __forceinline__ T row16_sum(T v)
     v += dpp_zero<0x140, 0xF>(v);
     return v;
 }
+// The sums over a wavefront of 28 values, four for each of seven gates.  Every exchange between lane groups halves the number of values that a
+// lane holds.  The lane that gets a sum returns it and which one in `at`; the others get at = -1.
+__device__ __forceinline__ float wave_sums28(const float (&v)[28], int lane, int &at)
+{
+    const int i16 = lane & 15, o = (lane >> 4) & 1, h = lane >> 5;
+    float mine = 0.f;
+#pragma unroll
+    for (int q = 0; q < 7; ++q) {                                     // row (h, o) holds sum 2 o + h of gate q
+        const float u = row16_sum(swap_add16(swap_add32(v[4 * q], v[4 * q + 1]), swap_add32(v[4 * q + 2], v[4 * q + 3])));
+        mine = i16 == q ? u : mine;
+    }
+    at = i16 < 7 ? 4 * i16 + 2 * o + h : -1;
+    return mine;
+}
 // Maximum over each row of 16 lanes, valid in all of its lanes.
 template <typename T>
 __device__ __forceinline__ T row16_max(T v)

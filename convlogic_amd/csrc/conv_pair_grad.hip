@@ -34,18 +34,13 @@ __device__ __forceinline__ PairCell pair_cell(const Geom &g, const PairPlan &p, 
     return r;
 }
 
-// The 28 sums of a workgroup: every exchange between lane groups halves the number of values a lane holds, then the wavefronts meet in LDS.
-__device__ __forceinline__ void pair_block_sums(float (&v)[28], float *__restrict__ meet, float *__restrict__ dst, int lane, int wave)
+// The 28 sums of a workgroup: those of its wavefronts meet in LDS.
+__device__ __forceinline__ void pair_block_sums(const float (&v)[28], float *__restrict__ meet, float *__restrict__ dst, int lane, int wave)
 {
-    const int i16 = lane & 15, o = (lane >> 4) & 1, h = lane >> 5;
-    float mine = 0.f;
-#pragma unroll
-    for (int q = 0; q < 7; ++q) {                                     // row (h, o) holds sum 2 o + h of gate q
-        const float u = row16_sum(swap_add16(swap_add32(v[4 * q], v[4 * q + 1]), swap_add32(v[4 * q + 2], v[4 * q + 3])));
-        mine = i16 == q ? u : mine;
-    }
+    int at;
+    const float mine = wave_sums28(v, lane, at);
     __syncthreads();                                                 // (the planes are done with)
-    if (i16 < 7) meet[wave * 28 + 4 * i16 + 2 * o + h] = mine;
+    if (at >= 0) meet[wave * 28 + at] = mine;
     __syncthreads();
     if (threadIdx.x < 28) {
         float s = meet[threadIdx.x];

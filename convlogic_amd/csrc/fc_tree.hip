@@ -311,18 +311,6 @@ __global__ __launch_bounds__(256) void fc_tree_finish_kernel(const float *__rest
 // root; what remains -- 16 gates per neuron, the softmax backward -- needs the rows of seven scattered neurons and is a
 // kernel of its own in neuron order (fc_tree_logit_grad_kernel): done here it held the wavefront for one more round trip and
 // read and wrote 64-byte pieces all over (655360 roots x 128 samples: 1742 us, 978 without it).
-__device__ __forceinline__ void tree_store_sums(float (&v)[28], float *__restrict__ sums, int j, int lane)
-{
-    const int i16 = lane & 15, o = (lane >> 4) & 1, h = lane >> 5;
-    float mine = 0.f;
-#pragma unroll
-    for (int q = 0; q < 7; ++q) {                                     // row (h, o) holds sum 2 o + h of gate q
-        const float u = row16_sum(swap_add16(swap_add32(v[4 * q], v[4 * q + 1]), swap_add32(v[4 * q + 2], v[4 * q + 3])));
-        mine = i16 == q ? u : mine;
-    }
-    if (i16 < 7) sums[(int64_t)j * 28 + 4 * i16 + 2 * o + h] = mine;
-}
-
 // SUMS, ROWS: for the gradients of the logits, of the input (a frozen end and an input without a gradient need one of them).
 template <int V, bool SUMS, bool ROWS>
 __global__ __launch_bounds__(kTreeBlock) void fc_tree_backward_kernel(const float *__restrict__ x, const int32_t *__restrict__ rows,
@@ -405,7 +393,11 @@ __global__ __launch_bounds__(kTreeBlock) void fc_tree_backward_kernel(const floa
                     store_samples<V>(rowgrad + (int64_t)min((uint64_t)(uint32_t)pj[q], (uint64_t)total_rows - 1) * pitch + s, v[q]);
             }
         }
-        if constexpr (SUMS) tree_store_sums(acc, sums, j, lane);
+        if constexpr (SUMS) {
+            int at;
+            const float sum = wave_sums28(acc, lane, at);
+            if (at >= 0) sums[(int64_t)j * 28 + at] = sum;
+        }
     }
 }
 
