@@ -287,7 +287,7 @@ def _cpu_reps(cpu_step, budget_s, max_reps):
 
 
 def _cpu_torch_leg(cpu_step, units_per_step, sample):
-    """cpu_baseline entry of a torch-CPU oracle step: all host threads the box grants (at most 16) for about 5 s, then
+    """cpu_baseline entry of a torch-CPU oracle step: all host threads the machine grants (at most 16) for about 5 s, then
     the same on one thread for about 3 s."""
     import torch
     threads = min(os.cpu_count() or 1, 16)

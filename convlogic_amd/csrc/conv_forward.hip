@@ -15,7 +15,7 @@
 // columns, each lane evaluates the tree at conv rows 2r and 2r+1, the horizontal neighbour comes over
 // DPP, and the even lane pools and writes.  The kernel index is uniform per wavefront, so gate
 // parameters and tap offsets sit in scalar registers.  Many channels with enough samples take the
-// wavefront-private staging of conv_pair.hip; choose_forward below has the rule.
+// wavefront-private staging of conv_pair.hip; pair_is_faster below has the rule.
 #include <stdlib.h>
 
 #include <algorithm>

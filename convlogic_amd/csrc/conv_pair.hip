@@ -13,7 +13,7 @@
 // Bound by LDS and the vector ALU together: per kernel and 64 cells 97 vector instructions of float gates and 16 two-value reads
 // ([128,4096,8,8] -> 16384: 240 us, the vector instructions alone 111; the kernel before read its taps from a padded copy, 355 us), 56 + 30 of
 // words ([1024,128,8,8] -> 512: 66 us).  With even and odd columns in one row the lanes of a read were two elements apart and met in
-// the banks two to four times: 265 and 84 us.  Which shapes come here: choose_forward in conv_forward.hip.
+// the banks two to four times: 265 and 84 us.  Which shapes come here: pair_is_faster in conv_forward.hip.
 #include <algorithm>
 
 #include "conv_ops.h"

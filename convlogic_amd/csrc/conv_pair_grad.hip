@@ -4,7 +4,7 @@
 // The kernel with lanes along a padded copy of x asks the vector cache for eight addresses per lane and cell, 16 clocks each of the
 // one that four SIMDs share: 128 of the 270 clocks it takes per 64 cells.  Here they come as two 16-byte loads of a
 // lane.  102 vector instructions per 64 cells bound it from there ([128,4096,8,8] -> 16384: 253 -> 172 us, 81 of them those;
-// [128,1024,16,16] -> 4096: 191 -> 165; [256,128,8,8] -> 512: 16.9 -> 14).
+// [128,1024,16,16] -> 4096: 191 -> 162; [256,128,8,8] -> 512: 16.9 -> 13).
 // The input gradient was built the same way (own planes resident, the other channel's staged per kernel, gradient planes in LDS) and
 // taken back: 620 to 640 us for both gradients against 597 with the kernel that gathers; a chain of scalar loads, staging
 // and read-add-write rounds per kernel of a list bounds both.
@@ -182,8 +182,8 @@ static int launch_pair_w_nl(const Geom &g, const PairPlan &p, int nb, const floa
 
 // Workgroups per kernel.  A lane adds one term per block of cells it visits to the same sum, so there are as many as keep that chain no longer
 // than in the kernel of the padded copy, which gives a thread 8 terms, 16 from 65536 cells of a kernel on, in at most 64 parts (one
-// part for each of 4096 kernels had 32 terms and an error 1.2 times as large at [128,1024,16,16] -> 4096, 161 us where four
-// take 169; 1.5 times at [1000,40,8,8] -> 2000).  A group's blocks of cells stay together, so a lane takes whole groups.  More workgroups up to
+// part for each of 4096 kernels had 32 terms and an error 1.2 times as large at [128,1024,16,16] -> 4096, 157 us where four
+// take 162; 1.5 times at [1000,40,8,8] -> 2000).  A group's blocks of cells stay together, so a lane takes whole groups.  More workgroups up to
 // 1024 in all ([256,32,16,16] -> 128, both gradients: 52.7 us without this kernel, 46.9 with 8 per kernel, 50.8 with
 // 16, 63 with 2), as long as a wavefront has four blocks of cells for its 28 reductions.
 constexpr int kMaxParts = 64;                                        // (what the scratch holds)
