@@ -13,7 +13,7 @@ from ..difflogic.difflogic import _feature_major, logic_layer_group_sum
 from ..difflogic.fc_tree import tree_eval, tree_packed, tree_plan, tree_train
 from ..difflogic.packbitstensor import PackBitsTensor
 from ..hip.convlogic_hip import bin_supported
-from . import packed_net
+from . import packed_net, train_net
 from .convlogic_layer import ConvLogicLayer
 
 
@@ -89,8 +89,8 @@ def _tree_tail(net):
 def _forward(owner, x):
     """The network on x.  Three things happen that a plain nn.Sequential call would not do: the three LogicLayers and the
     GroupSum at its end are evaluated as one operation where their wiring allows (`tree_tail`, default on; training steps,
-    evaluation and packed inference); in training the logits of the other layers are folded in one launch where that pays (`prefold`), and a
-    last LogicLayer and GroupSum that do not run as trees run as one autograd node (`fused_tail`, default on), whose
+    evaluation and packed inference), in training of a small network the blocks in front of them as well; else the logits of the other
+    layers are folded in one launch where that pays (`prefold`), and a last LogicLayer and GroupSum that do not run as trees run as one autograd node (`fused_tail`, default on), whose
     backward needs no GroupSum launch."""
     net = owner.network
     tail = _tree_tail(net) if owner.__dict__.get("tree_tail", True) else None
@@ -122,6 +122,10 @@ def _forward(owner, x):
         return _rest(net, h)
     plan = tree_plan(*tail[0]) if trees and all(m.training for m in tail[0]) else None
     mode = owner.__dict__.get("prefold", True)                       # True: where it pays, "always", False
+    if plan is not None and mode is True:
+        out = train_net.train(net, tail, plan, x, _called_for_itself)
+        if out is not None:
+            return out
     if mode:
         layers = [m for m in net if isinstance(m, (ConvLogicLayer, LogicLayer))]
         _prefold(owner, layers if plan is None else layers[:-3], x, mode)

@@ -159,92 +159,114 @@ std::vector<int64_t> pooled(const clg_conv_geom &g)
     return {g.n, g.c_out, std::max<int64_t>(ho, 0) / 2, std::max<int64_t>(wo, 0) / 2};
 }
 
-// plan, signature: the layer's backward plan.  pair: probabilities and folded coefficients [c, 7, 16], [c, 7, 4] in one buffer
-// that a network made for all its layers (or null).
+// What a block keeps of its forward pass, in the order in which it is saved.
+struct BlockState {
+    Tensor x, probs, sel, argmax, folded, padded;
+    static constexpr int kTensors = 6;
+    void save(variable_list &list) const { list.insert(list.end(), {x, probs, sel, argmax, folded, padded}); }
+    static BlockState from(const Tensor *t) { return {t[0], t[1], t[2], t[3], t[4], t[5]}; }
+};
+// signature: that of the layer's backward plan.  pair: probabilities and folded coefficients [c, 7, 16], [c, 7, 4] in one buffer
+// that a network made for all its layers (or null).  fm (in): the output may be feature-major; (out): it is, [c, h, w, n].
+Tensor block_forward(const Tensor &x_in, const Tensor &logits, const Tensor &sel_in, const Conv &conv, bool &fm, int64_t signature,
+                     const std::pair<Tensor, Tensor> *pair, bool need_x, BlockState &state)
+{
+    const Tensor x = x_in.contiguous(), sel = sel_in.contiguous();
+    const int64_t c = logits.size(0);
+    const clg_conv_geom g = conv.geom(x, c);
+    const auto s = pooled(g);
+    fm = fm && clg_convblock_fm_supported(CLG_F32, &g);
+    Tensor y = fm ? floats(x, {s[1], s[2], s[3], s[0]}) : floats(x, s), argmax = at::empty(s, x.options().dtype(at::kByte));
+    Tensor probs, folded;                                             // without a pair: probabilities and coefficients in one tensor, no folded
+    if (pair != nullptr) {
+        probs = pair->first, folded = pair->second;
+        need(probs, x, "prefolded probabilities", {c, 7, 16});
+        need(folded, x, "prefolded coefficients", {c, 7, 4});
+        TORCH_CHECK(folded.data_ptr<float>() == probs.data_ptr<float>() + probs.numel(),
+                    "prefolded: the folded coefficients must follow the probabilities in one buffer (fold_many)");
+    } else {
+        probs = floats(x, {c * (112 + 28)});
+    }
+    const Tensor scratch = bytes(x, clg_convblock_forward_scratch_bytes(CLG_F32, &g));
+    const int flags = CLG_FWD_W_LOGITS | (fm ? CLG_FWD_Y_FEATURE_MAJOR : 0) | CLG_FWD_FOLDED_OUT | (pair != nullptr ? CLG_FWD_FOLDED_IN : 0);
+    Tensor padded;
+    if (need_x && (signature & 1) == CLG_LISTS_SHORT && !fm) {        // the copy of x that the forward kernels stage and the backward reads
+        const int64_t elems = clg_convblock_padded_elems(CLG_F32, &g, 1);
+        if (elems > 0) padded = floats(x, {elems});
+    }
+    const int32_t *selection = static_cast<const int32_t *>(sel.data_ptr());
+    uint8_t *codes = static_cast<uint8_t *>(argmax.data_ptr());
+    if (padded.defined())
+        check(clg_convblock_forward_padded(CLG_F32, &g, x.data_ptr(), logits.data_ptr(), selection, y.data_ptr(), codes, probs.data_ptr(), flags,
+                                           scratch.data_ptr(), padded.data_ptr(), stream_of(x)));
+    else
+        check(clg_convblock_forward_ex(CLG_F32, &g, x.data_ptr(), logits.data_ptr(), selection, y.data_ptr(), codes, probs.data_ptr(), flags,
+                                       scratch.data_ptr(), stream_of(x)));
+    state = {x, probs, sel, argmax, folded, padded};
+    return y;
+}
+// -> gradients of x and of the logits; fm: the forward pass was feature-major
+std::pair<Tensor, Tensor> block_backward(const BlockState &state, const Conv &conv, bool fm, const Tensor &plan, int64_t signature, Tensor gy, bool need_x,
+                                         bool need_l)
+{
+    const Tensor &x = state.x, &probs = state.probs, &sel = state.sel;
+    const int64_t c = sel.size(0);
+    const float *folded = state.folded.defined() ? state.folded.data_ptr<float>() : probs.data_ptr<float>() + c * 112;
+    const int32_t *selection = static_cast<const int32_t *>(sel.data_ptr());
+    const uint8_t *codes = static_cast<const uint8_t *>(state.argmax.data_ptr());
+    const clg_conv_geom g = conv.geom(x, c);
+    Tensor gx, gl;
+    if (need_x) gx = at::empty_like(x);
+    if (need_l) {
+        fm = fm && !gy.is_contiguous() && gy.permute({1, 2, 3, 0}).is_contiguous();
+        const auto s = pooled(g);
+        if (fm) {
+            gy = gy.permute({1, 2, 3, 0});
+            need(gy, x, "grad_y", {s[1], s[2], s[3], s[0]});
+        } else {
+            gy = gy.contiguous();
+            need(gy, x, "grad_y", s);
+        }
+        gl = floats(x, {c, 7, 16});
+        const Tensor scratch = bytes(x, clg_convblock_backward_planned_scratch_bytes(CLG_F32, &g, signature));
+        const Tensor padded = fm || !need_x ? Tensor() : state.padded;
+        const int flags = CLG_BWD_WRT_LOGITS | (fm ? CLG_BWD_GY_FEATURE_MAJOR : 0);
+        if (padded.defined())
+            check(clg_convblock_backward_planned_padded(CLG_F32, &g, gy.data_ptr(), x.data_ptr(), probs.data_ptr(), folded, padded.data_ptr(),
+                                                        selection, codes, plan.data_ptr(), signature, gx.data_ptr(), gl.data_ptr(), flags,
+                                                        scratch.data_ptr(), stream_of(x)));
+        else
+            check(clg_convblock_backward_planned(CLG_F32, &g, gy.data_ptr(), x.data_ptr(), probs.data_ptr(), folded, selection, codes,
+                                                 plan.data_ptr(), signature, ptr(gx), gl.data_ptr(), flags, scratch.data_ptr(), stream_of(x)));
+    } else if (need_x) {
+        gy = gy.contiguous();
+        need(gy, x, "grad_y", pooled(g));
+        const Tensor scratch = bytes(x, clg_convblock_backward_x_scratch_bytes(CLG_F32, &g));
+        check(clg_convblock_backward_x(CLG_F32, &g, gy.data_ptr(), x.data_ptr(), probs.data_ptr(), selection, codes, gx.data_ptr(),
+                                       scratch.data_ptr(), stream_of(x)));
+    }
+    return {gx, gl};
+}
 struct Block : torch::autograd::Function<Block> {
-    static Tensor forward(AutogradContext *ctx, const Tensor &x_in, const Tensor &logits, const Tensor &sel_in, const Conv *conv, bool want_fm,
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &logits, const Tensor &sel, const Conv *conv, bool want_fm,
                           const Tensor *plan, int64_t signature, const std::pair<Tensor, Tensor> *pair, bool need_x)
     {
-        const Tensor x = x_in.contiguous(), sel = sel_in.contiguous();
-        const int64_t c = logits.size(0);
-        const clg_conv_geom g = conv->geom(x, c);
-        const auto s = pooled(g);
-        const bool fm = want_fm && clg_convblock_fm_supported(CLG_F32, &g);
-        Tensor y = fm ? floats(x, {s[1], s[2], s[3], s[0]}) : floats(x, s), argmax = at::empty(s, x.options().dtype(at::kByte));
-        Tensor probs, folded;                                         // without a pair: probabilities and coefficients in one tensor, no folded
-        if (pair != nullptr) {
-            probs = pair->first, folded = pair->second;
-            need(probs, x, "prefolded probabilities", {c, 7, 16});
-            need(folded, x, "prefolded coefficients", {c, 7, 4});
-            TORCH_CHECK(folded.data_ptr<float>() == probs.data_ptr<float>() + probs.numel(),
-                        "prefolded: the folded coefficients must follow the probabilities in one buffer (fold_many)");
-        } else {
-            probs = floats(x, {c * (112 + 28)});
-        }
-        const Tensor scratch = bytes(x, clg_convblock_forward_scratch_bytes(CLG_F32, &g));
-        const int flags = CLG_FWD_W_LOGITS | (fm ? CLG_FWD_Y_FEATURE_MAJOR : 0) | CLG_FWD_FOLDED_OUT | (pair != nullptr ? CLG_FWD_FOLDED_IN : 0);
-        Tensor padded;
-        if (need_x && (signature & 1) == CLG_LISTS_SHORT && !fm) {    // the copy of x that the forward kernels stage and the backward reads
-            const int64_t elems = clg_convblock_padded_elems(CLG_F32, &g, 1);
-            if (elems > 0) padded = floats(x, {elems});
-        }
-        const int32_t *selection = static_cast<const int32_t *>(sel.data_ptr());
-        uint8_t *codes = static_cast<uint8_t *>(argmax.data_ptr());
-        if (padded.defined())
-            check(clg_convblock_forward_padded(CLG_F32, &g, x.data_ptr(), logits.data_ptr(), selection, y.data_ptr(), codes, probs.data_ptr(), flags,
-                                               scratch.data_ptr(), padded.data_ptr(), stream_of(x)));
-        else
-            check(clg_convblock_forward_ex(CLG_F32, &g, x.data_ptr(), logits.data_ptr(), selection, y.data_ptr(), codes, probs.data_ptr(), flags,
-                                           scratch.data_ptr(), stream_of(x)));
-        ctx->save_for_backward({x, probs, sel, argmax, folded, padded});
-        ctx->saved_data["conv"] = conv->saved({fm, signature});
+        BlockState state;
+        const Tensor y = block_forward(x, logits, sel, *conv, want_fm, signature, pair, need_x, state);
+        variable_list saved;
+        state.save(saved);
+        ctx->save_for_backward(std::move(saved));
+        ctx->saved_data["conv"] = conv->saved({want_fm, signature});
         ctx->saved_data["plan"] = *plan;
-        return fm ? y.permute({3, 0, 1, 2}) : y;
+        return want_fm ? y.permute({3, 0, 1, 2}) : y;
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
         const auto saved = ctx->get_saved_variables();
-        const Tensor &x = saved[0], &probs = saved[1], &sel = saved[2], &argmax = saved[3];
         const auto ints = ctx->saved_data["conv"].toIntVector();
-        const Conv conv = Conv::from(ints);
-        const bool need_x = ctx->needs_input_grad(0), need_l = ctx->needs_input_grad(1);
-        const int64_t c = sel.size(0), signature = ints[7];
-        const float *folded = saved[4].defined() ? saved[4].data_ptr<float>() : probs.data_ptr<float>() + c * 112;
-        const int32_t *selection = static_cast<const int32_t *>(sel.data_ptr());
-        const uint8_t *codes = static_cast<const uint8_t *>(argmax.data_ptr());
-        const clg_conv_geom g = conv.geom(x, c);
-        Tensor gy = grads[0], gx, gl;
-        if (need_x) gx = at::empty_like(x);
-        if (need_l) {
-            const bool fm = ints[6] && !gy.is_contiguous() && gy.permute({1, 2, 3, 0}).is_contiguous();
-            const auto s = pooled(g);
-            if (fm) {
-                gy = gy.permute({1, 2, 3, 0});
-                need(gy, x, "grad_y", {s[1], s[2], s[3], s[0]});
-            } else {
-                gy = gy.contiguous();
-                need(gy, x, "grad_y", s);
-            }
-            gl = floats(x, {c, 7, 16});
-            const Tensor plan = ctx->saved_data["plan"].toTensor(),
-                         scratch = bytes(x, clg_convblock_backward_planned_scratch_bytes(CLG_F32, &g, signature));
-            const Tensor padded = fm || !need_x ? Tensor() : saved[5];
-            const int flags = CLG_BWD_WRT_LOGITS | (fm ? CLG_BWD_GY_FEATURE_MAJOR : 0);
-            if (padded.defined())
-                check(clg_convblock_backward_planned_padded(CLG_F32, &g, gy.data_ptr(), x.data_ptr(), probs.data_ptr(), folded,
-                                                            padded.data_ptr(), selection, codes, plan.data_ptr(), signature, gx.data_ptr(),
-                                                            gl.data_ptr(), flags, scratch.data_ptr(), stream_of(x)));
-            else
-                check(clg_convblock_backward_planned(CLG_F32, &g, gy.data_ptr(), x.data_ptr(), probs.data_ptr(), folded, selection, codes,
-                                                     plan.data_ptr(), signature, ptr(gx), gl.data_ptr(), flags, scratch.data_ptr(), stream_of(x)));
-        } else if (need_x) {
-            gy = gy.contiguous();
-            need(gy, x, "grad_y", pooled(g));
-            const Tensor scratch = bytes(x, clg_convblock_backward_x_scratch_bytes(CLG_F32, &g));
-            check(clg_convblock_backward_x(CLG_F32, &g, gy.data_ptr(), x.data_ptr(), probs.data_ptr(), selection, codes, gx.data_ptr(),
-                                           scratch.data_ptr(), stream_of(x)));
-        }
-        return {gx, gl, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+        const auto g = block_backward(BlockState::from(saved.data()), Conv::from(ints), ints[6], ctx->saved_data["plan"].toTensor(), ints[7], grads[0],
+                                      ctx->needs_input_grad(0), ctx->needs_input_grad(1));
+        return {g.first, g.second, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };
 Tensor block(const Tensor &x, const Tensor &logits, const Tensor &sel, std::array<int64_t, 6> conv, bool want_fm, const Tensor &plan,
@@ -255,46 +277,58 @@ Tensor block(const Tensor &x, const Tensor &logits, const Tensor &sel, std::arra
     return Block::apply(x, logits, sel, &cv, want_fm, &plan, signature, prefolded ? &*prefolded : nullptr, at::GradMode::is_enabled() && x.requires_grad());
 }
 
-// The block on 0/1 inputs, from the logits.  flag: device address of the layer's BinaryFlag.
+// The block on 0/1 inputs, from the logits.  flag: device address of the layer's BinaryFlag.  It keeps taps and keep; x itself is not needed
+// again.
+Tensor binary_forward(const Tensor &x_in, const Tensor &logits, const Tensor &sel_in, const Conv &conv, int64_t flag, Tensor &taps, Tensor &keep)
+{
+    const Tensor x = x_in.contiguous(), sel = sel_in.contiguous();
+    const clg_conv_geom g = conv.geom(x, logits.size(0));
+    keep = bytes(x, clg_convblock_bin_ctx_bytes(CLG_F32, &g));
+    const auto s = pooled(g);
+    Tensor y = floats(x, s);
+    taps = at::empty(s, x.options().dtype(at::kShort));
+    check(clg_convblock_bin_forward(CLG_F32, &g, x.data_ptr(), logits.data_ptr(), static_cast<const int32_t *>(sel.data_ptr()), y.data_ptr(),
+                                    static_cast<uint16_t *>(taps.data_ptr()), keep.data_ptr(), CLG_FWD_W_LOGITS, reinterpret_cast<int32_t *>(flag),
+                                    stream_of(x)));
+    return y;
+}
+// xs: shape of x
+std::pair<Tensor, Tensor> binary_backward(const Tensor &taps, const Tensor &keep, const Conv &cv, at::IntArrayRef xs, const Tensor &grad, bool need_x, bool need_l)
+{
+    const Tensor gy = grad.contiguous();
+    TORCH_CHECK(gy.is_cuda(), "grad_y must be a CUDA tensor");
+    TORCH_CHECK(gy.device() == taps.device(), "all tensors must be on one device, got ", taps.device(), " and ", gy.device());
+    need(gy, gy, "grad_y", taps.sizes());
+    const int64_t c = gy.size(1);
+    const clg_conv_geom g = {(int32_t)xs[0], (int32_t)xs[1], (int32_t)xs[2], (int32_t)xs[3], (int32_t)c, (int32_t)cv.sh, (int32_t)cv.sw,
+                             (int32_t)cv.ph, (int32_t)cv.pw, (int32_t)cv.kh, (int32_t)cv.kw};
+    Tensor gx, gl, scratch;
+    if (need_x) gx = floats(gy, xs);
+    if (need_l) {
+        gl = floats(gy, {c, 7, 16});
+        scratch = bytes(gy, clg_convblock_bin_backward_scratch_bytes(CLG_F32, &g));
+    }
+    if (need_x || need_l)
+        check(clg_convblock_bin_backward(CLG_F32, &g, gy.data_ptr(), static_cast<const uint16_t *>(taps.data_ptr()), keep.data_ptr(), ptr(gx), ptr(gl),
+                                         CLG_BWD_WRT_LOGITS, ptr(scratch), stream_of(gy)));
+    return {gx, gl};
+}
 struct BinaryBlock : torch::autograd::Function<BinaryBlock> {
-    static Tensor forward(AutogradContext *ctx, const Tensor &x_in, const Tensor &logits, const Tensor &sel_in, const Conv *conv, int64_t flag)
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &logits, const Tensor &sel, const Conv *conv, int64_t flag)
     {
-        const Tensor x = x_in.contiguous(), sel = sel_in.contiguous();
-        const clg_conv_geom g = conv->geom(x, logits.size(0));
-        const Tensor keep = bytes(x, clg_convblock_bin_ctx_bytes(CLG_F32, &g));
-        const auto s = pooled(g);
-        Tensor y = floats(x, s), taps = at::empty(s, x.options().dtype(at::kShort));
-        check(clg_convblock_bin_forward(CLG_F32, &g, x.data_ptr(), logits.data_ptr(), static_cast<const int32_t *>(sel.data_ptr()), y.data_ptr(),
-                                        static_cast<uint16_t *>(taps.data_ptr()), keep.data_ptr(), CLG_FWD_W_LOGITS,
-                                        reinterpret_cast<int32_t *>(flag), stream_of(x)));
-        ctx->save_for_backward({taps, keep});                        // x itself is not needed again
+        Tensor taps, keep;
+        const Tensor y = binary_forward(x, logits, sel, *conv, flag, taps, keep);
+        ctx->save_for_backward({taps, keep});
         ctx->saved_data["conv"] = conv->saved(x.sizes().vec());
         return y;
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
         const auto saved = ctx->get_saved_variables();
-        const Tensor &taps = saved[0], &keep = saved[1], gy = grads[0].contiguous();
-        TORCH_CHECK(gy.is_cuda(), "grad_y must be a CUDA tensor");
-        TORCH_CHECK(gy.device() == taps.device(), "all tensors must be on one device, got ", taps.device(), " and ", gy.device());
-        need(gy, gy, "grad_y", taps.sizes());
         const auto ints = ctx->saved_data["conv"].toIntVector();
-        const Conv cv = Conv::from(ints);
-        const std::vector<int64_t> xs(ints.begin() + 6, ints.end());
-        const int64_t c = gy.size(1);
-        const clg_conv_geom g = {(int32_t)xs[0], (int32_t)xs[1], (int32_t)xs[2], (int32_t)xs[3], (int32_t)c, (int32_t)cv.sh, (int32_t)cv.sw,
-                                 (int32_t)cv.ph, (int32_t)cv.pw, (int32_t)cv.kh, (int32_t)cv.kw};
-        const bool need_x = ctx->needs_input_grad(0), need_l = ctx->needs_input_grad(1);
-        Tensor gx, gl, scratch;
-        if (need_x) gx = floats(gy, xs);
-        if (need_l) {
-            gl = floats(gy, {c, 7, 16});
-            scratch = bytes(gy, clg_convblock_bin_backward_scratch_bytes(CLG_F32, &g));
-        }
-        if (need_x || need_l)
-            check(clg_convblock_bin_backward(CLG_F32, &g, gy.data_ptr(), static_cast<const uint16_t *>(taps.data_ptr()), keep.data_ptr(), ptr(gx),
-                                             ptr(gl), CLG_BWD_WRT_LOGITS, ptr(scratch), stream_of(gy)));
-        return {gx, gl, Tensor(), Tensor(), Tensor()};
+        const auto g = binary_backward(saved[0], saved[1], Conv::from(ints), at::IntArrayRef(ints).slice(6), grads[0], ctx->needs_input_grad(0),
+                                       ctx->needs_input_grad(1));
+        return {g.first, g.second, Tensor(), Tensor(), Tensor()};
     }
 };
 Tensor binary_block(const Tensor &x, const Tensor &logits, const Tensor &sel, std::array<int64_t, 6> conv, int64_t flag)
@@ -313,19 +347,43 @@ struct TreeArgs {
     int64_t roots, k;
     double tau;
 };
+const int32_t *i32(const Tensor &v) { return static_cast<const int32_t *>(v.data_ptr()); }
+float *f32(const Tensor &v) { return static_cast<float *>(ptr(v)); }
+// x feature-major -> class sums; coef and (need_l) probs are kept
+Tensor trees_forward(const Tensor &x, const Tensor &l0, const Tensor &l1, const Tensor &l2, const TreeArgs &t, bool need_l, Tensor &coef, Tensor &probs)
+{
+    const int64_t in_dim = x.size(0), batch = x.size(1);
+    coef = floats(x, {t.roots, 28});
+    if (need_l) probs = floats(x, {7 * t.roots, 16});                 // (the logits may be updated between forward and backward)
+    check(clg_fc_tree_fold(l0.data_ptr<float>(), l1.data_ptr<float>(), l2.data_ptr<float>(), i32(t.ids), f32(coef), f32(probs), t.roots, 0, stream_of(x)));
+    const int64_t elems = clg_fc_tree_partial_elems(t.roots, t.k, batch, batch);
+    Tensor out = floats(x, {batch, t.k}), partial = floats(x, {elems < 0 ? 0 : elems});
+    check(clg_fc_tree_forward(f32(x), i32(t.rows), f32(coef), f32(partial), f32(out), in_dim, t.roots, t.k, batch, batch, t.tau, stream_of(x)));
+    return out;
+}
+// -> gradients of x and of the three layers' logits, those that are wanted.  tables: rows, pos, slot
+std::array<Tensor, 4> trees_backward(const Tensor &x, const Tensor &start, const Tensor &coef, const Tensor &probs, const std::vector<Tensor> &tables, int64_t k,
+                                     double tau, const Tensor &grad, std::array<bool, 4> wanted)
+{
+    const int64_t in_dim = x.size(0), batch = x.size(1), roots = coef.size(0);
+    const Tensor go = grad.contiguous();
+    need(go, x, "grad_out", {batch, k});
+    std::array<Tensor, 4> g;
+    if (wanted[0]) g[0] = at::empty_like(x);
+    const int64_t neurons[3] = {4 * roots, 2 * roots, roots};
+    for (int i = 0; i < 3; ++i)
+        if (wanted[1 + i]) g[1 + i] = floats(x, {neurons[i], 16});
+    const int64_t rows = g[0].defined() ? 8 * roots * batch : 0;
+    const Tensor scratch = floats(x, {rows + 28 * roots});           // operand gradients, then sums
+    check(clg_fc_tree_backward(f32(x), i32(tables[0]), i32(tables[1]), i32(tables[2]), f32(coef), f32(go), f32(probs), f32(g[1]), f32(g[2]), f32(g[3]),
+                               f32(scratch), f32(scratch) + rows, idx(start), f32(g[0]), in_dim, roots, k, batch, batch, tau, stream_of(x)));
+    return g;
+}
 struct Trees : torch::autograd::Function<Trees> {
     static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &l0, const Tensor &l1, const Tensor &l2, const TreeArgs *t, bool need_l)
     {
-        const int64_t in_dim = x.size(0), batch = x.size(1);
-        const auto i32 = [](const Tensor &v) { return static_cast<const int32_t *>(v.data_ptr()); };
-        Tensor coef = floats(x, {t->roots, 28}), probs;
-        if (need_l) probs = floats(x, {7 * t->roots, 16});            // (the logits may be updated between forward and backward)
-        check(clg_fc_tree_fold(l0.data_ptr<float>(), l1.data_ptr<float>(), l2.data_ptr<float>(), i32(t->ids), coef.data_ptr<float>(),
-                               static_cast<float *>(ptr(probs)), t->roots, 0, stream_of(x)));
-        const int64_t elems = clg_fc_tree_partial_elems(t->roots, t->k, batch, batch);
-        Tensor out = floats(x, {batch, t->k}), partial = floats(x, {elems < 0 ? 0 : elems});
-        check(clg_fc_tree_forward(x.data_ptr<float>(), i32(t->rows), coef.data_ptr<float>(), partial.data_ptr<float>(), out.data_ptr<float>(), in_dim,
-                                  t->roots, t->k, batch, batch, t->tau, stream_of(x)));
+        Tensor coef, probs;
+        const Tensor out = trees_forward(x, l0, l1, l2, *t, need_l, coef, probs);
         variable_list saved = {x, t->start, coef, probs};
         saved.insert(saved.end(), t->wiring.begin(), t->wiring.end());
         ctx->save_for_backward(std::move(saved));
@@ -337,24 +395,10 @@ struct Trees : torch::autograd::Function<Trees> {
     static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
         const auto saved = ctx->get_saved_variables();
-        const Tensor &x = saved[0], &start = saved[1], &coef = saved[2], &probs = saved[3];
-        const auto tables = ctx->saved_data["tables"].toTensorVector();
-        const int64_t k = ctx->saved_data["k"].toInt(), in_dim = x.size(0), batch = x.size(1), roots = coef.size(0);
-        const auto i32 = [](const Tensor &v) { return static_cast<const int32_t *>(v.data_ptr()); };
-        const auto f32 = [](const Tensor &v) { return static_cast<float *>(ptr(v)); };
-        const Tensor go = grads[0].contiguous();
-        need(go, x, "grad_out", {batch, k});
-        Tensor gx, g[3];
-        if (ctx->needs_input_grad(0)) gx = at::empty_like(x);
-        const int64_t neurons[3] = {4 * roots, 2 * roots, roots};
-        for (int i = 0; i < 3; ++i)
-            if (ctx->needs_input_grad(1 + i)) g[i] = floats(x, {neurons[i], 16});
-        const int64_t rows = gx.defined() ? 8 * roots * batch : 0;
-        const Tensor scratch = floats(x, {rows + 28 * roots});       // operand gradients, then sums
-        check(clg_fc_tree_backward(f32(x), i32(tables[0]), i32(tables[1]), i32(tables[2]), f32(coef), f32(go), f32(probs), f32(g[0]), f32(g[1]),
-                                   f32(g[2]), f32(scratch), f32(scratch) + rows, idx(start), f32(gx), in_dim, roots, k, batch, batch,
-                                   ctx->saved_data["tau"].toDouble(), stream_of(x)));
-        return {gx, g[0], g[1], g[2], Tensor(), Tensor()};
+        const auto g = trees_backward(saved[0], saved[1], saved[2], saved[3], ctx->saved_data["tables"].toTensorVector(), ctx->saved_data["k"].toInt(),
+                                      ctx->saved_data["tau"].toDouble(), grads[0],
+                                      {ctx->needs_input_grad(0), ctx->needs_input_grad(1), ctx->needs_input_grad(2), ctx->needs_input_grad(3)});
+        return {g[0], g[1], g[2], g[3], Tensor(), Tensor()};
     }
 };
 Tensor trees(const Tensor &x, const Tensor &l0, const Tensor &l1, const Tensor &l2, const Tensor &start, std::vector<Tensor> wiring, const Tensor &rows,
@@ -365,6 +409,120 @@ Tensor trees(const Tensor &x, const Tensor &l0, const Tensor &l1, const Tensor &
     need(l2, x, "weights", {roots, 16});
     const TreeArgs t{start, rows, pos, ids, slot, std::move(wiring), roots, k, tau};
     return Trees::apply(x, l0, l1, l2, &t, at::GradMode::is_enabled() && (l0.requires_grad() || l1.requires_grad() || l2.requires_grad()));
+}
+
+// ---- a network: blocks, flattening, trees -------------------------------------------------------------------------------------
+// One node for what the modules' nodes do one after the other, with the same calls of the library: a step of a small network is bound by the
+// host, which takes longer from node to node (module calls in Python, views, the engine's queue) than for the launches of one.  MNIST
+// topology, k = 32, 100 images, a step with its loss: 344 -> 285 us; CIFAR, 256 images: 352 -> 330, the time of its kernels.
+struct NetBlock {
+    Tensor sel, plan;
+    Conv conv;
+    int64_t signature, flag;                                          // flag: not 0 for a block on 0/1 inputs, which has no plan
+    bool fm;
+};
+struct NetArgs {
+    std::vector<NetBlock> blocks;
+    TreeArgs trees;
+    std::vector<bool> wanted;                                         // of x and every logits
+};
+struct Network : torch::autograd::Function<Network> {
+    // per block and for the trees in front of their wiring: as many saved tensors
+    static constexpr int kEach = BlockState::kTensors, kTrees = 4;
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, at::TensorList logits, const NetArgs *a)
+    {
+        const size_t n = a->blocks.size();
+        variable_list saved;
+        std::vector<int64_t> ints;
+        std::vector<Tensor> plans;
+        Tensor h = x;
+        bool some = a->wanted[0], fm = false;                         // whether a gradient is wanted of what the block takes
+        for (size_t i = 0; i < n; ++i) {
+            const NetBlock &b = a->blocks[i];
+            BlockState state;
+            const auto shape = h.sizes().vec();
+            fm = b.fm;
+            if (b.flag != 0) {
+                fm = false;
+                h = binary_forward(h, logits[i], b.sel, b.conv, b.flag, state.x, state.probs);
+            } else {
+                h = block_forward(h, logits[i], b.sel, b.conv, fm, b.signature, nullptr, some, state);
+            }
+            state.save(saved);
+            const std::vector<int64_t> own{b.conv.sh, b.conv.sw, b.conv.ph, b.conv.pw, b.conv.kh, b.conv.kw, shape[0], shape[1], shape[2], shape[3],
+                                           b.flag != 0, b.signature, fm};
+            ints.insert(ints.end(), own.begin(), own.end());
+            plans.push_back(b.plan);
+            some = some || a->wanted[1 + i];
+        }
+        // features [c h w, n]
+        const int64_t batch = x.size(0);
+        h = fm ? h.view({-1, batch}) : transposed(h.view({batch, -1}));
+        const bool need_l = a->wanted[1 + n] || a->wanted[2 + n] || a->wanted[3 + n];
+        Tensor coef, probs;
+        const Tensor out = trees_forward(h, logits[n], logits[n + 1], logits[n + 2], a->trees, need_l, coef, probs);
+        saved.insert(saved.end(), {h, a->trees.start, coef, probs});
+        saved.insert(saved.end(), a->trees.wiring.begin(), a->trees.wiring.end());
+        ctx->save_for_backward(std::move(saved));
+        ctx->saved_data["blocks"] = std::move(ints);
+        ctx->saved_data["plans"] = std::move(plans);
+        ctx->saved_data["tables"] = std::vector<Tensor>{a->trees.rows, a->trees.pos, a->trees.slot};
+        ctx->saved_data["k"] = a->trees.k;
+        ctx->saved_data["tau"] = a->trees.tau;
+        return out;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads)
+    {
+        constexpr int kInts = 13;
+        const auto saved = ctx->get_saved_variables();
+        const auto ints = ctx->saved_data["blocks"].toIntVector();
+        const auto plans = ctx->saved_data["plans"].toTensorVector();
+        const size_t n = plans.size();
+        const auto wanted = [&](size_t i) { return ctx->needs_input_grad(i); };
+        std::vector<bool> below(n + 1);                               // whether a gradient is wanted of what block i, or the trees, take
+        below[0] = wanted(0);
+        for (size_t i = 0; i < n; ++i) below[i + 1] = below[i] || wanted(1 + i);
+        variable_list out(1 + n + 3 + 1);
+        const Tensor *t = saved.data() + n * kEach;
+        auto g = trees_backward(t[0], t[1], t[2], t[3], ctx->saved_data["tables"].toTensorVector(), ctx->saved_data["k"].toInt(),
+                                ctx->saved_data["tau"].toDouble(), grads[0], {below[n], wanted(1 + n), wanted(2 + n), wanted(3 + n)});
+        for (size_t i = 0; i < 3; ++i) out[1 + n + i] = g[1 + i];
+        Tensor h = g[0];
+        for (size_t i = n; i-- > 0 && (below[i] || wanted(1 + i));) {
+            const int64_t *own = ints.data() + i * kInts;
+            const Conv conv{own[0], own[1], own[2], own[3], own[4], own[5]};
+            const Tensor *kept = saved.data() + i * kEach;
+            const bool binary = own[10] != 0, fm = own[12] != 0;
+            if (i + 1 == n) {                                         // from [features, batch]
+                const auto s = pooled({(int32_t)own[6], (int32_t)own[7], (int32_t)own[8], (int32_t)own[9], (int32_t)(binary ? kept[0].size(1) : kept[2].size(0)),
+                                       (int32_t)own[0], (int32_t)own[1], (int32_t)own[2], (int32_t)own[3], (int32_t)own[4], (int32_t)own[5]});
+                h = fm ? h.view({s[1], s[2], s[3], s[0]}).permute({3, 0, 1, 2}) : transposed(h).view(s);
+            }
+            const auto gi = binary ? binary_backward(kept[0], kept[1], conv, at::IntArrayRef(own + 6, 4), h, below[i], wanted(1 + i))
+                                   : block_backward(BlockState::from(kept), conv, fm, plans[i], own[11], h, below[i], wanted(1 + i));
+            h = gi.first;
+            out[1 + i] = gi.second;
+        }
+        if (below[0]) out[0] = h;
+        return out;
+    }
+};
+// blocks: selection, stride / padding / kernel, plan, its signature, feature-major output, flag; logits of the blocks and of the three layers
+using NetBlockTuple = std::tuple<Tensor, std::array<int64_t, 6>, Tensor, int64_t, bool, int64_t>;
+Tensor network(const Tensor &x, const std::vector<Tensor> &logits, const std::vector<NetBlockTuple> &blocks, const Tensor &start, std::vector<Tensor> wiring,
+               const Tensor &rows, const Tensor &pos, const Tensor &ids, const Tensor &slot, int64_t roots, int64_t k, double tau)
+{
+    const size_t n = blocks.size();
+    TORCH_CHECK(n > 0 && logits.size() == n + 3, "logits of ", n, " blocks and three layers are needed, got ", logits.size());
+    NetArgs a{{}, {start, rows, pos, ids, slot, std::move(wiring), roots, k, tau}, {x.requires_grad()}};
+    for (size_t i = 0; i < n; ++i) {
+        const auto &[sel, cv, plan, signature, fm, flag] = blocks[i];
+        need(logits[i], x, "weights", {sel.size(0), 7, 16});
+        a.blocks.push_back({sel, plan, {cv[0], cv[1], cv[2], cv[3], cv[4], cv[5]}, signature, flag, fm});
+    }
+    for (int i = 0; i < 3; ++i) need(logits[n + i], x, "weights", {(4 >> i) * roots, 16});
+    for (const Tensor &l : logits) a.wanted.push_back(l.requires_grad());
+    return Network::apply(x, at::TensorList(logits), &a);
 }
 
 // grad_fn of a node's output in Python: a type of the name that the Python function's node has
@@ -387,9 +545,11 @@ PYBIND11_MODULE(_nodes, m)
     name_node<Block>("_FullConvLogicLogitsFunctionBackward");
     name_node<BinaryBlock>("_FullConvLogicBinaryFunctionBackward");
     name_node<Trees>("_TreeFunctionBackward");
+    name_node<Network>("_TreeNetworkFunctionBackward");
     m.def("feature_major", &feature_major, no_gil);
     m.def("fc_layer", &fc_layer, no_gil);
     m.def("block", &block, no_gil);
     m.def("binary_block", &binary_block, no_gil);
     m.def("trees", &trees, no_gil);
+    m.def("network", &network, no_gil);
 }

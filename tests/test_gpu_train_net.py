@@ -1,0 +1,139 @@
+"""A network's training step as one autograd node (convlogic/train_net.py) against its modules one after the other: outputs and gradients bit
+for bit, for every set of wanted gradients; and what is left to the modules."""
+import copy
+
+import pytest
+import torch
+
+import convlogic_amd as C
+from convlogic_amd.convlogic import train_net
+from tests.gpu_util import DEV
+
+pytestmark = pytest.mark.gpu
+
+
+def network(topology, k, channels):
+    torch.manual_seed(k)
+    model = C.ConvLogicCifarModel(k_param=k, input_channels=channels) if topology == "cifar" else C.ConvLogicMnistModel(k_param=k, input_channels=channels)
+    return model.to(DEV), 32 if topology == "cifar" else 28
+
+
+@pytest.fixture
+def at_once(monkeypatch):
+    calls, train = [], train_net.train
+
+    def spy(*a):
+        out = train(*a)
+        calls.append(out is not None)
+        return out
+    monkeypatch.setattr(train_net, "train", spy)
+    return calls
+
+
+def step(model, x, gy, tensors, by_modules):
+    model.prefold = not by_modules                                    # (any other value than True calls the modules)
+    y = model(x)
+    wanted = [t for t in tensors if t.requires_grad]
+    got = iter(torch.autograd.grad(y, wanted, gy))
+    return y, [next(got) if t.requires_grad else None for t in tensors]
+
+
+# batches below and from the 32 samples on from which the last CIFAR block writes feature-major; channels too many for the binary first block's
+# lists to be short, the first block without its promise
+@pytest.mark.parametrize("topology,k,channels,batch,binary", [("cifar", 8, 3, 5, True), ("cifar", 8, 9, 64, True), ("cifar", 16, 3, 33, False),
+                                                              ("mnist", 8, 1, 70, True), ("mnist", 9, 2, 1, True), ("mnist", 10, 1, 31, False)])
+def test_the_same_as_the_modules(at_once, topology, k, channels, batch, binary):
+    model, side = network(topology, k, channels)
+    model.network[0].binary_input = binary
+    x = (torch.rand(batch, channels, side, side, device=DEV) < 0.5).float()
+    params = list(model.parameters())
+    gy = torch.randn(batch, 10, device=DEV)
+    n = len(params)
+    frozen_sets = [set(), set(range(n)), *({i} for i in range(n)), set(range(n - 3)), set(range(n - 3, n)), {0, 1}, {n - 2, n - 1}]
+    for need_x in (False, True):
+        for frozen in frozen_sets:
+            if not need_x and len(frozen) == n:
+                continue
+            x.requires_grad_(need_x)
+            for i, p in enumerate(params):
+                p.requires_grad_(i not in frozen)
+            at_once.clear()
+            y, grads = step(model, x, gy, [x, *params], False)
+            assert at_once == [True]
+            y0, grads0 = step(model, x, gy, [x, *params], True)
+            assert at_once == [True] and torch.equal(y, y0)
+            for a, b in zip(grads, grads0, strict=True):
+                assert (a is None) == (b is None) and (a is None or (torch.equal(a, b) and a.stride() == b.stride()))
+
+
+def test_what_autograd_offers_around_the_node(at_once):
+    model, side = network("mnist", 8, 1)
+    x = (torch.rand(40, 1, side, side, device=DEV) < 0.5).float()
+    params = list(model.parameters())
+    want = torch.autograd.grad(model(x).sum(), params)
+    moved = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: moved.append(1) or t.cpu(), lambda t: t.to(DEV)):
+        got = torch.autograd.grad(model(x).sum(), params)
+    assert moved and all(torch.equal(a, b) for a, b in zip(got, want))
+    again = torch.utils.checkpoint.checkpoint(model, x, use_reentrant=False)
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(again.sum(), params), want))
+    y = model(x)
+    assert all(torch.equal(a, b) for _ in range(2) for a, b in zip(torch.autograd.grad(y.sum(), params, retain_graph=True), want))
+    y.sum().backward()
+    with pytest.raises(RuntimeError, match="second time"):
+        y.sum().backward()
+    y = model(x)
+    with torch.no_grad():
+        for p in params:
+            p.data.mul_(2)                                            # an optimizer's update between the passes
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(y.sum(), params), want))
+    y = model(x)
+    model.network[1].selection.add_(0)                                # the wiring written in between
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.sum().backward()
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(model)(torch.zeros(2, 4, 1, side, side, device=DEV))
+    assert all(at_once[:-1])
+
+
+def test_what_the_modules_do_for_themselves_stays_theirs(at_once):
+    model, side = network("mnist", 8, 1)
+    x = (torch.rand(20, 1, side, side, device=DEV) < 0.5).float()
+    want = model(x).detach()
+    assert at_once == [True]
+    seen = []
+    for module in (model.network[0], model.network[2], model.network[3]):
+        for register in (module.register_forward_hook, module.register_full_backward_hook):
+            at_once.clear()
+            handle = register(lambda *a: seen.append(1))
+            y = model(x)
+            y.sum().backward()
+            assert torch.equal(y, want) and seen and True not in at_once
+            handle.remove()
+            seen.clear()
+
+    def change(f):
+        other = copy.deepcopy(model)
+        f(other)
+        at_once.clear()
+        y = other(x)
+        assert True not in at_once and torch.equal(y, want)
+    change(lambda m: setattr(m, "prefold", "always"))
+    change(lambda m: setattr(m.network[1], "grad_factor", 2.0))
+    change(lambda m: setattr(m.network[1], "forward", m.network[1].forward))
+    at_once.clear()
+    assert torch.equal(model(x.expand(20, 1, side, side).flip(0).flip(0).transpose(2, 3).contiguous().transpose(2, 3)), want) and True not in at_once
+    with pytest.raises(RuntimeError):
+        model(x[:, :, 1:])
+    large, side = network("mnist", 128, 1)                            # more logits than small networks have
+    at_once.clear()
+    large((torch.rand(2, 1, side, side, device=DEV) < 0.5).float())
+    assert True not in at_once
+
+
+def test_a_broken_promise_of_binary_inputs_is_reported():
+    model, side = network("mnist", 8, 1)
+    model(torch.rand(4, 1, side, side, device=DEV))
+    torch.cuda.synchronize()
+    with pytest.raises(RuntimeError, match="0 and 1"):
+        model(torch.zeros(4, 1, side, side, device=DEV))
