@@ -52,10 +52,24 @@ namespace {
 // ---------------------------------------------------------------------------------------------
 // input gradient
 // ---------------------------------------------------------------------------------------------
+// kHitWide for a kernel whose taps (its eight at sq) are in more than two channels
+__device__ __forceinline__ int wide_kernel(const int32_t *__restrict__ sq, int cin)
+{
+    const int ch0 = tap_channel(sq[0], cin);
+    int ch1 = ch0;
+    bool wide = false;
+#pragma unroll
+    for (int t = 1; t < 8; ++t) {
+        const int ch = tap_channel(sq[t], cin);
+        wide |= ch != ch0 && ch1 != ch0 && ch != ch1;
+        ch1 = ch1 == ch0 ? ch : ch1;
+    }
+    return wide ? kHitWide : 0;
+}
 // Scratch of the input-gradient kernels, written by the preparation launches:
 //   folded [c][7][4]   coefficients (ab, a, b, one) of every gate
 //   count  [cin][2]    (number of kernels that read input channel ch, offset of its list in hits)
-//   hits               those kernels in increasing order, entry = kernel | tap mask << 16
+//   hits               those kernels in increasing order, entry = kernel | tap mask << 16 (| kHitWide)
 // (the reverse map "input channel -> kernels and taps reading it", built in a fixed order).  Small maps
 // are dense, hits[cin][c], filled by one wavefront per channel.  Large ones (cin * c above 2^20) are
 // compressed: lists back to back (at most 8 c entries), filled through integer atomics and then sorted per
@@ -130,7 +144,7 @@ __global__ __launch_bounds__(256) void convblock_prepare_kernel(const T *__restr
         const uint64_t vote = __ballot(mask != 0);
         if (mask) {
             const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(vote >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)vote, 0));
-            hits[(int64_t)ch * C + n + before] = c | (mask << 16);
+            hits[(int64_t)ch * C + n + before] = c | (mask << 16) | wide_kernel(sel + (int64_t)c * 8, cin);
         }
         n += __popcll(vote);
     }
@@ -203,7 +217,7 @@ __global__ __launch_bounds__(256) void hits_fill_kernel(const int32_t *__restric
         const int mask = first_use_mask(sq, t, cin);
         if (mask) {
             const int ch = tap_channel(sq[t], cin);
-            unsorted[count[2 * ch + 1] + atomicAdd(cursor + ch, 1)] = c | (mask << 16);
+            unsorted[count[2 * ch + 1] + atomicAdd(cursor + ch, 1)] = c | (mask << 16) | wide_kernel(sq, cin);
         }
     }
 }
@@ -1472,10 +1486,35 @@ int clg_allow_lds(const void *kernel, size_t bytes, const char *name)
     return CLG_OK;
 }
 
-static int64_t backward_x_scratch_bytes(const char *name, int dtype, const clg_conv_geom *gg, bool long_lists)
+// 4x4 images with one sample per lane (conv_small.hip): scratch = prepare tables | tap gradients
+static bool backward_4x4_wanted(const Geom &g)
+{
+    const char *e = clg_knob(K_BWD_4X4);
+    return clg_convblock_is_4x4(g) && g.c <= 65535 && (!e || atoi(e) != 0);
+}
+
+// A planned float32 call takes both gradients from planes staged two at a time (conv_pair_grad.hip) as long as the gradient planes between its two
+// kernels stay in the last-level cache of 256 MB.  Forward and backward of a block against the kernels below, 180 shapes of 6x6 to 20x20
+// images, 4 to 512 channels with lists of 2 to 16 kernels, 16 to 256 samples: 0.95 to 1.84 times as fast at up to 150 MB of planes, 21 of them
+// below 1.05 (lists of 2), 1.1 to 1.5 in between ([256,32,16,16] -> 128 70.7 -> 63.1 us, [16,32,6,6] -> 256 45 -> 25,
+// [64,512,12,12] -> 2048 184 -> 156); 0.82 to 1.07 at 256 MB and more ([128,1024,16,16] -> 4096 752 -> 853).  Fewer than four channels are
+// the tiled kernel's, whose wavefronts share a channel; lists longer than 16 on the average go by their length (lists_are_long).
+static bool backward_planes_wanted(const Geom &g, int dtype, PairPlan *p)
+{
+    if (dtype != CLG_F32 || backward_4x4_wanted(g) || !clg_plan_pair(g, 4, p, false) || !clg_pair_grad_w_wanted(g, *p) || !clg_pair_planes_fit(g, *p))
+        return false;
+    if (const char *e = clg_knob(K_BWDX_PLANES)) return atoi(e) != 0;
+    if (clg_knob(K_BWDX_DIRECT) != nullptr) return false;            // (one of the other kernels is asked for)
+    return g.cin >= 4 && g.c >= g.cin && g.c <= 8 * (int64_t)g.cin && clg_pair_planes_bytes(g) <= (size_t)160 << 20;
+}
+static size_t backward_planes_off(const Geom &g) { return (bwd_scratch_layout(g, 4, 1).total + 255) & ~(size_t)255; }
+
+static int64_t backward_x_scratch_bytes(const char *name, int dtype, const clg_conv_geom *gg, bool long_lists, bool planned = false)
 {
     Geom g;
     if (clg_convblock_check(gg, &g, dtype, name)) return -1;
+    PairPlan pp;
+    if (planned && backward_planes_wanted(g, dtype, &pp)) return (int64_t)(backward_planes_off(g) + clg_pair_planes_bytes(g));
     TilePlan p;
     int se = 0;
     const BwdXMode mode = choose_backward_x(g, elem_size(dtype), &p, &se, long_lists);
@@ -1620,12 +1659,6 @@ extern "C" int clg_convblock_backward_w(int dtype, const clg_conv_geom *gg, cons
                                      "clg_convblock_backward_w");
 }
 
-// 4x4 images with one sample per lane (conv_small.hip): scratch = prepare tables | tap gradients
-static bool backward_4x4_wanted(const Geom &g)
-{
-    const char *e = clg_knob(K_BWD_4X4);
-    return clg_convblock_is_4x4(g) && g.c <= 65535 && (!e || atoi(e) != 0);
-}
 static size_t backward_4x4_tg_off(const Geom &g, int dtype) { return (bwd_scratch_layout(g, elem_size(dtype), 1).total + 255) & ~(size_t)255; }
 
 static int convblock_backward_4x4(int dtype, const Geom &g, const void *grad_y, const void *x, const void *w, const int32_t *selection,
@@ -1646,9 +1679,9 @@ static int convblock_backward_4x4(int dtype, const Geom &g, const void *grad_y, 
                                       tb.count, tb.hits, grad_x, st, name);
 }
 
-static int64_t backward_scratch_bytes(const char *name, int dtype, const clg_conv_geom *gg, bool long_lists)
+static int64_t backward_scratch_bytes(const char *name, int dtype, const clg_conv_geom *gg, bool long_lists, bool planned = false)
 {
-    const int64_t a = backward_x_scratch_bytes(name, dtype, gg, long_lists), b = clg_convblock_backward_w_scratch_bytes(dtype, gg);
+    const int64_t a = backward_x_scratch_bytes(name, dtype, gg, long_lists, planned), b = clg_convblock_backward_w_scratch_bytes(dtype, gg);
     if (a < 0 || b < 0) return -1;
     int64_t total = ((a + 255) & ~255ll) + b;
     Geom g;
@@ -1665,7 +1698,7 @@ extern "C" int64_t clg_convblock_backward_scratch_bytes(int dtype, const clg_con
 }
 extern "C" int64_t clg_convblock_backward_planned_scratch_bytes(int dtype, const clg_conv_geom *gg, int64_t signature)
 {
-    return backward_scratch_bytes("clg_convblock_backward_planned_scratch_bytes", dtype, gg, (signature & 1) != 0);
+    return backward_scratch_bytes("clg_convblock_backward_planned_scratch_bytes", dtype, gg, (signature & 1) != 0, true);
 }
 
 extern "C" int clg_convblock_backward(int dtype, const clg_conv_geom *gg, const void *grad_y, const void *x, const void *w,
@@ -1737,14 +1770,20 @@ struct PlanInfo {
     int rs, chs;
     size_t total;
     int64_t signature;
+    bool planes;                                                     // both gradients by `pair`
+    PairPlan pair;
 };
 // long_lists is the lowest bit of the signature (0 where it makes no difference), so a planned call finds the kernels again.
 PlanInfo plan_info(const Geom &g, int dtype, bool long_lists)
 {
     PlanInfo pi;
     const int elem = elem_size(dtype);
-    int mode = 3, rs = 0, chs = 0;                                    // 3: one sample per lane on 4x4 images
-    if (!backward_4x4_wanted(g)) {
+    int mode = 3, rs = 0, chs = 0;                                    // 3: one sample per lane on 4x4 images, 4: gradient planes
+    pi.planes = backward_planes_wanted(g, dtype, &pi.pair);
+    if (pi.planes) {
+        mode = 4;
+        long_lists = false;
+    } else if (!backward_4x4_wanted(g)) {
         TilePlan p;
         int se = 0;
         mode = (int)choose_backward_x(g, elem, &p, &se);
@@ -1822,9 +1861,10 @@ extern "C" int clg_convblock_plan(int dtype, const clg_conv_geom *gg, const int3
 // One sample of the padded copy the planned backward pass reads when its input gradient is the direct kernel, else 0.
 int64_t clg_convblock_backward_padded_sample_elems(int dtype, const Geom &g)
 {
-    if (backward_4x4_wanted(g)) return 0;
     TilePlan p;
+    PairPlan pp;
     int se = 0;
+    if (backward_4x4_wanted(g) || backward_planes_wanted(g, dtype, &pp)) return 0;
     return choose_backward_x(g, elem_size(dtype), &p, &se) == kBwdXDirect ? se : 0;
 }
 
@@ -1855,10 +1895,21 @@ static int backward_planned_impl(const char *name, int dtype, const clg_conv_geo
         g.y_fm = fm ? 1 : 0;
         return convblock_backward_4x4(dtype, g, grad_y, x, w, selection, argmax, grad_x, grad_w, scratch, stream, probs, name, &pv);
     }
-    const int64_t a = backward_x_scratch_bytes(name, dtype, gg, long_lists);
+    const int64_t a = backward_x_scratch_bytes(name, dtype, gg, long_lists, true);
     if (a < 0) return CLG_EINVAL;
     SharedPad shared;
     void *w_scratch = reinterpret_cast<unsigned char *>(scratch) + ((a + 255) & ~255ll);
+    if (grad_x != nullptr && pi.planes) {
+        hipStream_t st = clg_stream(stream);
+        BwdTables tb;
+        if (int e = prepare_tables<float>(g, pi.lay, 0, 0, w, selection, scratch, st, no_pad_job<float>(), &pv, &tb)) return e;
+        const int nb = clg_pair_grad_w_parts(g, pi.pair);
+        float *planes = reinterpret_cast<float *>(reinterpret_cast<unsigned char *>(scratch) + backward_planes_off(g));
+        if (int e = clg_pair_grads(g, pi.pair, nb, (const float *)grad_y, (const float *)x, (const float *)tb.folded, selection, argmax, tb.count, tb.hits,
+                                   planes, (float *)w_scratch, (float *)grad_x, st, name))
+            return e;
+        return clg_launch_reduce_coef(CLG_F32, w_scratch, grad_w, g.c, nb, 7, st, name, probs);
+    }
     if (grad_x != nullptr)
         if (int e = convblock_backward_x_impl(dtype, gg, grad_y, x, w, selection, argmax, grad_x, scratch, stream, &shared, w_scratch, &pv,
                                               long_lists))

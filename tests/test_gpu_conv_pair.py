@@ -8,7 +8,7 @@ import torch
 import convlogic_amd as C
 from convlogic_amd.hip import convlogic_hip as H
 from oracle import convlogic_oracle as O
-from tests.gpu_util import DEV, check_pool_route, set_knobs
+from tests.gpu_util import DEV, assert_grad_close, check_pool_route, set_knobs
 
 pytestmark = pytest.mark.gpu
 # n, cin, h, w, cout, kernel, padding
@@ -167,6 +167,33 @@ def test_weight_gradient_against_float64_at_the_same_arg_max(n, cin, h, w, c, k,
         assert err.max() <= 2 * (gw0.double() - ref).abs().max() + 1e-6 * gy.abs().max()
         if wide and rep == 1:
             break
+
+
+# groups that overlap, rows that no 16-byte piece fits, more and fewer cells than lanes, 8 kernels of a list at a time and the rest
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("n,cin,h,w,c", [(9, 4, 8, 8, 32), (37, 12, 6, 6, 40), (1, 5, 16, 16, 20), (3, 6, 18, 20, 30), (21, 7, 10, 14, 9), (5, 4, 2, 4, 50)])
+def test_both_gradients_by_planes_against_float64(n, cin, h, w, c, wide, monkeypatch):
+    torch.manual_seed(n * 100 + h)
+    layer = C.ConvLogicLayer(cin, c, complete=True, implementation="cuda").to(DEV)
+    sel, probs, geo = _selection(layer, wide), torch.softmax(layer.weights.detach(), -1), (1, 1, 1, 1)
+    sel[0] = sel[0, 0] & ~0xFFFF | sel[0] & 0xFFFF                    # a kernel with all taps in one channel
+    x = torch.randn(n, cin, h, w, device=DEV)
+    y, am = H.full_convlogic_forward(x, probs, sel, *geo, 3, 3)
+    gy = torch.randn_like(y)
+    ref, _ = H.full_convlogic_backward(gy.double(), x.double(), probs.double(), am, sel, *geo)
+    got = []
+    for planes in ("0", "1"):
+        set_knobs(monkeypatch, CLG_BWDX_PLANES=planes)
+        plan = H.make_backward_plan(x, c, sel, *geo, 3, 3)
+        got.append([H.full_convlogic_backward_planned(gy, x, probs, None, am, sel, *plan, *geo, wrt_logits=False) for _ in range(2)])
+    for a, b in got:
+        assert all(torch.equal(u, v) for u, v in zip(a, b))
+    (gx0, gw0), (gx1, gw1) = got[0][0], got[1][0]
+    # the same terms with the same roundings, and as many additions in another order; the weight gradient is the same kernel's where it
+    # was taken before, else sums of as many terms
+    e0, e1 = ((g.double() - ref).norm().item() for g in (gx0, gx1))
+    assert e1 <= 1.25 * e0 + 2.0**-24 * ref.norm().item()
+    assert_grad_close(gw1, gw0, rel=1e-5)
 
 
 @pytest.mark.parametrize("n,cin,side,c", [(1000, 40, 8, 2000), (128, 64, 16, 2048), (300, 48, 16, 600)])
