@@ -10,7 +10,7 @@ import sys
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
-SOURCES = ["clg_api.hip", "conv_binary.hip", "logic_fc.hip", "fc_tree.hip", "packbits.hip", "binarize.hip", "conv_generic.hip", "conv_forward.hip", "conv_small.hip", "conv_pair.hip", "conv_pair_grad.hip", "conv_block.hip"]
+SOURCES = ["clg_api.hip", "conv_binary.hip", "logic_fc.hip", "fc_tree.hip", "packbits.hip", "binarize.hip", "conv_generic.hip", "conv_forward.hip", "conv_small.hip", "conv_pair.hip", "conv_pair_grad.hip", "conv_block.hip", "net_step.hip"]
 LIB = os.path.join(PKG, "libconvlogic_amd.so")
 NODES = os.path.join(PKG, "_nodes.so")
 

@@ -21,13 +21,12 @@
 
 #include <algorithm>
 
-#include "conv_tile.h"
+#include "conv_binary.h"
+#include "net_step.h"
 
 int clg_convblock_check(const clg_conv_geom *gg, Geom *g, int dtype, const char *name);
 
 namespace {
-
-constexpr int kFtab = 160;          // per kernel: F1[2][16], F2[8][16]
 
 // ---- context: what the forward leaves for the backward pass (one device buffer) --------------------------------
 struct BinCtx {
@@ -65,133 +64,7 @@ bool bin_supported(const Geom &g, int dtype)
 }
 
 // ---- set-up launch ------------------------------------------------------------------------------------------------
-// blocks [0, C): kernel c -- softmax / fold, the 256-entry table, the derivative tables, tap descriptors
-// blocks [C, C + list_blocks): per input channel, the kernels that read it (increasing order) with their tap masks
-// blocks from pack0 on: the image as bit rows, and the check that it is binary
-struct PrepArgs {
-    const float *x, *w;
-    const int32_t *sel;
-    uint32_t *bits;
-    float *lut, *probs, *folded, *ftab;
-    int32_t *tapinfo, *xtap, *count, *hits;
-    int32_t *bad;            // set to 1 when some x is neither 0 nor 1 (may be host memory the device can write)
-    int w_logits, list_blocks, pack0, RP, prs;
-    FastDiv d_h, d_cinh;
-};
-
-__global__ __launch_bounds__(256) void convblock_bin_prepare_kernel(PrepArgs a, Geom g)
-{
-    const int tid = threadIdx.x, lane = tid & 63;
-    if ((int)blockIdx.x < g.c) {
-        __shared__ float cf[28];
-        const int c = blockIdx.x;
-        if (tid < 7) {
-            const int64_t q = (int64_t)c * 7 + tid;
-            float pr[16];
-            if (a.w_logits) {
-                softmax16(a.w + q * 16, pr);
-            } else {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) pr[i] = a.w[q * 16 + i];
-            }
-#pragma unroll
-            for (int i = 0; i < 16; ++i) a.probs[q * 16 + i] = pr[i];
-            const Coef<float> k = fold16(pr);
-            cf[4 * tid] = k.ab, cf[4 * tid + 1] = k.a, cf[4 * tid + 2] = k.b, cf[4 * tid + 3] = k.one;
-            a.folded[q * 4] = k.ab, a.folded[q * 4 + 1] = k.a, a.folded[q * 4 + 2] = k.b, a.folded[q * 4 + 3] = k.one;
-        }
-        if (tid >= 64 && tid < 72) {
-            const int t = tid - 64;
-            const Tap tp = unpack_tap(a.sel[(int64_t)c * 8 + t], tap_limit(g));   // (forced into the layer's ranges)
-            const int sh = tp.rx - g.pw;                              // tap word = row word >> sh (<< -sh)
-            a.tapinfo[c * 8 + t] = ((tp.ch * a.RP + tp.ry) << 16) | ((sh < 0 ? -sh : 0) << 8) | (sh > 0 ? sh : 0);
-            a.xtap[c * 8 + t] = tp.ry * a.prs + tp.rx;                 // offset of the tap in a gradient plane
-        }
-        __syncthreads();
-        Tree<float> tr;
-#pragma unroll
-        for (int q = 0; q < 7; ++q) tr.g[q] = Coef<float>{cf[4 * q], cf[4 * q + 1], cf[4 * q + 2], cf[4 * q + 3]};
-        float tap[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) tap[i] = (float)((tid >> i) & 1);
-        const TreeVals<float> tv = eval_tree(tr, tap);
-        a.lut[(int64_t)c * 256 + tid] = tv.root;
-        if (tid < kFtab) {
-            // F1[q][nib of the OTHER side] = d root / d mid_q; F2[i][own nibble] = d mid / d leaf * d leaf / d tap_i
-            float v;
-            const int nib = tid & 15;
-            float nb[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) nb[i] = (float)((nib >> i) & 1);
-            auto coef = [&](int q) { return Coef<float>{cf[4 * q], cf[4 * q + 1], cf[4 * q + 2], cf[4 * q + 3]}; };   // (run-time gate index)
-            if (tid < 32) {
-                const int q = tid >> 4;                              // F1[q] is indexed by the nibble of side 1 - q
-                const int o = 1 - q;
-                const float l0 = gate(coef(2 * o), nb[0], nb[1]), l1 = gate(coef(2 * o + 1), nb[2], nb[3]);
-                const float mo = gate(coef(4 + o), l0, l1);
-                v = q == 0 ? gate_da(tr.g[6], mo) : gate_db(tr.g[6], mo);
-            } else {
-                const int i = (tid - 32) >> 4;                       // tap 0..7
-                const int p = i >> 1, q = p >> 1, pl = p & 1, s = i & 1;   // leaf, side, leaf inside the side, operand
-                const float pa = pl ? nb[0] : nb[2], pb = pl ? nb[1] : nb[3];            // taps of the partner leaf
-                const float oa = pl ? nb[2] : nb[0], ob = pl ? nb[3] : nb[1];            // taps of the own leaf
-                const float partner = gate(coef(2 * q + (1 - pl)), pa, pb);
-                const float dm = pl == 0 ? gate_da(coef(4 + q), partner) : gate_db(coef(4 + q), partner);
-                const float dl = s == 0 ? gate_da(coef(p), ob) : gate_db(coef(p), oa);
-                v = dm * dl;
-            }
-            a.ftab[(int64_t)c * kFtab + tid] = v;
-        }
-        return;
-    }
-    if ((int)blockIdx.x < g.c + a.list_blocks) {
-        // one wavefront per input channel: lanes test 64 kernels at a time, matches are appended in order
-        const int ch = uniform((int)(blockIdx.x - g.c) * 4 + (tid >> 6));
-        if (ch >= g.cin) return;
-        int n = 0;
-        for (int c0 = 0; c0 < g.c; c0 += kWave) {
-            const int c = c0 + lane;
-            int mask = 0;
-            if (c < g.c) {
-#pragma unroll
-                for (int t = 0; t < 8; ++t) mask |= (tap_channel(a.sel[c * 8 + t], g.cin) == ch) << t;
-            }
-            const uint64_t vote = __ballot(mask != 0);
-            if (mask) {
-                const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(vote >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)vote, 0));
-                a.hits[(int64_t)ch * g.c + n + before] = c | (mask << 16);
-            }
-            n += __popcll(vote);
-        }
-        if (lane == 0) {
-            a.count[2 * ch] = n;
-            a.count[2 * ch + 1] = ch * g.c;
-        }
-        return;
-    }
-    // bit rows: a wavefront packs two image rows per step (lane = row of the pair * 32 + column)
-    const int64_t rows = (int64_t)g.n * g.cin * g.h;
-    const int r = lane >> 5, col = lane & 31;
-    const int64_t wave0 = (int64_t)(blockIdx.x - a.pack0) * 4 + (tid >> 6), nwaves = (int64_t)(gridDim.x - a.pack0) * 4;
-    bool bad = false;
-    for (int64_t pair = wave0; pair * 2 < rows; pair += nwaves) {
-        const int64_t row = pair * 2 + r;
-        const bool ok = row < rows && col < g.w;
-        const float v = ok ? a.x[row * g.w + col] : 0.f;
-        bad = bad || (v != 0.f && v != 1.f);
-        const uint64_t m = __ballot(v != 0.f);
-        if (col == 0 && row < rows) {
-            const uint32_t plane = fdiv((uint32_t)row, a.d_h), iy = (uint32_t)row - plane * (uint32_t)g.h;
-            uint32_t *dst = a.bits + (int64_t)plane * a.RP;
-            dst[iy + g.ph] = (uint32_t)(r ? m >> 32 : m);
-            if (iy == 0)
-                for (int k = 0; k < g.ph; ++k) dst[k] = 0;
-            if (iy == (uint32_t)g.h - 1)
-                for (int k = 0; k < g.ph; ++k) dst[g.ph + g.h + k] = 0;
-        }
-    }
-    if (bad) *a.bad = 1;
-}
+__global__ __launch_bounds__(256) void convblock_bin_prepare_kernel(PrepArgs a, Geom g) { bin_prepare(a, g, blockIdx.x, gridDim.x); }
 
 // ---- forward --------------------------------------------------------------------------------------------------------
 struct BinFwd {
@@ -492,56 +365,7 @@ __global__ __launch_bounds__(HL) void convblock_bin_hist_kernel(const float *__r
     }
 }
 
-// grid: C, 256 threads: thread t weights the derivative of the tree at tap byte t with the histogram; the 28 coefficient
-// sums are added over t in a fixed order, then the transform to the 16 gates (and the softmax backward for logits).
-__global__ __launch_bounds__(256) void convblock_bin_wgrad_finish_kernel(const float *__restrict__ hpart, const float *__restrict__ folded,
-                                                                       const float *__restrict__ probs, float *__restrict__ gw, int parts)
-{
-    __shared__ float sums[28];
-    const int c = blockIdx.x, t = threadIdx.x;
-    float H = 0.f;
-    const float *hp = hpart + (int64_t)c * parts * 256 + t;
-    int k = 0;
-    for (; k + 8 <= parts; k += 8) {                                  // eight loads in flight, added in the order of one by one
-        float v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = hp[(k + u) * 256];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) H += v[u];
-    }
-    for (; k < parts; ++k) H += hp[k * 256];
-    Tree<float> tr;
-    const float *fc = folded + (int64_t)c * 28;
-#pragma unroll
-    for (int q = 0; q < 7; ++q) tr.g[q] = Coef<float>{fc[4 * q], fc[4 * q + 1], fc[4 * q + 2], fc[4 * q + 3]};
-    float tap[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) tap[i] = (float)((t >> i) & 1);
-    const TreeVals<float> tv = eval_tree(tr, tap);
-    float acc[28];
-    auto put = [&](int q, float g, float a, float b) {
-        const float ga = g * a;
-        acc[4 * q] = ga * b, acc[4 * q + 1] = ga, acc[4 * q + 2] = g * b, acc[4 * q + 3] = g;
-    };
-    put(6, H, tv.mid[0], tv.mid[1]);
-    const float g_m0 = H * gate_da(tr.g[6], tv.mid[1]), g_m1 = H * gate_db(tr.g[6], tv.mid[0]);
-    put(4, g_m0, tv.leaf[0], tv.leaf[1]);
-    put(5, g_m1, tv.leaf[2], tv.leaf[3]);
-    const float g_l0 = g_m0 * gate_da(tr.g[4], tv.leaf[1]), g_l1 = g_m0 * gate_db(tr.g[4], tv.leaf[0]);
-    const float g_l2 = g_m1 * gate_da(tr.g[5], tv.leaf[3]), g_l3 = g_m1 * gate_db(tr.g[5], tv.leaf[2]);
-    put(0, g_l0, tap[0], tap[1]);
-    put(1, g_l1, tap[2], tap[3]);
-    put(2, g_l2, tap[4], tap[5]);
-    put(3, g_l3, tap[6], tap[7]);
-    block_sum_store<float, 28, 256>(acc, sums);
-    __syncthreads();
-    if (t < 112) {
-        const int q = t >> 4, i = t & 15;
-        float gi = coef_transpose_row<float>(i, sums[4 * q], sums[4 * q + 1], sums[4 * q + 2], sums[4 * q + 3]);
-        if (probs != nullptr) gi = softmax16_backward(gi, probs[(int64_t)c * 112 + t]);
-        gw[(int64_t)c * 112 + t] = gi;
-    }
-}
+__global__ __launch_bounds__(256) void convblock_bin_wgrad_finish_kernel(BinSums s) { bin_sums(s, blockIdx.x); }
 
 // ---- input gradient ---------------------------------------------------------------------------------------------------
 struct BinBwdX {
@@ -733,20 +557,16 @@ extern "C" int64_t clg_convblock_bin_ctx_bytes(int dtype, const clg_conv_geom *g
     return (int64_t)bin_ctx(g).total;
 }
 
-extern "C" int clg_convblock_bin_forward(int dtype, const clg_conv_geom *gg, const void *x, const void *w, const int32_t *selection,
-                                         void *y, uint16_t *taps, void *ctx, int flags, int32_t *not_binary, void *stream)
+int clg_bin_prepare_args(const char *name, int dtype, const clg_conv_geom *gg, const void *x, const void *w, const int32_t *selection, void *ctx, bool w_logits,
+                         int32_t *not_binary, Geom *geom, PrepArgs *args, int *blocks)
 {
-    const char *name = "clg_convblock_bin_forward";
-    Geom g;
-    if (int e = clg_convblock_check(gg, &g, dtype, name)) return e;
+    if (int e = clg_convblock_check(gg, geom, dtype, name)) return e;
+    const Geom &g = *geom;
     CLG_REQUIRE(bin_supported(g, dtype), "%s: shape not supported by the binary-input kernels (clg_convblock_bin_supported)", name);
-    CLG_REQUIRE(x && w && selection && y && taps && ctx && not_binary, "%s: null pointer argument", name);
-    CLG_REQUIRE((flags & ~CLG_FWD_W_LOGITS) == 0, "%s: unknown flags 0x%x", name, flags);
+    CLG_REQUIRE(x && w && selection && ctx && not_binary, "%s: null pointer argument", name);
     const BinCtx cx = bin_ctx(g);
     unsigned char *base = reinterpret_cast<unsigned char *>(ctx);
-    hipStream_t st = clg_stream(stream);
-
-    PrepArgs a;
+    PrepArgs &a = *args;
     a.x = (const float *)x, a.w = (const float *)w, a.sel = selection;
     a.bits = reinterpret_cast<uint32_t *>(base + cx.bits_off);
     a.lut = reinterpret_cast<float *>(base + cx.lut_off);
@@ -758,7 +578,7 @@ extern "C" int clg_convblock_bin_forward(int dtype, const clg_conv_geom *gg, con
     a.count = reinterpret_cast<int32_t *>(base + cx.count_off);
     a.hits = reinterpret_cast<int32_t *>(base + cx.hits_off);
     a.bad = not_binary;
-    a.w_logits = (flags & CLG_FWD_W_LOGITS) ? 1 : 0;
+    a.w_logits = w_logits ? 1 : 0;
     a.list_blocks = (int)clg_ceil_div(g.cin, 4);
     a.pack0 = g.c + a.list_blocks;
     a.RP = cx.RP, a.prs = cx.prs;
@@ -766,11 +586,28 @@ extern "C" int clg_convblock_bin_forward(int dtype, const clg_conv_geom *gg, con
     a.d_cinh = make_fastdiv((uint32_t)(g.cin * g.h));
     const int64_t row_pairs = clg_ceil_div((int64_t)g.n * g.cin * g.h, 2);
     const int pack_blocks = (int)std::min<int64_t>(clg_ceil_div(row_pairs, 4 * 8), 2048);   // about 8 row pairs per wavefront
-    hipLaunchKernelGGL(convblock_bin_prepare_kernel, dim3((unsigned)(a.pack0 + std::max(pack_blocks, 1))), dim3(256), 0, st, a, g);
-    CLG_CHECK_LAUNCH("clg_convblock_bin_forward(prepare)");
+    *blocks = a.pack0 + std::max(pack_blocks, 1);
+    return CLG_OK;
+}
+
+extern "C" int clg_convblock_bin_forward(int dtype, const clg_conv_geom *gg, const void *x, const void *w, const int32_t *selection,
+                                         void *y, uint16_t *taps, void *ctx, int flags, int32_t *not_binary, void *stream)
+{
+    const char *name = "clg_convblock_bin_forward";
+    Geom g;
+    PrepArgs a;
+    int prepare_blocks;
+    if (int e = clg_bin_prepare_args(name, dtype, gg, x, w, selection, ctx, (flags & CLG_FWD_W_LOGITS) != 0, not_binary, &g, &a, &prepare_blocks)) return e;
+    CLG_REQUIRE(y && taps, "%s: null pointer argument", name);
+    CLG_REQUIRE((flags & ~(CLG_FWD_W_LOGITS | CLG_FWD_PREPARED)) == 0, "%s: unknown flags 0x%x", name, flags);
+    hipStream_t st = clg_stream(stream);
+    if ((flags & CLG_FWD_PREPARED) == 0) {
+        hipLaunchKernelGGL(convblock_bin_prepare_kernel, dim3((unsigned)prepare_blocks), dim3(256), 0, st, a, g);
+        CLG_CHECK_LAUNCH("clg_convblock_bin_forward(prepare)");
+    }
 
     BinFwd p;
-    p.hp = g.ho / 2, p.wp = g.wo / 2, p.RP = cx.RP;
+    p.hp = g.ho / 2, p.wp = g.wo / 2, p.RP = a.RP;
     // samples per workgroup: the smallest count that fills its last block of 64 lanes to at least 85 %
     int S = 1;
     for (int s = 1; s <= 32; s *= 2) {
@@ -778,7 +615,7 @@ extern "C" int clg_convblock_bin_forward(int dtype, const clg_conv_geom *gg, con
         S = s;
         if (lanes * 100 >= blocks * 64 * 85) break;
     }
-    const size_t img_per_sample = (size_t)g.cin * cx.RP * 4;
+    const size_t img_per_sample = (size_t)g.cin * a.RP * 4;
     if (const char *e = clg_knob(K_BIN_S)) S = std::min(64, std::max(1, atoi(e)));
     while (S > 1 && S * img_per_sample > 64 * 1024) S /= 2;
     CLG_REQUIRE(S * img_per_sample <= 96 * 1024, "%s: the bit planes of one sample (%zu bytes) do not fit LDS", name, img_per_sample);
@@ -803,7 +640,7 @@ extern "C" int clg_convblock_bin_forward(int dtype, const clg_conv_geom *gg, con
     if (const char *e = clg_knob(K_BIN_PIECE)) pc = atoi(e) == 0 ? 0 : (atoi(e) == 2 && pc ? 2 : pc);   // narrower pieces / rows written directly
     p.tr_words = pc ? kWave * (p.wp + 4) : 0;
     p.d_npc = make_fastdiv((uint32_t)std::max(1, pc ? p.wp / pc : 1));
-    const size_t lds = (size_t)CT * 1024 + (((size_t)S * g.cin * cx.RP + 3) & ~(size_t)3) * 4 + (size_t)nw * p.tr_words * 4;
+    const size_t lds = (size_t)CT * 1024 + (((size_t)S * g.cin * a.RP + 3) & ~(size_t)3) * 4 + (size_t)nw * p.tr_words * 4;
 #define CLG_BIN_FWD(PC)                                                                                                          \
     do {                                                                                                                         \
         if (int e = allow_lds(convblock_bin_forward_kernel<PC>, lds, name)) return e;                                            \
@@ -848,10 +685,9 @@ extern "C" int64_t clg_convblock_bin_backward_scratch_bytes(int dtype, const clg
     return (int64_t)g.c * hist_parts(g) * 256 * 4;
 }
 
-extern "C" int clg_convblock_bin_backward(int dtype, const clg_conv_geom *gg, const void *grad_y, const uint16_t *taps, const void *ctx,
-                                          void *grad_x, void *grad_w, int flags, void *scratch, void *stream)
+static int bin_backward(const char *name, int dtype, const clg_conv_geom *gg, const void *grad_y, const uint16_t *taps, const void *ctx, void *grad_x,
+                        void *grad_w, int flags, void *scratch, void *stream, clg_late_sums *late)
 {
-    const char *name = "clg_convblock_bin_backward";
     Geom g;
     if (int e = clg_convblock_check(gg, &g, dtype, name)) return e;
     CLG_REQUIRE(bin_supported(g, dtype), "%s: shape not supported by the binary-input kernels (clg_convblock_bin_supported)", name);
@@ -931,11 +767,29 @@ extern "C" int clg_convblock_bin_backward(int dtype, const clg_conv_geom *gg, co
         else CLG_BIN_HIST(16);
 #undef CLG_BIN_HIST
         CLG_CHECK_LAUNCH("clg_convblock_bin_backward(histogram)");
-        hipLaunchKernelGGL(convblock_bin_wgrad_finish_kernel, dim3((unsigned)g.c), dim3(256), 0, st, (const float *)scratch,
-                           reinterpret_cast<const float *>(base + cx.folded_off),
-                           (flags & CLG_BWD_WRT_LOGITS) ? reinterpret_cast<const float *>(base + cx.probs_off) : (const float *)nullptr,
-                           (float *)grad_w, h.parts);
+        const BinSums sums = {(const float *)scratch, reinterpret_cast<const float *>(base + cx.folded_off),
+                              (flags & CLG_BWD_WRT_LOGITS) ? reinterpret_cast<const float *>(base + cx.probs_off) : (const float *)nullptr,
+                              (float *)grad_w, h.parts};
+        if (late != nullptr) {
+            *late = clg_late(kLateBin, g.c, sums);
+            return CLG_OK;
+        }
+        hipLaunchKernelGGL(convblock_bin_wgrad_finish_kernel, dim3((unsigned)g.c), dim3(256), 0, st, sums);
         CLG_CHECK_LAUNCH("clg_convblock_bin_backward(finish)");
     }
     return CLG_OK;
+}
+
+extern "C" int clg_convblock_bin_backward(int dtype, const clg_conv_geom *gg, const void *grad_y, const uint16_t *taps, const void *ctx,
+                                          void *grad_x, void *grad_w, int flags, void *scratch, void *stream)
+{
+    return bin_backward("clg_convblock_bin_backward", dtype, gg, grad_y, taps, ctx, grad_x, grad_w, flags, scratch, stream, nullptr);
+}
+
+extern "C" int clg_convblock_bin_backward_late(int dtype, const clg_conv_geom *gg, const void *grad_y, const uint16_t *taps, const void *ctx,
+                                               void *grad_x, void *grad_w, int flags, void *scratch, clg_late_sums *late, void *stream)
+{
+    CLG_REQUIRE(late, "clg_convblock_bin_backward_late: null pointer argument");
+    *late = {};
+    return bin_backward("clg_convblock_bin_backward_late", dtype, gg, grad_y, taps, ctx, grad_x, grad_w, flags, scratch, stream, late);
 }

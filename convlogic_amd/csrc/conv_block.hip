@@ -45,7 +45,7 @@ int clg_convblock_backward_4x4(int dtype, const Geom &g, const void *x, const vo
                                const uint8_t *argmax, void *tg, void *gw, const void *probs, const int32_t *count, const int32_t *hits,
                                void *gx, hipStream_t st, const char *name);
 int clg_launch_reduce_coef(int dtype, const void *partial, void *out, int64_t rows, int nb, int G, hipStream_t st, const char *name,
-                           const void *probs);
+                           const void *probs, clg_late_sums *late);
 
 namespace {
 
@@ -1316,7 +1316,7 @@ int launch_backward_x_direct(const Geom &g, const TilePlan &p, int sample_elems,
 
 template <typename T>
 int launch_backward_w_padded(const Geom &g, const TilePlan &p, const WScratch &ws, const void *gy, const void *x, const void *w,
-                             const int32_t *sel, const uint8_t *argmax, void *gw, void *scratch, hipStream_t st, const void *probs)
+                             const int32_t *sel, const uint8_t *argmax, void *gw, void *scratch, hipStream_t st, const void *probs, clg_late_sums *late)
 {
     unsigned char *base = reinterpret_cast<unsigned char *>(scratch);
     T *partial = reinterpret_cast<T *>(base);
@@ -1339,13 +1339,13 @@ int launch_backward_w_padded(const Geom &g, const TilePlan &p, const WScratch &w
                            make_fastdiv((uint32_t)I), ws.sample_elems, 8);
     CLG_CHECK_LAUNCH("clg_convblock_backward_w(padded)");
     return clg_launch_reduce_coef(sizeof(T) == 8 ? CLG_F64 : CLG_F32, partial, gw, g.c, ws.nb, 7, st, "clg_convblock_backward_w(reduce)",
-                                  probs);
+                                  probs, late);
 }
 
 // weight gradient from the padded copy the input gradient of the same call has made
 template <typename T>
 int launch_backward_w_shared(const Geom &g, const SharedPad &sh, const void *gy, const uint8_t *argmax, void *gw, void *scratch,
-                             hipStream_t st, const void *probs)
+                             hipStream_t st, const void *probs, clg_late_sums *late)
 {
     const int64_t I = (int64_t)(g.ho / 2) * (g.wo / 2);
     int64_t nb = clg_ceil_div(I * g.n, 256 * cells_per_thread(I * g.n));
@@ -1361,7 +1361,7 @@ int launch_backward_w_shared(const Geom &g, const SharedPad &sh, const void *gy,
                            make_fastdiv((uint32_t)I), sh.sample_elems, 16);
     CLG_CHECK_LAUNCH("clg_convblock_backward_w(padded, shared copy)");
     return clg_launch_reduce_coef(sizeof(T) == 8 ? CLG_F64 : CLG_F32, partial, gw, g.c, (int)nb, 7, st,
-                                  "clg_convblock_backward_w(reduce)", probs);
+                                  "clg_convblock_backward_w(reduce)", probs, late);
 }
 
 // Plan of the LDS-staged weight gradient: S samples per staged group (their image elements travel through at most
@@ -1424,7 +1424,7 @@ bool plan_backward_w_tiled(const Geom &g, int elem, TiledWPlan *tw)
 
 template <typename T>
 int launch_backward_w_tiled(const Geom &g, const TiledWPlan &tw, const void *gy, const void *x, const void *w, const int32_t *sel,
-                            const uint8_t *argmax, void *gw, void *scratch, hipStream_t st, const void *probs)
+                            const uint8_t *argmax, void *gw, void *scratch, hipStream_t st, const void *probs, clg_late_sums *late)
 {
     const dim3 grid((unsigned)tw.nb, (unsigned)clg_ceil_div(g.c, tw.p.CT)), block(kTiledWWaves * kWave);
     const int nparts = tw.nb * (kTiledWWaves / tw.p.CT);
@@ -1447,7 +1447,7 @@ int launch_backward_w_tiled(const Geom &g, const TiledWPlan &tw, const void *gy,
 #undef CLG_BWDW_TILED
     CLG_CHECK_LAUNCH("clg_convblock_backward_w(tiled)");
     return clg_launch_reduce_coef(sizeof(T) == 8 ? CLG_F64 : CLG_F32, scratch, gw, g.c, nparts, 7, st, "clg_convblock_backward_w(reduce)",
-                                  probs);
+                                  probs, late);
 }
 
 int elem_size(int dtype) { return dtype == CLG_F64 ? 8 : 4; }
@@ -1614,7 +1614,7 @@ extern "C" int clg_convblock_backward_x(int dtype, const clg_conv_geom *gg, cons
 // grad_w w.r.t. the gate probabilities, or -- with probs = the softmax output w -- w.r.t. the logits
 static int convblock_backward_w_impl(int dtype, const clg_conv_geom *gg, const void *grad_y, const void *x, const void *w,
                                      const int32_t *selection, const uint8_t *argmax, void *grad_w, void *scratch, void *stream,
-                                     const void *probs, const char *name, const SharedPad *shared = nullptr)
+                                     const void *probs, const char *name, const SharedPad *shared = nullptr, clg_late_sums *late = nullptr)
 {
     Geom g;
     if (int e = clg_convblock_check(gg, &g, dtype, name)) return e;
@@ -1630,23 +1630,23 @@ static int convblock_backward_w_impl(int dtype, const clg_conv_geom *gg, const v
         if (int e = clg_pair_grad_w(g, pp, nb, (const float *)grad_y, (const float *)x, (const float *)shared->folded, selection, argmax, (float *)scratch,
                                     st, "clg_convblock_backward_w(two planes)"))
             return e;
-        return clg_launch_reduce_coef(CLG_F32, scratch, grad_w, g.c, nb, 7, st, "clg_convblock_backward_w(reduce)", probs);
+        return clg_launch_reduce_coef(CLG_F32, scratch, grad_w, g.c, nb, 7, st, "clg_convblock_backward_w(reduce)", probs, late);
     }
     if (shared != nullptr && shared->xp != nullptr && g.c <= 65535) {
-        if (dtype == CLG_F32) return launch_backward_w_shared<float>(g, *shared, grad_y, argmax, grad_w, scratch, clg_stream(stream), probs);
-        return launch_backward_w_shared<double>(g, *shared, grad_y, argmax, grad_w, scratch, clg_stream(stream), probs);
+        if (dtype == CLG_F32) return launch_backward_w_shared<float>(g, *shared, grad_y, argmax, grad_w, scratch, clg_stream(stream), probs, late);
+        return launch_backward_w_shared<double>(g, *shared, grad_y, argmax, grad_w, scratch, clg_stream(stream), probs, late);
     }
     TiledWPlan tw;
     const char *e_pad = clg_knob(K_BWDW_PADDED);
     if (!(e_pad && atoi(e_pad) != 0) && plan_backward_w_tiled(g, elem_size(dtype), &tw)) {     // images in LDS (CLG_BWDW_PADDED=1 forces the padded copy)
-        return launch_backward_w_tiled<float>(g, tw, grad_y, x, w, selection, argmax, grad_w, scratch, clg_stream(stream), probs);
+        return launch_backward_w_tiled<float>(g, tw, grad_y, x, w, selection, argmax, grad_w, scratch, clg_stream(stream), probs, late);
     }
     TilePlan p;
     WScratch ws;
     if ((!e_pad || atoi(e_pad) != 0) && plan_backward_w(g, elem_size(dtype), &p, &ws)) {
         if (dtype == CLG_F32)
-            return launch_backward_w_padded<float>(g, p, ws, grad_y, x, w, selection, argmax, grad_w, scratch, clg_stream(stream), probs);
-        return launch_backward_w_padded<double>(g, p, ws, grad_y, x, w, selection, argmax, grad_w, scratch, clg_stream(stream), probs);
+            return launch_backward_w_padded<float>(g, p, ws, grad_y, x, w, selection, argmax, grad_w, scratch, clg_stream(stream), probs, late);
+        return launch_backward_w_padded<double>(g, p, ws, grad_y, x, w, selection, argmax, grad_w, scratch, clg_stream(stream), probs, late);
     }
     return clg_convblock_backward_w_generic(dtype, g, grad_y, x, w, selection, argmax, grad_w, scratch, clg_stream(stream), probs);
 }
@@ -1870,7 +1870,7 @@ int64_t clg_convblock_backward_padded_sample_elems(int dtype, const Geom &g)
 
 static int backward_planned_impl(const char *name, int dtype, const clg_conv_geom *gg, const void *grad_y, const void *x, const void *w,
                                  const void *folded, const void *padded, const int32_t *selection, const uint8_t *argmax, void *plan,
-                                 int64_t signature, void *grad_x, void *grad_w, int flags, void *scratch, void *stream)
+                                 int64_t signature, void *grad_x, void *grad_w, int flags, void *scratch, void *stream, clg_late_sums *late = nullptr)
 {
     Geom g;
     if (int e = clg_convblock_check(gg, &g, dtype, name)) return e;
@@ -1908,13 +1908,13 @@ static int backward_planned_impl(const char *name, int dtype, const clg_conv_geo
         if (int e = clg_pair_grads(g, pi.pair, nb, (const float *)grad_y, (const float *)x, (const float *)tb.folded, selection, argmax, tb.count, tb.hits,
                                    planes, (float *)w_scratch, (float *)grad_x, st, name))
             return e;
-        return clg_launch_reduce_coef(CLG_F32, w_scratch, grad_w, g.c, nb, 7, st, name, probs);
+        return clg_launch_reduce_coef(CLG_F32, w_scratch, grad_w, g.c, nb, 7, st, name, probs, late);
     }
     if (grad_x != nullptr)
         if (int e = convblock_backward_x_impl(dtype, gg, grad_y, x, w, selection, argmax, grad_x, scratch, stream, &shared, w_scratch, &pv,
                                               long_lists))
             return e;
-    return convblock_backward_w_impl(dtype, gg, grad_y, x, w, selection, argmax, grad_w, w_scratch, stream, probs, name, &shared);
+    return convblock_backward_w_impl(dtype, gg, grad_y, x, w, selection, argmax, grad_w, w_scratch, stream, probs, name, &shared, late);
 }
 
 extern "C" int clg_convblock_backward_planned(int dtype, const clg_conv_geom *gg, const void *grad_y, const void *x, const void *w,
@@ -1925,16 +1925,31 @@ extern "C" int clg_convblock_backward_planned(int dtype, const clg_conv_geom *gg
                                  grad_x, grad_w, flags, scratch, stream);
 }
 
-extern "C" int clg_convblock_backward_planned_padded(int dtype, const clg_conv_geom *gg, const void *grad_y, const void *x, const void *w,
-                                                     const void *folded, const void *padded, const int32_t *selection,
-                                                     const uint8_t *argmax, void *plan, int64_t signature, void *grad_x, void *grad_w,
-                                                     int flags, void *scratch, void *stream)
+static int planned_padded(const char *name, int dtype, const clg_conv_geom *gg, const void *grad_y, const void *x, const void *w,
+                          const void *folded, const void *padded, const int32_t *selection,
+                          const uint8_t *argmax, void *plan, int64_t signature, void *grad_x, void *grad_w,
+                          int flags, void *scratch, void *stream, clg_late_sums *late)
 {
-    const char *name = "clg_convblock_backward_planned_padded";
     Geom g;
     if (int e = clg_convblock_check(gg, &g, dtype, name)) return e;
     CLG_REQUIRE(padded == nullptr || (grad_x != nullptr && clg_convblock_backward_padded_sample_elems(dtype, g) > 0 && (signature & 1) == 0),
                 "%s: a padded copy is only taken with grad_x, where clg_convblock_padded_elems() is not 0 and for a plan of short lists", name);
     return backward_planned_impl(name, dtype, gg, grad_y, x, w, folded, padded, selection, argmax, plan, signature, grad_x, grad_w, flags,
-                                 scratch, stream);
+                                 scratch, stream, late);
+}
+
+extern "C" int clg_convblock_backward_planned_padded(int dtype, const clg_conv_geom *gg, const void *grad_y, const void *x, const void *w,
+                                                     const void *folded, const void *padded, const int32_t *selection, const uint8_t *argmax, void *plan,
+                                                     int64_t signature, void *grad_x, void *grad_w, int flags, void *scratch, void *stream)
+{
+    return planned_padded("clg_convblock_backward_planned_padded", dtype, gg, grad_y, x, w, folded, padded, selection, argmax, plan, signature, grad_x, grad_w, flags, scratch, stream, nullptr);
+}
+
+extern "C" int clg_convblock_backward_planned_late(int dtype, const clg_conv_geom *gg, const void *grad_y, const void *x, const void *w,
+                                                   const void *folded, const void *padded, const int32_t *selection, const uint8_t *argmax, void *plan,
+                                                   int64_t signature, void *grad_x, void *grad_w, int flags, void *scratch, clg_late_sums *late, void *stream)
+{
+    CLG_REQUIRE(late, "clg_convblock_backward_planned_late: null pointer argument");
+    *late = {};
+    return planned_padded("clg_convblock_backward_planned_late", dtype, gg, grad_y, x, w, folded, padded, selection, argmax, plan, signature, grad_x, grad_w, flags, scratch, stream, late);
 }

@@ -108,4 +108,46 @@ __device__ __forceinline__ void block_sum_store(T (&acc)[K], T *__restrict__ dst
     }
 }
 
+// out[row*G + q][i] = sum_k COEF[k][i] * (sum_blk partial[row][blk][q*4 + k]): the gradient w.r.t. the gate
+// probabilities; with probs (the softmax output they came from) the gradient w.r.t. the logits instead.
+// The 16 lanes of a gate split the sum: lane i adds component i & 3 over the blocks blk = i >> 2 (mod 4), the four
+// stripes meet in a butterfly (same value in both partners), and every lane then holds the four totals.
+template <typename T>
+struct CoefSums {
+    const T *partial, *probs;
+    T *out;
+    int64_t rows;
+    int nb, G;
+};
+template <typename T>
+__device__ __forceinline__ void reduce_coef_partials(const CoefSums<T> &s, int64_t block)   // (of 256 threads)
+{
+    const T *__restrict__ partial = s.partial, *__restrict__ probs = s.probs;
+    T *__restrict__ out = s.out;
+    const int64_t rows = s.rows, e = block * 256 + threadIdx.x;
+    const int nb = s.nb, G = s.G;
+    const int i = threadIdx.x & 15;
+    const int64_t gate = e >> 4;                                     // row * G + q; a row of 16 lanes is live or dead as a whole
+    if (gate >= rows * G) return;
+    const int64_t row = gate / G;
+    const int q = (int)(gate - row * G);
+    const T *p = partial + (row * nb * G + q) * 4 + (i & 3);
+    T acc = 0;
+    int blk = i >> 2;
+    for (; blk + 28 < nb; blk += 32) {                               // eight loads in flight, added in the same order as one by one
+        T v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = p[(int64_t)(blk + 4 * u) * G * 4];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) acc += v[u];
+    }
+    for (; blk < nb; blk += 4) acc += p[(int64_t)blk * G * 4];
+    acc += __shfl_xor(acc, 4, 16);
+    acc += __shfl_xor(acc, 8, 16);
+    const T s0 = __shfl(acc, 0, 16), s1 = __shfl(acc, 1, 16), s2 = __shfl(acc, 2, 16), s3 = __shfl(acc, 3, 16);
+    T gi = coef_transpose_row<T>(i, s0, s1, s2, s3);
+    if (probs != nullptr) gi = softmax16_backward(gi, probs[e]);
+    out[e] = gi;
+}
+
 #endif

@@ -878,11 +878,14 @@ static int forward_ex_impl(const char *name, int dtype, const clg_conv_geom *gg,
     Geom g;
     if (int e = clg_convblock_check(gg, &g, dtype, name)) return e;
     CLG_REQUIRE(x && w && selection && y && argmax, "%s: null pointer argument", name);
-    CLG_REQUIRE((flags & ~(CLG_FWD_W_LOGITS | CLG_FWD_Y_FEATURE_MAJOR | CLG_FWD_FOLDED_OUT | CLG_FWD_FOLDED_IN)) == 0, "%s: unknown flags 0x%x",
+    CLG_REQUIRE((flags & ~(CLG_FWD_W_LOGITS | CLG_FWD_Y_FEATURE_MAJOR | CLG_FWD_FOLDED_OUT | CLG_FWD_FOLDED_IN | CLG_FWD_PREPARED)) == 0, "%s: unknown flags 0x%x",
                 name, flags);
     const bool given = (flags & CLG_FWD_FOLDED_IN) != 0;                // probabilities and coefficients are in probs_out already
     CLG_REQUIRE(!given || ((flags & CLG_FWD_W_LOGITS) && (flags & CLG_FWD_FOLDED_OUT)), "%s: CLG_FWD_FOLDED_IN goes with CLG_FWD_W_LOGITS | "
                 "CLG_FWD_FOLDED_OUT (it says that their outputs are there already)", name);
+    const bool prepared = (flags & CLG_FWD_PREPARED) != 0;
+    CLG_REQUIRE(!prepared || (given && dtype == CLG_F32 && scratch), "%s: CLG_FWD_PREPARED goes with CLG_FWD_FOLDED_IN, float32 and the scratch of "
+                "clg_train_prepare", name);
     bool logits = (flags & CLG_FWD_W_LOGITS) != 0;
     const bool fm = (flags & CLG_FWD_Y_FEATURE_MAJOR) != 0;
     bool want_folded = (flags & CLG_FWD_FOLDED_OUT) != 0;
@@ -917,7 +920,8 @@ static int forward_ex_impl(const char *name, int dtype, const clg_conv_geom *gg,
         float *probs = (float *)probs_out;
         return clg_forward_pair_f32(g, pp, (const float *)x, (const float *)w, selection, (float *)y, argmax, scratch, logits && !given, probs,
                                     given ? (const float *)folded_out : nullptr, (float *)padded_out, tp.rs, tp.chs,
-                                    g.cin * tp.chs + g.ph * tp.rs + g.pw, st, name, want_folded && !given ? (float *)folded_out : nullptr);
+                                    g.cin * tp.chs + g.ph * tp.rs + g.pw, st, name, want_folded && !given ? (float *)folded_out : nullptr,
+                                    prepared);
     }
     if (path == 4 || path == 5) {
         void *fold_to = want_folded ? folded_out : scratch;             // the kernels read them from wherever they are
@@ -980,6 +984,16 @@ static int forward_ex_impl(const char *name, int dtype, const clg_conv_geom *gg,
         return launch_forward_tiled<FloatOps<double>>(g, tp, x, w, selection, y, argmax, st, name, probs_out);
     }
     return fold_after(clg_convblock_forward_generic(dtype, g, x, w, selection, y, argmax, st));
+}
+
+int clg_forward_pair_plan(const char *name, const clg_conv_geom *gg, bool feature_major, Geom *g, PairPlan *p, bool *pair)
+{
+    if (int e = clg_convblock_check(gg, g, CLG_F32, name)) return e;
+    TilePlan tp;
+    DirectPlan dp;
+    g->y_fm = feature_major ? 1 : 0;
+    *pair = choose_forward(*g, 4, 28, true, &tp, &dp, p) == 6;
+    return CLG_OK;
 }
 
 extern "C" int clg_convblock_forward_ex(int dtype, const clg_conv_geom *gg, const void *x, const void *w, const int32_t *selection,

@@ -9,6 +9,7 @@
 // order into per-block partials that a second kernel sums in order; input gradients are gathered
 // per input pixel (one writer per element, no atomics).
 #include "conv_common.h"
+#include "net_step.h"
 
 namespace {
 
@@ -79,38 +80,8 @@ __global__ __launch_bounds__(kBlk) void conv4_backward_w_kernel(const T *__restr
     block_sum_store<T, 16, kBlk>(acc, partial + ((int64_t)c * nb + blockIdx.x) * 16);
 }
 
-// out[row*G + q][i] = sum_k COEF[k][i] * (sum_blk partial[row][blk][q*4 + k]): the gradient w.r.t. the gate
-// probabilities; with probs (the softmax output they came from) the gradient w.r.t. the logits instead.
-// The 16 lanes of a gate split the sum: lane i adds component i & 3 over the blocks blk = i >> 2 (mod 4), the four
-// stripes meet in a butterfly (same value in both partners), and every lane then holds the four totals.
 template <typename T>
-__global__ __launch_bounds__(256) void reduce_coef_partials_kernel(const T *__restrict__ partial, T *__restrict__ out, int64_t rows,
-                                                                 int nb, int G, const T *__restrict__ probs)
-{
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int i = threadIdx.x & 15;
-    const int64_t gate = e >> 4;                                     // row * G + q; a row of 16 lanes is live or dead as a whole
-    if (gate >= rows * G) return;
-    const int64_t row = gate / G;
-    const int q = (int)(gate - row * G);
-    const T *p = partial + (row * nb * G + q) * 4 + (i & 3);
-    T acc = 0;
-    int blk = i >> 2;
-    for (; blk + 28 < nb; blk += 32) {                               // eight loads in flight, added in the same order as one by one
-        T v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = p[(int64_t)(blk + 4 * u) * G * 4];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) acc += v[u];
-    }
-    for (; blk < nb; blk += 4) acc += p[(int64_t)blk * G * 4];
-    acc += __shfl_xor(acc, 4, 16);
-    acc += __shfl_xor(acc, 8, 16);
-    const T s0 = __shfl(acc, 0, 16), s1 = __shfl(acc, 1, 16), s2 = __shfl(acc, 2, 16), s3 = __shfl(acc, 3, 16);
-    T gi = coef_transpose_row<T>(i, s0, s1, s2, s3);
-    if (probs != nullptr) gi = softmax16_backward(gi, probs[e]);
-    out[e] = gi;
-}
+__global__ __launch_bounds__(256) void reduce_coef_partials_kernel(CoefSums<T> s) { reduce_coef_partials(s, blockIdx.x); }
 
 // One thread per input element; every (kernel, tap) that reads the element's channel is visited in
 // a fixed order, so the sum is reproducible.  Gradient of the 4-leaf layer (grad arrives per leaf gate
@@ -398,7 +369,7 @@ int launch_reduce(const void *partial, void *out, int64_t rows, int nb, int G, h
 {
     const int64_t total = rows * G * 16;
     hipLaunchKernelGGL(reduce_coef_partials_kernel<T>, dim3((unsigned)clg_ceil_div(total, 256)), dim3(256), 0, st,
-                       (const T *)partial, (T *)out, rows, nb, G, (const T *)probs);
+                       CoefSums<T>{(const T *)partial, (const T *)probs, (T *)out, rows, nb, G});
     CLG_CHECK_LAUNCH(name);
     return CLG_OK;
 }
@@ -533,9 +504,15 @@ extern "C" int clg_tree_backward_w(int dtype, const void *grad_y, const void *x,
     CLG_DISPATCH(dtype, return launch_reduce<T>(scratch, grad_w, c * xo, nb, 1, st, "clg_tree_backward_w(reduce)"));
 }
 
+// late (or null): takes the sums of a float32 block, which are launched later then
 int clg_launch_reduce_coef(int dtype, const void *partial, void *out, int64_t rows, int nb, int G, hipStream_t st, const char *name,
-                           const void *probs)
+                           const void *probs, clg_late_sums *late)
 {
+    const int64_t blocks = clg_ceil_div(rows * G * 16, 256);
+    if (late != nullptr && dtype == CLG_F32 && blocks < (1 << 24)) {
+        *late = clg_late(kLateCoef, (int)blocks, CoefSums<float>{(const float *)partial, (const float *)probs, (float *)out, rows, nb, G});
+        return CLG_OK;
+    }
     CLG_DISPATCH(dtype, return launch_reduce<T>(partial, out, rows, nb, G, st, name, probs));
 }
 

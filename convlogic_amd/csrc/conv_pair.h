@@ -24,12 +24,45 @@ __host__ __device__ inline int32_t pair_tap(int plane, int rs, int odd, int shif
 }
 constexpr int kPairTable = 12;          // per kernel: channel 0, channel 1 (-1: more than two), code, -, 8 taps;
                                         // behind the last one the geometry, for the rare path that needs all of it
+struct PairOffsets {
+    int plane, rs, odd, shift;
+};
+__host__ __device__ inline PairOffsets pair_offsets(const PairPlan &p) { return {p.plane, p.rs, p.odd, p.lead - p.pw}; }
+#if defined(__HIPCC__)
+// channels and taps of kernel q
+__device__ __forceinline__ void pair_table_row(int32_t *__restrict__ table, const int32_t *__restrict__ sel, int64_t q, const PairOffsets &at, const Geom &g)
+{
+    const TapLimit lim = tap_limit(g);
+    Tap tp[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) tp[t] = unpack_tap(sel[q * 8 + t], lim);
+    const int ch0 = tp[0].ch;
+    int ch1 = ch0;
+#pragma unroll
+    for (int t = 7; t >= 1; --t) ch1 = tp[t].ch != ch0 ? tp[t].ch : ch1;   // first channel that differs
+    bool wide = false;
+    int32_t *row = table + q * kPairTable;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        wide |= tp[t].ch != ch0 && tp[t].ch != ch1;
+        row[4 + t] = pair_tap(at.plane, at.rs, at.odd, at.shift, tp[t].ch != ch0, tp[t].ry, tp[t].rx);
+    }
+    row[0] = ch0;
+    row[1] = wide ? -1 : ch1;
+}
+#endif
 // elem: 4 (float) or 8 (words).  False where the shape is another kernel's.  split: even and odd columns apart, as the forward kernels
 // read them; without, as the weight gradient of floats does.
 bool clg_plan_pair(const Geom &g, int elem, PairPlan *p, bool split = true);
 int clg_forward_pair_f32(const Geom &g, const PairPlan &p, const float *x, const float *w, const int32_t *sel, float *y, uint8_t *argmax, void *scratch,
                          bool from_logits, float *probs_out, const float *folded_in, float *padded_out, int pad_rs, int pad_chs, int pad_sample,
-                         hipStream_t st, const char *name, float *folded_out = nullptr);
+                         hipStream_t st, const char *name, float *folded_out = nullptr, bool prepared = false);
+// The plan of a float32 block whose forward call takes this kernel (conv_forward.hip).
+int clg_forward_pair_plan(const char *name, const clg_conv_geom *gg, bool feature_major, Geom *g, PairPlan *p, bool *pair);
+static inline int32_t *clg_pair_table(const PairPlan &p, void *scratch)
+{
+    return reinterpret_cast<int32_t *>(reinterpret_cast<unsigned char *>(scratch) + p.folded_bytes);
+}
 // gates: null where the table at the start of the scratch is made already
 int clg_forward_pair_packed(const Geom &g, const PairPlan &p, const uint64_t *x, const uint8_t *gates, const int32_t *sel, uint64_t *y, void *scratch,
                             hipStream_t st, const char *name);

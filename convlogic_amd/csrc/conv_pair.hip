@@ -35,47 +35,16 @@ __global__ __launch_bounds__(256) void pair_prepare_kernel(const P *__restrict__
         return;
     }
     const int C = g.c;
-    const TapLimit lim = tap_limit(g);
     const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if constexpr (!Ops::kOrPool) {
         if (folded != nullptr && q < (int64_t)C * 7) {
-            T pr[16];
-            if (from_logits) {
-                softmax16(w + q * 16, pr);
-                if (probs_out != nullptr) {
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) probs_out[q * 16 + i] = pr[i];
-                }
-            } else {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) pr[i] = w[q * 16 + i];
-            }
-            const Coef<T> cf = fold16(pr);
-            folded[q * 4 + 0] = cf.ab;
-            folded[q * 4 + 1] = cf.a;
-            folded[q * 4 + 2] = cf.b;
-            folded[q * 4 + 3] = cf.one;
+            fold_gate<P, T>(w, q, from_logits, probs_out, folded);
         }
     }
     if (q == 0) *reinterpret_cast<Geom *>(table + (int64_t)C * kPairTable) = g;
     if (q < C) {
-        Tap tp[8];
-#pragma unroll
-        for (int t = 0; t < 8; ++t) tp[t] = unpack_tap(sel[q * 8 + t], lim);
-        const int ch0 = tp[0].ch;
-        int ch1 = ch0;
-#pragma unroll
-        for (int t = 7; t >= 1; --t) ch1 = tp[t].ch != ch0 ? tp[t].ch : ch1;   // first channel that differs
-        bool wide = false;
-        int32_t *row = table + q * kPairTable;
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            wide |= tp[t].ch != ch0 && tp[t].ch != ch1;
-            row[4 + t] = pair_tap(p.plane, p.rs, p.odd, p.lead - p.pw, tp[t].ch != ch0, tp[t].ry, tp[t].rx);
-        }
-        row[0] = ch0;
-        row[1] = wide ? -1 : ch1;
-        if constexpr (Ops::kOrPool) row[2] = (int32_t)tree_code(w + q * 7);
+        pair_table_row(table, sel, q, pair_offsets(p), g);
+        if constexpr (Ops::kOrPool) table[q * kPairTable + 2] = (int32_t)tree_code(w + q * 7);
     }
 }
 
@@ -330,16 +299,18 @@ bool clg_plan_pair(const Geom &g, int elem, PairPlan *p, bool split)
 // (null: scratch).  padded_out: where the zero-padded copy of x goes (strides rs, chs), or null.
 int clg_forward_pair_f32(const Geom &g, const PairPlan &p, const float *x, const float *w, const int32_t *sel, float *y, uint8_t *argmax, void *scratch,
                          bool from_logits, float *probs_out, const float *folded_in, float *padded_out, int pad_rs, int pad_chs, int pad_sample,
-                         hipStream_t st, const char *name, float *folded_out)
+                         hipStream_t st, const char *name, float *folded_out, bool prepared)
 {
     unsigned char *base = reinterpret_cast<unsigned char *>(scratch);
     float *folded = folded_out ? folded_out : reinterpret_cast<float *>(base);
-    int32_t *table = reinterpret_cast<int32_t *>(base + p.folded_bytes);
-    const PadJob<float> job = padded_out ? make_pad_job(x, padded_out, g, pad_rs, pad_chs, pad_sample) : no_pad_job<float>();
-    const unsigned prep = (unsigned)clg_ceil_div((int64_t)g.c * (folded_in ? 1 : 7), 256);
-    hipLaunchKernelGGL((pair_prepare_kernel<FloatOps<float>, float, float>), dim3(prep + pad_blocks(job)), dim3(256), 0, st, w, sel,
-                       folded_in ? (float *)nullptr : folded, table, p, g, job, (int)prep, from_logits ? 1 : 0, probs_out);
-    CLG_CHECK_LAUNCH(name);
+    int32_t *table = clg_pair_table(p, scratch);
+    if (!prepared || padded_out) {                                    // (prepared: coefficients and table are there)
+        const PadJob<float> job = padded_out ? make_pad_job(x, padded_out, g, pad_rs, pad_chs, pad_sample) : no_pad_job<float>();
+        const unsigned prep = (unsigned)clg_ceil_div((int64_t)g.c * (folded_in ? 1 : 7), 256);
+        hipLaunchKernelGGL((pair_prepare_kernel<FloatOps<float>, float, float>), dim3(prep + pad_blocks(job)), dim3(256), 0, st, w, sel,
+                           folded_in ? (float *)nullptr : folded, table, p, g, job, (int)prep, from_logits ? 1 : 0, probs_out);
+        CLG_CHECK_LAUNCH(name);
+    }
     const void *fc = folded_in ? (const void *)folded_in : (const void *)folded;
     using Ops = FloatOps<float>;
     if (p.loads <= 2) return launch_pair_nl<Ops, 2>(g, p, x, fc, table, sel, y, argmax, st, name);

@@ -227,6 +227,28 @@ static inline PadJob<T> no_pad_job()
 template <typename T>
 static inline unsigned pad_blocks(const PadJob<T> &j) { return (unsigned)clg_ceil_div(j.total, kPadPerBlock); }
 
+// Folded coefficients of gate q; from_logits: w holds the logits, whose softmax goes to probs_out (or null).
+template <typename P, typename T>
+__device__ __forceinline__ void fold_gate(const P *__restrict__ w, int64_t q, bool from_logits, T *__restrict__ probs_out, T *__restrict__ folded)
+{
+    T pr[16];
+    if (from_logits) {
+        softmax16(w + q * 16, pr);
+        if (probs_out != nullptr) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) probs_out[q * 16 + i] = pr[i];
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) pr[i] = w[q * 16 + i];
+    }
+    const Coef<T> cf = fold16(pr);
+    folded[q * 4 + 0] = cf.ab;
+    folded[q * 4 + 1] = cf.a;
+    folded[q * 4 + 2] = cf.b;
+    folded[q * 4 + 3] = cf.one;
+}
+
 // folded coefficients [c][28] and tap offsets [c][8] in the padded-image layout (either is skipped when null) in the
 // first blocks of the launch, the padded copy in the blocks from pad_block0 on: one launch sets a kernel up.
 // from_logits: w holds the logits, whose softmax goes to probs_out.
@@ -246,22 +268,7 @@ __global__ __launch_bounds__(256) void convblock_w_prepare_kernel(const P *__res
         taps[q] = tp.ch * chs + tp.ry * rs + tp.rx;
     }
     if (folded != nullptr && q < (int64_t)C * 7) {
-        P pr[16];
-        if (from_logits) {                                           // w holds logits: softmax here, written out for the backward pass
-            softmax16(w + q * 16, pr);
-            if (probs_out != nullptr) {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) probs_out[q * 16 + i] = pr[i];
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) pr[i] = w[q * 16 + i];
-        }
-        const Coef<P> cf = fold16(pr);
-        folded[q * 4 + 0] = cf.ab;
-        folded[q * 4 + 1] = cf.a;
-        folded[q * 4 + 2] = cf.b;
-        folded[q * 4 + 3] = cf.one;
+        fold_gate<P, P>(w, q, from_logits, probs_out, folded);
     }
 }
 #endif

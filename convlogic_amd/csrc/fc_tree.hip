@@ -24,7 +24,8 @@
 #include <algorithm>
 
 #include "conv_ops.h"
-#include "conv_pair.h"
+#include "fc_tree.h"
+#include "net_step.h"
 
 int clg_convblock_check(const clg_conv_geom *gg, Geom *g, int dtype, const char *name);
 
@@ -40,8 +41,6 @@ template <int V>
 struct Samples {
     float v[V];
 };
-// (vectors at any 4-byte boundary, which is all that a wide access to global memory needs: rows of an odd number of samples)
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
 template <int V>
 struct SamplesRaw;
@@ -114,17 +113,6 @@ __global__ __launch_bounds__(256) void fc_tree_plan_kernel(TreeWiring w, int32_t
 }
 
 // ---- coefficients ---------------------------------------------------------------------------------------------------
-// ids [roots][8]: the neurons of a tree, 0..3 of the first layer, 4..5 of the second; the root is neuron j of the third.
-// coef [roots][7][4]: fold16 of the softmax (training) or of the arg-max gate (evaluation) of their logits, in tree order, so
-// that a root's 28 coefficients are one run of 112 bytes.
-struct TreeLogits {
-    const float *l[3];
-};
-// (A bad id names a wrong neuron; it never leaves the logits or the probabilities, which are written at the same place.)
-__device__ __forceinline__ int64_t tree_neuron(const int32_t *__restrict__ ids, int j, int q, int roots)
-{
-    return q < 6 ? min((uint32_t)ids[(int64_t)j * 8 + q], (q < 4 ? 4u : 2u) * (uint32_t)roots - 1u) : (uint32_t)j;
-}
 __device__ __forceinline__ const float *tree_logits(const TreeLogits &lg, const int32_t *__restrict__ ids, int j, int q, int roots)
 {
     return (q < 4 ? lg.l[0] : (q < 6 ? lg.l[1] : lg.l[2])) + tree_neuron(ids, j, q, roots) * 16;
@@ -151,66 +139,7 @@ __device__ __forceinline__ int argmax16_quad(f32x4u mine)
     }
     return at;
 }
-// probs (or null): the probabilities, neurons of the first layer first.  The backward pass reads these: logits that an
-// optimizer updates between the two passes must not reach it.
-// A lane per gate does the arithmetic, four lanes per gate move its 64 bytes: the 16-byte pieces of a row go through LDS, so that an
-// access of a wavefront is 16 rows in place of 64 pieces of 64 rows (131072 features, 655360 roots: 211 -> 188 us, 94080 roots 38 -> 28; what is left
-// are 0.66 GB of rows, read and written in tree order).
-constexpr int kFoldPitch = 20;                                       // floats of a row in LDS: 16-byte pieces, lanes spread over the banks
-__global__ __launch_bounds__(256) void fc_tree_fold_kernel(TreeLogits lg, const int32_t *__restrict__ ids, float *__restrict__ coef,
-                                                         float *__restrict__ probs, int roots, int hard)
-{
-    __shared__ __align__(16) float rows[256 / kWave][kWave * kFoldPitch];
-    const int lane = threadIdx.x & (kWave - 1);
-    float *mine = rows[threadIdx.x >> 6];
-    const int64_t gates = (int64_t)roots * 7, e0 = (int64_t)blockIdx.x * 256 + (threadIdx.x & ~(kWave - 1)), e = e0 + lane;
-    if (e0 >= gates) return;                                          // (a whole wavefront; none meets another one)
-    const int64_t ec = e < gates ? e : gates - 1;
-    const int j = (int)(ec / 7), q = (int)(ec - (int64_t)j * 7);
-    const int layer = q < 4 ? 0 : (q < 6 ? 1 : 2);
-    const int neuron = (int)tree_neuron(ids, j, q, roots);
-    const int place = neuron + roots * (layer == 0 ? 0 : (layer == 1 ? 4 : 6));   // of the neuron among all (below 2^31: roots < 2^28)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int from = 16 * i + (lane >> 2), l = __shfl(layer, from, kWave), n = __shfl(neuron, from, kWave);
-        const float *w = l == 0 ? lg.l[0] : (l == 1 ? lg.l[1] : lg.l[2]);
-        const f32x4u v = reinterpret_cast<const f32x4u *>(w + (int64_t)n * 16)[lane & 3];
-        // (logits at any 4-byte boundary)
-        *reinterpret_cast<float4 *>(mine + from * kFoldPitch + 4 * (lane & 3)) = make_float4(v.x, v.y, v.z, v.w);
-    }
-    wave_fence();                                                     // (lanes read what others wrote)
-    float w[16], p[16];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float4 v = *reinterpret_cast<const float4 *>(mine + lane * kFoldPitch + 4 * i);
-        w[4 * i] = v.x, w[4 * i + 1] = v.y, w[4 * i + 2] = v.z, w[4 * i + 3] = v.w;
-    }
-    if (hard) {
-        float best = w[0];
-        int at = 0;
-#pragma unroll
-        for (int i = 1; i < 16; ++i)
-            if (w[i] > best || (w[i] != w[i] && best == best)) best = w[i], at = i;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) p[i] = i == at ? 1.f : 0.f;
-    } else {
-        softmax16(w, p);
-    }
-    const Coef<float> c = fold16(p);
-    if (e < gates) reinterpret_cast<float4 *>(coef)[e] = make_float4(c.ab, c.a, c.b, c.one);
-    if (probs == nullptr) return;
-    wave_fence();
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        *reinterpret_cast<float4 *>(mine + lane * kFoldPitch + 4 * i) = make_float4(p[4 * i], p[4 * i + 1], p[4 * i + 2], p[4 * i + 3]);
-    wave_fence();
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int from = 16 * i + (lane >> 2), at = __shfl(place, from, kWave);
-        const float4 v = *reinterpret_cast<const float4 *>(mine + from * kFoldPitch + 4 * (lane & 3));
-        if (e0 + from < gates) reinterpret_cast<float4 *>(probs + (int64_t)at * 16)[lane & 3] = v;
-    }
-}
+__global__ __launch_bounds__(256) void fc_tree_fold_kernel(TreeFold f) { tree_fold(f, blockIdx.x); }
 
 // ---- forward ----------------------------------------------------------------------------------------------------------
 // rows [roots][8]: the input rows of a tree.  A wavefront takes a root at a time, 64 lanes x V samples.
@@ -401,39 +330,7 @@ __global__ __launch_bounds__(kTreeBlock) void fc_tree_backward_kernel(const floa
     }
 }
 
-// Gradients of the logits, one thread per neuron of the three layers in order.  slot: where the neuron's four sums are (root * 7
-// + gate of the tree).  A layer whose gradient is not wanted has a null pointer.
-struct TreeGrads {
-    float *g[3];
-    int64_t end[3];       // neurons of the first one, two, three layers
-};
-__global__ __launch_bounds__(256) void fc_tree_logit_grad_kernel(const float *__restrict__ probs, TreeGrads gr, const float *__restrict__ sums,
-                                                               const int32_t *__restrict__ slot, int64_t slots)
-{
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= gr.end[2]) return;
-    const int layer = e < gr.end[0] ? 0 : (e < gr.end[1] ? 1 : 2);
-    const int64_t n = e - (layer ? gr.end[layer - 1] : 0);
-    if (gr.g[layer] == nullptr) return;
-    const float4 s = reinterpret_cast<const float4 *>(sums)[min((uint64_t)(uint32_t)slot[e], (uint64_t)slots - 1)];
-    const float4 *w = reinterpret_cast<const float4 *>(probs + e * 16);
-    float p[16], gi[16], dot = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float4 v = w[i];
-        p[4 * i] = v.x, p[4 * i + 1] = v.y, p[4 * i + 2] = v.z, p[4 * i + 3] = v.w;
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        gi[i] = coef_transpose_row<float>(i, s.x, s.y, s.z, s.w);
-        dot = fma_t(p[i], gi[i], dot);
-    }
-    float4 *dst = reinterpret_cast<float4 *>(gr.g[layer] + n * 16);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        dst[i] = make_float4(p[4 * i] * (gi[4 * i] - dot), p[4 * i + 1] * (gi[4 * i + 1] - dot), p[4 * i + 2] * (gi[4 * i + 2] - dot),
-                             p[4 * i + 3] * (gi[4 * i + 3] - dot));
-}
+__global__ __launch_bounds__(256) void fc_tree_logit_grad_kernel(TreeSums t) { tree_logit_grad(t, blockIdx.x); }
 
 // gx[i] = sum of the rows start[i] .. start[i + 1] of rowgrad, eight in flight, four partial sums
 template <int V>
@@ -484,13 +381,6 @@ int tree_vec_dividing(int64_t pitch, const void *x, const void *rowgrad)
     return (align & 15) == 0 ? fit : ((align & 7) == 0 && fit > 1 ? 2 : 1);
 }
 
-int check_tree(const char *name, int64_t in_dim, int64_t roots, int64_t k)
-{
-    CLG_REQUIRE(in_dim > 0 && roots > 0 && k > 0 && roots % k == 0, "%s: in_dim, roots and k must be positive and k divide roots", name);
-    CLG_REQUIRE(in_dim < (1ll << 31) && roots < (1ll << 28) && k <= 65535, "%s: in_dim below 2^31, roots below 2^28 and k up to 65535 only", name);
-    return CLG_OK;
-}
-
 // Row slices of a class, as clg_group_sum cuts them (a class sum of 65 536 values is rounded at 1e-7 of a logit in the
 // thousands: the softmax of the loss then shows the order of the additions, so the order is kept).  Only one or two large classes of a
 // small batch are cut into more slices than its 64, which would be the launch's only 64 or 128 workgroups.
@@ -504,12 +394,19 @@ int tree_slices(int64_t class_rows, int64_t batch, int64_t k)
 
 }  // namespace
 
+int clg_check_tree(const char *name, int64_t in_dim, int64_t roots, int64_t k)
+{
+    CLG_REQUIRE(in_dim > 0 && roots > 0 && k > 0 && roots % k == 0, "%s: in_dim, roots and k must be positive and k divide roots", name);
+    CLG_REQUIRE(in_dim < (1ll << 31) && roots < (1ll << 28) && k <= 65535, "%s: in_dim below 2^31, roots below 2^28 and k up to 65535 only", name);
+    return CLG_OK;
+}
+
 extern "C" int clg_fc_tree_plan(const int64_t *a0, const int64_t *b0, const int64_t *a1, const int64_t *b1, const int64_t *a2,
                                 const int64_t *b2, const int64_t *start, const int64_t *flat, int32_t *rows, int32_t *pos, int32_t *ids,
                                 int32_t *slot, int64_t in_dim, int64_t roots, void *stream)
 {
     const char *name = "clg_fc_tree_plan";
-    if (int e = check_tree(name, in_dim, roots, 1)) return e;
+    if (int e = clg_check_tree(name, in_dim, roots, 1)) return e;
     CLG_REQUIRE(a0 && b0 && a1 && b1 && a2 && b2 && start && flat && rows && pos && ids && slot, "%s: null pointer argument", name);
     const TreeWiring w = {{a0, a1, a2}, {b0, b1, b2}, start, flat};
     hipLaunchKernelGGL(fc_tree_no_slots_kernel, dim3((unsigned)clg_ceil_div(roots * 7, 256)), dim3(256), 0, clg_stream(stream), slot, roots * 7);
@@ -524,11 +421,10 @@ extern "C" int clg_fc_tree_fold(const float *logits0, const float *logits1, cons
                                 float *probs, int64_t roots, int hard, void *stream)
 {
     const char *name = "clg_fc_tree_fold";
-    if (int e = check_tree(name, 1, roots, 1)) return e;
+    if (int e = clg_check_tree(name, 1, roots, 1)) return e;
     CLG_REQUIRE(logits0 && logits1 && logits2 && ids && coef, "%s: null pointer argument", name);
-    const TreeLogits lg = {{logits0, logits1, logits2}};
-    hipLaunchKernelGGL(fc_tree_fold_kernel, dim3((unsigned)clg_ceil_div(roots * 7, 256)), dim3(256), 0, clg_stream(stream), lg, ids, coef,
-                       probs, (int)roots, hard);
+    const TreeFold f = {{{logits0, logits1, logits2}}, ids, coef, probs, (int)roots, hard};
+    hipLaunchKernelGGL(fc_tree_fold_kernel, dim3((unsigned)clg_ceil_div(roots * 7, 256)), dim3(256), 0, clg_stream(stream), f);
     CLG_CHECK_LAUNCH(name);
     return CLG_OK;
 }
@@ -543,7 +439,7 @@ extern "C" int clg_fc_tree_forward(const float *x, const int32_t *rows, const fl
                                    int64_t roots, int64_t k, int64_t batch, int64_t pitch, double tau, void *stream)
 {
     const char *name = "clg_fc_tree_forward";
-    if (int e = check_tree(name, in_dim, roots, k)) return e;
+    if (int e = clg_check_tree(name, in_dim, roots, k)) return e;
     CLG_REQUIRE(x && rows && coef && partial && out, "%s: null pointer argument", name);
     CLG_REQUIRE(batch > 0 && pitch >= batch && pitch < (1ll << 28) && tau != 0.0, "%s: the row pitch must hold the batch, tau must not be zero",
                 name);
@@ -564,19 +460,19 @@ extern "C" int clg_fc_tree_forward(const float *x, const int32_t *rows, const fl
 #define CLG_TREE_S(FLIGHT)                                                                                                    \
     hipLaunchKernelGGL((fc_tree_finish_kernel<FLIGHT>), dim3((unsigned)clg_ceil_div(batch * k, 256)), dim3(256), 0, st, (const float *)partial, \
                        out, slices, (int)k, pitch, batch, 1.f / (float)tau)
-    if (slices > 64) CLG_TREE_S(32);
+    if (slices > 8) CLG_TREE_S(32);
     else CLG_TREE_S(8);
 #undef CLG_TREE_S
     CLG_CHECK_LAUNCH(name);
     return CLG_OK;
 }
 
-extern "C" int clg_fc_tree_backward(const float *x, const int32_t *rows, const int32_t *pos, const int32_t *slot, const float *coef,
-                                    const float *grad_out, const float *probs, float *grad0, float *grad1, float *grad2, float *rowgrad,
-                                    float *sums, const int64_t *start, float *grad_x, int64_t in_dim, int64_t roots, int64_t k, int64_t batch, int64_t pitch, double tau, void *stream)
+static int tree_backward(const char *name, const float *x, const int32_t *rows, const int32_t *pos, const int32_t *slot, const float *coef,
+                         const float *grad_out, const float *probs, float *grad0, float *grad1, float *grad2, float *rowgrad, float *sums,
+                         const int64_t *start, float *grad_x, int64_t in_dim, int64_t roots, int64_t k, int64_t batch, int64_t pitch, double tau, void *stream,
+                         clg_late_sums *late)
 {
-    const char *name = "clg_fc_tree_backward";
-    if (int e = check_tree(name, in_dim, roots, k)) return e;
+    if (int e = clg_check_tree(name, in_dim, roots, k)) return e;
     const bool logits = grad0 || grad1 || grad2;
     CLG_REQUIRE(x && rows && coef && grad_out && (logits || grad_x), "%s: null pointer argument", name);
     CLG_REQUIRE(!logits || (slot && probs && sums), "%s: gradients of logits need slot, probs and sums", name);
@@ -614,10 +510,35 @@ extern "C" int clg_fc_tree_backward(const float *x, const int32_t *rows, const i
 #undef CLG_TREE_K
     CLG_CHECK_LAUNCH(name);
     if (!logits) return CLG_OK;
-    hipLaunchKernelGGL(fc_tree_logit_grad_kernel, dim3((unsigned)clg_ceil_div(7 * roots, 256)), dim3(256), 0, st, probs, gr, (const float *)sums, slot,
-                       7 * roots);
+    const TreeSums t = {gr, probs, sums, slot, 7 * roots};
+    const int64_t blocks = clg_ceil_div(7 * roots, 256);
+    if (late != nullptr) {
+        *late = clg_late(kLateTree, (int)blocks, t);
+        return CLG_OK;
+    }
+    hipLaunchKernelGGL(fc_tree_logit_grad_kernel, dim3((unsigned)blocks), dim3(256), 0, st, t);
     CLG_CHECK_LAUNCH(name);
     return CLG_OK;
+}
+
+extern "C" int clg_fc_tree_backward(const float *x, const int32_t *rows, const int32_t *pos, const int32_t *slot, const float *coef,
+                                    const float *grad_out, const float *probs, float *grad0, float *grad1, float *grad2, float *rowgrad,
+                                    float *sums, const int64_t *start, float *grad_x, int64_t in_dim, int64_t roots, int64_t k, int64_t batch,
+                                    int64_t pitch, double tau, void *stream)
+{
+    return tree_backward("clg_fc_tree_backward", x, rows, pos, slot, coef, grad_out, probs, grad0, grad1, grad2, rowgrad, sums, start, grad_x,
+                         in_dim, roots, k, batch, pitch, tau, stream, nullptr);
+}
+
+extern "C" int clg_fc_tree_backward_late(const float *x, const int32_t *rows, const int32_t *pos, const int32_t *slot, const float *coef,
+                                         const float *grad_out, const float *probs, float *grad0, float *grad1, float *grad2, float *rowgrad,
+                                         float *sums, const int64_t *start, float *grad_x, int64_t in_dim, int64_t roots, int64_t k, int64_t batch,
+                                         int64_t pitch, double tau, clg_late_sums *late, void *stream)
+{
+    CLG_REQUIRE(late, "clg_fc_tree_backward_late: null pointer argument");
+    *late = {};
+    return tree_backward("clg_fc_tree_backward_late", x, rows, pos, slot, coef, grad_out, probs, grad0, grad1, grad2, rowgrad, sums, start, grad_x,
+                         in_dim, roots, k, batch, pitch, tau, stream, late);
 }
 
 // ---- packed inference ---------------------------------------------------------------------------------------------------
@@ -927,7 +848,7 @@ extern "C" int clg_fc_tree_packed(const int64_t *x, const int32_t *rows, const i
                                   int64_t words, int64_t samples, void *stream)
 {
     const char *name = "clg_fc_tree_packed";
-    if (int e = check_tree(name, in_dim, roots, k)) return e;
+    if (int e = clg_check_tree(name, in_dim, roots, k)) return e;
     CLG_REQUIRE(x && rows && ids && logits0 && logits1 && logits2 && codes && out, "%s: null pointer argument", name);
     CLG_REQUIRE(words > 0 && samples > 0 && samples <= words * 64 && words < (1ll << 31), "%s: words %lld, samples %lld", name,
                 (long long)words, (long long)samples);
@@ -1002,7 +923,7 @@ extern "C" int64_t clg_net_packed_scratch_bytes(const clg_packed_block *blocks, 
                                                 int64_t samples)
 {
     const char *name = "clg_net_packed_scratch_bytes";
-    if (check_tree(name, in_dim, roots, k)) return -1;
+    if (clg_check_tree(name, in_dim, roots, k)) return -1;
     NetLayout l;
     return net_layout(name, blocks, n_blocks, in_dim, roots, k, samples, &l) ? -1 : (int64_t)l.total;
 }
@@ -1012,7 +933,7 @@ extern "C" int clg_net_packed(const clg_packed_block *blocks, int n_blocks, cons
                               double tau, int64_t in_dim, int64_t roots, int64_t k, int64_t samples, void *scratch, void *stream)
 {
     const char *name = "clg_net_packed";
-    if (int e = check_tree(name, in_dim, roots, k)) return e;
+    if (int e = clg_check_tree(name, in_dim, roots, k)) return e;
     NetLayout l;
     if (int e = net_layout(name, blocks, n_blocks, in_dim, roots, k, samples, &l)) return e;
     const int64_t words = blocks[0].geom.n;

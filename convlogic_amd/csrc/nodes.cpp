@@ -140,11 +140,12 @@ Tensor fc_layer(const Tensor &x, const Tensor &a, const Tensor &b, const Tensor 
 // ---- complete blocks -----------------------------------------------------------------------------------------------------
 struct Conv {                                                         // stride, padding and kernel of a block
     int64_t sh, sw, ph, pw, kh, kw;
-    clg_conv_geom geom(const Tensor &x, int64_t c_out) const
+    clg_conv_geom geom(at::IntArrayRef x, int64_t c_out) const
     {
-        return {(int32_t)x.size(0), (int32_t)x.size(1), (int32_t)x.size(2), (int32_t)x.size(3), (int32_t)c_out, (int32_t)sh, (int32_t)sw,
-                (int32_t)ph, (int32_t)pw, (int32_t)kh, (int32_t)kw};
+        return {(int32_t)x[0], (int32_t)x[1], (int32_t)x[2], (int32_t)x[3], (int32_t)c_out, (int32_t)sh, (int32_t)sw, (int32_t)ph, (int32_t)pw,
+                (int32_t)kh, (int32_t)kw};
     }
+    clg_conv_geom geom(const Tensor &x, int64_t c_out) const { return geom(x.sizes(), c_out); }
     c10::IValue saved(std::vector<int64_t> more) const
     {
         std::vector<int64_t> l{sh, sw, ph, pw, kh, kw};
@@ -166,10 +167,33 @@ struct BlockState {
     void save(variable_list &list) const { list.insert(list.end(), {x, probs, sel, argmax, folded, padded}); }
     static BlockState from(const Tensor *t) { return {t[0], t[1], t[2], t[3], t[4], t[5]}; }
 };
+// What clg_train_prepare has filled for a float32 block: probabilities and coefficients, and the scratch of its forward call.
+struct Prepared {
+    Tensor probs, scratch;
+    static Prepared room(const Tensor &like, const clg_conv_geom &g)
+    {
+        return {floats(like, {(int64_t)g.c_out * (112 + 28)}), bytes(like, clg_convblock_forward_scratch_bytes(CLG_F32, &g))};
+    }
+};
+// Sums that the backward calls of a network's layers leave for one launch, and the buffers they are in.
+struct Late {
+    std::vector<clg_late_sums> sums;
+    std::vector<Tensor> kept;
+    clg_late_sums *next(const Tensor &scratch)
+    {
+        kept.push_back(scratch);
+        sums.push_back({});
+        return &sums.back();
+    }
+    void run(void *stream)
+    {
+        if (!sums.empty()) check(clg_late_sums_run(sums.data(), (int)sums.size(), stream));
+    }
+};
 // signature: that of the layer's backward plan.  pair: probabilities and folded coefficients [c, 7, 16], [c, 7, 4] in one buffer
 // that a network made for all its layers (or null).  fm (in): the output may be feature-major; (out): it is, [c, h, w, n].
 Tensor block_forward(const Tensor &x_in, const Tensor &logits, const Tensor &sel_in, const Conv &conv, bool &fm, int64_t signature,
-                     const std::pair<Tensor, Tensor> *pair, bool need_x, BlockState &state)
+                     const std::pair<Tensor, Tensor> *pair, bool need_x, BlockState &state, const Prepared *made = nullptr)
 {
     const Tensor x = x_in.contiguous(), sel = sel_in.contiguous();
     const int64_t c = logits.size(0);
@@ -184,11 +208,14 @@ Tensor block_forward(const Tensor &x_in, const Tensor &logits, const Tensor &sel
         need(folded, x, "prefolded coefficients", {c, 7, 4});
         TORCH_CHECK(folded.data_ptr<float>() == probs.data_ptr<float>() + probs.numel(),
                     "prefolded: the folded coefficients must follow the probabilities in one buffer (fold_many)");
-    } else {
+    } else if (made == nullptr) {
         probs = floats(x, {c * (112 + 28)});
+    } else {
+        probs = made->probs;
     }
-    const Tensor scratch = bytes(x, clg_convblock_forward_scratch_bytes(CLG_F32, &g));
-    const int flags = CLG_FWD_W_LOGITS | (fm ? CLG_FWD_Y_FEATURE_MAJOR : 0) | CLG_FWD_FOLDED_OUT | (pair != nullptr ? CLG_FWD_FOLDED_IN : 0);
+    const Tensor scratch = made != nullptr ? made->scratch : bytes(x, clg_convblock_forward_scratch_bytes(CLG_F32, &g));
+    const int flags = CLG_FWD_W_LOGITS | (fm ? CLG_FWD_Y_FEATURE_MAJOR : 0) | CLG_FWD_FOLDED_OUT |
+                      (made != nullptr ? CLG_FWD_FOLDED_IN | CLG_FWD_PREPARED : (pair != nullptr ? CLG_FWD_FOLDED_IN : 0));
     Tensor padded;
     if (need_x && (signature & 1) == CLG_LISTS_SHORT && !fm) {        // the copy of x that the forward kernels stage and the backward reads
         const int64_t elems = clg_convblock_padded_elems(CLG_F32, &g, 1);
@@ -207,7 +234,7 @@ Tensor block_forward(const Tensor &x_in, const Tensor &logits, const Tensor &sel
 }
 // -> gradients of x and of the logits; fm: the forward pass was feature-major
 std::pair<Tensor, Tensor> block_backward(const BlockState &state, const Conv &conv, bool fm, const Tensor &plan, int64_t signature, Tensor gy, bool need_x,
-                                         bool need_l)
+                                         bool need_l, Late *late = nullptr)
 {
     const Tensor &x = state.x, &probs = state.probs, &sel = state.sel;
     const int64_t c = sel.size(0);
@@ -231,7 +258,11 @@ std::pair<Tensor, Tensor> block_backward(const BlockState &state, const Conv &co
         const Tensor scratch = bytes(x, clg_convblock_backward_planned_scratch_bytes(CLG_F32, &g, signature));
         const Tensor padded = fm || !need_x ? Tensor() : state.padded;
         const int flags = CLG_BWD_WRT_LOGITS | (fm ? CLG_BWD_GY_FEATURE_MAJOR : 0);
-        if (padded.defined())
+        if (late != nullptr)
+            check(clg_convblock_backward_planned_late(CLG_F32, &g, gy.data_ptr(), x.data_ptr(), probs.data_ptr(), folded, ptr(padded), selection, codes,
+                                                      plan.data_ptr(), signature, ptr(gx), gl.data_ptr(), flags, scratch.data_ptr(),
+                                                      late->next(scratch), stream_of(x)));
+        else if (padded.defined())
             check(clg_convblock_backward_planned_padded(CLG_F32, &g, gy.data_ptr(), x.data_ptr(), probs.data_ptr(), folded, padded.data_ptr(),
                                                         selection, codes, plan.data_ptr(), signature, gx.data_ptr(), gl.data_ptr(), flags,
                                                         scratch.data_ptr(), stream_of(x)));
@@ -278,22 +309,24 @@ Tensor block(const Tensor &x, const Tensor &logits, const Tensor &sel, std::arra
 }
 
 // The block on 0/1 inputs, from the logits.  flag: device address of the layer's BinaryFlag.  It keeps taps and keep; x itself is not needed
-// again.
-Tensor binary_forward(const Tensor &x_in, const Tensor &logits, const Tensor &sel_in, const Conv &conv, int64_t flag, Tensor &taps, Tensor &keep)
+// again.  made: clg_train_prepare has filled keep.
+Tensor binary_forward(const Tensor &x_in, const Tensor &logits, const Tensor &sel_in, const Conv &conv, int64_t flag, Tensor &taps, Tensor &keep,
+                      bool made = false)
 {
     const Tensor x = x_in.contiguous(), sel = sel_in.contiguous();
     const clg_conv_geom g = conv.geom(x, logits.size(0));
-    keep = bytes(x, clg_convblock_bin_ctx_bytes(CLG_F32, &g));
+    if (!made) keep = bytes(x, clg_convblock_bin_ctx_bytes(CLG_F32, &g));
     const auto s = pooled(g);
     Tensor y = floats(x, s);
     taps = at::empty(s, x.options().dtype(at::kShort));
     check(clg_convblock_bin_forward(CLG_F32, &g, x.data_ptr(), logits.data_ptr(), static_cast<const int32_t *>(sel.data_ptr()), y.data_ptr(),
-                                    static_cast<uint16_t *>(taps.data_ptr()), keep.data_ptr(), CLG_FWD_W_LOGITS, reinterpret_cast<int32_t *>(flag),
-                                    stream_of(x)));
+                                    static_cast<uint16_t *>(taps.data_ptr()), keep.data_ptr(), CLG_FWD_W_LOGITS | (made ? CLG_FWD_PREPARED : 0),
+                                    reinterpret_cast<int32_t *>(flag), stream_of(x)));
     return y;
 }
 // xs: shape of x
-std::pair<Tensor, Tensor> binary_backward(const Tensor &taps, const Tensor &keep, const Conv &cv, at::IntArrayRef xs, const Tensor &grad, bool need_x, bool need_l)
+std::pair<Tensor, Tensor> binary_backward(const Tensor &taps, const Tensor &keep, const Conv &cv, at::IntArrayRef xs, const Tensor &grad, bool need_x, bool need_l,
+                                          Late *late = nullptr)
 {
     const Tensor gy = grad.contiguous();
     TORCH_CHECK(gy.is_cuda(), "grad_y must be a CUDA tensor");
@@ -308,7 +341,10 @@ std::pair<Tensor, Tensor> binary_backward(const Tensor &taps, const Tensor &keep
         gl = floats(gy, {c, 7, 16});
         scratch = bytes(gy, clg_convblock_bin_backward_scratch_bytes(CLG_F32, &g));
     }
-    if (need_x || need_l)
+    if (need_l && late != nullptr)
+        check(clg_convblock_bin_backward_late(CLG_F32, &g, gy.data_ptr(), static_cast<const uint16_t *>(taps.data_ptr()), keep.data_ptr(), ptr(gx), ptr(gl),
+                                              CLG_BWD_WRT_LOGITS, ptr(scratch), late->next(scratch), stream_of(gy)));
+    else if (need_x || need_l)
         check(clg_convblock_bin_backward(CLG_F32, &g, gy.data_ptr(), static_cast<const uint16_t *>(taps.data_ptr()), keep.data_ptr(), ptr(gx), ptr(gl),
                                          CLG_BWD_WRT_LOGITS, ptr(scratch), stream_of(gy)));
     return {gx, gl};
@@ -349,13 +385,16 @@ struct TreeArgs {
 };
 const int32_t *i32(const Tensor &v) { return static_cast<const int32_t *>(v.data_ptr()); }
 float *f32(const Tensor &v) { return static_cast<float *>(ptr(v)); }
-// x feature-major -> class sums; coef and (need_l) probs are kept
+// x feature-major -> class sums; coef and (need_l) probs are kept, and made here unless coef is there
 Tensor trees_forward(const Tensor &x, const Tensor &l0, const Tensor &l1, const Tensor &l2, const TreeArgs &t, bool need_l, Tensor &coef, Tensor &probs)
 {
     const int64_t in_dim = x.size(0), batch = x.size(1);
-    coef = floats(x, {t.roots, 28});
-    if (need_l) probs = floats(x, {7 * t.roots, 16});                 // (the logits may be updated between forward and backward)
-    check(clg_fc_tree_fold(l0.data_ptr<float>(), l1.data_ptr<float>(), l2.data_ptr<float>(), i32(t.ids), f32(coef), f32(probs), t.roots, 0, stream_of(x)));
+    if (!coef.defined()) {
+        coef = floats(x, {t.roots, 28});
+        if (need_l) probs = floats(x, {7 * t.roots, 16});             // (the logits may be updated between forward and backward)
+        check(clg_fc_tree_fold(l0.data_ptr<float>(), l1.data_ptr<float>(), l2.data_ptr<float>(), i32(t.ids), f32(coef), f32(probs), t.roots, 0,
+                               stream_of(x)));
+    }
     const int64_t elems = clg_fc_tree_partial_elems(t.roots, t.k, batch, batch);
     Tensor out = floats(x, {batch, t.k}), partial = floats(x, {elems < 0 ? 0 : elems});
     check(clg_fc_tree_forward(f32(x), i32(t.rows), f32(coef), f32(partial), f32(out), in_dim, t.roots, t.k, batch, batch, t.tau, stream_of(x)));
@@ -363,7 +402,7 @@ Tensor trees_forward(const Tensor &x, const Tensor &l0, const Tensor &l1, const 
 }
 // -> gradients of x and of the three layers' logits, those that are wanted.  tables: rows, pos, slot
 std::array<Tensor, 4> trees_backward(const Tensor &x, const Tensor &start, const Tensor &coef, const Tensor &probs, const std::vector<Tensor> &tables, int64_t k,
-                                     double tau, const Tensor &grad, std::array<bool, 4> wanted)
+                                     double tau, const Tensor &grad, std::array<bool, 4> wanted, Late *late = nullptr)
 {
     const int64_t in_dim = x.size(0), batch = x.size(1), roots = coef.size(0);
     const Tensor go = grad.contiguous();
@@ -375,8 +414,13 @@ std::array<Tensor, 4> trees_backward(const Tensor &x, const Tensor &start, const
         if (wanted[1 + i]) g[1 + i] = floats(x, {neurons[i], 16});
     const int64_t rows = g[0].defined() ? 8 * roots * batch : 0;
     const Tensor scratch = floats(x, {rows + 28 * roots});           // operand gradients, then sums
-    check(clg_fc_tree_backward(f32(x), i32(tables[0]), i32(tables[1]), i32(tables[2]), f32(coef), f32(go), f32(probs), f32(g[1]), f32(g[2]), f32(g[3]),
-                               f32(scratch), f32(scratch) + rows, idx(start), f32(g[0]), in_dim, roots, k, batch, batch, tau, stream_of(x)));
+    if (late != nullptr)
+        check(clg_fc_tree_backward_late(f32(x), i32(tables[0]), i32(tables[1]), i32(tables[2]), f32(coef), f32(go), f32(probs), f32(g[1]), f32(g[2]),
+                                        f32(g[3]), f32(scratch), f32(scratch) + rows, idx(start), f32(g[0]), in_dim, roots, k, batch, batch, tau,
+                                        late->next(scratch), stream_of(x)));
+    else
+        check(clg_fc_tree_backward(f32(x), i32(tables[0]), i32(tables[1]), i32(tables[2]), f32(coef), f32(go), f32(probs), f32(g[1]), f32(g[2]), f32(g[3]),
+                                   f32(scratch), f32(scratch) + rows, idx(start), f32(g[0]), in_dim, roots, k, batch, batch, tau, stream_of(x)));
     return g;
 }
 struct Trees : torch::autograd::Function<Trees> {
@@ -412,7 +456,7 @@ Tensor trees(const Tensor &x, const Tensor &l0, const Tensor &l1, const Tensor &
 }
 
 // ---- a network: blocks, flattening, trees -------------------------------------------------------------------------------------
-// One node for what the modules' nodes do one after the other, with the same calls of the library: a step of a small network is bound by the
+// One node for what the modules' nodes do one after the other, with the same kernels: a step of a small network is bound by the
 // host, which takes longer from node to node (module calls in Python, views, the engine's queue) than for the launches of one.  MNIST
 // topology, k = 32, 100 images, a step with its loss: 344 -> 285 us; CIFAR, 256 images: 352 -> 330, the time of its kernels.
 struct NetBlock {
@@ -429,9 +473,35 @@ struct NetArgs {
 struct Network : torch::autograd::Function<Network> {
     // per block and for the trees in front of their wiring: as many saved tensors
     static constexpr int kEach = BlockState::kTensors, kTrees = 4;
+    static constexpr size_t kTogether = 16;                           // blocks that clg_train_prepare and clg_late_sums_run take
     static Tensor forward(AutogradContext *ctx, const Tensor &x, at::TensorList logits, const NetArgs *a)
     {
         const size_t n = a->blocks.size();
+        const bool need_l = a->wanted[1 + n] || a->wanted[2 + n] || a->wanted[3 + n];
+        // the set-up of all layers in one launch
+        Tensor coef, probs;
+        std::vector<Prepared> made(n);                                // (a binary block's: its keep)
+        const bool together = n <= kTogether;
+        if (together) {
+            std::vector<clg_train_block> first(n);
+            at::DimVector shape(x.sizes());
+            for (size_t i = 0; i < n; ++i) {
+                const NetBlock &b = a->blocks[i];
+                const clg_conv_geom g = b.conv.geom(shape, b.sel.size(0));
+                const auto next = pooled(g);
+                const bool binary = b.flag != 0;
+                if (binary) made[i].probs = bytes(x, clg_convblock_bin_ctx_bytes(CLG_F32, &g));
+                else made[i] = Prepared::room(x, g);
+                first[i] = {g, binary ? f32(x) : nullptr, f32(logits[i]), i32(b.sel), binary ? nullptr : f32(made[i].probs),
+                            binary ? ptr(made[i].probs) : ptr(made[i].scratch), reinterpret_cast<int32_t *>(b.flag),
+                            !binary && b.fm && clg_convblock_fm_supported(CLG_F32, &g)};
+                shape.assign(next.begin(), next.end());
+            }
+            coef = floats(x, {a->trees.roots, 28});
+            if (need_l) probs = floats(x, {7 * a->trees.roots, 16});
+            check(clg_train_prepare(first.data(), (int)n, f32(logits[n]), f32(logits[n + 1]), f32(logits[n + 2]), i32(a->trees.ids), f32(coef), f32(probs),
+                                    a->trees.roots, stream_of(x)));
+        }
         variable_list saved;
         std::vector<int64_t> ints;
         std::vector<Tensor> plans;
@@ -444,9 +514,10 @@ struct Network : torch::autograd::Function<Network> {
             fm = b.fm;
             if (b.flag != 0) {
                 fm = false;
-                h = binary_forward(h, logits[i], b.sel, b.conv, b.flag, state.x, state.probs);
+                state.probs = made[i].probs;
+                h = binary_forward(h, logits[i], b.sel, b.conv, b.flag, state.x, state.probs, together);
             } else {
-                h = block_forward(h, logits[i], b.sel, b.conv, fm, b.signature, nullptr, some, state);
+                h = block_forward(h, logits[i], b.sel, b.conv, fm, b.signature, nullptr, some, state, together ? &made[i] : nullptr);
             }
             state.save(saved);
             const std::vector<int64_t> own{b.conv.sh, b.conv.sw, b.conv.ph, b.conv.pw, b.conv.kh, b.conv.kw, shape[0], shape[1], shape[2], shape[3],
@@ -458,8 +529,6 @@ struct Network : torch::autograd::Function<Network> {
         // features [c h w, n]
         const int64_t batch = x.size(0);
         h = fm ? h.view({-1, batch}) : transposed(h.view({batch, -1}));
-        const bool need_l = a->wanted[1 + n] || a->wanted[2 + n] || a->wanted[3 + n];
-        Tensor coef, probs;
         const Tensor out = trees_forward(h, logits[n], logits[n + 1], logits[n + 2], a->trees, need_l, coef, probs);
         saved.insert(saved.end(), {h, a->trees.start, coef, probs});
         saved.insert(saved.end(), a->trees.wiring.begin(), a->trees.wiring.end());
@@ -484,8 +553,9 @@ struct Network : torch::autograd::Function<Network> {
         for (size_t i = 0; i < n; ++i) below[i + 1] = below[i] || wanted(1 + i);
         variable_list out(1 + n + 3 + 1);
         const Tensor *t = saved.data() + n * kEach;
+        Late sums, *late = n <= kTogether ? &sums : nullptr;
         auto g = trees_backward(t[0], t[1], t[2], t[3], ctx->saved_data["tables"].toTensorVector(), ctx->saved_data["k"].toInt(),
-                                ctx->saved_data["tau"].toDouble(), grads[0], {below[n], wanted(1 + n), wanted(2 + n), wanted(3 + n)});
+                                ctx->saved_data["tau"].toDouble(), grads[0], {below[n], wanted(1 + n), wanted(2 + n), wanted(3 + n)}, late);
         for (size_t i = 0; i < 3; ++i) out[1 + n + i] = g[1 + i];
         Tensor h = g[0];
         for (size_t i = n; i-- > 0 && (below[i] || wanted(1 + i));) {
@@ -498,12 +568,13 @@ struct Network : torch::autograd::Function<Network> {
                                        (int32_t)own[0], (int32_t)own[1], (int32_t)own[2], (int32_t)own[3], (int32_t)own[4], (int32_t)own[5]});
                 h = fm ? h.view({s[1], s[2], s[3], s[0]}).permute({3, 0, 1, 2}) : transposed(h).view(s);
             }
-            const auto gi = binary ? binary_backward(kept[0], kept[1], conv, at::IntArrayRef(own + 6, 4), h, below[i], wanted(1 + i))
-                                   : block_backward(BlockState::from(kept), conv, fm, plans[i], own[11], h, below[i], wanted(1 + i));
+            const auto gi = binary ? binary_backward(kept[0], kept[1], conv, at::IntArrayRef(own + 6, 4), h, below[i], wanted(1 + i), late)
+                                   : block_backward(BlockState::from(kept), conv, fm, plans[i], own[11], h, below[i], wanted(1 + i), late);
             h = gi.first;
             out[1 + i] = gi.second;
         }
         if (below[0]) out[0] = h;
+        sums.run(stream_of(t[0]));
         return out;
     }
 };

@@ -438,6 +438,7 @@ int clg_convblock_fm_supported(int dtype, const clg_conv_geom *g);
                               * probability part is left untouched (w already holds them) */
 #define CLG_FWD_FOLDED_IN 8  /* with the two flags above: probs_out ALREADY holds the probabilities and the folded coefficients of
                               * w's logits (clg_fold_many at the start of the step): no softmax or fold launch in this call */
+#define CLG_FWD_PREPARED 32  /* clg_train_prepare has made what this call's kernels read: with CLG_FWD_FOLDED_IN, and the same scratch */
 int clg_convblock_forward_ex(int dtype, const clg_conv_geom *g, const void *x, const void *w, const int32_t *selection, void *y,
                              uint8_t *argmax, void *probs_out, int flags, void *scratch, void *stream);
 /* The same for packed words: y laid out [c_out, ho/2, wo/2, groups], which IS the feature-major [features, words] layout
@@ -585,6 +586,41 @@ int clg_convblock_bin_forward(int dtype, const clg_conv_geom *g, const void *x, 
 int64_t clg_convblock_bin_backward_scratch_bytes(int dtype, const clg_conv_geom *g);
 int clg_convblock_bin_backward(int dtype, const clg_conv_geom *g, const void *grad_y, const uint16_t *taps, const void *ctx,
                                void *grad_x, void *grad_w, int flags, void *scratch, void *stream);
+
+/* A training step of a network of blocks and trees with one launch for the set-up of all layers and one for the sums that end their weight
+ * gradients.  clg_train_prepare: what clg_fc_tree_fold makes of the trees' logits and, per block, what its forward call with
+ * CLG_FWD_PREPARED reads -- for a float32 block clg_convblock_forward_ex / _padded (flags CLG_FWD_W_LOGITS | CLG_FWD_FOLDED_OUT | CLG_FWD_FOLDED_IN |
+ * CLG_FWD_PREPARED), for one on 0/1 inputs clg_convblock_bin_forward.  At most 16 blocks, one of them binary.
+ * The _late calls are those without the suffix, but for a last launch that they describe in *late where they would end with one;
+ * clg_late_sums_run launches those of up to 17 calls together.  Until then grad_w is not written, and the buffers of the calls, scratch
+ * included, stay as they are. */
+typedef struct clg_train_block {
+    clg_conv_geom geom;
+    const float *x;           /* binary block: its input, else NULL */
+    const float *logits;      /* [c_out, 7, 16] */
+    const int32_t *selection; /* [c_out, 8] */
+    float *probs;             /* float32 block: [c_out, 7, 16] then [c_out, 7, 4], probs_out of the forward call */
+    void *scratch;            /* the forward call's scratch; binary block: its ctx */
+    int32_t *not_binary;      /* binary block: its flag, else NULL */
+    int32_t feature_major;    /* float32 block: CLG_FWD_Y_FEATURE_MAJOR */
+} clg_train_block;
+int clg_train_prepare(const clg_train_block *blocks, int n_blocks, const float *logits0, const float *logits1, const float *logits2,
+                      const int32_t *ids, float *coef, float *probs, int64_t roots, void *stream);
+typedef struct clg_late_sums {
+    int32_t kind, blocks;     /* kind 0: nothing is left to do */
+    int64_t field[12];
+} clg_late_sums;
+int clg_convblock_backward_planned_late(int dtype, const clg_conv_geom *g, const void *grad_y, const void *x, const void *w,
+                                        const void *folded, const void *padded, const int32_t *selection, const uint8_t *argmax,
+                                        void *plan, int64_t signature, void *grad_x, void *grad_w, int flags, void *scratch,
+                                        clg_late_sums *late, void *stream);
+int clg_convblock_bin_backward_late(int dtype, const clg_conv_geom *g, const void *grad_y, const uint16_t *taps, const void *ctx,
+                                    void *grad_x, void *grad_w, int flags, void *scratch, clg_late_sums *late, void *stream);
+int clg_fc_tree_backward_late(const float *x, const int32_t *rows, const int32_t *pos, const int32_t *slot, const float *coef,
+                              const float *grad_out, const float *probs, float *grad0, float *grad1, float *grad2, float *rowgrad,
+                              float *sums, const int64_t *start, float *grad_x, int64_t in_dim, int64_t roots, int64_t k,
+                              int64_t batch, int64_t pitch, double tau, clg_late_sums *late, void *stream);
+int clg_late_sums_run(const clg_late_sums *late, int n, void *stream);
 
 /* ---------------------------------------------------------------------------------
  * input binarisation (the step in front of the first layer)

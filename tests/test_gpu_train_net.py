@@ -137,3 +137,20 @@ def test_a_broken_promise_of_binary_inputs_is_reported():
     torch.cuda.synchronize()
     with pytest.raises(RuntimeError, match="0 and 1"):
         model(torch.zeros(4, 1, side, side, device=DEV))
+
+
+# one launch sets up to 16 blocks up and ends their weight gradients, another one more is set up layer by layer
+@pytest.mark.parametrize("blocks,kernels", [(1, 3), (16, 5), (17, 5)])
+def test_any_number_of_blocks(at_once, blocks, kernels):
+    torch.manual_seed(blocks)
+    model = C.ConvLogicMnistModel(k_param=8)
+    channels = [2] + [kernels] * blocks
+    model.network = torch.nn.Sequential(*(C.ConvLogicLayer(a, b, kernel=3, padding=2, complete=True, implementation="cuda") for a, b in zip(channels, channels[1:])),
+                                        torch.nn.Flatten(), *(C.LogicLayer(a, b, implementation="cuda") for a, b in ((4 * kernels, 80), (80, 40), (40, 20))),
+                                        C.GroupSum(10))
+    model = model.to(DEV)
+    x = torch.rand(37, 2, 2, 2, device=DEV).requires_grad_(True)     # (2 x 2 images stay 2 x 2)
+    tensors, gy = [x, *model.parameters()], torch.randn(37, 10, device=DEV)
+    y, grads = step(model, x, gy, tensors, False)
+    y0, grads0 = step(model, x, gy, tensors, True)
+    assert at_once == [True] and torch.equal(y, y0) and all(torch.equal(a, b) for a, b in zip(grads, grads0, strict=True))
