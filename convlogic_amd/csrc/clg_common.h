@@ -33,7 +33,7 @@ void clg_set_error(const char *fmt, ...);
 // (C ABI) reads them again after the environment was changed.
 #define CLG_KNOBS(X)                                                                                                   \
     X(BWDW_CELLS) X(BWDW_PADDED) X(BWDX_PLANES) X(BWDX_BANDS) X(BWDX_CSR) X(BWDX_DIRECT) X(BWDX_HSW) X(BWDX_SPLIT) X(BWD_4X4)         \
-    X(EVAL_CHUNK_BYTES) X(EVAL_NPW) X(EVAL_WALK_R) X(EVAL_WALK_SEG) X(FWD_4X4) X(FWD_CT) X(FWD_DIRECT) X(FWD_NW)       \
+    X(EVAL_ROWS) X(EVAL_CHUNK_BYTES) X(EVAL_NPW) X(EVAL_WALK_R) X(EVAL_WALK_SEG) X(FWD_4X4) X(FWD_CT) X(FWD_DIRECT) X(FWD_NW)       \
     X(FWD_ONE_ROW) X(FWD_S) X(FWD_SOFTMAX_IN_KERNEL) X(FWD_SUBSET) X(GSUM_SLICES) X(PACKED_4X4_HALVES) X(PACK_TILE)    \
     X(BWDW_LDS) X(BIN_CT) X(BIN_S) X(BIN_NW) X(BIN_HSW) X(BIN_PARTS) X(BIN_PIECE) X(BIN_HL) X(FWD_KPL) X(FWD_PAIR) X(BWDW_PAIR)
 enum ClgKnob {
@@ -51,6 +51,20 @@ static inline hipStream_t clg_stream(void *s) { return reinterpret_cast<hipStrea
 constexpr int kWave = 64;  // CDNA wavefront
 
 // ---- device side ---------------------------------------------------------------------------
+// Division of a 31-bit value by a runtime constant: q = umulhi(x, mul) >> shr (d == 1: q = x).
+struct FastDiv {
+    uint32_t mul, shr, d;
+};
+static inline FastDiv make_fastdiv(uint32_t d)
+{
+    if (d <= 1) return FastDiv{0, 0, 1};
+    uint32_t lg = 0;
+    while ((1ull << lg) < d) ++lg;
+    const uint32_t p = 31 + lg;
+    const uint32_t mul = (uint32_t)(((1ull << p) + d - 1) / d);
+    return FastDiv{mul, p - 32, d};
+}
+
 #if defined(__HIPCC__)
 
 template <typename T>
@@ -243,6 +257,8 @@ __device__ __forceinline__ Tap unpack_tap(int32_t s, const TapLimit &lim)
     return Tap{tap_channel(s, lim.cin), min((s >> 8) & 0xFF, lim.kh - 1), min(s & 0xFF, lim.kw - 1)};
 }
 
+__device__ __forceinline__ uint32_t fdiv(uint32_t x, const FastDiv &f) { return f.d == 1 ? x : (__umulhi(x, f.mul) >> f.shr); }
+
 // ---- bitwise gates on packed samples ---------------------------------------------------------
 struct Masks {
     uint32_t f00, f01, f10, f11;  // all-ones / all-zeros per truth-table entry
@@ -264,5 +280,32 @@ __device__ __forceinline__ V gate_vec(const Masks &m, V a, V b)
     return (a & t1) | (~a & t0);
 }
 __device__ __forceinline__ uint32_t gate_bits(const Masks &m, uint32_t a, uint32_t b) { return gate_vec<uint32_t>(m, a, b); }
+
+
+// (vectors at any 4-byte boundary, which is all that a wide access to global memory needs: rows of an odd number of samples)
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// Index of the first maximum of 16 logits (a NaN counts as the maximum), as clg_gate_argmax, by four lanes: `mine` are the logits 4 (lane
+// & 3) .. + 3.  Valid in all four.  Values compare as integers: -0 and +0 equal, NaN on top.
+__device__ __forceinline__ int argmax16_quad(f32x4u mine)
+{
+    const float v[4] = {mine.x, mine.y, mine.z, mine.w};
+    uint32_t best = 0;
+    int at = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t u = __builtin_bit_cast(uint32_t, v[i] + 0.0f);
+        const uint32_t key = v[i] != v[i] ? 0xFFFFFFFFu : (u ^ ((u >> 31) ? 0xFFFFFFFFu : 0x80000000u));
+        if (i == 0 || key > best) best = key, at = i;
+    }
+    at += 4 * (threadIdx.x & 3);
+#pragma unroll
+    for (int by = 1; by <= 2; by <<= 1) {
+        const uint32_t key = by == 1 ? dpp_zero<0xB1, 0xF>(best) : dpp_zero<0x4E, 0xF>(best);
+        const int other = (int)(by == 1 ? dpp_zero<0xB1, 0xF>((uint32_t)at) : dpp_zero<0x4E, 0xF>((uint32_t)at));
+        if (key > best || (key == best && other < at)) best = key, at = other;
+    }
+    return at;
+}
 
 #endif  // __HIPCC__

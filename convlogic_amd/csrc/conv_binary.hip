@@ -96,7 +96,6 @@ __device__ __forceinline__ void transpose_bits8(uint32_t (&t)[8])
 #undef CLG_SWAP
 }
 
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u32x2u __attribute__((ext_vector_type(2), aligned(4)));
 typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
 

@@ -5,21 +5,6 @@
 
 constexpr int kLdsLimit = 160 * 1024;
 
-// Division of a 31-bit value by a runtime constant: q = umulhi(x, mul) >> shr (d == 1: q = x).
-struct FastDiv {
-    uint32_t mul, shr, d;
-};
-static inline FastDiv make_fastdiv(uint32_t d)
-{
-    if (d <= 1) return FastDiv{0, 0, 1};
-    uint32_t lg = 0;
-    while ((1ull << lg) < d) ++lg;
-    const uint32_t p = 31 + lg;
-    const uint32_t mul = (uint32_t)(((1ull << p) + d - 1) / d);
-    return FastDiv{mul, p - 32, d};
-}
-__device__ __forceinline__ uint32_t fdiv(uint32_t x, const FastDiv &f) { return f.d == 1 ? x : (__umulhi(x, f.mul) >> f.shr); }
-
 struct TilePlan {
     int S;              // samples per workgroup
     int G;              // samples sharing one wavefront pass (input gradient; 1 when a sample has >= 64 cells)

@@ -7,9 +7,6 @@
 
 namespace {
 
-// (vectors at any 4-byte boundary, which is all that a wide access to global memory needs: rows of an odd number of samples)
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
-
 // ---- coefficients ---------------------------------------------------------------------------------------------------
 // ids [roots][8]: the neurons of a tree, 0..3 of the first layer, 4..5 of the second; the root is neuron j of the third.
 // coef [roots][7][4]: fold16 of the softmax (training) or of the arg-max gate (evaluation) of their logits, in tree order, so

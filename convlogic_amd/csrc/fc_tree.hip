@@ -117,28 +117,6 @@ __device__ __forceinline__ const float *tree_logits(const TreeLogits &lg, const 
 {
     return (q < 4 ? lg.l[0] : (q < 6 ? lg.l[1] : lg.l[2])) + tree_neuron(ids, j, q, roots) * 16;
 }
-// Index of the first maximum of 16 logits (a NaN counts as the maximum), as clg_gate_argmax, by four lanes: `mine` are the logits 4 (lane
-// & 3) .. + 3.  Valid in all four.  Values compare as integers: -0 and +0 equal, NaN on top.
-__device__ __forceinline__ int argmax16_quad(f32x4u mine)
-{
-    const float v[4] = {mine.x, mine.y, mine.z, mine.w};
-    uint32_t best = 0;
-    int at = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t u = __builtin_bit_cast(uint32_t, v[i] + 0.0f);
-        const uint32_t key = v[i] != v[i] ? 0xFFFFFFFFu : (u ^ ((u >> 31) ? 0xFFFFFFFFu : 0x80000000u));
-        if (i == 0 || key > best) best = key, at = i;
-    }
-    at += 4 * (threadIdx.x & 3);
-#pragma unroll
-    for (int by = 1; by <= 2; by <<= 1) {
-        const uint32_t key = by == 1 ? dpp_zero<0xB1, 0xF>(best) : dpp_zero<0x4E, 0xF>(best);
-        const int other = (int)(by == 1 ? dpp_zero<0xB1, 0xF>((uint32_t)at) : dpp_zero<0x4E, 0xF>((uint32_t)at));
-        if (key > best || (key == best && other < at)) best = key, at = other;
-    }
-    return at;
-}
 __global__ __launch_bounds__(256) void fc_tree_fold_kernel(TreeFold f) { tree_fold(f, blockIdx.x); }
 
 // ---- forward ----------------------------------------------------------------------------------------------------------

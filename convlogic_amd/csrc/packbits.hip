@@ -6,6 +6,8 @@
 // and truth-table masks are wave-uniform) over a column chunk of its two input rows.
 #include <stdlib.h>
 
+#include <algorithm>
+
 #include "clg_common.h"
 
 namespace {
@@ -32,8 +34,7 @@ __device__ __forceinline__ int argmax16_uniform(float v)
 // the chunk as the slow index, so that all neurons of one column chunk run back to back and the
 // second read of an input row segment finds it in the last-level cache.
 // LOGITS: `gate` points to float32 logits [out_dim, 16] and the wavefront takes their arg-max itself, else to uint8 gate ids.
-// Short rows are bound by the chain index -> rows -> store of one wavefront, which hides the logits' load behind the rows';
-// 8000 neurons on rows of 313 4-byte words: 9.0 us, against 8.6 + 4.0 us with a launch for the gate ids.
+// Long rows of whole 16-byte vectors come here where there is no walk of the wiring, and rows below 16 bytes; the rest: eval_packed_rows_kernel.
 template <typename V, int UNROLL, bool LOGITS>
 __global__ __launch_bounds__(kEvalBlock) void eval_packed_kernel(const V *__restrict__ x, const int64_t *__restrict__ a,
                                                                const int64_t *__restrict__ b,
@@ -77,6 +78,57 @@ __global__ __launch_bounds__(kEvalBlock) void eval_packed_kernel(const V *__rest
     }
 }
 
+// Short rows: lanes run along the 16-byte pieces of `nj` neurons of the workgroup, all of them in flight at once, so that neither lanes without a
+// piece nor one round of loads after the other are paid for; four lanes per neuron find its gate meanwhile.  Rows of any number of bytes from 16 on: the
+// last piece of a row steps back to its last 16 bytes, some of which two lanes write then (the same values).  us per layer, a wavefront per neuron or a walk
+// -> here: 64000 neurons on rows of 64 bytes 15.7 -> 4.1, of 252 18.3 -> 9.6, 8000 on 1280 7.7 -> 4.4; one piece of a thread at a time instead of two
+// costs up to 10 %, stores that stay in the caches up to 25 (64000 on 8188: 250 us, 218).
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
+constexpr int kRowsMax = 64, kRowsUnroll = 2;                        // neurons of a workgroup, pieces of a thread
+template <bool LOGITS>
+__global__ __launch_bounds__(kEvalBlock) void eval_packed_rows_kernel(const uint8_t *__restrict__ x, const int64_t *__restrict__ a,
+                                                                    const int64_t *__restrict__ b, const void *__restrict__ gate,
+                                                                    uint8_t *__restrict__ y, int out_dim, int64_t row_bytes, uint32_t pieces,
+                                                                    FastDiv d_pieces, int nj, int64_t in_dim)
+{
+    __shared__ int ids[kRowsMax];
+    const int j0 = blockIdx.x * nj, here = min(nj, out_dim - j0), q = threadIdx.x >> 2;
+    const uint32_t total = (uint32_t)here * pieces;
+    f32x4u logits = 0.f;                                              // requested ahead of the rows: vector loads return in order
+    if (LOGITS && q < here) logits = reinterpret_cast<const f32x4u *>(reinterpret_cast<const float *>(gate) + (int64_t)(j0 + q) * 16)[threadIdx.x & 3];
+    u32x4 ra[kRowsUnroll], rb[kRowsUnroll];
+    int jn[kRowsUnroll];
+    int64_t off[kRowsUnroll];
+    auto request = [&](uint32_t first) {
+#pragma unroll
+        for (int u = 0; u < kRowsUnroll; ++u) {
+            const uint32_t e = first + u * kEvalBlock + threadIdx.x, ec = e < total ? e : 0;
+            jn[u] = (int)fdiv(ec, d_pieces);
+            off[u] = min((int64_t)(ec - jn[u] * pieces) * 16, row_bytes - 16);
+            ra[u] = *reinterpret_cast<const u32x4_any *>(x + clamp_index(a[j0 + jn[u]], in_dim) * row_bytes + off[u]);
+            rb[u] = *reinterpret_cast<const u32x4_any *>(x + clamp_index(b[j0 + jn[u]], in_dim) * row_bytes + off[u]);
+        }
+    };
+    request(0);
+    if constexpr (LOGITS) {
+        const int id = argmax16_quad(logits);
+        if ((threadIdx.x & 3) == 0 && q < here) ids[q] = id;
+    } else {
+        if ((int)threadIdx.x < here) ids[threadIdx.x] = reinterpret_cast<const uint8_t *>(gate)[j0 + threadIdx.x];
+    }
+    __syncthreads();
+    for (uint32_t first = 0;;) {
+#pragma unroll
+        for (int u = 0; u < kRowsUnroll; ++u)
+            if (first + u * kEvalBlock + threadIdx.x < total)
+                __builtin_nontemporal_store((u32x4_any)gate_vec(gate_masks(ids[jn[u]]), ra[u], rb[u]),
+                                            reinterpret_cast<u32x4_any *>(y + (int64_t)(j0 + jn[u]) * row_bytes + off[u]));
+        first += kRowsUnroll * kEvalBlock;
+        if (first >= total) return;
+        request(first);
+    }
+}
+
 // ---------------------------------------------------------------------------------------------
 // evaluation along a precomputed walk of the wiring graph
 // ---------------------------------------------------------------------------------------------
@@ -101,12 +153,13 @@ __device__ __forceinline__ int gate_id_uniform(const uint8_t *__restrict__ gate,
 
 // LOGITS: `gate` points to float32 logits [out_dim, 16] and the wavefront takes their arg-max itself (the layer's eval
 // call then needs no launch of its own for the gate ids); else to uint8 gate ids [out_dim].
+// Rows of any number of bytes from 16 on, row_vecs vectors of 16 bytes, the last of which steps back to the row's last 16 bytes.
 template <int R, bool LOGITS>
-__global__ __launch_bounds__(kEvalBlock) void eval_packed_walk_kernel(const u32x4 *__restrict__ x, const int64_t *__restrict__ a,
+__global__ __launch_bounds__(kEvalBlock) void eval_packed_walk_kernel(const uint8_t *__restrict__ x, const int64_t *__restrict__ a,
                                                                     const int64_t *__restrict__ b,
                                                                     const void *__restrict__ gate,
-                                                                    const int32_t *__restrict__ plan, u32x4 *__restrict__ y,
-                                                                    int steps, int seg_len, int64_t row_vecs, int64_t in_dim)
+                                                                    const int32_t *__restrict__ plan, uint8_t *__restrict__ y,
+                                                                    int steps, int seg_len, int64_t row_vecs, int64_t row_bytes, int64_t in_dim)
 {
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = uniform(threadIdx.x >> 6);
@@ -114,6 +167,9 @@ __global__ __launch_bounds__(kEvalBlock) void eval_packed_walk_kernel(const u32x
     if (k0 >= steps) return;
     const int k1 = k0 + seg_len < steps ? k0 + seg_len : steps;
     const int64_t col0 = (int64_t)blockIdx.y * (kWave * R) + lane;   // this lane's first vector in the row
+    int64_t at[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) at[r] = min((col0 + r * kWave) * 16, row_bytes - 16);
     u32x4 ra[R], rb[R], carry[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) carry[r] = (u32x4)0u;
@@ -121,14 +177,14 @@ __global__ __launch_bounds__(kEvalBlock) void eval_packed_walk_kernel(const u32x
         const int p = plan[k];
         const int j = min(p & 0x0FFFFFFF, steps - 1), keep = (p >> 30) & 1;   // one plan entry per neuron
         const int use = k == k0 ? 0 : (p >> 28) & 3;
-        const u32x4 *xa = x + clamp_index(a[j], in_dim) * row_vecs + col0;
-        const u32x4 *xb = x + clamp_index(b[j], in_dim) * row_vecs + col0;
+        const uint8_t *xa = x + clamp_index(a[j], in_dim) * row_bytes;
+        const uint8_t *xb = x + clamp_index(b[j], in_dim) * row_bytes;
         float logit = 0.f;                                            // requested ahead of the rows: vector loads return in order
         if constexpr (LOGITS) logit = reinterpret_cast<const float *>(gate)[(int64_t)j * 16 + (lane & 15)];
         if (use != 1 && use != 3) {
 #pragma unroll
             for (int r = 0; r < R; ++r)
-                if (col0 + r * kWave < row_vecs) ra[r] = xa[r * kWave];
+                if (col0 + r * kWave < row_vecs) ra[r] = *reinterpret_cast<const u32x4_any *>(xa + at[r]);
         } else {
 #pragma unroll
             for (int r = 0; r < R; ++r) ra[r] = carry[r];
@@ -136,7 +192,7 @@ __global__ __launch_bounds__(kEvalBlock) void eval_packed_walk_kernel(const u32x
         if (use < 2) {
 #pragma unroll
             for (int r = 0; r < R; ++r)
-                if (col0 + r * kWave < row_vecs) rb[r] = xb[r * kWave];
+                if (col0 + r * kWave < row_vecs) rb[r] = *reinterpret_cast<const u32x4_any *>(xb + at[r]);
         } else {
 #pragma unroll
             for (int r = 0; r < R; ++r) rb[r] = carry[r];
@@ -145,10 +201,10 @@ __global__ __launch_bounds__(kEvalBlock) void eval_packed_walk_kernel(const u32x
         if constexpr (LOGITS) id = argmax16_uniform(logit);
         else id = gate_id_uniform(reinterpret_cast<const uint8_t *>(gate), j, steps);
         const Masks m = gate_masks(id);
-        u32x4 *yj = y + (int64_t)j * row_vecs + col0;
+        uint8_t *yj = y + (int64_t)j * row_bytes;
 #pragma unroll
         for (int r = 0; r < R; ++r)
-            if (col0 + r * kWave < row_vecs) __builtin_nontemporal_store(gate_vec(m, ra[r], rb[r]), yj + r * kWave);
+            if (col0 + r * kWave < row_vecs) __builtin_nontemporal_store((u32x4_any)gate_vec(m, ra[r], rb[r]), reinterpret_cast<u32x4_any *>(yj + at[r]));
 #pragma unroll
         for (int r = 0; r < R; ++r) carry[r] = keep ? rb[r] : ra[r];
     }
@@ -640,6 +696,26 @@ void launch_eval(const void *x, const int64_t *a, const int64_t *b, const void *
                        b, gate, (V *)y, (int)out_dim, row_vecs, chunk_vecs, groups, neurons_per_wave, in_dim);
 }
 
+template <bool LOGITS>
+void launch_rows(const void *x, const int64_t *a, const int64_t *b, const void *gate, void *y, int64_t out_dim, int64_t row_bytes, hipStream_t st,
+                 int64_t in_dim)
+{
+    const uint32_t pieces = (uint32_t)clg_ceil_div(row_bytes, 16);
+    const int nj = (int)std::max<int64_t>(1, std::min<int64_t>(kRowsMax, kRowsUnroll * kEvalBlock / pieces));
+    hipLaunchKernelGGL(eval_packed_rows_kernel<LOGITS>, dim3((unsigned)clg_ceil_div(out_dim, nj)), dim3(kEvalBlock), 0, st, (const uint8_t *)x, a, b, gate,
+                       (uint8_t *)y, (int)out_dim, row_bytes, pieces, make_fastdiv(pieces), nj, in_dim);
+}
+
+// Layers whose rows are read once along a walk of the wiring (the others twice, but all at once): us at [neurons] x bytes, lanes along several neurons' rows
+// against the walk: [8000] x 3000 11.5 and 12.4, x 5000 18.5 and 17.3, [16000] x 1528 11.8 and 12.2, [32000] x 1020 15.9 and 15.3,
+// [64000] x 500 17.0 and 17.5, x 768 22.3 and 20.7, [16000] x 8188 56 and 49; below 30 MB a wavefront's chain of eight neurons is what a walk takes
+// ([2000] x 1280 3.9 and 7.3).
+bool walk_pays(int64_t row_bytes, int64_t out_dim)
+{
+    if (const char *e = clg_knob(K_EVAL_ROWS)) return atoi(e) == 0;
+    return row_bytes >= 640 && row_bytes * out_dim >= 30'000'000;
+}
+
 bool valid_elem(int e) { return e == 1 || e == 2 || e == 4 || e == 8; }
 
 }  // namespace
@@ -659,8 +735,10 @@ static int eval_packed(const char *name, int elem_size, const void *x, const int
     hipStream_t st = clg_stream(stream);
     const int64_t blocks_needed = clg_ceil_div(row_bytes, 2048) * clg_ceil_div(out_dim, 16);
     CLG_REQUIRE(blocks_needed < (1ll << 31), "%s: problem too large for one launch (%lld blocks)", name, (long long)blocks_needed);
-    if ((align & 15) == 0) launch_eval<u32x4, LOGITS>(x, a, b, gate, y, out_dim, row_bytes, st, in_dim);
-    else if ((align & 7) == 0) launch_eval<u32x2, LOGITS>(x, a, b, gate, y, out_dim, row_bytes, st, in_dim);
+    // without a plan, long rows of whole vectors go a wavefront per neuron and 4 KiB ([64000] x 8192: 196 us, 212 by pieces)
+    const bool whole = (align & 15) == 0 && row_bytes >= 1024 && walk_pays(row_bytes, out_dim);
+    if (row_bytes >= 16 && row_bytes < (1ll << 34) && !whole) launch_rows<LOGITS>(x, a, b, gate, y, out_dim, row_bytes, st, in_dim);
+    else if ((align & 15) == 0) launch_eval<u32x4, LOGITS>(x, a, b, gate, y, out_dim, row_bytes, st, in_dim);
     else if ((align & 3) == 0) launch_eval<uint32_t, LOGITS>(x, a, b, gate, y, out_dim, row_bytes, st, in_dim);
     else if constexpr (LOGITS)
         CLG_REQUIRE(false, "%s: rows must be whole 4-byte words at 4-byte aligned addresses; use clg_gate_argmax + clg_fc_eval_packed "
@@ -681,6 +759,8 @@ extern "C" int clg_fc_eval_packed(int elem_size, const void *x, const int64_t *a
 extern "C" int clg_fc_eval_packed_logits(int elem_size, const void *x, const int64_t *a, const int64_t *b, const float *logits,
                                          void *y, int64_t in_dim, int64_t out_dim, int64_t words, void *stream)
 {
+    CLG_REQUIRE((((uintptr_t)x | (uintptr_t)y | (uintptr_t)(words * elem_size)) & 3) == 0, "clg_fc_eval_packed_logits: rows must be whole 4-byte words at "
+                "4-byte aligned addresses; use clg_gate_argmax + clg_fc_eval_packed otherwise");
     return eval_packed<true>("clg_fc_eval_packed_logits", elem_size, x, a, b, logits, y, in_dim, out_dim, words, stream);
 }
 
@@ -897,7 +977,7 @@ template <bool LOGITS>
 int launch_walk(const char *name, int elem_size, const void *x, const int64_t *a, const int64_t *b, const void *gate, const int32_t *plan,
                 void *y, int64_t in_dim, int64_t out_dim, int64_t words, void *stream)
 {
-    const int64_t row_vecs = words * elem_size / 16;
+    const int64_t row_bytes = words * elem_size, row_vecs = clg_ceil_div(row_bytes, 16);
     const char *e_r = clg_knob(K_EVAL_WALK_R), *e_l = clg_knob(K_EVAL_WALK_SEG);
     int R = e_r ? atoi(e_r) : 4;
     while (R > 1 && (int64_t)kWave * (R / 2) >= row_vecs) R /= 2;
@@ -907,8 +987,8 @@ int launch_walk(const char *name, int elem_size, const void *x, const int64_t *a
     const dim3 grid((unsigned)clg_ceil_div(out_dim, (int64_t)kEvalWaves * seg), (unsigned)col_chunks), block(kEvalBlock);
     hipStream_t st = clg_stream(stream);
 #define CLG_WALK(RR)                                                                                                          \
-    hipLaunchKernelGGL((eval_packed_walk_kernel<RR, LOGITS>), grid, block, 0, st, (const u32x4 *)x, a, b, gate, plan, (u32x4 *)y, \
-                       (int)out_dim, seg, row_vecs, in_dim)
+    hipLaunchKernelGGL((eval_packed_walk_kernel<RR, LOGITS>), grid, block, 0, st, (const uint8_t *)x, a, b, gate, plan, (uint8_t *)y, \
+                       (int)out_dim, seg, row_vecs, row_bytes, in_dim)
     switch (R) {
     case 1: CLG_WALK(1); break;
     case 2: CLG_WALK(2); break;
@@ -919,6 +999,7 @@ int launch_walk(const char *name, int elem_size, const void *x, const int64_t *a
     CLG_CHECK_LAUNCH(name);
     return CLG_OK;
 }
+
 }  // namespace
 
 extern "C" int clg_fc_eval_packed_planned(int elem_size, const void *x, const int64_t *a, const int64_t *b, const uint8_t *gate,
@@ -931,7 +1012,7 @@ extern "C" int clg_fc_eval_packed_planned(int elem_size, const void *x, const in
     CLG_REQUIRE(x != y, "%s: x and y must not overlap", name);
     CLG_REQUIRE(in_dim > 0 && out_dim > 0 && words > 0, "%s: in_dim, out_dim and words must be positive", name);
     CLG_REQUIRE(out_dim < (1ll << 28), "%s: out_dim above 2^28-1 is not supported", name);
-    if (!walk_fits(elem_size, x, y, words)) return clg_fc_eval_packed(elem_size, x, a, b, gate, y, in_dim, out_dim, words, stream);
+    if (words * elem_size < 16 || !walk_pays(words * elem_size, out_dim)) return clg_fc_eval_packed(elem_size, x, a, b, gate, y, in_dim, out_dim, words, stream);
     return launch_walk<false>(name, elem_size, x, a, b, gate, plan, y, in_dim, out_dim, words, stream);
 }
 
@@ -953,4 +1034,20 @@ extern "C" int clg_fc_eval_packed_planned_logits(int elem_size, const void *x, c
     CLG_REQUIRE(walk_fits(elem_size, x, y, words), "%s: rows must be whole 16-byte vectors of at least 1 KiB at 16-byte aligned addresses "
                 "(clg_fc_eval_walk_fits); use clg_gate_argmax + clg_fc_eval_packed_planned otherwise", name);
     return launch_walk<true>(name, elem_size, x, a, b, logits, plan, y, in_dim, out_dim, words, stream);
+}
+
+extern "C" int clg_fc_eval_packed_layer(int elem_size, const void *x, const int64_t *a, const int64_t *b, const float *logits, const int32_t *plan, void *y,
+                                        int64_t in_dim, int64_t out_dim, int64_t words, void *stream)
+{
+    const char *name = "clg_fc_eval_packed_layer";
+    CLG_REQUIRE(valid_elem(elem_size), "%s: elem_size must be 1, 2, 4 or 8, got %d", name, elem_size);
+    CLG_REQUIRE(x && a && b && logits && plan && y, "%s: null pointer argument", name);
+    CLG_REQUIRE(x != y, "%s: x and y must not overlap", name);
+    CLG_REQUIRE(in_dim > 0 && out_dim > 0 && words > 0, "%s: in_dim, out_dim and words must be positive", name);
+    CLG_REQUIRE(out_dim < (1ll << 28), "%s: out_dim above 2^28-1 is not supported", name);
+    const int64_t row_bytes = words * elem_size;
+    CLG_REQUIRE(row_bytes >= 16 || (((uintptr_t)x | (uintptr_t)y | (uintptr_t)row_bytes) & 3) == 0, "%s: rows must be 16 bytes or more, or whole 4-byte words at "
+                "4-byte aligned addresses; use clg_gate_argmax + clg_fc_eval_packed otherwise", name);
+    if (row_bytes >= 16 && walk_pays(row_bytes, out_dim)) return launch_walk<true>(name, elem_size, x, a, b, logits, plan, y, in_dim, out_dim, words, stream);
+    return eval_packed<true>(name, elem_size, x, a, b, logits, y, in_dim, out_dim, words, stream);
 }

@@ -388,9 +388,8 @@ def eval_planned(x, a, b, w, plan):
 
 
 def eval_planned_logits(x, a, b, logits, plan):
-    """eval_planned(x, a, b, gate_argmax(logits), plan) -- in one launch where the logits are float32 and the rows whole
-    4-byte words (the kernels take the arg-max themselves; in plan order where the walk kernel takes the rows: whole
-    16-byte vectors of at least 1 KiB), in two launches otherwise.
+    """eval_planned(x, a, b, gate_argmax(logits), plan) -- in one launch where the logits are float32 and the rows 16 bytes
+    or more, or whole 4-byte words (the kernels take the arg-max themselves, in plan order where that pays), in two launches otherwise.
     LogicLayer.forward_cuda_eval (src/difflogic/difflogic.py:149-164)."""
     if x.dtype not in _WORD_DTYPE.values() or plan.dtype != torch.int32 or logits.dim() != 2 or logits.shape[1] != 16:
         raise RuntimeError("eval_planned_logits expects int8/16/32/64 words, logits [out, 16] and an int32 plan")
@@ -403,14 +402,10 @@ def eval_planned_logits(x, a, b, logits, plan):
     lib = _lib.load()
     y = torch.empty((out_dim, words), dtype=x.dtype, device=x.device)
     elem = x.element_size()
-    if logits.dtype != torch.float32 or (x.data_ptr() | y.data_ptr() | (words * elem)) & 3:
+    if logits.dtype != torch.float32 or (words * elem < 16 and (x.data_ptr() | y.data_ptr() | (words * elem)) & 3):
         return eval_planned(x, a, b, gate_argmax(logits), plan)
-    if not lib.clg_fc_eval_walk_fits(elem, x.data_ptr(), y.data_ptr(), words):
-        check(lib.clg_fc_eval_packed_logits(elem, x.data_ptr(), a.data_ptr(), b.data_ptr(), logits.data_ptr(), y.data_ptr(), in_dim,
-                                            out_dim, words, stream_ptr(x)))
-        return y
-    check(lib.clg_fc_eval_packed_planned_logits(elem, x.data_ptr(), a.data_ptr(), b.data_ptr(), logits.data_ptr(),
-                                                plan.data_ptr(), y.data_ptr(), in_dim, out_dim, words, stream_ptr(x)))
+    check(lib.clg_fc_eval_packed_layer(elem, x.data_ptr(), a.data_ptr(), b.data_ptr(), logits.data_ptr(), plan.data_ptr(), y.data_ptr(), in_dim,
+                                       out_dim, words, stream_ptr(x)))
     return y
 
 

@@ -277,6 +277,10 @@ int clg_fc_eval_walk_fits(int elem_size, const void *x, const void *y, int64_t w
 int clg_fc_eval_packed_planned_logits(int elem_size, const void *x /*[in_dim,words]*/, const int64_t *a, const int64_t *b,
                                       const float *logits /*[out_dim,16]*/, const int32_t *plan /*[out_dim]*/,
                                       void *y /*[out_dim,words]*/, int64_t in_dim, int64_t out_dim, int64_t words, void *stream);
+/* The layer whatever its rows: along the plan where that pays, else lanes along the rows of several neurons.  Rows below 16 bytes must be
+ * whole 4-byte words at 4-byte aligned addresses. */
+int clg_fc_eval_packed_layer(int elem_size, const void *x, const int64_t *a, const int64_t *b, const float *logits, const int32_t *plan,
+                             void *y, int64_t in_dim, int64_t out_dim, int64_t words, void *stream);
 
 /* clg_gate_argmax + clg_fc_eval_packed in ONE launch, for rows the walk kernel does not take: the same gate ids from the 16
  * float32 logits of a neuron.  Rows must be whole 4-byte words at 4-byte aligned addresses (CLG_EINVAL otherwise; use the

@@ -80,6 +80,31 @@ def test_eval_packed_bit_exact(bits, batch):
     assert got.dtype == TORCH_WORD[bits] and np.array_equal(got.cpu().numpy(), want)
 
 
+# rows of 15 bytes up to more than a workgroup takes at once, whole vectors and not, at odd addresses; one neuron, more of them than a workgroup takes and one
+# more or less; both the kernel of short rows and the walk
+@pytest.mark.parametrize("rows_kernel", ["0", "1"])
+@pytest.mark.parametrize("bits,row_bytes,out_dim,offset", [(8, 15, 70, 1), (8, 16, 65, 1), (8, 17, 64, 3), (16, 62, 63, 2), (8, 253, 53, 5), (32, 252, 1, 4),
+                                                          (32, 500, 40, 0), (8, 1025, 33, 7), (64, 1024, 31, 8), (64, 4104, 17, 0), (32, 8196, 9, 4),
+                                                          (8, 8209, 8, 0), (64, 8192, 129, 0)])
+def test_eval_packed_rows_of_any_length(monkeypatch, bits, row_bytes, out_dim, offset, rows_kernel):
+    rng = np.random.default_rng(row_bytes)
+    torch.manual_seed(row_bytes)
+    in_dim, dtype = 41, TORCH_WORD[bits]
+    raw = rng.integers(0, 256, offset + in_dim * row_bytes, dtype=np.uint8)
+    x = torch.from_numpy(raw).to(DEV)[offset:].view(dtype).view(in_dim, -1)
+    words = raw[offset:].copy().view(x.cpu().numpy().dtype).reshape(in_dim, -1)
+    a, b = torch.randint(0, in_dim, (out_dim,), device=DEV), torch.randint(0, in_dim, (out_dim,), device=DEV)
+    logits = torch.randint(-2, 3, (out_dim, 16), device=DEV).float()  # (ties: the first maximum)
+    logits[out_dim // 2, 5] = float("nan")
+    gate, plan = difflogic_hip.gate_argmax(logits), difflogic_hip.eval_plan(a, b, in_dim)
+    want = O.eval_packed(words, a.cpu().numpy(), b.cpu().numpy(), gate.cpu().numpy())
+    set_knobs(monkeypatch, CLG_EVAL_ROWS=rows_kernel)
+    got = [difflogic_hip.eval_planned_logits(x, a, b, logits, plan), difflogic_hip.eval_planned(x, a, b, gate, plan), difflogic_hip.eval(x, a, b, gate)]
+    monkeypatch.undo()
+    _lib.reload_knobs()
+    assert all(np.array_equal(y.cpu().numpy(), want) for y in got)
+
+
 @pytest.mark.parametrize("bits,batch,features,k", [(64, 256, 40, 10), (32, 100, 12, 3), (8, 9, 4, 2), (64, 5000, 2000, 10), (16, 33, 6, 6),
                                                    (64, 4133, 84, 4), (32, 4200, 30, 3), (8, 600, 9, 1), (64, 8192, 2400, 4),
                                                    (64, 4096, 7, 7), (64, 4096, 40000, 2)])
