@@ -33,7 +33,7 @@ void clg_set_error(const char *fmt, ...);
 // (C ABI) reads them again after the environment was changed.
 #define CLG_KNOBS(X)                                                                                                   \
     X(BWDW_CELLS) X(BWDW_PADDED) X(BWDX_PLANES) X(BWDX_BANDS) X(BWDX_CSR) X(BWDX_DIRECT) X(BWDX_HSW) X(BWDX_SPLIT) X(BWD_4X4)         \
-    X(EVAL_ROWS) X(EVAL_CHUNK_BYTES) X(EVAL_NPW) X(EVAL_WALK_R) X(EVAL_WALK_SEG) X(FWD_4X4) X(FWD_CT) X(FWD_DIRECT) X(FWD_NW)       \
+    X(STREAM_MB) X(EVAL_ROWS) X(EVAL_CHUNK_BYTES) X(EVAL_NPW) X(EVAL_WALK_R) X(EVAL_WALK_SEG) X(FWD_4X4) X(FWD_CT) X(FWD_DIRECT) X(FWD_NW)       \
     X(FWD_ONE_ROW) X(FWD_S) X(FWD_SOFTMAX_IN_KERNEL) X(FWD_SUBSET) X(GSUM_SLICES) X(PACKED_4X4_HALVES) X(PACK_TILE)    \
     X(BWDW_LDS) X(BIN_CT) X(BIN_S) X(BIN_NW) X(BIN_HSW) X(BIN_PARTS) X(BIN_PIECE) X(BIN_HL) X(FWD_KPL) X(FWD_PAIR) X(BWDW_PAIR)
 enum ClgKnob {
@@ -51,6 +51,14 @@ static inline hipStream_t clg_stream(void *s) { return reinterpret_cast<hipStrea
 constexpr int kWave = 64;  // CDNA wavefront
 
 // ---- device side ---------------------------------------------------------------------------
+// Whether a buffer of so many bytes that one kernel writes and a later one reads once goes past the L2 caches (nontemporal accesses): from `mb` on it
+// does not stay there, and its lines push out what the kernels read again and again.
+static inline bool clg_past_caches(int64_t bytes, int64_t mb)
+{
+    const char *e = clg_knob(K_STREAM_MB);
+    return bytes >= (e ? atoll(e) : mb) << 20;
+}
+
 // Division of a 31-bit value by a runtime constant: q = umulhi(x, mul) >> shr (d == 1: q = x).
 struct FastDiv {
     uint32_t mul, shr, d;
@@ -258,6 +266,20 @@ __device__ __forceinline__ Tap unpack_tap(int32_t s, const TapLimit &lim)
 }
 
 __device__ __forceinline__ uint32_t fdiv(uint32_t x, const FastDiv &f) { return f.d == 1 ? x : (__umulhi(x, f.mul) >> f.shr); }
+
+// (STREAM: clg_past_caches.  A template argument: of a run-time choice the compiler makes one plain access.)
+template <bool STREAM, typename V>
+__device__ __forceinline__ void store_vec(V *p, V v)
+{
+    if constexpr (STREAM) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+template <bool STREAM, typename V>
+__device__ __forceinline__ V load_vec(const V *p)
+{
+    if constexpr (STREAM) return __builtin_nontemporal_load(p);
+    else return *p;
+}
 
 // ---- bitwise gates on packed samples ---------------------------------------------------------
 struct Masks {

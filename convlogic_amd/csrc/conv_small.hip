@@ -345,7 +345,7 @@ __global__ __launch_bounds__(kLsWaves *kWave, 2) void convblock_eval_packed_4x4_
 constexpr int kGradStride = kLsPlane + kLsRow + 1; // gradient plane (taps of border cells fall into the halo); odd
 
 // the gradients of a tap at the 4 cells of a sample, as 16-byte pieces
-template <typename T>
+template <bool STREAM, typename T>
 __device__ __forceinline__ void store_cells(T *dst, const T *v)
 {
     constexpr int PER = 16 / (int)sizeof(T);
@@ -353,22 +353,22 @@ __device__ __forceinline__ void store_cells(T *dst, const T *v)
     for (int q = 0; q < 4 / PER; ++q) {
         u32x4 raw;
         __builtin_memcpy(&raw, v + q * PER, 16);
-        reinterpret_cast<u32x4 *>(dst)[q] = raw;
+        store_vec<STREAM>(reinterpret_cast<u32x4 *>(dst) + q, raw);
     }
 }
-template <typename T>
+template <bool STREAM, typename T>
 __device__ __forceinline__ void load_cells(T *v, const T *src)
 {
     constexpr int PER = 16 / (int)sizeof(T);
 #pragma unroll
     for (int q = 0; q < 4 / PER; ++q) {
-        const u32x4 raw = reinterpret_cast<const u32x4 *>(src)[q];
+        const u32x4 raw = load_vec<STREAM>(reinterpret_cast<const u32x4 *>(src) + q);
         __builtin_memcpy(v + q * PER, &raw, 16);
     }
 }
 
 // The wavefronts of a workgroup (1, 2 or 4) deal the 64-sample blocks among themselves.
-template <typename T>
+template <typename T, bool STREAM>
 __global__ __launch_bounds__(kLsWaves *kWave, sizeof(T) == 4 ? 3 : 1) void convblock_backward_4x4_kernel(
     const T *__restrict__ x, const T *__restrict__ folded, const int32_t *__restrict__ sel, const T *__restrict__ gy,
     const uint8_t *__restrict__ argmax, T *__restrict__ tg, uint32_t *__restrict__ tcodes, T *__restrict__ gw,
@@ -488,7 +488,7 @@ __global__ __launch_bounds__(kLsWaves *kWave, sizeof(T) == 4 ? 3 : 1) void convb
             }
             if (dst) {
 #pragma unroll
-                for (int k = 0; k < 8; ++k) store_cells(dst + k * tap_step, &gt[4 * k]);
+                for (int k = 0; k < 8; ++k) store_cells<STREAM>(dst + k * tap_step, &gt[4 * k]);
             }
         }
         // 28 sums of this kernel: lanes, then the wavefronts in order
@@ -514,7 +514,7 @@ __global__ __launch_bounds__(kLsWaves *kWave, sizeof(T) == 4 ? 3 : 1) void convb
 
 // grid: (64-sample blocks x channels) / kLsWaves.  count[2 ch] = kernels that read the channel, count[2 ch + 1] = where
 // their list starts in hits; an entry is kernel | tap mask << 16.
-template <typename T>
+template <typename T, bool STREAM>
 __global__ __launch_bounds__(kLsWaves *kWave) void convblock_backward_x_4x4_kernel(const T *__restrict__ tg,
                                                                                  const int32_t *__restrict__ count,
                                                                                  const int32_t *__restrict__ hits,
@@ -572,7 +572,7 @@ __global__ __launch_bounds__(kLsWaves *kWave) void convblock_backward_x_4x4_kern
             const uint32_t p = (uint32_t)__builtin_amdgcn_readlane(pair, last);
             const int c = p >> 16, t = (p >> 8) & 7;
             off[u] = p & 0xFF;
-            load_cells(val[u], tg + (((int64_t)c * 8 + t) * g.n + ns) * 4);
+            load_cells<STREAM>(val[u], tg + (((int64_t)c * 8 + t) * g.n + ns) * 4);
             code[u] = tcodes[(int64_t)c * g.n + ns];
         };
 #pragma unroll
@@ -610,7 +610,7 @@ __global__ __launch_bounds__(kLsWaves *kWave) void convblock_backward_x_4x4_kern
         for (int e = 0; e < 16; ++e) out[e] = plane[ls_at((e >> 2) + 1, (e & 3) + 1)];
         T *dst = gx + (n * g.cin + ch) * 16;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) store_cells(dst + 4 * q, &out[4 * q]);
+        for (int q = 0; q < 4; ++q) store_cells<false>(dst + 4 * q, &out[4 * q]);
     }
 }
 
@@ -686,9 +686,13 @@ static int launch_backward_4x4(const Geom &g, const void *x, const void *folded,
     while (ct > 1 && (g.c + ct - 1) / ct < 1024) ct >>= 1;
     const int sblocks = (g.n + kWave - 1) / kWave, waves = sblocks >= 4 ? 4 : (sblocks >= 2 ? 2 : 1);   // none without samples
     const size_t lds = (size_t)waves * kWave * kLsStride * sizeof(T);
-    if (int e = allow_lds(convblock_backward_4x4_kernel<T>, lds + 1024, name)) return e;
+    // (a step of the CIFAR topology, us without and with: 25 MB 248 and 250, 32 MB 282 and 270, 50 MB 425 and 416, 512 MB 44 less; samples
+    // that are not whole lines within 1 % either way)
+    const bool stream = clg_past_caches((int64_t)tg_elems_bytes(sizeof(T) == 8 ? CLG_F64 : CLG_F32, g), g.n % 8 == 0 ? 30 : 400);
     uint32_t *tcodes = reinterpret_cast<uint32_t *>(reinterpret_cast<unsigned char *>(tg) + tg_elems_bytes(sizeof(T) == 8 ? CLG_F64 : CLG_F32, g));
-    hipLaunchKernelGGL(convblock_backward_4x4_kernel<T>, dim3((unsigned)((g.c + ct - 1) / ct)), dim3(waves * kWave), lds, st,
+    auto main_kern = stream ? convblock_backward_4x4_kernel<T, true> : convblock_backward_4x4_kernel<T, false>;
+    if (int e = allow_lds(main_kern, lds + 1024, name)) return e;
+    hipLaunchKernelGGL(main_kern, dim3((unsigned)((g.c + ct - 1) / ct)), dim3(waves * kWave), lds, st,
                        (const T *)x, (const T *)folded, sel, (const T *)gy, argmax, gx != nullptr ? (T *)tg : (T *)nullptr, tcodes, (T *)gw,
                        (const T *)probs, g, ct);
     CLG_CHECK_LAUNCH(name);
@@ -696,9 +700,10 @@ static int launch_backward_4x4(const Geom &g, const void *x, const void *folded,
     const int64_t items = (int64_t)((g.n + kWave - 1) / kWave) * g.cin;
     CLG_REQUIRE((items + kLsWaves - 1) / kLsWaves < (1ll << 31), "%s: too many (sample block, channel) pairs for one launch", name);
     const size_t lds_x = (size_t)kLsWaves * kWave * kGradStride * sizeof(T);
-    if (int e = allow_lds(convblock_backward_x_4x4_kernel<T>, lds_x, name)) return e;
-    hipLaunchKernelGGL(convblock_backward_x_4x4_kernel<T>, dim3((unsigned)((items + kLsWaves - 1) / kLsWaves)), dim3(kLsWaves * kWave),
-                       lds_x, st, (const T *)tg, count, hits, sel, (const uint32_t *)tcodes, (T *)gx, g);
+    auto kern = stream ? convblock_backward_x_4x4_kernel<T, true> : convblock_backward_x_4x4_kernel<T, false>;
+    if (int e = allow_lds(kern, lds_x, name)) return e;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((items + kLsWaves - 1) / kLsWaves)), dim3(kLsWaves * kWave), lds_x, st, (const T *)tg, count, hits, sel,
+                       (const uint32_t *)tcodes, (T *)gx, g);
     CLG_CHECK_LAUNCH(name);
     return CLG_OK;
 }

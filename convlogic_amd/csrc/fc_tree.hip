@@ -50,15 +50,15 @@ template <>
 struct SamplesRaw<2> { using type = f32x2u; };
 template <>
 struct SamplesRaw<4> { using type = f32x4u; };
-template <int V>
+template <int V, bool STREAM = false>
 __device__ __forceinline__ Samples<V> load_samples(const float *p)
 {
-    return __builtin_bit_cast(Samples<V>, *reinterpret_cast<const typename SamplesRaw<V>::type *>(p));
+    return __builtin_bit_cast(Samples<V>, load_vec<STREAM>(reinterpret_cast<const typename SamplesRaw<V>::type *>(p)));
 }
-template <int V>
+template <int V, bool STREAM = false>
 __device__ __forceinline__ void store_samples(float *p, const Samples<V> &v)
 {
-    *reinterpret_cast<typename SamplesRaw<V>::type *>(p) = __builtin_bit_cast(typename SamplesRaw<V>::type, v);
+    store_vec<STREAM>(reinterpret_cast<typename SamplesRaw<V>::type *>(p), __builtin_bit_cast(typename SamplesRaw<V>::type, v));
 }
 // Where the lane whose samples begin at s reads and writes: the last lane of a row whose length V does not divide steps back to the
 // last V samples, which it shares with its neighbour (the same values, computed twice); lanes behind the row: 0.
@@ -219,7 +219,7 @@ __global__ __launch_bounds__(256) void fc_tree_finish_kernel(const float *__rest
 // kernel of its own in neuron order (fc_tree_logit_grad_kernel): done here it held the wavefront for one more round trip and
 // read and wrote 64-byte pieces all over (655360 roots x 128 samples: 1742 us, 978 without it).
 // SUMS, ROWS: for the gradients of the logits, of the input (a frozen end and an input without a gradient need one of them).
-template <int V, bool SUMS, bool ROWS>
+template <int V, bool SUMS, bool ROWS, bool STREAM>
 __global__ __launch_bounds__(kTreeBlock) void fc_tree_backward_kernel(const float *__restrict__ x, const int32_t *__restrict__ rows,
                                                                     const int32_t *__restrict__ pos, const float *__restrict__ coef,
                                                                     const float *__restrict__ grad_out,
@@ -297,7 +297,7 @@ __global__ __launch_bounds__(kTreeBlock) void fc_tree_backward_kernel(const floa
             if (ROWS && live) {
 #pragma unroll
                 for (int q = 0; q < 8; ++q)
-                    store_samples<V>(rowgrad + (int64_t)min((uint64_t)(uint32_t)pj[q], (uint64_t)total_rows - 1) * pitch + s, v[q]);
+                    store_samples<V, STREAM>(rowgrad + (int64_t)min((uint64_t)(uint32_t)pj[q], (uint64_t)total_rows - 1) * pitch + s, v[q]);
             }
         }
         if constexpr (SUMS) {
@@ -308,10 +308,14 @@ __global__ __launch_bounds__(kTreeBlock) void fc_tree_backward_kernel(const floa
     }
 }
 
-__global__ __launch_bounds__(256) void fc_tree_logit_grad_kernel(TreeSums t) { tree_logit_grad(t, blockIdx.x); }
+template <bool STREAM>
+__global__ __launch_bounds__(256) void fc_tree_logit_grad_kernel(TreeSums t)
+{
+    tree_logit_grad<STREAM>(t, blockIdx.x);
+}
 
 // gx[i] = sum of the rows start[i] .. start[i + 1] of rowgrad, eight in flight, four partial sums
-template <int V>
+template <int V, bool STREAM>
 __global__ __launch_bounds__(kTreeBlock) void fc_tree_gather_kernel(const float *__restrict__ rowgrad, const int64_t *__restrict__ start,
                                                                   float *__restrict__ gx, int in_dim, int64_t pitch, int64_t total_rows)
 {
@@ -326,7 +330,7 @@ __global__ __launch_bounds__(kTreeBlock) void fc_tree_gather_kernel(const float 
     for (; r + 8 <= end; r += 8, p += 8 * pitch) {
         Samples<V> v[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = load_samples<V>(p + u * pitch);
+        for (int u = 0; u < 8; ++u) v[u] = load_samples<V, STREAM>(p + u * pitch);
 #pragma unroll
         for (int u = 0; u < 8; ++u)
 #pragma unroll
@@ -335,7 +339,7 @@ __global__ __launch_bounds__(kTreeBlock) void fc_tree_gather_kernel(const float 
     if (r < end) {
         Samples<V> v[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = load_samples<V>(p + (r + u < end ? u : 0) * pitch);
+        for (int u = 0; u < 8; ++u) v[u] = load_samples<V, STREAM>(p + (r + u < end ? u : 0) * pitch);
 #pragma unroll
         for (int u = 0; u < 8; ++u)
 #pragma unroll
@@ -447,7 +451,7 @@ extern "C" int clg_fc_tree_forward(const float *x, const int32_t *rows, const fl
 
 static int tree_backward(const char *name, const float *x, const int32_t *rows, const int32_t *pos, const int32_t *slot, const float *coef,
                          const float *grad_out, const float *probs, float *grad0, float *grad1, float *grad2, float *rowgrad, float *sums,
-                         const int64_t *start, float *grad_x, int64_t in_dim, int64_t roots, int64_t k, int64_t batch, int64_t pitch, double tau, void *stream,
+                         const int64_t *start, float *grad_x, int64_t in_dim, int64_t roots, int64_t k, int64_t batch, int64_t pitch, double tau, void *stream_,
                          clg_late_sums *late)
 {
     if (int e = clg_check_tree(name, in_dim, roots, k)) return e;
@@ -458,13 +462,18 @@ static int tree_backward(const char *name, const float *x, const int32_t *rows, 
     CLG_REQUIRE(batch > 0 && pitch >= batch && pitch < (1ll << 28) && tau != 0.0, "%s: the row pitch must hold the batch, tau must not be zero",
                 name);
     const int vec = tree_vec_dividing(pitch, x, rowgrad), gvec = tree_vec(pitch);
-    hipStream_t st = clg_stream(stream);
+    hipStream_t st = clg_stream(stream_);
+    // Operand gradients: a step of the CIFAR topology, us through the caches and past them: rows of 1 KiB 62 MB 261 and 248, 80 MB 295 and 282, 160 MB 501 and 485,
+    // of 512 bytes 2.7 GB 4722 and 4550, no difference at 40.  Pieces of lines at the ends of rows cost what that gives: rows of 400 bytes, MNIST
+    // topology, 98 MB 229 and 232, 250 MB 519 and 495; of 508 bytes, which lanes write four at a time, 79 MB 194 and 216, of 804 294 MB 934 and 1002.
+    const bool stream = pitch % 4 == 0 && clg_past_caches(roots * 8 * pitch * 4, pitch % 16 == 0 ? 48 : 200);
     const TreeGrads gr = {{grad0, grad1, grad2}, {4 * roots, 6 * roots, 7 * roots}};
     const dim3 grid((unsigned)clg_ceil_div(roots, kTreeWaves));
     const dim3 ggrid((unsigned)clg_ceil_div(in_dim, kTreeWaves), (unsigned)clg_ceil_div(pitch, (int64_t)kWave * gvec));
     CLG_REQUIRE(ggrid.y <= 65535, "%s: batch too large", name);
 #define CLG_TREE_K(V, SUMS, ROWS)                                                                                                \
-    hipLaunchKernelGGL((fc_tree_backward_kernel<V, SUMS, ROWS>), grid, dim3(kTreeBlock), 0, st, x, rows, pos, coef, grad_out, sums, rowgrad, \
+    hipLaunchKernelGGL((ROWS && stream ? fc_tree_backward_kernel<V, SUMS, ROWS, ROWS> : fc_tree_backward_kernel<V, SUMS, ROWS, false>), grid, \
+                       dim3(kTreeBlock), 0, st, x, rows, pos, coef, grad_out, sums, rowgrad, \
                        (int)roots, (int)(roots / k), (int)k, batch, pitch, (int)in_dim, 1.f / (float)tau)
 #define CLG_TREE_B(V)                                                                                                            \
     do {                                                                                                                         \
@@ -473,8 +482,8 @@ static int tree_backward(const char *name, const float *x, const int32_t *rows, 
         else CLG_TREE_K(V, false, true);                                                                                         \
     } while (0)
 #define CLG_TREE_G(V)                                                                                                            \
-    hipLaunchKernelGGL((fc_tree_gather_kernel<V>), ggrid, dim3(kTreeBlock), 0, st, (const float *)rowgrad, start, grad_x, (int)in_dim, pitch, \
-                       roots * 8)
+    hipLaunchKernelGGL((stream ? fc_tree_gather_kernel<V, true> : fc_tree_gather_kernel<V, false>), ggrid, dim3(kTreeBlock), 0, st, \
+                       (const float *)rowgrad, start, grad_x, (int)in_dim, pitch, roots * 8)
     if (vec == 1) CLG_TREE_B(1);
     else if (vec == 2) CLG_TREE_B(2);
     else CLG_TREE_B(4);
@@ -489,12 +498,13 @@ static int tree_backward(const char *name, const float *x, const int32_t *rows, 
     CLG_CHECK_LAUNCH(name);
     if (!logits) return CLG_OK;
     const TreeSums t = {gr, probs, sums, slot, 7 * roots};
-    const int64_t blocks = clg_ceil_div(7 * roots, 256);
-    if (late != nullptr) {
+    const int64_t blocks = clg_ceil_div(7 * roots * 4, 256);
+    const bool stream_logits = clg_past_caches(7 * roots * 64, 100);
+    if (late != nullptr && !stream_logits) {
         *late = clg_late(kLateTree, (int)blocks, t);
         return CLG_OK;
     }
-    hipLaunchKernelGGL(fc_tree_logit_grad_kernel, dim3((unsigned)blocks), dim3(256), 0, st, t);
+    hipLaunchKernelGGL((stream_logits ? fc_tree_logit_grad_kernel<true> : fc_tree_logit_grad_kernel<false>), dim3((unsigned)blocks), dim3(256), 0, st, t);
     CLG_CHECK_LAUNCH(name);
     return CLG_OK;
 }

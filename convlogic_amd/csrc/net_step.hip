@@ -61,7 +61,7 @@ __global__ __launch_bounds__(256) void step_sums_kernel(StepSums s)
     while (i < s.n - 1 && b >= s.late[i].blocks) first = s.late[i++].blocks;
     const clg_late_sums &l = s.late[i];
     if (l.kind == kLateBin) bin_sums(reinterpret_cast<const BinSums &>(l.field), b - first);
-    else if (l.kind == kLateTree) tree_logit_grad(reinterpret_cast<const TreeSums &>(l.field), b - first);
+    else if (l.kind == kLateTree) tree_logit_grad<false>(reinterpret_cast<const TreeSums &>(l.field), b - first);
     else reduce_coef_partials(reinterpret_cast<const CoefSums<float> &>(l.field), b - first);
 }
 

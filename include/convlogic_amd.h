@@ -612,7 +612,7 @@ int clg_train_prepare(const clg_train_block *blocks, int n_blocks, const float *
                       const int32_t *ids, float *coef, float *probs, int64_t roots, void *stream);
 typedef struct clg_late_sums {
     int32_t kind, blocks;     /* kind 0: nothing is left to do */
-    int64_t field[12];
+    int64_t field[13];
 } clg_late_sums;
 int clg_convblock_backward_planned_late(int dtype, const clg_conv_geom *g, const void *grad_y, const void *x, const void *w,
                                         const void *folded, const void *padded, const int32_t *selection, const uint8_t *argmax,

@@ -7,7 +7,8 @@ import torch
 
 import convlogic_amd as C
 from convlogic_amd.convlogic import train_net
-from tests.gpu_util import DEV
+from convlogic_amd.hip import _lib
+from tests.gpu_util import DEV, set_knobs
 
 pytestmark = pytest.mark.gpu
 
@@ -154,3 +155,18 @@ def test_any_number_of_blocks(at_once, blocks, kernels):
     y, grads = step(model, x, gy, tensors, False)
     y0, grads0 = step(model, x, gy, tensors, True)
     assert at_once == [True] and torch.equal(y, y0) and all(torch.equal(a, b) for a, b in zip(grads, grads0, strict=True))
+
+
+# operand and tap gradients and the trees' logits past the caches or through them, rows of one to four samples per lane and ragged ones
+@pytest.mark.parametrize("k,batch", [(8, 33), (8, 64), (8, 127), (4, 256), (4, 301)])
+@pytest.mark.parametrize("by_modules", [False, True])
+def test_gradients_past_the_caches(monkeypatch, k, batch, by_modules):
+    model, side = network("cifar", k, 3)
+    x, gy = (torch.rand(batch, 3, side, side, device=DEV) < 0.5).float(), torch.randn(batch, 10, device=DEV)
+    got = []
+    for megabytes in ("0", "100000"):
+        set_knobs(monkeypatch, CLG_STREAM_MB=megabytes)
+        got.append(step(model, x, gy, list(model.parameters()), by_modules)[1])
+    monkeypatch.undo()
+    _lib.reload_knobs()
+    assert all(torch.equal(a, b) for a, b in zip(*got, strict=True))
