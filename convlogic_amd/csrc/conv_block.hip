@@ -1493,11 +1493,15 @@ static bool backward_4x4_wanted(const Geom &g)
     return clg_convblock_is_4x4(g) && g.c <= 65535 && (!e || atoi(e) != 0);
 }
 
-// A planned float32 call takes both gradients from planes staged two at a time (conv_pair_grad.hip) as long as the gradient planes between its two
-// kernels stay in the last-level cache of 256 MB.  Forward and backward of a block against the kernels below, 180 shapes of 6x6 to 20x20
+// A planned float32 call takes both gradients from planes staged two at a time (conv_pair_grad.hip) up to 450 MB of gradient planes between its two
+// kernels.  Forward and backward of a block against the kernels below, 180 shapes of 6x6 to 20x20
 // images, 4 to 512 channels with lists of 2 to 16 kernels, 16 to 256 samples: 0.95 to 1.84 times as fast at up to 150 MB of planes, 21 of them
 // below 1.05 (lists of 2), 1.1 to 1.5 in between ([256,32,16,16] -> 128 70.7 -> 63.1 us, [16,32,6,6] -> 256 45 -> 25,
-// [64,512,12,12] -> 2048 184 -> 156); 0.82 to 1.07 at 256 MB and more ([128,1024,16,16] -> 4096 752 -> 853).  Fewer than four channels are
+// [64,512,12,12] -> 2048 184 -> 156); 45 shapes of 90 to 420 MB 1.03 to 1.36 times ([71,749,20,20] -> 749 221 -> 167 us, [240,127,20,20] -> 508 323 -> 295,
+// [24,618,18,18] -> 4944 360 -> 337); 26 of 420 to 1100 MB 0.81 to 1.10, the slower ones from 477 on.  Images of 8 and 16 columns, which the kernels
+// below take without a division per position, only up to 70 MB: in the step of a whole network, where the planes' memory is not in the caches
+// any more, CIFAR topology, k = 32 with 256 images, 64 MB per block, 299 -> 272 us, k = 48 with 200, 75 MB, 342 -> 356, k = 100 with
+// 128, 406 -> 421, k = 250 with 200, 391 MB, 1401 -> 1473 (MNIST topology, 12 and 6 columns, k = 256 with 128, 108 MB, 568 -> 549).  Fewer than four channels are
 // the tiled kernel's, whose wavefronts share a channel; lists longer than 16 on the average go by their length (lists_are_long).
 static bool backward_planes_wanted(const Geom &g, int dtype, PairPlan *p)
 {
@@ -1505,7 +1509,7 @@ static bool backward_planes_wanted(const Geom &g, int dtype, PairPlan *p)
         return false;
     if (const char *e = clg_knob(K_BWDX_PLANES)) return atoi(e) != 0;
     if (clg_knob(K_BWDX_DIRECT) != nullptr) return false;            // (one of the other kernels is asked for)
-    return g.cin >= 4 && g.c >= g.cin && g.c <= 8 * (int64_t)g.cin && clg_pair_planes_bytes(g) <= (size_t)160 << 20;
+    return g.cin >= 4 && g.c >= g.cin && g.c <= 8 * (int64_t)g.cin && clg_pair_planes_bytes(g) <= (size_t)(g.w == 8 || g.w == 16 ? 70 : 450) << 20;
 }
 static size_t backward_planes_off(const Geom &g) { return (bwd_scratch_layout(g, 4, 1).total + 255) & ~(size_t)255; }
 
@@ -1903,9 +1907,9 @@ static int backward_planned_impl(const char *name, int dtype, const clg_conv_geo
         hipStream_t st = clg_stream(stream);
         BwdTables tb;
         if (int e = prepare_tables<float>(g, pi.lay, 0, 0, w, selection, scratch, st, no_pad_job<float>(), &pv, &tb)) return e;
-        const int nb = clg_pair_grad_w_parts(g, pi.pair);
+        int nb = 0;
         float *planes = reinterpret_cast<float *>(reinterpret_cast<unsigned char *>(scratch) + backward_planes_off(g));
-        if (int e = clg_pair_grads(g, pi.pair, nb, (const float *)grad_y, (const float *)x, (const float *)tb.folded, selection, argmax, tb.count, tb.hits,
+        if (int e = clg_pair_grads(g, pi.pair, &nb, (const float *)grad_y, (const float *)x, (const float *)tb.folded, selection, argmax, tb.count, tb.hits,
                                    planes, (float *)w_scratch, (float *)grad_x, st, name))
             return e;
         return clg_launch_reduce_coef(CLG_F32, w_scratch, grad_w, g.c, nb, 7, st, name, probs, late);

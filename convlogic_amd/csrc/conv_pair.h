@@ -77,11 +77,11 @@ int clg_pair_grad_w(const Geom &g, const PairPlan &p, int nb, const float *gy, c
                     const uint8_t *argmax, float *partial, hipStream_t st, const char *name);
 
 // Both gradients: the sums as above, and the input gradient by way of gradient planes per kernel and channel (clg_pair_planes_bytes), which
-// are summed per channel.  count, hits: the lists of conv_block.hip.
+// are summed per channel; nb: the parts that it has left.  count, hits: the lists of conv_block.hip.
 constexpr int kHitWide = 1 << 24;                                    // of a list entry: the kernel's taps are in more than two channels
 bool clg_pair_planes_fit(const Geom &g, const PairPlan &p);
 size_t clg_pair_planes_bytes(const Geom &g);
-int clg_pair_grads(const Geom &g, const PairPlan &p, int nb, const float *gy, const float *x, const float *folded, const int32_t *sel,
+int clg_pair_grads(const Geom &g, const PairPlan &p, int *nb, const float *gy, const float *x, const float *folded, const int32_t *sel,
                    const uint8_t *argmax, const int32_t *count, const int32_t *hits, float *planes, float *partial, float *gx, hipStream_t st,
                    const char *name);
 

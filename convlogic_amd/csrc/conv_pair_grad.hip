@@ -60,7 +60,7 @@ __device__ __forceinline__ void pair_block_sums(const float (&v)[28], float *__r
 // them.  partial [c][nb][28], added in order by reduce_coef_partials.
 // PLANES: the tap gradients as well, added to gradient planes beside the staged ones and written to planes [c][2][n][h w]: those of a kernel's
 // first and second channel, for plane_sums_kernel.  (Of a kernel with taps in more than two channels nothing is written.)
-template <int NL, int RS, bool ROWS, bool ONE, bool PLANES>
+template <int NL, int RS, bool ROWS, bool ONE, bool PLANES, bool STREAM>
 __global__ __launch_bounds__(kPairWaves *kWave) void convblock_backward_w_pair_kernel(const float *__restrict__ gy, const float *__restrict__ x,
                                                                                     const float *__restrict__ folded, const int32_t *__restrict__ sel,
                                                                                     const uint8_t *__restrict__ argmax, float *__restrict__ partial,
@@ -199,7 +199,7 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_backward_w_pair_k
                     for (int j = 0; j < 4; ++j) part[j] = grads[in.to[i][j]];
                     __builtin_memcpy(&v, part, 16);
                 }
-                if (!wide && out_sample[i] < p.G && n0 + out_sample[i] >= q * p.G) *reinterpret_cast<u32x4 *>(dst + out_at[i]) = v;
+                if (!wide && out_sample[i] < p.G && n0 + out_sample[i] >= q * p.G) store_vec<STREAM>(reinterpret_cast<u32x4 *>(dst + out_at[i]), v);
             }
         }
     }
@@ -208,6 +208,7 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_backward_w_pair_k
 
 // gx = the sum of a channel's gradient planes, in the order of the kernels: four consecutive elements per thread, `parts` workgroups per channel.
 // A kernel that wrote none (its list entry says so) is evaluated here, element by element.
+template <bool STREAM>
 __global__ __launch_bounds__(256) void plane_sums_kernel(const float *__restrict__ planes, const int32_t *__restrict__ count, const int32_t *__restrict__ hits,
                                                        const float *__restrict__ gy, const float *__restrict__ x, const float *__restrict__ folded,
                                                        const int32_t *__restrict__ sel, const uint8_t *__restrict__ argmax, float *__restrict__ gx, Geom g,
@@ -224,7 +225,7 @@ __global__ __launch_bounds__(256) void plane_sums_kernel(const float *__restrict
     const float *from = planes + e;
     f32x4 sum = 0.f;
     auto piece = [&](int ent) {
-        return *reinterpret_cast<const f32x4 *>(from + (int64_t)(2 * (ent & 0xFFFF) + ((ent >> 16) & 1 ? 0 : 1)) * plane);
+        return load_vec<STREAM>(reinterpret_cast<const f32x4 *>(from + (int64_t)(2 * (ent & 0xFFFF) + ((ent >> 16) & 1 ? 0 : 1)) * plane));
     };
     int k = 0;
     while (k < nhits) {
@@ -294,27 +295,27 @@ __global__ __launch_bounds__(256) void plane_sums_kernel(const float *__restrict
 
 }  // namespace
 
-template <int NL, int RS, bool ROWS, bool ONE, bool PLANES>
+template <int NL, int RS, bool ROWS, bool ONE, bool PLANES, bool STREAM>
 static int launch_pair_w(const Geom &g, const PairPlan &p, int nb, const float *gy, const float *x, const float *folded, const int32_t *sel,
                          const uint8_t *argmax, float *partial, float *planes, hipStream_t st, const char *name)
 {
     const size_t lds = (size_t)(PLANES ? 2 : 1) * kPairWaves * p.wave_elems * 4;
-    if (int e = allow_lds(convblock_backward_w_pair_kernel<NL, RS, ROWS, ONE, PLANES>, lds, name)) return e;
-    hipLaunchKernelGGL((convblock_backward_w_pair_kernel<NL, RS, ROWS, ONE, PLANES>), dim3((unsigned)(g.c * nb)), dim3(kPairWaves *kWave), lds, st, gy, x,
+    if (int e = allow_lds(convblock_backward_w_pair_kernel<NL, RS, ROWS, ONE, PLANES, STREAM>, lds, name)) return e;
+    hipLaunchKernelGGL((convblock_backward_w_pair_kernel<NL, RS, ROWS, ONE, PLANES, STREAM>), dim3((unsigned)(g.c * nb)), dim3(kPairWaves *kWave), lds, st, gy, x,
                        folded, sel, argmax, partial, planes, g, p, nb);
     CLG_CHECK_LAUNCH(name);
     return CLG_OK;
 }
-template <int NL, bool PLANES>
+template <int NL, bool PLANES, bool STREAM>
 static int launch_pair_w_nl(const Geom &g, const PairPlan &p, int nb, const float *gy, const float *x, const float *folded, const int32_t *sel,
                             const uint8_t *argmax, float *partial, float *planes, hipStream_t st, const char *name)
 {
     const bool one = p.G * (g.ho / 2) * (g.wo / 2) <= kWave;
-    auto *launch = launch_pair_w<NL, 0, true, false, PLANES>;
-    if (g.w % 4 != 0) launch = one ? launch_pair_w<NL, 0, false, true, PLANES> : launch_pair_w<NL, 0, false, false, PLANES>;
+    auto *launch = launch_pair_w<NL, 0, true, false, PLANES, STREAM>;
+    if (g.w % 4 != 0) launch = one ? launch_pair_w<NL, 0, false, true, PLANES, STREAM> : launch_pair_w<NL, 0, false, false, PLANES, STREAM>;
     else if (one)
-        launch = p.rs == 20 ? launch_pair_w<NL, 20, true, true, PLANES>
-                            : (p.rs == 12 ? launch_pair_w<NL, 12, true, true, PLANES> : launch_pair_w<NL, 0, true, true, PLANES>);
+        launch = p.rs == 20 ? launch_pair_w<NL, 20, true, true, PLANES, STREAM>
+                            : (p.rs == 12 ? launch_pair_w<NL, 12, true, true, PLANES, STREAM> : launch_pair_w<NL, 0, true, true, PLANES, STREAM>);
     return launch(g, p, nb, gy, x, folded, sel, argmax, partial, planes, st, name);
 }
 
@@ -341,6 +342,22 @@ int clg_pair_grad_w_parts(const Geom &g, const PairPlan &p)
     const int64_t fill = std::min<int64_t>(clg_ceil_div(1024, g.c), p.groups * ch.blocks / (4 * kPairWaves));
     return (int)std::max<int64_t>(1, std::min<int64_t>(kMaxParts, std::max(fill, clg_ceil_div(p.groups, groups * kPairWaves))));
 }
+// With the planes a CU holds four workgroups, or what LDS has room for, and a launch of a little more than all CUs hold takes twice as long ([200,48,16,16] ->
+// 192 in 7 parts: 1344 workgroups, 45 us; step of the k = 48
+// CIFAR network 362 -> 356 us with 10).  Of the numbers of parts from the shortest chain's on, the one with the fewest
+// rounds of the launch times groups of a wavefront, and as long as two for what a workgroup does before and after.
+static int planes_parts(const Geom &g, const PairPlan &p)
+{
+    const Chain ch = chain_of(g, p);
+    const int64_t groups = std::max<int64_t>(1, ch.limit / ch.blocks), least = std::min<int64_t>(kMaxParts, clg_ceil_div(p.groups, groups * kPairWaves));
+    const int64_t slots = 256 * std::max<int64_t>(1, std::min<int64_t>(4, kLdsLimit / (2ll * kPairWaves * p.wave_elems * 4)));
+    int64_t best = least, cost = INT64_MAX;
+    for (int64_t nb = least; nb <= std::min<int64_t>(kMaxParts, std::max(least, clg_ceil_div(p.groups, (int64_t)kPairWaves))); ++nb) {
+        const int64_t now = clg_ceil_div(g.c * nb, slots) * (clg_ceil_div(p.groups, nb * kPairWaves) * ch.blocks + 2);
+        if (now < cost) best = nb, cost = now;
+    }
+    return (int)best;
+}
 // Lanes that idle in every block of cells can make the chain longer than the other kernel's even with the most parts.
 bool clg_pair_grad_w_wanted(const Geom &g, const PairPlan &p)
 {
@@ -351,9 +368,9 @@ bool clg_pair_grad_w_wanted(const Geom &g, const PairPlan &p)
 int clg_pair_grad_w(const Geom &g, const PairPlan &p, int nb, const float *gy, const float *x, const float *folded, const int32_t *sel,
                     const uint8_t *argmax, float *partial, hipStream_t st, const char *name)
 {
-    if (p.loads <= 2) return launch_pair_w_nl<2, false>(g, p, nb, gy, x, folded, sel, argmax, partial, nullptr, st, name);
-    if (p.loads <= 4) return launch_pair_w_nl<4, false>(g, p, nb, gy, x, folded, sel, argmax, partial, nullptr, st, name);
-    return launch_pair_w_nl<8, false>(g, p, nb, gy, x, folded, sel, argmax, partial, nullptr, st, name);
+    if (p.loads <= 2) return launch_pair_w_nl<2, false, false>(g, p, nb, gy, x, folded, sel, argmax, partial, nullptr, st, name);
+    if (p.loads <= 4) return launch_pair_w_nl<4, false, false>(g, p, nb, gy, x, folded, sel, argmax, partial, nullptr, st, name);
+    return launch_pair_w_nl<8, false, false>(g, p, nb, gy, x, folded, sel, argmax, partial, nullptr, st, name);
 }
 
 bool clg_pair_planes_fit(const Geom &g, const PairPlan &p)
@@ -363,14 +380,21 @@ bool clg_pair_planes_fit(const Geom &g, const PairPlan &p)
 }
 size_t clg_pair_planes_bytes(const Geom &g) { return (size_t)2 * g.c * g.n * g.h * g.w * 4; }
 
-int clg_pair_grads(const Geom &g, const PairPlan &p, int nb, const float *gy, const float *x, const float *folded, const int32_t *sel, const uint8_t *argmax,
+int clg_pair_grads(const Geom &g, const PairPlan &p, int *parts_of_sums, const float *gy, const float *x, const float *folded, const int32_t *sel, const uint8_t *argmax,
                    const int32_t *count, const int32_t *hits, float *planes, float *partial, float *gx, hipStream_t st, const char *name)
 {
-    auto *launch = p.loads <= 2 ? launch_pair_w_nl<2, true> : launch_pair_w_nl<4, true>;
+    const int nb = *parts_of_sums = planes_parts(g, p);
+    // Past the caches where the planes, x and its gradient together are more than the last-level cache keeps between the two kernels: forward and backward, us
+    // through the caches and past them, [275,144,20,20] -> 144, 121 MB of planes and 2 x 63, 139 and 131, [268,233,10,10] -> 932, 191 and 2 x 25, 198 and 189,
+    // [126,381,14,14] -> 1143, 215 and 2 x 38, 236 and 210; [297,706,8,8] -> 706, 102 and 2 x 54, 104 and 111, [209,31,20,20] -> 248, 158 and 2 x 10, 142 and 147.
+    const bool stream = clg_past_caches((int64_t)clg_pair_planes_bytes(g) + (int64_t)g.n * g.cin * g.h * g.w * 8, 215);
+    auto *launch = p.loads <= 2 ? (stream ? launch_pair_w_nl<2, true, true> : launch_pair_w_nl<2, true, false>)
+                                : (stream ? launch_pair_w_nl<4, true, true> : launch_pair_w_nl<4, true, false>);
     if (int e = launch(g, p, nb, gy, x, folded, sel, argmax, partial, planes, st, name)) return e;
     const unsigned parts = (unsigned)clg_ceil_div((int64_t)g.n * g.h * g.w, 1024);
-    hipLaunchKernelGGL(plane_sums_kernel, dim3(parts * (unsigned)g.cin), dim3(256), 0, st, (const float *)planes, count, hits, gy, x, folded, sel, argmax, gx, g,
-                       parts, make_fastdiv(parts), make_fastdiv((uint32_t)(g.h * g.w)), make_fastdiv((uint32_t)g.w));
+    hipLaunchKernelGGL((stream ? plane_sums_kernel<true> : plane_sums_kernel<false>), dim3(parts * (unsigned)g.cin), dim3(256), 0, st, (const float *)planes,
+                       count, hits, gy, x, folded, sel, argmax, gx, g, parts, make_fastdiv(parts), make_fastdiv((uint32_t)(g.h * g.w)),
+                       make_fastdiv((uint32_t)g.w));
     CLG_CHECK_LAUNCH(name);
     return CLG_OK;
 }

@@ -194,6 +194,9 @@ def test_both_gradients_by_planes_against_float64(n, cin, h, w, c, wide, monkeyp
     e0, e1 = ((g.double() - ref).norm().item() for g in (gx0, gx1))
     assert e1 <= 1.25 * e0 + 2.0**-24 * ref.norm().item()
     assert_grad_close(gw1, gw0, rel=1e-5)
+    set_knobs(monkeypatch, CLG_STREAM_MB="0")                         # planes past the caches
+    again = H.full_convlogic_backward_planned(gy, x, probs, None, am, sel, *plan, *geo, wrt_logits=False)
+    assert torch.equal(again[0], gx1) and torch.equal(again[1], gw1)
 
 
 @pytest.mark.parametrize("n,cin,side,c", [(1000, 40, 8, 2000), (128, 64, 16, 2048), (300, 48, 16, 600)])
