@@ -25,13 +25,13 @@ namespace {
 
 // What a launch needs besides x and the selection, in one launch: table, folded coefficients (float gates; the softmax of logits
 // first), the zero-padded copy of x that the backward pass reads.
-template <typename Ops, typename P, typename T>
+template <typename Ops, typename P, typename T, bool STREAM>
 __global__ __launch_bounds__(256) void pair_prepare_kernel(const P *__restrict__ w, const int32_t *__restrict__ sel, T *__restrict__ folded,
                                                          int32_t *__restrict__ table, PairPlan p, Geom g, PadJob<T> pad,
                                                          int pad_block0, int from_logits, T *__restrict__ probs_out)
 {
     if ((int)blockIdx.x >= pad_block0) {
-        pad_image_elems(pad, blockIdx.x - pad_block0);
+        pad_image_elems<STREAM>(pad, blockIdx.x - pad_block0);
         return;
     }
     const int C = g.c;
@@ -307,7 +307,10 @@ int clg_forward_pair_f32(const Geom &g, const PairPlan &p, const float *x, const
     if (!prepared || padded_out) {                                    // (prepared: coefficients and table are there)
         const PadJob<float> job = padded_out ? make_pad_job(x, padded_out, g, pad_rs, pad_chs, pad_sample) : no_pad_job<float>();
         const unsigned prep = (unsigned)clg_ceil_div((int64_t)g.c * (folded_in ? 1 : 7), 256);
-        hipLaunchKernelGGL((pair_prepare_kernel<FloatOps<float>, float, float>), dim3(prep + pad_blocks(job)), dim3(256), 0, st, w, sel,
+        // (a large copy goes past the caches: it is read in the backward pass; [128,1024,16,16] and [128,4096,8,8], 160 and 215 MB, copy and forward
+        // 241 -> 225 and 229 -> 207 us; step of the CIFAR topology, 40 MB 1030 -> 1022 us, no difference at 28)
+        auto kern = clg_past_caches(job.total * 4, 36) ? pair_prepare_kernel<FloatOps<float>, float, float, true> : pair_prepare_kernel<FloatOps<float>, float, float, false>;
+        hipLaunchKernelGGL(kern, dim3(prep + pad_blocks(job)), dim3(256), 0, st, w, sel,
                            folded_in ? (float *)nullptr : folded, table, p, g, job, (int)prep, from_logits ? 1 : 0, probs_out);
         CLG_CHECK_LAUNCH(name);
     }
@@ -324,7 +327,7 @@ int clg_forward_pair_packed(const Geom &g, const PairPlan &p, const uint64_t *x,
     int32_t *table = reinterpret_cast<int32_t *>(scratch);
     const unsigned prep = (unsigned)clg_ceil_div(g.c, 256);
     if (gates != nullptr)
-        hipLaunchKernelGGL((pair_prepare_kernel<BitOpsAnf, uint8_t, float>), dim3(prep), dim3(256), 0, st, gates, sel, (float *)nullptr, table, p, g,
+        hipLaunchKernelGGL((pair_prepare_kernel<BitOpsAnf, uint8_t, float, false>), dim3(prep), dim3(256), 0, st, gates, sel, (float *)nullptr, table, p, g,
                        no_pad_job<float>(), (int)prep, 0, (float *)nullptr);
     CLG_CHECK_LAUNCH(name);
     if (p.loads <= 2) return launch_pair_nl<BitOpsAnf, 2>(g, p, x, nullptr, table, sel, y, nullptr, st, name);

@@ -150,7 +150,7 @@ struct PadJob {
 // With one element per thread 109 us at [128, 4096, 8, 8] and 85 us at [128, 1024, 16, 16], 3 TB/s bound by that arithmetic;
 // now 66 and 56 us, 4.6 and 5.1 TB/s, the rate of a large copy.
 constexpr int kPadPerThread = 4, kPadPerBlock = 256 * kPadPerThread;
-template <typename T>
+template <bool STREAM = false, typename T>
 __device__ __forceinline__ void pad_image_elems(const PadJob<T> &j, unsigned block)
 {
     const int64_t e0 = (int64_t)block * kPadPerBlock + threadIdx.x * kPadPerThread;
@@ -181,11 +181,11 @@ __device__ __forceinline__ void pad_image_elems(const PadJob<T> &j, unsigned blo
     }
     T *dst = j.xp + e0;
     if (left == kPadPerThread && (reinterpret_cast<uintptr_t>(j.xp) & 15) == 0) {
-        struct alignas(16) Four { T t[kPadPerThread]; };
-        Four f;
+        typedef T four __attribute__((ext_vector_type(kPadPerThread)));
+        four f;
 #pragma unroll
-        for (int k = 0; k < kPadPerThread; ++k) f.t[k] = v[k];
-        *reinterpret_cast<Four *>(dst) = f;
+        for (int k = 0; k < kPadPerThread; ++k) f[k] = v[k];
+        store_vec<STREAM>(reinterpret_cast<four *>(dst), f);
         return;
     }
 #pragma unroll

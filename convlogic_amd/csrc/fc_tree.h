@@ -89,6 +89,55 @@ __device__ __forceinline__ void tree_fold(const TreeFold &f, int64_t block)
     }
 }
 
+// The same for training, neuron by neuron in the order of the layers: logits and probabilities in whole lines, the 16 bytes of coefficients at the
+// neuron's slot (root * 7 + gate).  In tree order both are pieces of 64 bytes, half a line each (655360 roots: 193 us, here 169, the coefficients' pieces are what is left).
+struct TreeFoldSlots {
+    TreeLogits lg;
+    const int32_t *slot;
+    float *coef, *probs;
+    int64_t end[3];       // neurons of the first one, two, three layers
+};
+template <bool STREAM>
+__device__ __forceinline__ void tree_fold_slots(const TreeFoldSlots &f, int64_t block)
+{
+    __shared__ __align__(16) float rows[256 / kWave][kWave * kFoldPitch];
+    const int lane = threadIdx.x & (kWave - 1);
+    float *mine = rows[threadIdx.x >> 6];
+    const int64_t e0 = block * 256 + (threadIdx.x & ~(kWave - 1)), e = e0 + lane, all = f.end[2];
+    if (e0 >= all) return;                                            // (a whole wavefront; none meets another one)
+    const uint32_t slot = e < all ? (uint32_t)f.slot[e] : 0u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int from = 16 * i + (lane >> 2);
+        const int64_t n = min(e0 + from, all - 1);
+        const int layer = n < f.end[0] ? 0 : (n < f.end[1] ? 1 : 2);
+        const f32x4u v = reinterpret_cast<const f32x4u *>(f.lg.l[layer] + (n - (layer ? f.end[layer - 1] : 0)) * 16)[lane & 3];
+        *reinterpret_cast<float4 *>(mine + from * kFoldPitch + 4 * (lane & 3)) = make_float4(v.x, v.y, v.z, v.w);
+    }
+    wave_fence();                                                     // (lanes read what others wrote)
+    float w[16], p[16];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float4 v = *reinterpret_cast<const float4 *>(mine + lane * kFoldPitch + 4 * i);
+        w[4 * i] = v.x, w[4 * i + 1] = v.y, w[4 * i + 2] = v.z, w[4 * i + 3] = v.w;
+    }
+    softmax16(w, p);
+    const Coef<float> c = fold16(p);
+    if (e < all && slot < (uint64_t)all) reinterpret_cast<float4 *>(f.coef)[slot] = make_float4(c.ab, c.a, c.b, c.one);
+    if (f.probs == nullptr) return;
+    wave_fence();
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<float4 *>(mine + lane * kFoldPitch + 4 * i) = make_float4(p[4 * i], p[4 * i + 1], p[4 * i + 2], p[4 * i + 3]);
+    wave_fence();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int from = 16 * i + (lane >> 2);
+        const float4 v = *reinterpret_cast<const float4 *>(mine + from * kFoldPitch + 4 * (lane & 3));
+        if (e0 + from < all) store_vec<STREAM>(reinterpret_cast<f32x4u *>(f.probs + (e0 + from) * 16) + (lane & 3), f32x4u{v.x, v.y, v.z, v.w});
+    }
+}
+
 // ---- gradients of the logits --------------------------------------------------------------------------------------------
 // Gradients of the logits, four lanes per neuron of the three layers in order, four gates each: whole lines of probabilities and gradients.  slot:
 // where the neuron's four sums are (root * 7 + gate of the tree).  A layer whose gradient is not wanted has a null pointer.

@@ -118,6 +118,11 @@ __device__ __forceinline__ const float *tree_logits(const TreeLogits &lg, const 
     return (q < 4 ? lg.l[0] : (q < 6 ? lg.l[1] : lg.l[2])) + tree_neuron(ids, j, q, roots) * 16;
 }
 __global__ __launch_bounds__(256) void fc_tree_fold_kernel(TreeFold f) { tree_fold(f, blockIdx.x); }
+template <bool STREAM>
+__global__ __launch_bounds__(256) void fc_tree_fold_slots_kernel(TreeFoldSlots f)
+{
+    tree_fold_slots<STREAM>(f, blockIdx.x);
+}
 
 // ---- forward ----------------------------------------------------------------------------------------------------------
 // rows [roots][8]: the input rows of a tree.  A wavefront takes a root at a time, 64 lanes x V samples.
@@ -407,6 +412,20 @@ extern "C" int clg_fc_tree_fold(const float *logits0, const float *logits1, cons
     CLG_REQUIRE(logits0 && logits1 && logits2 && ids && coef, "%s: null pointer argument", name);
     const TreeFold f = {{{logits0, logits1, logits2}}, ids, coef, probs, (int)roots, hard};
     hipLaunchKernelGGL(fc_tree_fold_kernel, dim3((unsigned)clg_ceil_div(roots * 7, 256)), dim3(256), 0, clg_stream(stream), f);
+    CLG_CHECK_LAUNCH(name);
+    return CLG_OK;
+}
+
+extern "C" int clg_fc_tree_fold_slots(const float *logits0, const float *logits1, const float *logits2, const int32_t *slot, float *coef, float *probs,
+                                      int64_t roots, void *stream)
+{
+    const char *name = "clg_fc_tree_fold_slots";
+    if (int e = clg_check_tree(name, 1, roots, 1)) return e;
+    CLG_REQUIRE(logits0 && logits1 && logits2 && slot && coef, "%s: null pointer argument", name);
+    const TreeFoldSlots f = {{{logits0, logits1, logits2}}, slot, coef, probs, {4 * roots, 6 * roots, 7 * roots}};
+    const bool past = clg_past_caches(7 * roots * 64, 100);
+    hipLaunchKernelGGL((past ? fc_tree_fold_slots_kernel<true> : fc_tree_fold_slots_kernel<false>), dim3((unsigned)clg_ceil_div(roots * 7, 256)), dim3(256), 0,
+                       clg_stream(stream), f);
     CLG_CHECK_LAUNCH(name);
     return CLG_OK;
 }

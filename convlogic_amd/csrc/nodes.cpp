@@ -392,8 +392,8 @@ Tensor trees_forward(const Tensor &x, const Tensor &l0, const Tensor &l1, const 
     if (!coef.defined()) {
         coef = floats(x, {t.roots, 28});
         if (need_l) probs = floats(x, {7 * t.roots, 16});             // (the logits may be updated between forward and backward)
-        check(clg_fc_tree_fold(l0.data_ptr<float>(), l1.data_ptr<float>(), l2.data_ptr<float>(), i32(t.ids), f32(coef), f32(probs), t.roots, 0,
-                               stream_of(x)));
+        check(clg_fc_tree_fold_slots(l0.data_ptr<float>(), l1.data_ptr<float>(), l2.data_ptr<float>(), i32(t.slot), f32(coef), f32(probs), t.roots,
+                                     stream_of(x)));
     }
     const int64_t elems = clg_fc_tree_partial_elems(t.roots, t.k, batch, batch);
     Tensor out = floats(x, {batch, t.k}), partial = floats(x, {elems < 0 ? 0 : elems});

@@ -131,6 +131,7 @@ SIGNATURES = {
     "clg_convblock_bin_backward_late": (_i, [_i, _GP, _p, _p, _p, _p, _p, _i, _p, _p, _p]),
     "clg_fc_tree_backward_late": (_i, [_p] * 14 + [_i64, _i64, _i64, _i64, _i64, _f64, _p, _p]),
     "clg_late_sums_run": (_i, [_p, _i, _p]),
+    "clg_fc_tree_fold_slots": (_i, [_p] * 6 + [_i64, _p]),
     "clg_net_packed_scratch_bytes": (_i64, [_p, _i, _i64, _i64, _i64, _i64]),
     "clg_net_packed": (_i, [_p, _i] + [_p] * 9 + [_f64, _i64, _i64, _i64, _i64, _p, _p]),
 }

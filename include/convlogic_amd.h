@@ -552,6 +552,9 @@ int clg_fc_tree_plan(const int64_t *a0, const int64_t *b0, const int64_t *a1, co
  * layer first (may be NULL) */
 int clg_fc_tree_fold(const float *logits0, const float *logits1, const float *logits2, const int32_t *ids, float *coef,
                      float *probs, int64_t roots, int hard, void *stream);
+/* clg_fc_tree_fold (hard = 0) in the order of the neurons: for large layers; an entry of slot out of range is left out */
+int clg_fc_tree_fold_slots(const float *logits0, const float *logits1, const float *logits2, const int32_t *slot, float *coef,
+                           float *probs, int64_t roots, void *stream);
 /* floats of the `partial` buffer of clg_fc_tree_forward; negative for bad arguments */
 int64_t clg_fc_tree_partial_elems(int64_t roots, int64_t k, int64_t batch, int64_t pitch);
 /* out [batch, k] = class sums of the roots' values / tau */

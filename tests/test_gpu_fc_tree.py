@@ -8,7 +8,7 @@ import convlogic_amd as C
 from convlogic_amd.convlogic.model import _forward
 from convlogic_amd.difflogic import fc_tree
 from oracle import convlogic_oracle as O
-from tests.gpu_util import DEV, assert_grad_close
+from tests.gpu_util import DEV, assert_grad_close, set_knobs
 
 pytestmark = pytest.mark.gpu
 
@@ -531,3 +531,24 @@ def test_one_network_first_used_by_several_threads_and_streams():
             t.join()
         for (a, b), (c, d) in zip(got, want):
             assert torch.equal(a, c) and torch.equal(b, d)
+
+
+# neurons in their own order and roots in theirs: a wavefront's 64, parts of one, layers that end inside one
+@pytest.mark.parametrize("roots", [1, 9, 64, 130, 663])
+@pytest.mark.parametrize("stream_mb", ["0", "100000"])
+def test_folding_by_slots_gives_the_bits_of_folding_by_roots(roots, stream_mb, monkeypatch):
+    from convlogic_amd.hip import _lib
+    layers, _ = tail(max(2, roots), roots, 1, roots)
+    plan, lib = fc_tree.tree_plan(*layers), _lib.load()
+    logits = [torch.randn_like(m.weights) * 3 for m in layers]
+    set_knobs(monkeypatch, CLG_STREAM_MB=stream_mb)
+    got = []
+    for table, call in ((plan.ids, lambda *a: lib.clg_fc_tree_fold(*a, roots, 0, None)), (plan.slot, lambda *a: lib.clg_fc_tree_fold_slots(*a, roots, None))):
+        coef, probs = torch.full((roots, 28), 7.0, device=DEV), torch.full((7 * roots, 16), 7.0, device=DEV)
+        torch.cuda.synchronize()
+        assert call(*(w.data_ptr() for w in logits), table.data_ptr(), coef.data_ptr(), probs.data_ptr()) == 0
+        torch.cuda.synchronize()
+        got.append((coef, probs))
+    monkeypatch.undo()
+    _lib.reload_knobs()
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
