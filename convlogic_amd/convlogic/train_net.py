@@ -1,5 +1,6 @@
 """A training step of a whole small network -- complete blocks, nn.Flatten, three LogicLayers as trees, GroupSum -- as one autograd node
-(csrc/nodes.cpp): the same launches as of the modules one after the other, without the host's work between them."""
+(csrc/nodes.cpp): the kernels of the modules one after the other without the host's work between them, the set-up of all layers in one launch and
+the sums that end their weight gradients in another (csrc/net_step.hip)."""
 import ctypes
 import types
 
