@@ -181,7 +181,7 @@ __device__ __forceinline__ void pad_image_elems(const PadJob<T> &j, unsigned blo
     }
     T *dst = j.xp + e0;
     if (left == kPadPerThread && (reinterpret_cast<uintptr_t>(j.xp) & 15) == 0) {
-        typedef T four __attribute__((ext_vector_type(kPadPerThread)));
+        typedef T four __attribute__((ext_vector_type(kPadPerThread), aligned(16)));
         four f;
 #pragma unroll
         for (int k = 0; k < kPadPerThread; ++k) f[k] = v[k];

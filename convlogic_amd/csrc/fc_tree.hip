@@ -314,9 +314,9 @@ __global__ __launch_bounds__(kTreeBlock) void fc_tree_backward_kernel(const floa
 }
 
 template <bool STREAM>
-__global__ __launch_bounds__(256) void fc_tree_logit_grad_kernel(TreeSums t)
+__global__ __launch_bounds__(256) void fc_tree_logit_grad_kernel(TreeSums t, int64_t blocks)
 {
-    tree_logit_grad<STREAM>(t, blockIdx.x);
+    for (int64_t b = blockIdx.x; b < blocks; b += gridDim.x) tree_logit_grad<STREAM>(t, b);   // (28 lanes for each of 2^28 roots are no launch)
 }
 
 // gx[i] = sum of the rows start[i] .. start[i + 1] of rowgrad, eight in flight, four partial sums
@@ -523,7 +523,8 @@ static int tree_backward(const char *name, const float *x, const int32_t *rows, 
         *late = clg_late(kLateTree, (int)blocks, t);
         return CLG_OK;
     }
-    hipLaunchKernelGGL((stream_logits ? fc_tree_logit_grad_kernel<true> : fc_tree_logit_grad_kernel<false>), dim3((unsigned)blocks), dim3(256), 0, st, t);
+    hipLaunchKernelGGL((stream_logits ? fc_tree_logit_grad_kernel<true> : fc_tree_logit_grad_kernel<false>), dim3((unsigned)std::min<int64_t>(blocks, 1 << 23)),
+                       dim3(256), 0, st, t, blocks);
     CLG_CHECK_LAUNCH(name);
     return CLG_OK;
 }

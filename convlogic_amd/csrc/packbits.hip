@@ -702,8 +702,14 @@ void launch_rows(const void *x, const int64_t *a, const int64_t *b, const void *
 {
     const uint32_t pieces = (uint32_t)clg_ceil_div(row_bytes, 16);
     const int nj = (int)std::max<int64_t>(1, std::min<int64_t>(kRowsMax, kRowsUnroll * kEvalBlock / pieces));
-    hipLaunchKernelGGL(eval_packed_rows_kernel<LOGITS>, dim3((unsigned)clg_ceil_div(out_dim, nj)), dim3(kEvalBlock), 0, st, (const uint8_t *)x, a, b, gate,
-                       (uint8_t *)y, (int)out_dim, row_bytes, pieces, make_fastdiv(pieces), nj, in_dim);
+    // (a launch is fewer than 2^32 threads)
+    const int64_t most = (int64_t)((1 << 24) - 1) * nj;
+    for (int64_t j = 0; j < out_dim; j += most) {
+        const int64_t some = std::min(most, out_dim - j);
+        const void *gates = reinterpret_cast<const uint8_t *>(gate) + j * (LOGITS ? 64 : 1);
+        hipLaunchKernelGGL(eval_packed_rows_kernel<LOGITS>, dim3((unsigned)clg_ceil_div(some, nj)), dim3(kEvalBlock), 0, st, (const uint8_t *)x, a + j, b + j,
+                           gates, (uint8_t *)y + j * row_bytes, (int)some, row_bytes, pieces, make_fastdiv(pieces), nj, in_dim);
+    }
 }
 
 // Layers whose rows are read once along a walk of the wiring (the others twice, but all at once): us at [neurons] x bytes, lanes along several neurons' rows
