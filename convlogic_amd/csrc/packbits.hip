@@ -83,17 +83,21 @@ __global__ __launch_bounds__(kEvalBlock) void eval_packed_kernel(const V *__rest
 // last piece of a row steps back to its last 16 bytes, some of which two lanes write then (the same values).  us per layer, a wavefront per neuron or a walk
 // -> here: 64000 neurons on rows of 64 bytes 15.7 -> 4.1, of 252 18.3 -> 9.6, 8000 on 1280 7.7 -> 4.4; one piece of a thread at a time instead of two
 // costs up to 10 %, stores that stay in the caches up to 25 (64000 on 8188: 250 us, 218).
+// A row of more pieces than a workgroup has in flight is cut into parts of `per` pieces, a workgroup each: few neurons on long rows fill the chip too
+// (in one workgroup each 64 on 400 KiB took 60 us, here 12.4, 1 on 4 MiB 530, 3.5, 100 on 64 KiB 8.6, 4.0).  The parts are the slow index of the launch: the neurons of one part run back to
+// back and find the second use of an input row's piece in the caches.
 typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
 constexpr int kRowsMax = 64, kRowsUnroll = 2;                        // neurons of a workgroup, pieces of a thread
 template <bool LOGITS>
 __global__ __launch_bounds__(kEvalBlock) void eval_packed_rows_kernel(const uint8_t *__restrict__ x, const int64_t *__restrict__ a,
                                                                     const int64_t *__restrict__ b, const void *__restrict__ gate,
                                                                     uint8_t *__restrict__ y, int out_dim, int64_t row_bytes, uint32_t pieces,
-                                                                    FastDiv d_pieces, int nj, int64_t in_dim)
+                                                                    FastDiv d_pieces, int nj, FastDiv d_groups, uint32_t per, int64_t in_dim)
 {
     __shared__ int ids[kRowsMax];
-    const int j0 = blockIdx.x * nj, here = min(nj, out_dim - j0), q = threadIdx.x >> 2;
-    const uint32_t total = (uint32_t)here * pieces;
+    const uint32_t part = fdiv(blockIdx.x, d_groups);
+    const int j0 = (int)(blockIdx.x - part * d_groups.d) * nj, here = min(nj, out_dim - j0), q = threadIdx.x >> 2;
+    const uint32_t total = min((uint32_t)here * pieces, (part + 1) * per);   // (more than one part: of one neuron)
     f32x4u logits = 0.f;                                              // requested ahead of the rows: vector loads return in order
     if (LOGITS && q < here) logits = reinterpret_cast<const f32x4u *>(reinterpret_cast<const float *>(gate) + (int64_t)(j0 + q) * 16)[threadIdx.x & 3];
     u32x4 ra[kRowsUnroll], rb[kRowsUnroll];
@@ -109,7 +113,7 @@ __global__ __launch_bounds__(kEvalBlock) void eval_packed_rows_kernel(const uint
             rb[u] = *reinterpret_cast<const u32x4_any *>(x + clamp_index(b[j0 + jn[u]], in_dim) * row_bytes + off[u]);
         }
     };
-    request(0);
+    request(part * per);
     if constexpr (LOGITS) {
         const int id = argmax16_quad(logits);
         if ((threadIdx.x & 3) == 0 && q < here) ids[q] = id;
@@ -117,7 +121,7 @@ __global__ __launch_bounds__(kEvalBlock) void eval_packed_rows_kernel(const uint
         if ((int)threadIdx.x < here) ids[threadIdx.x] = reinterpret_cast<const uint8_t *>(gate)[j0 + threadIdx.x];
     }
     __syncthreads();
-    for (uint32_t first = 0;;) {
+    for (uint32_t first = part * per;;) {
 #pragma unroll
         for (int u = 0; u < kRowsUnroll; ++u)
             if (first + u * kEvalBlock + threadIdx.x < total)
@@ -702,24 +706,28 @@ void launch_rows(const void *x, const int64_t *a, const int64_t *b, const void *
 {
     const uint32_t pieces = (uint32_t)clg_ceil_div(row_bytes, 16);
     const int nj = (int)std::max<int64_t>(1, std::min<int64_t>(kRowsMax, kRowsUnroll * kEvalBlock / pieces));
-    // (a launch is fewer than 2^32 threads)
-    const int64_t most = (int64_t)((1 << 24) - 1) * nj;
+    const int64_t parts = nj > 1 ? 1 : clg_ceil_div(pieces, kRowsUnroll * kEvalBlock);
+    const uint32_t per = (uint32_t)clg_ceil_div((int64_t)nj * pieces, parts);
+    // (a launch is fewer than 2^32 threads; parts < 2^21, of 2^30 pieces)
+    const int64_t most = ((1 << 24) - 1) / parts * nj;
     for (int64_t j = 0; j < out_dim; j += most) {
-        const int64_t some = std::min(most, out_dim - j);
+        const int64_t some = std::min(most, out_dim - j), groups = clg_ceil_div(some, nj);
         const void *gates = reinterpret_cast<const uint8_t *>(gate) + j * (LOGITS ? 64 : 1);
-        hipLaunchKernelGGL(eval_packed_rows_kernel<LOGITS>, dim3((unsigned)clg_ceil_div(some, nj)), dim3(kEvalBlock), 0, st, (const uint8_t *)x, a + j, b + j,
-                           gates, (uint8_t *)y + j * row_bytes, (int)some, row_bytes, pieces, make_fastdiv(pieces), nj, in_dim);
+        hipLaunchKernelGGL(eval_packed_rows_kernel<LOGITS>, dim3((unsigned)(groups * parts)), dim3(kEvalBlock), 0, st, (const uint8_t *)x, a + j, b + j,
+                           gates, (uint8_t *)y + j * row_bytes, (int)some, row_bytes, pieces, make_fastdiv(pieces), nj, make_fastdiv((uint32_t)groups), per,
+                           in_dim);
     }
 }
 
 // Layers whose rows are read once along a walk of the wiring (the others twice, but all at once): us at [neurons] x bytes, lanes along several neurons' rows
 // against the walk: [8000] x 3000 11.5 and 12.4, x 5000 18.5 and 17.3, [16000] x 1528 11.8 and 12.2, [32000] x 1020 15.9 and 15.3,
 // [64000] x 500 17.0 and 17.5, x 768 22.3 and 20.7, [16000] x 8188 56 and 49; below 30 MB a wavefront's chain of eight neurons is what a walk takes
-// ([2000] x 1280 3.9 and 7.3).
+// ([2000] x 1280 3.9 and 7.3, [100] x 256 KiB 12.0 and 13.2, [20] x 512 KiB 5.0 and 8.7), on rows of 1 MiB and more below 20 MB ([28] x 1 MiB 14.1 and 9.9, [10] x
+// 2 MiB 10.6 and 8.9, [4] x 1 MiB 3.7 and 5.3).
 bool walk_pays(int64_t row_bytes, int64_t out_dim)
 {
     if (const char *e = clg_knob(K_EVAL_ROWS)) return atoi(e) == 0;
-    return row_bytes >= 640 && row_bytes * out_dim >= 30'000'000;
+    return row_bytes >= 640 && row_bytes * out_dim >= (row_bytes >= 1 << 20 ? 20'000'000 : 30'000'000);
 }
 
 bool valid_elem(int e) { return e == 1 || e == 2 || e == 4 || e == 8; }

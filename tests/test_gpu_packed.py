@@ -105,6 +105,42 @@ def test_eval_packed_rows_of_any_length(monkeypatch, bits, row_bytes, out_dim, o
     assert all(np.array_equal(y.cpu().numpy(), want) for y in got)
 
 
+# rows in parts of a workgroup each: one part and one piece more, a last part of a few pieces, rows that end inside a piece
+@pytest.mark.parametrize("bits,row_bytes,out_dim,offset", [(64, 8192, 3, 0), (64, 8200, 3, 8), (8, 8193, 2, 1), (8, 16384, 1, 0), (32, 24580, 5, 4), (8, 131071, 7, 3),
+                                                          (64, 1 << 20, 2, 0)])
+def test_few_neurons_on_long_rows(bits, row_bytes, out_dim, offset):
+    rng = np.random.default_rng(row_bytes)
+    torch.manual_seed(row_bytes)
+    raw = rng.integers(0, 256, offset + 4 * row_bytes, dtype=np.uint8)
+    x = torch.from_numpy(raw).to(DEV)[offset:].view(TORCH_WORD[bits]).view(4, -1)
+    words = raw[offset:].copy().view(x.cpu().numpy().dtype).reshape(4, -1)
+    a, b = torch.randint(0, 4, (out_dim,), device=DEV), torch.randint(0, 4, (out_dim,), device=DEV)
+    logits = torch.randn(out_dim, 16, device=DEV)
+    gate, plan = difflogic_hip.gate_argmax(logits), difflogic_hip.eval_plan(a, b, 4)
+    want = O.eval_packed(words, a.cpu().numpy(), b.cpu().numpy(), gate.cpu().numpy())
+    for y in (difflogic_hip.eval_planned_logits(x, a, b, logits, plan), difflogic_hip.eval_planned(x, a, b, gate, plan), difflogic_hip.eval(x, a, b, gate)):
+        assert np.array_equal(y.cpu().numpy(), want)
+
+
+def test_one_long_row_takes_as_long_as_its_bytes_do():
+    # one neuron on a row of 16 MiB and 2048 neurons on 8 KiB each, the same bytes: a workgroup for each 8 KiB either way (in one workgroup 4 MiB take 530 us)
+    def microseconds(out_dim, row_bytes):
+        x = torch.randint(-128, 127, (2 * out_dim, row_bytes), dtype=torch.int8, device=DEV)
+        a = torch.arange(out_dim, device=DEV)
+        logits, plan, times = torch.randn(out_dim, 16, device=DEV), difflogic_hip.eval_plan(a, a + out_dim, 2 * out_dim), []
+        for _ in range(8):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(10):
+                difflogic_hip.eval_planned_logits(x, a, a + out_dim, logits, plan)
+            end.record()
+            end.synchronize()
+            times.append(100 * start.elapsed_time(end))
+        return min(times)
+    few, many = microseconds(1, 1 << 24), microseconds(2048, 1 << 13)
+    assert few <= 4 * many + 20, (few, many)
+
+
 @pytest.mark.parametrize("bits,batch,features,k", [(64, 256, 40, 10), (32, 100, 12, 3), (8, 9, 4, 2), (64, 5000, 2000, 10), (16, 33, 6, 6),
                                                    (64, 4133, 84, 4), (32, 4200, 30, 3), (8, 600, 9, 1), (64, 8192, 2400, 4),
                                                    (64, 4096, 7, 7), (64, 4096, 40000, 2)])
