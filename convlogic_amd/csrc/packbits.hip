@@ -729,6 +729,20 @@ bool walk_pays(int64_t row_bytes, int64_t out_dim)
     if (const char *e = clg_knob(K_EVAL_ROWS)) return atoi(e) == 0;
     return row_bytes >= 640 && row_bytes * out_dim >= (row_bytes >= 1 << 20 ? 20'000'000 : 30'000'000);
 }
+// Vectors of a lane in the walk, whose grid holds 65535 column chunks of them: 268 MB of a row
+int walk_vecs(int64_t row_vecs)
+{
+    const char *e = clg_knob(K_EVAL_WALK_R);
+    int R = e ? atoi(e) : 4;
+    while (R > 1 && (int64_t)kWave * (R / 2) >= row_vecs) R /= 2;
+    return R;
+}
+constexpr int64_t kWalkChunks = 65535;
+bool walk_takes(int64_t row_bytes, int64_t out_dim)
+{
+    const int64_t row_vecs = clg_ceil_div(row_bytes, 16);
+    return row_bytes >= 16 && walk_pays(row_bytes, out_dim) && clg_ceil_div(row_vecs, (int64_t)kWave * walk_vecs(row_vecs)) <= kWalkChunks;
+}
 
 bool valid_elem(int e) { return e == 1 || e == 2 || e == 4 || e == 8; }
 
@@ -992,12 +1006,11 @@ int launch_walk(const char *name, int elem_size, const void *x, const int64_t *a
                 void *y, int64_t in_dim, int64_t out_dim, int64_t words, void *stream)
 {
     const int64_t row_bytes = words * elem_size, row_vecs = clg_ceil_div(row_bytes, 16);
-    const char *e_r = clg_knob(K_EVAL_WALK_R), *e_l = clg_knob(K_EVAL_WALK_SEG);
-    int R = e_r ? atoi(e_r) : 4;
-    while (R > 1 && (int64_t)kWave * (R / 2) >= row_vecs) R /= 2;
+    const char *e_l = clg_knob(K_EVAL_WALK_SEG);
+    const int R = walk_vecs(row_vecs);
     const int seg = e_l ? atoi(e_l) : 8;
     const int64_t col_chunks = clg_ceil_div(row_vecs, (int64_t)kWave * R);
-    CLG_REQUIRE(col_chunks <= 65535, "%s: rows above %lld bytes are not supported", name, 65535ll * kWave * R * 16);
+    CLG_REQUIRE(col_chunks <= kWalkChunks, "%s: rows above %lld bytes are not supported", name, (long long)kWalkChunks * kWave * R * 16);
     const dim3 grid((unsigned)clg_ceil_div(out_dim, (int64_t)kEvalWaves * seg), (unsigned)col_chunks), block(kEvalBlock);
     hipStream_t st = clg_stream(stream);
 #define CLG_WALK(RR)                                                                                                          \
@@ -1026,7 +1039,7 @@ extern "C" int clg_fc_eval_packed_planned(int elem_size, const void *x, const in
     CLG_REQUIRE(x != y, "%s: x and y must not overlap", name);
     CLG_REQUIRE(in_dim > 0 && out_dim > 0 && words > 0, "%s: in_dim, out_dim and words must be positive", name);
     CLG_REQUIRE(out_dim < (1ll << 28), "%s: out_dim above 2^28-1 is not supported", name);
-    if (words * elem_size < 16 || !walk_pays(words * elem_size, out_dim)) return clg_fc_eval_packed(elem_size, x, a, b, gate, y, in_dim, out_dim, words, stream);
+    if (!walk_takes(words * elem_size, out_dim)) return clg_fc_eval_packed(elem_size, x, a, b, gate, y, in_dim, out_dim, words, stream);
     return launch_walk<false>(name, elem_size, x, a, b, gate, plan, y, in_dim, out_dim, words, stream);
 }
 
@@ -1062,6 +1075,6 @@ extern "C" int clg_fc_eval_packed_layer(int elem_size, const void *x, const int6
     const int64_t row_bytes = words * elem_size;
     CLG_REQUIRE(row_bytes >= 16 || (((uintptr_t)x | (uintptr_t)y | (uintptr_t)row_bytes) & 3) == 0, "%s: rows must be 16 bytes or more, or whole 4-byte words at "
                 "4-byte aligned addresses; use clg_gate_argmax + clg_fc_eval_packed otherwise", name);
-    if (row_bytes >= 16 && walk_pays(row_bytes, out_dim)) return launch_walk<true>(name, elem_size, x, a, b, logits, plan, y, in_dim, out_dim, words, stream);
+    if (walk_takes(row_bytes, out_dim)) return launch_walk<true>(name, elem_size, x, a, b, logits, plan, y, in_dim, out_dim, words, stream);
     return eval_packed<true>(name, elem_size, x, a, b, logits, y, in_dim, out_dim, words, stream);
 }

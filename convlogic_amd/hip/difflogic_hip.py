@@ -402,7 +402,7 @@ def eval_planned_logits(x, a, b, logits, plan):
     lib = _lib.load()
     y = torch.empty((out_dim, words), dtype=x.dtype, device=x.device)
     elem = x.element_size()
-    if logits.dtype != torch.float32 or (words * elem < 16 and (x.data_ptr() | y.data_ptr() | (words * elem)) & 3):
+    if logits.dtype != torch.float32 or (not 16 <= words * elem < 1 << 34 and (x.data_ptr() | y.data_ptr() | (words * elem)) & 3):
         return eval_planned(x, a, b, gate_argmax(logits), plan)
     check(lib.clg_fc_eval_packed_layer(elem, x.data_ptr(), a.data_ptr(), b.data_ptr(), logits.data_ptr(), plan.data_ptr(), y.data_ptr(), in_dim,
                                        out_dim, words, stream_ptr(x)))

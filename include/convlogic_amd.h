@@ -277,8 +277,8 @@ int clg_fc_eval_walk_fits(int elem_size, const void *x, const void *y, int64_t w
 int clg_fc_eval_packed_planned_logits(int elem_size, const void *x /*[in_dim,words]*/, const int64_t *a, const int64_t *b,
                                       const float *logits /*[out_dim,16]*/, const int32_t *plan /*[out_dim]*/,
                                       void *y /*[out_dim,words]*/, int64_t in_dim, int64_t out_dim, int64_t words, void *stream);
-/* The layer whatever its rows: along the plan where that pays, else lanes along the rows of several neurons.  Rows below 16 bytes must be
- * whole 4-byte words at 4-byte aligned addresses. */
+/* The layer whatever its rows: along the plan where that pays, else lanes along the rows of several neurons.  Rows below 16 bytes, and from
+ * 2^34 on, must be whole 4-byte words at 4-byte aligned addresses. */
 int clg_fc_eval_packed_layer(int elem_size, const void *x, const int64_t *a, const int64_t *b, const float *logits, const int32_t *plan,
                              void *y, int64_t in_dim, int64_t out_dim, int64_t words, void *stream);
 

@@ -122,6 +122,16 @@ def test_few_neurons_on_long_rows(bits, row_bytes, out_dim, offset):
         assert np.array_equal(y.cpu().numpy(), want)
 
 
+def test_rows_past_the_column_chunks_of_the_walk():
+    row_bytes = 65535 * 4096 + 19                                     # (of 65535 chunks of 4 KiB)
+    x = torch.randint(-128, 127, (2, row_bytes), dtype=torch.int8, device=DEV)
+    a, b = torch.tensor([0], device=DEV), torch.tensor([1], device=DEV)
+    logits = torch.nn.functional.one_hot(torch.tensor([[6]], device=DEV)[0], 16).float()      # XOR
+    plan, want = difflogic_hip.eval_plan(a, b, 2), (x[0] ^ x[1]).view(1, -1)
+    assert torch.equal(difflogic_hip.eval_planned_logits(x, a, b, logits, plan), want)
+    assert torch.equal(difflogic_hip.eval_planned(x, a, b, difflogic_hip.gate_argmax(logits), plan), want)
+
+
 def test_one_long_row_takes_as_long_as_its_bytes_do():
     # one neuron on a row of 16 MiB and 2048 neurons on 8 KiB each, the same bytes: a workgroup for each 8 KiB either way (in one workgroup 4 MiB take 530 us)
     def microseconds(out_dim, row_bytes):
