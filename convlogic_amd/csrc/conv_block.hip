@@ -49,6 +49,14 @@ int clg_launch_reduce_coef(int dtype, const void *partial, void *out, int64_t ro
 
 namespace {
 
+// Where a call leaves the sums that end its weight gradient to a later launch (to: null where it launches them itself), and where their
+// parts go (null: to the start of the weight gradient's scratch).
+struct LateSums {
+    clg_late_sums *to = nullptr;
+    void *parts = nullptr;
+    void *parts_or(void *scratch) const { return parts != nullptr ? parts : scratch; }
+};
+
 // ---------------------------------------------------------------------------------------------
 // input gradient
 // ---------------------------------------------------------------------------------------------
@@ -1316,10 +1324,10 @@ int launch_backward_x_direct(const Geom &g, const TilePlan &p, int sample_elems,
 
 template <typename T>
 int launch_backward_w_padded(const Geom &g, const TilePlan &p, const WScratch &ws, const void *gy, const void *x, const void *w,
-                             const int32_t *sel, const uint8_t *argmax, void *gw, void *scratch, hipStream_t st, const void *probs, clg_late_sums *late)
+                             const int32_t *sel, const uint8_t *argmax, void *gw, void *scratch, hipStream_t st, const void *probs, const LateSums &late)
 {
     unsigned char *base = reinterpret_cast<unsigned char *>(scratch);
-    T *partial = reinterpret_cast<T *>(base);
+    T *partial = reinterpret_cast<T *>(late.parts_or(base));
     T *folded = reinterpret_cast<T *>(base + ws.folded_off);
     int32_t *taps = reinterpret_cast<int32_t *>(base + ws.taps_off);
     T *xp = reinterpret_cast<T *>(base + ws.xp_off);
@@ -1339,18 +1347,18 @@ int launch_backward_w_padded(const Geom &g, const TilePlan &p, const WScratch &w
                            make_fastdiv((uint32_t)I), ws.sample_elems, 8);
     CLG_CHECK_LAUNCH("clg_convblock_backward_w(padded)");
     return clg_launch_reduce_coef(sizeof(T) == 8 ? CLG_F64 : CLG_F32, partial, gw, g.c, ws.nb, 7, st, "clg_convblock_backward_w(reduce)",
-                                  probs, late);
+                                  probs, late.to);
 }
 
 // weight gradient from the padded copy the input gradient of the same call has made
 template <typename T>
 int launch_backward_w_shared(const Geom &g, const SharedPad &sh, const void *gy, const uint8_t *argmax, void *gw, void *scratch,
-                             hipStream_t st, const void *probs, clg_late_sums *late)
+                             hipStream_t st, const void *probs, const LateSums &late)
 {
     const int64_t I = (int64_t)(g.ho / 2) * (g.wo / 2);
     int64_t nb = clg_ceil_div(I * g.n, 256 * cells_per_thread(I * g.n));
     nb = nb < 1 ? 1 : (nb > 64 ? 64 : nb);
-    T *partial = reinterpret_cast<T *>(scratch);                      // [c][nb][28], within the any-shape kernel's [c][64][28]
+    T *partial = reinterpret_cast<T *>(late.parts_or(scratch));       // [c][nb][28], within the any-shape kernel's [c][64][28]
     if (fixed_cells(g, (int)sizeof(T)))
         hipLaunchKernelGGL((convblock_backward_w_padded_kernel<T, true>), dim3((unsigned)nb, (unsigned)g.c), dim3(256), 0, st,
                            (const T *)gy, (const T *)sh.xp, (const T *)sh.folded, sh.taps, argmax, partial, g, sh.p,
@@ -1361,7 +1369,7 @@ int launch_backward_w_shared(const Geom &g, const SharedPad &sh, const void *gy,
                            make_fastdiv((uint32_t)I), sh.sample_elems, 16);
     CLG_CHECK_LAUNCH("clg_convblock_backward_w(padded, shared copy)");
     return clg_launch_reduce_coef(sizeof(T) == 8 ? CLG_F64 : CLG_F32, partial, gw, g.c, (int)nb, 7, st,
-                                  "clg_convblock_backward_w(reduce)", probs, late);
+                                  "clg_convblock_backward_w(reduce)", probs, late.to);
 }
 
 // Plan of the LDS-staged weight gradient: S samples per staged group (their image elements travel through at most
@@ -1424,7 +1432,7 @@ bool plan_backward_w_tiled(const Geom &g, int elem, TiledWPlan *tw)
 
 template <typename T>
 int launch_backward_w_tiled(const Geom &g, const TiledWPlan &tw, const void *gy, const void *x, const void *w, const int32_t *sel,
-                            const uint8_t *argmax, void *gw, void *scratch, hipStream_t st, const void *probs, clg_late_sums *late)
+                            const uint8_t *argmax, void *gw, void *scratch, hipStream_t st, const void *probs, const LateSums &late)
 {
     const dim3 grid((unsigned)tw.nb, (unsigned)clg_ceil_div(g.c, tw.p.CT)), block(kTiledWWaves * kWave);
     const int nparts = tw.nb * (kTiledWWaves / tw.p.CT);
@@ -1439,15 +1447,15 @@ int launch_backward_w_tiled(const Geom &g, const TiledWPlan &tw, const void *gy,
     do {                                                                                                                          \
         if (int e = allow_lds(convblock_backward_w_tiled_kernel<T, VV>, tw.p.lds_bytes, "clg_convblock_backward_w")) return e;    \
         hipLaunchKernelGGL((convblock_backward_w_tiled_kernel<T, VV>), grid, block, tw.p.lds_bytes, st, (const T *)gy, (const T *)x, \
-                           (const T *)w, sel, argmax, (T *)scratch, g, tw.p, tw.rounds);                                          \
+                           (const T *)w, sel, argmax, (T *)late.parts_or(scratch), g, tw.p, tw.rounds);                           \
     } while (0)
     if (v == 4) CLG_BWDW_TILED(4);
     else if (v == 2) CLG_BWDW_TILED(2);
     else CLG_BWDW_TILED(1);
 #undef CLG_BWDW_TILED
     CLG_CHECK_LAUNCH("clg_convblock_backward_w(tiled)");
-    return clg_launch_reduce_coef(sizeof(T) == 8 ? CLG_F64 : CLG_F32, scratch, gw, g.c, nparts, 7, st, "clg_convblock_backward_w(reduce)",
-                                  probs, late);
+    return clg_launch_reduce_coef(sizeof(T) == 8 ? CLG_F64 : CLG_F32, late.parts_or(scratch), gw, g.c, nparts, 7, st,
+                                  "clg_convblock_backward_w(reduce)", probs, late.to);
 }
 
 int elem_size(int dtype) { return dtype == CLG_F64 ? 8 : 4; }
@@ -1618,7 +1626,7 @@ extern "C" int clg_convblock_backward_x(int dtype, const clg_conv_geom *gg, cons
 // grad_w w.r.t. the gate probabilities, or -- with probs = the softmax output w -- w.r.t. the logits
 static int convblock_backward_w_impl(int dtype, const clg_conv_geom *gg, const void *grad_y, const void *x, const void *w,
                                      const int32_t *selection, const uint8_t *argmax, void *grad_w, void *scratch, void *stream,
-                                     const void *probs, const char *name, const SharedPad *shared = nullptr, clg_late_sums *late = nullptr)
+                                     const void *probs, const char *name, const SharedPad *shared = nullptr, const LateSums &late = {})
 {
     Geom g;
     if (int e = clg_convblock_check(gg, &g, dtype, name)) return e;
@@ -1631,10 +1639,11 @@ static int convblock_backward_w_impl(int dtype, const clg_conv_geom *gg, const v
     if (pair) {
         const int nb = clg_pair_grad_w_parts(g, pp);
         hipStream_t st = clg_stream(stream);
-        if (int e = clg_pair_grad_w(g, pp, nb, (const float *)grad_y, (const float *)x, (const float *)shared->folded, selection, argmax, (float *)scratch,
-                                    st, "clg_convblock_backward_w(two planes)"))
+        float *parts = (float *)late.parts_or(scratch);
+        if (int e = clg_pair_grad_w(g, pp, nb, (const float *)grad_y, (const float *)x, (const float *)shared->folded, selection, argmax, parts, st,
+                                    "clg_convblock_backward_w(two planes)"))
             return e;
-        return clg_launch_reduce_coef(CLG_F32, scratch, grad_w, g.c, nb, 7, st, "clg_convblock_backward_w(reduce)", probs, late);
+        return clg_launch_reduce_coef(CLG_F32, parts, grad_w, g.c, nb, 7, st, "clg_convblock_backward_w(reduce)", probs, late.to);
     }
     if (shared != nullptr && shared->xp != nullptr && g.c <= 65535) {
         if (dtype == CLG_F32) return launch_backward_w_shared<float>(g, *shared, grad_y, argmax, grad_w, scratch, clg_stream(stream), probs, late);
@@ -1874,7 +1883,7 @@ int64_t clg_convblock_backward_padded_sample_elems(int dtype, const Geom &g)
 
 static int backward_planned_impl(const char *name, int dtype, const clg_conv_geom *gg, const void *grad_y, const void *x, const void *w,
                                  const void *folded, const void *padded, const int32_t *selection, const uint8_t *argmax, void *plan,
-                                 int64_t signature, void *grad_x, void *grad_w, int flags, void *scratch, void *stream, clg_late_sums *late = nullptr)
+                                 int64_t signature, void *grad_x, void *grad_w, int flags, void *scratch, void *stream, const LateSums &late = {})
 {
     Geom g;
     if (int e = clg_convblock_check(gg, &g, dtype, name)) return e;
@@ -1910,9 +1919,9 @@ static int backward_planned_impl(const char *name, int dtype, const clg_conv_geo
         int nb = 0;
         float *planes = reinterpret_cast<float *>(reinterpret_cast<unsigned char *>(scratch) + backward_planes_off(g));
         if (int e = clg_pair_grads(g, pi.pair, &nb, (const float *)grad_y, (const float *)x, (const float *)tb.folded, selection, argmax, tb.count, tb.hits,
-                                   planes, (float *)w_scratch, (float *)grad_x, st, name))
+                                   planes, (float *)late.parts_or(w_scratch), (float *)grad_x, st, name))
             return e;
-        return clg_launch_reduce_coef(CLG_F32, w_scratch, grad_w, g.c, nb, 7, st, name, probs, late);
+        return clg_launch_reduce_coef(CLG_F32, late.parts_or(w_scratch), grad_w, g.c, nb, 7, st, name, probs, late.to);
     }
     if (grad_x != nullptr)
         if (int e = convblock_backward_x_impl(dtype, gg, grad_y, x, w, selection, argmax, grad_x, scratch, stream, &shared, w_scratch, &pv,
@@ -1932,7 +1941,7 @@ extern "C" int clg_convblock_backward_planned(int dtype, const clg_conv_geom *gg
 static int planned_padded(const char *name, int dtype, const clg_conv_geom *gg, const void *grad_y, const void *x, const void *w,
                           const void *folded, const void *padded, const int32_t *selection,
                           const uint8_t *argmax, void *plan, int64_t signature, void *grad_x, void *grad_w,
-                          int flags, void *scratch, void *stream, clg_late_sums *late)
+                          int flags, void *scratch, void *stream, const LateSums &late)
 {
     Geom g;
     if (int e = clg_convblock_check(gg, &g, dtype, name)) return e;
@@ -1946,14 +1955,26 @@ extern "C" int clg_convblock_backward_planned_padded(int dtype, const clg_conv_g
                                                      const void *folded, const void *padded, const int32_t *selection, const uint8_t *argmax, void *plan,
                                                      int64_t signature, void *grad_x, void *grad_w, int flags, void *scratch, void *stream)
 {
-    return planned_padded("clg_convblock_backward_planned_padded", dtype, gg, grad_y, x, w, folded, padded, selection, argmax, plan, signature, grad_x, grad_w, flags, scratch, stream, nullptr);
+    return planned_padded("clg_convblock_backward_planned_padded", dtype, gg, grad_y, x, w, folded, padded, selection, argmax, plan, signature, grad_x, grad_w, flags, scratch, stream, {});
+}
+
+extern "C" int64_t clg_convblock_late_sums_bytes(int dtype, const clg_conv_geom *gg)
+{
+    Geom g;
+    if (clg_convblock_check(gg, &g, dtype, "clg_convblock_late_sums_bytes")) return -1;
+    if (dtype != CLG_F32 || backward_4x4_wanted(g)) return 0;
+    TiledWPlan tw;
+    const char *e_pad = clg_knob(K_BWDW_PADDED);
+    const bool tiled = !(e_pad && atoi(e_pad) != 0) && plan_backward_w_tiled(g, 4, &tw);
+    return (int64_t)g.c * std::max(64, tiled ? tw.nb * (kTiledWWaves / tw.p.CT) : 0) * 28 * 4;
 }
 
 extern "C" int clg_convblock_backward_planned_late(int dtype, const clg_conv_geom *gg, const void *grad_y, const void *x, const void *w,
                                                    const void *folded, const void *padded, const int32_t *selection, const uint8_t *argmax, void *plan,
-                                                   int64_t signature, void *grad_x, void *grad_w, int flags, void *scratch, clg_late_sums *late, void *stream)
+                                                   int64_t signature, void *grad_x, void *grad_w, int flags, void *scratch, void *sums, clg_late_sums *late,
+                                                   void *stream)
 {
     CLG_REQUIRE(late, "clg_convblock_backward_planned_late: null pointer argument");
     *late = {};
-    return planned_padded("clg_convblock_backward_planned_late", dtype, gg, grad_y, x, w, folded, padded, selection, argmax, plan, signature, grad_x, grad_w, flags, scratch, stream, late);
+    return planned_padded("clg_convblock_backward_planned_late", dtype, gg, grad_y, x, w, folded, padded, selection, argmax, plan, signature, grad_x, grad_w, flags, scratch, stream, {late, sums});
 }

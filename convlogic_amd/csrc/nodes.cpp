@@ -175,13 +175,15 @@ struct Prepared {
         return {floats(like, {(int64_t)g.c_out * (112 + 28)}), bytes(like, clg_convblock_forward_scratch_bytes(CLG_F32, &g))};
     }
 };
-// Sums that the backward calls of a network's layers leave for one launch, and the buffers they are in.
+// Sums that the backward calls of a network's layers leave for one launch, and the buffers their parts are in -- those alone, a layer's scratch
+// is the next one's: operand gradients and gradient planes of all layers held together were twice the memory of a step (CIFAR topology, k =
+// 100, 1024 images: 3.07 GB, 1.88 like this and by the modules).
 struct Late {
     std::vector<clg_late_sums> sums;
     std::vector<Tensor> kept;
-    clg_late_sums *next(const Tensor &scratch)
+    clg_late_sums *next(const Tensor &parts)
     {
-        kept.push_back(scratch);
+        kept.push_back(parts);
         sums.push_back({});
         return &sums.back();
     }
@@ -258,10 +260,12 @@ std::pair<Tensor, Tensor> block_backward(const BlockState &state, const Conv &co
         const Tensor scratch = bytes(x, clg_convblock_backward_planned_scratch_bytes(CLG_F32, &g, signature));
         const Tensor padded = fm || !need_x ? Tensor() : state.padded;
         const int flags = CLG_BWD_WRT_LOGITS | (fm ? CLG_BWD_GY_FEATURE_MAJOR : 0);
-        if (late != nullptr)
+        if (late != nullptr) {
+            const Tensor parts = bytes(x, clg_convblock_late_sums_bytes(CLG_F32, &g));
             check(clg_convblock_backward_planned_late(CLG_F32, &g, gy.data_ptr(), x.data_ptr(), probs.data_ptr(), folded, ptr(padded), selection, codes,
-                                                      plan.data_ptr(), signature, ptr(gx), gl.data_ptr(), flags, scratch.data_ptr(),
-                                                      late->next(scratch), stream_of(x)));
+                                                      plan.data_ptr(), signature, ptr(gx), gl.data_ptr(), flags, scratch.data_ptr(), parts.data_ptr(),
+                                                      late->next(parts), stream_of(x)));
+        }
         else if (padded.defined())
             check(clg_convblock_backward_planned_padded(CLG_F32, &g, gy.data_ptr(), x.data_ptr(), probs.data_ptr(), folded, padded.data_ptr(),
                                                         selection, codes, plan.data_ptr(), signature, gx.data_ptr(), gl.data_ptr(), flags,
@@ -413,14 +417,15 @@ std::array<Tensor, 4> trees_backward(const Tensor &x, const Tensor &start, const
     for (int i = 0; i < 3; ++i)
         if (wanted[1 + i]) g[1 + i] = floats(x, {neurons[i], 16});
     const int64_t rows = g[0].defined() ? 8 * roots * batch : 0;
-    const Tensor scratch = floats(x, {rows + 28 * roots});           // operand gradients, then sums
+    const Tensor scratch = floats(x, {rows + (late ? 0 : 28 * roots)}), kept = late ? floats(x, {28 * roots}) : Tensor();   // operand gradients, sums
+    float *sums = late ? f32(kept) : f32(scratch) + rows;
     if (late != nullptr)
         check(clg_fc_tree_backward_late(f32(x), i32(tables[0]), i32(tables[1]), i32(tables[2]), f32(coef), f32(go), f32(probs), f32(g[1]), f32(g[2]),
-                                        f32(g[3]), f32(scratch), f32(scratch) + rows, idx(start), f32(g[0]), in_dim, roots, k, batch, batch, tau,
-                                        late->next(scratch), stream_of(x)));
+                                        f32(g[3]), f32(scratch), sums, idx(start), f32(g[0]), in_dim, roots, k, batch, batch, tau, late->next(kept),
+                                        stream_of(x)));
     else
         check(clg_fc_tree_backward(f32(x), i32(tables[0]), i32(tables[1]), i32(tables[2]), f32(coef), f32(go), f32(probs), f32(g[1]), f32(g[2]), f32(g[3]),
-                                   f32(scratch), f32(scratch) + rows, idx(start), f32(g[0]), in_dim, roots, k, batch, batch, tau, stream_of(x)));
+                                   f32(scratch), sums, idx(start), f32(g[0]), in_dim, roots, k, batch, batch, tau, stream_of(x)));
     return g;
 }
 struct Trees : torch::autograd::Function<Trees> {
@@ -520,6 +525,7 @@ struct Network : torch::autograd::Function<Network> {
             } else {
                 h = block_forward(h, logits[i], b.sel, b.conv, fm, b.signature, nullptr, some, state, together ? &made[i] : nullptr);
             }
+            made[i] = {};
             state.save(saved);
             const std::vector<int64_t> own{b.conv.sh, b.conv.sw, b.conv.ph, b.conv.pw, b.conv.kh, b.conv.kw, shape[0], shape[1], shape[2], shape[3],
                                            b.flag != 0, b.signature, fm};

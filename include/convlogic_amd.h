@@ -599,8 +599,9 @@ int clg_convblock_bin_backward(int dtype, const clg_conv_geom *g, const void *gr
  * CLG_FWD_PREPARED reads -- for a float32 block clg_convblock_forward_ex / _padded (flags CLG_FWD_W_LOGITS | CLG_FWD_FOLDED_OUT | CLG_FWD_FOLDED_IN |
  * CLG_FWD_PREPARED), for one on 0/1 inputs clg_convblock_bin_forward.  At most 16 blocks, one of them binary.
  * The _late calls are those without the suffix, but for a last launch that they describe in *late where they would end with one;
- * clg_late_sums_run launches those of up to 17 calls together.  Until then grad_w is not written, and the buffers of the calls, scratch
- * included, stay as they are. */
+ * clg_late_sums_run launches those of up to 17 calls together.  Until then grad_w is not written, and what it is made of stays as it is: w
+ * or ctx (probs of the trees), and sums -- for a float32 block clg_convblock_late_sums_bytes() of its own, beside which scratch is free
+ * when the call has returned (NULL: in scratch), for the others as without the suffix (scratch of a binary block, sums of the trees). */
 typedef struct clg_train_block {
     clg_conv_geom geom;
     const float *x;           /* binary block: its input, else NULL */
@@ -617,10 +618,11 @@ typedef struct clg_late_sums {
     int32_t kind, blocks;     /* kind 0: nothing is left to do */
     int64_t field[13];
 } clg_late_sums;
+int64_t clg_convblock_late_sums_bytes(int dtype, const clg_conv_geom *g);
 int clg_convblock_backward_planned_late(int dtype, const clg_conv_geom *g, const void *grad_y, const void *x, const void *w,
                                         const void *folded, const void *padded, const int32_t *selection, const uint8_t *argmax,
                                         void *plan, int64_t signature, void *grad_x, void *grad_w, int flags, void *scratch,
-                                        clg_late_sums *late, void *stream);
+                                        void *sums, clg_late_sums *late, void *stream);
 int clg_convblock_bin_backward_late(int dtype, const clg_conv_geom *g, const void *grad_y, const uint16_t *taps, const void *ctx,
                                     void *grad_x, void *grad_w, int flags, void *scratch, clg_late_sums *late, void *stream);
 int clg_fc_tree_backward_late(const float *x, const int32_t *rows, const int32_t *pos, const int32_t *slot, const float *coef,

@@ -170,3 +170,22 @@ def test_gradients_past_the_caches(monkeypatch, k, batch, by_modules):
     monkeypatch.undo()
     _lib.reload_knobs()
     assert all(torch.equal(a, b) for a, b in zip(*got, strict=True))
+
+
+# batches at which scratch is most of a step's memory: by one node no more of it than by the modules, whose scratch is one layer's at a time
+@pytest.mark.parametrize("topology,k,channels,batch", [("cifar", 32, 9, 256), ("cifar", 16, 3, 512), ("mnist", 32, 1, 1000)])
+def test_memory_of_a_step(at_once, topology, k, channels, batch):
+    model, side = network(topology, k, channels)
+    x = (torch.rand(batch, channels, side, side, device=DEV) < 0.5).float()
+    peak = []
+    for by_modules in (False, True):
+        model.prefold = not by_modules
+        for counted in (False, True):                                 # (plans are made in the first step)
+            model.zero_grad()
+            torch.cuda.empty_cache()
+            torch.cuda.reset_peak_memory_stats()
+            before = torch.cuda.memory_allocated()
+            model(x).sum().backward()
+        peak.append(torch.cuda.max_memory_allocated() - before)
+    # what the node keeps longer than the modules: the saved activations of the layers behind (their gradients' scratch is larger), parts of the sums
+    assert True in at_once and peak[0] <= 1.1 * peak[1], peak
