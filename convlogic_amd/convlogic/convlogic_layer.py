@@ -97,7 +97,7 @@ class _FullConvLogicLogitsFunction(Function):
             # needs a gradient and the kernels of this shape read one -- the zero-padded copy of x it staged
             y, argmax, w_prob, folded, *rest = convlogic_hip.full_convlogic_forward_logits(
                 x1, logits.detach(), selection, *geo, kernel_h, kernel_w, feature_major=fm, want_folded=True, validate=False,
-                want_padded=ctx.needs_input_grad[0] and convlogic_hip.lists_of(plan[1]) == convlogic_hip.LISTS_SHORT, prefolded=prefolded)
+                want_padded=ctx.needs_input_grad[0], signature=plan[1], prefolded=prefolded)
             padded = rest[0] if rest else None
             ctx.save_for_backward(x1, w_prob, selection, argmax, folded, *(() if padded is None else (padded,)))
             return y.permute(3, 0, 1, 2) if fm else y
@@ -186,8 +186,13 @@ class _KeptPlan:
         self.recorded = False
 
     def make(self, like, sel, layer):
-        """In place where there are tables already, and for the same kernels: a recorded step reads them at their addresses."""
+        """In place where there are tables already, and for the same kernels: a recorded step reads them at their addresses.  (Tables that no
+        recording reads: made anew where a kernel has taps in more than two channels now, or has none any more.)"""
         tables, lists = (None, convlogic_hip.LISTS_LOOK) if self.plan is None else (self.plan[0], convlogic_hip.lists_of(self.plan[1]))
+        if self.plan is not None and not self.recorded:
+            wide = convlogic_hip.LISTS_WIDE if convlogic_hip.taps_are_wide(sel, layer.in_channels) else 0
+            if (lists & convlogic_hip.LISTS_WIDE) != wide:
+                tables, lists = None, convlogic_hip.LISTS_LOOK
         self.plan = convlogic_hip.make_backward_plan(like, layer.out_channels, sel, *layer.stride, *layer.padding, *layer.kernel, into=tables,
                                                      lists=lists)
 

@@ -1521,12 +1521,12 @@ static bool backward_planes_wanted(const Geom &g, int dtype, PairPlan *p)
 }
 static size_t backward_planes_off(const Geom &g) { return (bwd_scratch_layout(g, 4, 1).total + 255) & ~(size_t)255; }
 
-static int64_t backward_x_scratch_bytes(const char *name, int dtype, const clg_conv_geom *gg, bool long_lists, bool planned = false)
+static int64_t backward_x_scratch_bytes(const char *name, int dtype, const clg_conv_geom *gg, bool long_lists, bool planes = false)
 {
     Geom g;
     if (clg_convblock_check(gg, &g, dtype, name)) return -1;
     PairPlan pp;
-    if (planned && backward_planes_wanted(g, dtype, &pp)) return (int64_t)(backward_planes_off(g) + clg_pair_planes_bytes(g));
+    if (planes && backward_planes_wanted(g, dtype, &pp)) return (int64_t)(backward_planes_off(g) + clg_pair_planes_bytes(g));
     TilePlan p;
     int se = 0;
     const BwdXMode mode = choose_backward_x(g, elem_size(dtype), &p, &se, long_lists);
@@ -1692,9 +1692,9 @@ static int convblock_backward_4x4(int dtype, const Geom &g, const void *grad_y, 
                                       tb.count, tb.hits, grad_x, st, name);
 }
 
-static int64_t backward_scratch_bytes(const char *name, int dtype, const clg_conv_geom *gg, bool long_lists, bool planned = false)
+static int64_t backward_scratch_bytes(const char *name, int dtype, const clg_conv_geom *gg, bool long_lists, bool planes = false)
 {
-    const int64_t a = backward_x_scratch_bytes(name, dtype, gg, long_lists, planned), b = clg_convblock_backward_w_scratch_bytes(dtype, gg);
+    const int64_t a = backward_x_scratch_bytes(name, dtype, gg, long_lists, planes), b = clg_convblock_backward_w_scratch_bytes(dtype, gg);
     if (a < 0 || b < 0) return -1;
     int64_t total = ((a + 255) & ~255ll) + b;
     Geom g;
@@ -1711,7 +1711,7 @@ extern "C" int64_t clg_convblock_backward_scratch_bytes(int dtype, const clg_con
 }
 extern "C" int64_t clg_convblock_backward_planned_scratch_bytes(int dtype, const clg_conv_geom *gg, int64_t signature)
 {
-    return backward_scratch_bytes("clg_convblock_backward_planned_scratch_bytes", dtype, gg, (signature & 1) != 0, true);
+    return backward_scratch_bytes("clg_convblock_backward_planned_scratch_bytes", dtype, gg, (signature & CLG_LISTS_LONG) != 0, (signature & CLG_LISTS_WIDE) == 0);
 }
 
 extern "C" int clg_convblock_backward(int dtype, const clg_conv_geom *gg, const void *grad_y, const void *x, const void *w,
@@ -1786,13 +1786,16 @@ struct PlanInfo {
     bool planes;                                                     // both gradients by `pair`
     PairPlan pair;
 };
-// long_lists is the lowest bit of the signature (0 where it makes no difference), so a planned call finds the kernels again.
-PlanInfo plan_info(const Geom &g, int dtype, bool long_lists)
+// lists: CLG_LISTS_LONG, CLG_LISTS_WIDE or both.  They are the lowest bits of the signature (0 where they make no difference), so a planned call
+// finds the kernels again.
+PlanInfo plan_info(const Geom &g, int dtype, int lists)
 {
     PlanInfo pi;
+    bool long_lists = (lists & CLG_LISTS_LONG) != 0;
     const int elem = elem_size(dtype);
     int mode = 3, rs = 0, chs = 0;                                    // 3: one sample per lane on 4x4 images, 4: gradient planes
-    pi.planes = backward_planes_wanted(g, dtype, &pi.pair);
+    const bool wanted = backward_planes_wanted(g, dtype, &pi.pair), wide = wanted && (lists & CLG_LISTS_WIDE) != 0;
+    pi.planes = wanted && !wide;
     if (pi.planes) {
         mode = 4;
         long_lists = false;
@@ -1819,8 +1822,43 @@ PlanInfo plan_info(const Geom &g, int dtype, bool long_lists)
         h ^= (uint64_t)f;
         h *= 1099511628211ull;
     }
-    pi.signature = (int64_t)(h & 0x7ffffffffffffffeull) | (long_lists ? 1 : 0);
+    pi.signature = (int64_t)(h & 0x7ffffffffffffffcull) | (long_lists ? CLG_LISTS_LONG : 0) | (wide ? CLG_LISTS_WIDE : 0);
     return pi;
+}
+int lists_of(int64_t signature) { return (int)(signature & (CLG_LISTS_LONG | CLG_LISTS_WIDE)); }
+
+// from the device to the host, waiting for the stream
+std::unique_ptr<int32_t[]> host_copy(const void *from, size_t count, hipStream_t st, const char *name)
+{
+    std::unique_ptr<int32_t[]> to(new (std::nothrow) int32_t[count]);
+    if (to == nullptr) {
+        clg_set_error("%s: out of host memory", name);
+        return to;
+    }
+    hipError_t err = hipMemcpyAsync(to.get(), from, count * 4, hipMemcpyDeviceToHost, st);
+    if (err == hipSuccess) err = hipStreamSynchronize(st);
+    if (err != hipSuccess) {
+        clg_set_error("%s: the lists cannot be read (%s); inside a recording lists cannot be CLG_LISTS_LOOK", name, hipGetErrorString(err));
+        to.reset();
+    }
+    return to;
+}
+// Whether some kernel's taps are in more than two channels.  Gradient planes hold two channels of a kernel, plane_sums_kernel evaluates such a
+// one element by element for each of its channels: forward and backward of [256,128,8,8] -> 512, us by the other kernels and with planes, no such
+// kernel 67 and 60, 2 % of them 75 and 86, all 207 and 713; [64,512,12,12] -> 2048 176 and 145, 184 and 194, 454 and 2062; [16,32,6,6] -> 256 41 and 21, 43 and
+// 42, 66 and 481.  (A channel that many kernels read is no reason: all kernels on one channel 479 and 100, 1993 and 337, 211 and 41.)
+bool taps_are_wide(const Geom &g, const int32_t *selection)
+{
+    for (int64_t c = 0; c < g.c; ++c) {
+        int ch[2] = {-1, -1};
+        for (int t = 0; t < 8; ++t) {
+            const int at = std::min((selection[c * 8 + t] >> 16) & 0xFFFF, g.cin - 1);
+            if (ch[0] < 0 || at == ch[0]) ch[0] = at;
+            else if (ch[1] < 0 || at == ch[1]) ch[1] = at;
+            else return true;
+        }
+    }
+    return false;
 }
 }  // namespace
 
@@ -1828,7 +1866,7 @@ extern "C" int64_t clg_convblock_plan_bytes(int dtype, const clg_conv_geom *gg)
 {
     Geom g;
     if (clg_convblock_check(gg, &g, dtype, "clg_convblock_plan_bytes")) return -1;
-    return (int64_t)plan_info(g, dtype, false).total;                 // (the same tables for lists of any length)
+    return (int64_t)plan_info(g, dtype, CLG_LISTS_SHORT).total;       // (the same tables for every choice)
 }
 
 // lists and tap offsets by the set-up launch of the unplanned path (no weights: nothing is folded)
@@ -1845,21 +1883,26 @@ extern "C" int clg_convblock_plan_lists(int dtype, const clg_conv_geom *gg, cons
     Geom g;
     if (int e = clg_convblock_check(gg, &g, dtype, name)) return e;
     CLG_REQUIRE(selection && plan && signature, "%s: null pointer argument", name);
-    CLG_REQUIRE(lists >= CLG_LISTS_LOOK && lists <= CLG_LISTS_LONG, "%s: lists must be a CLG_LISTS_ value, got %d", name, lists);
+    CLG_REQUIRE(lists >= CLG_LISTS_LOOK && lists <= (CLG_LISTS_LONG | CLG_LISTS_WIDE), "%s: lists must be a CLG_LISTS_ value, got %d", name, lists);
     hipStream_t st = clg_stream(stream);
-    const PlanInfo pi = plan_info(g, dtype, lists == CLG_LISTS_LONG);
+    const PlanInfo pi = plan_info(g, dtype, lists == CLG_LISTS_LOOK ? CLG_LISTS_SHORT : lists);
     if (int e = make_plan(g, dtype, pi, selection, plan, st)) return e;
     *signature = pi.signature;
     if (lists != CLG_LISTS_LOOK) return CLG_OK;
-    const PlanInfo other = plan_info(g, dtype, true);
-    if (other.signature == pi.signature) return CLG_OK;
-    const size_t entries = 2 * (size_t)g.cin;
-    const std::unique_ptr<int32_t[]> count(new (std::nothrow) int32_t[entries]);
-    CLG_REQUIRE(count != nullptr, "%s: out of host memory", name);
-    hipError_t err = hipMemcpyAsync(count.get(), reinterpret_cast<unsigned char *>(plan) + pi.lay.count_off, entries * 4, hipMemcpyDeviceToHost, st);
-    if (err == hipSuccess) err = hipStreamSynchronize(st);
-    CLG_REQUIRE(err == hipSuccess, "%s: the lists cannot be read (%s); inside a recording lists cannot be CLG_LISTS_LOOK", name, hipGetErrorString(err));
-    if (!lists_are_long(g, elem_size(dtype), count.get())) return CLG_OK;
+    int found = CLG_LISTS_SHORT;
+    if (pi.planes) {
+        const auto taps = host_copy(selection, (size_t)g.c * 8, st, name);
+        if (taps == nullptr) return CLG_EINVAL;
+        if (!taps_are_wide(g, taps.get())) return CLG_OK;
+        found = CLG_LISTS_WIDE;
+    }
+    if (plan_info(g, dtype, found | CLG_LISTS_LONG).signature != plan_info(g, dtype, found).signature) {
+        const auto count = host_copy(reinterpret_cast<unsigned char *>(plan) + pi.lay.count_off, 2 * (size_t)g.cin, st, name);
+        if (count == nullptr) return CLG_EINVAL;
+        if (lists_are_long(g, elem_size(dtype), count.get())) found |= CLG_LISTS_LONG;
+    }
+    if (found == CLG_LISTS_SHORT) return CLG_OK;
+    const PlanInfo other = plan_info(g, dtype, found);
     if (int e = make_plan(g, dtype, other, selection, plan, st)) return e;
     *signature = other.signature;
     return CLG_OK;
@@ -1871,13 +1914,13 @@ extern "C" int clg_convblock_plan(int dtype, const clg_conv_geom *gg, const int3
     return clg_convblock_plan_lists(dtype, gg, selection, plan, CLG_LISTS_SHORT, signature, stream);
 }
 
-// One sample of the padded copy the planned backward pass reads when its input gradient is the direct kernel, else 0.
-int64_t clg_convblock_backward_padded_sample_elems(int dtype, const Geom &g)
+// One sample of the padded copy that the backward pass of a plan of these lists reads when its input gradient is the direct kernel, else 0.
+int64_t clg_convblock_backward_padded_sample_elems(int dtype, const Geom &g, int lists)
 {
     TilePlan p;
     PairPlan pp;
     int se = 0;
-    if (backward_4x4_wanted(g) || backward_planes_wanted(g, dtype, &pp)) return 0;
+    if ((lists & CLG_LISTS_LONG) != 0 || backward_4x4_wanted(g) || ((lists & CLG_LISTS_WIDE) == 0 && backward_planes_wanted(g, dtype, &pp))) return 0;
     return choose_backward_x(g, elem_size(dtype), &p, &se) == kBwdXDirect ? se : 0;
 }
 
@@ -1892,8 +1935,8 @@ static int backward_planned_impl(const char *name, int dtype, const clg_conv_geo
     const bool wrt_logits = (flags & CLG_BWD_WRT_LOGITS) != 0, fm = (flags & CLG_BWD_GY_FEATURE_MAJOR) != 0;
     CLG_REQUIRE(!fm || clg_convblock_fm_supported(dtype, gg), "%s: CLG_BWD_GY_FEATURE_MAJOR needs a shape for which "
                 "clg_convblock_fm_supported() holds (4x4 images, 3x3 kernel, stride 1, padding 1, n >= 32)", name);
-    const bool long_lists = (signature & 1) != 0;
-    const PlanInfo pi = plan_info(g, dtype, long_lists);
+    const bool long_lists = (signature & CLG_LISTS_LONG) != 0;
+    const PlanInfo pi = plan_info(g, dtype, lists_of(signature));
     CLG_REQUIRE(signature == pi.signature, "%s: the plan was made for another geometry, element type or kernel choice (make a new one "
                 "with clg_convblock_plan; the CLG_* knobs are part of the choice)", name);
     unsigned char *pb = reinterpret_cast<unsigned char *>(plan);
@@ -1908,7 +1951,7 @@ static int backward_planned_impl(const char *name, int dtype, const clg_conv_geo
         g.y_fm = fm ? 1 : 0;
         return convblock_backward_4x4(dtype, g, grad_y, x, w, selection, argmax, grad_x, grad_w, scratch, stream, probs, name, &pv);
     }
-    const int64_t a = backward_x_scratch_bytes(name, dtype, gg, long_lists, true);
+    const int64_t a = backward_x_scratch_bytes(name, dtype, gg, long_lists, pi.planes);
     if (a < 0) return CLG_EINVAL;
     SharedPad shared;
     void *w_scratch = reinterpret_cast<unsigned char *>(scratch) + ((a + 255) & ~255ll);
@@ -1945,7 +1988,7 @@ static int planned_padded(const char *name, int dtype, const clg_conv_geom *gg, 
 {
     Geom g;
     if (int e = clg_convblock_check(gg, &g, dtype, name)) return e;
-    CLG_REQUIRE(padded == nullptr || (grad_x != nullptr && clg_convblock_backward_padded_sample_elems(dtype, g) > 0 && (signature & 1) == 0),
+    CLG_REQUIRE(padded == nullptr || (grad_x != nullptr && clg_convblock_backward_padded_sample_elems(dtype, g, lists_of(signature)) > 0),
                 "%s: a padded copy is only taken with grad_x, where clg_convblock_padded_elems() is not 0 and for a plan of short lists", name);
     return backward_planned_impl(name, dtype, gg, grad_y, x, w, folded, padded, selection, argmax, plan, signature, grad_x, grad_w, flags,
                                  scratch, stream, late);

@@ -870,7 +870,7 @@ __global__ __launch_bounds__(256) void softmax16_rows_kernel(const T *__restrict
 }  // namespace
 
 // Forward of the complete block with options (flags: CLG_FWD_W_LOGITS, CLG_FWD_Y_FEATURE_MAJOR).
-int64_t clg_convblock_backward_padded_sample_elems(int dtype, const Geom &g);
+int64_t clg_convblock_backward_padded_sample_elems(int dtype, const Geom &g, int lists);
 
 static int forward_ex_impl(const char *name, int dtype, const clg_conv_geom *gg, const void *x, const void *w, const int32_t *selection,
                            void *y, uint8_t *argmax, void *probs_out, int flags, void *scratch, void *padded_out, void *stream)
@@ -1005,7 +1005,7 @@ extern "C" int clg_convblock_forward_ex(int dtype, const clg_conv_geom *gg, cons
 // Elements of the padded copy of x that clg_convblock_forward_padded leaves for clg_convblock_backward_planned_padded, or 0
 // when the pair has no use for one at this shape: the forward must stage or read the copy anyway (all channels in LDS, or
 // the direct kernel) and the backward must be the one that reads its taps from such a copy.
-extern "C" int64_t clg_convblock_padded_elems(int dtype, const clg_conv_geom *gg, int have_scratch)
+extern "C" int64_t clg_convblock_padded_elems_planned(int dtype, const clg_conv_geom *gg, int have_scratch, int64_t signature)
 {
     Geom g;
     if (clg_convblock_check(gg, &g, dtype, "clg_convblock_padded_elems")) return -1;
@@ -1015,10 +1015,14 @@ extern "C" int64_t clg_convblock_padded_elems(int dtype, const clg_conv_geom *gg
     PairPlan pp;
     const int path = choose_forward(g, elem, 28, have_scratch != 0, &tp, &dp, &pp);
     if (path != 0 && path != 2 && path != 5 && path != 6) return 0;
-    const int64_t se = clg_convblock_backward_padded_sample_elems(dtype, g);
+    const int64_t se = clg_convblock_backward_padded_sample_elems(dtype, g, (int)(signature & (CLG_LISTS_LONG | CLG_LISTS_WIDE)));
     if (se <= 0) return 0;
     const int64_t mine = path == 2 ? dp.sample_elems : (int64_t)g.cin * tp.chs + g.ph * tp.rs + g.pw;
     return se == mine ? se * g.n : 0;
+}
+extern "C" int64_t clg_convblock_padded_elems(int dtype, const clg_conv_geom *gg, int have_scratch)
+{
+    return clg_convblock_padded_elems_planned(dtype, gg, have_scratch, CLG_LISTS_SHORT);
 }
 
 extern "C" int clg_convblock_forward_padded(int dtype, const clg_conv_geom *gg, const void *x, const void *w, const int32_t *selection,
@@ -1027,7 +1031,7 @@ extern "C" int clg_convblock_forward_padded(int dtype, const clg_conv_geom *gg, 
 {
     const char *name = "clg_convblock_forward_padded";
     CLG_REQUIRE(padded_out, "%s: null pointer argument", name);
-    CLG_REQUIRE((flags & CLG_FWD_Y_FEATURE_MAJOR) == 0 && clg_convblock_padded_elems(dtype, gg, scratch != nullptr) > 0,
+    CLG_REQUIRE((flags & CLG_FWD_Y_FEATURE_MAJOR) == 0 && clg_convblock_padded_elems_planned(dtype, gg, scratch != nullptr, CLG_LISTS_WIDE) > 0,
                 "%s: no padded copy at this shape (clg_convblock_padded_elems)", name);
     return forward_ex_impl(name, dtype, gg, x, w, selection, y, argmax, probs_out, flags, scratch, padded_out, stream);
 }

@@ -219,8 +219,8 @@ Tensor block_forward(const Tensor &x_in, const Tensor &logits, const Tensor &sel
     const int flags = CLG_FWD_W_LOGITS | (fm ? CLG_FWD_Y_FEATURE_MAJOR : 0) | CLG_FWD_FOLDED_OUT |
                       (made != nullptr ? CLG_FWD_FOLDED_IN | CLG_FWD_PREPARED : (pair != nullptr ? CLG_FWD_FOLDED_IN : 0));
     Tensor padded;
-    if (need_x && (signature & 1) == CLG_LISTS_SHORT && !fm) {        // the copy of x that the forward kernels stage and the backward reads
-        const int64_t elems = clg_convblock_padded_elems(CLG_F32, &g, 1);
+    if (need_x && !fm) {                                              // the copy of x that the forward kernels stage and the backward reads
+        const int64_t elems = clg_convblock_padded_elems_planned(CLG_F32, &g, 1, signature);
         if (elems > 0) padded = floats(x, {elems});
     }
     const int32_t *selection = static_cast<const int32_t *>(sel.data_ptr());

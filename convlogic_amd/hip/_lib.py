@@ -100,6 +100,7 @@ SIGNATURES = {
     "clg_convblock_fm_supported": (_i, [_i, _GP]),
     "clg_convblock_forward_ex": (_i, [_i, _GP, _p, _p, _p, _p, _p, _p, _i, _p, _p]),
     "clg_convblock_padded_elems": (_i64, [_i, _GP, _i]),
+    "clg_convblock_padded_elems_planned": (_i64, [_i, _GP, _i, _i64]),
     "clg_convblock_forward_padded": (_i, [_i, _GP, _p, _p, _p, _p, _p, _p, _i, _p, _p, _p]),
     "clg_convblock_eval_packed_fm_supported": (_i, [_GP]),
     "clg_convblock_eval_packed_fm": (_i, [_GP, _p, _p, _p, _p, _p]),

@@ -338,13 +338,13 @@ def full_convlogic_forward_fm(x, weight, selection, stride_h, stride_w, pad_h, p
 
 
 def full_convlogic_forward_logits(x, logits, selection, stride_h, stride_w, pad_h, pad_w, kernel_h, kernel_w, feature_major=False,
-                                  want_folded=False, validate=True, want_padded=False, prefolded=None):
+                                  want_folded=False, validate=True, want_padded=False, prefolded=None, signature=0):
     """full_convlogic_forward() from the LOGITS [C, 7, 16]: the softmax is taken inside the launch that sets the gate
     parameters up.  -> (y, argmax, probs); with feature_major (where feature_major_supported) y is laid out
     [C, Ho/2, Wo/2, N] as from full_convlogic_forward_fm().  want_folded: -> (y, argmax, probs, folded [C, 7, 4]), the
     folded coefficients of every gate for full_convlogic_backward_planned().  want_padded (with want_folded): a fifth
     result, the zero-padded copy of x that the forward kernels stage anyway and the planned backward pass would otherwise
-    make in a launch of its own -- or None where the pair of kernels at this shape has no use for one.  prefolded (with
+    make in a launch of its own -- or None where the pair of kernels at this shape (and a plan of this signature) has no use for one.  prefolded (with
     want_folded): the (probs, folded) pair that difflogic_hip.fold_many() made from these logits -- the call then launches
     no softmax or fold of its own and returns that pair."""
     if validate:
@@ -372,7 +372,7 @@ def full_convlogic_forward_logits(x, logits, selection, stride_h, stride_w, pad_
     flags = 1 | (2 if feature_major else 0) | (4 if want_folded else 0) | (8 if prefolded is not None and want_folded else 0)
     padded = None
     if want_padded and want_folded and not feature_major:
-        elems = lib.clg_convblock_padded_elems(dtype_code(x), ctypes.byref(g), 1 if scratch is not None else 0)
+        elems = lib.clg_convblock_padded_elems_planned(dtype_code(x), ctypes.byref(g), 1 if scratch is not None else 0, signature)
         if elems > 0:
             padded = torch.empty((elems,), dtype=x.dtype, device=x.device)
     if padded is not None:
@@ -390,7 +390,7 @@ def full_convlogic_forward_logits(x, logits, selection, stride_h, stride_w, pad_
     return y, argmax, probs
 
 
-LISTS_LOOK, LISTS_SHORT = -1, 0                                       # CLG_LISTS_* (include/convlogic_amd.h)
+LISTS_LOOK, LISTS_SHORT, LISTS_LONG, LISTS_WIDE = -1, 0, 1, 2         # CLG_LISTS_* (include/convlogic_amd.h)
 
 
 def make_backward_plan(x, c_out, selection, stride_h, stride_w, pad_h, pad_w, kernel_h, kernel_w, into=None, lists=LISTS_SHORT):
@@ -416,8 +416,15 @@ def make_backward_plan(x, c_out, selection, stride_h, stride_w, pad_h, pad_w, ke
 
 
 def lists_of(signature):
-    """What a plan's kernels were chosen for: LISTS_SHORT, or 1 for a channel that many kernels read (they take no padded copy of x)."""
-    return signature & 1
+    """What a plan's kernels were chosen for: LISTS_SHORT, or of LISTS_LONG for a channel that many kernels read (they take no padded copy of x) and
+    LISTS_WIDE for kernels with taps in more than two channels."""
+    return signature & (LISTS_LONG | LISTS_WIDE)
+
+
+def taps_are_wide(selection, channels):
+    """Whether the taps of some kernel are in more than two channels (waits for the device)."""
+    ch = ((selection >> 16) & 0xFFFF).clamp(max=channels - 1).sort(1).values
+    return bool(((ch[:, 1:] != ch[:, :-1]).sum(1) > 1).any())
 
 
 def full_convlogic_backward_planned(grad_y, x, weight, folded, argmax, selection, plan, signature, stride_h, stride_w, pad_h, pad_w,
@@ -453,7 +460,7 @@ def full_convlogic_backward_planned(grad_y, x, weight, folded, argmax, selection
     if padded is not None and need_grad_x:
         # the padded copy of x that full_convlogic_forward_logits(want_padded=True) left: no launch to make one
         if validate:
-            check_input(padded, "padded", x.dtype, (lib.clg_convblock_padded_elems(dt, ctypes.byref(g), 1),))
+            check_input(padded, "padded", x.dtype, (lib.clg_convblock_padded_elems_planned(dt, ctypes.byref(g), 1, signature & LISTS_WIDE),))
         check(lib.clg_convblock_backward_planned_padded(dt, ctypes.byref(g), grad_y.data_ptr(), x.data_ptr(), weight.data_ptr(),
                                                         folded.data_ptr() if folded is not None else None, padded.data_ptr(),
                                                         selection.data_ptr(), argmax.data_ptr(), plan.data_ptr(), signature, gx.data_ptr(),

@@ -473,11 +473,14 @@ int64_t clg_convblock_plan_bytes(int dtype, const clg_conv_geom *g);
 int clg_convblock_plan(int dtype, const clg_conv_geom *g, const int32_t *selection, void *plan, int64_t *signature, void *stream);
 /* The same, where the caller knows more of the selection than that its taps are spread over the channels like random ones.
  * CLG_LISTS_LONG: so many kernels read one channel that the kernels for short lists, where a list is one wavefront's work,
- * are the slower ones.  CLG_LISTS_LOOK: looks at the lists and chooses (waits for the stream; not inside a recording).  The choice is the lowest bit
- * of the signature; plans made again in the memory of one that is in use must be given it as `lists`. */
+ * are the slower ones.  CLG_LISTS_WIDE (alone or with CLG_LISTS_LONG): the taps of some kernel are in more than two channels, which the kernels that
+ * keep a plane for each of a kernel's two channels evaluate one by one.  CLG_LISTS_LOOK: looks at the lists and chooses (waits for the stream; not
+ * inside a recording).  The choice is the lowest two bits of the signature; plans made again in the memory of one that is in use must be given it as
+ * `lists`. */
 #define CLG_LISTS_LOOK -1
 #define CLG_LISTS_SHORT 0
 #define CLG_LISTS_LONG 1
+#define CLG_LISTS_WIDE 2
 int clg_convblock_plan_lists(int dtype, const clg_conv_geom *g, const int32_t *selection, void *plan, int lists, int64_t *signature,
                              void *stream);
 /* scratch of the planned calls (clg_convblock_backward_scratch_bytes for a plan of short lists) */
@@ -495,13 +498,15 @@ int clg_convblock_backward_planned(int dtype, const clg_conv_geom *g, const void
 /* The padded hand-off.  The forward kernels of most shapes stage a zero-padded copy of x (in LDS, or in their scratch), and
  * the input gradient of layers with many channels reads its taps from exactly such a copy, which the backward call
  * otherwise makes in a launch of its own.  clg_convblock_padded_elems(): elements of that copy (n samples of
- * c_in * (h + ph) * (w + pw) + ph * (w + pw) + pw) when both sides have use for it at this shape, else 0.
+ * c_in * (h + ph) * (w + pw) + ph * (w + pw) + pw) when both sides have use for it at this shape, else 0;
+ * clg_convblock_padded_elems_planned(): with a plan of this signature.
  * clg_convblock_forward_padded = clg_convblock_forward_ex that also leaves the copy in padded_out;
  * clg_convblock_backward_planned_padded = clg_convblock_backward_planned that reads it (`padded` may be NULL: the plain
  * call) -- same values.  The reference pads x once per weight-gradient call (torch::constant_pad_nd,
  * src/convlogic/cuda/full_convlogic_kernel.cu:635) and bounds-checks every tap elsewhere (:16-33, :241-257); here one
  * padded copy per step serves the forward and both gradients. */
 int64_t clg_convblock_padded_elems(int dtype, const clg_conv_geom *g, int have_scratch);
+int64_t clg_convblock_padded_elems_planned(int dtype, const clg_conv_geom *g, int have_scratch, int64_t signature);
 int clg_convblock_forward_padded(int dtype, const clg_conv_geom *g, const void *x, const void *w, const int32_t *selection, void *y,
                                  uint8_t *argmax, void *probs_out, int flags, void *scratch, void *padded_out, void *stream);
 int clg_convblock_backward_planned_padded(int dtype, const clg_conv_geom *g, const void *grad_y, const void *x, const void *w,

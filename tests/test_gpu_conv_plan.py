@@ -166,6 +166,57 @@ def test_a_channel_that_many_kernels_read_keeps_the_kernels_of_long_lists(shape,
     assert_grad_close(gx, x.grad, rel=1e-4)
 
 
+def wide(sel, cin, part):
+    """the selection with the taps of every `part`-th kernel in any channels"""
+    ch = torch.randint(0, cin, sel.shape, device=sel.device, dtype=torch.int32)
+    return torch.where((torch.arange(sel.shape[0], device=sel.device) % part == 0).view(-1, 1), (ch << 16) | (sel & 0xFFFF), sel)
+
+
+# both gradients by planes unless some kernel's taps are in more than two channels: then by the kernels without planes, bit for bit (one with a padded
+# copy from the forward call, one whose channels with many kernels take the kernels of long lists)
+@pytest.mark.parametrize("shape", [(16, 32, 256, 6), (256, 32, 128, 16), (32, 16, 128, 20)])
+def test_taps_in_many_channels_take_the_kernels_without_planes(shape, monkeypatch):
+    n, cin, cout, side = shape
+    torch.manual_seed(n)
+    layer, lib = C.ConvLogicLayer(cin, cout, padding=1, complete=True, implementation="cuda").to(DEV), _lib.load()
+    x, geo = torch.rand(n, cin, side, side, device=DEV), (1, 1, 1, 1)
+    def gradients(sel, lists):
+        plan, sig = convlogic_hip.make_backward_plan(x, cout, sel, *geo, 3, 3, lists=lists)
+        geom = ctypes.byref(convlogic_hip._geom(x, cout, *geo, 3, 3))
+        y, am, probs, folded, padded = convlogic_hip.full_convlogic_forward_logits(x, layer.weights.detach(), sel, *geo, 3, 3, want_folded=True, want_padded=True,
+                                                                                   signature=sig)
+        torch.manual_seed(1)
+        gy = torch.randn_like(y)
+        got = convlogic_hip.full_convlogic_backward_planned(gy, x, probs, folded, am, sel, plan, sig, *geo, padded=padded)
+        return sig, lib.clg_convblock_backward_planned_scratch_bytes(0, geom, sig), None if padded is None else padded.numel(), got
+    for sel, is_wide in ((layer.selection, 0), (wide(layer.selection, cin, cout), 2), (wide(layer.selection, cin, 1), 2), (wide(crowded(layer.selection, False), cin, 2), 2)):
+        sig, scratch, padded, got = gradients(sel, -1)
+        assert convlogic_hip.lists_of(sig) & 2 == is_wide
+        for lists in (sig & 3, 0, 1, 2, 3):                           # (any choice is a right one)
+            again = gradients(sel, lists)
+            assert lists != sig & 3 or (again[:3] == (sig, scratch, padded) and all(torch.equal(a, b) for a, b in zip(got, again[3])))
+            for a, b in zip(got, again[3]):
+                assert_grad_close(a, b, rel=1e-4)
+        if is_wide:
+            set_knobs(monkeypatch, CLG_BWDX_PLANES="0")
+            _, scratch0, padded0, want = gradients(sel, -1)
+            set_knobs(monkeypatch, CLG_BWDX_PLANES=None)
+            assert (scratch, padded) == (scratch0, padded0) and all(torch.equal(a, b) for a, b in zip(got, want))
+    # a plan in use whose layer is given such a selection, and one without
+    x.requires_grad_(True)
+    for sel in (layer.selection.clone(), wide(layer.selection, cin, 1), layer.selection.clone()):
+        with torch.no_grad():
+            layer.selection.copy_(sel)
+        y = layer(x)
+        torch.manual_seed(1)
+        got = torch.autograd.grad(y, [x, layer.weights], torch.randn_like(y))
+        (kept,) = layer._plans.values()
+        x.requires_grad_(False)
+        sig, _, _, want = gradients(sel, -1)
+        x.requires_grad_(True)
+        assert kept.plan[1] == sig and all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 def test_a_kept_plan_is_complete():
     # what a first call leaves for calls on other streams: the tables of a block's plan and of a network's trees
     torch.manual_seed(5)
