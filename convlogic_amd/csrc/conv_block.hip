@@ -1713,6 +1713,14 @@ extern "C" int64_t clg_convblock_backward_planned_scratch_bytes(int dtype, const
 {
     return backward_scratch_bytes("clg_convblock_backward_planned_scratch_bytes", dtype, gg, (signature & CLG_LISTS_LONG) != 0, (signature & CLG_LISTS_WIDE) == 0);
 }
+// (no gradient planes: they are the input gradient's)
+extern "C" int64_t clg_convblock_backward_planned_w_scratch_bytes(int dtype, const clg_conv_geom *gg)
+{
+    const char *name = "clg_convblock_backward_planned_w_scratch_bytes";
+    Geom g;
+    if (clg_convblock_check(gg, &g, dtype, name)) return -1;
+    return backward_4x4_wanted(g) ? backward_scratch_bytes(name, dtype, gg, false) : clg_convblock_backward_w_scratch_bytes(dtype, gg);
+}
 
 extern "C" int clg_convblock_backward(int dtype, const clg_conv_geom *gg, const void *grad_y, const void *x, const void *w,
                                       const int32_t *selection, const uint8_t *argmax, void *grad_x, void *grad_w, void *scratch,
@@ -1951,7 +1959,7 @@ static int backward_planned_impl(const char *name, int dtype, const clg_conv_geo
         g.y_fm = fm ? 1 : 0;
         return convblock_backward_4x4(dtype, g, grad_y, x, w, selection, argmax, grad_x, grad_w, scratch, stream, probs, name, &pv);
     }
-    const int64_t a = backward_x_scratch_bytes(name, dtype, gg, long_lists, pi.planes);
+    const int64_t a = grad_x != nullptr ? backward_x_scratch_bytes(name, dtype, gg, long_lists, pi.planes) : 0;
     if (a < 0) return CLG_EINVAL;
     SharedPad shared;
     void *w_scratch = reinterpret_cast<unsigned char *>(scratch) + ((a + 255) & ~255ll);

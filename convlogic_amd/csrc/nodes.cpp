@@ -257,7 +257,8 @@ std::pair<Tensor, Tensor> block_backward(const BlockState &state, const Conv &co
             need(gy, x, "grad_y", s);
         }
         gl = floats(x, {c, 7, 16});
-        const Tensor scratch = bytes(x, clg_convblock_backward_planned_scratch_bytes(CLG_F32, &g, signature));
+        const Tensor scratch = bytes(x, need_x ? clg_convblock_backward_planned_scratch_bytes(CLG_F32, &g, signature)
+                                              : clg_convblock_backward_planned_w_scratch_bytes(CLG_F32, &g));
         const Tensor padded = fm || !need_x ? Tensor() : state.padded;
         const int flags = CLG_BWD_WRT_LOGITS | (fm ? CLG_BWD_GY_FEATURE_MAJOR : 0);
         if (late != nullptr) {

@@ -113,6 +113,7 @@ SIGNATURES = {
     "clg_convblock_plan": (_i, [_i, _GP, _p, _p, _p, _p]),
     "clg_convblock_plan_lists": (_i, [_i, _GP, _p, _p, _i, _p, _p]),
     "clg_convblock_backward_planned_scratch_bytes": (_i64, [_i, _GP, _i64]),
+    "clg_convblock_backward_planned_w_scratch_bytes": (_i64, [_i, _GP]),
     "clg_convblock_backward_planned": (_i, [_i, _GP, _p, _p, _p, _p, _p, _p, _p, _i64, _p, _p, _i, _p, _p]),
     "clg_convblock_backward_planned_padded": (_i, [_i, _GP, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _p, _p, _i, _p, _p]),
     "clg_convblock_bin_supported": (_i, [_i, _GP]),

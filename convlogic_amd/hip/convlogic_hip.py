@@ -453,7 +453,8 @@ def full_convlogic_backward_planned(grad_y, x, weight, folded, argmax, selection
         check_input(plan, "plan", torch.uint8)
         if plan.numel() < lib.clg_convblock_plan_bytes(dt, ctypes.byref(g)):
             raise RuntimeError("plan is smaller than clg_convblock_plan_bytes() for this geometry")
-    scratch = _scratch(lib.clg_convblock_backward_planned_scratch_bytes(dt, ctypes.byref(g), signature), x.device)
+    scratch = _scratch(lib.clg_convblock_backward_planned_scratch_bytes(dt, ctypes.byref(g), signature) if need_grad_x
+                       else lib.clg_convblock_backward_planned_w_scratch_bytes(dt, ctypes.byref(g)), x.device)
     gx = torch.empty_like(x) if need_grad_x else None
     gw = torch.empty((g.c_out, 7, 16), dtype=x.dtype, device=x.device)
     flags = (1 if wrt_logits else 0) | (2 if feature_major else 0)

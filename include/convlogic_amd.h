@@ -485,11 +485,12 @@ int clg_convblock_plan_lists(int dtype, const clg_conv_geom *g, const int32_t *s
                              void *stream);
 /* scratch of the planned calls (clg_convblock_backward_scratch_bytes for a plan of short lists) */
 int64_t clg_convblock_backward_planned_scratch_bytes(int dtype, const clg_conv_geom *g, int64_t signature);
+int64_t clg_convblock_backward_planned_w_scratch_bytes(int dtype, const clg_conv_geom *g);   /* of a call without grad_x */
 #define CLG_BWD_WRT_LOGITS 1       /* w = softmax(logits): grad_w is the gradient w.r.t. the logits */
 #define CLG_BWD_GY_FEATURE_MAJOR 2 /* grad_y laid out [c_out, ho/2, wo/2, n] (shapes of clg_convblock_fm_supported) */
 /* clg_convblock_backward / clg_convblock_backward_logits / clg_convblock_backward_fm (chosen by flags) with a plan: no list building per call, and with folded [c_out, 7, 4] (written by clg_convblock_forward_ex with
  * CLG_FWD_FOLDED_OUT for the same w; may be NULL) no set-up launch is left for blocks whose images fit LDS.  grad_x may
- * be NULL.  scratch: clg_convblock_backward_planned_scratch_bytes().  Same values as the unplanned entry points.
+ * be NULL (scratch is then clg_convblock_backward_planned_w_scratch_bytes(), else clg_convblock_backward_planned_scratch_bytes()).  Same values as the unplanned entry points.
  * Replaces full_convlogic_backward_x + full_convlogic_backward_weight (src/convlogic/convlogic_layer.py:71-82). */
 int clg_convblock_backward_planned(int dtype, const clg_conv_geom *g, const void *grad_y, const void *x, const void *w,
                                    const void *folded, const int32_t *selection, const uint8_t *argmax, void *plan,

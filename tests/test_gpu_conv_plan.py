@@ -217,6 +217,27 @@ def test_taps_in_many_channels_take_the_kernels_without_planes(shape, monkeypatc
         assert kept.plan[1] == sig and all(torch.equal(a, b) for a, b in zip(got, want))
 
 
+@pytest.mark.parametrize("shape", [(256, 8, 32, 16), (300, 16, 128, 12)])
+def test_a_first_block_takes_no_gradient_planes(shape):
+    n, cin, cout, side = shape
+    layer, x = C.ConvLogicLayer(cin, cout, padding=1, complete=True, implementation="cuda").to(DEV), torch.rand(n, cin, side, side, device=DEV)
+    geom, (_, sig) = ctypes.byref(convlogic_hip._geom(x, cout, 1, 1, 1, 1, 3, 3)), layer._backward_plan(x, layer.selection)
+    planes = 2 * cout * x[:, 0].numel() * 4
+    assert _lib.load().clg_convblock_backward_planned_scratch_bytes(0, geom, sig) >= planes
+    y = layer(x)
+    gy = torch.randn_like(y)
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    (got,) = torch.autograd.grad(y, [layer.weights], gy)
+    assert torch.cuda.max_memory_allocated() - before < planes // 2
+    y = layer(x.requires_grad_(True))
+    want = torch.autograd.grad(y, [x, layer.weights], gy)[1]
+    # two orders of the same terms, each at most |grad_y|, that a gradient of a gate adds with coefficients of absolute sum <= 5, the softmax at most
+    # doubling it; 12 roundings make a term, 16 additions a lane's sum, 73 join lanes, wavefronts and parts
+    bound = 2 * 2 * 5 * (12 + 16 + 73) * 2.0**-24 * gy.abs().double().sum((0, 2, 3))
+    assert ((got.double() - want.double()).abs().amax((1, 2)) <= bound).all()
+
+
 def test_a_kept_plan_is_complete():
     # what a first call leaves for calls on other streams: the tables of a block's plan and of a network's trees
     torch.manual_seed(5)
