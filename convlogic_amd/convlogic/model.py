@@ -10,6 +10,7 @@ from torch import nn
 
 from ..difflogic import GroupSum, LogicLayer
 from ..difflogic.difflogic import _feature_major, logic_layer_group_sum
+from ..difflogic import fc_tree
 from ..difflogic.fc_tree import tree_eval, tree_packed, tree_plan, tree_train
 from ..difflogic.packbitstensor import PackBitsTensor
 from ..hip.convlogic_hip import bin_supported
@@ -195,7 +196,7 @@ def _many_small_classes(roots, k, words):
 def _trees_take(h, first):
     """True for what the modules themselves would accept (they raise for anything else), up to the kernels' grid"""
     return (h.dim() == 2 and h.shape[1] == first.in_dim and h.dtype == torch.float32 and h.device == first._parameters["weights"].device
-            and h.shape[0] <= 1 << 20)
+            and h.shape[0] <= fc_tree.MAX_BATCH)
 
 
 def _head_of(net, h):

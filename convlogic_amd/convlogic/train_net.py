@@ -7,6 +7,7 @@ import types
 import torch
 from torch import nn
 
+from ..difflogic import fc_tree
 from ..difflogic.fc_tree import wiring_of
 from ..hip import _lib
 from ..hip._lib import ConvGeom
@@ -37,7 +38,7 @@ def blocks_of(net, called_for_itself, device):
 def train(net, tail, plan, x, called_for_itself):
     """Class sums / tau of a training step, or None where the modules have to be called."""
     layers, group_sum = tail
-    if type(x) is not torch.Tensor or x.dim() != 4 or not x.is_contiguous() or _lib.traced() or layers[0]._parameters["weights"].device != x.device:
+    if type(x) is not torch.Tensor or x.dim() != 4 or x.shape[0] > fc_tree.MAX_BATCH or not x.is_contiguous() or _lib.traced() or layers[0]._parameters["weights"].device != x.device:
         return None
     blocks = blocks_of(net, called_for_itself, x.device)
     if blocks is None or 16 * 7 * (plan.roots + sum(m.out_channels for m in blocks)) > MAX_LOGITS:

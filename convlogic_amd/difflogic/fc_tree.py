@@ -10,6 +10,8 @@ import torch
 from ..hip import _lib
 from ..hip._lib import check, stream_ptr
 
+MAX_BATCH = 1 << 20                                                   # samples of a call, within what the kernels' grids hold
+
 # per first layer: the _Entry of every pair of layers that was seen behind it; kept outside the modules so that copies and pickles
 # carry no derived buffers
 _PLANS = weakref.WeakKeyDictionary()

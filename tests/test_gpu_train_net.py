@@ -132,6 +132,18 @@ def test_what_the_modules_do_for_themselves_stays_theirs(at_once):
     assert True not in at_once
 
 
+def test_a_batch_that_the_trees_do_not_take_is_the_modules(at_once, monkeypatch):
+    model, side = network("mnist", 8, 1)
+    x = (torch.rand(20, 1, side, side, device=DEV) < 0.5).float()
+    want = model(x)
+    monkeypatch.setattr(train_net.fc_tree, "MAX_BATCH", 19)
+    got = model(x)
+    # (the modules' class sums add the rows of a class in another order)
+    assert at_once == [True, False] and (got - want).abs().max() <= 1e-5 * want.abs().max()
+    monkeypatch.setattr(train_net.fc_tree, "MAX_BATCH", 20)
+    assert torch.equal(model(x), want) and at_once[-1]
+
+
 def test_a_broken_promise_of_binary_inputs_is_reported():
     model, side = network("mnist", 8, 1)
     model(torch.rand(4, 1, side, side, device=DEV))
