@@ -1507,17 +1507,20 @@ static bool backward_4x4_wanted(const Geom &g)
 // below 1.05 (lists of 2), 1.1 to 1.5 in between ([256,32,16,16] -> 128 70.7 -> 63.1 us, [16,32,6,6] -> 256 45 -> 25,
 // [64,512,12,12] -> 2048 184 -> 156); 45 shapes of 90 to 420 MB 1.03 to 1.36 times ([71,749,20,20] -> 749 221 -> 167 us, [240,127,20,20] -> 508 323 -> 295,
 // [24,618,18,18] -> 4944 360 -> 337); 26 of 420 to 1100 MB 0.81 to 1.10, the slower ones from 477 on.  Images of 8 and 16 columns, which the kernels
-// below take without a division per position, only up to 70 MB: in the step of a whole network, where the planes' memory is not in the caches
-// any more, CIFAR topology, k = 32 with 256 images, 64 MB per block, 299 -> 272 us, k = 48 with 200, 75 MB, 342 -> 356, k = 100 with
-// 128, 406 -> 421, k = 250 with 200, 391 MB, 1401 -> 1473 (MNIST topology, 12 and 6 columns, k = 256 with 128, 108 MB, 568 -> 549).  Fewer than four channels are
-// the tiled kernel's, whose wavefronts share a channel; lists longer than 16 on the average go by their length (lists_are_long).
+// below take without a division per position, only up to 128 MB.  Replayed step of the CIFAR topology, two such blocks, us without planes and with them, 50
+// networks of k = 24 to 400: 47 to 128 MB per block 0.99 to 1.10 times as fast (k = 32 with 256 images, 64 MB, 293 -> 267; k = 48 with 200, 75 MB, 339 -> 318; k = 100
+// with 128, 100 MB, 408 -> 396), from there on either way, 0.94 to 1.05 (k = 24 with 813, 152 MB, 579 -> 596; k = 380 with 51, 151 MB, 739 -> 728; k = 150 with 150,
+// 176 MB, 712 -> 739; k = 64 with 400, 200 MB, 703 -> 670; k = 250 with 200, 391 MB, 1389 -> 1470): what is left of the planes in the 256 MB of the last-level
+// cache decides, and they are one of several large buffers of a step.  (MNIST topology, 12 and 6 columns, k = 256 with 128, 108 MB, 568 -> 549.)  Fewer than four channels are
+// the tiled kernel's, whose wavefronts share a channel; lists longer than 16 on the average go by their length (lists_are_long), selections with taps in
+// more than two channels of a kernel by taps_are_wide.
 static bool backward_planes_wanted(const Geom &g, int dtype, PairPlan *p)
 {
     if (dtype != CLG_F32 || backward_4x4_wanted(g) || !clg_plan_pair(g, 4, p, false) || !clg_pair_grad_w_wanted(g, *p) || !clg_pair_planes_fit(g, *p))
         return false;
     if (const char *e = clg_knob(K_BWDX_PLANES)) return atoi(e) != 0;
     if (clg_knob(K_BWDX_DIRECT) != nullptr) return false;            // (one of the other kernels is asked for)
-    return g.cin >= 4 && g.c >= g.cin && g.c <= 8 * (int64_t)g.cin && clg_pair_planes_bytes(g) <= (size_t)(g.w == 8 || g.w == 16 ? 70 : 450) << 20;
+    return g.cin >= 4 && g.c >= g.cin && g.c <= 8 * (int64_t)g.cin && clg_pair_planes_bytes(g) <= (size_t)(g.w == 8 || g.w == 16 ? 128 : 450) << 20;
 }
 static size_t backward_planes_off(const Geom &g) { return (bwd_scratch_layout(g, 4, 1).total + 255) & ~(size_t)255; }
 
