@@ -170,7 +170,7 @@ def _pair(v):
 
 
 def _same_buffer(of, buffer):
-    """True when `of` = (buffer, version) is of this buffer as it is now.  The buffer itself is compared (and so held): another
+    """True when `of` = (buffer, version, ...) is of this buffer as it is now.  The buffer itself is compared (and so held): another
     one may have its address and version, for instance after a move to another device and back."""
     return of is not None and of[0] is buffer and of[1] == buffer._version
 
@@ -188,11 +188,11 @@ class _KeptPlan:
     def make(self, like, sel, layer):
         """In place where there are tables already, and for the same kernels: a recorded step reads them at their addresses.  (Tables that no
         recording reads: made anew where a kernel has taps in more than two channels now, or has none any more.)"""
-        tables, lists = (None, convlogic_hip.LISTS_LOOK) if self.plan is None else (self.plan[0], convlogic_hip.lists_of(self.plan[1]))
-        if self.plan is not None and not self.recorded:
-            wide = convlogic_hip.LISTS_WIDE if convlogic_hip.taps_are_wide(sel, layer.in_channels) else 0
-            if (lists & convlogic_hip.LISTS_WIDE) != wide:
-                tables, lists = None, convlogic_hip.LISTS_LOOK
+        wide = layer.taps_are_wide()
+        look = convlogic_hip.LISTS_LOOK_NARROW if wide is False else convlogic_hip.LISTS_LOOK
+        tables, lists = (None, look) if self.plan is None else (self.plan[0], convlogic_hip.lists_of(self.plan[1]))
+        if self.plan is not None and not self.recorded and wide != bool(lists & convlogic_hip.LISTS_WIDE):
+            tables, lists = None, look
         self.plan = convlogic_hip.make_backward_plan(like, layer.out_channels, sel, *layer.stride, *layer.padding, *layer.kernel, into=tables,
                                                      lists=lists)
 
@@ -245,11 +245,20 @@ class ConvLogicLayer(nn.Module):
             return
         if sel.dtype != torch.int32 or tuple(sel.shape) != (self.out_channels, 8):
             raise ValueError(f"selection must be int32 [{self.out_channels}, 8], got {sel.dtype} {tuple(sel.shape)}")
-        ch, row, col = self.unpack_selection(sel)
-        if sel.numel() and (int(ch.max()) >= self.in_channels or int(row.max()) >= self.kernel[0] or int(col.max()) >= self.kernel[1]):
+        if sel.is_cuda and self.out_channels <= 4096:                # (one copy to the host: one wait for the device; large ones take longer to copy)
+            inside, wide = convlogic_hip.look_at_selection(sel.cpu().contiguous(), self.in_channels, *self.kernel)
+        else:
+            (ch, row, col), wide = self.unpack_selection(sel), None
+            inside = not sel.numel() or (int(ch.max()) < self.in_channels and int(row.max()) < self.kernel[0] and int(col.max()) < self.kernel[1])
+        if not inside:
             raise ValueError(f"selection names a tap outside {self.in_channels} input channels and a "
                              f"{self.kernel[0]}x{self.kernel[1]} receptive field")
-        self._selection_checked = (sel, sel._version)
+        self._selection_checked = (sel, sel._version, wide)
+
+    def taps_are_wide(self):
+        """Whether the taps of some kernel are in more than two channels, or None where nobody looked."""
+        self._check_selection()
+        return self._selection_checked[2]
 
     def invalidate(self):
         """Forces the next call to check the selection buffer again and to make the backward plans again (after a write

@@ -1858,12 +1858,12 @@ std::unique_ptr<int32_t[]> host_copy(const void *from, size_t count, hipStream_t
 // one element by element for each of its channels: forward and backward of [256,128,8,8] -> 512, us by the other kernels and with planes, no such
 // kernel 67 and 60, 2 % of them 75 and 86, all 207 and 713; [64,512,12,12] -> 2048 176 and 145, 184 and 194, 454 and 2062; [16,32,6,6] -> 256 41 and 21, 43 and
 // 42, 66 and 481.  (A channel that many kernels read is no reason: all kernels on one channel 479 and 100, 1993 and 337, 211 and 41.)
-bool taps_are_wide(const Geom &g, const int32_t *selection)
+bool taps_are_wide(const int32_t *selection, int64_t kernels, int cin)
 {
-    for (int64_t c = 0; c < g.c; ++c) {
+    for (int64_t c = 0; c < kernels; ++c) {
         int ch[2] = {-1, -1};
         for (int t = 0; t < 8; ++t) {
-            const int at = std::min((selection[c * 8 + t] >> 16) & 0xFFFF, g.cin - 1);
+            const int at = std::min((selection[c * 8 + t] >> 16) & 0xFFFF, cin - 1);
             if (ch[0] < 0 || at == ch[0]) ch[0] = at;
             else if (ch[1] < 0 || at == ch[1]) ch[1] = at;
             else return true;
@@ -1872,6 +1872,16 @@ bool taps_are_wide(const Geom &g, const int32_t *selection)
     return false;
 }
 }  // namespace
+
+extern "C" int clg_selection_look(const int32_t *selection, int64_t c_out, int c_in, int kernel_h, int kernel_w)
+{
+    bool outside = false;
+    for (int64_t i = 0; i < c_out * 8; ++i) {
+        const int32_t s = selection[i];
+        outside |= ((s >> 16) & 0xFFFF) >= c_in || ((s >> 8) & 0xFF) >= kernel_h || (s & 0xFF) >= kernel_w;
+    }
+    return (outside ? 1 : 0) | (taps_are_wide(selection, c_out, c_in) ? 2 : 0);
+}
 
 extern "C" int64_t clg_convblock_plan_bytes(int dtype, const clg_conv_geom *gg)
 {
@@ -1894,17 +1904,18 @@ extern "C" int clg_convblock_plan_lists(int dtype, const clg_conv_geom *gg, cons
     Geom g;
     if (int e = clg_convblock_check(gg, &g, dtype, name)) return e;
     CLG_REQUIRE(selection && plan && signature, "%s: null pointer argument", name);
-    CLG_REQUIRE(lists >= CLG_LISTS_LOOK && lists <= (CLG_LISTS_LONG | CLG_LISTS_WIDE), "%s: lists must be a CLG_LISTS_ value, got %d", name, lists);
+    CLG_REQUIRE(lists >= CLG_LISTS_LOOK_NARROW && lists <= (CLG_LISTS_LONG | CLG_LISTS_WIDE), "%s: lists must be a CLG_LISTS_ value, got %d", name, lists);
     hipStream_t st = clg_stream(stream);
-    const PlanInfo pi = plan_info(g, dtype, lists == CLG_LISTS_LOOK ? CLG_LISTS_SHORT : lists);
+    const PlanInfo pi = plan_info(g, dtype, std::max(lists, CLG_LISTS_SHORT));
     if (int e = make_plan(g, dtype, pi, selection, plan, st)) return e;
     *signature = pi.signature;
-    if (lists != CLG_LISTS_LOOK) return CLG_OK;
+    if (lists >= CLG_LISTS_SHORT) return CLG_OK;
     int found = CLG_LISTS_SHORT;
     if (pi.planes) {
+        if (lists == CLG_LISTS_LOOK_NARROW) return CLG_OK;
         const auto taps = host_copy(selection, (size_t)g.c * 8, st, name);
         if (taps == nullptr) return CLG_EINVAL;
-        if (!taps_are_wide(g, taps.get())) return CLG_OK;
+        if (!taps_are_wide(taps.get(), g.c, g.cin)) return CLG_OK;
         found = CLG_LISTS_WIDE;
     }
     if (plan_info(g, dtype, found | CLG_LISTS_LONG).signature != plan_info(g, dtype, found).signature) {

@@ -129,6 +129,7 @@ SIGNATURES = {
     "clg_fc_tree_backward": (_i, [_p] * 14 + [_i64, _i64, _i64, _i64, _i64, _f64, _p]),
     "clg_fc_tree_packed": (_i, [_p] * 8 + [_i64, _i64, _i64, _i64, _i64, _p]),
     "clg_train_prepare": (_i, [_p, _i] + [_p] * 6 + [_i64, _p]),
+    "clg_selection_look": (_i, [_p, _i64, _i, _i, _i]),
     "clg_convblock_late_sums_bytes": (_i64, [_i, _GP]),
     "clg_convblock_backward_planned_late": (_i, [_i, _GP] + [_p] * 8 + [_i64, _p, _p, _i, _p, _p, _p, _p]),
     "clg_convblock_bin_backward_late": (_i, [_i, _GP, _p, _p, _p, _p, _p, _i, _p, _p, _p]),

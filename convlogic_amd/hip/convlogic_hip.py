@@ -390,7 +390,13 @@ def full_convlogic_forward_logits(x, logits, selection, stride_h, stride_w, pad_
     return y, argmax, probs
 
 
-LISTS_LOOK, LISTS_SHORT, LISTS_LONG, LISTS_WIDE = -1, 0, 1, 2         # CLG_LISTS_* (include/convlogic_amd.h)
+LISTS_LOOK_NARROW, LISTS_LOOK, LISTS_SHORT, LISTS_LONG, LISTS_WIDE = -2, -1, 0, 1, 2      # CLG_LISTS_* (include/convlogic_amd.h)
+
+
+def look_at_selection(selection, channels, kernel_h, kernel_w):
+    """-> (whether every tap of a selection in host memory is inside the layer's ranges, whether some kernel's taps are in more than two channels)"""
+    found = _lib.load().clg_selection_look(selection.data_ptr(), selection.shape[0], channels, kernel_h, kernel_w)
+    return not found & 1, bool(found & 2)
 
 
 def make_backward_plan(x, c_out, selection, stride_h, stride_w, pad_h, pad_w, kernel_h, kernel_w, into=None, lists=LISTS_SHORT):
@@ -398,8 +404,8 @@ def make_backward_plan(x, c_out, selection, stride_h, stride_w, pad_h, pad_w, ke
     signature).  Depends only on the selection and the geometry; built once and reused by every
     full_convlogic_backward_planned() call of the layer (the reverse map the reference's LogicLayer builds at
     construction, src/difflogic/difflogic.py:71-87, for the fused block).  Of x only shape, dtype and device are looked at.
-    into: the bytes of an earlier plan for the same geometry, which are written again.  lists: LISTS_SHORT, LISTS_LOOK (waits for the
-    stream) or lists_of() an earlier plan."""
+    into: the bytes of an earlier plan for the same geometry, which are written again.  lists: LISTS_SHORT, LISTS_LOOK or
+    LISTS_LOOK_NARROW (may wait for the stream) or lists_of() an earlier plan."""
     if isinstance(x, torch.Tensor):
         check_input(x, "x")
     if len(x.shape) != 4:
@@ -419,12 +425,6 @@ def lists_of(signature):
     """What a plan's kernels were chosen for: LISTS_SHORT, or of LISTS_LONG for a channel that many kernels read (they take no padded copy of x) and
     LISTS_WIDE for kernels with taps in more than two channels."""
     return signature & (LISTS_LONG | LISTS_WIDE)
-
-
-def taps_are_wide(selection, channels):
-    """Whether the taps of some kernel are in more than two channels (waits for the device)."""
-    ch = ((selection >> 16) & 0xFFFF).clamp(max=channels - 1).sort(1).values
-    return bool(((ch[:, 1:] != ch[:, :-1]).sum(1) > 1).any())
 
 
 def full_convlogic_backward_planned(grad_y, x, weight, folded, argmax, selection, plan, signature, stride_h, stride_w, pad_h, pad_w,

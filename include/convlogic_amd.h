@@ -475,12 +475,15 @@ int clg_convblock_plan(int dtype, const clg_conv_geom *g, const int32_t *selecti
  * CLG_LISTS_LONG: so many kernels read one channel that the kernels for short lists, where a list is one wavefront's work,
  * are the slower ones.  CLG_LISTS_WIDE (alone or with CLG_LISTS_LONG): the taps of some kernel are in more than two channels, which the kernels that
  * keep a plane for each of a kernel's two channels evaluate one by one.  CLG_LISTS_LOOK: looks at the lists and chooses (waits for the stream; not
- * inside a recording).  The choice is the lowest two bits of the signature; plans made again in the memory of one that is in use must be given it as
+ * inside a recording), CLG_LISTS_LOOK_NARROW: the same for a selection known to have no such kernel.  The choice is the lowest two bits of the signature; plans made again in the memory of one that is in use must be given it as
  * `lists`. */
+#define CLG_LISTS_LOOK_NARROW -2
 #define CLG_LISTS_LOOK -1
 #define CLG_LISTS_SHORT 0
 #define CLG_LISTS_LONG 1
 #define CLG_LISTS_WIDE 2
+int clg_selection_look(const int32_t *selection, int64_t c_out, int c_in, int kernel_h, int kernel_w);   /* of a selection in host memory: 1 (some tap is
+                                                               outside the ranges) | 2 (some kernel's taps are in more than two channels) */
 int clg_convblock_plan_lists(int dtype, const clg_conv_geom *g, const int32_t *selection, void *plan, int lists, int64_t *signature,
                              void *stream);
 /* scratch of the planned calls (clg_convblock_backward_scratch_bytes for a plan of short lists) */
