@@ -180,10 +180,18 @@ struct Prepared {
 // 100, 1024 images: 3.07 GB, 1.88 like this and by the modules).
 struct Late {
     std::vector<clg_late_sums> sums;
-    std::vector<Tensor> kept;
-    clg_late_sums *next(const Tensor &parts)
+    Tensor parts, histogram;                                          // (of a binary block: the only one's scratch)
+    int64_t used = 0, block = 0;                                      // block: bytes of the parts of the block at hand
+    static int64_t aligned(int64_t n) { return (n + 255) & ~(int64_t)255; }
+    void *take(int64_t n)                                             // of parts, which hold as much as all layers take
     {
-        kept.push_back(parts);
+        TORCH_CHECK(used + n <= parts.numel(), "late sums: more parts than room");
+        void *at = static_cast<char *>(parts.data_ptr()) + used;
+        used += aligned(n);
+        return at;
+    }
+    clg_late_sums *next()
+    {
         sums.push_back({});
         return &sums.back();
     }
@@ -261,12 +269,10 @@ std::pair<Tensor, Tensor> block_backward(const BlockState &state, const Conv &co
                                               : clg_convblock_backward_planned_w_scratch_bytes(CLG_F32, &g));
         const Tensor padded = fm || !need_x ? Tensor() : state.padded;
         const int flags = CLG_BWD_WRT_LOGITS | (fm ? CLG_BWD_GY_FEATURE_MAJOR : 0);
-        if (late != nullptr) {
-            const Tensor parts = bytes(x, clg_convblock_late_sums_bytes(CLG_F32, &g));
+        if (late != nullptr)
             check(clg_convblock_backward_planned_late(CLG_F32, &g, gy.data_ptr(), x.data_ptr(), probs.data_ptr(), folded, ptr(padded), selection, codes,
-                                                      plan.data_ptr(), signature, ptr(gx), gl.data_ptr(), flags, scratch.data_ptr(), parts.data_ptr(),
-                                                      late->next(parts), stream_of(x)));
-        }
+                                                      plan.data_ptr(), signature, ptr(gx), gl.data_ptr(), flags, scratch.data_ptr(),
+                                                      late->take(late->block), late->next(), stream_of(x)));
         else if (padded.defined())
             check(clg_convblock_backward_planned_padded(CLG_F32, &g, gy.data_ptr(), x.data_ptr(), probs.data_ptr(), folded, padded.data_ptr(),
                                                         selection, codes, plan.data_ptr(), signature, gx.data_ptr(), gl.data_ptr(), flags,
@@ -346,10 +352,11 @@ std::pair<Tensor, Tensor> binary_backward(const Tensor &taps, const Tensor &keep
         gl = floats(gy, {c, 7, 16});
         scratch = bytes(gy, clg_convblock_bin_backward_scratch_bytes(CLG_F32, &g));
     }
-    if (need_l && late != nullptr)
+    if (need_l && late != nullptr) {
+        late->histogram = scratch;
         check(clg_convblock_bin_backward_late(CLG_F32, &g, gy.data_ptr(), static_cast<const uint16_t *>(taps.data_ptr()), keep.data_ptr(), ptr(gx), ptr(gl),
-                                              CLG_BWD_WRT_LOGITS, ptr(scratch), late->next(scratch), stream_of(gy)));
-    else if (need_x || need_l)
+                                              CLG_BWD_WRT_LOGITS, ptr(scratch), late->next(), stream_of(gy)));
+    } else if (need_x || need_l)
         check(clg_convblock_bin_backward(CLG_F32, &g, gy.data_ptr(), static_cast<const uint16_t *>(taps.data_ptr()), keep.data_ptr(), ptr(gx), ptr(gl),
                                          CLG_BWD_WRT_LOGITS, ptr(scratch), stream_of(gy)));
     return {gx, gl};
@@ -418,11 +425,11 @@ std::array<Tensor, 4> trees_backward(const Tensor &x, const Tensor &start, const
     for (int i = 0; i < 3; ++i)
         if (wanted[1 + i]) g[1 + i] = floats(x, {neurons[i], 16});
     const int64_t rows = g[0].defined() ? 8 * roots * batch : 0;
-    const Tensor scratch = floats(x, {rows + (late ? 0 : 28 * roots)}), kept = late ? floats(x, {28 * roots}) : Tensor();   // operand gradients, sums
-    float *sums = late ? f32(kept) : f32(scratch) + rows;
+    const Tensor scratch = floats(x, {rows + (late ? 0 : 28 * roots)});   // operand gradients, then sums
+    float *sums = late ? static_cast<float *>(late->take(112 * roots)) : f32(scratch) + rows;
     if (late != nullptr)
         check(clg_fc_tree_backward_late(f32(x), i32(tables[0]), i32(tables[1]), i32(tables[2]), f32(coef), f32(go), f32(probs), f32(g[1]), f32(g[2]),
-                                        f32(g[3]), f32(scratch), sums, idx(start), f32(g[0]), in_dim, roots, k, batch, batch, tau, late->next(kept),
+                                        f32(g[3]), f32(scratch), sums, idx(start), f32(g[0]), in_dim, roots, k, batch, batch, tau, late->next(),
                                         stream_of(x)));
     else
         check(clg_fc_tree_backward(f32(x), i32(tables[0]), i32(tables[1]), i32(tables[2]), f32(coef), f32(go), f32(probs), f32(g[1]), f32(g[2]), f32(g[3]),
@@ -562,6 +569,17 @@ struct Network : torch::autograd::Function<Network> {
         variable_list out(1 + n + 3 + 1);
         const Tensor *t = saved.data() + n * kEach;
         Late sums, *late = n <= kTogether ? &sums : nullptr;
+        std::vector<int64_t> parts_of(n);
+        if (late != nullptr) {
+            int64_t parts = Late::aligned(112 * t[2].size(0));
+            for (size_t i = 0; i < n; ++i) {
+                const int64_t *own = ints.data() + i * kInts;
+                if (own[10] != 0 || !wanted(1 + i)) continue;
+                const clg_conv_geom geom = Conv{own[0], own[1], own[2], own[3], own[4], own[5]}.geom(at::IntArrayRef(own + 6, 4), saved[i * kEach + 2].size(0));
+                parts += Late::aligned(parts_of[i] = clg_convblock_late_sums_bytes(CLG_F32, &geom));
+            }
+            sums.parts = bytes(t[0], parts);
+        }
         auto g = trees_backward(t[0], t[1], t[2], t[3], ctx->saved_data["tables"].toTensorVector(), ctx->saved_data["k"].toInt(),
                                 ctx->saved_data["tau"].toDouble(), grads[0], {below[n], wanted(1 + n), wanted(2 + n), wanted(3 + n)}, late);
         for (size_t i = 0; i < 3; ++i) out[1 + n + i] = g[1 + i];
@@ -576,6 +594,7 @@ struct Network : torch::autograd::Function<Network> {
                                        (int32_t)own[0], (int32_t)own[1], (int32_t)own[2], (int32_t)own[3], (int32_t)own[4], (int32_t)own[5]});
                 h = fm ? h.view({s[1], s[2], s[3], s[0]}).permute({3, 0, 1, 2}) : transposed(h).view(s);
             }
+            sums.block = parts_of[i];
             const auto gi = binary ? binary_backward(kept[0], kept[1], conv, at::IntArrayRef(own + 6, 4), h, below[i], wanted(1 + i), late)
                                    : block_backward(BlockState::from(kept), conv, fm, plans[i], own[11], h, below[i], wanted(1 + i), late);
             h = gi.first;
