@@ -34,7 +34,7 @@ __device__ __forceinline__ int argmax16_uniform(float v)
 // the chunk as the slow index, so that all neurons of one column chunk run back to back and the
 // second read of an input row segment finds it in the last-level cache.
 // LOGITS: `gate` points to float32 logits [out_dim, 16] and the wavefront takes their arg-max itself, else to uint8 gate ids.
-// Long rows of whole 16-byte vectors come here where there is no walk of the wiring, and rows below 16 bytes; the rest: eval_packed_rows_kernel.
+// Rows of whole 16-byte vectors from 1 MiB on come here where there is no walk of the wiring, and rows below 16 bytes; the rest: eval_packed_rows_kernel.
 template <typename V, int UNROLL, bool LOGITS>
 __global__ __launch_bounds__(kEvalBlock) void eval_packed_kernel(const V *__restrict__ x, const int64_t *__restrict__ a,
                                                                const int64_t *__restrict__ b,
@@ -82,7 +82,7 @@ __global__ __launch_bounds__(kEvalBlock) void eval_packed_kernel(const V *__rest
 // piece nor one round of loads after the other are paid for; four lanes per neuron find its gate meanwhile.  Rows of any number of bytes from 16 on: the
 // last piece of a row steps back to its last 16 bytes, some of which two lanes write then (the same values).  us per layer, a wavefront per neuron or a walk
 // -> here: 64000 neurons on rows of 64 bytes 15.7 -> 4.1, of 252 18.3 -> 9.6, 8000 on 1280 7.7 -> 4.4; one piece of a thread at a time instead of two
-// costs up to 10 %, stores that stay in the caches up to 25 (64000 on 8188: 250 us, 218).
+// costs up to 10 %, stores that stay in the caches up to 25 (64000 on 8188: 250 us, 219).
 // A row of more pieces than a workgroup has in flight is cut into parts of `per` pieces, a workgroup each: few neurons on long rows fill the chip too
 // (in one workgroup each 64 on 400 KiB took 60 us, here 12.4, 1 on 4 MiB 530, 3.5, 100 on 64 KiB 8.6, 4.0).  The parts are the slow index of the launch: the neurons of one part run back to
 // back and find the second use of an input row's piece in the caches.
@@ -748,7 +748,7 @@ bool valid_elem(int e) { return e == 1 || e == 2 || e == 4 || e == 8; }
 
 }  // namespace
 
-// LOGITS: `gate` holds float32 logits; rows must then be whole 4-byte words at 4-byte aligned addresses
+// LOGITS: `gate` holds float32 logits; rows below 16 bytes, and from 2^34 on, must then be whole 4-byte words at 4-byte aligned addresses
 template <bool LOGITS>
 static int eval_packed(const char *name, int elem_size, const void *x, const int64_t *a, const int64_t *b, const void *gate, void *y,
                        int64_t in_dim, int64_t out_dim, int64_t words, void *stream)
@@ -763,8 +763,9 @@ static int eval_packed(const char *name, int elem_size, const void *x, const int
     hipStream_t st = clg_stream(stream);
     const int64_t blocks_needed = clg_ceil_div(row_bytes, 2048) * clg_ceil_div(out_dim, 16);
     CLG_REQUIRE(blocks_needed < (1ll << 31), "%s: problem too large for one launch (%lld blocks)", name, (long long)blocks_needed);
-    // without a plan, long rows of whole vectors go a wavefront per neuron and 4 KiB ([64000] x 8192: 196 us, 212 by pieces)
-    const bool whole = (align & 15) == 0 && row_bytes >= 1024 && walk_pays(row_bytes, out_dim);
+    // without a plan, rows of whole vectors go a wavefront per neuron and 4 KiB from 1 MiB on ([10] x 2 MiB 8.4 us, 11.4 by pieces, [10] x 16 MiB 57.7 and 62.4, [100] x
+    // 4 MiB 165 and 172, [50] x 4 MiB 84.7 and 84.6; shorter ones [64000] x 8192 214.8 and 213.1, [500] x 64 KiB 16.1 and 15.1)
+    const bool whole = (align & 15) == 0 && row_bytes >= 1 << 20;
     if (row_bytes >= 16 && row_bytes < (1ll << 34) && !whole) launch_rows<LOGITS>(x, a, b, gate, y, out_dim, row_bytes, st, in_dim);
     else if ((align & 15) == 0) launch_eval<u32x4, LOGITS>(x, a, b, gate, y, out_dim, row_bytes, st, in_dim);
     else if ((align & 3) == 0) launch_eval<uint32_t, LOGITS>(x, a, b, gate, y, out_dim, row_bytes, st, in_dim);
@@ -992,8 +993,8 @@ extern "C" int clg_fc_eval_plan(const int64_t *a, const int64_t *b, int64_t in_d
 }
 
 namespace {
-// rows the walk kernel takes: whole 16-byte vectors at 16-byte aligned addresses, at least 1 KiB long (shorter rows gain
-// nothing from carrying a row in registers)
+// rows that clg_fc_eval_packed_planned_logits promises to take: whole 16-byte vectors at 16-byte aligned addresses, at least 1 KiB long.  (The
+// kernels behind it take any; clg_fc_eval_packed_layer lets them.)
 bool walk_fits(int elem_size, const void *x, const void *y, int64_t words)
 {
     const int64_t row_bytes = words * elem_size;
@@ -1048,33 +1049,32 @@ extern "C" int clg_fc_eval_walk_fits(int elem_size, const void *x, const void *y
     return valid_elem(elem_size) && x && y && words > 0 && walk_fits(elem_size, x, y, words) ? 1 : 0;
 }
 
-extern "C" int clg_fc_eval_packed_planned_logits(int elem_size, const void *x, const int64_t *a, const int64_t *b, const float *logits,
-                                                 const int32_t *plan, void *y, int64_t in_dim, int64_t out_dim, int64_t words,
-                                                 void *stream)
+static int eval_packed_layer(const char *name, int elem_size, const void *x, const int64_t *a, const int64_t *b, const float *logits, const int32_t *plan,
+                             void *y, int64_t in_dim, int64_t out_dim, int64_t words, void *stream, bool whole_vectors)
 {
-    const char *name = "clg_fc_eval_packed_planned_logits";
     CLG_REQUIRE(valid_elem(elem_size), "%s: elem_size must be 1, 2, 4 or 8, got %d", name, elem_size);
     CLG_REQUIRE(x && a && b && logits && plan && y, "%s: null pointer argument", name);
     CLG_REQUIRE(x != y, "%s: x and y must not overlap", name);
     CLG_REQUIRE(in_dim > 0 && out_dim > 0 && words > 0, "%s: in_dim, out_dim and words must be positive", name);
     CLG_REQUIRE(out_dim < (1ll << 28), "%s: out_dim above 2^28-1 is not supported", name);
-    CLG_REQUIRE(walk_fits(elem_size, x, y, words), "%s: rows must be whole 16-byte vectors of at least 1 KiB at 16-byte aligned addresses "
+    CLG_REQUIRE(!whole_vectors || walk_fits(elem_size, x, y, words), "%s: rows must be whole 16-byte vectors of at least 1 KiB at 16-byte aligned addresses "
                 "(clg_fc_eval_walk_fits); use clg_gate_argmax + clg_fc_eval_packed_planned otherwise", name);
-    return launch_walk<true>(name, elem_size, x, a, b, logits, plan, y, in_dim, out_dim, words, stream);
-}
-
-extern "C" int clg_fc_eval_packed_layer(int elem_size, const void *x, const int64_t *a, const int64_t *b, const float *logits, const int32_t *plan, void *y,
-                                        int64_t in_dim, int64_t out_dim, int64_t words, void *stream)
-{
-    const char *name = "clg_fc_eval_packed_layer";
-    CLG_REQUIRE(valid_elem(elem_size), "%s: elem_size must be 1, 2, 4 or 8, got %d", name, elem_size);
-    CLG_REQUIRE(x && a && b && logits && plan && y, "%s: null pointer argument", name);
-    CLG_REQUIRE(x != y, "%s: x and y must not overlap", name);
-    CLG_REQUIRE(in_dim > 0 && out_dim > 0 && words > 0, "%s: in_dim, out_dim and words must be positive", name);
-    CLG_REQUIRE(out_dim < (1ll << 28), "%s: out_dim above 2^28-1 is not supported", name);
     const int64_t row_bytes = words * elem_size;
     CLG_REQUIRE(row_bytes >= 16 || (((uintptr_t)x | (uintptr_t)y | (uintptr_t)row_bytes) & 3) == 0, "%s: rows must be 16 bytes or more, or whole 4-byte words at "
                 "4-byte aligned addresses; use clg_gate_argmax + clg_fc_eval_packed otherwise", name);
     if (walk_takes(row_bytes, out_dim)) return launch_walk<true>(name, elem_size, x, a, b, logits, plan, y, in_dim, out_dim, words, stream);
     return eval_packed<true>(name, elem_size, x, a, b, logits, y, in_dim, out_dim, words, stream);
+}
+
+extern "C" int clg_fc_eval_packed_planned_logits(int elem_size, const void *x, const int64_t *a, const int64_t *b, const float *logits,
+                                                 const int32_t *plan, void *y, int64_t in_dim, int64_t out_dim, int64_t words,
+                                                 void *stream)
+{
+    return eval_packed_layer("clg_fc_eval_packed_planned_logits", elem_size, x, a, b, logits, plan, y, in_dim, out_dim, words, stream, true);
+}
+
+extern "C" int clg_fc_eval_packed_layer(int elem_size, const void *x, const int64_t *a, const int64_t *b, const float *logits, const int32_t *plan, void *y,
+                                        int64_t in_dim, int64_t out_dim, int64_t words, void *stream)
+{
+    return eval_packed_layer("clg_fc_eval_packed_layer", elem_size, x, a, b, logits, plan, y, in_dim, out_dim, words, stream, false);
 }

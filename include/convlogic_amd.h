@@ -269,8 +269,8 @@ int clg_fc_eval_packed_planned(int elem_size, const void *x /*[in_dim,words]*/, 
 
 /* clg_gate_argmax + clg_fc_eval_packed_planned in ONE launch: the kernel takes the arg-max of the 16 float32 logits of a
  * neuron itself (first maximum, a NaN counts as the maximum: the same gate ids, tested), so a packed layer call is a
- * single launch.  Needs rows the walk kernel takes -- clg_fc_eval_walk_fits(): whole 16-byte vectors, at least 1 KiB, x
- * and y 16-byte aligned -- and is rejected with CLG_EINVAL otherwise (use the two calls then).
+ * single launch.  For rows for which clg_fc_eval_walk_fits() holds -- whole 16-byte vectors, at least 1 KiB, x and y 16-byte aligned --, rejected
+ * with CLG_EINVAL otherwise; clg_fc_eval_packed_layer() is the same for other rows as well.
  * Replaces `self.weights.argmax(-1).to(torch.uint8)` + difflogic_cuda.eval of LogicLayer.forward_cuda_eval
  * (src/difflogic/difflogic.py:149-164; src/difflogic/cuda/difflogic_kernel.cu:295-330). */
 int clg_fc_eval_walk_fits(int elem_size, const void *x, const void *y, int64_t words);
@@ -282,7 +282,7 @@ int clg_fc_eval_packed_planned_logits(int elem_size, const void *x /*[in_dim,wor
 int clg_fc_eval_packed_layer(int elem_size, const void *x, const int64_t *a, const int64_t *b, const float *logits, const int32_t *plan,
                              void *y, int64_t in_dim, int64_t out_dim, int64_t words, void *stream);
 
-/* clg_gate_argmax + clg_fc_eval_packed in ONE launch, for rows the walk kernel does not take: the same gate ids from the 16
+/* clg_gate_argmax + clg_fc_eval_packed in ONE launch, without a plan: the same gate ids from the 16
  * float32 logits of a neuron.  Rows must be whole 4-byte words at 4-byte aligned addresses (CLG_EINVAL otherwise; use the
  * two calls then).  Replaces the same lines of LogicLayer.forward_cuda_eval as clg_fc_eval_packed_planned_logits. */
 int clg_fc_eval_packed_logits(int elem_size, const void *x /*[in_dim,words]*/, const int64_t *a, const int64_t *b,
