@@ -624,9 +624,6 @@ def bench_c5(steps, warmup, cpu=True):
 
     def leaves():
         m2 = copy.deepcopy(model)
-        # a step replayed from a graph has no host cost, so the network folds all its layers' logits in one launch (the
-        # model's option for that; by default only networks whose eager step the GPU bounds do)
-        m2.prefold = "always"
         return [m2] + [p for p in m2.parameters()]
 
     def run(lv):
@@ -646,8 +643,7 @@ def bench_c5(steps, warmup, cpu=True):
     out = {"workload": f"C5: ConvLogicCifarModel k={k}, 9 input channels, batch {n}, float32 training step (fwd + CE loss + bwd)",
            "metric": "convlogic_fwd_bwd_Ggate_evals_per_s", "value": ge / sec / 1e9, "unit": "Ggate-evals/s", "ms_per_step": sec * 1e3,
            "dtype": "f32", "ms_per_step_hip_graph": graph_ms, "value_hip_graph": (ge / (graph_ms * 1e-3) / 1e9) if graph_ms else None,
-           "hip_graph_note": "the graphed step runs the model with prefold = 'always' (one launch folds the logits of all layers); "
-                             "the eager step runs the model's defaults",
+           "hip_graph_note": "both steps run the model's defaults",
            "roofline": _roof("whole training step (all kernels)", alg, graph_ms if graph_ms else sec * 1e3, _traffic_fields("c5", "step_bytes"))}
 
     # packed inference of the same network: thresholds + packing fused, 65536 samples

@@ -49,9 +49,11 @@ def _prefold(owner, layers, x, mode=True):
         _FOLD_PLANS[owner] = ((x.dtype, x.device, len(layers)), picked, plan)
     if plan is None:
         return
-    # An eager step of a small network is bound by the host, where the bookkeeping of this launch costs more than the
-    # layers' own allocations save (C5: +15 us per step): by default only networks whose step the GPU bounds fold ahead;
-    # prefold = "always" is for small networks whose step is replayed from a HIP graph (C5: 0.385 -> 0.379 ms).
+    # An eager step of a small network whose modules are called is bound by the host, where the bookkeeping of this launch costs more than
+    # the layers' own allocations save (+15 us per step): by default only networks whose step the GPU bounds fold ahead.  "always" is for smaller
+    # ones that are replayed from a HIP graph and cannot run as one node (train_net.py), which by default sets all layers up in one launch and is
+    # the faster way: replayed step of the k = 32 CIFAR network with 256 images 267 us as one node, 291 with "always", 292 without; MNIST, 100
+    # images, 140, 163 and 161.
     if mode != "always" and plan.total < _PREFOLD_MIN_ELEMS:
         return
     for m, (probs, folded) in zip(picked, difflogic_hip.fold_many([w.detach() for w in weights], plan)):
@@ -90,8 +92,8 @@ def _tree_tail(net):
 def _forward(owner, x):
     """The network on x.  Three things happen that a plain nn.Sequential call would not do: the three LogicLayers and the
     GroupSum at its end are evaluated as one operation where their wiring allows (`tree_tail`, default on; training steps,
-    evaluation and packed inference), in training of a small network the blocks in front of them as well; else the logits of the other
-    layers are folded in one launch where that pays (`prefold`), and a last LogicLayer and GroupSum that do not run as trees run as one autograd node (`fused_tail`, default on), whose
+    evaluation and packed inference), in training of a small network the blocks in front of them as well (unless `prefold` is set); else the
+    logits of the other layers are folded in one launch where that pays (`prefold`), and a last LogicLayer and GroupSum that do not run as trees run as one autograd node (`fused_tail`, default on), whose
     backward needs no GroupSum launch."""
     net = owner.network
     tail = _tree_tail(net) if owner.__dict__.get("tree_tail", True) else None

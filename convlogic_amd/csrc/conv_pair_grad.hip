@@ -207,7 +207,8 @@ __global__ __launch_bounds__(kPairWaves *kWave) void convblock_backward_w_pair_k
 }
 
 // gx = the sum of a channel's gradient planes, in the order of the kernels: four consecutive elements per thread, `parts` workgroups per channel.
-// A kernel that wrote none (its list entry says so) is evaluated here, element by element.
+// A kernel that wrote none (its list entry says so) is evaluated here, element by element: slow (taps_are_wide in conv_block.hip), and so only
+// in plans that were made, or are read, by a recording.
 template <bool STREAM>
 __global__ __launch_bounds__(256) void plane_sums_kernel(const float *__restrict__ planes, const int32_t *__restrict__ count, const int32_t *__restrict__ hits,
                                                        const float *__restrict__ gy, const float *__restrict__ x, const float *__restrict__ folded,

@@ -686,8 +686,8 @@ static int launch_backward_4x4(const Geom &g, const void *x, const void *folded,
     while (ct > 1 && (g.c + ct - 1) / ct < 1024) ct >>= 1;
     const int sblocks = (g.n + kWave - 1) / kWave, waves = sblocks >= 4 ? 4 : (sblocks >= 2 ? 2 : 1);   // none without samples
     const size_t lds = (size_t)waves * kWave * kLsStride * sizeof(T);
-    // (a step of the CIFAR topology, us without and with: 25 MB 248 and 250, 32 MB 282 and 270, 50 MB 425 and 416, 512 MB 44 less; samples
-    // that are not whole lines within 1 % either way)
+    // (replayed step of the CIFAR topology, us without and with: 30 to 39 MB within 1 % but for 337 and 328 (k = 100, 96 images), 50 MB 404 and 395, 462 and 467, 64 MB
+    // 467 and 460, 512 MB 44 less; samples that are not whole lines within 1 % either way)
     const bool stream = clg_past_caches((int64_t)tg_elems_bytes(sizeof(T) == 8 ? CLG_F64 : CLG_F32, g), g.n % 8 == 0 ? 30 : 400);
     uint32_t *tcodes = reinterpret_cast<uint32_t *>(reinterpret_cast<unsigned char *>(tg) + tg_elems_bytes(sizeof(T) == 8 ? CLG_F64 : CLG_F32, g));
     auto main_kern = stream ? convblock_backward_4x4_kernel<T, true> : convblock_backward_4x4_kernel<T, false>;

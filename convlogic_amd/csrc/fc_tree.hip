@@ -482,8 +482,8 @@ static int tree_backward(const char *name, const float *x, const int32_t *rows, 
                 name);
     const int vec = tree_vec_dividing(pitch, x, rowgrad), gvec = tree_vec(pitch);
     hipStream_t st = clg_stream(stream_);
-    // Operand gradients: a step of the CIFAR topology, us through the caches and past them: rows of 1 KiB 62 MB 261 and 248, 80 MB 295 and 282, 160 MB 501 and 485,
-    // of 512 bytes 2.7 GB 4722 and 4550, no difference at 40.  Pieces of lines at the ends of rows cost what that gives: rows of 400 bytes, MNIST
+    // Operand gradients: replayed step of the CIFAR topology, us through the caches and past them: 60 to 82 MB within 1 % but for 274 and 267 (k = 64, 128 images, 80 MB),
+    // 94 MB 345 and 328, 100 MB 332 and 318, 125 MB 419 and 395, 160 MB 479 and 460, rows of 512 bytes 2.7 GB 4722 and 4550.  Pieces of lines at the ends of rows cost what that gives: rows of 400 bytes, MNIST
     // topology, 98 MB 229 and 232, 250 MB 519 and 495; of 508 bytes, which lanes write four at a time, 79 MB 194 and 216, of 804 294 MB 934 and 1002.
     const bool stream = pitch % 4 == 0 && clg_past_caches(roots * 8 * pitch * 4, pitch % 16 == 0 ? 48 : 200);
     const TreeGrads gr = {{grad0, grad1, grad2}, {4 * roots, 6 * roots, 7 * roots}};
