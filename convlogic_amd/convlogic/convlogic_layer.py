@@ -182,7 +182,7 @@ class _KeptPlan:
     """A backward plan of a layer, the selection it was made from (buffer and version) and whether a recording reads it."""
 
     def __init__(self):
-        self.plan = self.wiring = None
+        self.plan = self.wiring = self.wide = None
         self.recorded = False
 
     def make(self, like, sel, layer):
@@ -191,8 +191,9 @@ class _KeptPlan:
         wide = layer.taps_are_wide()
         look = convlogic_hip.LISTS_LOOK_NARROW if wide is False else convlogic_hip.LISTS_LOOK
         tables, lists = (None, look) if self.plan is None else (self.plan[0], convlogic_hip.lists_of(self.plan[1]))
-        if self.plan is not None and not self.recorded and wide != bool(lists & convlogic_hip.LISTS_WIDE):
+        if self.plan is not None and not self.recorded and wide != self.wide:
             tables, lists = None, look
+        self.wide = wide
         self.plan = convlogic_hip.make_backward_plan(like, layer.out_channels, sel, *layer.stride, *layer.padding, *layer.kernel, into=tables,
                                                      lists=lists)
 
@@ -245,7 +246,7 @@ class ConvLogicLayer(nn.Module):
             return
         if sel.dtype != torch.int32 or tuple(sel.shape) != (self.out_channels, 8):
             raise ValueError(f"selection must be int32 [{self.out_channels}, 8], got {sel.dtype} {tuple(sel.shape)}")
-        if sel.is_cuda and self.out_channels <= 4096:                # (one copy to the host: one wait for the device; large ones take longer to copy)
+        if sel.is_cuda and self.implementation == "cuda" and self.out_channels <= 4096:      # (one copy to the host: one wait for the device; large ones take longer to copy)
             inside, wide = convlogic_hip.look_at_selection(sel.cpu().contiguous(), self.in_channels, *self.kernel)
         else:
             (ch, row, col), wide = self.unpack_selection(sel), None

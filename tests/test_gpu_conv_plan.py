@@ -217,6 +217,21 @@ def test_taps_in_many_channels_take_the_kernels_without_planes(shape, monkeypatc
         assert kept.plan[1] == sig and all(torch.equal(a, b) for a, b in zip(got, want))
 
 
+@pytest.mark.parametrize("cout", [256, 4100])                          # (whose selections are, and are not, looked at on the host)
+def test_a_plan_is_made_again_in_its_place(cout):
+    layer = C.ConvLogicLayer(600 if cout > 4096 else 32, cout, padding=1, complete=True, implementation="cuda").to(DEV)
+    x = torch.rand(2, layer.in_channels, 6, 6, device=DEV)
+    before, sig = layer._backward_plan(x, layer.selection)
+    layer.selection.add_(0)                                           # (as a broadcast of the buffers does)
+    layer._check_selection()
+    after, again = layer._backward_plan(x, layer.selection)
+    assert after.data_ptr() == before.data_ptr() and again == sig and len(layer._plans) == 1
+    with torch.no_grad():
+        layer.selection[7, 3] = layer.in_channels << 16               # a channel outside
+    with pytest.raises(ValueError, match="outside"):
+        layer(x)
+
+
 @pytest.mark.parametrize("shape", [(256, 8, 32, 16), (300, 16, 128, 12)])
 def test_a_first_block_takes_no_gradient_planes(shape):
     n, cin, cout, side = shape
